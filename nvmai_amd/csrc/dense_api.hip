@@ -8,6 +8,42 @@ using namespace nvmai;
 
 namespace nvmai {
 
+// A float as three BF16 values that add up to it exactly (8 + 8 + 8 bits of mantissa, by truncation; below 2^-110 the
+// last bits may be lost).  Infinities and NaN stay in the first one.
+__device__ __forceinline__ void dense_split3(float x, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+    const uint32_t u = __float_as_uint(x);
+    const bool finite = (u & 0x7F800000u) != 0x7F800000u;
+    const float r1 = x - __uint_as_float(u & 0xFFFF0000u);
+    const float r2 = r1 - __uint_as_float(__float_as_uint(r1) & 0xFFFF0000u);
+    hi = (u >> 16) | (!finite && (u & 0x007FFFFFu) ? 0x40u : 0u);
+    mid = finite ? __float_as_uint(r1) >> 16 : 0u;
+    lo = finite ? __float_as_uint(r2) >> 16 : 0u;
+}
+
+// Rows of floats -> [row][3][k] BF16, the smallest part first.  Bound by its bytes (4 read, 6 written per value).
+__global__ __launch_bounds__(256) void dense_split_kernel(const float* x, uint32_t x_stride, uint32_t k, uint16_t* planes) {
+    const uint32_t at = (blockIdx.x * 256u + threadIdx.x) * 8u, row = blockIdx.y;
+    if (at >= k) return;
+    const float4 v[2] = {*reinterpret_cast<const float4*>(x + (size_t)row * x_stride + at), *reinterpret_cast<const float4*>(x + (size_t)row * x_stride + at + 4u)};
+    const float f[8] = {v[0].x, v[0].y, v[0].z, v[0].w, v[1].x, v[1].y, v[1].z, v[1].w};
+    uint32_t out[3][4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        uint32_t a[3], b[3];
+        dense_split3(f[2 * e], a[0], a[1], a[2]);
+        dense_split3(f[2 * e + 1], b[0], b[1], b[2]);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) out[q][e] = a[q] | (b[q] << 16);
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+        *reinterpret_cast<uint4*>(planes + ((size_t)row * 3u + (2 - q)) * k + at) = make_uint4(out[q][0], out[q][1], out[q][2], out[q][3]);
+}
+
+void dense_split(hipStream_t s, const float* x, uint32_t x_stride, uint32_t rows, uint32_t k, uint16_t* planes) {
+    dense_split_kernel<<<dim3((k + 2047) / 2048, rows), 256, 0, s>>>(x, x_stride, k, planes);
+}
+
 int dense_linear_check(const nvmai_hip_ctx* ctx, const DenseLinearParams& p) {
     if (!ctx || !p.w || !p.x || (!p.y && !p.y_f32)) return NVMAI_ERR_INVALID_ARG;
     if (ctx->act != NVMAI_ACT_BF16 && ctx->act != NVMAI_ACT_FP32) return NVMAI_ERR_UNSUPPORTED;
@@ -36,11 +72,29 @@ int dense_linear(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p) 
 
 }  // namespace nvmai
 
+namespace {
+
+// An entry point's own call: the planes of 32-bit rows lie in the workspace.  Where a stream that is being captured finds it
+// too small the product is made without them.
+int dense_linear_call(nvmai_hip_ctx* ctx, nvmai_stream stream, DenseLinearParams p) {
+    const int rc = dense_linear_check(ctx, p);
+    if (rc) return rc;
+    if (ctx->act == NVMAI_ACT_FP32 && p.rows > 4) {
+        const size_t bytes = dense_plane_bytes(p.rows, p.k);
+        const int got = ws_begin(ctx, stream, ws_round(bytes));
+        if (got == NVMAI_OK) p.planes = ws_take<uint16_t>(ctx, bytes / 2);
+        else if (got != NVMAI_ERR_SCRATCH) return got;
+    }
+    return dense_linear(ctx, (hipStream_t)stream, p);
+}
+
+}  // namespace
+
 extern "C" int nvmai_hip_dense_linear(nvmai_hip_ctx* ctx, nvmai_stream stream, const uint16_t* w, uint32_t w_stride,
                                       const void* x, uint32_t x_stride, uint32_t rows, uint32_t n, uint32_t k, void* y,
                                       float* y_f32, uint32_t y_stride, int activation) {
     const DenseLinearParams p{w, x, y, y_f32, w_stride, x_stride, y_stride, rows, n, k, activation};
-    return dense_linear(ctx, (hipStream_t)stream, p);
+    return dense_linear_call(ctx, stream, p);
 }
 
 extern "C" int nvmai_hip_dense_linear_ex(nvmai_hip_ctx* ctx, nvmai_stream stream, const uint16_t* w, uint32_t w_stride, const void* x,
@@ -49,7 +103,7 @@ extern "C" int nvmai_hip_dense_linear_ex(nvmai_hip_ctx* ctx, nvmai_stream stream
     if (!e) return NVMAI_ERR_INVALID_ARG;
     const DenseLinearParams p{w, x, y, y_f32, w_stride, x_stride, y_stride, rows, n, k, e->activation, e->bias, e->mul, e->mul_ids,
                               e->mul_stride, e->mul_rows};
-    return dense_linear(ctx, (hipStream_t)stream, p);
+    return dense_linear_call(ctx, stream, p);
 }
 
 extern "C" int nvmai_hip_embed_rows(nvmai_hip_ctx* ctx, nvmai_stream stream, const uint16_t* table, uint32_t table_stride,

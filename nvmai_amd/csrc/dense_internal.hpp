@@ -16,7 +16,19 @@ struct DenseLinearParams {
     const uint16_t* mul;    // BF16 table [mul_rows, mul_stride]: y[t, r] *= mul[mul_ids[t], r]; or nullptr
     const uint32_t* mul_ids;
     uint32_t mul_stride, mul_rows;
+    uint16_t* planes;       // dense_plane_bytes of scratch for the rows of a 32-bit context, or nullptr
 };
+
+// 32-bit rows are multiplied as three BF16 planes, at most this many rows (128 MB) at a time.
+inline uint32_t dense_plane_rows(uint32_t k) {
+    const uint32_t rows = (128u << 20) / (6u * k) / 256u * 256u;
+    return rows ? (rows < 32768u ? rows : 32768u) : 256u;
+}
+void dense_split(hipStream_t s, const float* x, uint32_t x_stride, uint32_t rows, uint32_t k, uint16_t* planes);
+inline size_t dense_plane_bytes(uint32_t rows, uint32_t k) {
+    const uint32_t most = dense_plane_rows(k);
+    return (size_t)(rows < most ? rows : most) * k * 6u;
+}
 
 int dense_linear_check(const nvmai_hip_ctx* ctx, const DenseLinearParams& p);
 // The launches behind it by what stands between sum and store (dense_*_api.hip, built side by side).
@@ -24,6 +36,7 @@ int dense_launch_erf(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams&
 int dense_launch_bias(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p);
 int dense_launch_pairs(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p);
 int dense_launch_full(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p);
+// Launches it.  In a 32-bit context p.planes is the caller's scratch: a call between ws_takes must not start the workspace anew.
 int dense_linear(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p);
 
 }  // namespace nvmai

@@ -17,24 +17,87 @@ __device__ __forceinline__ dn_f4 dn_mfma(const uint4& a, const uint4& b, dn_f4 c
 // z/2 (1 + erf(z / sqrt 2))
 __device__ __forceinline__ float gelu_erf(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
 
+// The same by formula 7.1.26 of Abramowitz and Stegun, erfc(x) = (a1 t + .. + a5 t^5) e^(-x^2), t = 1 / (1 + p x), off by at most
+// 1.5e-7: about a third of erff's instructions and no branch, for results of 16-bit contexts.  z < 0 takes erfc itself (one
+// minus erf would cancel).
+__device__ __forceinline__ float gelu_erf_fast(float z) {
+    const float x = fabsf(z) * 0.70710678118654752f, t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, x, 1.0f));
+    const float poly = t * fmaf(t, fmaf(t, fmaf(t, fmaf(t, 1.061405429f, -1.453152027f), 1.421413741f), -0.284496736f), 0.254829592f);
+    const float c = poly * __builtin_amdgcn_exp2f(-1.4426950408889634f * x * x);
+    return 0.5f * z * (z < 0.0f ? c : 2.0f - c);
+}
+
 // z/2 (1 + tanh(sqrt(2/pi) (z + 0.044715 z^3)))
 __device__ __forceinline__ float gelu_tanh(float z) { return 0.5f * z * (1.0f + tanhf(0.79788456080286536f * fmaf(0.044715f * z * z, z, z))); }
+
+// z / (1 + e^(-2 u)), which is the same, through the hardware's exponential and reciprocal: for results of 16-bit contexts.
+__device__ __forceinline__ float gelu_tanh_fast(float z) {
+    const float u = 0.79788456080286536f * fmaf(0.044715f * z * z, z, z);
+    return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-2.8853900817779268f * u));
+}
 
 // What stands between a sum and its store, fixed when a kernel is built: a tile's store is unrolled many times, and code
 // that a call does not need costs instruction fetches in all of them.  PLAIN: the activation NONE; ERF: GELU_ERF; BIAS: a
 // bias; PAIRS: SILU_PAIRS; FULL: bias, any activation, the token's own multiplier.
 enum DenseEpilogue : int { DE_PLAIN, DE_ERF, DE_BIAS, DE_PAIRS, DE_FULL };
 
-template <int EPI>
+template <int ACT>
+__device__ __forceinline__ float dense_activate(int activation, float v) {
+    if (activation == NVMAI_LINEAR_GELU_ERF) return ACT == ACT_FP32 ? gelu_erf(v) : gelu_erf_fast(v);
+    if (activation == NVMAI_LINEAR_GELU_TANH) return ACT == ACT_FP32 ? gelu_tanh(v) : gelu_tanh_fast(v);
+    return v;
+}
+
+template <int EPI, int ACT>
 __device__ __forceinline__ float dense_finish(const DenseLinearParams& p, uint32_t t, uint32_t r, float v) {
-    if (EPI == DE_ERF) return gelu_erf(v);
+    if (EPI == DE_ERF) return dense_activate<ACT>(NVMAI_LINEAR_GELU_ERF, v);
     if (EPI == DE_BIAS) return v + bf16_to_f32(p.bias[r]);
     if (EPI != DE_FULL) return v;
     if (p.bias) v += bf16_to_f32(p.bias[r]);
-    v = p.activation == NVMAI_LINEAR_GELU_ERF ? gelu_erf(v) : p.activation == NVMAI_LINEAR_GELU_TANH ? gelu_tanh(v) : v;
+    v = dense_activate<ACT>(p.activation, v);
     if (p.mul) {                                     // an id past the table: zero
         const uint32_t id = p.mul_ids[t];
         v *= id < p.mul_rows ? bf16_to_f32(p.mul[(size_t)id * p.mul_stride + r]) : 0.0f;
+    }
+    return v;
+}
+
+// The biases of four neighbouring rows (r0 a multiple of 4; past the matrix: what is there is not used).
+template <int EPI>
+__device__ __forceinline__ dn_f4 dense_bias4(const DenseLinearParams& p, uint32_t r0) {
+    dn_f4 b{0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (EPI == DE_BIAS || EPI == DE_FULL) {
+        if (p.bias && r0 + 4u <= p.n)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) b[j] = bf16_to_f32(p.bias[r0 + j]);
+    }
+    return b;
+}
+
+// dense_finish of four neighbouring rows whose biases the caller holds.
+template <int EPI, int ACT>
+__device__ __forceinline__ dn_f4 dense_finish4(const DenseLinearParams& p, uint32_t t, uint32_t r0, dn_f4 v, dn_f4 bias) {
+    if constexpr (EPI == DE_FULL) {
+        dn_f4 m{1.0f, 1.0f, 1.0f, 1.0f};
+        if (p.mul) {
+            const uint32_t id = p.mul_ids[t];
+            const uint16_t* at = p.mul + (size_t)min(id, p.mul_rows - 1u) * p.mul_stride + r0;
+            const float live = id < p.mul_rows ? 1.0f : 0.0f;
+            if ((reinterpret_cast<uintptr_t>(p.mul) & 7u) == 0 && (p.mul_stride & 3u) == 0) {
+                const uint2 q = *reinterpret_cast<const uint2*>(at);
+                m = dn_f4{__uint_as_float(q.x << 16), __uint_as_float(q.x & 0xFFFF0000u), __uint_as_float(q.y << 16), __uint_as_float(q.y & 0xFFFF0000u)};
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) m[j] = bf16_to_f32(at[j]);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) m[j] = live != 0.0f ? m[j] : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = dense_activate<ACT>(p.activation, v[j] + bias[j]) * m[j];
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = EPI == DE_ERF ? dense_activate<ACT>(NVMAI_LINEAR_GELU_ERF, v[j]) : EPI == DE_BIAS ? v[j] + bias[j] : v[j];
     }
     return v;
 }
@@ -47,7 +110,7 @@ __device__ __forceinline__ void dense_put(const DenseLinearParams& p, uint32_t t
 
 template <int EPI, int ACT>
 __device__ __forceinline__ void dense_store(const DenseLinearParams& p, uint32_t t, uint32_t r, float v) {
-    dense_put<ACT>(p, t, r, dense_finish<EPI>(p, t, r, v));
+    dense_put<ACT>(p, t, r, dense_finish<EPI, ACT>(p, t, r, v));
 }
 
 // Rows 2 j and 2 j + 1 of the matrix make output j: silu(gate) * up.
@@ -55,30 +118,38 @@ template <int ACT>
 __device__ __forceinline__ float dense_pair(float gate, float up) { return (ACT == ACT_FP32 ? silu(gate) : silu_fast(gate)) * up; }
 
 // Four neighbouring outputs of one token (r0 a multiple of 4).
-template <int EPI>
-__device__ __forceinline__ void dense_store4_bf16(const DenseLinearParams& p, uint32_t t, uint32_t r0, dn_f4 v) {
+template <int EPI, int ACT>
+__device__ __forceinline__ void dense_store4(const DenseLinearParams& p, uint32_t t, uint32_t r0, dn_f4 v, dn_f4 bias) {
     if (EPI == DE_PAIRS) {                           // n and the row stride are even
-        const float a = dense_pair<ACT_BF16>(v[0], v[1]), b = dense_pair<ACT_BF16>(v[2], v[3]);
+        const float a = dense_pair<ACT>(v[0], v[1]), b = dense_pair<ACT>(v[2], v[3]);
         if (r0 + 4u <= p.n) {
-            if (p.y) *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(p.y) + (size_t)t * p.y_stride + r0 / 2u) = f32_to_bf16(a) | ((uint32_t)f32_to_bf16(b) << 16);
+            if (p.y) {
+                act_t<ACT>* y = static_cast<act_t<ACT>*>(p.y) + (size_t)t * p.y_stride + r0 / 2u;
+                if constexpr (ACT == ACT_FP32) *reinterpret_cast<float2*>(y) = float2{a, b};
+                else *reinterpret_cast<uint32_t*>(y) = f32_to_bf16(a) | ((uint32_t)f32_to_bf16(b) << 16);
+            }
             if (p.y_f32) *reinterpret_cast<float2*>(p.y_f32 + (size_t)t * p.y_stride + r0 / 2u) = float2{a, b};
         } else if (r0 < p.n) {
-            dense_put<ACT_BF16>(p, t, r0 / 2u, a);
+            dense_put<ACT>(p, t, r0 / 2u, a);
         }
     } else if (r0 + 4u <= p.n && (p.y_stride & 3u) == 0) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = dense_finish<EPI>(p, t, r0 + j, v[j]);
+        v = dense_finish4<EPI, ACT>(p, t, r0, v, bias);
         if (p.y) {
-            uint2 q;
-            q.x = f32_to_bf16(v[0]) | ((uint32_t)f32_to_bf16(v[1]) << 16);
-            q.y = f32_to_bf16(v[2]) | ((uint32_t)f32_to_bf16(v[3]) << 16);
-            *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.y) + (size_t)t * p.y_stride + r0) = q;
+            act_t<ACT>* y = static_cast<act_t<ACT>*>(p.y) + (size_t)t * p.y_stride + r0;
+            if constexpr (ACT == ACT_FP32) {
+                *reinterpret_cast<dn_f4*>(y) = v;
+            } else {
+                uint2 q;
+                q.x = f32_to_bf16(v[0]) | ((uint32_t)f32_to_bf16(v[1]) << 16);
+                q.y = f32_to_bf16(v[2]) | ((uint32_t)f32_to_bf16(v[3]) << 16);
+                *reinterpret_cast<uint2*>(y) = q;
+            }
         }
         if (p.y_f32) *reinterpret_cast<dn_f4*>(p.y_f32 + (size_t)t * p.y_stride + r0) = v;
     } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-            if (r0 + j < p.n) dense_store<EPI, ACT_BF16>(p, t, r0 + j, v[j]);
+            if (r0 + j < p.n) dense_store<EPI, ACT>(p, t, r0 + j, v[j]);
     }
 }
 
@@ -221,91 +292,191 @@ __global__ __launch_bounds__(64 * NW) void dense_skinny_kernel(DenseLinearParams
 #pragma unroll
             for (int w = 0; w < NW - 1; ++w) acc[r][t] += *reinterpret_cast<const dn_f4*>(&part[w][lane][4 * (r * TT + t)]);
             // acc[r][t][j] = y[token 16 t + i, row r0 + 16 r + 4 g + j]
-            if (16u * t + i < p.rows) dense_store4_bf16<EPI>(p, 16u * t + i, r0 + 16u * r + 4u * g, acc[r][t]);
+            if (16u * t + i < p.rows) dense_store4<EPI, ACT_BF16>(p, 16u * t + i, r0 + 16u * r + 4u * g, acc[r][t], dense_bias4<EPI>(p, r0 + 16u * r + 4u * g));
         }
 }
 
-// ---- many input rows: tiles of BN weight rows x BM tokens, k in steps of 64 through double-buffered LDS --------
-// Four waves, each a quarter of the tile (BN / 2 x BM / 2) in 16 x 16 x 32 products.  A tile's rows are 128 bytes
-// of LDS; the eight 16-byte pieces of row r lie in the order piece ^ (r % 8), so that the sixteen rows of an
-// operand read fall into different banks.  Loads go straight from memory into LDS.
-template <int EPI, int BN, int BM>
-__global__ __launch_bounds__(256) void dense_gemm_kernel(DenseLinearParams p, uint32_t tiles_n, uint32_t tiles_m) {
-    constexpr int LA = BN / 32, LB = BM / 32;                // 1 KB pieces per wave
-    constexpr int TN = BN / 32, TM = BM / 32;                // 16 x 16 tiles per wave
+// ---- many input rows: tiles of BN weight rows x BM tokens, k in steps of 64 through a ring of S stages in LDS ----------
+// Four waves, each a quarter of the tile (BN / 2 x BM / 2) in 32 x 32 x 16 products.  Bound by the rate at which a compute
+// unit takes operands into LDS (about 60 bytes per ns; a tile of 256 x 256 is where the products take as long) and, below
+// one tile per compute unit, by the latency of a step.  A tile's rows are 128 bytes of LDS; the eight 16-byte pieces of
+// row r lie in the order piece ^ (r % 8), so that the rows of an operand read fall into different banks.
+//   A stage is multiplied in four phases of 16 k.  The operands of the next phase are read, and a quarter of the stage S - 1
+// ahead is requested, between the products of a phase: a wave alone on its SIMD has products to issue at all times, and
+// requests spread over the phases keep the wave from waiting at the memory pipe (in one burst behind the barrier: 96 us for
+// 2048 x 2048 x 8192 in tiles of 256 x 128, spread 93, and 125 with a branch around the burst).  One barrier per stage,
+// before its last phase: by then every wave has read the stage to its end (its place is free for stage + S) and waits for
+// its own part of the next one.  Requests are never conditional, so the counter's meaning is the same in every step; a
+// stage past the last reads no bytes (a buffer of size 0).  Stages are separate arrays: the compiler then knows
+// which requests a read of LDS has to wait for.
+//   32-bit activations come as three BF16 planes (dense_split), [row][plane][k], the smallest first: the products of a step
+// of 64 k are exact, and their sum goes to a running total of its own, which keeps the rounding of a long k small.
+// Measured (tiles of 128 x 128 x 64 in two stages before): 2048 x 8192 x 2048 77 -> 61 us, 2048 x 2048 x 8192 140 -> 67, 1501 x
+// 2048 x 2048 34 -> 17, 512 x 2048 x 2048 33 -> 9.5 (rows x n x k, cold weights).
+typedef float dn_f16 __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ dn_f16 dn_mfma32(const uint4& a, const uint4& b, dn_f16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(dn_b8, a), __builtin_bit_cast(dn_b8, b), c, 0, 0, 0);
+}
+
+// Every read of LDS done, all but the last N requests landed, for every wave of the block.
+template <int N>
+__device__ __forceinline__ void dense_stage_barrier() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"(N) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#endif
+}
+
+constexpr int dense_stages(int act, int bn, int bm) {        // of 160 KB; two blocks per compute unit where the tile is small
+    return act == ACT_FP32 ? 3 : bn + bm <= 192 ? 5 : bn + bm <= 256 ? 4 : bn + bm <= 384 ? 3 : 2;
+}
+
+template <int EPI, int ACT, int BN, int BM>
+__global__ __launch_bounds__(256, BN + BM <= 128 ? 2 : 1) void dense_tile_kernel(DenseLinearParams p, uint32_t tiles_n, uint32_t tiles_m) {
+    constexpr bool SPLIT = ACT == ACT_FP32;
+    constexpr int S = dense_stages(ACT, BN, BM);
+    constexpr int LA = BN / 32, LB = BM / 32, L = LA + LB;   // 1 KB requests per wave and stage
+    constexpr int TN = BN / 64, TM = BM / 64;                // 32 x 32 tiles per wave
     constexpr uint32_t STAGE = (BN + BM) * 128u;
-    __shared__ __attribute__((aligned(16))) uint8_t lds[2 * STAGE];
+    __shared__ __attribute__((aligned(1024))) uint8_t l0[STAGE], l1[STAGE], l2[S > 2 ? STAGE : 16], l3[S > 3 ? STAGE : 16], l4[S > 4 ? STAGE : 16];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // blocks are dealt to the eight XCDs in turn: give each XCD a run of neighbouring tiles (shared L2 lines)
-    const uint32_t total = tiles_n * tiles_m, xcd = blockIdx.x & 7u, nth = blockIdx.x >> 3;
-    const uint32_t base = total / 8u, extra = total % 8u;
+    const uint32_t all = tiles_n * tiles_m, xcd = blockIdx.x & 7u, nth = blockIdx.x >> 3;
+    const uint32_t base = all / 8u, extra = all % 8u;
     const uint32_t tile = xcd * base + min(xcd, extra) + nth;
     // in bands of eight token tiles, weight tiles outermost within the band
     const uint32_t band = tile / (8u * tiles_n), in_band = tile % (8u * tiles_n);
     const uint32_t band_m = min(8u, tiles_m - band * 8u);
     const uint32_t m0 = (band * 8u + in_band % band_m) * BM, n0 = (in_band / band_m) * BN;
 
-    [[maybe_unused]] const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(p.w), 0, (int)(uint32_t)((size_t)(p.n - 1u) * p.w_stride * 2u + p.k * 2u), 0x00020000);
-    [[maybe_unused]] const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<void*>(p.x), 0, (int)(uint32_t)((size_t)(p.rows - 1u) * p.x_stride * 2u + p.k * 2u), 0x00020000);
-    uint32_t aoff[LA], boff[LB];
-    const uint32_t lr = lane >> 3, piece = (lane & 7u) ^ (lr & 7u);
-#pragma unroll
-    for (int j = 0; j < LA; ++j) aoff[j] = min(n0 + (wave * LA + j) * 8u + lr, p.n - 1u) * p.w_stride * 2u + piece * 16u;
-#pragma unroll
-    for (int j = 0; j < LB; ++j) boff[j] = min(m0 + (wave * LB + j) * 8u + lr, p.rows - 1u) * p.x_stride * 2u + piece * 16u;
-    auto issue = [&](uint32_t st, uint8_t* dst) {
+    const uint32_t steps = p.k / 64u * (SPLIT ? 3u : 1u);
+    [[maybe_unused]] const uint32_t w_bytes = (p.n - 1u) * p.w_stride * 2u + p.k * 2u;
+    [[maybe_unused]] const uint32_t x_bytes = (p.rows - 1u) * p.x_stride * 2u + p.k * (SPLIT ? 6u : 2u);
+    const uint32_t lr = lane >> 3, piece = ((lane & 7u) ^ (lr & 7u)) * 16u;
+    // rows past the last: the last one, whose sums are not stored
+    [[maybe_unused]] const uint32_t a8 = p.w_stride * 16u, a0 = (n0 + wave * (LA * 8u) + lr) * p.w_stride * 2u + piece, amax = (p.n - 1u) * p.w_stride * 2u + piece;
+    [[maybe_unused]] const uint32_t b8 = p.x_stride * 16u, b0 = (m0 + wave * (LB * 8u) + lr) * p.x_stride * 2u + piece, bmax = (p.rows - 1u) * p.x_stride * 2u + piece;
+    auto buf = [&](int j) -> uint8_t* { return j == 0 ? l0 : j == 1 ? l1 : j == 2 ? l2 : j == 3 ? l3 : l4; };
+    // requests [from, to) of stage st into its place j = st % S (the plane of a 32-bit input, S = 3)
+    auto request = [&](uint32_t st, int j, int from, int to) {
 #if defined(__HIP_DEVICE_COMPILE__)     // the host pass rejects the 16-byte form of the load
+        const bool live = st < steps;
+        const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.w), 0, live ? (int)w_bytes : 0, 0x00020000);
+        const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.x), 0, live ? (int)x_bytes : 0, 0x00020000);
+        const uint32_t wk = (SPLIT ? st / 3u : st) * 128u, xk = SPLIT ? wk + j * p.k * 2u : wk;
+        uint8_t* dst = buf(j);
 #pragma unroll
-        for (int j = 0; j < LA; ++j)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (__attribute__((address_space(3))) void*)(dst + (wave * LA + j) * 1024u), 16, aoff[j], st * 128u, 0, 0);
-#pragma unroll
-        for (int j = 0; j < LB; ++j)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (__attribute__((address_space(3))) void*)(dst + BN * 128u + (wave * LB + j) * 1024u), 16, boff[j], st * 128u, 0, 0);
+        for (int r = 0; r < L; ++r) {
+            if (r < from || r >= to) continue;
+            if (r < LA) __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (__attribute__((address_space(3))) void*)(dst + (wave * LA + r) * 1024u), 16, min(a0 + r * a8, amax), wk, 0, 0);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void*)(dst + BN * 128u + (wave * LB + r - LA) * 1024u), 16, min(b0 + (r - LA) * b8, bmax), xk, 0, 0);
+        }
 #endif
     };
-    dn_f4 acc[TN][TM];
+    const uint32_t i = lane & 31u, g = lane >> 5;
+    const uint32_t wn = (wave >> 1) * (BN / 2), wm = (wave & 1u) * (BM / 2);
+    const uint32_t arow = (wn + i) * 128u, brow = BN * 128u + (wm + i) * 128u;
+    uint4 fa[2][TN], fb[2][TM];
+    auto fetch = [&](int j, uint32_t q) {                    // the operands of phase q of the stage at place j
+        const uint32_t sw = ((q * 2u + g) ^ (i & 7u)) * 16u;
+#pragma unroll
+        for (int b = 0; b < TM; ++b) fb[q & 1u][b] = *reinterpret_cast<const uint4*>(buf(j) + brow + 4096u * b + sw);
+#pragma unroll
+        for (int a = 0; a < TN; ++a) fa[q & 1u][a] = *reinterpret_cast<const uint4*>(buf(j) + arow + 4096u * a + sw);
+    };
+    dn_f16 acc[TN][TM];
+    [[maybe_unused]] dn_f16 total[SPLIT ? TN : 1][SPLIT ? TM : 1];
 #pragma unroll
     for (int a = 0; a < TN; ++a)
 #pragma unroll
-        for (int b = 0; b < TM; ++b) acc[a][b] = dn_f4{0.0f, 0.0f, 0.0f, 0.0f};
-    const uint32_t i = lane & 15u, g = lane >> 4;
-    const uint32_t wn = (wave >> 1) * (BN / 2), wm = (wave & 1u) * (BM / 2);
-    const uint32_t steps = p.k / 64u;
-    issue(0, lds);
-    __syncthreads();
-    for (uint32_t st = 0; st < steps; ++st) {
-        uint8_t* cur = lds + (st & 1u) * STAGE;
-        if (st + 1u < steps) issue(st + 1u, lds + ((st + 1u) & 1u) * STAGE);
-#pragma unroll
-        for (uint32_t ks = 0; ks < 2; ++ks) {
-            const uint32_t sw = ((ks * 4u + g) ^ (i & 7u)) * 16u;
-            uint4 af[TN], bf[TM];
-#pragma unroll
-            for (int a = 0; a < TN; ++a) af[a] = *reinterpret_cast<const uint4*>(cur + (wn + 16 * a + i) * 128u + sw);
-#pragma unroll
-            for (int b = 0; b < TM; ++b) bf[b] = *reinterpret_cast<const uint4*>(cur + BN * 128u + (wm + 16 * b + i) * 128u + sw);
-#pragma unroll
-            for (int a = 0; a < TN; ++a)
-#pragma unroll
-                for (int b = 0; b < TM; ++b) acc[a][b] = dn_mfma(af[a], bf[b], acc[a][b]);
+        for (int b = 0; b < TM; ++b) {
+            acc[a][b] = dn_f16{};
+            if constexpr (SPLIT) total[a][b] = dn_f16{};
         }
-        __syncthreads();                 // the next stage has landed, this one may be overwritten
+    auto multiply = [&](int q, auto requests, bool fresh) {
+        constexpr int NP = TN * TM, NF = TN + TM, NR = decltype(requests)::value;
+#pragma unroll
+        for (int a = 0; a < TN; ++a)
+#pragma unroll
+            for (int b = 0; b < TM; ++b) acc[a][b] = dn_mfma32(fa[q & 1][a], fb[q & 1][b], fresh ? dn_f16{} : acc[a][b]);
+#pragma unroll
+        for (int k = 0; k < NP; ++k) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);                                     // a product,
+            __builtin_amdgcn_sched_group_barrier(0x100, (NF + NP - 1) / NP, 0);                  // the next phase's operands,
+            if constexpr (NR > 0) __builtin_amdgcn_sched_group_barrier(0x20, (NR + NP - 1) / NP, 0);  // and the requests
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+#define NVMAI_SHARE(q) (L * (q) / 4)
+    auto step = [&](uint32_t st, int j) {
+        constexpr int B = S - 1;
+        fetch(j, 1);
+        request(st + B, (j + B) % S, NVMAI_SHARE(1), NVMAI_SHARE(2));
+        multiply(0, std::integral_constant<int, NVMAI_SHARE(2) - NVMAI_SHARE(1)>{}, SPLIT && j == 0);
+        fetch(j, 2);
+        request(st + B, (j + B) % S, NVMAI_SHARE(2), NVMAI_SHARE(3));
+        multiply(1, std::integral_constant<int, NVMAI_SHARE(3) - NVMAI_SHARE(2)>{}, false);
+        fetch(j, 3);
+        request(st + B, (j + B) % S, NVMAI_SHARE(3), NVMAI_SHARE(4));
+        multiply(2, std::integral_constant<int, NVMAI_SHARE(4) - NVMAI_SHARE(3)>{}, false);
+        dense_stage_barrier<(S - 2) * L>();
+        fetch((j + 1) % S, 0);
+        request(st + S, j, 0, NVMAI_SHARE(1));
+        multiply(3, std::integral_constant<int, NVMAI_SHARE(1)>{}, false);
+        if constexpr (SPLIT) {
+            if (j == 2) {
+#pragma unroll
+                for (int a = 0; a < TN; ++a)
+#pragma unroll
+                    for (int b = 0; b < TM; ++b) total[a][b] += acc[a][b];
+            }
+        }
+    };
+#pragma unroll
+    for (int j = 0; j < S; ++j) request(j, j, 0, j == S - 1 ? NVMAI_SHARE(1) : L);
+    dense_stage_barrier<(S - 2) * L + NVMAI_SHARE(1)>();
+#undef NVMAI_SHARE
+    fetch(0, 0);
+    uint32_t st = 0;
+    for (; st + (uint32_t)S <= steps; st += S) {
+#pragma unroll
+        for (int j = 0; j < S; ++j) step(st + j, j);
     }
 #pragma unroll
+    for (int j = 0; j < S - 1; ++j)
+        if (st + (uint32_t)j < steps) step(st + j, j);
+    dense_stage_barrier<0>();                                // no request outlives its block; the stages' places are free
+    // The sums change places through LDS, 32 tokens of the wave's part at a time, so that neighbouring lanes hold
+    // neighbouring outputs of one token (stores of whole lines) and what stands between sum and store is a short loop: unrolled
+    // over the sums of a tile it is longer than the instruction cache (GELU on 256 x 128: 122 us instead of 71 for 2048 x 8192 x 2048).
+    constexpr uint32_t ROWS = BN / 2, PITCH = ROWS + 4, PER = ROWS / 4, AT_ONCE = 64 / PER;
+    constexpr int UNROLL = EPI == DE_ERF ? 2 : 4;
+    float* turn = reinterpret_cast<float*>((wave & 1u) ? l1 : l0) + (wave >> 1) * (32u * PITCH);
+    static_assert(2u * 32u * PITCH * 4u <= STAGE, "two waves per stage");
+    const uint32_t r = n0 + wn + lane % PER * 4u;
+    const dn_f4 bias = dense_bias4<EPI>(p, r);
+#pragma unroll
     for (int b = 0; b < TM; ++b) {
-        const uint32_t t = m0 + wm + 16 * b + i;
-        if (t >= p.rows) continue;
 #pragma unroll
         for (int a = 0; a < TN; ++a) {
-            const uint32_t r = n0 + wn + 16 * a + 4u * g;
-            if (r < p.n) dense_store4_bf16<EPI>(p, t, r, acc[a][b]);
+            dn_f16 v = acc[a][b];
+            if constexpr (SPLIT) v = total[a][b];
+#pragma unroll
+            for (int h = 0; h < 4; ++h)                      // element 4 h + e of a lane: row 8 h + 4 g + e, token i
+                *reinterpret_cast<dn_f4*>(turn + i * PITCH + 32 * a + 8 * h + 4u * g) = dn_f4{v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]};
+        }
+#pragma unroll UNROLL
+        for (uint32_t k = 0; k < 32u / AT_ONCE; ++k) {
+            const uint32_t at = lane / PER + k * AT_ONCE, t = m0 + wm + 32 * b + at;
+            const dn_f4 v = *reinterpret_cast<const dn_f4*>(turn + at * PITCH + lane % PER * 4u);
+            if (t < p.rows && r < p.n) dense_store4<EPI, ACT>(p, t, r, v, bias);
         }
     }
 }
 
-// ---- 32-bit activations, more than four rows: 64 x 64 tiles on the vector pipe, BF16 weights widened, fp32 FMA ------------
+// ---- 32-bit activations, more than four rows, no place for their planes (a call that is captured before any other has
+// sized the workspace): 64 x 64 tiles on the vector pipe, BF16 weights widened, fp32 FMA ---------------------------------
 // Sums are two-level (a step of 16 k, then the running total), which keeps the rounding error of a long k small.
 template <int EPI>
 __global__ __launch_bounds__(256) void dense_f32_kernel(DenseLinearParams p) {
@@ -369,12 +540,105 @@ int gemv(const DenseLinearParams& p, hipStream_t s) {
     return launch_status();
 }
 
+// Which tile: the one whose rounds over the compute units take the least time.  A step of 64 k takes `full` where every unit
+// has a tile and `lone` where few have one (in 10 ns; measured at k 2048 and 8192 over 65 .. 4096 rows and 256 .. 11264 weight
+// rows: the choice is the fastest of the five or within a tenth of it).  Large tiles read each operand less often, small
+// ones leave fewer units idle.
+struct DenseTile {
+    uint32_t bn, bm, lone, full;
+};
+constexpr DenseTile DENSE_TILES[] = {{64, 64, 19, 21}, {128, 64, 24, 34}, {128, 128, 30, 55}, {256, 128, 50, 100}, {256, 256, 115, 185}};
+
+struct DensePlan {
+    int tile;
+    uint64_t ns;
+};
+
+inline DensePlan dense_plan_tile(uint32_t n, uint32_t rows, uint32_t steps, uint32_t cus, int count) {
+    DensePlan best{0, ~0ull};
+    for (int c = 0; c < count; ++c) {
+        const DenseTile& t = DENSE_TILES[c];
+        const uint64_t tiles = (uint64_t)((n + t.bn - 1) / t.bn) * ((rows + t.bm - 1) / t.bm), rest = tiles % cus;
+        const uint64_t cost = tiles / cus * t.full + (rest ? t.lone + (t.full - t.lone) * rest / cus : 0);
+        const uint64_t ns = cost * 10 * steps + 4000;        // and a launch, the first requests, the stores
+        if (ns < best.ns) best = {c, ns};
+    }
+    return best;
+}
+
+// The matrix's rows in one launch, or in two where that is shorter: a last round that few units take part in is left to
+// smaller tiles (8208 weight rows, 2048 tokens: one round of 256 x 256 and a sixteenth of one, 105 -> 76 us in all).
+// Returns how many rows the first launch takes.
+inline uint32_t dense_plan(uint32_t n, uint32_t rows, uint32_t steps, uint32_t cus, int count) {
+    DensePlan best = dense_plan_tile(n, rows, steps, cus, count);
+    uint32_t first = n;
+    for (int c = 0; c < count; ++c) {
+        const uint32_t tm = (rows + DENSE_TILES[c].bm - 1) / DENSE_TILES[c].bm, tn = n / DENSE_TILES[c].bn;
+        const uint32_t rounds = (uint32_t)((uint64_t)tn * tm / cus);
+        const uint32_t cut = rounds ? (uint32_t)((uint64_t)rounds * cus / tm) * DENSE_TILES[c].bn : 0;
+        if (cut == 0 || cut >= n) continue;
+        const uint64_t ns = dense_plan_tile(cut, rows, steps, cus, count).ns + dense_plan_tile(n - cut, rows, steps, cus, count).ns;
+        if (ns < best.ns) { best.ns = ns; first = cut; }
+    }
+    return first;
+}
+
+template <int EPI, int ACT, int COUNT>
+void launch_tile(hipStream_t s, const DenseLinearParams& p, int c) {
+    const uint32_t tn = (p.n + DENSE_TILES[c].bn - 1) / DENSE_TILES[c].bn, tm = (p.rows + DENSE_TILES[c].bm - 1) / DENSE_TILES[c].bm;
+    if (c == 0) dense_tile_kernel<EPI, ACT, 64, 64><<<tn * tm, 256, 0, s>>>(p, tn, tm);
+    else if (c == 1) dense_tile_kernel<EPI, ACT, 128, 64><<<tn * tm, 256, 0, s>>>(p, tn, tm);
+    else if (c == 2) dense_tile_kernel<EPI, ACT, 128, 128><<<tn * tm, 256, 0, s>>>(p, tn, tm);
+    if constexpr (COUNT > 3) {
+        if (c == 3) dense_tile_kernel<EPI, ACT, 256, 128><<<tn * tm, 256, 0, s>>>(p, tn, tm);
+        else if (c == 4) dense_tile_kernel<EPI, ACT, 256, 256><<<tn * tm, 256, 0, s>>>(p, tn, tm);
+    }
+}
+
+template <int EPI, int ACT>
+void launch_tiles(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p) {
+    constexpr int COUNT = ACT == ACT_FP32 ? 3 : 5;           // 32-bit inputs keep a running total beside the sums: no registers for the larger tiles
+    const uint32_t cus = (uint32_t)ctx->compute_units, steps = p.k / 64u * (ACT == ACT_FP32 ? 3u : 1u);
+    const uint32_t first = dense_plan(p.n, p.rows, steps, cus, COUNT);
+    DenseLinearParams q = p;
+    q.n = first;
+    launch_tile<EPI, ACT, COUNT>(s, q, dense_plan_tile(q.n, q.rows, steps, cus, COUNT).tile);
+    if (first == p.n) return;
+    q.n = p.n - first;                                       // first is a multiple of 64: every operand stays aligned
+    q.w = p.w + (size_t)first * p.w_stride;
+    const uint32_t out = EPI == DE_PAIRS ? first / 2 : first;
+    if (p.y) q.y = static_cast<act_t<ACT>*>(p.y) + out;
+    if (p.y_f32) q.y_f32 = p.y_f32 + out;
+    if (p.bias) q.bias = p.bias + first;
+    if (p.mul) q.mul = p.mul + first;
+    launch_tile<EPI, ACT, COUNT>(s, q, dense_plan_tile(q.n, q.rows, steps, cus, COUNT).tile);
+}
+
+// 32-bit inputs: their planes, in portions of rows, then the product.
+template <int EPI>
+int launch_split(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p) {
+    const uint32_t most = dense_plane_rows(p.k);
+    for (uint32_t at = 0; at < p.rows; at += most) {
+        DenseLinearParams q = p;
+        q.rows = p.rows - at < most ? p.rows - at : most;
+        dense_split(s, static_cast<const float*>(p.x) + (size_t)at * p.x_stride, p.x_stride, q.rows, p.k, p.planes);
+        q.x = p.planes;
+        q.x_stride = 3 * p.k;
+        if (p.y) q.y = static_cast<float*>(p.y) + (size_t)at * p.y_stride;
+        if (p.y_f32) q.y_f32 = p.y_f32 + (size_t)at * p.y_stride;
+        if (p.mul_ids) q.mul_ids = p.mul_ids + at;
+        launch_tiles<EPI, ACT_FP32>(ctx, s, q);
+    }
+    return launch_status();
+}
+
 template <int EPI>
 int dense_launch(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p) {
     if (p.rows <= 4) return ctx->act == NVMAI_ACT_FP32 ? gemv<EPI, ACT_FP32>(p, s) : gemv<EPI, ACT_BF16>(p, s);
     if (ctx->act == NVMAI_ACT_FP32) {
         const dim3 grid((p.n + 63) / 64, (p.rows + 63) / 64);
         if (grid.y > 65535) return NVMAI_ERR_UNSUPPORTED;
+        if (p.planes) return launch_split<EPI>(ctx, s, p);
         dense_f32_kernel<EPI><<<grid, 256, 0, s>>>(p);
         return launch_status();
     }
@@ -396,17 +660,7 @@ int dense_launch(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p) 
 #undef NVMAI_SKINNY
         return launch_status();
     }
-    // the largest tile that still gives every compute unit one
-    const uint32_t cus = (uint32_t)ctx->compute_units;
-    auto tiles = [](uint32_t v, uint32_t b) { return (v + b - 1) / b; };
-    if (tiles(p.n, 128) * tiles(p.rows, 128) >= cus)
-        dense_gemm_kernel<EPI, 128, 128><<<tiles(p.n, 128) * tiles(p.rows, 128), 256, 0, s>>>(p, tiles(p.n, 128), tiles(p.rows, 128));
-    else if (tiles(p.n, 64) * tiles(p.rows, 128) >= cus)
-        dense_gemm_kernel<EPI, 64, 128><<<tiles(p.n, 64) * tiles(p.rows, 128), 256, 0, s>>>(p, tiles(p.n, 64), tiles(p.rows, 128));
-    else if (tiles(p.n, 64) * tiles(p.rows, 64) <= cus)      // one tile per compute unit waits for each of its loads: halve them
-        dense_gemm_kernel<EPI, 32, 64><<<tiles(p.n, 32) * tiles(p.rows, 64), 256, 0, s>>>(p, tiles(p.n, 32), tiles(p.rows, 64));
-    else
-        dense_gemm_kernel<EPI, 64, 64><<<tiles(p.n, 64) * tiles(p.rows, 64), 256, 0, s>>>(p, tiles(p.n, 64), tiles(p.rows, 64));
+    launch_tiles<EPI, ACT_BF16>(ctx, s, p);
     return launch_status();
 }
 

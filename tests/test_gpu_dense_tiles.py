@@ -1,0 +1,103 @@
+"""The tiled products behind dense_linear at the edges of their tiles, rounds and pipelines, against float64 on the device."""
+import pytest
+import torch
+
+from gpu_util import say
+
+pytestmark = pytest.mark.gpu
+
+
+def operands(rows, n, k, dtype, seed):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    w = (torch.randn((n, k), device="cuda", generator=gen) * k ** -0.5).to(torch.bfloat16)
+    return w, torch.randn((rows, k), device="cuda", generator=gen).to(dtype)
+
+
+def check(got, want, tol):
+    assert float((got.double() - want).abs().max() / want.abs().max()) < tol
+
+
+# A sum of k products of order k^-1/2 in fp32, rounded at most k / 16 + 16 times: 2^-24 sqrt(k / 16 + 16) of the largest value
+# and below 1e-6 at these k; the bound is twice that.
+@pytest.mark.parametrize("act", ["bf16", "fp32"])
+@pytest.mark.parametrize("k", [64, 128, 192, 256, 320, 448])          # one to seven steps: every remainder of a ring of 2, 3, 4 or 5 stages
+@pytest.mark.parametrize("rows,n", [(65, 250), (300, 64), (1000, 2047), (300, 8190), (2048, 2170), (2047, 8192)])  # each tile, ragged
+def test_tiles(act, k, rows, n):
+    import nvmai_amd as nv
+    say("dense tiles", act, rows, n, k)
+    ctx = nv.Context(0, nv.ACT_FP32 if act == "fp32" else nv.ACT_BF16)
+    w, x = operands(rows, n, k, ctx.dtype, rows + n + k)
+    want = x.double() @ w.double().T
+    stride = n + 5
+    y, y32 = torch.full((rows, stride), 7.0, dtype=ctx.dtype, device="cuda"), torch.full((rows, stride), 7.0, device="cuda")
+    nv.dense_linear(ctx, w, x, y=y, y_f32=y32)
+    check(y32[:, :n], want, 2e-6)
+    check(y[:, :n], want, 2e-6 if act == "fp32" else 2 ** -8)
+    assert bool((y[:, n:] == 7).all()) and bool((y32[:, n:] == 7).all())
+
+
+# 2048 rows x 8208: a full round of the largest tile and sixteen weight rows in a launch of their own
+@pytest.mark.parametrize("kind", ["plain", "erf", "bias", "pairs", "full"])
+def test_two_launches_with_every_epilogue(kind):
+    import nvmai_amd as nv
+    say("dense in two launches", kind)
+    ctx = nv.Context(0, nv.ACT_BF16)
+    rows, n, k = 2048, 8208, 512
+    w, x = operands(rows, n, k, ctx.dtype, 11)
+    gen = torch.Generator(device="cuda").manual_seed(12)
+    bias, mul = torch.randn(n, device="cuda", generator=gen).to(torch.bfloat16), torch.randn((50, n), device="cuda", generator=gen).to(torch.bfloat16)
+    ids = torch.randint(0, 52, (rows,), device="cuda", generator=gen, dtype=torch.int32)            # two of them past the table
+    want = x.double() @ w.double().T
+    gelu = torch.nn.functional.gelu
+    if kind == "erf":
+        args, want = dict(activation=nv.LINEAR_GELU_ERF), gelu(want)
+    elif kind == "bias":
+        args, want = dict(bias=bias), want + bias.double()
+    elif kind == "pairs":
+        args, want = dict(activation=nv.LINEAR_SILU_PAIRS), torch.nn.functional.silu(want[:, ::2]) * want[:, 1::2]
+    elif kind == "full":
+        table = torch.cat([mul.double(), torch.zeros((2, n), dtype=torch.float64, device="cuda")])
+        args, want = dict(bias=bias, activation=nv.LINEAR_GELU_TANH, mul=mul, mul_ids=ids), gelu(want + bias.double(), approximate="tanh") * table[ids.long()]
+    else:
+        args = {}
+    y32 = torch.full((rows, n), 7.0, device="cuda")
+    y32 = y32[:, :n // 2].contiguous() if kind == "pairs" else y32
+    nv.dense_linear(ctx, w, x, y_f32=y32, **args)
+    check(y32, want, 3e-6)              # the sum's 2e-6, and 1e-6 for a GELU by hardware exponentials
+
+
+def test_32_bit_values_keep_every_bit():
+    """The planes of 32-bit rows hold them exactly: unit rows of the matrix give the inputs back, whatever their size."""
+    import nvmai_amd as nv
+    ctx = nv.Context(0, nv.ACT_FP32)
+    x = torch.randn((70, 64), device="cuda", generator=torch.Generator(device="cuda").manual_seed(3))
+    x = x * torch.logspace(-30, 30, 70, device="cuda")[:, None]
+    x[0, 0], x[1, 1], x[2, 2], x[3, 3] = float("inf"), float("-inf"), float("nan"), 3.4028234663852886e38
+    y = torch.empty((70, 64), device="cuda")
+    nv.dense_linear(ctx, torch.eye(64, device="cuda", dtype=torch.bfloat16), x, y_f32=y)
+    rest = torch.ones(70, dtype=torch.bool)
+    rest[:3] = False                    # an infinity or NaN meets zeros in its row
+    assert torch.equal(y[rest.cuda()], x[rest.cuda()])
+    one = torch.ones((64, 64), device="cuda", dtype=torch.bfloat16)
+    nv.dense_linear(ctx, one, x, y_f32=y)
+    assert bool((y[0] == float("inf")).all()) and bool((y[1] == float("-inf")).all()) and bool(y[2].isnan().all())
+
+
+def test_a_captured_call_without_workspace_still_runs():
+    """The planes lie in the workspace; a call that is captured before anything has sized it takes a form without them."""
+    import nvmai_amd as nv
+    say("captured 32-bit product")
+    w, x = operands(100, 200, 256, torch.float32, 5)
+    want, y = x.double() @ w.double().T, torch.zeros((100, 200), device="cuda")
+    warm, ctx = nv.Context(0, nv.ACT_FP32), nv.Context(0, nv.ACT_FP32)
+    nv.dense_linear(warm, w, x, y_f32=torch.empty_like(y))            # loads the module
+    torch.cuda.synchronize()
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(graph, stream=stream):
+            nv.dense_linear(ctx, w, x, y_f32=y)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        check(y, want, 2e-6)
