@@ -62,10 +62,7 @@ int absorbed(const LatentAttnParams& p, hipStream_t s) {
 
 template <int NP, int RP, int DV>
 int launch_flash(const LatentAttnParams& p, hipStream_t s) {
-    const size_t lds = 2 * ((size_t)64 * (NP + RP) * 2 + (size_t)DV * 128);
-    const int rc = raise_lds(reinterpret_cast<const void*>(latent_flash_kernel<NP, RP, DV>), lds);
-    if (rc) return rc;
-    latent_flash_kernel<NP, RP, DV><<<(p.n_rows + 127) / 128 * p.heads, 256, lds, s>>>(p);
+    latent_flash_kernel<NP, RP, DV><<<(p.n_rows + 127) / 128 * p.heads, 256, 0, s>>>(p);
     return launch_status();
 }
 

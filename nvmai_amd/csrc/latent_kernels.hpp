@@ -577,6 +577,9 @@ __global__ __launch_bounds__(256) void latent_expanded_plain_kernel(LatentAttnPa
 // LDS pieces of 16 bytes are exchanged within a row (la_swizzle) so that the eight lanes that a read serves at once
 // fall into different banks.  NP, RP: the two parts of a key, DV: value dims, padded with zeros (a lane whose column
 // does not exist loads from past the end of the buffer, which reads as zero).
+// The two stages are arrays of their own and the loop is written out for both: from halves of one array the compiler cannot
+// tell that a read of this tile does not touch the tile on its way, and waits for it before the first product (139 -> 114 us,
+// 2048 queries behind 2048 tokens, 16 heads of 192 / 128).
 template <int W>                         // row width in pieces
 __device__ __forceinline__ uint32_t la_swizzle(uint32_t key) {
     return W >= 8 ? (key & 3u) | ((key >> 1) & 4u) : (key >> 3) & (W - 1u);
@@ -589,8 +592,7 @@ __global__ __launch_bounds__(256, NP + RP + DV <= 320 ? 2 : 1) void latent_flash
     constexpr int KN = NP / 32, KR = RP / 32, NV = DV / 16;
     constexpr int LN = NP / 32, LR = RP / 32, LV = DV / 32;      // 1 KB loads per wave and tile
     constexpr uint32_t AT_R = 64u * NP * 2u, AT_V = AT_R + 64u * RP * 2u, STAGE = AT_V + DV * 128u;
-    extern __shared__ __attribute__((aligned(16))) float la_lds[];
-    uint8_t* lds = reinterpret_cast<uint8_t*>(la_lds);
+    __shared__ __attribute__((aligned(1024))) uint8_t even[STAGE], odd[STAGE];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 15u, g = lane >> 4;
     // Blocks are dealt to the eight XCDs in turn: an XCD keeps to its own heads (their keys stay in its L2) where
     // the heads divide.  Even rounds take the query blocks with the most keys first, odd ones last: a compute unit's
@@ -660,13 +662,10 @@ __global__ __launch_bounds__(256, NP + RP + DV <= 320 ? 2 : 1) void latent_flash
     const uint32_t w_lo = first_key(p.rows.position + wt0, p.window) - p.key0, w_hi = p.rows.position + wt1 + 1u - p.key0;
     const uint32_t full_lo = first_key(p.rows.position + wt1, p.window) - p.key0, full_hi = p.rows.position + wt0 + 1u - p.key0;
     const uint32_t krow = 8u * (i >> 2) + (i & 3u);              // key of this lane's row in an even score tile
-    issue(k_lo, lds);
-    uint32_t stage = 0;
-    for (uint32_t k0 = k_lo; k0 < k_hi; k0 += 64u, stage ^= 1u) {
+    auto tile = [&](uint32_t k0, const uint8_t* cur, uint8_t* next) {
         __syncthreads();                             // this tile has landed; everyone is done with the other stage
-        if (k0 + 64u < k_hi) issue(k0 + 64u, lds + (stage ^ 1u) * STAGE);
-        if (!wave_live || k0 >= w_hi || k0 + 64u <= w_lo) continue;             // wave-uniform
-        const uint8_t* cur = lds + stage * STAGE;
+        if (k0 + 64u < k_hi) issue(k0 + 64u, next);
+        if (!wave_live || k0 >= w_hi || k0 + 64u <= w_lo) return;               // wave-uniform
         la_f4 s[2][4];
 #pragma unroll
         for (int b = 0; b < 2; ++b)
@@ -737,6 +736,11 @@ __global__ __launch_bounds__(256, NP + RP + DV <= 320 ? 2 : 1) void latent_flash
 #pragma unroll
                 for (int b = 0; b < 2; ++b) acc[b][n] = la_mfma(a, pf[b][h], acc[b][n]);
             }
+    };
+    issue(k_lo, even);
+    for (uint32_t k0 = k_lo; k0 < k_hi; k0 += 128u) {
+        tile(k0, even, odd);
+        if (k0 + 64u < k_hi) tile(k0 + 64u, odd, even);
     }
     if (!wave_live) return;
 #pragma unroll

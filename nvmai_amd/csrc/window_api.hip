@@ -30,12 +30,6 @@ int check_map(const nvmai_row_map* map, const nvmai_kv_ring* cache, uint32_t win
 KvRing ring_of(const nvmai_kv_ring* c) { return KvRing{c->k, c->v, c->kv_heads, c->key_dim, c->value_dim, c->pinned, c->ring}; }
 SeqRows rows_of(const nvmai_row_map* m) { return SeqRows{m->slots, m->positions, m->slot, m->position}; }
 
-int raise_lds(const void* kernel, size_t bytes) {
-    if (bytes > 160 * 1024) return NVMAI_ERR_UNSUPPORTED;
-    if (bytes > 64 * 1024) NVMAI_HIP_TRY(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
-    return NVMAI_OK;
-}
-
 template <int CT>
 void epilogue(const WindowEpilogueParams& p, hipStream_t s) {
     const uint32_t G = p.cache.kv_heads, units = p.heads + (p.k_norm ? (p.values ? 2 * G : G) : 0);
@@ -51,10 +45,7 @@ void epilogue(const WindowEpilogueParams& p, hipStream_t s) {
 
 template <int DK, int DV, bool BOUND>
 int launch_flash_as(const WindowParams& p, hipStream_t s) {
-    const size_t lds = 2 * ((size_t)64 * DK * 2 + (size_t)DV * 128);
-    const int rc = raise_lds(reinterpret_cast<const void*>(window_flash_kernel<DK, DV, BOUND>), lds);
-    if (rc) return rc;
-    window_flash_kernel<DK, DV, BOUND><<<(p.n_rows + 127) / 128 * p.heads, 256, lds, s>>>(p);
+    window_flash_kernel<DK, DV, BOUND><<<(p.n_rows + 127) / 128 * p.heads, 256, 0, s>>>(p);
     return launch_status();
 }
 
