@@ -191,6 +191,12 @@ extern "C" int nvmai_hip_latent_attention(nvmai_hip_ctx* ctx, nvmai_stream strea
         if (c.rotary_dims) latent_rotate_q_kernel<ACT_BF16><<<rows, 256, lds_rot, s>>>(p);
     }
     if ((rc = dense_linear(ctx, s, lk)) || (rc = dense_linear(ctx, s, lv))) return rc;
+    if (f32 && c.nope_dim <= 128 && c.rope_dim <= 64 && c.value_dim <= 128) {
+        const uint32_t blocks = (rows + 15) / 16 * c.heads;
+        if (c.value_dim <= 64) latent_flash32_kernel<128, 64, 64><<<blocks, 256, 0, s>>>(p);
+        else latent_flash32_kernel<128, 64, 128><<<blocks, 256, 0, s>>>(p);
+        return launch_status();
+    }
     if (!flash) {
         const size_t lds = ((size_t)dq + c.value_dim + 256 + 8) * 4;
         if (f32) {

@@ -108,6 +108,14 @@ extern "C" int nvmai_hip_window_attention(nvmai_hip_ctx* ctx, nvmai_stream strea
     const uint64_t total = (uint64_t)cache->pinned + cache->ring;
     const bool can_flash = can16 && known && !f32 && total * (dk > dv ? dk : dv) * 2 < 0x7FFFFFFFull && out_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 7u) == 0;
     if ((form == NVMAI_WINDOW_SPLIT && !can16) || (form == NVMAI_WINDOW_FLASH && !can_flash)) return NVMAI_ERR_UNSUPPORTED;
+    // a prompt's rows in 32 bits, a block of 16 queries at a time: from 16 rows on (a block per row and head before)
+    if (form == NVMAI_FORM_AUTO && cache32 && f32 && known && rows >= 16 && dk <= 128 && dv <= 128 && aligned16(q) && q_stride % 4 == 0 && aligned16(cache->k) &&
+        aligned16(cache->v)) {
+        const uint32_t blocks = (rows + 15) / 16 * c.heads;
+        if (dk <= 64 && dv <= 64) window_flash32_kernel<64, 64><<<blocks, 256, 0, s>>>(p);
+        else window_flash32_kernel<128, 128><<<blocks, 256, 0, s>>>(p);
+        return launch_status();
+    }
     if (form == NVMAI_FORM_AUTO) form = can_flash && rows >= 32 ? NVMAI_WINDOW_FLASH : can16 ? NVMAI_WINDOW_SPLIT : NVMAI_WINDOW_PLAIN;
     if (form == NVMAI_WINDOW_PLAIN) {
         if (cache32) return plain<ACT_FP32, ACT_FP32>(p, s);

@@ -16,6 +16,7 @@
 //   * plain: any sizes and types, a thread per key.
 #pragma once
 
+#include "flash32.hpp"
 #include "rows.hpp"
 
 namespace nvmai {
@@ -381,6 +382,50 @@ __global__ __launch_bounds__(256) void window_plain_kernel(WindowParams p) {
     const float gate = (p.gate ? wa_sigmoid(p.gate[(size_t)row * p.gate_stride + head]) : 1.0f) * p.out_scale;
     for (uint32_t j = tid; j < dv; j += 256u)
         static_cast<act_t<ACT>*>(p.out)[(size_t)row * p.out_stride + head * dv + j] = f32_to_act<ACT>(acc[j] / l * gate);
+}
+
+// ---- flash form in 32 bits: 16 queries of one head per block (flash32.hpp) --------------------------------------
+// 700 rows, 8 heads of 128 / 128: 1133 -> 44 us (the plain form before).
+template <int DK, int DV>
+__global__ __launch_bounds__(256, 2) void window_flash32_kernel(WindowParams p) {
+    constexpr int NV = DV / 16;
+    __shared__ __attribute__((aligned(16))) float shared[NV * 1024 + 128];
+    const uint32_t lane = threadIdx.x & 63u, i = lane & 15u, g = lane >> 4, dk = p.cache.dk, dv = p.cache.dv, total = p.cache.rows();
+    // neighbouring heads (which share a kv head) on one XCD; the queries with the most keys come first
+    const uint32_t nq = (p.n_rows + 15u) / 16u, nth = blockIdx.x % p.heads, q0 = (nq - 1u - blockIdx.x / p.heads) * 16u;
+    const uint32_t head = p.heads % 8u == 0u ? (nth % 8u) * (p.heads / 8u) + nth / 8u : nth;
+    const uint32_t row = min(q0 + i, p.n_rows - 1u), start = p.rows.position, pos = start + row, last = start + min(q0 + 15u, p.n_rows - 1u);
+    // tiles of 16 positions: the kept ones, then from the window's first one to the last query's
+    const uint32_t first_t = first_key(start + q0, p.window) / 16u, kept = min((p.keep + 15u) / 16u, first_t);
+    const size_t own = (size_t)p.rows.slot * p.cache.kv_heads + head / (p.heads / p.cache.kv_heads);
+    const float* q = static_cast<const float*>(p.q) + (size_t)row * p.q_stride + head * dk + 4u * g;
+    const float* k = static_cast<const float*>(p.cache.k) + own * total * dk + 4u * g;
+    const float* v = static_cast<const float*>(p.cache.v) + own * dv * total + (size_t)i * total + 4u * g;
+    const f32_f4 none{0.0f, 0.0f, 0.0f, 0.0f};
+    const float slope = p.alibi ? wa_slope_log2(head, p.heads) : 0.0f;
+    const float gate = (p.gate ? wa_sigmoid(p.gate[(size_t)row * p.gate_stride + head]) : 1.0f) * p.out_scale;
+    auto position_of = [&](uint32_t t) { return (t < kept ? t : first_t + t - kept) * 16u; };
+    flash32_block<DK / 16, NV, true>(kept + last / 16u - first_t + 1u, shared,
+        [&](int c) { return 16u * c < dk ? *reinterpret_cast<const f32_f4*>(q + 16 * c) : none; },
+        [&](uint32_t t, int c) { return 16u * c < dk ? *reinterpret_cast<const f32_f4*>(k + (size_t)(p.cache.row_of(position_of(t)) + i) * dk + 16 * c) : none; },
+        [&](uint32_t t, int n) {
+            // positions past the last query's have not been written: what lies there is not multiplied, not even by zero
+            const uint32_t at = position_of(t);
+            f32_f4 x = 16u * n < dv ? *reinterpret_cast<const f32_f4*>(v + (size_t)(16 * n) * total + p.cache.row_of(at)) : none;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) x[j] = at + 4u * g + j <= last ? x[j] : 0.0f;
+            return x;
+        },
+        [&](uint32_t t, int j, float s) {
+            const uint32_t key = position_of(t) + 4u * g + j;
+            s *= p.a;
+            if (p.capped) s = p.b * tanhf(s);
+            s = fmaf(-slope, (float)(int32_t)(pos - key), s);
+            return wa_visible(pos, key, p.window, p.keep) ? s : 2.0f * FLASH32_NONE;
+        },
+        [&](uint32_t d, float o) {
+            if (q0 + i < p.n_rows && d < dv) static_cast<float*>(p.out)[(size_t)row * p.out_stride + head * dv + d] = o * gate;
+        });
 }
 
 // ---- flash form ------------------------------------------------------------------------------------------
