@@ -328,8 +328,10 @@ __device__ __forceinline__ void dense_stage_barrier() {
 #endif
 }
 
-constexpr int dense_stages(int act, int bn, int bm) {        // of 160 KB; two blocks per compute unit where the tile is small
-    return act == ACT_FP32 ? 3 : bn + bm <= 192 ? 5 : bn + bm <= 256 ? 4 : bn + bm <= 384 ? 3 : 2;
+// Of 160 KB; two blocks per compute unit where the tile is small.  Planes come in threes: six stages where they fit (64 x 64, 700 x
+// 1024 x 1024 in 32 bits: 17.4 us with three, 13.5 with six).
+constexpr int dense_stages(int act, int bn, int bm) {
+    return act == ACT_FP32 ? (bn + bm <= 192 ? 6 : 3) : bn + bm <= 192 ? 5 : bn + bm <= 256 ? 4 : bn + bm <= 384 ? 3 : 2;
 }
 
 template <int EPI, int ACT, int BN, int BM>
@@ -339,7 +341,7 @@ __global__ __launch_bounds__(256, BN + BM <= 128 ? 2 : 1) void dense_tile_kernel
     constexpr int LA = BN / 32, LB = BM / 32, L = LA + LB;   // 1 KB requests per wave and stage
     constexpr int TN = BN / 64, TM = BM / 64;                // 32 x 32 tiles per wave
     constexpr uint32_t STAGE = (BN + BM) * 128u;
-    __shared__ __attribute__((aligned(1024))) uint8_t l0[STAGE], l1[STAGE], l2[S > 2 ? STAGE : 16], l3[S > 3 ? STAGE : 16], l4[S > 4 ? STAGE : 16];
+    __shared__ __attribute__((aligned(1024))) uint8_t l0[STAGE], l1[STAGE], l2[S > 2 ? STAGE : 16], l3[S > 3 ? STAGE : 16], l4[S > 4 ? STAGE : 16], l5[S > 5 ? STAGE : 16];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // blocks are dealt to the eight XCDs in turn: give each XCD a run of neighbouring tiles (shared L2 lines)
     const uint32_t all = tiles_n * tiles_m, xcd = blockIdx.x & 7u, nth = blockIdx.x >> 3;
@@ -357,14 +359,14 @@ __global__ __launch_bounds__(256, BN + BM <= 128 ? 2 : 1) void dense_tile_kernel
     // rows past the last: the last one, whose sums are not stored
     [[maybe_unused]] const uint32_t a8 = p.w_stride * 16u, a0 = (n0 + wave * (LA * 8u) + lr) * p.w_stride * 2u + piece, amax = (p.n - 1u) * p.w_stride * 2u + piece;
     [[maybe_unused]] const uint32_t b8 = p.x_stride * 16u, b0 = (m0 + wave * (LB * 8u) + lr) * p.x_stride * 2u + piece, bmax = (p.rows - 1u) * p.x_stride * 2u + piece;
-    auto buf = [&](int j) -> uint8_t* { return j == 0 ? l0 : j == 1 ? l1 : j == 2 ? l2 : j == 3 ? l3 : l4; };
-    // requests [from, to) of stage st into its place j = st % S (the plane of a 32-bit input, S = 3)
+    auto buf = [&](int j) -> uint8_t* { return j == 0 ? l0 : j == 1 ? l1 : j == 2 ? l2 : j == 3 ? l3 : j == 4 ? l4 : l5; };
+    // requests [from, to) of stage st into its place j = st % S (of a 32-bit input: plane j % 3, S is 3 or 6)
     auto request = [&](uint32_t st, int j, int from, int to) {
 #if defined(__HIP_DEVICE_COMPILE__)     // the host pass rejects the 16-byte form of the load
         const bool live = st < steps;
         const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.w), 0, live ? (int)w_bytes : 0, 0x00020000);
         const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.x), 0, live ? (int)x_bytes : 0, 0x00020000);
-        const uint32_t wk = (SPLIT ? st / 3u : st) * 128u, xk = SPLIT ? wk + j * p.k * 2u : wk;
+        const uint32_t wk = (SPLIT ? st / 3u : st) * 128u, xk = SPLIT ? wk + j % 3 * p.k * 2u : wk;
         uint8_t* dst = buf(j);
 #pragma unroll
         for (int r = 0; r < L; ++r) {
@@ -413,7 +415,7 @@ __global__ __launch_bounds__(256, BN + BM <= 128 ? 2 : 1) void dense_tile_kernel
         constexpr int B = S - 1;
         fetch(j, 1);
         request(st + B, (j + B) % S, NVMAI_SHARE(1), NVMAI_SHARE(2));
-        multiply(0, std::integral_constant<int, NVMAI_SHARE(2) - NVMAI_SHARE(1)>{}, SPLIT && j == 0);
+        multiply(0, std::integral_constant<int, NVMAI_SHARE(2) - NVMAI_SHARE(1)>{}, SPLIT && j % 3 == 0);
         fetch(j, 2);
         request(st + B, (j + B) % S, NVMAI_SHARE(2), NVMAI_SHARE(3));
         multiply(1, std::integral_constant<int, NVMAI_SHARE(3) - NVMAI_SHARE(2)>{}, false);
@@ -425,7 +427,7 @@ __global__ __launch_bounds__(256, BN + BM <= 128 ? 2 : 1) void dense_tile_kernel
         request(st + S, j, 0, NVMAI_SHARE(1));
         multiply(3, std::integral_constant<int, NVMAI_SHARE(1)>{}, false);
         if constexpr (SPLIT) {
-            if (j == 2) {
+            if (j % 3 == 2) {
 #pragma unroll
                 for (int a = 0; a < TN; ++a)
 #pragma unroll
