@@ -156,6 +156,11 @@ struct AttnParams {
     uint32_t ring;             // not 0: row of key p is p % ring (generic kernel only)
     uint32_t cols_q;           // sequences sharing one block of the matrix-core kernel
     uint32_t direct;           // num_chunks == 1: the partial kernel normalises and writes out itself
+    // A ragged batch dealt out by length (0: num_chunks chunks for every sequence): blocks per KV head, and per sequence its
+    // first block and how many it has, which the partial kernel writes for the combine.  Partial rows then lie
+    // [num_kv_heads, slots, heads of a KV head].
+    uint32_t slots;
+    uint32_t* seq_slots;       // [2][batch]
     // optional output gate (RealForwardRunner.swift:2272-2276, utility.metal:47-58): the combine
     // kernel writes round(out) / (1 + exp(-gate)) -- the rounded row first, as the separate
     // elementwise launch reads it, so the bits are the same.  Row of sequence b at gate + b * gate_stride.
@@ -173,6 +178,46 @@ __device__ __forceinline__ void attn_range(const AttnParams& p, uint32_t b, uint
         lo = p.kv_starts ? p.kv_starts[b] : p.kv_start;
     }
     if (lo > hi) lo = hi;
+}
+
+// Wave-wide sum through the DPP ladder, in every lane.
+__device__ __forceinline__ uint32_t attn_wave_sum(uint32_t v) {
+#define NVMAI_DPP_ADD(CTRL, ROWS) v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, true)
+    NVMAI_DPP_ADD(0xB1, 0xF);
+    NVMAI_DPP_ADD(0x4E, 0xF);
+    NVMAI_DPP_ADD(0x141, 0xF);
+    NVMAI_DPP_ADD(0x140, 0xF);
+    NVMAI_DPP_ADD(0x142, 0xA);
+    NVMAI_DPP_ADD(0x143, 0xC);
+#undef NVMAI_DPP_ADD
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// Block `slot` of a KV head in a ragged batch of at most 64: which sequence, which of its chunks, how long a chunk is.  The lanes
+// look at a sequence each; the chunk length (a multiple of 32, 128 at least) is the one with which half a chunk per sequence is left
+// over, or where that does not fit a whole one, which always does.  A sequence without keys has one block, which leaves an
+// empty partial row.  false: a block that is left over.
+__device__ __forceinline__ bool attn_deal(const AttnParams& p, uint32_t slot, uint32_t& b, uint32_t& chunk, uint32_t& chunk_len, uint32_t& first, uint32_t& count) {
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t lo = 0, hi = 0;
+    if (lane < p.batch) attn_range(p, lane, lo, hi);
+    const uint32_t len = hi - lo, total = attn_wave_sum(len);
+    uint32_t n = 0;
+    for (uint32_t part = 2; part >= 1; --part) {
+        const uint32_t share = p.slots - p.batch / part;                 // slots >= 2 batch
+        chunk_len = max(((total + share - 1u) / share + 31u) & ~31u, 128u);
+        n = lane < p.batch ? max((len + chunk_len - 1u) / chunk_len, 1u) : 0u;
+        if (attn_wave_sum(n) <= p.slots) break;
+    }
+    b = 0;
+    first = 0;
+    for (;; ++b) {
+        count = (uint32_t)__builtin_amdgcn_readlane((int)n, (int)b);
+        if (slot - first < count || b + 1u == p.batch) break;
+        first += count;
+    }
+    chunk = slot - first;
+    return chunk < count;
 }
 
 __device__ __forceinline__ float kv_load(const uint8_t* row, const KvFormat& f, uint32_t e) {   // attention.metal:89-117
@@ -249,9 +294,18 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams p) {
     __shared__ float part[4][64];
     const size_t bh = blockIdx.x;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const float* mr = p.m_part + bh * p.num_chunks;
-    const float* dr = p.d_part + bh * p.num_chunks;
-    const float* orow = p.o_part + bh * p.num_chunks * p.head_dim;
+    // where this head's partial rows begin, how many there are and how far apart
+    size_t row0 = bh * p.num_chunks;
+    uint32_t count = p.num_chunks, pitch = 1;
+    if (p.slots) {
+        const uint32_t seq = (uint32_t)(bh / p.num_q_heads), head = (uint32_t)(bh % p.num_q_heads);
+        pitch = p.num_q_heads / p.num_kv_heads;
+        row0 = ((size_t)(head / pitch) * p.slots + p.seq_slots[seq]) * pitch + head % pitch;
+        count = p.seq_slots[p.batch + seq];
+    }
+    const float* mr = p.m_part + row0;
+    const float* dr = p.d_part + row0;
+    const float* orow = p.o_part + row0 * p.head_dim;
     const uint32_t dim = blockIdx.y * 64 + lane;
     uint16_t* out_row = (uint16_t*)p.out + (bh / p.num_q_heads) * p.out_stride + (bh % p.num_q_heads) * p.head_dim;
     const uint16_t* gate_row = p.gate ? p.gate + (bh / p.num_q_heads) * p.gate_stride + (bh % p.num_q_heads) * p.head_dim : nullptr;
@@ -262,10 +316,10 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams p) {
     float mv[2], dv[2];
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) {
-        const uint32_t c = threadIdx.x + 256u * s2, cc = min(c, p.num_chunks - 1u);
+        const uint32_t c = threadIdx.x + 256u * s2, cc = min(c, count - 1u) * pitch;
         const float m_c = mr[cc], d_c = dr[cc];
-        mv[s2] = c < p.num_chunks ? m_c : -INFINITY;
-        dv[s2] = c < p.num_chunks ? d_c : 0.0f;
+        mv[s2] = c < count ? m_c : -INFINITY;
+        dv[s2] = c < count ? d_c : 0.0f;
     }
     auto gated = [&](float v) -> uint16_t {
         uint16_t o = f32_to_act<ACT>(v);
@@ -285,7 +339,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams p) {
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) {
         const uint32_t c = threadIdx.x + 256u * s2;
-        if (c < p.num_chunks) {
+        if (c < count) {
             const float w = expf(mv[s2] - mg);
             wgt[c] = w;
             dloc += dv[s2] * w;
@@ -299,7 +353,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams p) {
     if (dim < p.head_dim) {
         const float* oc = orow + dim;
 #pragma unroll 16
-        for (uint32_t c = wave; c < p.num_chunks; c += 4) acc += oc[(size_t)c * p.head_dim] * wgt[c];
+        for (uint32_t c = wave; c < count; c += 4) acc += oc[(size_t)c * pitch * p.head_dim] * wgt[c];
     }
     part[wave][lane] = acc;
     __syncthreads();
@@ -377,13 +431,30 @@ __global__ __launch_bounds__(256, 2) void attn_partial_mfma_kernel(AttnParams p)
     const int i = lane & 15, r = lane >> 4;
     float* bc = bc_all + wave * 64;                                // broadcast scratch
     float* merge = reinterpret_cast<float*>(kst);                  // after the loop
-    const uint32_t chunk = blockIdx.x % p.num_chunks;
-    const uint32_t kvh = (blockIdx.x / p.num_chunks) % p.num_kv_heads;
-    const uint32_t n_qb = (p.batch + p.cols_q - 1) / p.cols_q;
-    uint32_t qb = blockIdx.x / (p.num_chunks * p.num_kv_heads);
-    if (p.causal) qb = n_qb - 1u - qb;                             // the longest key ranges start first
-    const uint32_t b = qb * p.cols_q;                              // first sequence of this block
     const uint32_t qpk = p.num_q_heads / p.num_kv_heads;           // <= 16
+    uint32_t chunk, kvh, b, chunk_len = p.chunk_len;               // b: first sequence of this block
+    size_t part_row;                                               // partial row of (b, first head of kvh, this chunk)
+    uint32_t part_pitch;                                           // rows from one head to the next
+    if (p.slots) {                                                 // one sequence per block (cols_q is 1)
+        uint32_t first, count;
+        kvh = blockIdx.x / p.slots;
+        if (!attn_deal(p, blockIdx.x % p.slots, b, chunk, chunk_len, first, count)) return;
+        if (chunk == 0 && kvh == 0 && threadIdx.x == 0) {
+            p.seq_slots[b] = first;
+            p.seq_slots[p.batch + b] = count;
+        }
+        part_row = ((size_t)kvh * p.slots + first + chunk) * qpk;
+        part_pitch = 1;
+    } else {
+        chunk = blockIdx.x % p.num_chunks;
+        kvh = (blockIdx.x / p.num_chunks) % p.num_kv_heads;
+        const uint32_t n_qb = (p.batch + p.cols_q - 1) / p.cols_q;
+        uint32_t qb = blockIdx.x / (p.num_chunks * p.num_kv_heads);
+        if (p.causal) qb = n_qb - 1u - qb;                         // the longest key ranges start first
+        b = qb * p.cols_q;
+        part_row = ((size_t)b * p.num_q_heads + kvh * qpk) * p.num_chunks + chunk;
+        part_pitch = p.num_chunks;
+    }
     // Column i of the score tile is (sequence b + i / qpk, q head i % qpk of this kv head): a decode
     // step has cols_q = 1, a prefill chunk packs 16 / qpk query tokens into the sixteen columns.
     const uint32_t cols = min(p.cols_q, p.batch - b) * qpk;        // live columns
@@ -400,7 +471,7 @@ __global__ __launch_bounds__(256, 2) void attn_partial_mfma_kernel(AttnParams p)
     }
     blo = __builtin_amdgcn_readfirstlane(blo);                     // the union of the block's ranges
     bhi = __builtin_amdgcn_readfirstlane(bhi);
-    const uint32_t p0 = min(blo + chunk * p.chunk_len, bhi), p1 = min(p0 + p.chunk_len, bhi);
+    const uint32_t p0 = min(blo + chunk * chunk_len, bhi), p1 = min(p0 + chunk_len, bhi);
     const uint32_t groups_total = (p.f.elements + 63) / 64;
     const uint32_t code_off = kvh * ATTN_HD * BITS / 8;            // this head's codes inside a row
     const uint32_t meta_sc = p.f.value_bytes + 2 * (kvh * 4);      // 4 fp16 scales of this head
@@ -784,7 +855,7 @@ __global__ __launch_bounds__(256, 2) void attn_partial_mfma_kernel(AttnParams p)
         return;
     }
     if (r == 0 && live) {
-        const size_t at = ((size_t)my_b * p.num_q_heads + my_h) * p.num_chunks + chunk;
+        const size_t at = part_row + ((size_t)(my_b - b) * p.num_q_heads + (my_h - kvh * qpk)) * part_pitch;
         p.m_part[at] = m_run;
         p.d_part[at] = d_run;
     }
@@ -792,7 +863,7 @@ __global__ __launch_bounds__(256, 2) void attn_partial_mfma_kernel(AttnParams p)
     for (int t = 0; t < 4; ++t) {
         const uint32_t c = 4 * r + t;
         if (c >= cols) continue;
-        float* dst = p.o_part + (((size_t)(b + c / qpk) * p.num_q_heads + kvh * qpk + c % qpk) * p.num_chunks + chunk) * ATTN_HD;
+        float* dst = p.o_part + (part_row + ((size_t)(c / qpk) * p.num_q_heads + c % qpk) * part_pitch) * ATTN_HD;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             const float4 o4 = {oacc[g][0][t], oacc[g][1][t], oacc[g][2][t], oacc[g][3][t]};
