@@ -214,6 +214,38 @@ void run_router_t(const RouterParams& rp, uint32_t cpl, dim3 grid, hipStream_t s
     else router_logits_kernel<ACT, 8><<<grid, 256, lds, s>>>(rp);
 }
 
+template <int ACT, bool EFF, int SPLIT, int U>
+bool launch_router_chains(const RouterParams& rp, const RowsDesc& r, uint32_t n_rows, float* out, uint32_t out_ld, hipStream_t s) {
+    const size_t tokens = (size_t)(EFF ? 17 : 16) * router_chain_pitch(rp.d), sums = 8 * 4096;
+    const size_t lds = tokens > sums ? tokens : sums;
+    const void* kernel = reinterpret_cast<const void*>(router_chain_kernel<ACT, EFF, SPLIT, U>);
+    if (lds > 64 * 1024 && hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return false;
+    const dim3 grid((n_rows + 128 / SPLIT - 1) / (128 / SPLIT), (rp.tokens + 15) / 16);
+    router_chain_kernel<ACT, EFF, SPLIT, U><<<grid, 512, lds, s>>>(rp, r, n_rows, out, out_ld);
+    return true;
+}
+
+template <int ACT, int SPLIT, int U>
+bool launch_router_chains_any(const RouterParams& rp, const RowsDesc& r, uint32_t n_rows, float* out, uint32_t out_ld, hipStream_t s) {
+    return rp.eff_scale ? launch_router_chains<ACT, true, SPLIT, U>(rp, r, n_rows, out, out_ld, s)
+                        : launch_router_chains<ACT, false, SPLIT, U>(rp, r, n_rows, out, out_ld, s);
+}
+
+// Dense rows of a multiple of 256 elements (every lane's chain is as long; no more than 4096, the caller's limit), inputs
+// that can be read 16 bytes at a time.  Four waves per tile while two blocks a CU hold the call (256 rows with their
+// selection: 17 us at 512 tokens against 22.6 with two waves and 23.4 on the vector pipe), else two (4096 tokens: 63
+// against 70, and 97).
+template <int ACT>
+bool run_router_chains(const RouterParams& rp, const RowsDesc& r, uint32_t n_rows, float* out, uint32_t out_ld, hipStream_t s) {
+    if (r.kind != 16 || rp.d % 256 || !rp.x_vec || (rp.eff_scale && !aligned16(rp.eff_scale))) return false;
+    const bool few = (size_t)((n_rows + 31) / 32) * ((rp.tokens + 15) / 16) <= 512;
+    if (rp.d % 1024)
+        return few ? launch_router_chains_any<ACT, 4, 1>(rp, r, n_rows, out, out_ld, s)
+                   : launch_router_chains_any<ACT, 2, 1>(rp, r, n_rows, out, out_ld, s);
+    return few ? launch_router_chains_any<ACT, 4, 4>(rp, r, n_rows, out, out_ld, s)
+               : launch_router_chains_any<ACT, 2, 4>(rp, r, n_rows, out, out_ld, s);
+}
+
 // d <= 2048 dense / 4096 at 8 bit / 8192 at 4 bit (8 chunks per lane).
 template <int ACT>
 void run_router_tiled(const RouterParams& rp, const RowsDesc& r, uint32_t n_rows, float* out, uint32_t out_ld,
@@ -232,6 +264,7 @@ void run_router_tiled(const RouterParams& rp, const RowsDesc& r, uint32_t n_rows
 #undef NVMAI_SINGLE
         return;
     }
+    if (run_router_chains<ACT>(rp, r, n_rows, out, out_ld, s)) return;
     const size_t lds = (size_t)RT_TOK * rp.d * 2;
     const uint32_t per_block = 8 * (r.kind == 4 ? 2 : 4);
     dim3 grid((n_rows + per_block - 1) / per_block, (rp.tokens + RT_TOK - 1) / RT_TOK);

@@ -1015,6 +1015,130 @@ __global__ __launch_bounds__(256, KIND == 16 ? 4 : 2) void router_logits_tiled_k
         }
 }
 
+// ---- the same for dense rows, on the matrix pipe ---------------------------------------------------
+// A product with one step of k per instruction adds fma(w, x, sum) to every sum, which is the multiply-add of the
+// order above: v_mfma_f32_16x16x1_4b_f32 runs four of the 32 lanes' chains of sixteen rows x sixteen tokens at a time,
+// at twice the rate of the vector pipe's multiply-adds, and the conversions from 16 bits are shared by sixteen rows or
+// tokens.  A wave runs chains 4 n .. 4 n + 3 to their ends and adds the chains in the order of the butterfly: n ^ 4,
+// n ^ 2, n ^ 1 (offsets 16, 8, 4) as they end, then the four of an instruction (offsets 2, 1).
+// SPLIT (2 or 4) waves share a tile of sixteen rows, each with the chains whose n is its own modulo SPLIT; U chunks of
+// a row are under way per wave (d / 256 is a multiple of it).  The block's sixteen tokens lie in LDS as stored, rows 16
+// bytes off a multiple of 256: a read touches every bank once; under EFF the scales are a row of their own behind them.
+// Bound by the matrix pipe: 4096 tokens of 2048 against 256 rows take 52 us against 89 on the vector pipe, 82 TFLOP/s.
+typedef float rt_f4 __attribute__((ext_vector_type(4)));
+typedef float rt_f16 __attribute__((ext_vector_type(16)));
+
+__host__ __device__ constexpr uint32_t router_chain_pitch(uint32_t d) { return d * 2u + 16u; }
+
+template <int ACT, bool EFF, int SPLIT, int U>
+__global__ __launch_bounds__(512) void router_chain_kernel(RouterParams p, RowsDesc r, uint32_t n_rows, float* out, uint32_t out_ld) {
+    extern __shared__ uint4 router_lds[];
+    char* xl = reinterpret_cast<char*>(router_lds);
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, i = lane & 15u, b = lane >> 4;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), share = wave % SPLIT;
+    const uint32_t row0 = (blockIdx.x * (8u / SPLIT) + wave / SPLIT) * 16u, t0 = blockIdx.y * 16u;
+    const uint32_t pitch = router_chain_pitch(p.d), its = p.d / 256u;
+    // chain 4 n + b takes the 16-byte chunks 4 n + b + 32 it; rows past the end repeat the last one, unused
+    const uint16_t* wr = static_cast<const uint16_t*>(r.w) + (size_t)min(row0 + i, n_rows - 1u) * p.d + 8u * b;
+    auto start = [&](uint32_t g) {                   // n of the wave's g-th group: partners follow each other
+        return SPLIT == 4 ? share + 4u * g : share + ((g & 1u) << 2) + (g & 2u);
+    };
+    uint4 w[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) w[u] = *reinterpret_cast<const uint4*>(wr + start(0) * 32u + u * 256u);
+    {
+        const uint16_t* x = static_cast<const uint16_t*>(p.x);
+        const uint32_t per_row = p.d / 8u, total = 16u * per_row;
+#pragma unroll 8
+        for (uint32_t e = tid; e < total; e += 512u) {
+            const uint32_t t = e / per_row, c = e % per_row;         // tokens past the end repeat the last one, unused
+            *reinterpret_cast<uint4*>(xl + t * pitch + c * 16u) =
+                *reinterpret_cast<const uint4*>(x + (size_t)min(t0 + t, p.tokens - 1u) * p.x_stride + c * 8u);
+        }
+    }
+    if (EFF) for (uint32_t c = tid * 8u; c < p.d; c += 4096u) *reinterpret_cast<uint4*>(xl + 16u * pitch + c * 2u) = *reinterpret_cast<const uint4*>(p.eff_scale + c);
+    __syncthreads();
+    constexpr int LEVELS = SPLIT == 4 ? 1 : 2;
+    rt_f16 acc, level[LEVELS];
+    uint4 xr;                                        // the next step's chunks of the tokens
+    auto read_x = [&](uint32_t e0) { xr = *reinterpret_cast<const uint4*>(xl + i * pitch + e0 * 2u); };
+    read_x(start(0) * 32u + 8u * b);
+#pragma unroll 1
+    for (uint32_t g = 0; g < 8u / SPLIT; ++g) {
+        const uint32_t here = start(g), next = start(min(g + 1u, 8u / SPLIT - 1u));
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc[j] = 0.0f;
+#pragma unroll 1
+        for (uint32_t k = 0; k < its; k += U) {
+            const bool last = k + U >= its;
+            const uint32_t ahead = last ? 0u : k + U;
+            const uint16_t* wn = wr + (last ? next : here) * 32u;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                float q[8];                          // converted before the next request: the same registers take it
+                act2_to_f32<ACT_BF16>(w[u].x, q[0], q[1]); act2_to_f32<ACT_BF16>(w[u].y, q[2], q[3]);
+                act2_to_f32<ACT_BF16>(w[u].z, q[4], q[5]); act2_to_f32<ACT_BF16>(w[u].w, q[6], q[7]);
+                __builtin_amdgcn_sched_barrier(0);
+                w[u] = *reinterpret_cast<const uint4*>(wn + (ahead + u) * 256u);
+                const uint32_t e0 = here * 32u + 8u * b + (k + u) * 256u;
+                float x[8], ef[8];
+                if (EFF) {
+                    const uint4 e = *reinterpret_cast<const uint4*>(xl + 16u * pitch + e0 * 2u);
+                    act2_to_f32<ACT_BF16>(e.x, ef[0], ef[1]); act2_to_f32<ACT_BF16>(e.y, ef[2], ef[3]);
+                    act2_to_f32<ACT_BF16>(e.z, ef[4], ef[5]); act2_to_f32<ACT_BF16>(e.w, ef[6], ef[7]);
+                }
+                const uint4 v = xr;
+                act2_to_f32<ACT>(v.x, x[0], x[1]); act2_to_f32<ACT>(v.y, x[2], x[3]);
+                act2_to_f32<ACT>(v.z, x[4], x[5]); act2_to_f32<ACT>(v.w, x[6], x[7]);
+                if (EFF) {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) x[j] = __fmul_rn(x[j], ef[j]);
+                }
+                read_x(k + u + 1 < its ? e0 + 256u : next * 32u + 8u * b);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x1f32(q[j], x[j], acc, 0, 0, 0);
+            }
+        }
+        // the groups' sums by a binary counter: a group's partner is the one before it, a pair's the pair before it
+#pragma unroll
+        for (int v = 0; v < LEVELS; ++v) {
+            const bool add = (g >> v) & 1u;
+            if (add) {
+                acc += level[v];
+            } else {
+                level[v] = acc;
+                break;
+            }
+        }
+    }
+    {                                                // n ^ 2 and n ^ 1, or n ^ 1, across the waves of a tile
+        __syncthreads();                             // the tokens have been read
+        rt_f4* part = reinterpret_cast<rt_f4*>(xl) + wave * 256u + lane;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) part[j * 64] = rt_f4{acc[4 * j], acc[4 * j + 1], acc[4 * j + 2], acc[4 * j + 3]};
+        __syncthreads();
+        if (share) return;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            rt_f4 a = part[j * 64], c = part[256 + j * 64];
+            if (SPLIT == 4) {
+                a += part[512 + j * 64];
+                c += part[768 + j * 64];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[4 * j + e] = a[e] + c[e];
+        }
+    }
+    // block v of the product is chain 4 n + v; a lane holds rows 4 b .. 4 b + 3 of its token
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float sum = (acc[e] + acc[8 + e]) + (acc[4 + e] + acc[12 + e]);
+        const uint32_t token = t0 + i, row = row0 + 4u * b + e;
+        if (token < p.tokens && row < n_rows) out[(size_t)token * out_ld + row] = sum;
+    }
+}
+
 // One row (the shared expert's gate row) against many tokens: a half-wave per token, its inputs read
 // straight from memory (16 bytes per lane and load; nothing is shared between tokens but the one row,
 // which every half-wave reads from cache), all of a lane's loads requested before the first sum.  The
