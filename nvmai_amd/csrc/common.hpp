@@ -213,6 +213,15 @@ __device__ __forceinline__ void unpack_chunk(const uint4& w, float* q) {
     }
 }
 
+// All of each wave's requests into LDS landed and its reads of LDS done, for every wave of the block: what a kernel that loads
+// straight into LDS has to pass before it reads what other waves requested.  __syncthreads() alone does not wait for
+// such loads.  The wait is the builtin, which the compiler counts with: behind inline asm it adds waits of its own
+// at the next read, for the requests made since.
+__device__ __forceinline__ void lds_landed_barrier() {
+    __builtin_amdgcn_s_waitcnt(0x0070);              // vmcnt(0) lgkmcnt(0)
+    __syncthreads();
+}
+
 __device__ __forceinline__ float silu(float v) { return v / (1.0f + expf(-v)); }
 
 // silu through the hardware exp2 and reciprocal (about 1e-6 relative): for kernels

@@ -703,7 +703,9 @@ __global__ __launch_bounds__(256, NP + RP + DV <= 320 ? 2 : 1) void latent_flash
     const uint32_t full_lo = first_key(p.rows.position + wt1, p.window) - p.key0, full_hi = p.rows.position + wt0 + 1u - p.key0;
     const uint32_t krow = 8u * (i >> 2) + (i & 3u);              // key of this lane's row in an even score tile
     auto tile = [&](uint32_t k0, const uint8_t* cur, uint8_t* next) {
-        __syncthreads();                             // this tile has landed; everyone is done with the other stage
+        // This tile has landed and everyone is done with the other stage.  The wait stands here by name: a workgroup's barrier
+        // does not wait for loads into LDS, and a wave that skips a tile waits for its part of it all the same.
+        lds_landed_barrier();
         if (k0 + 64u < k_hi) issue(k0 + 64u, next);
         if (!wave_live || k0 >= w_hi || k0 + 64u <= w_lo) return;               // wave-uniform
         la_f4 s[2][4];

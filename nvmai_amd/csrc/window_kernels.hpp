@@ -517,7 +517,9 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void window_flash_kern
     const uint32_t krow = 8u * (i >> 2) + (i & 3u);              // key of this lane's row in an even score tile
     const float slope = p.alibi ? wa_slope_log2(head, p.heads) : 0.0f;
     auto tile = [&](uint32_t n, const uint8_t* cur, uint8_t* next) {
-        __syncthreads();                             // this tile has landed; everyone is done with the other stage
+        // This tile has landed and everyone is done with the other stage.  The wait stands here by name: a workgroup's barrier
+        // does not wait for loads into LDS, and a wave that skips a tile waits for its part of it all the same.
+        lds_landed_barrier();
         if (n + 1u < count) issue(n + 1u, next);
         const uint32_t k0 = position_of(n);
         if (!wave_live || k0 >= w_hi || (k0 + 64u <= w_lo && k0 >= p.keep)) return;                // wave-uniform
