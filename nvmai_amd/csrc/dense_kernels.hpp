@@ -81,17 +81,17 @@ __device__ __forceinline__ dn_f4 dense_finish4(const DenseLinearParams& p, uint3
         dn_f4 m{1.0f, 1.0f, 1.0f, 1.0f};
         if (p.mul) {
             const uint32_t id = p.mul_ids[t];
-            const uint16_t* at = p.mul + (size_t)min(id, p.mul_rows - 1u) * p.mul_stride + r0;
-            const float live = id < p.mul_rows ? 1.0f : 0.0f;
-            if ((reinterpret_cast<uintptr_t>(p.mul) & 7u) == 0 && (p.mul_stride & 3u) == 0) {
-                const uint2 q = *reinterpret_cast<const uint2*>(at);
-                m = dn_f4{__uint_as_float(q.x << 16), __uint_as_float(q.x & 0xFFFF0000u), __uint_as_float(q.y << 16), __uint_as_float(q.y & 0xFFFF0000u)};
-            } else {
+            m = dn_f4{0.0f, 0.0f, 0.0f, 0.0f};
+            if (id < p.mul_rows) {                   // an id past the table, which may have no row at all, reads nothing
+                const uint16_t* at = p.mul + (size_t)id * p.mul_stride + r0;
+                if ((reinterpret_cast<uintptr_t>(p.mul) & 7u) == 0 && (p.mul_stride & 3u) == 0) {
+                    const uint2 q = *reinterpret_cast<const uint2*>(at);
+                    m = dn_f4{__uint_as_float(q.x << 16), __uint_as_float(q.x & 0xFFFF0000u), __uint_as_float(q.y << 16), __uint_as_float(q.y & 0xFFFF0000u)};
+                } else {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) m[j] = bf16_to_f32(at[j]);
+                    for (int j = 0; j < 4; ++j) m[j] = bf16_to_f32(at[j]);
+                }
             }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) m[j] = live != 0.0f ? m[j] : 0.0f;
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[j] = dense_activate<ACT>(p.activation, v[j] + bias[j]) * m[j];

@@ -66,6 +66,33 @@ def test_two_launches_with_every_epilogue(kind):
     check(y32, want, 3e-6)              # the sum's 2e-6, and 1e-6 for a GELU by hardware exponentials
 
 
+# rows: a wave per weight row, the short products, the tiles; strides: four multipliers at once, one by one
+@pytest.mark.parametrize("act", ["bf16", "fp32"])
+@pytest.mark.parametrize("rows", [3, 40, 200])
+@pytest.mark.parametrize("n,stride", [(128, 128), (126, 131)])
+def test_a_table_without_rows_multiplies_by_zero(act, rows, n, stride):
+    """Nothing of the table is read: what lies there is not a number, and the ids are as large as they can be."""
+    import ctypes as C
+
+    import nvmai_amd as nv
+    from nvmai_amd._lib import LinearEpilogue, check, lib
+    say("multipliers past the table", act, rows, n)
+    ctx = nv.Context(0, nv.ACT_FP32 if act == "fp32" else nv.ACT_BF16)
+    w, x = operands(rows, n, 64, ctx.dtype, rows)
+    table = torch.full((3, stride), float("nan"), device="cuda", dtype=torch.bfloat16)
+    table[0] = 2.0
+    ids = torch.full((rows,), -1, dtype=torch.int32, device="cuda")
+    ids[::2] = 0
+    stream = torch.cuda.current_stream().cuda_stream
+    for table_rows in (0, 1):
+        y = torch.full((rows, n), 7.0, device="cuda")
+        e = LinearEpilogue(nv.LINEAR_NONE, None, table.data_ptr(), ids.data_ptr(), stride, table_rows)
+        check(lib.nvmai_hip_dense_linear_ex(ctx.handle, stream, w.data_ptr(), 64, x.data_ptr(), 64, rows, n, 64, None, y.data_ptr(), n, C.byref(e)), "dense")
+        want = x.double() @ w.double().T * 2.0 * table_rows
+        want[1::2] = 0.0
+        assert float((y.double() - want).abs().max()) < 1e-5 and bool((y[1::2] == 0).all())
+
+
 def test_32_bit_values_keep_every_bit():
     """The planes of 32-bit rows hold them exactly: unit rows of the matrix give the inputs back, whatever their size."""
     import nvmai_amd as nv
