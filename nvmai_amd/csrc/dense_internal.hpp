@@ -19,10 +19,11 @@ struct DenseLinearParams {
     uint16_t* planes;       // dense_plane_bytes of scratch for the rows of a 32-bit context, or nullptr
 };
 
-// 32-bit rows are multiplied as three BF16 planes, at most this many rows (128 MB) at a time.
+// 32-bit rows are multiplied as three BF16 planes, at most this many rows at a time: 128 MB of planes, or one row's (1.3 GB for
+// the longest that a call accepts), so that byte offsets inside them stay within 32 bits.
 inline uint32_t dense_plane_rows(uint32_t k) {
-    const uint32_t rows = (128u << 20) / (6u * k) / 256u * 256u;
-    return rows ? (rows < 32768u ? rows : 32768u) : 256u;
+    const uint64_t rows = (128u << 20) / (6ull * k);
+    return rows >= 32768u ? 32768u : rows >= 256u ? (uint32_t)(rows / 256u * 256u) : rows ? (uint32_t)rows : 1u;
 }
 void dense_split(hipStream_t s, const float* x, uint32_t x_stride, uint32_t rows, uint32_t k, uint16_t* planes);
 inline size_t dense_plane_bytes(uint32_t rows, uint32_t k) {

@@ -128,3 +128,24 @@ def test_a_captured_call_without_workspace_still_runs():
         graph.replay()
         torch.cuda.synchronize()
         check(y, want, 2e-6)
+
+
+# 2560 rows of 8192 k fill the portion of planes that is made at a time, 47 rows of 475,776, and seven of three million
+@pytest.mark.parametrize("rows,n,k", [(2565, 72, 8192), (2560, 8, 8192), (5130, 40, 8192), (100, 24, 475776), (257, 16, 2800000)])
+def test_32_bit_rows_in_portions(rows, n, k):
+    """Every portion's rows of x, the outputs and the ids; sums of a long k in a total per 64."""
+    import nvmai_amd as nv
+    say("32-bit rows in portions", rows, n, k)
+    ctx = nv.Context(0, nv.ACT_FP32)
+    w, x = operands(rows, n, k, torch.float32, k)
+    want = torch.cat([x[a:a + 64].double() @ w.double().T for a in range(0, rows, 64)])
+    y, y32 = (torch.full((rows, n), 7.0, device="cuda") for _ in range(2))
+    nv.dense_linear(ctx, w, x, y=y, y_f32=y32)
+    # a total per 64 k: rounded k / 64 times, 2^-24 sqrt(k / 64) of the largest value and below 1.3e-5 at the longest k; twice that
+    tol = max(2e-6, 2 * 2 ** -24 * (k / 64) ** 0.5)
+    check(y32, want, tol)
+    assert torch.equal(y, y32)
+    bias, mul = torch.randn(n, device="cuda").to(torch.bfloat16), torch.randn((50, n), device="cuda").to(torch.bfloat16)
+    ids = torch.arange(rows, device="cuda", dtype=torch.int32) * 7 % 50
+    nv.dense_linear(ctx, w, x, y_f32=y32, bias=bias, activation=nv.LINEAR_GELU_TANH, mul=mul, mul_ids=ids)
+    check(y32, torch.nn.functional.gelu(want + bias.double(), approximate="tanh") * mul.double()[ids.long()], 2 * tol)
