@@ -17,23 +17,28 @@ __device__ __forceinline__ dn_f4 dn_mfma(const uint4& a, const uint4& b, dn_f4 c
 // z/2 (1 + erf(z / sqrt 2))
 __device__ __forceinline__ float gelu_erf(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
 
-// The same by formula 7.1.26 of Abramowitz and Stegun, erfc(x) = (a1 t + .. + a5 t^5) e^(-x^2), t = 1 / (1 + p x), off by at most
-// 1.5e-7: about a third of erff's instructions and no branch, for results of 16-bit contexts.  z < 0 takes erfc itself (one
-// minus erf would cancel).
-__device__ __forceinline__ float gelu_erf_fast(float z) {
-    const float x = fabsf(z) * 0.70710678118654752f, t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, x, 1.0f));
-    const float poly = t * fmaf(t, fmaf(t, fmaf(t, fmaf(t, 1.061405429f, -1.453152027f), 1.421413741f), -0.284496736f), 0.254829592f);
-    const float c = poly * __builtin_amdgcn_exp2f(-1.4426950408889634f * x * x);
-    return 0.5f * z * (z < 0.0f ? c : 2.0f - c);
-}
-
 // z/2 (1 + tanh(sqrt(2/pi) (z + 0.044715 z^3)))
 __device__ __forceinline__ float gelu_tanh(float z) { return 0.5f * z * (1.0f + tanhf(0.79788456080286536f * fmaf(0.044715f * z * z, z, z))); }
 
-// z / (1 + e^(-2 u)), which is the same, through the hardware's exponential and reciprocal: for results of 16-bit contexts.
-__device__ __forceinline__ float gelu_tanh_fast(float z) {
-    const float u = 0.79788456080286536f * fmaf(0.044715f * z * z, z, z);
-    return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-2.8853900817779268f * u));
+// Both without the library's branches, for the tiles, whose stores erff and tanhf lengthen by a third (2048 x 8192 x 2048 with
+// GELU_ERF: 85 us, 75 with this, 62 without an activation).  z Phi(z), Phi(z) = 1/2 + z R(z^2) for |z| < 1, and past it
+// s or 1 - s with s = Phi(-|z|), which does not cancel: e^(-z^2 / 2) times a polynomial in 1 / (1 + 0.34 |z|), or 1 / (1 + e^(2 |u|)).  The
+// polynomials are minimax fits to erf, erfc e^(z^2 / 2) and tanh in double.  Largest error against 64 bits on the device, in 2^-24 of z / 2,
+// beside that of erff's form (tanhf's is alike): z in -8 .. -4 0.00 and 0.50, -4 .. -2 0.26 and 0.76, -2 .. -1 1.4 and 1.6, -1 .. 0 1.5 and 1.7,
+// 0 .. 1 3.0 and 3.3, 1 .. 8 3.2 and 4.1.
+__device__ __forceinline__ float gelu_join(float z, float inner, float tail) { return z * (fabsf(z) < 1.0f ? fmaf(z, inner, 0.5f) : z < 0.0f ? tail : 1.0f - tail); }
+
+__device__ __forceinline__ float gelu_erf_parts(float z) {
+    const float q = z * z, t = __builtin_amdgcn_rcpf(fmaf(0.34f, fabsf(z), 1.0f));
+    const float inner = fmaf(q, fmaf(q, fmaf(q, fmaf(q, fmaf(q, -7.530304e-06f, 1.13143644e-04f), -1.1859847e-03f), 9.973171e-03f), -6.649033e-02f), 0.3989423f);
+    const float tail = fmaf(t, fmaf(t, fmaf(t, fmaf(t, fmaf(t, -0.12013893f, 0.37782046f), -0.1036036f), 0.22889116f), 0.11511663f), 1.8795595e-03f);
+    return gelu_join(z, inner, tail * __builtin_amdgcn_exp2f(-0.72134752044448170f * q));
+}
+
+__device__ __forceinline__ float gelu_tanh_parts(float z) {
+    const float q = z * z, u = 0.79788456080286536f * fmaf(0.044715f * q, z, z);
+    const float inner = fmaf(q, fmaf(q, fmaf(q, fmaf(q, fmaf(q, -7.0424426e-06f, 1.1754699e-04f), -1.2428056e-03f), 1.0201477e-02f), -6.681947e-02f), 0.3989423f);
+    return gelu_join(z, inner, __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(2.8853900817779268f * fabsf(u))));
 }
 
 // What stands between a sum and its store, fixed when a kernel is built: a tile's store is unrolled many times, and code
@@ -41,20 +46,21 @@ __device__ __forceinline__ float gelu_tanh_fast(float z) {
 // bias; PAIRS: SILU_PAIRS; FULL: bias, any activation, the token's own multiplier.
 enum DenseEpilogue : int { DE_PLAIN, DE_ERF, DE_BIAS, DE_PAIRS, DE_FULL };
 
-template <int ACT>
+// PARTS: the forms for tiles, in 16-bit contexts.
+template <bool PARTS>
 __device__ __forceinline__ float dense_activate(int activation, float v) {
-    if (activation == NVMAI_LINEAR_GELU_ERF) return ACT == ACT_FP32 ? gelu_erf(v) : gelu_erf_fast(v);
-    if (activation == NVMAI_LINEAR_GELU_TANH) return ACT == ACT_FP32 ? gelu_tanh(v) : gelu_tanh_fast(v);
+    if (activation == NVMAI_LINEAR_GELU_ERF) return PARTS ? gelu_erf_parts(v) : gelu_erf(v);
+    if (activation == NVMAI_LINEAR_GELU_TANH) return PARTS ? gelu_tanh_parts(v) : gelu_tanh(v);
     return v;
 }
 
-template <int EPI, int ACT>
+template <int EPI, bool PARTS>
 __device__ __forceinline__ float dense_finish(const DenseLinearParams& p, uint32_t t, uint32_t r, float v) {
-    if (EPI == DE_ERF) return dense_activate<ACT>(NVMAI_LINEAR_GELU_ERF, v);
+    if (EPI == DE_ERF) return dense_activate<PARTS>(NVMAI_LINEAR_GELU_ERF, v);
     if (EPI == DE_BIAS) return v + bf16_to_f32(p.bias[r]);
     if (EPI != DE_FULL) return v;
     if (p.bias) v += bf16_to_f32(p.bias[r]);
-    v = dense_activate<ACT>(p.activation, v);
+    v = dense_activate<PARTS>(p.activation, v);
     if (p.mul) {                                     // an id past the table: zero
         const uint32_t id = p.mul_ids[t];
         v *= id < p.mul_rows ? bf16_to_f32(p.mul[(size_t)id * p.mul_stride + r]) : 0.0f;
@@ -75,7 +81,7 @@ __device__ __forceinline__ dn_f4 dense_bias4(const DenseLinearParams& p, uint32_
 }
 
 // dense_finish of four neighbouring rows whose biases the caller holds.
-template <int EPI, int ACT>
+template <int EPI, bool PARTS>
 __device__ __forceinline__ dn_f4 dense_finish4(const DenseLinearParams& p, uint32_t t, uint32_t r0, dn_f4 v, dn_f4 bias) {
     if constexpr (EPI == DE_FULL) {
         dn_f4 m{1.0f, 1.0f, 1.0f, 1.0f};
@@ -94,10 +100,10 @@ __device__ __forceinline__ dn_f4 dense_finish4(const DenseLinearParams& p, uint3
             }
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = dense_activate<ACT>(p.activation, v[j] + bias[j]) * m[j];
+        for (int j = 0; j < 4; ++j) v[j] = dense_activate<PARTS>(p.activation, v[j] + bias[j]) * m[j];
     } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = EPI == DE_ERF ? dense_activate<ACT>(NVMAI_LINEAR_GELU_ERF, v[j]) : EPI == DE_BIAS ? v[j] + bias[j] : v[j];
+        for (int j = 0; j < 4; ++j) v[j] = EPI == DE_ERF ? dense_activate<PARTS>(NVMAI_LINEAR_GELU_ERF, v[j]) : EPI == DE_BIAS ? v[j] + bias[j] : v[j];
     }
     return v;
 }
@@ -108,9 +114,9 @@ __device__ __forceinline__ void dense_put(const DenseLinearParams& p, uint32_t t
     if (p.y_f32) p.y_f32[(size_t)t * p.y_stride + r] = v;
 }
 
-template <int EPI, int ACT>
+template <int EPI, int ACT, bool PARTS = false>
 __device__ __forceinline__ void dense_store(const DenseLinearParams& p, uint32_t t, uint32_t r, float v) {
-    dense_put<ACT>(p, t, r, dense_finish<EPI, ACT>(p, t, r, v));
+    dense_put<ACT>(p, t, r, dense_finish<EPI, PARTS>(p, t, r, v));
 }
 
 // Rows 2 j and 2 j + 1 of the matrix make output j: silu(gate) * up.
@@ -118,7 +124,7 @@ template <int ACT>
 __device__ __forceinline__ float dense_pair(float gate, float up) { return (ACT == ACT_FP32 ? silu(gate) : silu_fast(gate)) * up; }
 
 // Four neighbouring outputs of one token (r0 a multiple of 4).
-template <int EPI, int ACT>
+template <int EPI, int ACT, bool PARTS = false>
 __device__ __forceinline__ void dense_store4(const DenseLinearParams& p, uint32_t t, uint32_t r0, dn_f4 v, dn_f4 bias) {
     if (EPI == DE_PAIRS) {                           // n and the row stride are even
         const float a = dense_pair<ACT>(v[0], v[1]), b = dense_pair<ACT>(v[2], v[3]);
@@ -133,7 +139,7 @@ __device__ __forceinline__ void dense_store4(const DenseLinearParams& p, uint32_
             dense_put<ACT>(p, t, r0 / 2u, a);
         }
     } else if (r0 + 4u <= p.n && (p.y_stride & 3u) == 0) {
-        v = dense_finish4<EPI, ACT>(p, t, r0, v, bias);
+        v = dense_finish4<EPI, PARTS>(p, t, r0, v, bias);
         if (p.y) {
             act_t<ACT>* y = static_cast<act_t<ACT>*>(p.y) + (size_t)t * p.y_stride + r0;
             if constexpr (ACT == ACT_FP32) {
@@ -149,7 +155,7 @@ __device__ __forceinline__ void dense_store4(const DenseLinearParams& p, uint32_
     } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-            if (r0 + j < p.n) dense_store<EPI, ACT>(p, t, r0 + j, v[j]);
+            if (r0 + j < p.n) dense_store<EPI, ACT, PARTS>(p, t, r0 + j, v[j]);
     }
 }
 
@@ -472,7 +478,7 @@ __global__ __launch_bounds__(256, BN + BM <= 128 ? 2 : 1) void dense_tile_kernel
         for (uint32_t k = 0; k < 32u / AT_ONCE; ++k) {
             const uint32_t at = lane / PER + k * AT_ONCE, t = m0 + wm + 32 * b + at;
             const dn_f4 v = *reinterpret_cast<const dn_f4*>(turn + at * PITCH + lane % PER * 4u);
-            if (t < p.rows && r < p.n) dense_store4<EPI, ACT>(p, t, r, v, bias);
+            if (t < p.rows && r < p.n) dense_store4<EPI, ACT, !SPLIT>(p, t, r, v, bias);
         }
     }
 }

@@ -149,3 +149,24 @@ def test_32_bit_rows_in_portions(rows, n, k):
     ids = torch.arange(rows, device="cuda", dtype=torch.int32) * 7 % 50
     nv.dense_linear(ctx, w, x, y_f32=y32, bias=bias, activation=nv.LINEAR_GELU_TANH, mul=mul, mul_ids=ids)
     check(y32, torch.nn.functional.gelu(want + bias.double(), approximate="tanh") * mul.double()[ids.long()], 2 * tol)
+
+
+@pytest.mark.parametrize("act", ["bf16", "fp32"])
+@pytest.mark.parametrize("rows", [3, 40, 200, 2000])
+def test_gelu_in_32_bit_precision(act, rows):
+    """Unit rows of the matrix hand the inputs on, so only the activation rounds.  z/2 (1 + erf(z / sqrt 2)) for z in [-4, 1]: the argument is
+    off by 2^-25, erff by two units of 2^-24, the sum rounds by 2^-24 and the product by 2^-23 at most, in all below 6 * 2^-24 of z / 2."""
+    import nvmai_amd as nv
+    say("gelu", act, rows)
+    ctx = nv.Context(0, nv.ACT_FP32 if act == "fp32" else nv.ACT_BF16)
+    eye = torch.eye(64, device="cuda", dtype=torch.bfloat16)
+    x = (torch.rand((rows, 64), device="cuda", generator=torch.Generator(device="cuda").manual_seed(rows)) * 5.0 - 4.0).to(torch.bfloat16)
+    z = x.double()
+    y = torch.empty((rows, 64), device="cuda")
+    nv.dense_linear(ctx, eye, x.to(ctx.dtype), y_f32=y, activation=nv.LINEAR_GELU_ERF)
+    want = 0.5 * z * torch.special.erfc(-z * 0.5 ** 0.5)
+    assert bool(((y.double() - want).abs() <= 6 * 2.0 ** -24 * z.abs() / 2).all())
+    tanh = torch.empty((rows, 64), device="cuda")
+    nv.dense_linear(ctx, eye, x.to(ctx.dtype), y_f32=tanh, activation=nv.LINEAR_GELU_TANH)
+    want = torch.nn.functional.gelu(z, approximate="tanh")
+    assert bool(((tanh.double() - want).abs() <= 6 * 2.0 ** -24 * z.abs() / 2).all())
