@@ -334,6 +334,22 @@ __device__ __forceinline__ void dense_stage_barrier() {
 #endif
 }
 
+// One sum of the planes again, in fp32 multiply-adds of the values that the planes stand for.  An infinite weight makes NaN of a
+// value's lower planes where they are zero, and planes of sums that overflow can cancel: a NaN comes from here or not at all.
+__device__ __forceinline__ float dense_sum_again(const DenseLinearParams& p, uint32_t t, uint32_t r) {
+    const uint16_t *w = p.w + (size_t)r * p.w_stride, *x = static_cast<const uint16_t*>(p.x) + (size_t)t * p.x_stride;
+    float total = 0.0f;
+#pragma unroll 1
+    for (uint32_t k0 = 0; k0 < p.k; k0 += 64u) {
+        float sum = 0.0f;
+#pragma unroll 1
+        for (uint32_t k = k0; k < k0 + 64u; ++k)
+            sum = fmaf(bf16_to_f32(w[k]), (bf16_to_f32(x[2u * p.k + k]) + bf16_to_f32(x[p.k + k])) + bf16_to_f32(x[k]), sum);
+        total += sum;
+    }
+    return total;
+}
+
 // Of 160 KB; two blocks per compute unit where the tile is small.  Planes come in threes: six stages where they fit (64 x 64, 700 x
 // 1024 x 1024 in 32 bits: 17.4 us with three, 13.5 with six).
 constexpr int dense_stages(int act, int bn, int bm) {
@@ -466,6 +482,7 @@ __global__ __launch_bounds__(256, BN + BM <= 128 ? 2 : 1) void dense_tile_kernel
     const dn_f4 bias = dense_bias4<EPI>(p, r);
 #pragma unroll
     for (int b = 0; b < TM; ++b) {
+        [[maybe_unused]] bool again = false;
 #pragma unroll
         for (int a = 0; a < TN; ++a) {
             dn_f16 v = acc[a][b];
@@ -473,6 +490,21 @@ __global__ __launch_bounds__(256, BN + BM <= 128 ? 2 : 1) void dense_tile_kernel
 #pragma unroll
             for (int h = 0; h < 4; ++h)                      // element 4 h + e of a lane: row 8 h + 4 g + e, token i
                 *reinterpret_cast<dn_f4*>(turn + i * PITCH + 32 * a + 8 * h + 4u * g) = dn_f4{v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]};
+            if constexpr (SPLIT) {
+                bool none = false;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) none |= v[e] != v[e];
+                again |= none;
+            }
+        }
+        if constexpr (SPLIT) {
+            if (__any(again)) {
+                for (uint32_t e = lane; e < 32u * ROWS; e += 64u) {
+                    const uint32_t t = m0 + wm + 32 * b + e / ROWS, row = n0 + wn + e % ROWS;
+                    float& sum = turn[e / ROWS * PITCH + e % ROWS];
+                    if (sum != sum && t < p.rows && row < p.n) sum = dense_sum_again(p, t, row);
+                }
+            }
         }
 #pragma unroll UNROLL
         for (uint32_t k = 0; k < 32u / AT_ONCE; ++k) {

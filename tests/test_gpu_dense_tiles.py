@@ -170,3 +170,24 @@ def test_gelu_in_32_bit_precision(act, rows):
     nv.dense_linear(ctx, eye, x.to(ctx.dtype), y_f32=tanh, activation=nv.LINEAR_GELU_TANH)
     want = torch.nn.functional.gelu(z, approximate="tanh")
     assert bool(((tanh.double() - want).abs() <= 6 * 2.0 ** -24 * z.abs() / 2).all())
+
+
+# tiles of every size a 32-bit context has, one row a wave
+@pytest.mark.parametrize("rows,n", [(3, 70), (70, 70), (700, 500), (2048, 2100)])
+def test_infinite_weights_meet_32_bit_rows(rows, n):
+    """An infinite weight gives an infinity of the input's sign, NaN only against zero or another infinity: whatever the planes of the
+    input are (1.0 has zeros in two of them)."""
+    import nvmai_amd as nv
+    say("infinite weights", rows, n)
+    k, inf = 192, float("inf")
+    w, x = operands(rows, n, k, torch.float32, 9)
+    x[:, 5] = torch.tensor([1.0, -2.0, 0.1, 0.0, 1e30], device="cuda").repeat(rows)[:rows]
+    w[3, 5], w[n - 1, 5], w[n - 1, 70], w[20, 191] = inf, -inf, inf, -inf
+    x[2, 100] = inf
+    y = torch.empty((rows, n), device="cuda")
+    nv.dense_linear(nv.Context(0, nv.ACT_FP32), w, x, y_f32=y)
+    want = (x.cpu().double() @ w.cpu().double().T).cuda()
+    assert torch.equal(y.isnan(), want.isnan())
+    assert torch.equal(y.isinf(), want.isinf()) and torch.equal(y[y.isinf()].double(), want[want.isinf()])
+    finite = want.isfinite()
+    assert int(finite.sum()) > (n - 4) * (rows - 1) and float((y.double() - want)[finite].abs().max()) < 1e24      # 1e30 among the inputs
