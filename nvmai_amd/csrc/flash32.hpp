@@ -18,10 +18,14 @@ constexpr float FLASH32_NONE = -1e30f;      // maximum of no scores; a masked sc
 // pipe (157 TFLOP/s) at thousands.
 //   KC: chunks of 16 dims; NV: 16-wide parts of the values.  query(c), key(tile, c): 16 bytes of dims 16 c + 4 g of query / key i
 // (zeros where there are none).  VT: values(tile, n) is value 16 n + i of keys 4 g .. 4 g + 3; otherwise values(tile, j * NV / 4 + b)
-// is values 64 b + 4 i .. + 3 of key 4 g + j.  score(tile, j, s): the score of key 4 g + j in powers of two, masked.  put(value, v): the
-// block's result of query i at a value index.  shared: NV * 1024 + 128 floats.
-template <int KC, int NV, bool VT, class Query, class Key, class Values, class Score, class Put>
-__device__ __forceinline__ void flash32_block(uint32_t tiles, float* shared, Query query, Key key, Values values, Score score, Put put) {
+// is values 64 b + 4 i .. + 3 of key 4 g + j.  score(tile, j, s): the score of key 4 g + j in powers of two.  whole(tile): every query of the
+// block sees all of the tile (the same in all lanes); sees(tile, j, query): a query of the block sees key 4 g + j.  put(value, v): the block's
+// result of query i at a value index.  shared: NV * 1024 + 128 floats.
+//   A key that a query does not see has probability zero, and zero times an infinity or NaN among its values would be NaN.  A tile
+// that is not seen whole is looked over for such values, and where there are any it is multiplied for one query at a time, with the
+// values of the keys that this query does not see set to zero.
+template <int KC, int NV, bool VT, class Query, class Key, class Values, class Score, class Whole, class Sees, class Put>
+__device__ __forceinline__ void flash32_block(uint32_t tiles, float* shared, Query query, Key key, Values values, Score score, Whole whole, Sees sees, Put put) {
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, i = lane & 15u, g = lane >> 4;
     f32_f4 q[KC], k[KC], v[NV], acc[NV];
 #pragma unroll
@@ -49,6 +53,11 @@ __device__ __forceinline__ void flash32_block(uint32_t tiles, float* shared, Que
         s += s1;
 #pragma unroll
         for (int j = 0; j < 4; ++j) s[j] = score(t, j, s[j]);
+        const bool part = !whole(t);
+        if (part) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s[j] = sees(t, j, i) ? s[j] : 2.0f * FLASH32_NONE;
+        }
         float tm = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
         tm = fmaxf(tm, shfl_xor_f(tm, 16));
         tm = fmaxf(tm, shfl_xor_f(tm, 32));
@@ -63,11 +72,35 @@ __device__ __forceinline__ void flash32_block(uint32_t tiles, float* shared, Que
 #pragma unroll
         for (int j = 0; j < 4; ++j) s[j] = __builtin_amdgcn_exp2f(s[j] - m);
         l += (s[0] + s[1]) + (s[2] + s[3]);
+        auto value = [&](int n, int j) { return VT ? v[n][j] : v[j * (NV / 4) + n / 4][n % 4]; };      // of key 4 g + j
+        if (part) {
+            uint32_t largest = 0;
+#pragma unroll
+            for (int n = 0; n < NV; ++n)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) largest = max(largest, __float_as_uint(v[n][j]) & 0x7FFFFFFFu);
+            if (__any(largest >= 0x7F800000u)) {
+#pragma unroll 1
+                for (uint32_t one = 0; one < 16u; ++one) {
+                    bool seen[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) seen[j] = sees(t, j, one);
+#pragma unroll
+                    for (int n = 0; n < NV; ++n) {
+                        f32_f4 sum{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(seen[j] ? value(n, j) : 0.0f, i == one ? s[j] : 0.0f, sum, 0, 0, 0);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) acc[n][j] += i == one ? sum[j] : 0.0f;
+                    }
+                }
+                continue;
+            }
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
-            for (int n = 0; n < NV; ++n)
-                acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(VT ? v[n][j] : v[j * (NV / 4) + n / 4][n % 4], s[j], acc[n], 0, 0, 0);
+            for (int n = 0; n < NV; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(value(n, j), s[j], acc[n], 0, 0, 0);
     }
     l += shfl_xor_f(l, 16);
     l += shfl_xor_f(l, 32);

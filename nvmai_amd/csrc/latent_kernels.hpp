@@ -578,9 +578,9 @@ __global__ __launch_bounds__(256, 2) void latent_flash32_kernel(LatentAttnParams
     const uint32_t lane = threadIdx.x & 63u, i = lane & 15u, g = lane >> 4;
     // the heads of a row of blocks lie on the XCDs in turn; the queries with the most keys come first
     const uint32_t nq = (p.n_rows + 15u) / 16u, head = blockIdx.x % p.heads, q0 = (nq - 1u - blockIdx.x / p.heads) * 16u;
-    const uint32_t row = min(q0 + i, p.n_rows - 1u), pos = p.rows.position + row, last = p.rows.position + min(q0 + 15u, p.n_rows - 1u);
+    const uint32_t row = min(q0 + i, p.n_rows - 1u), last = p.rows.position + min(q0 + 15u, p.n_rows - 1u);
     // keys are numbered from key0; rows past the last key are zeros up to a multiple of 64
-    const uint32_t lo = first_key(pos, p.window) - p.key0, hi = pos + 1u - p.key0, first_t = (first_key(p.rows.position + q0, p.window) - p.key0) / 16u;
+    const uint32_t first_t = (first_key(p.rows.position + q0, p.window) - p.key0) / 16u;
     const float* q = static_cast<const float*>(p.q) + (size_t)row * p.q_stride + head * (p.nope + p.rot) + 4u * g;
     const float* kn = static_cast<const float*>(p.kn) + head * p.nope + 4u * g;
     const float* kr = static_cast<const float*>(p.lat) + p.rank + 4u * g;
@@ -599,9 +599,14 @@ __global__ __launch_bounds__(256, 2) void latent_flash32_kernel(LatentAttnParams
             const uint32_t key = (first_t + t) * 16u + 4u * g + n / (NV / 4), d = 64u * (n % (NV / 4));
             return d + 4u * i < p.vdim ? *reinterpret_cast<const f32_f4*>(v + (size_t)key * p.v_stride + d) : none;
         },
-        [&](uint32_t t, int j, float s) {
-            const uint32_t key = (first_t + t) * 16u + 4u * g + j;
-            return key >= lo && key < hi ? s * p.scale_log2 : 2.0f * FLASH32_NONE;
+        [&](uint32_t, int, float s) { return s * p.scale_log2; },
+        [&](uint32_t t) {
+            const uint32_t at = (first_t + t) * 16u;
+            return at >= first_key(last, p.window) - p.key0 && at + 15u <= p.rows.position + q0 - p.key0;
+        },
+        [&](uint32_t t, int j, uint32_t query) {
+            const uint32_t key = (first_t + t) * 16u + 4u * g + j, pos = p.rows.position + min(q0 + query, p.n_rows - 1u);
+            return key >= first_key(pos, p.window) - p.key0 && key < pos + 1u - p.key0;
         },
         [&](uint32_t d, float o) {
             if (q0 + i < p.n_rows && d < p.vdim) static_cast<float*>(p.out)[(size_t)row * p.out_stride + head * p.vdim + d] = o * gate;

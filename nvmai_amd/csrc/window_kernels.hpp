@@ -420,9 +420,13 @@ __global__ __launch_bounds__(256, 2) void window_flash32_kernel(WindowParams p) 
             const uint32_t key = position_of(t) + 4u * g + j;
             s *= p.a;
             if (p.capped) s = p.b * tanhf(s);
-            s = fmaf(-slope, (float)(int32_t)(pos - key), s);
-            return wa_visible(pos, key, p.window, p.keep) ? s : 2.0f * FLASH32_NONE;
+            return fmaf(-slope, (float)(int32_t)(pos - key), s);
         },
+        [&](uint32_t t) {
+            const uint32_t at = position_of(t);
+            return at + 15u <= start + q0 && (at >= first_key(last, p.window) || at + 15u < p.keep);
+        },
+        [&](uint32_t t, int j, uint32_t query) { return wa_visible(start + min(q0 + query, p.n_rows - 1u), position_of(t) + 4u * g + j, p.window, p.keep); },
         [&](uint32_t d, float o) {
             if (q0 + i < p.n_rows && d < dv) static_cast<float*>(p.out)[(size_t)row * p.out_stride + head * dv + d] = o * gate;
         });
