@@ -133,8 +133,9 @@ int run_attention(nvmai_hip_ctx* ctx, nvmai_stream stream, AttnParams p, const n
     p.num_chunks = nc; p.chunk_len = chunk_len;
     // A ragged batch over long contexts: the same blocks and partial rows, dealt out by the sequences' lengths.  With as many
     // chunks for every sequence the longest ones' set the time and the others' blocks end early.  Finding its place costs a
-    // block about a microsecond; chunks of DEAL_FROM keys take 20 and more.  Eight 8-bit sequences of 64K to 128K: 174 -> 160 us, of 20K to 40K: 67 -> 59; two
-    // blocks per compute unit (4 bit) even the lengths out by themselves (115 us either way).
+    // block about a microsecond; chunks of DEAL_FROM keys take 20 and more.  8-bit, us without and with: 8 sequences of 64K to 128K
+    // 167 -> 144, 16 of 16K to 32K 93 -> 83, 32 of 1K to 32K 161 -> 95, 64 of 4K to 8K 107 -> 105; equal lengths keep the uniform split
+    // (8 x 128K 204 -> 205, 16 x 32K 104 -> 104).  Two blocks per compute unit (4 bit) even the lengths out by themselves (117 us either way).
     constexpr uint32_t DEAL_FROM = 2048;
     const bool deal = fast && k->bits == 8 && p.seq_lens && p.cols_q == 1 && nc > 1 && chunk_len >= DEAL_FROM && p.batch > 1 && p.batch <= 64 && nc * p.batch <= ATTN_MAX_CHUNKS;
     if (!p.direct) {
@@ -155,8 +156,11 @@ int run_attention(nvmai_hip_ctx* ctx, nvmai_stream stream, AttnParams p, const n
         ProfScope ps(ctx, NVMAI_PROF_ATTN_PARTIAL, s);
         if (fast) {
             dim3 grid(seq_blocks * p.num_kv_heads * nc);      // dealt out: cols_q is 1, so slots * num_kv_heads
-#define NVMAI_ATTN(ACT, BITS) attn_partial_mfma_kernel<ACT, BITS><<<grid, 256, 0, s>>>(p)
-            if (ctx->act == ACT_BF16) { if (k->bits == 8) NVMAI_ATTN(ACT_BF16, 8); else NVMAI_ATTN(ACT_BF16, 4); }
+#define NVMAI_ATTN(ACT, BITS) attn_partial_mfma_kernel<ACT, BITS, false><<<grid, 256, 0, s>>>(p)
+            if (p.slots) {
+                if (ctx->act == ACT_BF16) attn_partial_mfma_kernel<ACT_BF16, 8, true><<<grid, 256, 0, s>>>(p);
+                else attn_partial_mfma_kernel<ACT_FP16, 8, true><<<grid, 256, 0, s>>>(p);
+            } else if (ctx->act == ACT_BF16) { if (k->bits == 8) NVMAI_ATTN(ACT_BF16, 8); else NVMAI_ATTN(ACT_BF16, 4); }
             else { if (k->bits == 8) NVMAI_ATTN(ACT_FP16, 8); else NVMAI_ATTN(ACT_FP16, 4); }
 #undef NVMAI_ATTN
         } else {
@@ -168,8 +172,14 @@ int run_attention(nvmai_hip_ctx* ctx, nvmai_stream stream, AttnParams p, const n
     if (!p.direct) {
         ProfScope ps(ctx, NVMAI_PROF_ATTN_COMBINE, s);
         const dim3 cgrid((uint32_t)heads_total, (p.head_dim + 63) / 64);
-        if (ctx->act == ACT_BF16) attn_combine_kernel<ACT_BF16><<<cgrid, 256, 0, s>>>(p);
-        else attn_combine_kernel<ACT_FP16><<<cgrid, 256, 0, s>>>(p);
+#define NVMAI_COMBINE(ACT)                                                          \
+    do {                                                                            \
+        if (p.slots) attn_combine_kernel<ACT, true><<<cgrid, 256, 0, s>>>(p);       \
+        else attn_combine_kernel<ACT, false><<<cgrid, 256, 0, s>>>(p);              \
+    } while (0)
+        if (ctx->act == ACT_BF16) NVMAI_COMBINE(ACT_BF16);
+        else NVMAI_COMBINE(ACT_FP16);
+#undef NVMAI_COMBINE
     }
     return launch_status();
 }

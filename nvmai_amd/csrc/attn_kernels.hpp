@@ -156,8 +156,8 @@ struct AttnParams {
     uint32_t ring;             // not 0: row of key p is p % ring (generic kernel only)
     uint32_t cols_q;           // sequences sharing one block of the matrix-core kernel
     uint32_t direct;           // num_chunks == 1: the partial kernel normalises and writes out itself
-    // A ragged batch dealt out by length (0: num_chunks chunks for every sequence): blocks per KV head, and per sequence its
-    // first block and how many it has, which the partial kernel writes for the combine.  Partial rows then lie
+    // A ragged batch dealt out by length (the kernels' DEAL): blocks per KV head (num_chunks * batch), and per sequence its first
+    // block and how many it has, which the partial kernel writes for the combine.  Partial rows then lie
     // [num_kv_heads, slots, heads of a KV head].
     uint32_t slots;
     uint32_t* seq_slots;       // [2][batch]
@@ -193,22 +193,28 @@ __device__ __forceinline__ uint32_t attn_wave_sum(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
-// Block `slot` of a KV head in a ragged batch of at most 64: which sequence, which of its chunks, how long a chunk is.  The lanes
-// look at a sequence each; the chunk length (a multiple of 32, 128 at least) is the one with which half a chunk per sequence is left
-// over, or where that does not fit a whole one, which always does.  A sequence without keys has one block, which leaves an
-// empty partial row.  false: a block that is left over.
+// Block `slot` of a KV head in a ragged batch of at most 64: which sequence, which of its chunks, how long a chunk is (a multiple of 32,
+// 128 at least).  The lanes look at a sequence each.  The shortest of four lengths whose chunks fit into the slots (num_chunks per
+// sequence): all slots filled (equal sequences: the uniform split), half a chunk per sequence left over, a whole one, which always
+// fits, and the longest sequence in num_chunks, which fits too: no chunk is longer than without dealing.  A sequence without
+// keys has one block, which leaves an empty partial row.  false: a block that is left over.
 __device__ __forceinline__ bool attn_deal(const AttnParams& p, uint32_t slot, uint32_t& b, uint32_t& chunk, uint32_t& chunk_len, uint32_t& first, uint32_t& count) {
     const uint32_t lane = threadIdx.x & 63u;
     uint32_t lo = 0, hi = 0;
     if (lane < p.batch) attn_range(p, lane, lo, hi);
-    const uint32_t len = hi - lo, total = attn_wave_sum(len);
-    uint32_t n = 0;
-    for (uint32_t part = 2; part >= 1; --part) {
-        const uint32_t share = p.slots - p.batch / part;                 // slots >= 2 batch
-        chunk_len = max(((total + share - 1u) / share + 31u) & ~31u, 128u);
-        n = lane < p.batch ? max((len + chunk_len - 1u) / chunk_len, 1u) : 0u;
-        if (attn_wave_sum(n) <= p.slots) break;
+    const uint32_t len = hi - lo, total = attn_wave_sum(len), longest = ~wave_min_u32(~len);
+    auto in_blocks = [](uint32_t keys, uint32_t blocks) { return max(((keys + blocks - 1u) / blocks + 31u) & ~31u, 128u); };
+    auto blocks = [&](uint32_t of) { return lane < p.batch ? max((len + of - 1u) / of, 1u) : 0u; };
+    chunk_len = min(in_blocks(longest, p.num_chunks), in_blocks(total, p.slots - p.batch));           // slots >= 2 batch
+    for (uint32_t left = 0; left <= 1u; ++left) {
+        const uint32_t shorter = in_blocks(total, p.slots - left * (p.batch / 2u));
+        if (shorter >= chunk_len) break;
+        if (attn_wave_sum(blocks(shorter)) <= p.slots) {
+            chunk_len = shorter;
+            break;
+        }
     }
+    const uint32_t n = blocks(chunk_len);
     b = 0;
     first = 0;
     for (;; ++b) {
@@ -287,7 +293,7 @@ __global__ __launch_bounds__(256) void attn_partial_generic_kernel(AttnParams p)
 // ceil(head_dim / 64)); the four waves of a block split the chunks of 64 output dims.
 constexpr uint32_t ATTN_MAX_CHUNKS = 512;
 
-template <int ACT>
+template <int ACT, bool DEAL>
 __global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams p) {
     __shared__ float wgt[ATTN_MAX_CHUNKS];
     __shared__ float red[8];
@@ -297,7 +303,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams p) {
     // where this head's partial rows begin, how many there are and how far apart
     size_t row0 = bh * p.num_chunks;
     uint32_t count = p.num_chunks, pitch = 1;
-    if (p.slots) {
+    if constexpr (DEAL) {
         const uint32_t seq = (uint32_t)(bh / p.num_q_heads), head = (uint32_t)(bh % p.num_q_heads);
         pitch = p.num_q_heads / p.num_kv_heads;
         row0 = ((size_t)(head / pitch) * p.slots + p.seq_slots[seq]) * pitch + head % pitch;
@@ -404,7 +410,7 @@ __device__ __forceinline__ float attn_exp(float x) { return __builtin_amdgcn_exp
 constexpr int ATTN_HD = 256;
 constexpr int ATTN_STEP = 32;
 
-template <int ACT, int BITS>
+template <int ACT, int BITS, bool DEAL>
 __global__ __launch_bounds__(256, 2) void attn_partial_mfma_kernel(AttnParams p) {
     // LDS.  Every wave owns a K region and a V region, filled by buffer_load ... lds without
     // touching registers: 32 tokens x the codes of this KV head, the 16-byte chunks of a token
@@ -435,7 +441,7 @@ __global__ __launch_bounds__(256, 2) void attn_partial_mfma_kernel(AttnParams p)
     uint32_t chunk, kvh, b, chunk_len = p.chunk_len;               // b: first sequence of this block
     size_t part_row;                                               // partial row of (b, first head of kvh, this chunk)
     uint32_t part_pitch;                                           // rows from one head to the next
-    if (p.slots) {                                                 // one sequence per block (cols_q is 1)
+    if constexpr (DEAL) {                                          // one sequence per block (cols_q is 1)
         uint32_t first, count;
         kvh = blockIdx.x / p.slots;
         if (!attn_deal(p, blockIdx.x % p.slots, b, chunk, chunk_len, first, count)) return;

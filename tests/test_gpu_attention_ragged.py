@@ -39,3 +39,23 @@ def test_dealt_out_by_length(bits, lens, heads):
             want = att.encode_full(q[b:b + 1], kb, vb, 256, nq, nkv, n, kv_start=0 if begin is None else begin[b])[0].float()
             # the same sums in chunks of another length: two roundings to BF16 apart
             assert float((out[b].float() - want).abs().max() / want.abs().max()) < 2 ** -7, b
+
+
+@pytest.mark.parametrize("lens", [[40000] * 8, [16384] * 48, [8192] * 64, [8191] * 64, [50001] * 3], ids=lambda v: "%dx%d" % (len(v), v[0]))
+@pytest.mark.parametrize("heads", [(16, 2), (8, 8)], ids=["gqa", "mha"])
+def test_equal_lengths_are_cut_as_an_even_batch(lens, heads):
+    """No chunk is longer than in the uniform split, and equal sequences get that split back: the bits of a call that knows the length."""
+    import nvmai_amd as nv
+    say("ragged with equal lengths", heads, len(lens), lens[0])
+    ctx = nv.Context(0, nv.ACT_BF16)
+    gen = torch.Generator(device="cuda").manual_seed(len(lens))
+    (nq, nkv), B, n = heads, len(lens), lens[0]
+    k, v = (nv.KVCache(B, n, nkv * 256, 8) for _ in range(2))
+    rows = torch.randn((n, nkv * 256), device="cuda", generator=gen).to(torch.bfloat16)
+    for c in (k, v):
+        for b in range(B):
+            nv.KVCacheQuantizer(ctx).encode(rows.roll(b + (c is v), 0), nkv * 256, c.view(b), n, nkv * 256)
+    q = torch.randn((B, nq, 256), device="cuda", generator=gen).to(torch.bfloat16)
+    att = nv.Attention(ctx)
+    got = att.encode_ragged(q, k, v, 256, nq, nkv, torch.tensor(lens, dtype=torch.int32, device="cuda"), n)
+    assert torch.equal(got, att.encode_full(q, k, v, 256, nq, nkv, n))
