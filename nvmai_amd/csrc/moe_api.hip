@@ -236,9 +236,9 @@ bool launch_router_chains_any(const RouterParams& rp, const RowsDesc& r, uint32_
 // selection: 17 us at 512 tokens against 22.6 with two waves and 23.4 on the vector pipe), else two (4096 tokens: 63
 // against 70, and 97).
 template <int ACT>
-bool run_router_chains(const RouterParams& rp, const RowsDesc& r, uint32_t n_rows, float* out, uint32_t out_ld, hipStream_t s) {
+bool run_router_chains(const RouterParams& rp, uint32_t cus, const RowsDesc& r, uint32_t n_rows, float* out, uint32_t out_ld, hipStream_t s) {
     if (r.kind != 16 || rp.d % 256 || !rp.x_vec || (rp.eff_scale && !aligned16(rp.eff_scale))) return false;
-    const bool few = (size_t)((n_rows + 31) / 32) * ((rp.tokens + 15) / 16) <= 512;
+    const bool few = (size_t)((n_rows + 31) / 32) * ((rp.tokens + 15) / 16) <= 2 * (size_t)cus;
     if (rp.d % 1024)
         return few ? launch_router_chains_any<ACT, 4, 1>(rp, r, n_rows, out, out_ld, s)
                    : launch_router_chains_any<ACT, 2, 1>(rp, r, n_rows, out, out_ld, s);
@@ -248,7 +248,7 @@ bool run_router_chains(const RouterParams& rp, const RowsDesc& r, uint32_t n_row
 
 // d <= 2048 dense / 4096 at 8 bit / 8192 at 4 bit (8 chunks per lane).
 template <int ACT>
-void run_router_tiled(const RouterParams& rp, const RowsDesc& r, uint32_t n_rows, float* out, uint32_t out_ld,
+void run_router_tiled(const RouterParams& rp, uint32_t cus, const RowsDesc& r, uint32_t n_rows, float* out, uint32_t out_ld,
                       hipStream_t s) {
     const uint32_t cpl = (rows_chunks(r.kind, rp.d) + 31) / 32;
     if (n_rows == 1 && rp.x_vec && cpl <= 8) {      // one row (the shared expert's gate): a half-wave per token, no staging
@@ -264,7 +264,7 @@ void run_router_tiled(const RouterParams& rp, const RowsDesc& r, uint32_t n_rows
 #undef NVMAI_SINGLE
         return;
     }
-    if (run_router_chains<ACT>(rp, r, n_rows, out, out_ld, s)) return;
+    if (run_router_chains<ACT>(rp, cus, r, n_rows, out, out_ld, s)) return;
     const size_t lds = (size_t)RT_TOK * rp.d * 2;
     const uint32_t per_block = 8 * (r.kind == 4 ? 2 : 4);
     dim3 grid((n_rows + per_block - 1) / per_block, (rp.tokens + RT_TOK - 1) / RT_TOK);
@@ -279,16 +279,18 @@ void run_router_tiled(const RouterParams& rp, const RowsDesc& r, uint32_t n_rows
 #undef NVMAI_TILED
 }
 
-int run_router(int act, RouterParams& rp, hipStream_t s) {
+int run_router(const nvmai_hip_ctx* ctx, RouterParams& rp, hipStream_t s) {
+    const int act = ctx->act;
+    const uint32_t cus = (uint32_t)ctx->compute_units;
     rp.x_vec = aligned16(rp.x) && (rp.x_stride % 8 == 0);
     // Many tokens (a prefill block): the register-tiled kernel, same logits bit for bit
     if (rp.tokens >= 64 && (size_t)RT_TOK * rp.d * 2 <= 65536) {
         if (act == ACT_BF16) {
-            if (rp.num_experts) run_router_tiled<ACT_BF16>(rp, rp.router, rp.num_experts, rp.logits, rp.num_experts, s);
-            if (rp.gate.kind) run_router_tiled<ACT_BF16>(rp, rp.gate, 1, rp.gate_logit, 1, s);
+            if (rp.num_experts) run_router_tiled<ACT_BF16>(rp, cus, rp.router, rp.num_experts, rp.logits, rp.num_experts, s);
+            if (rp.gate.kind) run_router_tiled<ACT_BF16>(rp, cus, rp.gate, 1, rp.gate_logit, 1, s);
         } else {
-            if (rp.num_experts) run_router_tiled<ACT_FP16>(rp, rp.router, rp.num_experts, rp.logits, rp.num_experts, s);
-            if (rp.gate.kind) run_router_tiled<ACT_FP16>(rp, rp.gate, 1, rp.gate_logit, 1, s);
+            if (rp.num_experts) run_router_tiled<ACT_FP16>(rp, cus, rp.router, rp.num_experts, rp.logits, rp.num_experts, s);
+            if (rp.gate.kind) run_router_tiled<ACT_FP16>(rp, cus, rp.gate, 1, rp.gate_logit, 1, s);
         }
         return NVMAI_OK;
     }
@@ -668,7 +670,7 @@ extern "C" int nvmai_hip_moe_router_topk(nvmai_hip_ctx* ctx, nvmai_stream stream
     rp.router = to_desc(router);
     rp.x = hidden; rp.eff_scale = eff_scale; rp.x_stride = hidden_stride; rp.tokens = n_tokens;
     rp.num_experts = num_experts; rp.d = d; rp.logits = logits; rp.gate_logit = nullptr;
-    rc = run_router(ctx->act, rp, s);
+    rc = run_router(ctx, rp, s);
     if (rc) return rc;
     SelectParams sp{logits, per_expert_scale, n_tokens, num_experts, top_k, out_idx, out_w};
     select_topk_kernel<<<(n_tokens + 3) / 4, 256, 0, s>>>(sp);
@@ -832,7 +834,7 @@ extern "C" int nvmai_hip_shared_expert(nvmai_hip_ctx* ctx, nvmai_stream stream, 
             rp.gate = to_desc(shared_gate);
             rp.x = x; rp.x_stride = x_stride; rp.tokens = n_tokens; rp.num_experts = 0; rp.d = d;
             rp.logits = dummy_logits; rp.gate_logit = gate_logit;
-            rc = run_router(ctx->act, rp, s);
+            rc = run_router(ctx, rp, s);
             if (rc) return rc;
         }
         return nvmai::expert_ffn_dense(ctx, s, (const uint8_t*)blob, off, bits, x, x_stride, n_tokens, d, f, act, tmp,
@@ -858,7 +860,7 @@ extern "C" int nvmai_hip_shared_expert(nvmai_hip_ctx* ctx, nvmai_stream stream, 
                 rp.gate = to_desc(shared_gate);
                 rp.x = x; rp.x_stride = x_stride; rp.tokens = n_tokens; rp.num_experts = 0; rp.d = d;
                 rp.logits = dummy_logits; rp.gate_logit = gate_logit;
-                rc = run_router(ctx->act, rp, s);
+                rc = run_router(ctx, rp, s);
                 if (rc) return rc;
             }
             RowsParams p{};
@@ -898,7 +900,7 @@ extern "C" int nvmai_hip_shared_expert(nvmai_hip_ctx* ctx, nvmai_stream stream, 
         rp.gate = to_desc(shared_gate);
         rp.x = x; rp.x_stride = x_stride; rp.tokens = n_tokens; rp.num_experts = 0; rp.d = d;
         rp.logits = dummy_logits; rp.gate_logit = gate_logit;
-        rc = run_router(ctx->act, rp, s);
+        rc = run_router(ctx, rp, s);
         if (rc) return rc;
     }
     RowsParams p{};
@@ -1030,7 +1032,7 @@ int decode_layer_impl(nvmai_hip_ctx* ctx, nvmai_stream stream, const nvmai_moe_l
     GroupParams gp{sp, (uint32_t)maxtok, has_shared ? 1 : 0, entries, n_entries, stats, pair_token, pair_id,
                    ctx->tickets};
     if (fused_decode_ok(T, K, has_shared, D, F, L->bits)) {
-        { ProfScope ps(ctx, NVMAI_PROF_ROUTER, s); rc = run_router(ctx->act, rp, s); }
+        { ProfScope ps(ctx, NVMAI_PROF_ROUTER, s); rc = run_router(ctx, rp, s); }
         if (rc) return rc;
         RowsParams p{};
         p.src.pool_base = (const uint8_t*)L->experts_base;
@@ -1055,7 +1057,7 @@ int decode_layer_impl(nvmai_hip_ctx* ctx, nvmai_stream stream, const nvmai_moe_l
     // Two launches on purpose: one that also selects and groups in its last blocks needs a
     // device-scope release (an L2 write-back on this multi-die part) from every one of its
     // hundreds of producer blocks, and measured 18 us slower per step.
-    { ProfScope ps(ctx, NVMAI_PROF_ROUTER, s); rc = run_router(ctx->act, rp, s); }
+    { ProfScope ps(ctx, NVMAI_PROF_ROUTER, s); rc = run_router(ctx, rp, s); }
     if (rc) return rc;
     {
         ProfScope ps(ctx, NVMAI_PROF_GROUP, s);
