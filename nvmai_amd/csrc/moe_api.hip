@@ -219,7 +219,10 @@ bool launch_router_chains(const RouterParams& rp, const RowsDesc& r, uint32_t n_
     const size_t tokens = (size_t)(EFF ? 17 : 16) * router_chain_pitch(rp.d), sums = 8 * 4096;
     const size_t lds = tokens > sums ? tokens : sums;
     const void* kernel = reinterpret_cast<const void*>(router_chain_kernel<ACT, EFF, SPLIT, U>);
-    if (lds > 64 * 1024 && hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return false;
+    if (lds > 64 * 1024 && hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
+        (void)hipGetLastError();                     // the other kernel is launched instead
+        return false;
+    }
     const dim3 grid((n_rows + 128 / SPLIT - 1) / (128 / SPLIT), (rp.tokens + 15) / 16);
     router_chain_kernel<ACT, EFF, SPLIT, U><<<grid, 512, lds, s>>>(rp, r, n_rows, out, out_ld);
     return true;
