@@ -17,7 +17,11 @@
  *     nvmai_hip_ctx_destroy, so a captured graph stays valid whatever is called
  *     later.  A call that would have to grow while its stream is being captured
  *     returns NVMAI_ERR_SCRATCH and launches nothing: run the same call eagerly once,
- *     or nvmai_hip_ctx_reserve, before capturing.
+ *     or nvmai_hip_ctx_reserve, before capturing.  Three kinds of call that have a form with
+ *     less or no workspace record that one instead, slower and with other roundings:
+ *     nvmai_hip_dense_linear[_ex] and the expanded nvmai_hip_latent_attention of a 32-bit
+ *     context (products without BF16 planes), and nvmai_hip_attention_decode_ragged (chunks of
+ *     one length for every sequence).  They do the same where memory cannot be allocated.
  * Data formats (reference file:line):
  *   - weights: affine group-64 codes, 4 bit (two per byte, element 2k in the low
  *     nibble of byte k) or 8 bit, plus one BF16 scale and one BF16 bias per group
@@ -754,8 +758,10 @@ enum { NVMAI_LINEAR_NONE = 0, NVMAI_LINEAR_GELU_ERF = 1, NVMAI_LINEAR_GELU_TANH 
 enum { NVMAI_FORM_AUTO = 0, NVMAI_GLA_RECURRENT = 1, NVMAI_GLA_CHUNKED = 2, NVMAI_LATENT_ABSORBED = 1, NVMAI_LATENT_EXPANDED = 2 };
 
 /* y[t, :] = act(W x[t, :]) for any number of rows: a wave per weight row up to 4 rows, split-k matrix-core products
- * up to 64, LDS-tiled matrix-core products above; fp32 FMA in a 32-bit context.  y (activations) and / or y_f32, one
- * row stride for both. */
+ * up to 64, LDS-tiled matrix-core products above.  In a 32-bit context: fp32 FMA up to 4 rows; above, the rows as three BF16
+ * planes in the workspace (6 k bytes a row, 128 MB at most), whose products with the weights are exact, summed in fp32.  A
+ * value's planes add up to it where it is 2^-110 or more in magnitude and to within 2^-133 below that.  y (activations)
+ * and / or y_f32, one row stride for both. */
 int nvmai_hip_dense_linear(nvmai_hip_ctx* ctx, nvmai_stream stream, const uint16_t* w, uint32_t w_stride, const void* x,
                            uint32_t x_stride, uint32_t rows, uint32_t n, uint32_t k, void* y, float* y_f32, uint32_t y_stride,
                            int activation);

@@ -140,14 +140,13 @@ int run_attention(nvmai_hip_ctx* ctx, nvmai_stream stream, AttnParams p, const n
     const bool deal = fast && k->bits == 8 && p.seq_lens && p.cols_q == 1 && nc > 1 && chunk_len >= DEAL_FROM && p.batch > 1 && p.batch <= 64 && nc * p.batch <= ATTN_MAX_CHUNKS;
     if (!p.direct) {
         const size_t own = 2 * ws_round(heads_total * nc * 4) + ws_round(heads_total * nc * p.head_dim * 4), more = ws_round(2 * p.batch * 4);
-        int rc = deal ? ws_begin(ctx, stream, own + more) : NVMAI_ERR_SCRATCH;
-        if (rc == NVMAI_OK) {
+        if (deal && ws_begin(ctx, stream, own + more) == NVMAI_OK) {
             p.slots = nc * p.batch;
             p.seq_slots = ws_take<uint32_t>(ctx, 2 * p.batch);
-        } else if (rc == NVMAI_ERR_SCRATCH) {                    // not dealt out, or no place for the table under a capture
-            rc = ws_begin(ctx, stream, own);
+        } else {                                                 // not dealt out, or no place for the table (under a capture)
+            const int rc = ws_begin(ctx, stream, own);
+            if (rc) return rc;
         }
-        if (rc) return rc;
         p.m_part = ws_take<float>(ctx, heads_total * nc);
         p.d_part = ws_take<float>(ctx, heads_total * nc);
         p.o_part = ws_take<float>(ctx, heads_total * nc * p.head_dim);

@@ -69,7 +69,10 @@ inline int ws_begin(nvmai_hip_ctx* ctx, nvmai_stream stream, size_t bytes) {
     size_t cap = ctx->ws_cap ? ctx->ws_cap : (size_t)1 << 20;
     while (cap < bytes) cap *= 2;
     uint8_t* block = nullptr;
-    NVMAI_HIP_TRY(hipMalloc(reinterpret_cast<void**>(&block), cap));
+    if (hipMalloc(reinterpret_cast<void**>(&block), cap) != hipSuccess) {
+        (void)hipGetLastError();         // a caller may have a form that needs less
+        return NVMAI_ERR_HIP;
+    }
     if (ctx->ws) ctx->ws_retired.push_back(ctx->ws);
     ctx->ws = block;
     ctx->ws_cap = cap;

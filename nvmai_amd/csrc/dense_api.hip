@@ -74,16 +74,14 @@ int dense_linear(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p) 
 
 namespace {
 
-// An entry point's own call: the planes of 32-bit rows lie in the workspace.  Where a stream that is being captured finds it
-// too small the product is made without them.
+// An entry point's own call: the planes of 32-bit rows lie in the workspace.  Where it cannot be made large enough (while the
+// stream is being captured, or without memory) the product is made without them.
 int dense_linear_call(nvmai_hip_ctx* ctx, nvmai_stream stream, DenseLinearParams p) {
     const int rc = dense_linear_check(ctx, p);
     if (rc) return rc;
     if (ctx->act == NVMAI_ACT_FP32 && p.rows > 4) {
         const size_t bytes = dense_plane_bytes(p.rows, p.k);
-        const int got = ws_begin(ctx, stream, ws_round(bytes));
-        if (got == NVMAI_OK) p.planes = ws_take<uint16_t>(ctx, bytes / 2);
-        else if (got != NVMAI_ERR_SCRATCH) return got;
+        if (ws_begin(ctx, stream, ws_round(bytes)) == NVMAI_OK) p.planes = ws_take<uint16_t>(ctx, bytes / 2);
     }
     return dense_linear(ctx, (hipStream_t)stream, p);
 }

@@ -171,16 +171,17 @@ extern "C" int nvmai_hip_latent_attention(nvmai_hip_ctx* ctx, nvmai_stream strea
     flash = flash && widest * 2 < 0x7FFFFFFFull && (uint64_t)vh * (p.nk_pad + 64) * 2 < 0x7FFFFFFFull;
     p.v_stride = odd_lines(flash ? p.nk_pad : vh);
     const size_t n_lat = (size_t)p.nk_pad * cache->row_stride, n_kn = (size_t)p.nk_pad * p.kn_stride, n_v = (size_t)(flash ? vh : p.nk_pad) * p.v_stride;
-    const size_t n_planes = f32 ? dense_plane_bytes(p.nk_pad, c.rank) / 2 : 0;
-    rc = ws_begin(ctx, stream, ws_round(n_lat * esz) + ws_round(n_kn * esz) + ws_round(n_v * esz) + ws_round(n_planes * 2));
-    if (rc) return rc;
+    const size_t n_planes = f32 ? dense_plane_bytes(p.nk_pad, c.rank) / 2 : 0, own = ws_round(n_lat * esz) + ws_round(n_kn * esz) + ws_round(n_v * esz);
+    // without room for the planes (under a capture) the two products are made without them
+    const bool planes = f32 && ws_begin(ctx, stream, own + ws_round(n_planes * 2)) == NVMAI_OK;
+    if (!planes && (rc = ws_begin(ctx, stream, own))) return rc;
     p.lat = ws_take<uint8_t>(ctx, n_lat * esz);
     p.kn = ws_take<uint8_t>(ctx, n_kn * esz);
     p.v = ws_take<uint8_t>(ctx, n_v * esz);
     DenseLinearParams lk{uk, p.lat, p.kn, nullptr, c.rank, cache->row_stride, p.kn_stride, p.nk_pad, nh, c.rank, NVMAI_LINEAR_NONE};
     DenseLinearParams lv = flash ? DenseLinearParams{static_cast<const uint16_t*>(p.lat), uv, p.v, nullptr, cache->row_stride, c.rank, p.v_stride, vh, p.nk_pad, c.rank, NVMAI_LINEAR_NONE}
                                        : DenseLinearParams{uv, p.lat, p.v, nullptr, c.rank, cache->row_stride, p.v_stride, p.nk_pad, vh, c.rank, NVMAI_LINEAR_NONE};
-    if (f32) lk.planes = lv.planes = ws_take<uint16_t>(ctx, n_planes);
+    if (planes) lk.planes = lv.planes = ws_take<uint16_t>(ctx, n_planes);
     if ((rc = dense_linear_check(ctx, lk)) || (rc = dense_linear_check(ctx, lv))) return rc;
     const size_t lds_rot = (size_t)c.rotary_dims * 4;
     if (f32) {

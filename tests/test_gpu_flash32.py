@@ -69,3 +69,30 @@ def test_latent_rows_that_are_not_numbers_stay_with_the_queries_that_see_them(he
         sees = np.array([j <= i and (window == 0 or i - j < window) for i in range(n)])
         assert np.isnan(got[sees]).all() and np.isfinite(got[~sees]).all()
         assert (np.abs(got - want)[~sees] < 2e-6 * np.abs(want).max()).all()
+
+
+def test_a_captured_latent_prompt_runs_without_room_for_planes():
+    """A workspace that holds the keys and values (3.5 MB) but not the planes of their products (1 MB more): recorded without them."""
+    import torch
+
+    import nvmai_amd as nv
+    say("captured 32-bit latent prompt")
+    ctx, n = nv.Context(0, nv.ACT_FP32), 300
+    L = Latent(ctx, np.random.default_rng(5), 8, 128, 64, 128, 512, 0, n)
+    want = L.run([n], nv.LATENT_EXPANDED)
+    small = nv.Context(0, nv.ACT_FP32)
+    small.reserve(4 << 20)
+    op = nv.LatentAttention(small, L.heads, L.nope, L.rot, L.vdim, L.rank, L.count, L.scale, L.window, L.rotary, L.base, L.eps)
+    q, gate = L.q.clone(), L.proj[:, L.qc + L.rank + L.rot:]
+    y = torch.zeros((n, L.heads * L.vdim), device="cuda")
+    torch.cuda.synchronize()
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(graph, stream=stream):
+            op.encode(q, gate, L.uk, L.uv, L.cache, nv.row_map(0, 0), y, nv.LATENT_EXPANDED)
+    for _ in range(3):
+        q.copy_(L.q)                                 # the call rotates it in place
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.abs(y.double().cpu().numpy() - want).max() < 2e-5 * np.abs(want).max()
