@@ -36,34 +36,57 @@ def test_tiles(act, k, rows, n):
     assert bool((y[:, n:] == 7).all()) and bool((y32[:, n:] == 7).all())
 
 
-# 2048 rows x 8208: a full round of the largest tile and sixteen weight rows in a launch of their own
-@pytest.mark.parametrize("kind", ["plain", "erf", "bias", "pairs", "full"])
-def test_two_launches_with_every_epilogue(kind):
+def launches(call):
+    """How many launches a call makes, by the nodes of a graph that records it."""
+    import ctypes as C
+    graph, stream = torch.cuda.CUDAGraph(keep_graph=True), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(graph, stream=stream):
+            call()
+    n = C.c_size_t(0)
+    assert C.CDLL("libamdhip64.so").hipGraphGetNodes(C.c_void_p(graph.raw_cuda_graph()), None, C.byref(n)) == 0
+    return n.value
+
+
+def epilogue(kind, rows, n, want, table_rows=50):
+    """The arguments of one kind of epilogue, and float64 sums `want` taken through it."""
     import nvmai_amd as nv
-    say("dense in two launches", kind)
-    ctx = nv.Context(0, nv.ACT_BF16)
-    rows, n, k = 2048, 8208, 512
-    w, x = operands(rows, n, k, ctx.dtype, 11)
     gen = torch.Generator(device="cuda").manual_seed(12)
-    bias, mul = torch.randn(n, device="cuda", generator=gen).to(torch.bfloat16), torch.randn((50, n), device="cuda", generator=gen).to(torch.bfloat16)
-    ids = torch.randint(0, 52, (rows,), device="cuda", generator=gen, dtype=torch.int32)            # two of them past the table
-    want = x.double() @ w.double().T
+    bias, mul = torch.randn(n, device="cuda", generator=gen).to(torch.bfloat16), torch.randn((table_rows, n), device="cuda", generator=gen).to(torch.bfloat16)
+    ids = torch.randint(0, table_rows + 2, (rows,), device="cuda", generator=gen, dtype=torch.int32)      # two of them past the table
     gelu = torch.nn.functional.gelu
     if kind == "erf":
-        args, want = dict(activation=nv.LINEAR_GELU_ERF), gelu(want)
-    elif kind == "bias":
-        args, want = dict(bias=bias), want + bias.double()
-    elif kind == "pairs":
-        args, want = dict(activation=nv.LINEAR_SILU_PAIRS), torch.nn.functional.silu(want[:, ::2]) * want[:, 1::2]
-    elif kind == "full":
+        return dict(activation=nv.LINEAR_GELU_ERF), gelu(want)
+    if kind == "bias":
+        return dict(bias=bias), want + bias.double()
+    if kind == "pairs":
+        return dict(activation=nv.LINEAR_SILU_PAIRS), torch.nn.functional.silu(want[:, ::2]) * want[:, 1::2]
+    if kind == "full":
         table = torch.cat([mul.double(), torch.zeros((2, n), dtype=torch.float64, device="cuda")])
-        args, want = dict(bias=bias, activation=nv.LINEAR_GELU_TANH, mul=mul, mul_ids=ids), gelu(want + bias.double(), approximate="tanh") * table[ids.long()]
-    else:
-        args = {}
-    y32 = torch.full((rows, n), 7.0, device="cuda")
-    y32 = y32[:, :n // 2].contiguous() if kind == "pairs" else y32
-    nv.dense_linear(ctx, w, x, y_f32=y32, **args)
-    check(y32, want, 3e-6)              # the sum's 2e-6, and 1e-6 for a GELU by hardware exponentials
+        return dict(bias=bias, activation=nv.LINEAR_GELU_TANH, mul=mul, mul_ids=ids), gelu(want + bias.double(), approximate="tanh") * table[ids.long()]
+    return {}, want
+
+
+KINDS = ["plain", "erf", "bias", "pairs", "full"]
+
+
+# 2048 rows x 8208: full rounds of large tiles and sixteen weight rows in a launch of their own, from 576 k on; 32-bit rows make
+# their planes in a launch before that
+@pytest.mark.parametrize("act", ["bf16", "fp32"])
+@pytest.mark.parametrize("kind", KINDS)
+def test_two_launches_with_every_epilogue(kind, act):
+    import nvmai_amd as nv
+    say("dense in two launches", kind, act)
+    ctx = nv.Context(0, nv.ACT_FP32 if act == "fp32" else nv.ACT_BF16)
+    rows, n, k = 2048, 8208, 1024
+    w, x = operands(rows, n, k, ctx.dtype, 11)
+    args, want = epilogue(kind, rows, n, x.double() @ w.double().T)
+    y32 = torch.full((rows, want.shape[1]), 7.0, device="cuda")
+    call = lambda: nv.dense_linear(ctx, w, x, y_f32=y32, **args)
+    call()
+    check(y32, want, 3e-6)              # the sum's 2e-6, and 1e-6 for a GELU or SiLU by hardware exponentials
+    assert launches(call) == (3 if act == "fp32" else 2)
 
 
 # rows: a wave per weight row, the short products, the tiles; strides: four multipliers at once, one by one
@@ -191,3 +214,37 @@ def test_infinite_weights_meet_32_bit_rows(rows, n):
     assert torch.equal(y.isinf(), want.isinf()) and torch.equal(y[y.isinf()].double(), want[want.isinf()])
     finite = want.isfinite()
     assert int(finite.sum()) > (n - 4) * (rows - 1) and float((y.double() - want)[finite].abs().max()) < 1e24      # 1e30 among the inputs
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_captured_calls_without_workspace_with_every_epilogue(kind):
+    """The form without planes, recorded while there is no workspace, ragged at the edges of its tiles of 64."""
+    import nvmai_amd as nv
+    say("captured 32-bit product", kind)
+    rows, n, k = 100, 204, 320
+    w, x = operands(rows, n, k, torch.float32, 5)
+    args, want = epilogue(kind, rows, n, x.double() @ w.double().T)
+    warm, ctx = nv.Context(0, nv.ACT_FP32), nv.Context(0, nv.ACT_FP32)
+    y = torch.zeros(want.shape, device="cuda")
+    nv.dense_linear(warm, w, x, y_f32=y, **args)                      # loads the module
+    check(y, want, 3e-6)
+    torch.cuda.synchronize()
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(graph, stream=stream):
+            nv.dense_linear(ctx, w, x, y_f32=y, **args)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        check(y, want, 3e-6)
+
+
+@pytest.mark.parametrize("exponent", [-109, -111, -120, -126, -133, -149])
+def test_32_bit_values_below_the_planes_range(exponent):
+    """Exact down to 2^-110, within 2^-133 below it."""
+    import nvmai_amd as nv
+    x = ((torch.rand((70, 64), device="cuda", dtype=torch.float64, generator=torch.Generator(device="cuda").manual_seed(1)) + 1) * 2.0 ** exponent).float()
+    y = torch.empty((70, 64), device="cuda")
+    nv.dense_linear(nv.Context(0, nv.ACT_FP32), torch.eye(64, device="cuda", dtype=torch.bfloat16), x, y_f32=y)
+    assert float((y.double() - x.double()).abs().max()) <= (0.0 if exponent > -110 else 2.0 ** -133)
