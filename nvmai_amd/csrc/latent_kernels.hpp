@@ -713,6 +713,11 @@ __global__ __launch_bounds__(256, NP + RP + DV <= 320 ? 2 : 1) void latent_flash
         lds_landed_barrier();
         if (k0 + 64u < k_hi) issue(k0 + 64u, next);
         if (!wave_live || k0 >= w_hi || k0 + 64u <= w_lo) return;               // wave-uniform
+        // The largest size has no registers for the addresses of both stages' rows all through the loop and spilled fifteen: it makes
+        // them anew for every tile (8 heads of 384 / 256, 4096 queries: 285 us in one array, 283 now; 16 heads under a window of 1024: 213,
+        // 215 with the spills, 208 now).
+        uint32_t row = krow;
+        if (NP + RP + DV > 512) asm volatile("" : "+v"(row));
         la_f4 s[2][4];
 #pragma unroll
         for (int b = 0; b < 2; ++b)
@@ -723,7 +728,7 @@ __global__ __launch_bounds__(256, NP + RP + DV <= 320 ? 2 : 1) void latent_flash
             uint4 a[4];
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                const uint32_t key = 32u * (t >> 1) + 4u * (t & 1) + krow;
+                const uint32_t key = 32u * (t >> 1) + 4u * (t & 1) + row;
                 a[t] = st < KN ? *reinterpret_cast<const uint4*>(cur + key * (NP * 2u) + ((4u * st + g) ^ la_swizzle<NP / 8>(key)) * 16u)
                                : *reinterpret_cast<const uint4*>(cur + AT_R + key * (RP * 2u) + ((4u * (st - KN) + g) ^ la_swizzle<RP / 8>(key)) * 16u);
             }
