@@ -350,14 +350,16 @@ __device__ __forceinline__ float dense_sum_again(const DenseLinearParams& p, uin
     return total;
 }
 
-// Of 160 KB; two blocks per compute unit where the tile is small.  Planes come in threes: six stages where they fit (64 x 64, 700 x
-// 1024 x 1024 in 32 bits: 17.4 us with three, 13.5 with six).
+// Of 160 KB, one block per compute unit; 64 x 64 tiles of 16-bit inputs fit twice.  Planes come in threes: six stages where they fit
+// (64 x 64, 700 x 1024 x 1024 in 32 bits: 17.4 us with three, 13.5 with six).
 constexpr int dense_stages(int act, int bn, int bm) {
     return act == ACT_FP32 ? (bn + bm <= 192 ? 6 : 3) : bn + bm <= 192 ? 5 : bn + bm <= 256 ? 4 : bn + bm <= 384 ? 3 : 2;
 }
 
+constexpr int dense_blocks(int act, int bn, int bm) { return 2 * dense_stages(act, bn, bm) * (bn + bm) * 128 <= 160 * 1024 ? 2 : 1; }
+
 template <int EPI, int ACT, int BN, int BM>
-__global__ __launch_bounds__(256, BN + BM <= 128 ? 2 : 1) void dense_tile_kernel(DenseLinearParams p, uint32_t tiles_n, uint32_t tiles_m) {
+__global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_kernel(DenseLinearParams p, uint32_t tiles_n, uint32_t tiles_m) {
     constexpr bool SPLIT = ACT == ACT_FP32;
     constexpr int S = dense_stages(ACT, BN, BM);
     constexpr int LA = BN / 32, LB = BM / 32, L = LA + LB;   // 1 KB requests per wave and stage
