@@ -570,7 +570,7 @@ __global__ __launch_bounds__(256) void latent_expanded_plain_kernel(LatentAttnPa
 }
 
 // ---- expanded, 32 bits: 16 queries of one head per block (flash32.hpp) --------------------------------------
-// 700 rows, 8 heads of 192 / 128: 279 -> 38 us (a block per row and head, keys one by one on the vector pipe, before).
+// 700 rows, 8 heads of 192 / 128: 279 -> 40 us (a block per row and head, keys one by one on the vector pipe, before).
 template <int NP, int RP, int DV>
 __global__ __launch_bounds__(256, 2) void latent_flash32_kernel(LatentAttnParams p) {
     constexpr int KN = NP / 16, KR = RP / 16, NV = DV / 16;
@@ -623,7 +623,7 @@ __global__ __launch_bounds__(256, 2) void latent_flash32_kernel(LatentAttnParams
 // fall into different banks.  NP, RP: the two parts of a key, DV: value dims, padded with zeros (a lane whose column
 // does not exist loads from past the end of the buffer, which reads as zero).
 // The two stages are arrays of their own and the loop is written out for both: from halves of one array the compiler cannot
-// tell that a read of this tile does not touch the tile on its way, and waits for it before the first product (139 -> 114 us,
+// tell that a read of this tile does not touch the tile on its way, and waits for it before the first product (139 -> 121 us,
 // 2048 queries behind 2048 tokens, 16 heads of 192 / 128).
 template <int W>                         // row width in pieces
 __device__ __forceinline__ uint32_t la_swizzle(uint32_t key) {
