@@ -334,20 +334,33 @@ __device__ __forceinline__ void dense_stage_barrier() {
 #endif
 }
 
-// One sum of the planes again, in fp32 multiply-adds of the values that the planes stand for.  An infinite weight makes NaN of a
-// value's lower planes where they are zero, and planes of sums that overflow can cancel: a NaN comes from here or not at all.
-__device__ __forceinline__ float dense_sum_again(const DenseLinearParams& p, uint32_t t, uint32_t r) {
+// One sum of the planes again by a whole wave, in fp32 multiply-adds of the values that the planes stand for.  An infinite weight makes
+// NaN of a value's lower planes where they are zero, and planes of sums that overflow can cancel: a NaN comes from here or not
+// at all.  It ends where the sum has become NaN, which it stays; poisoned: by an input that is NaN, so that all sums of its row are.
+__device__ __forceinline__ float dense_sum_again(const DenseLinearParams& p, uint32_t t, uint32_t r, bool& poisoned) {
     const uint16_t *w = p.w + (size_t)r * p.w_stride, *x = static_cast<const uint16_t*>(p.x) + (size_t)t * p.x_stride;
-    float total = 0.0f;
+    const uint32_t lane = threadIdx.x & 63u;
+    float sum = 0.0f;
+    bool none = false;
 #pragma unroll 1
-    for (uint32_t k0 = 0; k0 < p.k; k0 += 64u) {
-        float sum = 0.0f;
-#pragma unroll 1
-        for (uint32_t k = k0; k < k0 + 64u; ++k)
-            sum = fmaf(bf16_to_f32(w[k]), (bf16_to_f32(x[2u * p.k + k]) + bf16_to_f32(x[p.k + k])) + bf16_to_f32(x[k]), sum);
-        total += sum;
+    for (uint32_t k0 = 0; k0 < p.k; k0 += 512u) {
+        const uint32_t k = k0 + lane * 8u;
+        if (k < p.k) {
+            const uint4 a = *reinterpret_cast<const uint4*>(w + k), lo = *reinterpret_cast<const uint4*>(x + k),
+                        mid = *reinterpret_cast<const uint4*>(x + p.k + k), hi = *reinterpret_cast<const uint4*>(x + 2u * p.k + k);
+            const uint32_t av[4] = {a.x, a.y, a.z, a.w}, lv[4] = {lo.x, lo.y, lo.z, lo.w}, mv[4] = {mid.x, mid.y, mid.z, mid.w}, hv[4] = {hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                auto part = [&](const uint32_t* v) { return bf16_to_f32((uint16_t)(v[e / 2] >> (16 * (e & 1)))); };
+                const float value = (part(hv) + part(mv)) + part(lv);
+                none |= value != value;
+                sum = fmaf(part(av), value, sum);
+            }
+        }
+        if (__any(sum != sum)) break;
     }
-    return total;
+    poisoned = __any(none);
+    return wave_sum_bcast(sum);
 }
 
 // Of 160 KB, one block per compute unit; 64 x 64 tiles of 16-bit inputs fit twice.  Planes come in threes: six stages where they fit
@@ -501,10 +514,18 @@ __global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_ker
         }
         if constexpr (SPLIT) {
             if (__any(again)) {
-                for (uint32_t e = lane; e < 32u * ROWS; e += 64u) {
-                    const uint32_t t = m0 + wm + 32 * b + e / ROWS, row = n0 + wn + e % ROWS;
-                    float& sum = turn[e / ROWS * PITCH + e % ROWS];
-                    if (sum != sum && t < p.rows && row < p.n) sum = dense_sum_again(p, t, row);
+                uint32_t poisoned_token = 32;                // sums of one token follow each other
+                for (uint32_t e0 = 0; e0 < 32u * ROWS; e0 += 64u) {
+                    const uint32_t own = e0 + lane;
+                    const float old = turn[own / ROWS * PITCH + own % ROWS];
+                    for (uint64_t left = __ballot(old != old); left != 0; left &= left - 1) {
+                        const uint32_t e = e0 + (uint32_t)__builtin_ctzll(left), token = e / ROWS, t = m0 + wm + 32 * b + token, row = n0 + wn + e % ROWS;
+                        if (token == poisoned_token || t >= p.rows || row >= p.n) continue;
+                        bool poisoned;
+                        const float sum = dense_sum_again(p, t, row, poisoned);
+                        if (poisoned) poisoned_token = token;
+                        else if (lane == 0) turn[token * PITCH + e % ROWS] = sum;
+                    }
                 }
             }
         }

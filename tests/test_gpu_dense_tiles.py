@@ -248,3 +248,23 @@ def test_32_bit_values_below_the_planes_range(exponent):
     y = torch.empty((70, 64), device="cuda")
     nv.dense_linear(nv.Context(0, nv.ACT_FP32), torch.eye(64, device="cuda", dtype=torch.bfloat16), x, y_f32=y)
     assert float((y.double() - x.double()).abs().max()) <= (0.0 if exponent > -110 else 2.0 ** -133)
+
+
+@pytest.mark.parametrize("rows,n,k", [(70, 70, 64), (300, 260, 1088), (2048, 2100, 576)])
+def test_32_bit_rows_that_are_not_numbers(rows, n, k):
+    """A NaN makes NaN of its own row, whatever weights it meets; the other rows are what they were."""
+    import nvmai_amd as nv
+    say("32-bit rows that are not numbers", rows, n, k)
+    ctx = nv.Context(0, nv.ACT_FP32)
+    w, x = operands(rows, n, k, torch.float32, 13)
+    clean = nv.dense_linear(ctx, w, x, y_f32=torch.empty((rows, n), device="cuda")).clone()
+    bad = sorted({0, 5, 31, 32, rows // 2, rows - 1})
+    for j, t in enumerate(bad):
+        x[t, (j * 97 + k - 1) % k] = float("nan")
+    w[n - 1, 3], w[1, k - 1] = float("inf"), float("-inf")
+    y = nv.dense_linear(ctx, w, x, y_f32=torch.empty((rows, n), device="cuda"))
+    fine = torch.ones(rows, dtype=torch.bool, device="cuda")
+    fine[bad] = False
+    assert bool(y[~fine].isnan().all())
+    assert torch.equal(y[fine][:, 2:n - 1], clean[fine][:, 2:n - 1])
+    assert torch.equal(y[fine, n - 1], torch.sign(x[fine, 3]) * float("inf")) and torch.equal(y[fine, 1], torch.sign(x[fine, k - 1]) * float("-inf"))
