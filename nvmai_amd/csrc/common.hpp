@@ -222,6 +222,20 @@ __device__ __forceinline__ void lds_landed_barrier() {
     __syncthreads();
 }
 
+// How the flash attention of prompts (latent_flash_kernel, window_flash_kernel) takes a call's queries.  Four waves of 32 queries
+// (WHOLE) leave one wave on a SIMD until there are two blocks per compute unit, and its products and its softmax then wait
+// for each other.  Up to one such block per unit, eight waves per block share the keys (HALVES), and where that leaves units without work
+// until the longest block ends, or where the stages of two blocks fit the 160 KB of a unit (lds: bytes of one), blocks of 64 queries
+// (HALVES16, sixteen per wave) do.  Measured, WHOLE / HALVES / HALVES16, 16 heads: windowed 128 / 128 and capped 1000 queries 30 / 26 / 17 us, 1501 43 / 36 / 34,
+// 2048 60 / 51 / 57, 2048 behind 2048 116 / 94 / 116, 4096 at once 124 / 155 / 155, 8 heads 64 / 52 / 37 at 2048; 64 / 64, 2048 45 / 38 / 27; latent 192 / 128
+// 1000 33 / 29 / 20, 1501 48 / 40 / 37, 2048 64 / 53 / 59, 2048 behind 2048 126 / 100 / 125, 4096 at once 135 / 165 / 170.
+enum class FlashForm { WHOLE, HALVES, HALVES16 };
+
+inline FlashForm flash_form(uint32_t rows, uint32_t heads, uint32_t cus, uint32_t lds) {
+    if ((uint64_t)((rows + 127) / 128) * heads > cus) return FlashForm::WHOLE;
+    return 2 * lds <= 160 * 1024 || (uint64_t)((rows + 63) / 64) * heads * 4 <= (uint64_t)cus * 7 ? FlashForm::HALVES16 : FlashForm::HALVES;
+}
+
 __device__ __forceinline__ float silu(float v) { return v / (1.0f + expf(-v)); }
 
 // silu through the hardware exp2 and reciprocal (about 1e-6 relative): for kernels

@@ -61,14 +61,29 @@ int absorbed(const LatentAttnParams& p, hipStream_t s) {
 }
 
 template <int NP, int RP, int DV>
-int launch_flash(const LatentAttnParams& p, hipStream_t s) {
-    latent_flash_kernel<NP, RP, DV><<<(p.n_rows + 127) / 128 * p.heads, 256, 0, s>>>(p);
+int launch_flash(const LatentAttnParams& p, uint32_t cus, hipStream_t s) {
+    const uint32_t blocks = (p.n_rows + 127) / 128 * p.heads;
+    if constexpr (NP + RP + DV <= 320) {                     // the stages of both halves fit
+        constexpr uint32_t LDS = 4 * 128 * (NP + RP + DV);
+        const FlashForm form = flash_form(p.n_rows, p.heads, cus, LDS);
+        if (form == FlashForm::HALVES16) {
+            latent_flash_halves_kernel<NP, RP, DV, 1><<<(p.n_rows + 63) / 64 * p.heads, 512, 0, s>>>(p);
+            return launch_status();
+        }
+        if constexpr (2 * LDS > 160 * 1024) {
+            if (form == FlashForm::HALVES) {
+                latent_flash_halves_kernel<NP, RP, DV, 2><<<blocks, 512, 0, s>>>(p);
+                return launch_status();
+            }
+        }
+    }
+    latent_flash_kernel<NP, RP, DV><<<blocks, 256, 0, s>>>(p);
     return launch_status();
 }
 
 template <int NP, int RP>
-int launch_flash_v(const LatentAttnParams& p, hipStream_t s) {
-    return p.vdim <= 64 ? launch_flash<NP, RP, 64>(p, s) : launch_flash<NP, RP, 128>(p, s);
+int launch_flash_v(const LatentAttnParams& p, uint32_t cus, hipStream_t s) {
+    return p.vdim <= 64 ? launch_flash<NP, RP, 64>(p, cus, s) : launch_flash<NP, RP, 128>(p, cus, s);
 }
 
 }  // namespace
@@ -209,7 +224,8 @@ extern "C" int nvmai_hip_latent_attention(nvmai_hip_ctx* ctx, nvmai_stream strea
         }
         return launch_status();
     }
-    if (c.nope_dim > 128 || c.rope_dim > 64 || c.value_dim > 128) return launch_flash<256, 128, 256>(p, s);
-    if (c.nope_dim <= 64) return c.rope_dim <= 32 ? launch_flash_v<64, 32>(p, s) : launch_flash_v<64, 64>(p, s);
-    return c.rope_dim <= 32 ? launch_flash_v<128, 32>(p, s) : launch_flash_v<128, 64>(p, s);
+    const uint32_t cus = (uint32_t)ctx->compute_units;
+    if (c.nope_dim > 128 || c.rope_dim > 64 || c.value_dim > 128) return launch_flash<256, 128, 256>(p, cus, s);
+    if (c.nope_dim <= 64) return c.rope_dim <= 32 ? launch_flash_v<64, 32>(p, cus, s) : launch_flash_v<64, 64>(p, cus, s);
+    return c.rope_dim <= 32 ? launch_flash_v<128, 32>(p, cus, s) : launch_flash_v<128, 64>(p, cus, s);
 }

@@ -614,7 +614,7 @@ __global__ __launch_bounds__(256, 2) void latent_flash32_kernel(LatentAttnParams
 }
 
 // ---- expanded: flash attention over a window, BF16 -------------------------------------------------------
-// 128 queries of one head per block, 32 per wave; K rows (in two regions, the head's own part and the shared rotated
+// 64 QB queries of one head per block, 16 QB per wave (flash_form says which form when); K rows (in two regions, the head's own part and the shared rotated
 // part) and V^T rows in tiles of 64 keys, loaded straight into LDS, the next tile under the current tile's products.
 // S^T[key, query] = K Q^T and O^T[value, query] += V^T P^T.  Row m of score tile 2 h (2 h + 1) is key
 // 32 h + 8 (m / 4) + m % 4 (+ 4): a lane's registers of the two tiles are then the keys 8 g .. 8 g + 7, in order, and
@@ -632,25 +632,26 @@ __device__ __forceinline__ uint32_t la_swizzle(uint32_t key) {
 
 constexpr uint32_t LA_OUT_OF_BOUNDS = 0x80000000u;
 
-template <int NP, int RP, int DV>
-__global__ __launch_bounds__(256, NP + RP + DV <= 320 ? 2 : 1) void latent_flash_kernel(LatentAttnParams p) {
+template <int NP, int RP, int DV, int GROUPS, int QB>
+__device__ __forceinline__ void latent_flash_body(const LatentAttnParams& p) {
     constexpr int KN = NP / 32, KR = RP / 32, NV = DV / 16;
     constexpr int LN = NP / 32, LR = RP / 32, LV = DV / 32;      // 1 KB loads per wave and tile
     constexpr uint32_t AT_R = 64u * NP * 2u, AT_V = AT_R + 64u * RP * 2u, STAGE = AT_V + DV * 128u;
-    __shared__ __attribute__((aligned(1024))) uint8_t even[STAGE], odd[STAGE];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 15u, g = lane >> 4;
+    __shared__ __attribute__((aligned(1024))) uint8_t even[GROUPS * STAGE], odd[GROUPS * STAGE];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, i = lane & 15u, g = lane >> 4;
+    const uint32_t nth_wave = __builtin_amdgcn_readfirstlane(tid >> 6), wave = nth_wave & 3u, group = GROUPS > 1 ? nth_wave >> 2 : 0u;
     // Blocks are dealt to the eight XCDs in turn: an XCD keeps to its own heads (their keys stay in its L2) where
     // the heads divide.  Even rounds take the query blocks with the most keys first, odd ones last: a compute unit's
     // two blocks then add up to the same work.
-    const uint32_t nqb = (p.n_rows + 127u) / 128u, id = blockIdx.x;
+    const uint32_t nqb = (p.n_rows + 64u * QB - 1u) / (64u * QB), id = blockIdx.x;
     const uint32_t nth = p.heads % 8u == 0u ? id / 8u : id, round = nth / nqb, in_round = nth % nqb;
     const uint32_t head = p.heads % 8u == 0u ? round * 8u + id % 8u : round, qb = round & 1u ? in_round : nqb - 1u - in_round;
-    const uint32_t q0 = qb * 128u, dq = p.nope + p.rot;
+    const uint32_t q0 = qb * (64u * QB), dq = p.nope + p.rot;
     const uint16_t* q = static_cast<const uint16_t*>(p.q) + head * dq;
-    uint4 qf[2][KN + KR];
+    uint4 qf[QB][KN + KR];
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-        const uint16_t* qr = q + (size_t)min(q0 + wave * 32u + 16u * b + i, p.n_rows - 1u) * p.q_stride;
+    for (int b = 0; b < QB; ++b) {
+        const uint16_t* qr = q + (size_t)min(q0 + wave * (16u * QB) + 16u * b + i, p.n_rows - 1u) * p.q_stride;
 #pragma unroll
         for (int s = 0; s < KN + KR; ++s) {
             const uint32_t d = s < KN ? 32u * s + 8u * g : 32u * (s - KN) + 8u * g, n = s < KN ? p.nope : p.rot;
@@ -658,14 +659,17 @@ __global__ __launch_bounds__(256, NP + RP + DV <= 320 ? 2 : 1) void latent_flash
             qf[b][s] = d < n ? v : make_uint4(0u, 0u, 0u, 0u);
         }
     }
-    la_f4 acc[2][NV];
-    float m[2] = {LA_NONE, LA_NONE}, l[2] = {0.0f, 0.0f};
+    la_f4 acc[QB][NV];
+    float m[QB], l[QB];
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < QB; ++b) {
+        m[b] = LA_NONE;
+        l[b] = 0.0f;
 #pragma unroll
         for (int n = 0; n < NV; ++n) acc[b][n] = la_f4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
     // keys are numbered from key0
-    const uint32_t last_t = min(q0 + 127u, p.n_rows - 1u);
+    const uint32_t last_t = min(q0 + 64u * QB - 1u, p.n_rows - 1u);
     const uint32_t k_lo = (first_key(p.rows.position + q0, p.window) - p.key0) & ~63u;
     const uint32_t k_hi = p.rows.position + last_t + 1u - p.key0;
     const uint32_t kn_bytes = p.kn_stride * 2u, lat_bytes = p.cache.row_stride * 2u, v_bytes = p.v_stride * 2u;
@@ -702,7 +706,7 @@ __global__ __launch_bounds__(256, NP + RP + DV <= 320 ? 2 : 1) void latent_flash
 #endif
     };
     // this wave's own range of keys, and the part of it that every one of its queries sees
-    const uint32_t wt0 = q0 + wave * 32u, wt1 = min(wt0 + 31u, p.n_rows - 1u);
+    const uint32_t wt0 = q0 + wave * (16u * QB), wt1 = min(wt0 + 16u * QB - 1u, p.n_rows - 1u);
     const bool wave_live = wt0 < p.n_rows;
     const uint32_t w_lo = first_key(p.rows.position + wt0, p.window) - p.key0, w_hi = p.rows.position + wt1 + 1u - p.key0;
     const uint32_t full_lo = first_key(p.rows.position + wt1, p.window) - p.key0, full_hi = p.rows.position + wt0 + 1u - p.key0;
@@ -711,16 +715,16 @@ __global__ __launch_bounds__(256, NP + RP + DV <= 320 ? 2 : 1) void latent_flash
         // This tile has landed and everyone is done with the other stage.  The wait stands here by name: a workgroup's barrier
         // does not wait for loads into LDS, and a wave that skips a tile waits for its part of it all the same.
         lds_landed_barrier();
-        if (k0 + 64u < k_hi) issue(k0 + 64u, next);
+        if (k0 + 64u * GROUPS < k_hi) issue(k0 + 64u * GROUPS, next);
         if (!wave_live || k0 >= w_hi || k0 + 64u <= w_lo) return;               // wave-uniform
         // The largest size has no registers for the addresses of both stages' rows all through the loop and spilled fifteen: it makes
         // them anew for every tile (8 heads of 384 / 256, 4096 queries: 285 us in one array, 283 now; 16 heads under a window of 1024: 213,
         // 215 with the spills, 208 now).
         uint32_t row = krow;
         if (NP + RP + DV > 512) asm volatile("" : "+v"(row));
-        la_f4 s[2][4];
+        la_f4 s[QB][4];
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
+        for (int b = 0; b < QB; ++b)
 #pragma unroll
             for (int t = 0; t < 4; ++t) s[b][t] = la_f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -735,12 +739,12 @@ __global__ __launch_bounds__(256, NP + RP + DV <= 320 ? 2 : 1) void latent_flash
 #pragma unroll
             for (int t = 0; t < 4; ++t)
 #pragma unroll
-                for (int b = 0; b < 2; ++b) s[b][t] = la_mfma(a[t], qf[b][st], s[b][t]);
+                for (int b = 0; b < QB; ++b) s[b][t] = la_mfma(a[t], qf[b][st], s[b][t]);
         }
         const bool masked = k0 < full_lo || k0 + 64u > full_hi;
-        uint4 pf[2][2];
+        uint4 pf[QB][2];
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
+        for (int b = 0; b < QB; ++b) {
 #pragma unroll
             for (int t = 0; t < 4; ++t) s[b][t] *= p.scale_log2;
             if (masked) {
@@ -786,17 +790,44 @@ __global__ __launch_bounds__(256, NP + RP + DV <= 320 ? 2 : 1) void latent_flash
             for (int n = 0; n < NV; ++n) {
                 const uint4 a = *reinterpret_cast<const uint4*>(cur + AT_V + (16u * n + i) * 128u + ((4u * h + g) ^ (i & 7u)) * 16u);
 #pragma unroll
-                for (int b = 0; b < 2; ++b) acc[b][n] = la_mfma(a, pf[b][h], acc[b][n]);
+                for (int b = 0; b < QB; ++b) acc[b][n] = la_mfma(a, pf[b][h], acc[b][n]);
             }
     };
-    issue(k_lo, even);
-    for (uint32_t k0 = k_lo; k0 < k_hi; k0 += 128u) {
-        tile(k0, even, odd);
-        if (k0 + 64u < k_hi) tile(k0 + 64u, odd, even);
+    uint8_t *const here = even + group * STAGE, *const there = odd + group * STAGE;
+    const uint32_t own = 64u * group;
+    if (k_lo + own < k_hi) issue(k_lo + own, here);
+    for (uint32_t k0 = k_lo; k0 < k_hi; k0 += 128u * GROUPS) {
+        tile(k0 + own, here, there);
+        if (k0 + 64u * GROUPS < k_hi) tile(k0 + 64u * GROUPS + own, there, here);
+    }
+    if constexpr (GROUPS > 1) {
+        // the second group's sums go to the first one through LDS, sixteen queries of a wave at a time
+        static_assert(GROUPS == 2 && 4u * NV * 1024u <= GROUPS * STAGE, "one array holds the sums, the other the rest");
+        la_f4* sums = reinterpret_cast<la_f4*>(even) + wave * (NV * 64u) + lane;
+        float* rest = reinterpret_cast<float*>(odd) + wave * 128u + lane;
+#pragma unroll
+        for (int b = 0; b < QB; ++b) {
+            lds_landed_barrier();
+            if (group == 1u) {
+#pragma unroll
+                for (int n = 0; n < NV; ++n) sums[n * 64] = acc[b][n];
+                rest[0] = m[b];
+                rest[64] = l[b];
+            }
+            lds_landed_barrier();
+            if (group == 0u) {
+                // both groups without a key so far: weights of 1 for sums of 0
+                const float m1 = rest[0], mn = fmaxf(m[b], m1), f0 = __builtin_amdgcn_exp2f(m[b] - mn), f1 = __builtin_amdgcn_exp2f(m1 - mn);
+                l[b] = l[b] * f0 + rest[64] * f1;
+#pragma unroll
+                for (int n = 0; n < NV; ++n) acc[b][n] = acc[b][n] * f0 + sums[n * 64] * f1;
+            }
+        }
+        if (group == 1u) return;
     }
     if (!wave_live) return;
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
+    for (int b = 0; b < QB; ++b) {
         float sum = l[b];
         sum += shfl_xor_f(sum, 16);
         sum += shfl_xor_f(sum, 32);
@@ -811,6 +842,18 @@ __global__ __launch_bounds__(256, NP + RP + DV <= 320 ? 2 : 1) void latent_flash
             if (d < p.vdim) *reinterpret_cast<uint2*>(out + d) = make_uint2(la_pack2(acc[b][n][0] * f, acc[b][n][1] * f), la_pack2(acc[b][n][2] * f, acc[b][n][3] * f));
         }
     }
+}
+
+template <int NP, int RP, int DV>
+__global__ __launch_bounds__(256, NP + RP + DV <= 320 ? 2 : 1) void latent_flash_kernel(LatentAttnParams p) {
+    latent_flash_body<NP, RP, DV, 1, 2>(p);
+}
+
+// Blocks of eight waves: two groups of four share a block's keys, a tile each at a time, and bring their sums together at the end.
+// Bound by products and softmax of the waves on a SIMD (a tile of a wave: 0.53 us and 0.5).
+template <int NP, int RP, int DV, int QB>
+__global__ __launch_bounds__(512, 1) void latent_flash_halves_kernel(LatentAttnParams p) {
+    latent_flash_body<NP, RP, DV, 2, QB>(p);
 }
 
 }  // namespace nvmai

@@ -44,14 +44,29 @@ void epilogue(const WindowEpilogueParams& p, hipStream_t s) {
 }
 
 template <int DK, int DV, bool BOUND>
-int launch_flash_as(const WindowParams& p, hipStream_t s) {
-    window_flash_kernel<DK, DV, BOUND><<<(p.n_rows + 127) / 128 * p.heads, 256, 0, s>>>(p);
+int launch_flash_as(const WindowParams& p, uint32_t cus, hipStream_t s) {
+    const uint32_t blocks = (p.n_rows + 127) / 128 * p.heads;
+    if constexpr (DK + DV <= 256) {                          // the stages of both halves fit
+        constexpr uint32_t LDS = 4 * 128 * (DK + DV);
+        const FlashForm form = flash_form(p.n_rows, p.heads, cus, LDS);
+        if (form == FlashForm::HALVES16) {
+            window_flash_halves_kernel<DK, DV, BOUND, 1><<<(p.n_rows + 63) / 64 * p.heads, 512, 0, s>>>(p);
+            return launch_status();
+        }
+        if constexpr (2 * LDS > 160 * 1024) {
+            if (form == FlashForm::HALVES) {
+                window_flash_halves_kernel<DK, DV, BOUND, 2><<<blocks, 512, 0, s>>>(p);
+                return launch_status();
+            }
+        }
+    }
+    window_flash_kernel<DK, DV, BOUND><<<blocks, 256, 0, s>>>(p);
     return launch_status();
 }
 
 template <int DK, int DV>
-int launch_flash(const WindowParams& p, hipStream_t s) {
-    return p.capped && !p.alibi && p.b <= WA_BOUND ? launch_flash_as<DK, DV, true>(p, s) : launch_flash_as<DK, DV, false>(p, s);
+int launch_flash(const WindowParams& p, uint32_t cus, hipStream_t s) {
+    return p.capped && !p.alibi && p.b <= WA_BOUND ? launch_flash_as<DK, DV, true>(p, cus, s) : launch_flash_as<DK, DV, false>(p, cus, s);
 }
 
 template <int ACT, int CT>
@@ -122,9 +137,9 @@ extern "C" int nvmai_hip_window_attention(nvmai_hip_ctx* ctx, nvmai_stream strea
         return f32 ? plain<ACT_FP32, ACT_BF16>(p, s) : plain<ACT_BF16, ACT_BF16>(p, s);
     }
     if (form == NVMAI_WINDOW_FLASH) {
-        if (dk > 128 || dv > 128) return launch_flash<256, 256>(p, s);
-        if (dk <= 64) return dv <= 64 ? launch_flash<64, 64>(p, s) : launch_flash<64, 128>(p, s);
-        return dv <= 64 ? launch_flash<128, 64>(p, s) : launch_flash<128, 128>(p, s);
+        if (dk > 128 || dv > 128) return launch_flash<256, 256>(p, (uint32_t)ctx->compute_units, s);
+        if (dk <= 64) return dv <= 64 ? launch_flash<64, 64>(p, (uint32_t)ctx->compute_units, s) : launch_flash<64, 128>(p, (uint32_t)ctx->compute_units, s);
+        return dv <= 64 ? launch_flash<128, 64>(p, (uint32_t)ctx->compute_units, s) : launch_flash<128, 128>(p, (uint32_t)ctx->compute_units, s);
     }
     // tiles of 32 positions that a row can look at
     const uint32_t last = known ? map->position + rows - 1 : max_position;

@@ -12,7 +12,7 @@
 // Values are stored transposed: 16 bytes of a row are eight positions of one channel, an A operand of the second product
 // as they lie.
 //   * split: decoding and short portions, sixteen heads of one kv head per block, waves and blocks share the tiles;
-//   * flash: prompts, 128 queries of one head per block, tiles of 64 keys through LDS;
+//   * flash: prompts, 64 or 128 queries of one head per block, tiles of 64 keys through LDS;
 //   * plain: any sizes and types, a thread per key.
 #pragma once
 
@@ -433,7 +433,7 @@ __global__ __launch_bounds__(256, 2) void window_flash32_kernel(WindowParams p) 
 }
 
 // ---- flash form ------------------------------------------------------------------------------------------
-// 128 queries of one head per block, 32 per wave; K and V^T tiles of 64 keys, loaded straight into LDS, the next tile
+// 64 QB queries of one head per block, 16 QB per wave (flash_form says which form when); K and V^T tiles of 64 keys, loaded straight into LDS, the next tile
 // under the current tile's products.  S^T[key, query] = K Q^T, O^T[value, query] += V^T P^T, with the order of keys of the split
 // form.  LDS pieces of 16 bytes are exchanged within a row so that the lanes a read serves at once fall into different
 // banks.  DK, DV: sizes padded with zeros (a lane whose column does not exist loads from past the end of the
@@ -449,26 +449,27 @@ __device__ __forceinline__ uint32_t wa_swizzle(uint32_t key) {
 constexpr uint32_t WA_OUT_OF_BOUNDS = 0x80000000u;
 constexpr float WA_BOUND = 80.0f;
 
-template <int DK, int DV, bool BOUND>
-__global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void window_flash_kernel(WindowParams p) {
+template <int DK, int DV, bool BOUND, int GROUPS, int QB>
+__device__ __forceinline__ void window_flash_body(const WindowParams& p) {
     constexpr int KS = DK / 32, VS = DV / 16;
     constexpr int LK = DK / 32, LV = DV / 32;        // 1 KB loads per wave and tile
     constexpr uint32_t AT_V = 64u * DK * 2u, STAGE = AT_V + DV * 128u;
-    __shared__ __attribute__((aligned(1024))) uint8_t even[STAGE], odd[STAGE];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 15u, g = lane >> 4;
+    __shared__ __attribute__((aligned(1024))) uint8_t even[GROUPS * STAGE], odd[GROUPS * STAGE];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, i = lane & 15u, g = lane >> 4;
+    const uint32_t nth_wave = __builtin_amdgcn_readfirstlane(tid >> 6), wave = nth_wave & 3u, group = GROUPS > 1 ? nth_wave >> 2 : 0u;
     // Blocks are dealt to the eight XCDs in turn: an XCD keeps to its own heads (their keys stay in its L2) where
     // the heads divide.  Even rounds take the query blocks with the most keys first, odd ones last: a compute unit's
     // two blocks then add up to the same work.
-    const uint32_t nqb = (p.n_rows + 127u) / 128u, id = blockIdx.x;
+    const uint32_t nqb = (p.n_rows + 64u * QB - 1u) / (64u * QB), id = blockIdx.x;
     const uint32_t nth = p.heads % 8u == 0u ? id / 8u : id, round = nth / nqb, in_round = nth % nqb;
     // neighbouring heads (which share a kv head) on one XCD
     const uint32_t head = p.heads % 8u == 0u ? (id % 8u) * (p.heads / 8u) + round : round, qb = round & 1u ? in_round : nqb - 1u - in_round;
-    const uint32_t q0 = qb * 128u, dk = p.cache.dk, dv = p.cache.dv, total = p.cache.rows(), start = p.rows.position;
+    const uint32_t q0 = qb * (64u * QB), dk = p.cache.dk, dv = p.cache.dv, total = p.cache.rows(), start = p.rows.position;
     const uint16_t* q = static_cast<const uint16_t*>(p.q) + head * dk;
-    uint4 qf[2][KS];
+    uint4 qf[QB][KS];
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-        const uint16_t* qr = q + (size_t)min(q0 + wave * 32u + 16u * b + i, p.n_rows - 1u) * p.q_stride;
+    for (int b = 0; b < QB; ++b) {
+        const uint16_t* qr = q + (size_t)min(q0 + wave * (16u * QB) + 16u * b + i, p.n_rows - 1u) * p.q_stride;
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
             const uint32_t d = 32u * s + 8u * g;
@@ -476,13 +477,16 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void window_flash_kern
             qf[b][s] = d < dk ? v : make_uint4(0u, 0u, 0u, 0u);
         }
     }
-    wa_f4 acc[2][VS];
-    float m[2] = {WA_NONE, WA_NONE}, l[2] = {0.0f, 0.0f};
+    wa_f4 acc[QB][VS];
+    float m[QB], l[QB];
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < QB; ++b) {
+        m[b] = WA_NONE;
+        l[b] = 0.0f;
 #pragma unroll
         for (int n = 0; n < VS; ++n) acc[b][n] = wa_f4{0.0f, 0.0f, 0.0f, 0.0f};
-    const uint32_t last = start + min(q0 + 127u, p.n_rows - 1u);
+    }
+    const uint32_t last = start + min(q0 + 64u * QB - 1u, p.n_rows - 1u);
     // tiles of 64 positions: the kept ones, then from the window's first one to the last query's
     const uint32_t first_t = first_key(start + q0, p.window) / 64u, kept = min((p.keep + 63u) / 64u, first_t), count = kept + last / 64u - first_t + 1u;
     const size_t own = (size_t)p.rows.slot * p.cache.kv_heads + head / (p.heads / p.cache.kv_heads);
@@ -514,7 +518,7 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void window_flash_kern
 #endif
     };
     // this wave's queries, the keys some of them see beside the kept ones, and those that all of them see
-    const uint32_t wt0 = q0 + wave * 32u, wt1 = min(wt0 + 31u, p.n_rows - 1u);
+    const uint32_t wt0 = q0 + wave * (16u * QB), wt1 = min(wt0 + 16u * QB - 1u, p.n_rows - 1u);
     const bool wave_live = wt0 < p.n_rows;
     const uint32_t w_lo = first_key(start + wt0, p.window), w_hi = start + wt1 + 1u;
     const uint32_t full_lo = first_key(start + wt1, p.window), full_hi = start + wt0 + 1u;
@@ -524,12 +528,12 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void window_flash_kern
         // This tile has landed and everyone is done with the other stage.  The wait stands here by name: a workgroup's barrier
         // does not wait for loads into LDS, and a wave that skips a tile waits for its part of it all the same.
         lds_landed_barrier();
-        if (n + 1u < count) issue(n + 1u, next);
+        if (n + GROUPS < count) issue(n + GROUPS, next);
         const uint32_t k0 = position_of(n);
-        if (!wave_live || k0 >= w_hi || (k0 + 64u <= w_lo && k0 >= p.keep)) return;                // wave-uniform
-        wa_f4 s[2][4];
+        if ((GROUPS > 1 && n >= count) || !wave_live || k0 >= w_hi || (k0 + 64u <= w_lo && k0 >= p.keep)) return;                // wave-uniform
+        wa_f4 s[QB][4];
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
+        for (int b = 0; b < QB; ++b)
 #pragma unroll
             for (int t = 0; t < 4; ++t) s[b][t] = wa_f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -543,12 +547,12 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void window_flash_kern
 #pragma unroll
             for (int t = 0; t < 4; ++t)
 #pragma unroll
-                for (int b = 0; b < 2; ++b) s[b][t] = wa_mfma(a[t], qf[b][st], s[b][t]);
+                for (int b = 0; b < QB; ++b) s[b][t] = wa_mfma(a[t], qf[b][st], s[b][t]);
         }
         const bool masked = k0 < full_lo || k0 + 64u > full_hi;
-        uint4 pf[2][2];
+        uint4 pf[QB][2];
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
+        for (int b = 0; b < QB; ++b) {
             const uint32_t pos = start + min(wt0 + 16u * b + i, p.n_rows - 1u);
             uint32_t w[8];
             if (BOUND) {
@@ -629,18 +633,44 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void window_flash_kern
             for (int t = 0; t < VS; ++t) {
                 const uint4 a = *reinterpret_cast<const uint4*>(cur + AT_V + (16u * t + i) * 128u + ((4u * h + g) ^ (i & 7u)) * 16u);
 #pragma unroll
-                for (int b = 0; b < 2; ++b) acc[b][t] = wa_mfma(a, pf[b][h], acc[b][t]);
+                for (int b = 0; b < QB; ++b) acc[b][t] = wa_mfma(a, pf[b][h], acc[b][t]);
             }
     };
-    issue(0, even);
     // two arrays, written out: a read of this tile does not wait for the tile on its way (1501 queries, 16 heads: 59 -> 43 us)
-    for (uint32_t n = 0; n < count; n += 2u) {
-        tile(n, even, odd);
-        if (n + 1u < count) tile(n + 1u, odd, even);
+    uint8_t *const here = even + group * STAGE, *const there = odd + group * STAGE;
+    if (group < count) issue(group, here);
+    for (uint32_t n = 0; n < count; n += 2u * GROUPS) {
+        tile(n + group, here, there);
+        if (n + GROUPS < count) tile(n + GROUPS + group, there, here);
+    }
+    if constexpr (GROUPS > 1) {
+        // the second group's sums go to the first one through LDS, sixteen queries of a wave at a time
+        static_assert(GROUPS == 2 && 4u * VS * 1024u <= GROUPS * STAGE, "one array holds the sums, the other the rest");
+        wa_f4* sums = reinterpret_cast<wa_f4*>(even) + wave * (VS * 64u) + lane;
+        float* rest = reinterpret_cast<float*>(odd) + wave * 128u + lane;
+#pragma unroll
+        for (int b = 0; b < QB; ++b) {
+            lds_landed_barrier();
+            if (group == 1u) {
+#pragma unroll
+                for (int t = 0; t < VS; ++t) sums[t * 64] = acc[b][t];
+                rest[0] = m[b];
+                rest[64] = l[b];
+            }
+            lds_landed_barrier();
+            if (group == 0u) {
+                // both groups without a key so far: weights of 1 for sums of 0
+                const float m1 = rest[0], mn = fmaxf(m[b], m1), f0 = BOUND ? 1.0f : __builtin_amdgcn_exp2f(m[b] - mn), f1 = BOUND ? 1.0f : __builtin_amdgcn_exp2f(m1 - mn);
+                l[b] = l[b] * f0 + rest[64] * f1;
+#pragma unroll
+                for (int t = 0; t < VS; ++t) acc[b][t] = acc[b][t] * f0 + sums[t * 64] * f1;
+            }
+        }
+        if (group == 1u) return;
     }
     if (!wave_live) return;
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
+    for (int b = 0; b < QB; ++b) {
         float sum = l[b];
         sum += shfl_xor_f(sum, 16);
         sum += shfl_xor_f(sum, 32);
@@ -655,6 +685,18 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void window_flash_kern
             if (d < dv) *reinterpret_cast<uint2*>(out + d) = make_uint2(wa_pack2(acc[b][t][0] * f, acc[b][t][1] * f), wa_pack2(acc[b][t][2] * f, acc[b][t][3] * f));
         }
     }
+}
+
+template <int DK, int DV, bool BOUND>
+__global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void window_flash_kernel(WindowParams p) {
+    window_flash_body<DK, DV, BOUND, 1, 2>(p);
+}
+
+// Blocks of eight waves: two groups of four share a block's keys, a tile each at a time, and bring their sums together at the end.
+// Bound by the vector pipe (a tile of a wave: 0.43 us of products, 0.5 to 0.9 of softmax) where a unit's eight waves are all at work.
+template <int DK, int DV, bool BOUND, int QB>
+__global__ __launch_bounds__(512, 1) void window_flash_halves_kernel(WindowParams p) {
+    window_flash_body<DK, DV, BOUND, 2, QB>(p);
 }
 
 }  // namespace nvmai

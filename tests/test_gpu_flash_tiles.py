@@ -36,3 +36,20 @@ def test_latent(heads, nope, rot, vdim, rank, n, window):
     for portions in ([n], [n - 33, 33]):
         got = L.run(portions, FORMS["expanded"])
         assert np.abs(got - want).max() < 2e-2 * np.abs(want).max(), portions
+
+
+# rows and heads on either side of what each form of the launch is for (256 compute units): 64 queries per block up to 448 blocks, 128 by eight waves up
+# to 256, by four beyond; waves and groups without a key, one tile, an odd number of tiles
+@pytest.mark.parametrize("heads,n", [(16, 33), (16, 65), (16, 1792), (16, 1793), (16, 2048), (24, 1409), (43, 700)])
+def test_forms_of_the_launch(heads, n):
+    import nvmai_amd as nv
+    for softcap, alibi, size in ((6.0, False, None), (0.0, True, 300)):
+        w = Window("bfloat16", heads, 1, 128, 128, size, 4, softcap, alibi, True, capacity=n + 63)
+        data = w.rows(n, n)
+        say("windowed flash, forms", heads, n, softcap)
+        close(w.run(data, nv.row_map(0, 0), nv.WINDOW_FLASH), w.run(data, nv.row_map(0, 0), nv.WINDOW_PLAIN), bar("bfloat16"), "prompt")
+    L = Latent(nv.Context(0, nv.ACT_BF16), np.random.default_rng(n), heads, 128, 64, 128, 64, 500, n)
+    say("latent flash, forms", heads, n)
+    want = L.run([n], FORMS["absorbed"])
+    got = L.run([n], FORMS["expanded"])
+    assert np.abs(got - want).max() < 2e-2 * np.abs(want).max()
