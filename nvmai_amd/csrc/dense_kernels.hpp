@@ -363,10 +363,26 @@ __device__ __forceinline__ float dense_sum_again(const DenseLinearParams& p, uin
     return wave_sum_bcast(sum);
 }
 
+// Which tile a block takes.
+struct DenseTileAt {
+    uint32_t m, n;
+};
+
+__device__ __forceinline__ DenseTileAt dense_tile_at(uint32_t tiles_n, uint32_t tiles_m) {
+    // blocks are dealt to the eight XCDs in turn: give each XCD a run of neighbouring tiles (shared L2 lines)
+    const uint32_t all = tiles_n * tiles_m, xcd = blockIdx.x & 7u, nth = blockIdx.x >> 3;
+    const uint32_t base = all / 8u, extra = all % 8u;
+    const uint32_t tile = xcd * base + min(xcd, extra) + nth;
+    // in bands of eight token tiles, weight tiles outermost within the band
+    const uint32_t band = tile / (8u * tiles_n), in_band = tile % (8u * tiles_n);
+    const uint32_t band_m = min(8u, tiles_m - band * 8u);
+    return {band * 8u + in_band % band_m, in_band / band_m};
+}
+
 // Of 160 KB, one block per compute unit; 64 x 64 tiles of 16-bit inputs fit twice.  Planes come in threes: six stages where they fit
 // (64 x 64, 700 x 1024 x 1024 in 32 bits: 17.4 us with three, 13.5 with six).
 constexpr int dense_stages(int act, int bn, int bm) {
-    return act == ACT_FP32 ? (bn + bm <= 192 ? 6 : 3) : bn + bm <= 192 ? 5 : bn + bm <= 256 ? 4 : bn + bm <= 384 ? 3 : 2;
+    return act == ACT_FP32 ? (bn + bm <= 192 ? 6 : 3) : bn + bm <= 192 ? 5 : bn + bm <= 256 ? 4 : 3;
 }
 
 constexpr int dense_blocks(int act, int bn, int bm) { return 2 * dense_stages(act, bn, bm) * (bn + bm) * 128 <= 160 * 1024 ? 2 : 1; }
@@ -378,16 +394,10 @@ __global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_ker
     constexpr int LA = BN / 32, LB = BM / 32, L = LA + LB;   // 1 KB requests per wave and stage
     constexpr int TN = BN / 64, TM = BM / 64;                // 32 x 32 tiles per wave
     constexpr uint32_t STAGE = (BN + BM) * 128u;
-    __shared__ __attribute__((aligned(1024))) uint8_t l0[STAGE], l1[STAGE], l2[S > 2 ? STAGE : 16], l3[S > 3 ? STAGE : 16], l4[S > 4 ? STAGE : 16], l5[S > 5 ? STAGE : 16];
+    __shared__ __attribute__((aligned(1024))) uint8_t l0[STAGE], l1[STAGE], l2[STAGE], l3[S > 3 ? STAGE : 16], l4[S > 4 ? STAGE : 16], l5[S > 5 ? STAGE : 16];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // blocks are dealt to the eight XCDs in turn: give each XCD a run of neighbouring tiles (shared L2 lines)
-    const uint32_t all = tiles_n * tiles_m, xcd = blockIdx.x & 7u, nth = blockIdx.x >> 3;
-    const uint32_t base = all / 8u, extra = all % 8u;
-    const uint32_t tile = xcd * base + min(xcd, extra) + nth;
-    // in bands of eight token tiles, weight tiles outermost within the band
-    const uint32_t band = tile / (8u * tiles_n), in_band = tile % (8u * tiles_n);
-    const uint32_t band_m = min(8u, tiles_m - band * 8u);
-    const uint32_t m0 = (band * 8u + in_band % band_m) * BM, n0 = (in_band / band_m) * BN;
+    const DenseTileAt at = dense_tile_at(tiles_n, tiles_m);
+    const uint32_t m0 = at.m * BM, n0 = at.n * BN;
 
     const uint32_t steps = p.k / 64u * (SPLIT ? 3u : 1u);
     [[maybe_unused]] const uint32_t w_bytes = (p.n - 1u) * p.w_stride * 2u + p.k * 2u;
@@ -531,9 +541,146 @@ __global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_ker
         }
 #pragma unroll UNROLL
         for (uint32_t k = 0; k < 32u / AT_ONCE; ++k) {
-            const uint32_t at = lane / PER + k * AT_ONCE, t = m0 + wm + 32 * b + at;
-            const dn_f4 v = *reinterpret_cast<const dn_f4*>(turn + at * PITCH + lane % PER * 4u);
+            const uint32_t token = lane / PER + k * AT_ONCE, t = m0 + wm + 32 * b + token;
+            const dn_f4 v = *reinterpret_cast<const dn_f4*>(turn + token * PITCH + lane % PER * 4u);
             if (t < p.rows && r < p.n) dense_store4<EPI, ACT, !SPLIT>(p, t, r, v, bias);
+        }
+    }
+}
+
+// ---- the same in tiles of 256 x 256, 16-bit activations --------------------------------------------------------------------
+// Two stages of 64 KB are all that fits, and a ring that frees a stage as a whole leaves the last requests for the next one a quarter of a
+// stage to arrive.  Here a stage is two halves of both operands (rows 0 .. 63 of every 128, and the others), freed and asked for one by one:
+// a wave's part is four products of half by half, in the order (0, 0), (1, 0), (1, 1), (0, 1), so that the halves 0 are read while the
+// last two products of the stage before run and the halves 1 during the first two; a half is then out of LDS for registers (128 of them hold a
+// stage) one to one and a half stages before its successor is needed.  Barriers stand behind the first four of the sixteen matrix instructions of
+// a product: the reads before them arrive in the meantime.  Requests go out evenly over the stage.  Pieces lie in the order piece ^ (r / 2 % 8):
+// the sixteen lanes that a read serves at once cover 256 bytes.  Bound by the rate of requests into LDS (49 us of the 61 below without the products) and the
+// clock that the products leave.  Rows x n x k, cold weights, former ring of two stages: 2048 x 8192 x 2048 67 -> 61 us, 4096 x 8192 x 2048
+// 126 -> 116, 8192 x 8192 x 8192 823 -> 759.  Not kept: a third place for the halves 0 (no change), requests of 64 bytes per row in stages of 32 k (half
+// the rate).
+template <int EPI>
+__global__ __launch_bounds__(256, 1) void dense_wide_kernel(DenseLinearParams p, uint32_t tiles_n, uint32_t tiles_m) {
+    constexpr uint32_t HALF = 128u * 128u;
+    // weights and tokens: place (stage % 2), half
+    __shared__ __attribute__((aligned(1024))) uint8_t w00[HALF], w01[HALF], w10[HALF], w11[HALF], x00[HALF], x01[HALF], x10[HALF], x11[HALF];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const DenseTileAt at = dense_tile_at(tiles_n, tiles_m);
+    const uint32_t m0 = at.m * 256u, n0 = at.n * 256u;
+    const uint32_t steps = p.k / 64u;
+    [[maybe_unused]] const uint32_t w_bytes = (p.n - 1u) * p.w_stride * 2u + p.k * 2u, x_bytes = (p.rows - 1u) * p.x_stride * 2u + p.k * 2u;
+    auto swizzle = [](uint32_t row) { return (row >> 1) & 7u; };
+    // request r of a wave: rows 32 wave + 8 r .. + 7 of a half (8 r + lane / 8 has two values of the swizzle)
+    const uint32_t lr = lane >> 3;
+    [[maybe_unused]] const uint32_t piece[2] = {((lane & 7u) ^ swizzle(lr)) * 16u, ((lane & 7u) ^ swizzle(lr + 8u)) * 16u};
+    const uint32_t row = (wave & 1u) * 32u + (wave >> 1) * 128u + lr;
+    [[maybe_unused]] const uint32_t w8 = p.w_stride * 16u, w0 = (n0 + row) * p.w_stride * 2u, wmax = (p.n - 1u) * p.w_stride * 2u;
+    [[maybe_unused]] const uint32_t x8 = p.x_stride * 16u, x0 = (m0 + row) * p.x_stride * 2u, xmax = (p.rows - 1u) * p.x_stride * 2u;
+    auto wbuf = [&](int j, int h) -> uint8_t* { return j == 0 ? (h == 0 ? w00 : w01) : (h == 0 ? w10 : w11); };
+    auto xbuf = [&](int j, int h) -> uint8_t* { return j == 0 ? (h == 0 ? x00 : x01) : (h == 0 ? x10 : x11); };
+    // request q of eight (four of weights, four of tokens) of half h of stage st into its place j = st % 2
+    auto request = [&](uint32_t st, int j, int h, int q) {
+#if defined(__HIP_DEVICE_COMPILE__)     // the host pass rejects the 16-byte form of the load
+        const bool live = st < steps;
+        const uint32_t k = st * 128u, r = (uint32_t)q & 3u;
+        if (q < 4) {
+            const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.w), 0, live ? (int)w_bytes : 0, 0x00020000);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (__attribute__((address_space(3))) void*)(wbuf(j, h) + (wave * 4u + r) * 1024u), 16, min(w0 + (8u * h + r) * w8, wmax) + piece[r & 1u], k, 0, 0);
+        } else {
+            const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.x), 0, live ? (int)x_bytes : 0, 0x00020000);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void*)(xbuf(j, h) + (wave * 4u + r) * 1024u), 16, min(x0 + (8u * h + r) * x8, xmax) + piece[r & 1u], k, 0, 0);
+        }
+#endif
+    };
+    const uint32_t i = lane & 31u, g = lane >> 5;
+    const uint32_t wn = (wave >> 1) * 128u, wm = (wave & 1u) * 128u;
+    const uint32_t arow = ((wave >> 1) * 64u + i) * 128u, brow = ((wave & 1u) * 64u + i) * 128u;
+    uint4 A[2][2][4], B[2][2][4];                            // [half][tile of 32][16 k]
+    // operand e of eight of a half
+    auto read_w = [&](int j, int h, int e) { A[h][e & 1][e >> 1] = *reinterpret_cast<const uint4*>(wbuf(j, h) + arow + 4096u * (e & 1) + (((e & ~1u) + g) ^ swizzle(i)) * 16u); };
+    auto read_x = [&](int j, int h, int e) { B[h][e & 1][e >> 1] = *reinterpret_cast<const uint4*>(xbuf(j, h) + brow + 4096u * (e & 1) + (((e & ~1u) + g) ^ swizzle(i)) * 16u); };
+    dn_f16 acc[4][4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) acc[a][b] = dn_f16{};
+    // matrix instruction e of sixteen of the product of two halves
+    auto multiply = [&](int ha, int hb, int e) {
+        const int k = e >> 2, a = (e >> 1) & 1, b = e & 1;
+        acc[2 * ha + a][2 * hb + b] = dn_mfma32(A[ha][a][k], B[hb][b][k], acc[2 * ha + a][2 * hb + b]);
+    };
+    // The half products (h, h) and (1 - h, h): the halves 1 - of the weights, then of the tokens, are read under the first two, those of the
+    // next stage under the last two, where the weights' half 0 is still an operand and is replaced behind its last use.
+    auto stage = [&](uint32_t st, int j) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int next = h == 0 ? j : 1 - j;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) multiply(h, h, e);
+            __builtin_amdgcn_sched_barrier(0);
+            dense_stage_barrier<16>();                       // two halves of both operands stay on their way
+#pragma unroll
+            for (int e = 4; e < 16; ++e) {
+                multiply(h, h, e);
+                if (e < 12) {
+                    if (h == 0) read_w(next, 1, e - 4);
+                    else read_x(next, 0, e - 4);
+                }
+                if (e % 3 == 0) request(st + 2u, j, h, e / 3 - 2);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                multiply(1 - h, h, e);
+                if (h == 0) {
+                    if (e < 8) read_x(next, 1, e);
+                } else if ((e & 3) == 3) {
+                    read_w(next, 0, e >> 2 << 1);
+                    read_w(next, 0, (e >> 2 << 1) + 1);
+                }
+                if (e % 4 == 1) request(st + 2u, j, h, 4 + e / 4);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int q = 0; q < 8; ++q) request(j, j, h, q);
+    dense_stage_barrier<24>();
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        read_w(0, 0, e);
+        read_x(0, 0, e);
+    }
+    uint32_t st = 0;
+    for (; st + 2u <= steps; st += 2u) {
+        stage(st, 0);
+        stage(st + 1u, 1);
+    }
+    if (st < steps) stage(st, 0);
+    dense_stage_barrier<0>();                                // no request outlives its block; the places are free
+    // The sums change places as in dense_tile_kernel, in a row of 128 per token whose pieces of four are exchanged by the token.
+    float* turn = reinterpret_cast<float*>(wave == 0u ? w00 : wave == 1u ? w01 : wave == 2u ? w10 : w11);
+    constexpr int UNROLL = EPI == DE_ERF ? 2 : 4;
+    const uint32_t r = n0 + wn + lane % 32u * 4u;
+    const dn_f4 bias = dense_bias4<EPI>(p, r);
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            const dn_f16 v = acc[a][b];
+#pragma unroll
+            for (int h = 0; h < 4; ++h)                      // element 4 h + e of a lane: row 8 h + 4 g + e, token i
+                *reinterpret_cast<dn_f4*>(turn + i * 128u + (((8u * a + 2u * h + g) ^ i) * 4u)) = dn_f4{v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]};
+        }
+#pragma unroll UNROLL
+        for (uint32_t k = 0; k < 16u; ++k) {
+            const uint32_t token = lane / 32u + k * 2u, t = m0 + wm + 32 * b + token;
+            const dn_f4 v = *reinterpret_cast<const dn_f4*>(turn + token * 128u + ((lane % 32u) ^ token) * 4u);
+            if (t < p.rows && r < p.n) dense_store4<EPI, ACT_BF16, true>(p, t, r, v, bias);
         }
     }
 }
@@ -610,7 +757,7 @@ int gemv(const DenseLinearParams& p, hipStream_t s) {
 struct DenseTile {
     uint32_t bn, bm, lone, full;
 };
-constexpr DenseTile DENSE_TILES[] = {{64, 64, 19, 21}, {128, 64, 24, 34}, {128, 128, 30, 55}, {256, 128, 50, 100}, {256, 256, 115, 185}};
+constexpr DenseTile DENSE_TILES[] = {{64, 64, 19, 21}, {128, 64, 24, 34}, {128, 128, 30, 55}, {256, 128, 50, 100}, {256, 256, 105, 168}};
 
 struct DensePlan {
     int tile;
@@ -654,7 +801,7 @@ void launch_tile(hipStream_t s, const DenseLinearParams& p, int c) {
     else if (c == 2) dense_tile_kernel<EPI, ACT, 128, 128><<<tn * tm, 256, 0, s>>>(p, tn, tm);
     if constexpr (COUNT > 3) {
         if (c == 3) dense_tile_kernel<EPI, ACT, 256, 128><<<tn * tm, 256, 0, s>>>(p, tn, tm);
-        else if (c == 4) dense_tile_kernel<EPI, ACT, 256, 256><<<tn * tm, 256, 0, s>>>(p, tn, tm);
+        else if (c == 4) dense_wide_kernel<EPI><<<tn * tm, 256, 0, s>>>(p, tn, tm);
     }
 }
 
