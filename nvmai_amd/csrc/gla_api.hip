@@ -26,14 +26,22 @@ int gla_recurrent(const GlaParams& p, uint32_t batch, hipStream_t s) {
     return gla_recurrent_sized<ACT, 0, 1024>(p, batch, s);
 }
 
-template <int ACT, int KT>
-void gla_spans(const GlaParams& p, uint32_t subs, uint32_t spans, hipStream_t s) {
+template <int ACT, int KT, bool ONE>
+void gla_spans_by(const GlaParams& p, uint32_t spans, hipStream_t s) {
     const dim3 grid(spans, p.heads);
     const uint32_t threads = p.dv * 4u;              // a wave per sixteen value columns
-    gla_span_kernel<ACT, KT, false><<<grid, threads, 0, s>>>(p);
-    gla_span_decay_kernel<<<dim3((p.heads * p.dk + 255) / 256, spans), 256, 0, s>>>(p, subs);
+    gla_span_kernel<ACT, KT, false, ONE><<<grid, threads, 0, s>>>(p);
     gla_scan_kernel<<<dim3((p.dk * p.dv / 4 + 255) / 256, p.heads), 256, 0, s>>>(p, spans);
-    gla_span_kernel<ACT, KT, true><<<grid, threads, 0, s>>>(p);
+    gla_span_kernel<ACT, KT, true, false><<<grid, threads, 0, s>>>(p);
+}
+
+template <int ACT, int KT>
+void gla_spans(const GlaParams& p, uint32_t spans, hipStream_t s) {
+    // a piece of a sub-chunk's 64 KT and a decay per thread; at 256 key channels there are no registers for them
+    if constexpr (KT <= 8) {
+        if (KT * 16 <= (int)p.dv) return gla_spans_by<ACT, KT, true>(p, spans, s);
+    }
+    gla_spans_by<ACT, KT, false>(p, spans, s);
 }
 
 template <int ACT>
@@ -48,10 +56,10 @@ int gla_chunked(const GlaParams& p, hipStream_t s) {
     if (lds > 128 * 1024) return NVMAI_ERR_UNSUPPORTED;
     gla_prep_kernel<<<dim3(subs, p.heads), 256, lds, s>>>(p);
     const uint32_t kt = (p.dk + 15) / 16;
-    if (kt <= 2) gla_spans<ACT, 2>(p, subs, spans, s);
-    else if (kt <= 4) gla_spans<ACT, 4>(p, subs, spans, s);
-    else if (kt <= 8) gla_spans<ACT, 8>(p, subs, spans, s);
-    else gla_spans<ACT, 16>(p, subs, spans, s);
+    if (kt <= 2) gla_spans<ACT, 2>(p, spans, s);
+    else if (kt <= 4) gla_spans<ACT, 4>(p, spans, s);
+    else if (kt <= 8) gla_spans<ACT, 8>(p, spans, s);
+    else gla_spans<ACT, 16>(p, spans, s);
     return launch_status();
 }
 

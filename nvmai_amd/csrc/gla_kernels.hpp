@@ -41,7 +41,7 @@ struct GlaParams {
     float *qd, *kd;                      // [sub, head, 16, dk]
     float* edge;                         // [sub, head, dk]        2^b_16
     float* att;                          // [sub, head, 16, 16]    A
-    float* spans;                        // [span, head, dk, dv]
+    float* spans;                        // [span, head, dv / 16, dk / 16, 64, 4]: tiles of 16 x 16 as a wave's accumulators hold them
     float* span_decay;                   // [span, head, dk]
 };
 
@@ -289,63 +289,98 @@ __global__ __launch_bounds__(256) void gla_prep_kernel(GlaParams p) {
 
 // ---- chunked: a span's sub-chunks in order ---------------------------------------------------------------
 // Wave w owns the value columns 16 w .. 16 w + 15.  OUT = false: from a zero state, the span's own contribution
-// goes to spans / span_decay.  OUT = true: from the state in spans, the outputs.
-template <int ACT, int KT, bool OUT>
+// goes to spans, the product of its sub-chunks' decays to span_decay.  OUT = true: from the state in spans, the outputs.
+// A sub-chunk's values and gates are requested before the products of the one ahead of it.  ONE (without OUT, whose
+// registers are full): so are its decayed keys and decays, of which a thread then has one piece of 16 bytes and one number.
+// Bound by memory (2048 rows, 16 heads of 128 / 128: 67 MB without OUT, 109 with) and, below two blocks per compute unit, by the latency of a
+// sub-chunk.  Without OUT 18.2 us, 20.4 without ONE, and 700 rows, 8 heads 9.9 and 11.5 (both with the decays of the span, which were a launch of
+// 4.5 us); with OUT 36.5, 39.5 as long as the state's loads stood under conditions (the compiler then waits for them one by one).
+template <int ACT, int KT, bool OUT, bool ONE>
 __global__ __launch_bounds__(1024) void gla_span_kernel(GlaParams p) {
     constexpr uint32_t KR = 16u * KT, KLD = KR + 16u, QLD = KR + 4u;
     __shared__ __attribute__((aligned(16))) float kds[16 * KLD];
     __shared__ __attribute__((aligned(16))) float qds[OUT ? 16 * QLD : 4];
     __shared__ __attribute__((aligned(16))) float es[KR];
     __shared__ float as[OUT ? 16 * 17 : 1];
-    __shared__ float ssq[OUT ? 16 * 16 : 1];
+    __shared__ __attribute__((aligned(16))) float ssq[OUT ? 16 * 16 : 1];
     const uint32_t tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63u, wave = tid >> 6, i = lane & 15u, g = lane >> 4;
     const uint32_t span = blockIdx.x, head = blockIdx.y, dk = p.dk, dv = p.dv, waves = nthr >> 6;
     const uint32_t col = 16u * wave + i;
     const size_t cell_s = (size_t)span * p.heads + head;
-    float* S = p.spans + cell_s * dk * dv;
+    const uint32_t first = span * p.span, count = min(p.span, (p.rows + GLA_SUB - 1u) / GLA_SUB - first);
+    const gla_f4 zero = gla_f4{0.0f, 0.0f, 0.0f, 0.0f};
+    gla_f4* S = reinterpret_cast<gla_f4*>(p.spans + cell_s * dk * dv) + wave * (dk * 4u);
+    // What sub-chunk c brings: this thread's pieces and its operands, as they lie in memory (from the last place where there is none: a
+    // load under a condition waits for the loads ahead of it, and so does a select beside one); put() and the loop make the others zero.
+    static_assert(!(OUT && ONE), "no registers");
+    gla_f4 kn = zero;
+    float en = 0.0f, vn[4], gn[4];
+    // (addresses: a uniform base and a 32-bit offset of the lane, which takes one register instead of two)
+    auto piece = [&](uint32_t sub, uint32_t e, const float* from) {
+        const uint32_t t = e / (KR / 4u), d = (e % (KR / 4u)) * 4u, at = t * dk + min(d, dk - 4u);
+        return *reinterpret_cast<const gla_f4*>(from + ((size_t)sub * p.heads + head) * (16u * dk) + at);
+    };
+    auto fetch = [&](uint32_t c) {
+        const uint32_t sub = first + c, t0 = sub * GLA_SUB;
+        [[maybe_unused]] const size_t cell = (size_t)sub * p.heads + head;
+        if constexpr (ONE) {
+            kn = piece(sub, min(tid, 4u * KR - 1u), p.kd);
+            en = p.edge[cell * dk + min(tid, dk - 1u)];
+        }
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) vn[ks] = (p.v + (size_t)t0 * p.proj_stride + head * dv)[min(4u * ks + g, p.rows - 1u - t0) * p.proj_stride + col];
+        if (OUT) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) gn[r] = (p.g + (size_t)t0 * p.proj_stride + head * dv)[min(4u * g + r, p.rows - 1u - t0) * p.proj_stride + col];
+        }
+    };
+    auto put = [&](uint32_t c) {
+        [[maybe_unused]] const uint32_t sub = first + c;
+        [[maybe_unused]] const size_t cell = (size_t)sub * p.heads + head;
+        auto place = [&](uint32_t e, const gla_f4& k, const gla_f4& q) {
+            const uint32_t t = e / (KR / 4u), d = (e % (KR / 4u)) * 4u;
+            *reinterpret_cast<gla_f4*>(kds + t * KLD + d) = d < dk ? k : zero;
+            if (OUT) *reinterpret_cast<gla_f4*>(qds + t * QLD + d) = d < dk ? q : zero;
+        };
+        if constexpr (ONE) {
+            if (tid < 4u * KR) place(tid, kn, zero);
+            if (tid < KR) es[tid] = tid < dk ? en : 0.0f;
+        } else {
+            for (uint32_t e = tid; e < 4u * KR; e += nthr) place(e, piece(sub, e, p.kd), OUT ? piece(sub, e, p.qd) : zero);
+            for (uint32_t d = tid; d < KR; d += nthr) es[d] = d < dk ? p.edge[cell * dk + d] : 0.0f;
+            if (OUT)
+                for (uint32_t e = tid; e < 256u; e += nthr) as[(e >> 4) * 17u + (e & 15u)] = p.att[cell * 256u + e];
+        }
+    };
+    fetch(0);
     gla_f4 acc[KT];
 #pragma unroll
     for (int t = 0; t < KT; ++t) {
-        acc[t] = gla_f4{0.0f, 0.0f, 0.0f, 0.0f};
-        if (OUT) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const uint32_t row = 16u * t + 4u * g + r;
-                if (row < dk) acc[t][r] = S[(size_t)row * dv + col];
-            }
+        acc[t] = zero;
+        if (OUT && 16u * t < dk) acc[t] = S[64u * t + lane];         // uniform
+    }
+    if (!OUT) {
+        for (uint32_t d = tid; d < dk; d += nthr) {
+            float e = 1.0f;
+            for (uint32_t c = 0; c < count; ++c) e *= p.edge[((size_t)(first + c) * p.heads + head) * dk + d];
+            p.span_decay[cell_s * dk + d] = e;
         }
     }
-    for (uint32_t c = 0; c < p.span; ++c) {
-        const uint32_t sub = span * p.span + c, t0 = sub * GLA_SUB;
-        if (t0 >= p.rows) break;                     // uniform
-        const size_t cell = (size_t)sub * p.heads + head;
+    const float nw = OUT ? bf16_to_f32(p.norm_weight[col]) : 0.0f;
+    for (uint32_t c = 0; c < count; ++c) {
+        const uint32_t t0 = (first + c) * GLA_SUB;
         __syncthreads();
-        for (uint32_t e = tid; e < 16u * KR / 4u; e += nthr) {
-            const uint32_t t = e / (KR / 4u), d = (e % (KR / 4u)) * 4u;
-            const gla_f4 zero = gla_f4{0.0f, 0.0f, 0.0f, 0.0f};
-            const size_t at = (cell * 16u + t) * dk + d;
-            *reinterpret_cast<gla_f4*>(kds + t * KLD + d) = d < dk ? *reinterpret_cast<const gla_f4*>(p.kd + at) : zero;
-            if (OUT) *reinterpret_cast<gla_f4*>(qds + t * QLD + d) = d < dk ? *reinterpret_cast<const gla_f4*>(p.qd + at) : zero;
-        }
-        for (uint32_t d = tid; d < KR; d += nthr) es[d] = d < dk ? p.edge[cell * dk + d] : 0.0f;
-        if (OUT)
-            for (uint32_t e = tid; e < 256u; e += nthr) as[(e >> 4) * 17u + (e & 15u)] = p.att[cell * 256u + e];
-        float vb[4];                                 // B operand: row 4 ks + g, this lane's column
+        put(c);
+        float vb[4], gate[4];                        // B operand: row 4 ks + g, this lane's column
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const uint32_t t = t0 + 4u * ks + g;
-            const float v = p.v[(size_t)min(t, p.rows - 1u) * p.proj_stride + head * dv + col];
-            vb[ks] = t < p.rows ? v : 0.0f;
+        for (int r = 0; r < 4; ++r) {
+            vb[r] = t0 + 4u * r + g < p.rows ? vn[r] : 0.0f;
+            if (OUT) gate[r] = gn[r];
         }
-        float gate[4];
-        if (OUT) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                gate[r] = p.g[(size_t)min(t0 + 4u * g + r, p.rows - 1u) * p.proj_stride + head * dv + col];
-        }
+        if (c + 1u < count) fetch(c + 1u);           // uniform
         __syncthreads();
         if (OUT) {
-            gla_f4 o0 = gla_f4{0.0f, 0.0f, 0.0f, 0.0f}, o1 = o0;
+            gla_f4 o0 = zero, o1 = zero;
 #pragma unroll
             for (int t = 0; t < KT; ++t) {
                 const gla_f4 q = *reinterpret_cast<const gla_f4*>(qds + i * QLD + 16 * t + 4u * g);
@@ -365,15 +400,13 @@ __global__ __launch_bounds__(1024) void gla_span_kernel(GlaParams p) {
                 for (int r = 0; r < 4; ++r) ssq[wave * 16u + 4u * g + r] = sq[r];
             }
             __syncthreads();
-            const float nw = bf16_to_f32(p.norm_weight[col]);
+            gla_f4 sum = zero;
+            for (uint32_t w = 0; w < waves; ++w) sum += *reinterpret_cast<const gla_f4*>(ssq + w * 16u + 4u * g);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                float sum = 0.0f;
-                for (uint32_t w = 0; w < waves; ++w) sum += ssq[w * 16u + 4u * g + r];
-                const float inv = 1.0f / sqrtf(sum / (float)p.dv_count + p.eps);
-                const uint32_t t = t0 + 4u * g + r;
-                if (t < p.rows)
-                    static_cast<act_t<ACT>*>(p.out)[(size_t)t * p.out_stride + head * dv + col] = f32_to_act<ACT>(o0[r] * inv * nw * gla_silu(gate[r]));
+                const float inv = 1.0f / sqrtf(sum[r] / (float)p.dv_count + p.eps);
+                if (t0 + 4u * g + r < p.rows)
+                    (static_cast<act_t<ACT>*>(p.out) + (size_t)t0 * p.out_stride + head * dv)[(4u * g + r) * p.out_stride + col] = f32_to_act<ACT>(o0[r] * inv * nw * gla_silu(gate[r]));
             }
             if (c + 1u == p.span) break;           // the state after the span came from the scan
         }
@@ -389,11 +422,7 @@ __global__ __launch_bounds__(1024) void gla_span_kernel(GlaParams p) {
     if (OUT) return;
 #pragma unroll
     for (int t = 0; t < KT; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const uint32_t row = 16u * t + 4u * g + r;
-            if (row < dk) S[(size_t)row * dv + col] = acc[t][r];
-        }
+        if (16u * t < dk) S[64u * t + lane] = acc[t];
 }
 
 // spans: each span's own contribution -> the state it starts from; the sequence's state ends after the last span.
@@ -401,21 +430,23 @@ __global__ __launch_bounds__(256) void gla_scan_kernel(GlaParams p, uint32_t n_s
     constexpr int AHEAD = 8;
     const uint32_t per_head = p.dk * p.dv / 4u, at = blockIdx.x * 256u + threadIdx.x, head = blockIdx.y;
     if (at >= per_head) return;
-    const uint32_t row = at * 4u / p.dv;
-    gla_f4* state = reinterpret_cast<gla_f4*>(p.state + ((size_t)p.slot0 * p.heads + head) * p.dk * p.dv) + at;
+    // rows row .. row + 3 of one column
+    const uint32_t lane = at & 63u, tile = at >> 6, col = tile / (p.dk / 16u) * 16u + (lane & 15u), row = tile % (p.dk / 16u) * 16u + (lane >> 4) * 4u;
+    float* state = p.state + ((size_t)p.slot0 * p.heads + head) * p.dk * p.dv + row * p.dv + col;
     gla_f4* own = reinterpret_cast<gla_f4*>(p.spans + (size_t)head * p.dk * p.dv) + at;
     const size_t step = (size_t)p.heads * per_head;
     const float* dec = p.span_decay + (size_t)head * p.dk + row;
     const size_t dstep = (size_t)p.heads * p.dk;
-    gla_f4 S = *state;
+    gla_f4 S;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[r] = state[r * p.dv];
     for (uint32_t n0 = 0; n0 < n_spans; n0 += AHEAD) {
-        gla_f4 add[AHEAD];
-        float d[AHEAD];
+        gla_f4 add[AHEAD], d[AHEAD];
 #pragma unroll
         for (int u = 0; u < AHEAD; ++u) {
             const uint32_t n = min(n0 + u, n_spans - 1u);
             add[u] = own[n * step];
-            d[u] = dec[n * dstep];
+            d[u] = *reinterpret_cast<const gla_f4*>(dec + n * dstep);
         }
 #pragma unroll
         for (int u = 0; u < AHEAD; ++u)
@@ -424,17 +455,8 @@ __global__ __launch_bounds__(256) void gla_scan_kernel(GlaParams p, uint32_t n_s
                 S = S * d[u] + add[u];
             }
     }
-    *state = S;
-}
-
-// the decay of a whole span: the product of its sub-chunks'
-__global__ __launch_bounds__(256) void gla_span_decay_kernel(GlaParams p, uint32_t n_subs) {
-    const uint32_t at = blockIdx.x * 256u + threadIdx.x, span = blockIdx.y;
-    if (at >= p.heads * p.dk) return;
-    float d = 1.0f;
-    for (uint32_t c = 0; c < p.span; ++c)
-        if (span * p.span + c < n_subs) d *= p.edge[(size_t)(span * p.span + c) * p.heads * p.dk + at];
-    p.span_decay[(size_t)span * p.heads * p.dk + at] = d;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) state[r * p.dv] = S[r];
 }
 
 }  // namespace nvmai
