@@ -525,6 +525,14 @@ int nvmai_hip_sample_topk64(nvmai_hip_ctx* ctx, nvmai_stream stream, const uint1
                             float top_p, const uint64_t* seeds, uint32_t top_k, uint32_t* out_token,
                             uint32_t* top64_out);
 
+/* Both of the above in three launches instead of four, with the same bits in probs, token and candidates
+ * (v <= 262144). */
+int nvmai_hip_softmax_sample_topk64(nvmai_hip_ctx* ctx, nvmai_stream stream, const void* logits,
+                                    uint32_t logits_stride, uint16_t* probs, uint32_t probs_stride,
+                                    uint32_t rows, uint32_t v, float softcap, float temperature,
+                                    float top_p, const uint64_t* seeds, uint32_t top_k,
+                                    uint32_t* out_token, uint32_t* top64_out);
+
 /* Sample.encode (LogitOutput.swift:157-199; kernel logit.metal:315-585), the kernel's three
  * paths: temperature <= 0 is greedy argmax (lowest index wins ties); top_k == 0 with top_p
  * outside (0, 1) is the Gumbel-max draw argmax(log p / T + g) with g from SplitMix64 of

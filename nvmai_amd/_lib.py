@@ -172,6 +172,7 @@ SIGNATURES = {
     "nvmai_attention_split_geometry": [u32, u32, u32, u32, C.c_int, C.POINTER(u32), C.POINTER(u32),
                                        C.POINTER(u32), C.POINTER(u32)],
     "nvmai_hip_softmax_tiled": [vp, vp, vp, u32, vp, u32, u32, u32, C.c_float],
+    "nvmai_hip_softmax_sample_topk64": [vp, vp, vp, u32, vp, u32, u32, u32, C.c_float, C.c_float, C.c_float, C.POINTER(u64), u32, vp, vp],
     "nvmai_hip_sample_topk64": [vp, vp, vp, u32, u32, u32, C.c_float, C.c_float, C.POINTER(u64), u32, vp, vp],
     "nvmai_prefill_grouping_check": [C.c_int64] * 5 + [C.c_int, C.c_int64],
     "nvmai_hip_prefill_make_pairs": [vp, vp, vp, vp, u32, u32, vp],

@@ -45,29 +45,73 @@ extern "C" int nvmai_hip_softmax_tiled(nvmai_hip_ctx* ctx, nvmai_stream stream, 
     return launch_status();
 }
 
+namespace {
+// What both entry points of the tiled sampler refuse.
+int check_topk64(const uint64_t* seeds, const uint32_t* out_token, uint32_t rows, uint32_t v, float temperature, uint32_t top_k) {
+    if (!seeds || !out_token) return NVMAI_ERR_INVALID_ARG;
+    if (v == 0 || v > 262144) return NVMAI_ERR_UNSUPPORTED;      // SampleTopK64Error.unsupportedVocabulary
+    if (!(temperature > 0.0f)) return NVMAI_ERR_INVALID_ARG;     // LogitOutput.swift:280-281
+    if (top_k < 1 || top_k > 64) return NVMAI_ERR_INVALID_ARG;   // LogitOutput.swift:282-283
+    return rows > SAMPLE_MAX_ROWS ? NVMAI_ERR_INVALID_ARG : NVMAI_OK;
+}
+
+void launch_final(const uint64_t* keys, uint32_t runs, uint32_t rows, float temperature, float top_p, const uint64_t* seeds, uint32_t top_k,
+                  uint32_t* out_token, uint32_t* top64_out, hipStream_t s) {
+    SeedArray sa{};
+    for (uint32_t r = 0; r < rows; ++r) sa.s[r] = seeds[r];
+    sample_topk64_final_kernel<<<dim3(rows), 1024, 0, s>>>(keys, runs, temperature, top_p, sa, top_k, out_token, top64_out);
+}
+
+template <int ACT>
+void launch_softmax_top64(const void* logits, uint32_t logits_stride, uint16_t* probs, uint32_t probs_stride, uint32_t rows, uint32_t v,
+                          float softcap, float* tmax, float* tsum, uint64_t* keys, uint32_t runs, hipStream_t s) {
+    const uint32_t tiles = (v + SOFTMAX_TILE - 1) / SOFTMAX_TILE;
+    softmax_stage1_kernel<ACT><<<dim3(tiles, rows), 256, 0, s>>>(logits, v, logits_stride, softcap, tmax, tsum, tiles);
+    softmax_top64_kernel<ACT><<<dim3(tiles, rows), 1024, 0, s>>>(logits, v, logits_stride, softcap, tmax, tsum, tiles, probs, probs_stride, keys,
+                                                                 runs * SAMPLE_KEEP);
+}
+}  // namespace
+
 extern "C" int nvmai_hip_sample_topk64(nvmai_hip_ctx* ctx, nvmai_stream stream, const uint16_t* probs,
                                        uint32_t probs_stride, uint32_t rows, uint32_t v, float temperature,
                                        float top_p, const uint64_t* seeds, uint32_t top_k, uint32_t* out_token,
                                        uint32_t* top64_out) {
-    if (!ctx || !probs || !seeds || !out_token || probs_stride < v) return NVMAI_ERR_INVALID_ARG;
-    if (v == 0 || v > 262144) return NVMAI_ERR_UNSUPPORTED;      // SampleTopK64Error.unsupportedVocabulary
-    if (!(temperature > 0.0f)) return NVMAI_ERR_INVALID_ARG;     // LogitOutput.swift:280-281
-    if (top_k < 1 || top_k > 64) return NVMAI_ERR_INVALID_ARG;   // LogitOutput.swift:282-283
-    if (rows == 0) return NVMAI_OK;
-    if (rows > SAMPLE_MAX_ROWS) return NVMAI_ERR_INVALID_ARG;
+    if (!ctx || !probs || probs_stride < v) return NVMAI_ERR_INVALID_ARG;
+    int rc = check_topk64(seeds, out_token, rows, v, temperature, top_k);
+    if (rc || rows == 0) return rc;
     hipStream_t s = (hipStream_t)stream;
-    const uint32_t g1 = (v + SAMPLE_TILE - 1) / SAMPLE_TILE, c1 = g1 * SAMPLE_KEEP;
-    const uint32_t g2 = (c1 + SAMPLE_TILE - 1) / SAMPLE_TILE, c2 = g2 * SAMPLE_KEEP;
-    int rc = ws_begin(ctx, stream, ws_round((size_t)rows * c1 * 8) + ws_round((size_t)rows * c2 * 8));
+    const uint32_t runs = (v + SAMPLE_TILE - 1) / SAMPLE_TILE;
+    rc = ws_begin(ctx, stream, ws_round((size_t)rows * runs * SAMPLE_KEEP * 8));
     if (rc) return rc;
-    uint64_t* s1 = ws_take<uint64_t>(ctx, (size_t)rows * c1);
-    uint64_t* s2 = ws_take<uint64_t>(ctx, (size_t)rows * c2);
-    SeedArray sa{};
-    for (uint32_t r = 0; r < rows; ++r) sa.s[r] = seeds[r];
+    uint64_t* keys = ws_take<uint64_t>(ctx, (size_t)rows * runs * SAMPLE_KEEP);
     ProfScope ps(ctx, NVMAI_PROF_SAMPLE, s);
-    sample_topk64_stage1_kernel<<<dim3(g1, rows), 256, 0, s>>>(probs, v, probs_stride, s1, c1);
-    sample_topk64_reduce_kernel<<<dim3(g2, rows), 256, 0, s>>>(s1, c1, c1, s2, c2);
-    sample_topk64_final_kernel<<<dim3(rows), 256, 0, s>>>(s2, c2, c2, temperature, top_p, sa, top_k, out_token, top64_out);
+    sample_topk64_stage1_kernel<<<dim3(runs, rows), 256, 0, s>>>(probs, v, probs_stride, keys, runs * SAMPLE_KEEP);
+    launch_final(keys, runs, rows, temperature, top_p, seeds, top_k, out_token, top64_out, s);
+    return launch_status();
+}
+
+extern "C" int nvmai_hip_softmax_sample_topk64(nvmai_hip_ctx* ctx, nvmai_stream stream, const void* logits, uint32_t logits_stride,
+                                               uint16_t* probs, uint32_t probs_stride, uint32_t rows, uint32_t v, float softcap,
+                                               float temperature, float top_p, const uint64_t* seeds, uint32_t top_k,
+                                               uint32_t* out_token, uint32_t* top64_out) {
+    if (!ctx || !logits || !probs || logits_stride < v || probs_stride < v) return NVMAI_ERR_INVALID_ARG;
+    int rc = check_topk64(seeds, out_token, rows, v, temperature, top_k);
+    if (rc || rows == 0) return rc;
+    hipStream_t s = (hipStream_t)stream;
+    const uint32_t runs = (v + SAMPLE_TILE - 1) / SAMPLE_TILE, tiles = (v + SOFTMAX_TILE - 1) / SOFTMAX_TILE;
+    rc = ws_begin(ctx, stream, 2 * ws_round((size_t)rows * tiles * 4) + ws_round((size_t)rows * runs * SAMPLE_KEEP * 8));
+    if (rc) return rc;
+    float* tmax = ws_take<float>(ctx, (size_t)rows * tiles);
+    float* tsum = ws_take<float>(ctx, (size_t)rows * tiles);
+    uint64_t* keys = ws_take<uint64_t>(ctx, (size_t)rows * runs * SAMPLE_KEEP);
+    {
+        ProfScope ps(ctx, NVMAI_PROF_SOFTMAX, s);
+        if (ctx->act == ACT_FP32) launch_softmax_top64<ACT_FP32>(logits, logits_stride, probs, probs_stride, rows, v, softcap, tmax, tsum, keys, runs, s);
+        else if (ctx->act == ACT_BF16) launch_softmax_top64<ACT_BF16>(logits, logits_stride, probs, probs_stride, rows, v, softcap, tmax, tsum, keys, runs, s);
+        else launch_softmax_top64<ACT_FP16>(logits, logits_stride, probs, probs_stride, rows, v, softcap, tmax, tsum, keys, runs, s);
+    }
+    ProfScope ps(ctx, NVMAI_PROF_SAMPLE, s);
+    launch_final(keys, runs, rows, temperature, top_p, seeds, top_k, out_token, top64_out, s);
     return launch_status();
 }
 
@@ -151,14 +195,16 @@ extern "C" int nvmai_hip_sampler_sample(nvmai_hip_ctx* ctx, nvmai_stream stream,
     }
     // one front end serves both paths here: the tiled and the single-group softmax of the
     // reference agree to 1e-5 and differ only in how the work is cut
-    int rc = nvmai_hip_softmax_tiled(ctx, stream, logits, v, probs, v, 1, v, logit_softcap);
-    if (rc) return rc;
-    const uint64_t seed = config->has_seed ? nvmai_sampler_seed_for(config->seed, position) : clock_seed();
+    int rc;
     const float top_p = has_p ? config->top_p : 1.0f;
     if (sampler_path == NVMAI_SAMPLER_TILED && T > 0.0f && has_k && config->top_k <= 64 && v <= 262144) {   // :211-214
-        rc = nvmai_hip_sample_topk64(ctx, stream, probs, v, 1, v, T, top_p, &seed, (uint32_t)config->top_k, out_token,
-                                     nullptr);
+        const uint64_t seed = config->has_seed ? nvmai_sampler_seed_for(config->seed, position) : clock_seed();
+        rc = nvmai_hip_softmax_sample_topk64(ctx, stream, logits, v, probs, v, 1, v, logit_softcap, T, top_p, &seed, (uint32_t)config->top_k,
+                                             out_token, nullptr);
     } else {
+        rc = nvmai_hip_softmax_tiled(ctx, stream, logits, v, probs, v, 1, v, logit_softcap);
+        if (rc) return rc;
+        const uint64_t seed = config->has_seed ? nvmai_sampler_seed_for(config->seed, position) : clock_seed();
         const uint32_t pos = (uint32_t)position;
         rc = nvmai_hip_sample(ctx, stream, probs, v, 1, v, T, has_k ? (uint32_t)config->top_k : 0u, top_p, &seed, &pos,
                               out_token);

@@ -30,19 +30,22 @@ __device__ __forceinline__ void softmax_merge(float& m, float& d, float m2, floa
 // Every thread ends with the block's state: the maximum first (max reductions only), then each
 // state's sum rescaled to it once, then plain sums.  Equal to folding softmax_merge over the
 // states up to the rounding of the additions.
+template <int WAVES>
 __device__ __forceinline__ void block_softmax_merge(float& m, float& d, float* lds) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const float wm = wave_max_f32(m);
     if (lane == 0) lds[wave] = wm;
     __syncthreads();
     float bm = lds[0];
-    for (int w = 1; w < (int)(blockDim.x >> 6); ++w) bm = fmaxf(bm, lds[w]);
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) bm = fmaxf(bm, lds[w]);
     const float scaled = (m == -INFINITY) ? 0.0f : d * __expf(m - bm);
     const float ws = wave_sum_bcast(scaled);
-    if (lane == 0) lds[4 + wave] = ws;
+    if (lane == 0) lds[WAVES + wave] = ws;
     __syncthreads();
-    float bd = lds[4];
-    for (int w = 1; w < (int)(blockDim.x >> 6); ++w) bd += lds[4 + w];
+    float bd = lds[WAVES];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) bd += lds[WAVES + w];
     __syncthreads();
     m = bm;
     d = bd;
@@ -103,7 +106,7 @@ __global__ __launch_bounds__(256) void softmax_stage1_kernel(const void* logits,
 #pragma unroll
         for (int j = 0; j < SOFTMAX_PER_THREAD; ++j) d += __expf(x[j] - m);   // exp(-inf) = 0 past the end
     }
-    block_softmax_merge(m, d, lds);
+    block_softmax_merge<4>(m, d, lds);
     if (threadIdx.x == 0) { tile_max[(size_t)row * tiles + tile] = m; tile_sum[(size_t)row * tiles + tile] = d; }
 }
 
@@ -123,7 +126,7 @@ __global__ __launch_bounds__(256) void softmax_normalize_kernel(const void* logi
     float m = -INFINITY, d = 0.0f;
     for (uint32_t t = threadIdx.x; t < tiles; t += 256)
         softmax_merge(m, d, tile_max[(size_t)row * tiles + t], tile_sum[(size_t)row * tiles + t]);
-    block_softmax_merge(m, d, lds);
+    block_softmax_merge<4>(m, d, lds);
     const float inv = d > 0.0f ? 1.0f / d : 0.0f;
     uint16_t* out = probs + (size_t)row * probs_stride;
     uint16_t pr[SOFTMAX_PER_THREAD];
@@ -258,16 +261,16 @@ __device__ __forceinline__ K wave_top64(K k[4], int lane, bool sorted) {
     return lane_merge64(m0 > m1 ? m0 : m1, lane, true);
 }
 
-// The best SAMPLE_KEEP of the block's 1024 keys (any assignment of keys to threads and
-// registers), descending, returned in lanes 0..63 of wave 0 (`valid` there); `cand` is 256 keys
+// The best SAMPLE_KEEP of the 1024 keys of four neighbouring waves (any assignment of keys to threads and
+// registers), descending, returned in the lanes of the first of them (`valid` there); `cand` is 256 keys
 // of LDS.
 template <typename K>
 __device__ __forceinline__ K tile_top64(K mine[4], K* cand, bool& valid) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3;
     cand[wave * 64 + lane] = wave_top64(mine, lane, false);
     __syncthreads();
     valid = wave == 0;
-    K best = 0;
+    K best{};
     if (wave == 0) {
         K k[4];
 #pragma unroll
@@ -284,6 +287,14 @@ __device__ __forceinline__ K tile_top64(K mine[4], K* cand, bool& valid) {
 __device__ __forceinline__ uint32_t tile_key(uint16_t h, uint32_t pos) {
     const uint32_t image = h ^ ((h >> 15) ? 0xFFFFu : 0x8000u);
     return (image << 16) | (uint32_t)(SAMPLE_TILE - pos);
+}
+
+// The 64-bit key of a selected one; fewer than 64 entries in the tile: the key of none.
+__device__ __forceinline__ uint64_t tile_key_64(uint32_t key, uint32_t base) {
+    if (!key) return sample_key(-INFINITY, 0xFFFFFFFFu);
+    const uint32_t image = key >> 16;
+    const uint16_t h = (uint16_t)(image ^ ((image >> 15) ? 0x8000u : 0xFFFFu));
+    return sample_key(f16_to_f32(h), base + SAMPLE_TILE - (key & 0xFFFFu));
 }
 
 __global__ __launch_bounds__(256) void sample_topk64_stage1_kernel(const uint16_t* probs, uint32_t v,
@@ -306,32 +317,63 @@ __global__ __launch_bounds__(256) void sample_topk64_stage1_kernel(const uint16_
     }
     bool valid;
     const uint32_t best = tile_top64(mine, cand, valid);
-    if (valid) {
-        uint64_t key = sample_key(-INFINITY, 0xFFFFFFFFu);        // fewer than 64 entries in the tile
-        if (best) {
-            const uint32_t image = best >> 16;
-            const uint16_t h = (uint16_t)(image ^ ((image >> 15) ? 0x8000u : 0xFFFFu));
-            key = sample_key(f16_to_f32(h), base + SAMPLE_TILE - (best & 0xFFFFu));
-        }
-        out[(size_t)row * out_row_stride + blockIdx.x * SAMPLE_KEEP + threadIdx.x] = key;
-    }
+    if (valid) out[(size_t)row * out_row_stride + blockIdx.x * SAMPLE_KEEP + threadIdx.x] = tile_key_64(best, base);
 }
 
-// Reduce (logit.metal:656-682): top 64 of each 1024 surviving candidates.
-__global__ __launch_bounds__(256) void sample_topk64_reduce_kernel(const uint64_t* in, uint32_t count,
-                                                                   uint32_t in_row_stride, uint64_t* out,
-                                                                   uint32_t out_row_stride) {
-    __shared__ uint64_t cand[256];
-    const uint32_t row = blockIdx.y, base = blockIdx.x * SAMPLE_TILE;
-    uint64_t mine[4];
+// Merge, normalize and the top 64 of each 1024 entries in one launch: a block takes the 4096 entries of a softmax tile, a thread four
+// neighbouring ones, four waves a tile of the sampler.  The same bits as the two kernels above (v <= 262144: the tiles' partial
+// states are one wave's, whatever the block's size).
+template <int ACT>
+__global__ __launch_bounds__(1024) void softmax_top64_kernel(const void* logits, uint32_t v, uint32_t row_stride, float softcap,
+                                                             const float* tile_max, const float* tile_sum, uint32_t tiles,
+                                                             uint16_t* probs, uint32_t probs_stride, uint64_t* out,
+                                                             uint32_t out_row_stride) {
+    __shared__ float lds[32];
+    __shared__ uint32_t cand[4][256];
+    const uint32_t row = blockIdx.y, base = blockIdx.x * SOFTMAX_TILE, first = base + 4u * threadIdx.x;
+    const act_t<ACT>* z = (const act_t<ACT>*)logits + (size_t)row * row_stride;
+    const bool whole = base + SOFTMAX_TILE <= v;
+    float x[4];
+    if (whole && (reinterpret_cast<uintptr_t>(z + base) & (4u * sizeof(act_t<ACT>) - 1u)) == 0) {
+        if constexpr (ACT == ACT_FP32) {
+            const float4 q = *reinterpret_cast<const float4*>(z + first);
+            x[0] = q.x; x[1] = q.y; x[2] = q.z; x[3] = q.w;
+        } else {
+            const uint2 q = *reinterpret_cast<const uint2*>(z + first);
+            act2_to_f32<ACT>(q.x, x[0], x[1]);
+            act2_to_f32<ACT>(q.y, x[2], x[3]);
+        }
+    } else {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const uint32_t src = base + r * 256 + threadIdx.x;
-        mine[r] = src < count ? in[(size_t)row * in_row_stride + src] : sample_key(-INFINITY, 0xFFFFFFFFu);
+        for (int j = 0; j < 4; ++j) x[j] = act_to_f32<ACT>(z[min(first + j, v - 1u)]);
     }
+    const uint32_t t = min(threadIdx.x, tiles - 1u);
+    const float tm = tile_max[(size_t)row * tiles + t], ts = tile_sum[(size_t)row * tiles + t];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = first + j < v ? softcap_value(x[j], softcap) : -INFINITY;
+    float m = threadIdx.x < tiles ? tm : -INFINITY, d = threadIdx.x < tiles && tm != -INFINITY ? ts : 0.0f;
+    block_softmax_merge<16>(m, d, lds);
+    const float inv = d > 0.0f ? 1.0f / d : 0.0f;
+    uint16_t* to = probs + (size_t)row * probs_stride;
+    uint32_t mine[4], pr[4];
+    const uint32_t place = 4u * (threadIdx.x & 255u);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        pr[j] = f32_to_f16(__expf(x[j] - m) * inv);
+        mine[j] = first + j < v ? tile_key((uint16_t)pr[j], place + j) : 0u;
+    }
+    if (whole && (reinterpret_cast<uintptr_t>(to + base) & 7u) == 0) {
+        *reinterpret_cast<uint2*>(to + first) = make_uint2(pr[0] | (pr[1] << 16), pr[2] | (pr[3] << 16));
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (first + j < v) to[first + j] = (uint16_t)pr[j];
+    }
+    const uint32_t group = threadIdx.x >> 8, tile = 4u * blockIdx.x + group;
     bool valid;
-    const uint64_t best = tile_top64(mine, cand, valid);
-    if (valid) out[(size_t)row * out_row_stride + blockIdx.x * SAMPLE_KEEP + threadIdx.x] = best;
+    const uint32_t best = tile_top64(mine, cand[group], valid);
+    if (valid && tile * SAMPLE_TILE < v)
+        out[(size_t)row * out_row_stride + tile * SAMPLE_KEEP + (threadIdx.x & 63u)] = tile_key_64(best, tile * SAMPLE_TILE);
 }
 
 // Selection over the sorted candidates (logit.metal:704-757 == :517-571): cap at k,
@@ -364,24 +406,53 @@ __device__ inline uint32_t sample_select(float* val, const uint32_t* idx, uint32
     return picked;
 }
 
-// Final (logit.metal:684-758).  seeds: one per row.  top64 (optional): the 64 sorted
-// candidates per row as (value bits, index) pairs.
-__global__ __launch_bounds__(256) void sample_topk64_final_kernel(const uint64_t* in, uint32_t count,
-                                                                  uint32_t in_row_stride, float temperature,
-                                                                  float top_p, SeedArray seeds,
-                                                                  uint32_t top_k, uint32_t* out_token,
-                                                                  uint32_t* top64) {
-    __shared__ uint64_t cand[256];
-    const uint32_t row = blockIdx.x;
-    uint64_t mine[4];
+// Reduce and final (logit.metal:656-758) in one launch: `runs` descending runs of 64 per row, at most 256.  Each of the
+// sixteen waves selects from every sixteenth of them, then four waves from four each, then the first.  Bound by the chain of dependent
+// exchanges, which is short because the runs are sorted: one row of 24,832 entries 7.5 us, where a launch per step, each sorting anew, took 6.1 + 11.8.
+// seeds: one per row.  top64 (optional): the 64 sorted candidates per row as (value bits, index) pairs.
+__global__ __launch_bounds__(1024) void sample_topk64_final_kernel(const uint64_t* in, uint32_t runs, float temperature,
+                                                                   float top_p, SeedArray seeds,
+                                                                   uint32_t top_k, uint32_t* out_token,
+                                                                   uint32_t* top64) {
+    __shared__ uint64_t cand[16 * SAMPLE_KEEP], last[4 * SAMPLE_KEEP];
+    const uint32_t row = blockIdx.x, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const uint64_t* from = in + (size_t)row * runs * SAMPLE_KEEP;
+    const uint64_t none = sample_key(-INFINITY, 0xFFFFFFFFu);
+    // runs wave + 16 (4 n + r), the odd ones ascending
+    auto fetch = [&](uint32_t n, uint64_t* k) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const uint32_t i = r * 256 + threadIdx.x;
-        mine[r] = i < count ? in[(size_t)row * in_row_stride + i] : sample_key(-INFINITY, 0xFFFFFFFFu);
+        for (uint32_t r = 0; r < 4; ++r) k[r] = from[min(wave + 16u * (4u * n + r), runs - 1u) * SAMPLE_KEEP + ((r & 1u) ? 63 - lane : lane)];
+    };
+    uint64_t k[4], ahead[4], best = none;
+    const uint32_t rounds = (runs + 63u) / 64u;
+    fetch(0, ahead);
+    for (uint32_t n = 0; n < rounds; ++n) {
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) k[r] = wave + 16u * (4u * n + r) < runs ? ahead[r] : none;
+        if (n + 1u < rounds) fetch(n + 1u, ahead);
+        const uint64_t top = wave_top64(k, lane, true);
+        if (n == 0) {
+            best = top;
+        } else {
+            // two descending runs: the larger of one and the other reversed is a bitonic run
+            const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)top, 63 - lane), hi = (uint32_t)__shfl((int)(uint32_t)(top >> 32), 63 - lane);
+            const uint64_t turned = ((uint64_t)hi << 32) | lo;
+            best = lane_merge64(best > turned ? best : turned, lane, true);
+        }
     }
-    bool valid;
-    const uint64_t best = tile_top64(mine, cand, valid);
-    if (!valid) return;                                            // wave 0 goes on: lane = candidate
+    cand[threadIdx.x] = best;
+    __syncthreads();
+    if (wave < 4u) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) k[r] = cand[(4 * wave + r) * SAMPLE_KEEP + ((r & 1) ? 63 - lane : lane)];
+        last[threadIdx.x] = wave_top64(k, lane, true);
+    }
+    __syncthreads();
+    if (wave != 0u) return;                                        // wave 0 goes on: lane = candidate
+#pragma unroll
+    for (int r = 0; r < 4; ++r) k[r] = last[r * SAMPLE_KEEP + ((r & 1) ? 63 - lane : lane)];
+    best = wave_top64(k, lane, true);
     const float val = key_value(best);
     const uint32_t idx = key_index(best);
     if (top64) {
@@ -402,31 +473,37 @@ __global__ __launch_bounds__(256) void sample_topk64_final_kernel(const uint64_t
         float cum = 0.0f;
         uint32_t cut = kept;
         bool found = false;
+        for (uint32_t i0 = 0; i0 < kept && !found; i0 += 8u) {
 #pragma unroll
-        for (int i = 0; i < SAMPLE_KEEP; ++i) {
-            cum = __fadd_rn(cum, readlane_f(val, i));
-            const bool hit = !found && (uint32_t)i < kept && cum >= top_p;
-            cut = hit ? (uint32_t)i + 1u : cut;
-            found = found || hit;
+            for (uint32_t i = i0; i < i0 + 8u; ++i) {
+                cum = __fadd_rn(cum, readlane_f(val, (int)i));
+                const bool hit = !found && i < kept && cum >= top_p;
+                cut = hit ? i + 1u : cut;
+                found = found || hit;
+            }
         }
         kept = cut;
     }
     float surviving = 0.0f;
+    for (uint32_t i0 = 0; i0 < kept; i0 += 8u) {
 #pragma unroll
-    for (int i = 0; i < SAMPLE_KEEP; ++i)
-        surviving = (uint32_t)i < kept ? __fadd_rn(surviving, readlane_f(powed, i)) : surviving;
+        for (uint32_t i = i0; i < i0 + 8u; ++i)
+            surviving = i < kept ? __fadd_rn(surviving, readlane_f(powed, (int)i)) : surviving;
+    }
     uint64_t rng = seeds.s[row];
     (void)xorshift64star(rng);
     const float u = __fmul_rn(uniform01(rng), surviving);
     float run = 0.0f;
     uint32_t picked = (uint32_t)__builtin_amdgcn_readlane((int)idx, 0);
     bool found = false;
+    for (uint32_t i0 = 0; i0 < kept && !found; i0 += 8u) {
 #pragma unroll
-    for (int i = 0; i < SAMPLE_KEEP; ++i) {
-        run = __fadd_rn(run, readlane_f(powed, i));
-        const bool hit = !found && (uint32_t)i < kept && u <= run;
-        picked = hit ? (uint32_t)__builtin_amdgcn_readlane((int)idx, i) : picked;
-        found = found || hit;
+        for (uint32_t i = i0; i < i0 + 8u; ++i) {
+            run = __fadd_rn(run, readlane_f(powed, (int)i));
+            const bool hit = !found && i < kept && u <= run;
+            picked = hit ? (uint32_t)__builtin_amdgcn_readlane((int)idx, (int)i) : picked;
+            found = found || hit;
+        }
     }
     if (threadIdx.x == 0) out_token[row] = picked;
 }

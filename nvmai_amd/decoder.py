@@ -335,12 +335,7 @@ class StepDecoder:
     def sample(self, seeds, temperature=0.6, top_k=20, top_p=0.95):
         """Softcap + softmax and the tiled top-k sampler (Sampler.sample's production path): tokens in
         self.next_tokens."""
-        self.softmax.encode(self.logits, self.probs, softcap=self.cfg.logit_softcap)
-        check(lib.nvmai_hip_sample_topk64(self.ctx.handle, ops._stream(), ops._ptr(self.probs), self.probs.stride(0),
-                                          self.batch, self.cfg.vocab, temperature, top_p,
-                                          (C.c_uint64 * self.batch)(*seeds), top_k, ops._ptr(self.next_tokens), None),
-              "sample_topk64")
-        return self.next_tokens
+        return ops.softmax_sample_topk64(self.ctx, self.logits, self.probs, temperature, top_p, seeds, top_k, self.cfg.logit_softcap, self.next_tokens)
 
     def step(self, position, seeds, temperature=0.6, top_k=20, top_p=0.95):
         """tokens (self.tokens) at `position` -> next tokens (self.next_tokens)."""

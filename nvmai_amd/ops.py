@@ -781,6 +781,16 @@ class SampleTopK64:
         return (out, top) if want_top64 else out
 
 
+def softmax_sample_topk64(ctx, logits, probs, temperature, top_p, seeds, top_k=64, softcap=30.0, out=None, top64=None):
+    """LogitSoftcapSoftmaxTiled and SampleTopK64 in one call: logits [rows, vocab] -> probs (FP16) and one token per row; top64: an int32
+    buffer [rows, 64, 2] for the candidates."""
+    rows, vocab = logits.shape
+    out = torch.empty(rows, dtype=torch.int32, device=logits.device) if out is None else out
+    check(lib.nvmai_hip_softmax_sample_topk64(ctx.handle, _stream(), _ptr(logits), logits.stride(0), _ptr(probs), probs.stride(0), rows, vocab, softcap,
+                                              temperature, top_p, _seed_array(seeds, rows), top_k, _ptr(out), _ptr(top64)), "softmax_sample_topk64")
+    return out
+
+
 class Sample:
     """Mirror of Sample (LogitOutput.swift:152-199): the generic sampler."""
 

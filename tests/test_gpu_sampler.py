@@ -135,6 +135,31 @@ def test_softmax_then_sampler_pipeline(nv, ctx):
         assert tok[r] == O.sample_topk64(ph[r], 0.6, 0.95, seeds[r], 20)
 
 
+# entries below, at and past the tiles of both steps (1024 and 4096) and the counts of runs that the selection treats apart (16 waves, four runs per
+# wave and round)
+@pytest.mark.parametrize("v", [1, 63, 65, 1023, 1025, 4095, 4097, 5000, 24832, 65536, 65537, 131073, 248320, 262144])
+def test_one_call_gives_the_bits_of_softmax_and_sampler(nv, ctx, v):
+    say("softmax and sampler in one call", ctx.act, v)
+    rng = np.random.default_rng(v)
+    for rows, pad, softcap, scale in ((1, 0, 0.0, 4.0), (3, 1, 30.0, 40.0), (2, 8, 0.0, 0.0)):
+        wide = act_tensor(round_act(gauss(rng, (rows, v + pad), scale), ctx.act), ctx)
+        logits = wide[:, pad:] if pad == 1 else wide[:, :v]
+        if v > 100:
+            logits[0, 7:v:3] = float("-inf")
+        probs, got = (torch.full((rows, v + pad), 5.0, dtype=torch.float16, device="cuda") for _ in range(2))
+        lib, check = nv.ops.lib, nv.ops.check
+        check(lib.nvmai_hip_softmax_tiled(ctx.handle, nv.ops._stream(), logits.data_ptr(), logits.stride(0), probs.data_ptr(), probs.stride(0), rows, v, softcap),
+              "softmax")
+        seeds = [nv.sampler_seed_for(77, r + v) for r in range(rows)]
+        top = torch.zeros((rows, 64, 2), dtype=torch.int32, device="cuda")
+        for t, p, k in ((0.6, 0.95, 20), (1.0, 1.0, 64), (1.3, 0.5, 1)):
+            token, want_top = nv.SampleTopK64(ctx, v).encode(probs[:, :v].contiguous(), t, p, seeds, k, want_top64=True)
+            out = nv.ops.softmax_sample_topk64(ctx, logits, got, t, p, seeds, k, softcap, top64=top)
+            assert torch.equal(probs.view(torch.int16), got.view(torch.int16)) and torch.equal(out, token) and torch.equal(top, want_top)
+            for r in range(rows):
+                assert int(out[r]) & 0xFFFFFFFF == O.sample_topk64(u16(probs[r, :v]), t, p, seeds[r], k)
+
+
 def test_gumbel_max_path_matches_oracle(nv, ctx):
     say("gumbel sampler", ctx.act)
     # top_k == 0 and top_p outside (0, 1): logit.metal:391-429; scores must be the same bits
