@@ -118,6 +118,16 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+    v = max(v, (uint32_t)dpp_keep<0xB1, 0xF>((int)v));
+    v = max(v, (uint32_t)dpp_keep<0x4E, 0xF>((int)v));
+    v = max(v, (uint32_t)dpp_keep<0x141, 0xF>((int)v));
+    v = max(v, (uint32_t)dpp_keep<0x140, 0xF>((int)v));
+    v = max(v, (uint32_t)dpp_keep<0x142, 0xA>((int)v));
+    v = max(v, (uint32_t)dpp_keep<0x143, 0xC>((int)v));
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
 // Lane of a SEG-lane segment that holds seg_reduce_sum's result.
 template <int SEG>
 __device__ __forceinline__ bool seg_result_lane(int lane) {

@@ -1064,7 +1064,10 @@ int decode_layer_impl(nvmai_hip_ctx* ctx, nvmai_stream stream, const nvmai_moe_l
     if (rc) return rc;
     {
         ProfScope ps(ctx, NVMAI_PROF_GROUP, s);
-        if (T <= 4) select_group_one_block_kernel<<<1, 256, (4 * E + 8 + pairs) * 4, s>>>(gp);
+        // a wave per token of one block (8 tokens 5.9 us, 16 7.2), or several blocks that meet at a ticket (7.4, 8.6; 24 tokens 9.3, 32 10.0 where
+        // one block takes 10.0 and 11.8: four selections on a SIMD are bound by their instructions)
+        const size_t one = (4 * E + 8 + 2 * (size_t)pairs) * 4;
+        if (T <= 16 && one <= 64 * 1024) select_group_one_block_kernel<<<1, 64 * (T < 4 ? 4 : T), one, s>>>(gp);
         else select_group_kernel<<<(T + 3) / 4, 256, (4 * E + 8 + pairs) * 4, s>>>(gp);
     }
 

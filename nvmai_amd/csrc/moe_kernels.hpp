@@ -1216,25 +1216,17 @@ __device__ __forceinline__ bool better(float v, uint32_t i, float v2, uint32_t i
     return v > v2 || (v == v2 && i < i2);
 }
 
-// Selection for token t by one wave: lane r < top_k ends with the r-th best (score, index).
-__device__ __forceinline__ void select_topk_core(const SelectParams& p, uint32_t t, int lane, float& my_score,
-                                                 uint32_t& my_idx) {
-    float val[TOPK_MAX_PER_LANE];
-    bool taken[TOPK_MAX_PER_LANE];
+// The rounds of select_topk_core by pairs (score, index).
+template <int PER>
+__device__ __forceinline__ void select_topk_pairs(const SelectParams& p, const float* val, int lane, float& my_score, uint32_t& my_idx) {
+    bool taken[PER];
 #pragma unroll
-    for (int j = 0; j < TOPK_MAX_PER_LANE; ++j) {
-        const uint32_t e = lane + 64 * j;
-        const size_t at = (size_t)t * p.num_experts + e;
-        val[j] = e >= p.num_experts ? 0.0f : p.logits[at];
-        taken[j] = e >= p.num_experts;
-    }
-    my_score = 0.0f;
-    my_idx = 0;
+    for (int j = 0; j < PER; ++j) taken[j] = (uint32_t)(lane + 64 * j) >= p.num_experts;
     for (uint32_t round = 0; round < p.top_k; ++round) {
         float bv = -INFINITY;
         uint32_t bi = 0xFFFFFFFFu;
 #pragma unroll
-        for (int j = 0; j < TOPK_MAX_PER_LANE; ++j) {
+        for (int j = 0; j < PER; ++j) {
             const uint32_t e = lane + 64 * j;
             if (!taken[j] && (bi == 0xFFFFFFFFu || better(val[j], e, bv, bi))) { bv = val[j]; bi = e; }
         }
@@ -1244,10 +1236,64 @@ __device__ __forceinline__ void select_topk_core(const SelectParams& p, uint32_t
         bv = wm;
         if (bi == 0xFFFFFFFFu) { bi = 0; bv = -INFINITY; }   // fewer candidates than k
 #pragma unroll
-        for (int j = 0; j < TOPK_MAX_PER_LANE; ++j)
+        for (int j = 0; j < PER; ++j)
             if ((uint32_t)(lane + 64 * j) == bi) taken[j] = true;
         if ((uint32_t)lane == round) { my_score = bv; my_idx = bi; }
     }
+}
+
+// Selection for token t by one wave: lane r < top_k ends with the r-th best (score, index).  PER: scores per lane.
+// A round is one maximum over the wave of unsigned images that order like the scores (0: taken, or past the last expert), and a
+// compare per score that finds the lowest index that has it: about thirty vector instructions at 256 experts, where a compare of (score, index)
+// pairs within the lanes and two reductions were a hundred (one token, 4 bits: the launch that selects for itself 8.7 -> 7.1 us).  Rows with a NaN go the
+// other way, in which it hides what stands behind it in its lane.
+template <int PER>
+__device__ __forceinline__ void select_topk_core(const SelectParams& p, uint32_t t, int lane, float& my_score,
+                                                 uint32_t& my_idx) {
+    float val[PER];
+    bool none = false;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const uint32_t e = lane + 64 * j;
+        val[j] = p.logits[(size_t)t * p.num_experts + min(e, p.num_experts - 1u)];
+    }
+#pragma unroll
+    for (int j = 0; j < PER; ++j) none |= (uint32_t)(lane + 64 * j) < p.num_experts && val[j] != val[j];
+    my_score = 0.0f;
+    my_idx = 0;
+    if (__any(none)) {
+        select_topk_pairs<PER>(p, val, lane, my_score, my_idx);
+        return;
+    }
+    uint32_t key[PER], mine = 0;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const uint32_t u = __float_as_uint(val[j] + 0.0f);             // -0 and 0 are equal
+        key[j] = (uint32_t)(lane + 64 * j) < p.num_experts ? u ^ ((uint32_t)((int)u >> 31) | 0x80000000u) : 0u;
+    }
+    for (uint32_t round = 0; round < p.top_k; ++round) {
+        uint32_t most = key[0];
+#pragma unroll
+        for (int j = 1; j < PER; ++j) most = max(most, key[j]);
+        most = wave_max_u32(most);
+        uint32_t best = 0;                                             // where no candidate is left: expert 0, -inf
+#pragma unroll
+        for (int j = PER - 1; j >= 0; --j) {
+            const uint64_t has = __ballot(key[j] == most);
+            best = has ? 64u * j + (uint32_t)__builtin_ctzll(has) : best;
+        }
+        best = most ? best : 0u;
+#pragma unroll
+        for (int j = 0; j < PER; ++j) key[j] = (uint32_t)(lane + 64 * j) == best ? 0u : key[j];
+        if ((uint32_t)lane == round) { mine = most; my_idx = best; }
+    }
+    if ((uint32_t)lane < p.top_k) my_score = mine ? __uint_as_float(mine ^ ((uint32_t)((int)~mine >> 31) | 0x80000000u)) : -INFINITY;
+}
+
+__device__ __forceinline__ void select_topk_core(const SelectParams& p, uint32_t t, int lane, float& my_score,
+                                                 uint32_t& my_idx) {
+    if (p.num_experts <= 256) select_topk_core<4>(p, t, lane, my_score, my_idx);
+    else select_topk_core<TOPK_MAX_PER_LANE>(p, t, lane, my_score, my_idx);
 }
 
 // Softmax over the selected scores (in the lanes below top_k) times the expert's gain; stores
@@ -1257,7 +1303,7 @@ __device__ __forceinline__ void select_store_routes(const SelectParams& p, uint3
     const float max_s = readlane_f(my_score, 0);
     const float ex = expf(my_score - max_s);
     float sum = 0.0f;
-    for (uint32_t i = 0; i < p.top_k; ++i) sum = __fadd_rn(sum, __shfl(ex, (int)i, 64));
+    for (uint32_t i = 0; i < p.top_k; ++i) sum = __fadd_rn(sum, readlane_f(ex, (int)i));
     if ((uint32_t)lane < p.top_k) {
         const float gain = p.per_expert_scale ? bf16_to_f32(p.per_expert_scale[my_idx]) : 1.0f;
         const float w = __fmul_rn(__fdiv_rn(ex, sum), gain);
@@ -1266,11 +1312,13 @@ __device__ __forceinline__ void select_store_routes(const SelectParams& p, uint3
     }
 }
 
-__device__ void select_topk_wave(const SelectParams& p, uint32_t t, int lane) {
+// Returns the index of the lane's rank.
+__device__ uint32_t select_topk_wave(const SelectParams& p, uint32_t t, int lane) {
     float my_score;
     uint32_t my_idx;
     select_topk_core(p, t, lane, my_score, my_idx);
     select_store_routes(p, t, lane, my_score, my_idx);
+    return my_idx;
 }
 
 __global__ __launch_bounds__(256) void select_topk_kernel(SelectParams p) {
@@ -1299,8 +1347,9 @@ struct GroupParams {
     uint32_t* ticket;          // zero between launches; counts finished blocks
 };
 
-// The work list from every token's routed experts; one block, after all indices are written.
-__device__ void build_work_list(const GroupParams& p, uint32_t* lds) {
+// The work list from every token's routed experts, idx[token * top_k + rank]; one block, after all indices are written.
+template <typename Idx>
+__device__ __forceinline__ void build_work_list(const GroupParams& p, uint32_t* lds, const Idx* idx) {
     const uint32_t tokens = p.sel.tokens, top_k = p.sel.top_k, E = p.sel.num_experts;
     const uint32_t n_pairs = tokens * top_k;
     const uint32_t tid = threadIdx.x;
@@ -1310,7 +1359,6 @@ __device__ void build_work_list(const GroupParams& p, uint32_t* lds) {
     uint32_t* slotr = lds + 3 * E;        // [E] remainder entry of the expert inside its class
     uint32_t* misc = lds + 4 * E;         // [0] pair cursor, [1..4] entries per class, [5] distinct
     uint32_t* rank = lds + 4 * E + 8;     // [n_pairs] rank of the pair inside its expert
-    const volatile uint32_t* idx = p.sel.out_idx;   // written by other blocks: read past L1
     for (uint32_t i = tid; i < 4 * E + 8; i += blockDim.x) lds[i] = 0;
     __syncthreads();
     for (uint32_t i = tid; i < n_pairs; i += blockDim.x) rank[i] = atomicAdd(&cnt[idx[i]], 1u);
@@ -1374,18 +1422,21 @@ __global__ __launch_bounds__(256) void select_group_kernel(GroupParams p) {
     __syncthreads();
     if (lds[0] != gridDim.x - 1) return;  // uniform per block
     __syncthreads();
-    build_work_list(p, lds);
+    build_work_list(p, lds, const_cast<const volatile uint32_t*>(p.sel.out_idx));       // written by other blocks: read past L1
 }
 
-// The same for at most four tokens in ONE block: nothing crosses a block, so the device-scope
+// The same in ONE block, a wave per token: nothing crosses a block, so the device-scope
 // release of the multi-block kernel (an L2 write-back on this multi-die part) and its ticket
-// are not needed.
-__global__ __launch_bounds__(256) void select_group_one_block_kernel(GroupParams p) {
+// are not needed, and the indices stay in LDS.
+__global__ __launch_bounds__(1024) void select_group_one_block_kernel(GroupParams p) {
     extern __shared__ uint32_t lds[];
-    const uint32_t t = threadIdx.x >> 6;
-    if (t < p.sel.tokens) select_topk_wave(p.sel, t, threadIdx.x & 63);
-    __syncthreads();
-    build_work_list(p, lds);
+    const uint32_t tokens = p.sel.tokens, top_k = p.sel.top_k, lane = threadIdx.x & 63u, waves = blockDim.x >> 6;
+    uint32_t* idx = lds + 4u * p.sel.num_experts + 8u + tokens * top_k;
+    for (uint32_t t = threadIdx.x >> 6; t < tokens; t += waves) {
+        const uint32_t mine = select_topk_wave(p.sel, t, (int)lane);
+        if (lane < top_k) idx[t * top_k + lane] = mine;
+    }
+    build_work_list(p, lds, idx);                    // its first barrier stands before the first index is read
 }
 
 // Dense work list: `count` inputs through the expert in slot `slot`.

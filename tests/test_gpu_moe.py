@@ -712,3 +712,52 @@ def test_affine_gemv_prenorm_equals_the_separate_calls(nv, ctx, bits):
     y2 = nv.affine_gemv_prenorm(ctx, p_, s_, b_, bits, h_in, delta, w, h_in, m, n, normed_scratch=scratch)
     torch.cuda.synchronize()
     assert torch.equal(h_in, h_ref) and torch.equal(y2.view(torch.int16), y_ref.view(torch.int16))
+
+
+def _pairs_topk(logits, k):
+    """k rounds of the best (score, lowest index); a lane (index mod 64) offers the first of its scores left, or one behind it that is better, so
+    that a NaN which is first hides what stands behind it."""
+    left, out = np.ones(len(logits), bool), []
+    for _ in range(k):
+        best = None
+        for lane in range(min(64, len(logits))):
+            mine = None
+            for e in range(lane, len(logits), 64):
+                if left[e] and (mine is None or logits[e] > logits[mine]):
+                    mine = e
+            if mine is not None and not np.isnan(logits[mine]) and (best is None or logits[mine] > logits[best] or (logits[mine] == logits[best] and mine < best)):
+                best = mine
+        out.append(0 if best is None else best)                         # expert 0 where none is offered
+        left[out[-1]] = False
+    return out
+
+
+@pytest.mark.parametrize("E", [1, 63, 64, 65, 200, 256, 257, 300, 512])
+def test_selection_of_ties_zeros_infinities_and_nan(nv, ctx_bf16, E):
+    say("selection", E)
+    rng, D = np.random.default_rng(E), 256
+    # column t of the rows is token t's scores where its input is one-hot
+    w = np.zeros((E, D), np.float32)
+    w[:, 0] = rng.integers(-2, 3, E)                                    # ties
+    w[:, 1] = np.where(rng.random(E) < 0.5, 0.0, -0.0)
+    w[:, 2] = rng.standard_normal(E)
+    w[:, 3] = np.where(rng.random(E) < 0.3, -3e38, rng.standard_normal(E))    # times 4: -inf
+    w[:, 4] = np.where(rng.random(E) < 0.1, 3e38, -1.0)                 # times 4: inf
+    w[:, 5] = np.where(rng.random(E) < 0.2, 3e38, rng.standard_normal(E))     # and column 100
+    w[:, 100] = np.where(w[:, 5] > 1e38, -3e38, 0.0)                    # of another chain: inf - inf
+    w[:, 7] = -3e38
+    x = np.zeros((70, D), np.float32)
+    x[np.arange(8), np.arange(8)] = [1, -1, 1, 4, 4, 4, 1, 4]
+    x[5, 100] = 4
+    x[8:] = rng.standard_normal((62, D)) * (np.arange(D) < 3)
+    w, x = O.round_bf16(w), O.round_bf16(x)
+    desc = nv.rows_desc(16, dev(O.bf16_bits(w).view(np.int16)))
+    for tokens, k in ((9, min(E, 8)), (70, min(E, 64))):
+        idx, wt, logits = nv.MoE(ctx_bf16).encode_router(desc, act_tensor(x[:tokens], ctx_bf16), E, D, k, want_logits=True)
+        torch.cuda.synchronize()
+        lo = logits.cpu().numpy()
+        assert np.isnan(lo[5]).any() == bool((w[:, 5] > 1e38).any()) and np.isneginf(lo[7]).all()
+        for t in range(tokens):
+            assert list(u32(idx[t])) == _pairs_topk(lo[t], k), (E, t)
+            if np.isfinite(lo[t]).all():
+                assert np.abs(u16(wt[t]).astype(np.int32) - O.router_topk(lo[t], k, None)[1].astype(np.int32)).max() <= 1
