@@ -805,6 +805,15 @@ int nvmai_hip_rms_residual(nvmai_hip_ctx* ctx, nvmai_stream stream, float* x, ui
                            uint32_t delta_stride, const uint16_t* post_weight, float post_add, const uint16_t* next_weight,
                            float next_add, void* out, uint32_t out_stride, uint32_t rows, uint32_t d, float eps);
 
+/* The end of a sublayer and the product that opens the next one, in 32-bit contexts, for one or two rows of at most 2048:
+ *   x_out  = x + RMS(delta) * (post_add + post_weight)     (x_out not x: other blocks still read it)
+ *   y      = the product of nvmai_hip_dense_linear_ex with x_out as its input
+ * Other contexts and sizes: NVMAI_ERR_UNSUPPORTED (nvmai_hip_rms_residual and nvmai_hip_dense_linear_ex take them). */
+int nvmai_hip_rms_residual_linear(nvmai_hip_ctx* ctx, nvmai_stream stream, const float* x, uint32_t x_stride, const float* delta,
+                                  uint32_t delta_stride, const uint16_t* post_weight, float post_add, float eps, float* x_out,
+                                  uint32_t x_out_stride, const uint16_t* w, uint32_t w_stride, uint32_t rows, uint32_t n, uint32_t k,
+                                  float* y, uint32_t y_stride, const nvmai_linear_epilogue* e);
+
 /* out[t, :] = row token_ids[t] of a BF16 table, as floats; an id >= vocab gives zeros. */
 int nvmai_hip_embed_rows(nvmai_hip_ctx* ctx, nvmai_stream stream, const uint16_t* table, uint32_t table_stride,
                          const uint32_t* token_ids, uint32_t n_tokens, float* out, uint32_t out_stride, uint32_t d, uint32_t vocab);

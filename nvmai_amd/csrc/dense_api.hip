@@ -104,6 +104,20 @@ extern "C" int nvmai_hip_dense_linear_ex(nvmai_hip_ctx* ctx, nvmai_stream stream
     return dense_linear_call(ctx, stream, p);
 }
 
+extern "C" int nvmai_hip_rms_residual_linear(nvmai_hip_ctx* ctx, nvmai_stream stream, const float* x, uint32_t x_stride, const float* delta,
+                                             uint32_t delta_stride, const uint16_t* post_weight, float post_add, float eps, float* x_out,
+                                             uint32_t x_out_stride, const uint16_t* w, uint32_t w_stride, uint32_t rows, uint32_t n, uint32_t k,
+                                             float* y, uint32_t y_stride, const nvmai_linear_epilogue* e) {
+    if (!ctx || !e || !delta || !post_weight || !x_out || x_out == x) return NVMAI_ERR_INVALID_ARG;
+    if (ctx->act != NVMAI_ACT_FP32 || rows > DENSE_RMS_ROWS || k > DENSE_RMS_K) return NVMAI_ERR_UNSUPPORTED;
+    DenseLinearParams p{w, x, y, nullptr, w_stride, x_stride, y_stride, rows, n, k, e->activation, e->bias, e->mul, e->mul_ids, e->mul_stride, e->mul_rows};
+    p.rms_delta = delta; p.rms_w = post_weight; p.rms_out = x_out; p.rms_delta_stride = delta_stride; p.rms_out_stride = x_out_stride;
+    p.rms_add = post_add; p.rms_eps = eps;
+    if (delta_stride < k || x_out_stride < k) return NVMAI_ERR_INVALID_ARG;
+    if (!aligned16(delta) || !aligned16(post_weight) || !aligned16(x_out) || delta_stride % 4 || x_out_stride % 4) return NVMAI_ERR_ALIGNMENT;
+    return dense_linear(ctx, (hipStream_t)stream, p);
+}
+
 extern "C" int nvmai_hip_embed_rows(nvmai_hip_ctx* ctx, nvmai_stream stream, const uint16_t* table, uint32_t table_stride,
                                     const uint32_t* token_ids, uint32_t n_tokens, float* out, uint32_t out_stride, uint32_t d,
                                     uint32_t vocab) {

@@ -17,7 +17,16 @@ struct DenseLinearParams {
     const uint32_t* mul_ids;
     uint32_t mul_stride, mul_rows;
     uint16_t* planes;       // dense_plane_bytes of scratch for the rows of a 32-bit context, or nullptr
+    // the rows that are multiplied are x + RMS(rms_delta) * (rms_add + rms_w), which go to rms_out as well (rms_out not x); nullptr: x
+    const float* rms_delta;
+    const uint16_t* rms_w;
+    float* rms_out;
+    uint32_t rms_delta_stride, rms_out_stride;
+    float rms_add, rms_eps;
 };
+
+// What the form with rms_delta takes beside a 32-bit context: a row is held in the registers of one wave.
+constexpr uint32_t DENSE_RMS_ROWS = 2, DENSE_RMS_K = 2048;
 
 // 32-bit rows are multiplied as three BF16 planes, at most this many rows at a time: 128 MB of planes, or one row's (1.3 GB for
 // the longest that a call accepts), so that byte offsets inside them stay within 32 bits.

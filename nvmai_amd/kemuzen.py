@@ -355,9 +355,9 @@ class KemuzenDecoder(DenseDecoder):
         y = self._buf("scan", T, heads * vdim_p, torch.float32).view(heads, T, vdim_p)         # head by head
         return self.scans[i, ctx].encode(proj, w["conv"], w["conv_bias"], w["a_log"], w["dt_bias"], w["skip"], *self.states[i], rows_at, y)
 
-    def _mix(self, ctx, i, h, rows_at):
-        m, w, T = self.cfg.layers[i][0], self.w.layers[i], h.shape[0]
-        proj = ops.dense_linear(ctx, w["in_proj"], h, y_f32=self._buf("proj", T, w["in_proj"].shape[0], torch.float32), bias=w["in_bias"])
+    def _mix(self, ctx, i, linear, T, rows_at):
+        m, w = self.cfg.layers[i][0], self.w.layers[i]
+        proj = linear(w["in_proj"], y_f32=self._buf("proj", T, w["in_proj"].shape[0], torch.float32), bias=w["in_bias"])
         out, at = self._buf("mixed", T, w["o"].shape[1], ctx.dtype), w["at"]
         if m.kind == "attention":
             self._window(ctx, i, m, proj, rows_at, out)
@@ -379,25 +379,40 @@ class KemuzenDecoder(DenseDecoder):
         ctx, D = self.pass_context(T), cfg.width
         x = self._buf("residual", T, D, torch.float32)
         h, last = self._buf("input", T, cfg.width_p, ctx.dtype), self._buf("normed", T, cfg.width_p, self.ctx.dtype)
+        # Short passes: the end of a sublayer goes with the product that opens the next one, from one of two residuals to the other.
+        joined = self.residual_hook is None and D == cfg.width_p and ops.joins_rms(ctx, T, D)
+        other, ended = self._buf("residual2", T, D, torch.float32) if joined else None, None
         ops.embed_positions(ctx, self.w.embed, tokens, D, cfg.vocab, cfg.embed_scale, self.inv_freq, rows_at, x, h)
+
+        def linear(weight, y=None, y_f32=None, **epilogue):      # of the layer's input
+            nonlocal x, other, ended
+            if ended is None:
+                return ops.dense_linear(ctx, weight, h, y=y, y_f32=y_f32, **epilogue)
+            (delta, post, add), ended = ended, None
+            x, other = other, x
+            return ops.rms_residual_linear(ctx, other, delta, post, add, x, weight, y_f32 if y is None else y, cfg.eps, **epilogue)
+
         for i, (m, ff) in enumerate(cfg.layers):
             w = self.w.layers[i]
             left = (ff is not None) + (cfg.side > 0)         # sublayers of this layer still to come
 
             def close(delta, weight, add):           # the end of a sublayer; behind the model's last one the final norm (in the head's type)
+                nonlocal ended
                 if i + 1 == len(cfg.layers) and left == 0:
                     ops.rms_residual(self.ctx, x, D, delta, weight, add, self.w.final_norm, 1.0, last, cfg.eps)
+                elif joined:
+                    ended = delta, weight, add
                 else:
                     ops.rms_residual(ctx, x, D, delta, weight, add, out=h, eps=cfg.eps)
-            close(self._mix(ctx, i, h, rows_at), w["norm1"], 1.0)
+            close(self._mix(ctx, i, linear, T, rows_at), w["norm1"], 1.0)
             if ff is not None:
                 left -= 1
-                act = ops.dense_linear(ctx, w["gate_up"], h, y=self._buf("ff", T, w["down"].shape[1], ctx.dtype), activation=ops.LINEAR_SILU_PAIRS)
+                act = linear(w["gate_up"], y=self._buf("ff", T, w["down"].shape[1], ctx.dtype), activation=ops.LINEAR_SILU_PAIRS)
                 close(ops.dense_linear(ctx, w["down"], act, y_f32=self._buf("delta", T, cfg.width_p, torch.float32)), w["norm2"], 1.0)
             if cfg.side:
                 left -= 1
-                g = ops.dense_linear(ctx, w["side_gate"], h, y=self._buf("side", T, w["side_proj"].shape[1], ctx.dtype),
-                                     activation=ops.LINEAR_GELU_TANH, mul=w["side_embed"], mul_ids=tokens)
+                g = linear(w["side_gate"], y=self._buf("side", T, w["side_proj"].shape[1], ctx.dtype), activation=ops.LINEAR_GELU_TANH, mul=w["side_embed"],
+                           mul_ids=tokens)
                 close(ops.dense_linear(ctx, w["side_proj"], g, y_f32=self._buf("delta", T, cfg.width_p, torch.float32)), w["side_norm"], 0.0)
             if self.residual_hook is not None:
                 self.residual_hook(i, x)

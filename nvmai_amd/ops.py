@@ -1143,6 +1143,21 @@ def rms_residual(ctx, x, d, delta=None, post=None, post_add=0.0, next_norm=None,
     return out
 
 
+def joins_rms(ctx, rows, k):
+    """Whether rms_residual_linear takes the rows."""
+    return ctx.act == ACT_FP32 and rows <= 2 and k <= 2048
+
+
+def rms_residual_linear(ctx, x, delta, post, post_add, x_out, weight, y, eps=1e-6, activation=LINEAR_NONE, bias=None, mul=None, mul_ids=None):
+    """x_out = x + RMS(delta) * (post_add + post), then dense_linear of x_out, in one launch (32-bit contexts, joins_rms)."""
+    n, k = weight.shape
+    e = LinearEpilogue(activation, _ptr(bias), _ptr(mul), _ptr(mul_ids), 0 if mul is None else mul.stride(0), 0 if mul is None else mul.shape[0])
+    check(lib.nvmai_hip_rms_residual_linear(ctx.handle, _stream(), _ptr(x), x.stride(0), _ptr(delta), delta.stride(0), _ptr(post), post_add, eps, _ptr(x_out),
+                                            x_out.stride(0), _ptr(weight), weight.stride(0), x.shape[0], n, k, _ptr(y), y.stride(0), C.byref(e)),
+          "rms_residual_linear")
+    return y
+
+
 def embed_rows(ctx, table, token_ids, d, vocab, out):
     """Rows of a BF16 table as 32-bit residual rows."""
     check(lib.nvmai_hip_embed_rows(ctx.handle, _stream(), _ptr(table), table.stride(0), _ptr(token_ids), token_ids.numel(),

@@ -105,6 +105,38 @@ def test_rms_norms_over_the_residual(dtype, d, stride):
             assert (out[:, d:] == 7.0).all()
 
 
+@pytest.mark.parametrize("rows", [1, 2])
+@pytest.mark.parametrize("k", [64, 512, 1024, 1088, 1984, 2048])
+@pytest.mark.parametrize("n", [1, 6, 257, 9000])
+def test_the_end_of_a_sublayer_with_the_next_product(rows, k, n):
+    import nvmai_amd as nv
+    ctx, eps = context("float32"), 1e-3
+    w, post, bias = bf(randn(1, n, k, std=k ** -0.5)), bf(randn(2, k)), bf(randn(3, n))
+    table, ids = bf(randn(4, 7, n)), torch.tensor([6, 9], dtype=torch.int32, device="cuda")[:rows]
+    x, delta = randn(5, rows, k + 8), randn(6, rows, k + 4, std=3.0)
+    say("rms_residual_linear", rows, k, n)
+    rows_in = f64(x)[:, :k] + K.rms(f64(delta)[:, :k], eps) * (1.0 + f64(post))
+    base = rows_in @ f64(w).T
+    mul = np.where((f64(ids) < 7)[:, None], f64(table)[np.minimum(ids.cpu().numpy(), 6)], 0.0)
+    for kw, want in [(dict(), base), (dict(bias=bias), base + f64(bias)),
+                     (dict(activation=nv.LINEAR_GELU_TANH, mul=table, mul_ids=ids), K.gelu_tanh(base) * mul),
+                     (dict(activation=nv.LINEAR_SILU_PAIRS), K.silu(base[:, 0:n - n % 2:2]) * base[:, 1::2])]:
+        pairs = "activation" in kw and "mul" not in kw
+        if pairs and n % 2:
+            continue
+        out, y = torch.full((rows, k + 4), 7.0, device="cuda"), torch.full((rows, n + n % 2 + 2), 7.0, device="cuda")
+        old = x.clone()
+        nv.ops.rms_residual_linear(ctx, x[:, :k], delta[:, :k], post, 1.0, out, w, y, eps, **kw)
+        close(f64(out)[:, :k], rows_in, 1e-6, "residual")
+        m = want.shape[1]
+        close(f64(y)[:, :m], want, 3e-6, "product", least=1.0)             # sums of terms whose squares add up to about one
+        assert (out[:, k:] == 7.0).all() and (y[:, m:] == 7.0).all() and torch.equal(x, old)
+    with pytest.raises(nv.NvmaiError):
+        nv.ops.rms_residual_linear(ctx, x[:, :k], delta[:, :k], post, 1.0, x, w, y, eps)
+    with pytest.raises(nv.NvmaiError):
+        nv.ops.rms_residual_linear(context("bfloat16"), x[:, :k], delta[:, :k], post, 1.0, out, w, y, eps)
+
+
 @pytest.mark.parametrize("dtype", TYPES)
 @pytest.mark.parametrize("width", [1, 5, 72, 700])
 def test_embeddings_with_sinusoids(dtype, width):
