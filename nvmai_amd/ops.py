@@ -19,11 +19,15 @@ _ACT_TORCH = {ACT_BF16: torch.bfloat16, ACT_FP16: torch.float16, ACT_FP32: torch
 
 
 def _ptr(t):
-    return None if t is None else C.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current stream of the current device.  torch.cuda.current_stream() makes a Stream object of it by way of a dozen Python
+    calls, a third of what a call here takes on the host; until the first CUDA call of a process it also sets the device up."""
+    if torch.cuda.is_initialized():
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return torch.cuda.current_stream().cuda_stream
 
 
 class Context:
