@@ -357,54 +357,117 @@ __global__ __launch_bounds__(256) void dense_gemv_rms_kernel(DenseLinearParams p
     }
 }
 
+// Every read of LDS done, all but the last N requests landed, for every wave of the block.
+template <int N>
+__device__ __forceinline__ void dense_stage_barrier() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"(N) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#endif
+}
+
+// All but this wave's last N requests have landed.
+template <int N>
+__device__ __forceinline__ void dense_landed() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#endif
+}
+
+// This wave's reads of LDS are done.
+__device__ __forceinline__ void dense_read() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#endif
+}
+
 // ---- 5 .. 64 input rows: 16 NR weight rows per block, the waves split k, MFMA, sums through LDS ---------
-// Weight rows are the A operand as they lie in memory: lane (i = lane % 16, g = lane / 16) loads the 32 bytes
-// W[r0 + i, k + 16 g .. + 16), four lanes cover 128 contiguous bytes of a row; the inputs are the B operand in
-// the same order of k, read from L2 once per NR row tiles.
+// Steps of 64 k go round the NW waves, and every wave has a ring of S steps of its own in LDS: weights and inputs are requested in whole
+// lines of 128 bytes and read back as operands (no barrier: a wave waits for its own requests alone).  Requested as operands, which is
+// sixteen rows by lane, a load costs the address unit a cycle per lane, and that was what it took.  16 rows: 2048 x 8192 18 -> 13.3 us, 8192 x 2048
+// 10.1 -> 9.6, 2048 x 2048 6.0 -> 4.2, 1024 x 4096 9.5 -> 5.2, 49,664 x 2048 49 -> 44 (4.6 TB/s).  A line's pieces of 16 bytes lie in the order piece ^ (row / 2 % 8): the sixteen lanes that a read serves at once cover 256
+// bytes.  Stages are arrays of their own, so that a read does not wait for the requests behind it.
+constexpr int skinny_stages(int tt, int nr, int nw) {
+    return nw * (nr + tt) * 2048 * 4 <= 128 * 1024 ? 4 : nw * (nr + tt) * 2048 * 3 <= 144 * 1024 ? 3 : 2;
+}
+
 template <int EPI, int TT, int NR, int NW>
 __global__ __launch_bounds__(64 * NW) void dense_skinny_kernel(DenseLinearParams p) {
-    __shared__ __attribute__((aligned(16))) float part[NW - 1][64][TT * NR * 4];
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, i = lane & 15u, g = lane >> 4;
+    constexpr int S = skinny_stages(TT, NR, NW), L = 2 * (NR + TT);         // 1 KB requests per step
+    constexpr uint32_t STEP = L * 1024u;
+    static_assert((NW - 1) * TT * NR <= NW * L, "one stage holds the sums");
+    __shared__ __attribute__((aligned(1024))) uint8_t l0[NW * STEP], l1[NW * STEP], l2[S > 2 ? NW * STEP : 16], l3[S > 3 ? NW * STEP : 16];
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i = lane & 15u, g = lane >> 4;
     const uint32_t r0 = blockIdx.x * (16u * NR);
-    const uint16_t* wp[NR];
+    const uint32_t steps = p.k / 64u, count = steps > wave ? (steps - wave + NW - 1u) / NW : 0u;
+    [[maybe_unused]] const uint32_t w_bytes = (p.n - 1u) * p.w_stride * 2u + p.k * 2u, x_bytes = (p.rows - 1u) * p.x_stride * 2u + p.k * 2u;
+    auto buf = [&](int j) -> uint8_t* { return (j == 0 ? l0 : j == 1 ? l1 : j == 2 ? l2 : l3) + wave * STEP; };
+    // request q: rows 8 q .. 8 q + 7 of the weights' 16 NR, then of the inputs' 16 TT (rows past the last: the last one, whose sums are not stored)
+    const uint32_t lr = lane >> 3;
+    uint32_t off[L];
 #pragma unroll
-    for (int r = 0; r < NR; ++r) wp[r] = p.w + (size_t)min(r0 + 16u * r + i, p.n - 1u) * p.w_stride + g * 16u;
-    const uint16_t* x = static_cast<const uint16_t*>(p.x);
-    const uint16_t* xp[TT];
+    for (int q = 0; q < L; ++q) {
+        const uint32_t row = 8u * (q < 2 * NR ? q : q - 2 * NR) + lr, piece = ((lane & 7u) ^ ((row >> 1) & 7u)) * 16u;
+        off[q] = (q < 2 * NR ? min(r0 + row, p.n - 1u) * p.w_stride : min(row, p.rows - 1u) * p.x_stride) * 2u + piece;
+    }
+    auto request = [&](uint32_t nth, int j) {
+#if defined(__HIP_DEVICE_COMPILE__)     // the host pass rejects the 16-byte form of the load
+        const bool live = nth < count;                       // a step past the last reads no bytes
+        const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.w), 0, live ? (int)w_bytes : 0, 0x00020000);
+        const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.x), 0, live ? (int)x_bytes : 0, 0x00020000);
+        const uint32_t k = (wave + nth * NW) * 128u;
 #pragma unroll
-    for (int t = 0; t < TT; ++t) xp[t] = x + (size_t)min(16u * t + i, p.rows - 1u) * p.x_stride + g * 16u;
+        for (int q = 0; q < L; ++q)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(q < 2 * NR ? wr : xr, (__attribute__((address_space(3))) void*)(buf(j) + q * 1024u), 16, off[q], k, 0, 0);
+#endif
+    };
+    const uint32_t at0 = i * 128u + ((g ^ ((i >> 1) & 7u)) * 16u), at1 = i * 128u + (((4u + g) ^ ((i >> 1) & 7u)) * 16u);
     dn_f4 acc[NR][TT];
 #pragma unroll
     for (int r = 0; r < NR; ++r)
 #pragma unroll
         for (int t = 0; t < TT; ++t) acc[r][t] = dn_f4{0.0f, 0.0f, 0.0f, 0.0f};
-    const uint32_t steps = p.k / 64u;
-#pragma unroll 4
-    for (uint32_t st = wave; st < steps; st += NW) {
-        uint4 a0[NR], a1[NR], b0[TT], b1[TT];
+#pragma unroll
+    for (int j = 0; j < S; ++j) request(j, j);
+    auto step = [&](uint32_t nth, int j) {
+        dense_landed<(S - 1) * L>();
+        uint4 a[NR][2], b[TT][2];
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
-            a0[r] = *reinterpret_cast<const uint4*>(wp[r] + st * 64u);
-            a1[r] = *reinterpret_cast<const uint4*>(wp[r] + st * 64u + 8u);
+            a[r][0] = *reinterpret_cast<const uint4*>(buf(j) + 2048u * r + at0);
+            a[r][1] = *reinterpret_cast<const uint4*>(buf(j) + 2048u * r + at1);
         }
 #pragma unroll
         for (int t = 0; t < TT; ++t) {
-            b0[t] = *reinterpret_cast<const uint4*>(xp[t] + st * 64u);
-            b1[t] = *reinterpret_cast<const uint4*>(xp[t] + st * 64u + 8u);
+            b[t][0] = *reinterpret_cast<const uint4*>(buf(j) + 2048u * (NR + t) + at0);
+            b[t][1] = *reinterpret_cast<const uint4*>(buf(j) + 2048u * (NR + t) + at1);
         }
+        dense_read();                                        // the operands are in registers: the place is free
+        request(nth + S, j);
 #pragma unroll
-        for (int r = 0; r < NR; ++r)
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int t = 0; t < TT; ++t) {
-                acc[r][t] = dn_mfma(a0[r], b0[t], acc[r][t]);
-                acc[r][t] = dn_mfma(a1[r], b1[t], acc[r][t]);
-            }
+            for (int r = 0; r < NR; ++r)
+#pragma unroll
+                for (int t = 0; t < TT; ++t) acc[r][t] = dn_mfma(a[r][h], b[t][h], acc[r][t]);
+    };
+    uint32_t nth = 0;
+    for (; nth + (uint32_t)S <= count; nth += S) {
+#pragma unroll
+        for (int j = 0; j < S; ++j) step(nth + j, j);
     }
+#pragma unroll
+    for (int j = 0; j < S - 1; ++j)
+        if (nth + (uint32_t)j < count) step(nth + j, j);
+    dense_stage_barrier<0>();                                // no request outlives its wave, and no other wave reads its places any more
+    float* part = reinterpret_cast<float*>(l0);
     if (wave != 0) {
 #pragma unroll
         for (int r = 0; r < NR; ++r)
 #pragma unroll
-            for (int t = 0; t < TT; ++t) *reinterpret_cast<dn_f4*>(&part[wave - 1][lane][4 * (r * TT + t)]) = acc[r][t];
+            for (int t = 0; t < TT; ++t) *reinterpret_cast<dn_f4*>(part + (((wave - 1u) * (NR * TT) + r * TT + t) * 64u + lane) * 4u) = acc[r][t];
     }
     __syncthreads();
     if (wave != 0) return;
@@ -413,7 +476,7 @@ __global__ __launch_bounds__(64 * NW) void dense_skinny_kernel(DenseLinearParams
 #pragma unroll
         for (int t = 0; t < TT; ++t) {
 #pragma unroll
-            for (int w = 0; w < NW - 1; ++w) acc[r][t] += *reinterpret_cast<const dn_f4*>(&part[w][lane][4 * (r * TT + t)]);
+            for (int w = 0; w < NW - 1; ++w) acc[r][t] += *reinterpret_cast<const dn_f4*>(part + ((w * (NR * TT) + r * TT + t) * 64u + lane) * 4u);
             // acc[r][t][j] = y[token 16 t + i, row r0 + 16 r + 4 g + j]
             if (16u * t + i < p.rows) dense_store4<EPI, ACT_BF16>(p, 16u * t + i, r0 + 16u * r + 4u * g, acc[r][t], dense_bias4<EPI>(p, r0 + 16u * r + 4u * g));
         }
@@ -440,15 +503,6 @@ typedef float dn_f16 __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ dn_f16 dn_mfma32(const uint4& a, const uint4& b, dn_f16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(dn_b8, a), __builtin_bit_cast(dn_b8, b), c, 0, 0, 0);
-}
-
-// Every read of LDS done, all but the last N requests landed, for every wave of the block.
-template <int N>
-__device__ __forceinline__ void dense_stage_barrier() {
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"(N) : "memory");
-    __builtin_amdgcn_sched_barrier(0);
-#endif
 }
 
 // One sum of the planes again by a whole wave, in fp32 multiply-adds of the values that the planes stand for.  An infinite weight makes
@@ -989,21 +1043,25 @@ int dense_launch(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p) 
         return launch_status();
     }
     if (p.rows <= 64) {
-        // row tiles per block: as many as leave every compute unit several blocks; waves: about four steps of k each
-        const int nr = p.n >= 32768 ? 4 : p.n >= 8192 ? 2 : 1;
-        const uint32_t blocks = (p.n + 16 * nr - 1) / (16 * nr);
-#define NVMAI_SKINNY(TT)                                                              \
-    do {                                                                              \
-        if (nr == 4) dense_skinny_kernel<EPI, TT, 4, 4><<<blocks, 256, 0, s>>>(p);         \
-        else if (nr == 2) dense_skinny_kernel<EPI, TT, 2, 4><<<blocks, 256, 0, s>>>(p);    \
-        else if (p.k <= 1024) dense_skinny_kernel<EPI, TT, 1, 4><<<blocks, 256, 0, s>>>(p); \
-        else if (p.k <= 2048) dense_skinny_kernel<EPI, TT, 1, 8><<<blocks, 512, 0, s>>>(p); \
-        else dense_skinny_kernel<EPI, TT, 1, 16><<<blocks, 1024, 0, s>>>(p);               \
-    } while (0)
-        if (p.rows <= 16) NVMAI_SKINNY(1);
-        else if (p.rows <= 32) NVMAI_SKINNY(2);
-        else NVMAI_SKINNY(4);
-#undef NVMAI_SKINNY
+        // Two waves leave room for several blocks per compute unit; four where a row is long and the blocks are few (16 rows: 2048 x 8192 14.0
+        // and 13.3 us, 1024 x 4096 5.5 and 5.2, 2048 x 2048 4.2 and 4.3).  Several row tiles per block where the inputs, which every
+        // block reads, would weigh more than its weights (32 rows: 8192 x 2048 11.5 -> 10.0 us; 64: 14.5 -> 12.3, 49,664 x 2048 83 -> 65 with four).
+        auto launch = [&](auto tt, auto nr, auto nw) {
+            constexpr int TT = decltype(tt)::value, NR = decltype(nr)::value, NW = decltype(nw)::value;
+            dense_skinny_kernel<EPI, TT, NR, NW><<<(p.n + 16 * NR - 1) / (16 * NR), 64 * NW, 0, s>>>(p);
+        };
+        constexpr std::integral_constant<int, 1> one{};
+        constexpr std::integral_constant<int, 2> two{};
+        constexpr std::integral_constant<int, 4> four{};
+        if (p.rows <= 16) {
+            if (p.k <= 2048) launch(one, one, two);
+            else launch(one, one, four);
+        } else if (p.rows <= 32) {
+            if (p.n < 8192) launch(two, one, two);
+            else launch(two, two, two);
+        } else if (p.n < 8192) launch(four, one, two);
+        else if (p.n < 32768) launch(four, two, two);
+        else launch(four, four, four);
         return launch_status();
     }
     launch_tiles<EPI, ACT_BF16>(ctx, s, p);
