@@ -259,7 +259,7 @@ extern "C" int nvmai_hip_prefill_grouped_moe(nvmai_hip_ctx* ctx, nvmai_stream st
     MTile* mtiles = ws_take<MTile>(ctx, (size_t)GEMM_XCDS * max_mtiles);
     uint32_t* qwords = ws_take<uint32_t>(ctx, GEMM_XCDS);   // list lengths
     hipStream_t s = (hipStream_t)stream;
-    prefill_mtiles_kernel<<<1, 256, 0, s>>>(reinterpret_cast<const PrefillGroup*>(grouping->groups), grouping->info,
+    prefill_mtiles_kernel<<<1, MTILES_THREADS, 0, s>>>(reinterpret_cast<const PrefillGroup*>(grouping->groups), grouping->info,
                                             mtiles, max_mtiles, grouped_list_max(max_mtiles), qwords,
                                             reinterpret_cast<uint4*>(route_partials),
                                             n_pairs * d * 2 / 16);

@@ -241,6 +241,15 @@ def test_reduce_token_major_rank_order(nv, ctx):
     assert torch.equal(h2.cpu(), want.cpu())
 
 
+# the work lists: experts on both sides of the 256 items that one pass ranks, of a whole and of a partial row of eight, one very
+# popular expert cut into many items (3000 tokens of one choice: 2 experts, 24 M tiles), and more experts than a list's first scan
+@pytest.mark.parametrize("E,k,tokens", [(2, 1, 3000), (7, 2, 300), (255, 4, 700), (259, 4, 700), (600, 4, 900)])
+def test_grouped_moe_work_lists(nv, ctx_bf16, E, k, tokens):
+    say("prefill work lists", E, k, tokens)
+    rng = np.random.default_rng(E * 7 + tokens)
+    _prefill_case(nv, ctx_bf16, rng, 128, 64, E, k, 4, tokens, check_tokens=np.arange(0, tokens, max(1, tokens // 64)))
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 def test_grouped_moe_production_shape(nv, ctx_bf16, bits):
     say("prefill grouped moe production", bits)
