@@ -29,13 +29,24 @@ int raise_lds(const void* kernel, size_t bytes) {
     return NVMAI_OK;
 }
 
+// Whether the rows of the cache go through LDS to the matrix cores.
+bool latent_staged(bool cache32, uint32_t rank, uint32_t row_stride) { return !cache32 && rank <= 1024 && row_stride - rank <= 128; }
+
 template <int NT>
 int launch_partial(const LatentAttnParams& p, hipStream_t s) {
-    const size_t lds = (size_t)p.rank * 80;
-    const int rc = raise_lds(reinterpret_cast<const void*>(latent_partial_mfma_kernel<NT>), lds);
-    if (rc) return rc;
-    latent_partial_mfma_kernel<NT><<<dim3(p.splits, (p.heads + 15) / 16, p.n_rows), 256, lds, s>>>(p);
+    latent_partial_mfma_kernel<NT><<<dim3(p.splits, (p.heads + 15) / 16, p.n_rows), 256, 0, s>>>(p);
     return NVMAI_OK;
+}
+
+// How many splits of `most`: of the form through LDS one block per compute unit is resident, so the fewest whose rounds per split are not
+// a tenth above the least (16 rows of 4096 keys: 16 splits 23.7 us and 8.5 to combine them).
+uint32_t latent_splits(uint32_t blocks, uint32_t cus, uint32_t most) {
+    uint32_t best = 1, best_rounds = (blocks + cus - 1) / cus;
+    for (uint32_t n = 2; n <= most; ++n) {
+        const uint32_t rounds = (uint32_t)(((uint64_t)blocks * n + cus - 1) / cus);
+        if ((uint64_t)rounds * best * 10 < (uint64_t)best_rounds * n * 9) { best = n; best_rounds = rounds; }
+    }
+    return best;
 }
 
 template <int ACT, int CT>
@@ -44,8 +55,7 @@ int absorbed(const LatentAttnParams& p, hipStream_t s) {
     int rc = raise_lds(reinterpret_cast<const void*>(latent_absorb_kernel<ACT, CT>), lds_a);
     if (rc) return rc;
     latent_absorb_kernel<ACT, CT><<<dim3(p.heads, p.n_rows, (p.rank + 127) / 128 + 1), 256, lds_a, s>>>(p);
-    const uint32_t rest = p.cache.row_stride - p.rank;
-    if (CT == ACT_BF16 && p.rank <= 1024 && rest <= 128) {
+    if (latent_staged(CT == ACT_FP32, p.rank, p.cache.row_stride)) {
         rc = p.rank <= 128 ? launch_partial<2>(p, s) : p.rank <= 256 ? launch_partial<4>(p, s) : p.rank <= 512 ? launch_partial<8>(p, s) : launch_partial<16>(p, s);
     } else {
         const size_t lds = ((size_t)p.cache.row_stride + p.rank + 256 + 8) * 4;
@@ -156,13 +166,15 @@ extern "C" int nvmai_hip_latent_attention(nvmai_hip_ctx* ctx, nvmai_stream strea
     if (!expand) {
         uint32_t keys = known ? last : cache->capacity;
         if (c.window && c.window < keys) keys = c.window;
-        // about two blocks per compute unit, at least 32 keys each
-        const uint32_t groups = cache32 ? c.heads : (c.heads + 15) / 16;
-        const uint32_t want = 2u * (uint32_t)ctx->compute_units / (rows * groups) + 1u;
-        const uint32_t per = ((keys + want - 1) / want + 31) / 32 * 32;
-        p.split_keys = per;
-        p.splits = (keys + per - 1) / per;
-        const size_t cells = (size_t)rows * c.heads * p.splits, n_qa = (size_t)rows * c.heads * cache->row_stride;
+        // about two blocks per compute unit, or one of those that fill it; at least 32 keys each
+        const uint32_t groups = cache32 ? c.heads : (c.heads + 15) / 16, cus = (uint32_t)ctx->compute_units;
+        const uint32_t most = 2u * cus / (rows * groups) + 1u;
+        const uint32_t want = latent_staged(cache32, c.rank, cache->row_stride) ? latent_splits(rows * groups, cus, most) : most;
+        auto keys_per = [&](uint32_t n) { return ((keys + n - 1) / n + 31) / 32 * 32; };
+        p.split_keys = keys_per(want);
+        p.splits = (keys + p.split_keys - 1) / p.split_keys;
+        // room for the most splits: a call of few rows then needs no more than one of many rows before it
+        const size_t cells = (size_t)rows * c.heads * ((keys + keys_per(most) - 1) / keys_per(most)), n_qa = (size_t)rows * c.heads * cache->row_stride;
         rc = ws_begin(ctx, stream, ws_round(n_qa * esz) + ws_round(cells * c.rank * 4) + 2 * ws_round(cells * 4));
         if (rc) return rc;
         p.qa = ws_take<uint8_t>(ctx, n_qa * esz);

@@ -23,6 +23,33 @@ __device__ __forceinline__ la_f4 la_mfma(const uint4& a, const uint4& b, la_f4 c
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(la_b8, a), __builtin_bit_cast(la_b8, b), c, 0, 0, 0);
 }
 
+// Every read of LDS done, all but the last N requests landed, for every wave of the block.
+template <int N>
+__device__ __forceinline__ void la_stage_barrier() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"(N) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#endif
+}
+
+// The reads and writes of LDS done for every wave of the block; requests from memory stay on their way.
+__device__ __forceinline__ void la_lds_barrier() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#endif
+}
+
+// Four rows of sixteen 16-bit values per sixteen lanes, lane t at value 4 (t % 4) of row t / 4: lane t gets value t of every row.
+__device__ __forceinline__ uint2 la_read_transposed(const uint8_t* lds) {
+    uint2 r{};
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef short s4 __attribute__((ext_vector_type(4)));
+    r = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4*)lds));
+#endif
+    return r;
+}
+
 // Two floats rounded to BF16 (nearest even) in one dword: one hardware conversion.
 typedef float la_f2 __attribute__((ext_vector_type(2)));
 typedef __bf16 la_b2 __attribute__((ext_vector_type(2)));
@@ -232,62 +259,97 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(LatentAttnParams p) 
 }
 
 // ---- absorbed: scores and sums over one split of the window, sixteen heads per block --------------------
-// Per 32 keys: S^T[key, head] = K Q^T with the waves splitting the row's elements (cache rows are the A operand as
-// they lie in memory), the partial scores summed through LDS, the softmax in registers, and
-// O^T[latent, head] += C^T P^T with the waves splitting the latent.  C^T comes from LDS: a thread transposes four
-// keys x eight latents on the way in.  The score registers of a lane are the B operand of the second product when
-// its eight keys are read as 4 g .. 4 g + 3 and 16 + 4 g .. 16 + 4 g + 3, so the columns of C^T lie in that order.
-// P enters as two BF16 halves (hi + lo): fp32 weights.
+// Bound by the bytes of the cached rows.  A stage is 32 keys, which lie one behind the other in memory: their rows go to LDS in whole lines, once, and a ring of
+// stages keeps the next ones on their way.  S^T[key, head] = K Q^T with the waves splitting the row's elements, the partial scores summed
+// through LDS, the softmax in registers, and O^T[latent, head] += C^T P^T with the waves splitting the latent; C^T is read out of the same rows by
+// transposing reads.  The score registers of a lane are the B operand of the second product when its eight keys are
+// read as 4 g .. 4 g + 3 and 16 + 4 g .. 16 + 4 g + 3.  P enters as two BF16 halves (hi + lo): fp32 weights.
+// A row's pieces of 16 bytes lie in the order piece ^ swizzle(row): sixteen rows read at one piece then cover 256 bytes.  A stage ends
+// with the split and at the end of the ring; rows past it, and stages past the last, are filled with zeros.
+// 16 sequences x 4096 keys of 1152 bytes, 16 heads: 31.3 -> 23.7 us (3.2 TB/s of rows with the launch; every row was loaded twice, once by sixteen rows a
+// lane apart, transposed in registers, and nothing was on its way while a tile was worked on), and half as many splits to combine: 9.6 -> 8.5.
+constexpr int latent_stages(int nt) { return nt <= 8 ? 3 : 2; }          // of 160 KB, one block per compute unit
+
 template <int NT>
-__global__ __launch_bounds__(256) void latent_partial_mfma_kernel(LatentAttnParams p) {
+__global__ __launch_bounds__(256, 1) void latent_partial_mfma_kernel(LatentAttnParams p) {
     constexpr int NQ = (2 * NT + 7) / 4;             // 32-element steps of a row per wave: rank <= 64 NT, rest <= 128
-    constexpr int NV = (NT + 3) / 4;                 // transposed units per thread
-    extern __shared__ __attribute__((aligned(16))) float la_lds[];
-    uint16_t* ct = reinterpret_cast<uint16_t*>(la_lds);      // [rank][40]: 32 keys, rows 16 bytes off a power of two
+    constexpr int S = latent_stages(NT), L = NT + 2; // 1 KB requests per wave and stage
+    constexpr uint32_t STAGE = 4096u * L;
+    __shared__ __attribute__((aligned(1024))) uint8_t l0[STAGE], l1[STAGE], l2[S > 2 ? STAGE : 16];
     __shared__ __attribute__((aligned(16))) float sc[4][16][36];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, i = lane & 15u, g = lane >> 4;
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i = lane & 15u, g = lane >> 4;
     const uint32_t split = blockIdx.x, h0 = blockIdx.y * 16u, row = blockIdx.z;
-    const uint32_t position = p.rows.position_of(row), first = first_key(position, p.window);
+    const uint32_t position = __builtin_amdgcn_readfirstlane(p.rows.position_of(row)), first = first_key(position, p.window);
     const uint32_t lo = first + split * p.split_keys, hi = min(position + 1u, lo + p.split_keys);
     const uint32_t head = min(h0 + i, p.heads - 1u);
     const size_t cell = ((size_t)row * p.heads + head) * p.splits + split;
     if (lo >= hi) {                                  // uniform
-        if (tid < 16u && h0 + tid < p.heads) { p.part_m[cell] = LA_NONE; p.part_l[cell] = 0.0f; }
+        if (threadIdx.x < 16u && h0 + threadIdx.x < p.heads) { p.part_m[cell] = LA_NONE; p.part_l[cell] = 0.0f; }
         return;
     }
-    const uint32_t rs = p.cache.row_stride, steps = rs / 32u, tiles = p.rank / 16u;
-    const uint16_t* cache = static_cast<const uint16_t*>(p.cache.base) + (size_t)p.rows.slot_of(row) * p.cache.slot_stride;
+    const uint32_t rs = p.cache.row_stride, steps = rs / 32u, tiles = p.rank / 16u, pitch = rs * 2u, pieces = rs / 8u;
+    const uint32_t shift = pieces % 8u ? 2u : 1u, mask = pieces % 8u ? 3u : 7u;       // pieces is a multiple of four
+    auto swizzle = [&](uint32_t r) { return (r >> shift) & mask; };
+    [[maybe_unused]] const uint16_t* cache = static_cast<const uint16_t*>(p.cache.base) + (size_t)__builtin_amdgcn_readfirstlane(p.rows.slot_of(row)) * p.cache.slot_stride;
     const uint16_t* q = static_cast<const uint16_t*>(p.qa) + ((size_t)row * p.heads + head) * rs;
     uint4 qf[NQ];
 #pragma unroll
     for (int n = 0; n < NQ; ++n) qf[n] = *reinterpret_cast<const uint4*>(q + min(wave + 4u * n, steps - 1u) * 32u + 8u * g);
+    __builtin_amdgcn_sched_barrier(0);               // ahead of the stages' requests: they are waited for one by one, in order
+    auto buf = [&](int j) -> uint8_t* { return j == 0 ? l0 : j == 1 ? l1 : l2; };
+    uint32_t off[L];                                 // what a request brings: places past the 32 rows lie behind every stage's last byte
+    {
+        uint32_t key = (wave * (L * 64u) + lane) / pieces, piece = (wave * (L * 64u) + lane) % pieces;
+        const uint32_t more_keys = 64u / pieces, more = 64u % pieces;
+#pragma unroll
+        for (int n = 0; n < L; ++n) {
+            off[n] = key * pitch + (piece ^ swizzle(key)) * 16u;
+            const bool carry = piece + more >= pieces;
+            key += more_keys + (carry ? 1u : 0u);
+            piece += more - (carry ? pieces : 0u);
+        }
+    }
+    const uint32_t cap = p.cache.capacity;
+    auto keys_of = [&](uint32_t k, uint32_t ring) { return k < hi ? min(32u, min(hi - k, cap - ring)) : 0u; };
+    uint32_t ahead = lo, ahead_ring = __builtin_amdgcn_readfirstlane(lo % cap);
+    auto request = [&](int j) {
+        const uint32_t n_keys = __builtin_amdgcn_readfirstlane(keys_of(ahead, ahead_ring));
+#if defined(__HIP_DEVICE_COMPILE__)     // the host pass rejects the 16-byte form of the load
+        const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(cache + (size_t)ahead_ring * rs), 0, (int)(n_keys * pitch), 0x00020000);
+#pragma unroll
+        for (int n = 0; n < L; ++n)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, (__attribute__((address_space(3))) void*)(buf(j) + (wave * L + n) * 1024u), 16, off[n], 0, 0, 0);
+#endif
+        ahead += n_keys;
+        ahead_ring += n_keys;
+        if (ahead_ring == cap) ahead_ring = 0;
+    };
+    uint32_t ka[NQ];                                 // the piece of step wave + 4 n in row i (row 16 + i has the same swizzle)
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) ka[n] = i * pitch + (((min(wave + 4u * n, steps - 1u) * 4u + g) ^ swizzle(i)) * 16u);
+    const uint32_t vrow = 4u * g + (i >> 2), va = vrow * pitch + (((2u * wave + ((i >> 1) & 1u)) ^ swizzle(vrow)) * 16u) + 8u * (i & 1u);
     la_f4 acc[NT];
 #pragma unroll
     for (int n = 0; n < NT; ++n) acc[n] = la_f4{0.0f, 0.0f, 0.0f, 0.0f};
     float m = LA_NONE, l = 0.0f;
-    const uint32_t units = p.rank;                   // 8 groups of four keys x rank / 8 pieces
-    for (uint32_t k0 = lo; k0 < hi; k0 += 32u) {
-        const uint32_t ring0 = k0 % p.cache.capacity, most = hi - 1u - k0;
-        auto row_of = [&](uint32_t key) {            // keys past the split repeat its last one
-            uint32_t r = ring0 + min(key, most);
-            r -= r >= p.cache.capacity ? p.cache.capacity : 0u;
-            return cache + (size_t)r * rs;
-        };
-        uint4 vv[NV][4];
+    uint32_t k0 = lo, ring = ahead_ring;
 #pragma unroll
-        for (int n = 0; n < NV; ++n) {
-            const uint32_t u = min(tid + 256u * n, units - 1u), kg = u & 7u, piece = u >> 3;
+    for (int j = 0; j < S - 1; ++j) request(j);
+#if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) vv[n][e] = *reinterpret_cast<const uint4*>(row_of(4u * kg + e) + piece * 8u);
-        }
-        const uint16_t *ka = row_of(i) + 8u * g, *kb = row_of(16u + i) + 8u * g;
+    for (int n = 0; n < NQ; ++n) asm volatile("" : "+v"(qf[n].x), "+v"(qf[n].y), "+v"(qf[n].z), "+v"(qf[n].w));    // waited for here, where the stages need not be
+#endif
+    auto stage = [&](int j) {
+        const uint32_t n_keys = keys_of(k0, ring);
+        la_stage_barrier<(S - 2) * L>();             // this stage has landed, and every wave has read the one before it to its end
+        request((j + S - 1) % S);
+        const uint8_t* at = buf(j);
         la_f4 s0 = la_f4{0.0f, 0.0f, 0.0f, 0.0f}, s1 = s0;
         uint4 fa[NQ], fb[NQ];
 #pragma unroll
         for (int n = 0; n < NQ; ++n) {
-            const uint32_t at = min(wave + 4u * n, steps - 1u) * 32u;
-            fa[n] = *reinterpret_cast<const uint4*>(ka + at);
-            fb[n] = *reinterpret_cast<const uint4*>(kb + at);
+            fa[n] = *reinterpret_cast<const uint4*>(at + ka[n]);
+            fb[n] = *reinterpret_cast<const uint4*>(at + 16u * pitch + ka[n]);
         }
 #pragma unroll
         for (int n = 0; n < NQ; ++n)
@@ -297,24 +359,7 @@ __global__ __launch_bounds__(256) void latent_partial_mfma_kernel(LatentAttnPara
             }
         *reinterpret_cast<la_f4*>(&sc[wave][i][4u * g]) = s0;
         *reinterpret_cast<la_f4*>(&sc[wave][i][16u + 4u * g]) = s1;
-#pragma unroll
-        for (int n = 0; n < NV; ++n) {
-            const uint32_t u = tid + 256u * n, kg = u & 7u, piece = u >> 3;
-            if (u < units) {
-                const uint32_t at = kg < 4u ? 8u * kg : 8u * (kg - 4u) + 4u;
-                const uint32_t a[4][4] = {{vv[n][0].x, vv[n][0].y, vv[n][0].z, vv[n][0].w}, {vv[n][1].x, vv[n][1].y, vv[n][1].z, vv[n][1].w},
-                                          {vv[n][2].x, vv[n][2].y, vv[n][2].z, vv[n][2].w}, {vv[n][3].x, vv[n][3].y, vv[n][3].z, vv[n][3].w}};
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;     // high or low halves of two dwords
-                    uint2 w;
-                    w.x = __builtin_amdgcn_perm(a[1][e >> 1], a[0][e >> 1], sel);
-                    w.y = __builtin_amdgcn_perm(a[3][e >> 1], a[2][e >> 1], sel);
-                    *reinterpret_cast<uint2*>(&ct[(piece * 8u + e) * 40u + at]) = w;
-                }
-            }
-        }
-        __syncthreads();
+        la_lds_barrier();
         float s[8];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -322,11 +367,11 @@ __global__ __launch_bounds__(256) void latent_partial_mfma_kernel(LatentAttnPara
 #pragma unroll
             for (int w = 1; w < 4; ++w) v += *reinterpret_cast<const la_f4*>(&sc[w][i][16 * h + 4u * g]);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) s[4 * h + j] = k0 + 16u * h + 4u * g + j < hi ? v[j] * p.scale_log2 : LA_NONE;
+            for (int e = 0; e < 4; ++e) s[4 * h + e] = 16u * h + 4u * g + e < n_keys ? v[e] * p.scale_log2 : LA_NONE;
         }
         float tm = s[0];
 #pragma unroll
-        for (int j = 1; j < 8; ++j) tm = fmaxf(tm, s[j]);
+        for (int e = 1; e < 8; ++e) tm = fmaxf(tm, s[e]);
         tm = fmaxf(tm, shfl_xor_f(tm, 16));
         tm = fmaxf(tm, shfl_xor_f(tm, 32));
         const float mn = fmaxf(m, tm), alpha = __builtin_amdgcn_exp2f(m - mn);
@@ -334,11 +379,11 @@ __global__ __launch_bounds__(256) void latent_partial_mfma_kernel(LatentAttnPara
         float ts = 0.0f;
         uint16_t ph[8], pl[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float e = s[j] > LA_NONE ? __builtin_amdgcn_exp2f(s[j] - mn) : 0.0f;
+        for (int j8 = 0; j8 < 8; ++j8) {
+            const float e = s[j8] > LA_NONE ? __builtin_amdgcn_exp2f(s[j8] - mn) : 0.0f;
             ts += e;
-            ph[j] = f32_to_bf16(e);
-            pl[j] = f32_to_bf16(e - bf16_to_f32(ph[j]));
+            ph[j8] = f32_to_bf16(e);
+            pl[j8] = f32_to_bf16(e - bf16_to_f32(ph[j8]));
         }
         ts += shfl_xor_f(ts, 16);
         ts += shfl_xor_f(ts, 32);
@@ -349,17 +394,24 @@ __global__ __launch_bounds__(256) void latent_partial_mfma_kernel(LatentAttnPara
         bl.x = pl[0] | ((uint32_t)pl[1] << 16); bl.y = pl[2] | ((uint32_t)pl[3] << 16);
         bl.z = pl[4] | ((uint32_t)pl[5] << 16); bl.w = pl[6] | ((uint32_t)pl[7] << 16);
 #pragma unroll
-        for (int n = 0; n < NT; ++n) {
-            const uint32_t tile = wave + 4u * n;
-            if (tile < tiles) {                      // uniform
-                const uint4 a = *reinterpret_cast<const uint4*>(&ct[(16u * tile + i) * 40u + 8u * g]);
-                acc[n] *= alpha;
-                acc[n] = la_mfma(a, bh, acc[n]);
-                acc[n] = la_mfma(a, bl, acc[n]);
-            }
+        for (int n = 0; n < NT; ++n) {               // tiles past the rank: other values of the stage, sums that are not stored
+            const uint2 a0 = la_read_transposed(at + va + 128u * n), a1 = la_read_transposed(at + 16u * pitch + va + 128u * n);
+            const uint4 a = {a0.x, a0.y, a1.x, a1.y};
+            acc[n] *= alpha;
+            acc[n] = la_mfma(a, bh, acc[n]);
+            acc[n] = la_mfma(a, bl, acc[n]);
         }
-        __syncthreads();
+        k0 += n_keys;
+        ring += n_keys;
+        if (ring == cap) ring = 0;
+        return k0 < hi;
+    };
+    for (bool more = true; more;) {
+#pragma unroll
+        for (int j = 0; j < S; ++j)
+            if (more) more = stage(j);
     }
+    la_stage_barrier<0>();                           // no request outlives its block
     if (h0 + i >= p.heads) return;
 #pragma unroll
     for (int n = 0; n < NT; ++n) {

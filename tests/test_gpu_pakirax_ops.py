@@ -358,6 +358,18 @@ def test_latent_ring_wraps_and_slots_are_reused(ctx):
         L.run([61], nv.FORM_AUTO, base=100)         # window + 60 rows do not fit the ring
 
 
+@pytest.mark.parametrize("heads,rot,rank", [(2, 16, 64), (17, 32, 192), (3, 128, 256), (2, 64, 512), (2, 48, 576), (1, 128, 1024)])
+def test_latent_splits_of_several_stages_over_the_end_of_the_ring(ctx, heads, rot, rank):
+    """Portions whose rows fill the device, so that one split holds a window of several stages of 32 keys: every size of the stages in LDS,
+    rows of an odd number of 64 bytes, a ring that ends inside a stage, windows that end inside one."""
+    say("latent stages", ctx.dtype, heads, rot, rank)
+    rng = np.random.default_rng(rank + rot)
+    window, n = 203, 700
+    L = Latent(ctx, rng, heads, 32, rot, 32, rank, window, n, capacity=window + 250 - 1)
+    got = L.run([250, 250, 200], FORMS["absorbed"])
+    check_latent(ctx, L, got, [0, 1, 31, 32, 33, 202, 203, 249, 250, 451, 452, 453, 480, 500, 655, 699])
+
+
 def test_latent_positions_far_along_and_partial_rotation(ctx):
     """Large positions (the angle is reduced in double) and a rotation of a part of the rope dims."""
     rng = np.random.default_rng(31)
