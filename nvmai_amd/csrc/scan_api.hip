@@ -46,8 +46,22 @@ void filter(const ScanParams& p, hipStream_t s) {
     else scan_filter_kernel<DELTA, 4, TAPS, FAST><<<grid, 256, 0, s>>>(p);
 }
 
+// Heads of one block of the preparation: it makes k k^T and q k^T once for all of them, which takes as long as one head of the delta rule or four of
+// the state-space form, and two blocks fit a compute unit.  Many heads where the blocks are many, few where units would be idle (us for 5, 24
+// and 32 chunks; delta rule, 16 key heads of 2: one head per block 26, 56 and 64, two 39, 48 and 53; state-space, one group of 64: 1 11.6, 27 and 33, 4 15.8, 18.9 and 19.1, 8 25, 26 and 26).
+uint32_t prep_heads(bool delta, uint32_t chunks, uint32_t key_heads, uint32_t ratio, uint32_t slots) {
+    uint32_t best = 1;
+    uint64_t least = ~0ull;
+    for (uint32_t per = 1; per <= ratio && per <= 8; ++per) {
+        const uint64_t blocks = (uint64_t)chunks * key_heads * ((ratio + per - 1) / per);
+        const uint64_t cost = (blocks + slots - 1) / slots * ((delta ? 1 : 4) + per);
+        if (cost < least) { least = cost; best = per; }
+    }
+    return best;
+}
+
 template <bool DELTA>
-int chunked(const ScanParams& p, uint32_t chunks, bool fast, hipStream_t s) {
+int chunked(const ScanParams& p, uint32_t chunks, bool fast, uint32_t cus, hipStream_t s) {
     const size_t q_part = (size_t)64 * (p.dk + 4), l_part = DELTA ? 64 * 68 : 0, lds = (q_part + (q_part > l_part ? q_part : l_part)) * 4;
     if (lds > 159 * 1024) return NVMAI_ERR_UNSUPPORTED;
     if (lds > 63 * 1024) NVMAI_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(scan_prep_kernel<DELTA>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -55,8 +69,7 @@ int chunked(const ScanParams& p, uint32_t chunks, bool fast, hipStream_t s) {
     else if (fast) filter<DELTA, 4, true>(p, s);
     else filter<DELTA, 4, false>(p, s);
     if (p.taps > 1) scan_history_kernel<<<dim3((p.channels + 255) / 256, p.taps - 1), 256, 0, s>>>(p);
-    // heads of one block: the state-space form shares q k^T among the heads of a group
-    const uint32_t ratio = p.heads / p.key_heads, per = DELTA ? 1 : ratio < 8 ? ratio : 8;
+    const uint32_t ratio = p.heads / p.key_heads, per = prep_heads(DELTA, chunks, p.key_heads, ratio, 2 * cus);
     scan_prep_kernel<DELTA><<<dim3(chunks, p.key_heads * ((ratio + per - 1) / per)), 256, lds, s>>>(p, per);
     const dim3 grid(p.heads, p.dv / 16);
     if (p.dk <= 64) scan_chain_kernel<DELTA, 4, 2><<<grid, 512, 0, s>>>(p, chunks);
@@ -122,7 +135,7 @@ extern "C" int nvmai_hip_scan(nvmai_hip_ctx* ctx, nvmai_stream stream, const nvm
     p.u0 = ws_take<float>(ctx, n_u0);
     p.k_t = ws_take<float>(ctx, n_k);
     const bool fast = ctx->act != NVMAI_ACT_FP32;    // the filter's activation by the hardware exponential (1e-6)
-    return delta ? chunked<true>(p, chunks, fast, s) : chunked<false>(p, chunks, fast, s);
+    return delta ? chunked<true>(p, chunks, fast, (uint32_t)ctx->compute_units, s) : chunked<false>(p, chunks, fast, (uint32_t)ctx->compute_units, s);
 }
 
 extern "C" int nvmai_hip_gated_norm(nvmai_hip_ctx* ctx, nvmai_stream stream, const float* x, uint32_t x_stride, uint64_t x_head_stride,

@@ -438,6 +438,20 @@ def test_scan_forms_match_the_oracle(kind, shape):
             assert s.state_error(slot) < 5e-6
 
 
+@pytest.mark.parametrize("kind,shape,n", [(0, (48, 16, 16, 16, 4), 709), (0, (20, 1, 16, 16, 4), 2000), (1, (60, 3, 16, 16, 4), 577), (1, (64, 1, 32, 16, 4), 1501)])
+def test_scan_chunks_whose_blocks_take_several_heads(kind, shape, n):
+    """More (chunk, head) pairs than the device holds blocks: two to four heads share a block, the last of a group fewer.
+    Tolerance: that of the shorter prompts above, in proportion to the rows that a sum runs over."""
+    import nvmai_amd as nv
+    say("scan heads", kind, shape, n)
+    s = Scan(kind, *shape)
+    rows = s.rows(n, n)
+    want = s.want(rows)
+    tol = 5e-6 * n / 150
+    close(s.run(rows, nv.row_map(0, 0), nv.SCAN_CHUNKED), want, tol, "%d rows" % n)
+    assert s.state_error(0) < tol
+
+
 @pytest.mark.parametrize("kind", [0, 1])
 @pytest.mark.parametrize("taps", [1, 4, 6])
 def test_scan_portions_carry_state_and_filter_inputs(kind, taps):
