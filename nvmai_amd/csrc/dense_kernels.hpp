@@ -393,14 +393,15 @@ constexpr int skinny_stages(int tt, int nr, int nw) {
     return nw * (nr + tt) * 2048 * 4 <= 128 * 1024 ? 4 : nw * (nr + tt) * 2048 * 3 <= 144 * 1024 ? 3 : 2;
 }
 
-template <int EPI, int TT, int NR, int NW>
+template <int EPI, int TT, int NR, int NW, bool HALF = false>
 __global__ __launch_bounds__(64 * NW) void dense_skinny_kernel(DenseLinearParams p) {
-    constexpr int S = skinny_stages(TT, NR, NW), L = 2 * (NR + TT);         // 1 KB requests per step
+    static_assert(!HALF || NR == 1, "eight weight rows, the operand's other eight repeat them");
+    constexpr int S = skinny_stages(TT, NR, NW), LW = HALF ? 1 : 2 * NR, L = LW + 2 * TT;      // 1 KB requests per step
     constexpr uint32_t STEP = L * 1024u;
     static_assert((NW - 1) * TT * NR <= NW * L, "one stage holds the sums");
     __shared__ __attribute__((aligned(1024))) uint8_t l0[NW * STEP], l1[NW * STEP], l2[S > 2 ? NW * STEP : 16], l3[S > 3 ? NW * STEP : 16];
     const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i = lane & 15u, g = lane >> 4;
-    const uint32_t r0 = blockIdx.x * (16u * NR);
+    const uint32_t r0 = blockIdx.x * (HALF ? 8u : 16u * NR);
     const uint32_t steps = p.k / 64u, count = steps > wave ? (steps - wave + NW - 1u) / NW : 0u;
     [[maybe_unused]] const uint32_t w_bytes = (p.n - 1u) * p.w_stride * 2u + p.k * 2u, x_bytes = (p.rows - 1u) * p.x_stride * 2u + p.k * 2u;
     auto buf = [&](int j) -> uint8_t* { return (j == 0 ? l0 : j == 1 ? l1 : j == 2 ? l2 : l3) + wave * STEP; };
@@ -409,8 +410,8 @@ __global__ __launch_bounds__(64 * NW) void dense_skinny_kernel(DenseLinearParams
     uint32_t off[L];
 #pragma unroll
     for (int q = 0; q < L; ++q) {
-        const uint32_t row = 8u * (q < 2 * NR ? q : q - 2 * NR) + lr, piece = ((lane & 7u) ^ ((row >> 1) & 7u)) * 16u;
-        off[q] = (q < 2 * NR ? min(r0 + row, p.n - 1u) * p.w_stride : min(row, p.rows - 1u) * p.x_stride) * 2u + piece;
+        const uint32_t row = 8u * (q < LW ? q : q - LW) + lr, piece = ((lane & 7u) ^ ((row >> 1) & 7u)) * 16u;
+        off[q] = (q < LW ? min(r0 + row, p.n - 1u) * p.w_stride : min(row, p.rows - 1u) * p.x_stride) * 2u + piece;
     }
     auto request = [&](uint32_t nth, int j) {
 #if defined(__HIP_DEVICE_COMPILE__)     // the host pass rejects the 16-byte form of the load
@@ -420,10 +421,12 @@ __global__ __launch_bounds__(64 * NW) void dense_skinny_kernel(DenseLinearParams
         const uint32_t k = (wave + nth * NW) * 128u;
 #pragma unroll
         for (int q = 0; q < L; ++q)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(q < 2 * NR ? wr : xr, (__attribute__((address_space(3))) void*)(buf(j) + q * 1024u), 16, off[q], k, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(q < LW ? wr : xr, (__attribute__((address_space(3))) void*)(buf(j) + q * 1024u), 16, off[q], k, 0, 0);
 #endif
     };
     const uint32_t at0 = i * 128u + ((g ^ ((i >> 1) & 7u)) * 16u), at1 = i * 128u + (((4u + g) ^ ((i >> 1) & 7u)) * 16u);
+    const uint32_t i8 = i & 7u;
+    [[maybe_unused]] const uint32_t half0 = i8 * 128u + ((g ^ (i8 >> 1)) * 16u), half1 = i8 * 128u + (((4u + g) ^ (i8 >> 1)) * 16u);
     dn_f4 acc[NR][TT];
 #pragma unroll
     for (int r = 0; r < NR; ++r)
@@ -436,13 +439,13 @@ __global__ __launch_bounds__(64 * NW) void dense_skinny_kernel(DenseLinearParams
         uint4 a[NR][2], b[TT][2];
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
-            a[r][0] = *reinterpret_cast<const uint4*>(buf(j) + 2048u * r + at0);
-            a[r][1] = *reinterpret_cast<const uint4*>(buf(j) + 2048u * r + at1);
+            a[r][0] = *reinterpret_cast<const uint4*>(buf(j) + 2048u * r + (HALF ? half0 : at0));
+            a[r][1] = *reinterpret_cast<const uint4*>(buf(j) + 2048u * r + (HALF ? half1 : at1));
         }
 #pragma unroll
         for (int t = 0; t < TT; ++t) {
-            b[t][0] = *reinterpret_cast<const uint4*>(buf(j) + 2048u * (NR + t) + at0);
-            b[t][1] = *reinterpret_cast<const uint4*>(buf(j) + 2048u * (NR + t) + at1);
+            b[t][0] = *reinterpret_cast<const uint4*>(buf(j) + 1024u * LW + 2048u * t + at0);
+            b[t][1] = *reinterpret_cast<const uint4*>(buf(j) + 1024u * LW + 2048u * t + at1);
         }
         dense_read();                                        // the operands are in registers: the place is free
         request(nth + S, j);
@@ -478,7 +481,7 @@ __global__ __launch_bounds__(64 * NW) void dense_skinny_kernel(DenseLinearParams
 #pragma unroll
             for (int w = 0; w < NW - 1; ++w) acc[r][t] += *reinterpret_cast<const dn_f4*>(part + ((w * (NR * TT) + r * TT + t) * 64u + lane) * 4u);
             // acc[r][t][j] = y[token 16 t + i, row r0 + 16 r + 4 g + j]
-            if (16u * t + i < p.rows) dense_store4<EPI, ACT_BF16>(p, 16u * t + i, r0 + 16u * r + 4u * g, acc[r][t], dense_bias4<EPI>(p, r0 + 16u * r + 4u * g));
+            if (16u * t + i < p.rows && (!HALF || g < 2u)) dense_store4<EPI, ACT_BF16>(p, 16u * t + i, r0 + 16u * r + 4u * g, acc[r][t], dense_bias4<EPI>(p, r0 + 16u * r + 4u * g));
         }
 }
 
@@ -1054,7 +1057,10 @@ int dense_launch(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p) 
         constexpr std::integral_constant<int, 2> two{};
         constexpr std::integral_constant<int, 4> four{};
         if (p.rows <= 16) {
-            if (p.k <= 2048) launch(one, one, two);
+            // eight weight rows per block where sixteen leave half the units without one (2048 x 8192 12.8 -> 10.5 us, 2048 x 2048 5.3 -> 4.9,
+            // 1024 x 4096 7.2 -> 6.1, 520 x 16,384 19.0 -> 14.2, a launch's gap included)
+            if (p.k >= 2048 && (p.n + 15) / 16 * 2 <= (uint32_t)ctx->compute_units) dense_skinny_kernel<EPI, 1, 1, 4, true><<<(p.n + 7) / 8, 256, 0, s>>>(p);
+            else if (p.k <= 2048) launch(one, one, two);
             else launch(one, one, four);
         } else if (p.rows <= 32) {
             if (p.n < 8192) launch(two, one, two);
