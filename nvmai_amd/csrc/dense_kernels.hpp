@@ -387,18 +387,33 @@ __device__ __forceinline__ void dense_read() {
 // Steps of 64 k go round the NW waves, and every wave has a ring of S steps of its own in LDS: weights and inputs are requested in whole
 // lines of 128 bytes and read back as operands (no barrier: a wave waits for its own requests alone).  Requested as operands, which is
 // sixteen rows by lane, a load costs the address unit a cycle per lane, and that was what it took.  16 rows: 2048 x 8192 18 -> 13.3 us, 8192 x 2048
-// 10.1 -> 9.6, 2048 x 2048 6.0 -> 4.2, 1024 x 4096 9.5 -> 5.2, 49,664 x 2048 49 -> 44 (4.6 TB/s).  A line's pieces of 16 bytes lie in the order piece ^ (row / 2 % 8): the sixteen lanes that a read serves at once cover 256
+// 10.1 -> 9.6, 2048 x 2048 6.0 -> 4.2, 1024 x 4096 9.5 -> 5.2, 49,664 x 2048 49 -> 44 (4.6 TB/s).  A line's pieces of 16 bytes lie in the order piece ^ skinny_swizzle(row): the sixteen lanes that a read serves at once cover 256
 // bytes.  Stages are arrays of their own, so that a read does not wait for the requests behind it.
+// An output is the sum of P = NW V partial sums: step s goes to the (s mod P)th, a wave's V of them in accumulators of its own, and they are added in
+// order.  P is the launch's rule of n and k alone (skinny_sums), so that neither the waves nor the rows of a block change a bit; with
+// one chain of products per wave the sums were up to 2.9 times as far from those in 64 bits (2048 x 8192, 17 rows 4.0e-7 and 1.5e-7), at 0 to 10 % less time.
 constexpr int skinny_stages(int tt, int nr, int nw) {
     return nw * (nr + tt) * 2048 * 4 <= 128 * 1024 ? 4 : nw * (nr + tt) * 2048 * 3 <= 144 * 1024 ? 3 : 2;
 }
 
-template <int EPI, int TT, int NR, int NW, bool HALF = false>
-__global__ __launch_bounds__(64 * NW) void dense_skinny_kernel(DenseLinearParams p) {
+// Partial sums of an output: chains of at most sixteen products up to 8192 k; many weight rows, four chains.
+inline uint32_t skinny_sums(uint32_t n, uint32_t k) { return n >= 8192 || k <= 1024 ? 4 : k <= 2048 ? 8 : 16; }
+
+// A lane's operand is the pieces 2 g and 2 g + 1 of row i; a read serves the rows 0 .. 3 and 12 .. 15 of one g with 4 .. 11 of the next at once, or sixteen rows
+// of one: pairs of rows in the order 0 1 4 5 6 7 2 3 cover eight pieces either way.
+__device__ __forceinline__ uint32_t skinny_swizzle(uint32_t row) { return (0x32765410u >> (row >> 1 << 2)) & 7u; }
+
+// The threads that the compiler is told of: 512 leave a wave 256 registers, where the sums need no copies between the two halves of the register file
+// (256 x 2048, 33 rows 7.2 us, 6.1 so; 2048 x 1536 6.5 and 5.6).  The largest sums are faster with them (6144 x 5632, 33 rows 29.1 and 31.3).
+constexpr int skinny_threads(int tt, int nw, int v) { return tt * v >= 32 ? 64 * nw : 512; }
+
+template <int EPI, int TT, int NR, int NW, int V, bool HALF = false>
+__global__ __launch_bounds__(skinny_threads(TT, NW, V)) void dense_skinny_kernel(DenseLinearParams p) {
     static_assert(!HALF || NR == 1, "eight weight rows, the operand's other eight repeat them");
     constexpr int S = skinny_stages(TT, NR, NW), LW = HALF ? 1 : 2 * NR, L = LW + 2 * TT;      // 1 KB requests per step
-    constexpr uint32_t STEP = L * 1024u;
-    static_assert((NW - 1) * TT * NR <= NW * L, "one stage holds the sums");
+    constexpr int U = S > V ? S : V;                         // steps of a turn round both the ring and the sums
+    constexpr uint32_t STEP = L * 1024u, SUMS = NW * TT * NR * 1024u;
+    static_assert(U % S == 0 && U % V == 0 && SUMS * ((V + S - 1) / S) <= NW * STEP, "the stages hold the sums");
     __shared__ __attribute__((aligned(1024))) uint8_t l0[NW * STEP], l1[NW * STEP], l2[S > 2 ? NW * STEP : 16], l3[S > 3 ? NW * STEP : 16];
     const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i = lane & 15u, g = lane >> 4;
     const uint32_t r0 = blockIdx.x * (HALF ? 8u : 16u * NR);
@@ -410,7 +425,7 @@ __global__ __launch_bounds__(64 * NW) void dense_skinny_kernel(DenseLinearParams
     uint32_t off[L];
 #pragma unroll
     for (int q = 0; q < L; ++q) {
-        const uint32_t row = 8u * (q < LW ? q : q - LW) + lr, piece = ((lane & 7u) ^ ((row >> 1) & 7u)) * 16u;
+        const uint32_t row = 8u * (q < LW ? q : q - LW) + lr, piece = ((lane & 7u) ^ skinny_swizzle(row & 15u)) * 16u;
         off[q] = (q < LW ? min(r0 + row, p.n - 1u) * p.w_stride : min(row, p.rows - 1u) * p.x_stride) * 2u + piece;
     }
     auto request = [&](uint32_t nth, int j) {
@@ -424,17 +439,19 @@ __global__ __launch_bounds__(64 * NW) void dense_skinny_kernel(DenseLinearParams
             __builtin_amdgcn_raw_ptr_buffer_load_lds(q < LW ? wr : xr, (__attribute__((address_space(3))) void*)(buf(j) + q * 1024u), 16, off[q], k, 0, 0);
 #endif
     };
-    const uint32_t at0 = i * 128u + ((g ^ ((i >> 1) & 7u)) * 16u), at1 = i * 128u + (((4u + g) ^ ((i >> 1) & 7u)) * 16u);
-    const uint32_t i8 = i & 7u;
-    [[maybe_unused]] const uint32_t half0 = i8 * 128u + ((g ^ (i8 >> 1)) * 16u), half1 = i8 * 128u + (((4u + g) ^ (i8 >> 1)) * 16u);
-    dn_f4 acc[NR][TT];
+    const uint32_t at0 = i * 128u + (((2u * g) ^ skinny_swizzle(i)) * 16u), at1 = at0 ^ 16u;
+    [[maybe_unused]] const uint32_t half0 = (i & 7u) * 128u + (((2u * g) ^ skinny_swizzle(i & 7u)) * 16u), half1 = half0 ^ 16u;
+    dn_f4 acc[V][NR][TT];
 #pragma unroll
-    for (int r = 0; r < NR; ++r)
+    for (int v = 0; v < V; ++v)
 #pragma unroll
-        for (int t = 0; t < TT; ++t) acc[r][t] = dn_f4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int r = 0; r < NR; ++r)
+#pragma unroll
+            for (int t = 0; t < TT; ++t) acc[v][r][t] = dn_f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int j = 0; j < S; ++j) request(j, j);
-    auto step = [&](uint32_t nth, int j) {
+    auto step = [&](uint32_t nth, int n) {                   // nth % U = n
+        const int j = n % S, v = n % V;
         dense_landed<(S - 1) * L>();
         uint4 a[NR][2], b[TT][2];
 #pragma unroll
@@ -454,35 +471,42 @@ __global__ __launch_bounds__(64 * NW) void dense_skinny_kernel(DenseLinearParams
 #pragma unroll
             for (int r = 0; r < NR; ++r)
 #pragma unroll
-                for (int t = 0; t < TT; ++t) acc[r][t] = dn_mfma(a[r][h], b[t][h], acc[r][t]);
+                for (int t = 0; t < TT; ++t) acc[v][r][t] = dn_mfma(a[r][h], b[t][h], acc[v][r][t]);
     };
     uint32_t nth = 0;
-    for (; nth + (uint32_t)S <= count; nth += S) {
+    for (; nth + (uint32_t)U <= count; nth += U) {
 #pragma unroll
-        for (int j = 0; j < S; ++j) step(nth + j, j);
+        for (int n = 0; n < U; ++n) step(nth + n, n);
     }
 #pragma unroll
-    for (int j = 0; j < S - 1; ++j)
-        if (nth + (uint32_t)j < count) step(nth + j, j);
+    for (int n = 0; n < U - 1; ++n)
+        if (nth + (uint32_t)n < count) step(nth + n, n);
     dense_stage_barrier<0>();                                // no request outlives its wave, and no other wave reads its places any more
-    float* part = reinterpret_cast<float*>(l0);
-    if (wave != 0) {
+    // The waves take the tiles of the sums in turn: part(v, w, at) is wave w's v-th sum of tile at, which is for another wave.
+    auto part = [&](int v, int w, int at) {
+        return reinterpret_cast<dn_f4*>((v % S == 0 ? l0 : v % S == 1 ? l1 : v % S == 2 ? l2 : l3) + v / S * SUMS + (w * NR * TT + at) * 1024u) + lane;
+    };
 #pragma unroll
-        for (int r = 0; r < NR; ++r)
+    for (int v = 0; v < V; ++v)
 #pragma unroll
-            for (int t = 0; t < TT; ++t) *reinterpret_cast<dn_f4*>(part + (((wave - 1u) * (NR * TT) + r * TT + t) * 64u + lane) * 4u) = acc[r][t];
-    }
+        for (int at = 0; at < NR * TT; ++at)
+            if (at % NW != (int)wave) *part(v, (int)wave, at) = acc[v][at / TT][at % TT];
     __syncthreads();
-    if (wave != 0) return;
 #pragma unroll
-    for (int r = 0; r < NR; ++r)
+    for (int at = 0; at < NR * TT; ++at) {
+        const int r = at / TT, t = at % TT;
+        if (at % NW != (int)wave) continue;
+        dn_f4 sum;
 #pragma unroll
-        for (int t = 0; t < TT; ++t) {
+        for (int v = 0; v < V; ++v)
 #pragma unroll
-            for (int w = 0; w < NW - 1; ++w) acc[r][t] += *reinterpret_cast<const dn_f4*>(part + ((w * (NR * TT) + r * TT + t) * 64u + lane) * 4u);
-            // acc[r][t][j] = y[token 16 t + i, row r0 + 16 r + 4 g + j]
-            if (16u * t + i < p.rows && (!HALF || g < 2u)) dense_store4<EPI, ACT_BF16>(p, 16u * t + i, r0 + 16u * r + 4u * g, acc[r][t], dense_bias4<EPI>(p, r0 + 16u * r + 4u * g));
-        }
+            for (int w = 0; w < NW; ++w) {
+                const dn_f4 add = w == at % NW ? acc[v][r][t] : *part(v, w, at);
+                sum = v + w == 0 ? add : sum + add;
+            }
+        // sum[j] = y[token 16 t + i, row r0 + 16 r + 4 g + j]
+        if (16u * t + i < p.rows && (!HALF || g < 2u)) dense_store4<EPI, ACT_BF16>(p, 16u * t + i, r0 + 16u * r + 4u * g, sum, dense_bias4<EPI>(p, r0 + 16u * r + 4u * g));
+    }
 }
 
 // ---- many input rows: tiles of BN weight rows x BM tokens, k in steps of 64 through a ring of S stages in LDS ----------
@@ -1049,9 +1073,16 @@ int dense_launch(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p) 
         // Two waves leave room for several blocks per compute unit; four where a row is long and the blocks are few (16 rows: 2048 x 8192 14.0
         // and 13.3 us, 1024 x 4096 5.5 and 5.2, 2048 x 2048 4.2 and 4.3).  Several row tiles per block where the inputs, which every
         // block reads, would weigh more than its weights (32 rows: 8192 x 2048 11.5 -> 10.0 us; 64: 14.5 -> 12.3, 49,664 x 2048 83 -> 65 with four).
+        const uint32_t sums = skinny_sums(p.n, p.k);
         auto launch = [&](auto tt, auto nr, auto nw) {
             constexpr int TT = decltype(tt)::value, NR = decltype(nr)::value, NW = decltype(nw)::value;
-            dense_skinny_kernel<EPI, TT, NR, NW><<<(p.n + 16 * NR - 1) / (16 * NR), 64 * NW, 0, s>>>(p);
+            const uint32_t blocks = (p.n + 16 * NR - 1) / (16 * NR);
+            if constexpr (NR == 1) {                          // four waves: k past 2048
+                if (sums == 16) return dense_skinny_kernel<EPI, TT, NR, NW, 16 / NW><<<blocks, 64 * NW, 0, s>>>(p);
+                if constexpr (NW == 2)
+                    if (sums == 8) return dense_skinny_kernel<EPI, TT, NR, NW, 8 / NW><<<blocks, 64 * NW, 0, s>>>(p);
+            }
+            dense_skinny_kernel<EPI, TT, NR, NW, 4 / NW><<<blocks, 64 * NW, 0, s>>>(p);
         };
         constexpr std::integral_constant<int, 1> one{};
         constexpr std::integral_constant<int, 2> two{};
@@ -1059,8 +1090,10 @@ int dense_launch(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p) 
         if (p.rows <= 16) {
             // eight weight rows per block where sixteen leave half the units without one (2048 x 8192 12.8 -> 10.5 us, 2048 x 2048 5.3 -> 4.9,
             // 1024 x 4096 7.2 -> 6.1, 520 x 16,384 19.0 -> 14.2, a launch's gap included)
-            if (p.k >= 2048 && (p.n + 15) / 16 * 2 <= (uint32_t)ctx->compute_units) dense_skinny_kernel<EPI, 1, 1, 4, true><<<(p.n + 7) / 8, 256, 0, s>>>(p);
-            else if (p.k <= 2048) launch(one, one, two);
+            if (p.k >= 2048 && (p.n + 15) / 16 * 2 <= (uint32_t)ctx->compute_units) {
+                if (sums == 16) dense_skinny_kernel<EPI, 1, 1, 4, 4, true><<<(p.n + 7) / 8, 256, 0, s>>>(p);
+                else dense_skinny_kernel<EPI, 1, 1, 4, 2, true><<<(p.n + 7) / 8, 256, 0, s>>>(p);
+            } else if (p.k <= 2048) launch(one, one, two);
             else launch(one, one, four);
         } else if (p.rows <= 32) {
             if (p.n < 8192) launch(two, one, two);
