@@ -241,7 +241,7 @@ __global__ __launch_bounds__(256) void dense_gemv_kernel(DenseLinearParams p) {
 }
 
 // ---- 1 or 2 input rows in 32 bits that are the end of a sublayer: x + RMS(delta) (add + w), then the product -------------------
-// A block norms the rows once, eight values per thread, and hands them to its waves through LDS while their first weight rows are on
+// A block norms the rows once, four values of every 1024 per thread as norm_residual_kernel does (the same bits as the two launches), and hands them to its waves through LDS while their first weight rows are on
 // their way; a wave keeps them in registers (k <= 512 S) and goes over `turns` times RW weight rows, the next ones requested before the
 // current ones are multiplied.  The first block stores the sum.  (With each wave norming for itself and one weight row per wave the loads of x, delta and
 // w, five times a weight row's, took the time: 16.1 us for 12,352 x 2048.)  As fast as dense_gemv_kernel alone (11.5 us, 12.5 with the norm; 11,264
@@ -253,18 +253,20 @@ __global__ __launch_bounds__(256) void dense_gemv_rms_kernel(DenseLinearParams p
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t first = (blockIdx.x * 4u + wave) * turns * RW;
     const float* x = static_cast<const float*>(p.x);
-    // this thread's values: 8 tid .. 8 tid + 7 (S = 2: the upper half of the block has none)
-    const bool own = 8u * tid < p.k;
-    const uint32_t mine = min(8u * tid, p.k - 8u);
-    dn_f4 xv[NT][2], dv[NT][2];
+    // this thread's values: 4 (tid + 256 u) .. + 3
+    constexpr int P = S / 2;
+    dn_f4 xv[NT][P], dv[NT][P];
+    uint2 nv[P];
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+    for (int u = 0; u < P; ++u) {
+        const uint32_t at = min(4u * tid + 1024u * u, p.k - 4u);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            dv[t][u] = reinterpret_cast<const dn_f4*>(p.rms_delta + (size_t)t * p.rms_delta_stride + mine)[u];
-            xv[t][u] = reinterpret_cast<const dn_f4*>(x + (size_t)t * p.x_stride + mine)[u];
+        for (int t = 0; t < NT; ++t) {
+            dv[t][u] = *reinterpret_cast<const dn_f4*>(p.rms_delta + (size_t)t * p.rms_delta_stride + at);
+            xv[t][u] = *reinterpret_cast<const dn_f4*>(x + (size_t)t * p.x_stride + at);
         }
-    const uint4 nv = *reinterpret_cast<const uint4*>(p.rms_w + mine);
+        nv[u] = *reinterpret_cast<const uint2*>(p.rms_w + at);
+    }
     uint4 wv[S][RW];
     auto fetch = [&](uint32_t r0) {
 #pragma unroll
@@ -280,27 +282,28 @@ __global__ __launch_bounds__(256) void dense_gemv_rms_kernel(DenseLinearParams p
     for (int t = 0; t < NT; ++t) {
         float q = 0.0f;
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < P; ++u)
+            if (4u * tid + 1024u * u < p.k)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) q = fmaf(dv[t][u][e], dv[t][u][e], q);
-        const float sum = wave_sum_bcast(own ? q : 0.0f);
+                for (int e = 0; e < 4; ++e) q = fmaf(dv[t][u][e], dv[t][u][e], q);
+        const float sum = wave_sum_bcast(q);
         if (lane == 0) part[t][wave] = sum;
     }
     __syncthreads();
-    float nw[8];
-    act2_to_f32<ACT_BF16>(nv.x, nw[0], nw[1]);
-    act2_to_f32<ACT_BF16>(nv.y, nw[2], nw[3]);
-    act2_to_f32<ACT_BF16>(nv.z, nw[4], nw[5]);
-    act2_to_f32<ACT_BF16>(nv.w, nw[6], nw[7]);
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        const float inv = 1.0f / sqrtf(((part[t][0] + part[t][1]) + (part[t][2] + part[t][3])) / (float)p.k + p.rms_eps);
+    for (int u = 0; u < P; ++u) {
+        const uint32_t at = 4u * tid + 1024u * u;
+        const bool own = at < p.k;
+        float nw[4];
+        act2_to_f32<ACT_BF16>(nv[u].x, nw[0], nw[1]);
+        act2_to_f32<ACT_BF16>(nv[u].y, nw[2], nw[3]);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+        for (int t = 0; t < NT; ++t) {
+            const float inv = 1.0f / sqrtf(((part[t][0] + part[t][1]) + (part[t][2] + part[t][3])) / (float)p.k + p.rms_eps);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) xv[t][u][e] += dv[t][u][e] * inv * (nw[4 * u + e] + p.rms_add);
-            if (own && blockIdx.x == 0) reinterpret_cast<dn_f4*>(p.rms_out + (size_t)t * p.rms_out_stride + 8u * tid)[u] = xv[t][u];
-            if (8u * tid < 512u * S) reinterpret_cast<dn_f4*>(rows[t] + 8u * tid)[u] = own ? xv[t][u] : dn_f4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int e = 0; e < 4; ++e) xv[t][u][e] += dv[t][u][e] * inv * (nw[e] + p.rms_add);
+            if (own && blockIdx.x == 0) *reinterpret_cast<dn_f4*>(p.rms_out + (size_t)t * p.rms_out_stride + at) = xv[t][u];
+            *reinterpret_cast<dn_f4*>(rows[t] + at) = own ? xv[t][u] : dn_f4{0.0f, 0.0f, 0.0f, 0.0f};
         }
     }
     __syncthreads();

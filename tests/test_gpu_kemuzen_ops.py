@@ -137,6 +137,26 @@ def test_the_end_of_a_sublayer_with_the_next_product(rows, k, n):
         nv.ops.rms_residual_linear(context("bfloat16"), x[:, :k], delta[:, :k], post, 1.0, out, w, y, eps)
 
 
+# n: one and several weight rows per wave, the last wave's cut short (pairs: a wave takes two of them at a time up to 12,288)
+@pytest.mark.parametrize("rows", [1, 2])
+@pytest.mark.parametrize("k", [64, 1024, 1088, 1984, 2048])
+@pytest.mark.parametrize("n", [2, 258, 9002, 12346, 24602])
+def test_the_joined_launch_gives_the_bits_of_the_two(rows, k, n):
+    import nvmai_amd as nv
+    say("rms_residual_linear, bits", rows, k, n)
+    ctx, gen = context("float32"), torch.Generator(device="cuda").manual_seed(n + k)
+    normal = lambda *s: torch.empty(s, device="cuda").normal_(0.0, 1.0, generator=gen)
+    w, post, bias = bf(normal(n, k) * k ** -0.5), bf(normal(k)), bf(normal(n))
+    x, delta = normal(rows, k), normal(rows, k) * 3.0
+    both, h = x.clone(), torch.zeros_like(x)
+    nv.ops.rms_residual(ctx, both, k, delta, post, 1.0, out=h, eps=1e-5)
+    for kw, m in ((dict(), n), (dict(bias=bias), n), (dict(activation=nv.LINEAR_SILU_PAIRS), n // 2)):
+        (want, got), out = (torch.full((rows, m + m % 2 + 4), 7.0, device="cuda") for _ in range(2)), torch.zeros_like(x)
+        nv.dense_linear(ctx, w, h, y_f32=want, **kw)
+        nv.ops.rms_residual_linear(ctx, x, delta, post, 1.0, out, w, got, 1e-5, **kw)
+        assert torch.equal(out, both) and torch.equal(got, want)
+
+
 @pytest.mark.parametrize("dtype", TYPES)
 @pytest.mark.parametrize("width", [1, 5, 72, 700])
 def test_embeddings_with_sinusoids(dtype, width):
