@@ -806,8 +806,9 @@ int nvmai_hip_rms_residual(nvmai_hip_ctx* ctx, nvmai_stream stream, float* x, ui
                            float next_add, void* out, uint32_t out_stride, uint32_t rows, uint32_t d, float eps);
 
 /* The end of a sublayer and the product that opens the next one, in 32-bit contexts, for one or two rows of at most 2048:
- *   x_out  = x + RMS(delta) * (post_add + post_weight)     (x_out not x: other blocks still read it)
+ *   x_out  = x + RMS(delta) * (post_add + post_weight)
  *   y      = the product of nvmai_hip_dense_linear_ex with x_out as its input
+ * The rows of x_out and y share no memory with each other or with those of x and delta (NVMAI_ERR_INVALID_ARG): other blocks still read them.
  * Other contexts and sizes: NVMAI_ERR_UNSUPPORTED (nvmai_hip_rms_residual and nvmai_hip_dense_linear_ex take them). */
 int nvmai_hip_rms_residual_linear(nvmai_hip_ctx* ctx, nvmai_stream stream, const float* x, uint32_t x_stride, const float* delta,
                                   uint32_t delta_stride, const uint16_t* post_weight, float post_add, float eps, float* x_out,

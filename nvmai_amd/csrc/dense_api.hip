@@ -86,6 +86,21 @@ int dense_linear_call(nvmai_hip_ctx* ctx, nvmai_stream stream, DenseLinearParams
     return dense_linear(ctx, (hipStream_t)stream, p);
 }
 
+// Rows of floats, and whether those of two of them share a value.
+struct FloatRows {
+    const float* base;
+    uint32_t stride, cols;
+};
+
+bool overlap(const FloatRows& a, const FloatRows& b, uint32_t rows) {
+    for (uint32_t i = 0; i < rows; ++i)
+        for (uint32_t j = 0; j < rows; ++j) {
+            const uintptr_t p = reinterpret_cast<uintptr_t>(a.base + (size_t)i * a.stride), q = reinterpret_cast<uintptr_t>(b.base + (size_t)j * b.stride);
+            if (p < q + (size_t)b.cols * 4u && q < p + (size_t)a.cols * 4u) return true;
+        }
+    return false;
+}
+
 }  // namespace
 
 extern "C" int nvmai_hip_dense_linear(nvmai_hip_ctx* ctx, nvmai_stream stream, const uint16_t* w, uint32_t w_stride,
@@ -108,13 +123,18 @@ extern "C" int nvmai_hip_rms_residual_linear(nvmai_hip_ctx* ctx, nvmai_stream st
                                              uint32_t delta_stride, const uint16_t* post_weight, float post_add, float eps, float* x_out,
                                              uint32_t x_out_stride, const uint16_t* w, uint32_t w_stride, uint32_t rows, uint32_t n, uint32_t k,
                                              float* y, uint32_t y_stride, const nvmai_linear_epilogue* e) {
-    if (!ctx || !e || !delta || !post_weight || !x_out || x_out == x) return NVMAI_ERR_INVALID_ARG;
+    if (!ctx || !e || !delta || !post_weight || !x_out) return NVMAI_ERR_INVALID_ARG;
     if (ctx->act != NVMAI_ACT_FP32 || rows > DENSE_RMS_ROWS || k > DENSE_RMS_K) return NVMAI_ERR_UNSUPPORTED;
     DenseLinearParams p{w, x, y, nullptr, w_stride, x_stride, y_stride, rows, n, k, e->activation, e->bias, e->mul, e->mul_ids, e->mul_stride, e->mul_rows};
     p.rms_delta = delta; p.rms_w = post_weight; p.rms_out = x_out; p.rms_delta_stride = delta_stride; p.rms_out_stride = x_out_stride;
     p.rms_add = post_add; p.rms_eps = eps;
     if (delta_stride < k || x_out_stride < k) return NVMAI_ERR_INVALID_ARG;
     if (!aligned16(delta) || !aligned16(post_weight) || !aligned16(x_out) || delta_stride % 4 || x_out_stride % 4) return NVMAI_ERR_ALIGNMENT;
+    // every block reads x and delta whole, while the first one stores x_out and others that have ended store y
+    const FloatRows out{x_out, x_out_stride, k}, product{y, y_stride, e->activation == NVMAI_LINEAR_SILU_PAIRS ? n / 2 : n};
+    for (const FloatRows& in : {FloatRows{x, x_stride, k}, FloatRows{delta, delta_stride, k}})
+        if (overlap(in, out, rows) || overlap(in, product, rows)) return NVMAI_ERR_INVALID_ARG;
+    if (overlap(out, product, rows)) return NVMAI_ERR_INVALID_ARG;
     return dense_linear(ctx, (hipStream_t)stream, p);
 }
 

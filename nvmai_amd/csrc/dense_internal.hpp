@@ -17,7 +17,7 @@ struct DenseLinearParams {
     const uint32_t* mul_ids;
     uint32_t mul_stride, mul_rows;
     uint16_t* planes;       // dense_plane_bytes of scratch for the rows of a 32-bit context, or nullptr
-    // the rows that are multiplied are x + RMS(rms_delta) * (rms_add + rms_w), which go to rms_out as well (rms_out not x); nullptr: x
+    // the rows that are multiplied are x + RMS(rms_delta) * (rms_add + rms_w), which go to rms_out as well (y and rms_out: neither x nor rms_delta); nullptr: x
     const float* rms_delta;
     const uint16_t* rms_w;
     float* rms_out;

@@ -157,6 +157,34 @@ def test_the_joined_launch_gives_the_bits_of_the_two(rows, k, n):
         assert torch.equal(out, both) and torch.equal(got, want)
 
 
+def test_the_joined_launch_refuses_outputs_over_its_inputs():
+    """Blocks read the inputs while others store: nothing is launched where an output's row shares a value with an input's or with the other
+    output's.  Rows side by side in one buffer share none."""
+    import nvmai_amd as nv
+    ctx, k, n = context("float32"), 64, 12
+    w, post = bf(randn(1, n, k, std=k ** -0.5)), bf(randn(2, k))
+    buf = randn(3, 2, 5 * k)
+    piece = lambda at, rows=2: buf[:rows, at:at + k]
+    x, delta, out, y = piece(0), piece(k), piece(2 * k), piece(3 * k)
+    for rows in (1, 2):
+        for bad in (dict(out=x), dict(out=delta), dict(y=x), dict(y=delta), dict(y=out), dict(out=piece(k - 4)), dict(out=piece(2 * k - 4)), dict(y=piece(2 * k - 8)),
+                    dict(y=piece(3 * k - 4)), dict(y=piece(k + 60))):
+            say("outputs over inputs", rows, sorted(bad))
+            a = dict(dict(x=x, delta=delta, out=out, y=y), **bad)
+            with pytest.raises(nv.NvmaiError) as e:
+                nv.ops.rms_residual_linear(ctx, a["x"][:rows], a["delta"][:rows], post, 1.0, a["out"][:rows], w, a["y"][:rows], 1e-3)
+            assert e.value.name == "invalid_arg"
+    flat = buf.flatten()                             # one row's output is the other row's input
+    with pytest.raises(nv.NvmaiError):
+        nv.ops.rms_residual_linear(ctx, x, delta, post, 1.0, flat[5 * k:5 * k + 2 * k].view(2, k), w, y, 1e-3)
+    apart = [t.clone() for t in (x, delta, out, y)]
+    nv.ops.rms_residual_linear(ctx, x, delta, post, 1.0, out, w, y[:, :n], 1e-3)
+    nv.ops.rms_residual_linear(ctx, apart[0], apart[1], post, 1.0, apart[2], w, apart[3][:, :n], 1e-3)
+    assert all(torch.equal(a, b) for a, b in zip((x, delta, out, y), apart))
+    pairs = torch.cat([randn(4, 2, n // 2 + 2), randn(5, 2, k + 4)], 1)      # SILU_PAIRS stores half as many columns: the next rows begin behind them
+    nv.ops.rms_residual_linear(ctx, x, delta, post, 1.0, pairs[:, 8:8 + k], w, pairs[:, :8], 1e-3, activation=nv.LINEAR_SILU_PAIRS)
+
+
 @pytest.mark.parametrize("dtype", TYPES)
 @pytest.mark.parametrize("width", [1, 5, 72, 700])
 def test_embeddings_with_sinusoids(dtype, width):
