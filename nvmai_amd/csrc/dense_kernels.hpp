@@ -386,7 +386,7 @@ __device__ __forceinline__ void dense_read() {
 #endif
 }
 
-// ---- 5 .. 64 input rows: 16 NR weight rows per block, the waves split k, MFMA, sums through LDS ---------
+// ---- 5 .. 64 input rows: 16 NR weight rows per block (HALF: eight), the waves split k, MFMA, sums through LDS ---------
 // Steps of 64 k go round the NW waves, and every wave has a ring of S steps of its own in LDS: weights and inputs are requested in whole
 // lines of 128 bytes and read back as operands (no barrier: a wave waits for its own requests alone).  Requested as operands, which is
 // sixteen rows by lane, a load costs the address unit a cycle per lane, and that was what it took.  16 rows: 2048 x 8192 18 -> 13.3 us, 8192 x 2048
@@ -1073,9 +1073,10 @@ int dense_launch(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p) 
         return launch_status();
     }
     if (p.rows <= 64) {
-        // Two waves leave room for several blocks per compute unit; four where a row is long and the blocks are few (16 rows: 2048 x 8192 14.0
-        // and 13.3 us, 1024 x 4096 5.5 and 5.2, 2048 x 2048 4.2 and 4.3).  Several row tiles per block where the inputs, which every
-        // block reads, would weigh more than its weights (32 rows: 8192 x 2048 11.5 -> 10.0 us; 64: 14.5 -> 12.3, 49,664 x 2048 83 -> 65 with four).
+        // Two waves leave room for several blocks per compute unit.  Several row tiles per block where the inputs, which every block reads, would
+        // weigh more than its weights (32 rows: 8192 x 2048 11.5 -> 10.0 us; 64: 14.5 -> 12.3, 49,664 x 2048 83 -> 65 with four).  Past 16 rows, against sixteen
+        // waves that load operands (17 and 64 rows): 2048 x 8192 19.5 -> 15.7 and 46.2 -> 24.2 us, 2048 x 5632 14.5 -> 11.6 and 33.9 -> 19.4, 2128 x 2048 8.4 -> 5.9 and
+        // 14.2 -> 8.6, 1024 x 2816 8.3 -> 5.8 and 15.8 -> 8.9.
         const uint32_t sums = skinny_sums(p.n, p.k);
         auto launch = [&](auto tt, auto nr, auto nw) {
             constexpr int TT = decltype(tt)::value, NR = decltype(nr)::value, NW = decltype(nw)::value;
@@ -1091,12 +1092,14 @@ int dense_launch(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p) 
         constexpr std::integral_constant<int, 2> two{};
         constexpr std::integral_constant<int, 4> four{};
         if (p.rows <= 16) {
-            // eight weight rows per block where sixteen leave half the units without one (2048 x 8192 12.8 -> 10.5 us, 2048 x 2048 5.3 -> 4.9,
-            // 1024 x 4096 7.2 -> 6.1, 520 x 16,384 19.0 -> 14.2, a launch's gap included)
-            if (p.k >= 2048 && (p.n + 15) / 16 * 2 <= (uint32_t)ctx->compute_units) {
+            // Eight weight rows per block where sixteen leave half the units without one, past rows of 1024 (sixteen weight rows in two waves and eight, us for 5 rows:
+            // 2048 x 8192 14.1 and 10.0, 2048 x 2112 5.6 and 4.6, 1024 x 4096 7.5 and 5.6, 2048 x 1536 3.7 and 3.5, 2048 x 1024 3.1 and 3.2, 2048 x 512 2.8 and 2.9).
+            // Four waves where a row is long and the blocks are few, or the row so long that two take too many turns (two and four: 2064 x 4096 8.2 and 7.3,
+            // 4096 x 2816 8.3 and 7.1, 8190 x 8192 31.7 and 30.0; but 6144 x 2112 8.0 and 8.8, 12,352 x 2816 16.8 and 17.4, 3072 x 1536 4.6 and 4.5, 2048 x 1024 3.1 and 3.3).
+            if (p.k > 1024 && (p.n + 15) / 16 * 2 <= (uint32_t)ctx->compute_units) {
                 if (sums == 16) dense_skinny_kernel<EPI, 1, 1, 4, 4, true><<<(p.n + 7) / 8, 256, 0, s>>>(p);
                 else dense_skinny_kernel<EPI, 1, 1, 4, 2, true><<<(p.n + 7) / 8, 256, 0, s>>>(p);
-            } else if (p.k <= 2048) launch(one, one, two);
+            } else if (p.k <= 2048 || (p.n > 4096 && p.k < 4096)) launch(one, one, two);
             else launch(one, one, four);
         } else if (p.rows <= 32) {
             if (p.n < 8192) launch(two, one, two);
