@@ -47,8 +47,10 @@ void filter(const ScanParams& p, hipStream_t s) {
 }
 
 // Heads of one block of the preparation: it makes k k^T and q k^T once for all of them, which takes as long as one head of the delta rule or four of
-// the state-space form, and two blocks fit a compute unit.  Many heads where the blocks are many, few where units would be idle (us for 5, 24
+// the state-space form; slots: the blocks that fit the device at once.  Many heads where the blocks are many, few where units would be idle (us for 5, 24
 // and 32 chunks; delta rule, 16 key heads of 2: one head per block 26, 56 and 64, two 39, 48 and 53; state-space, one group of 64: 1 11.6, 27 and 33, 4 15.8, 18.9 and 19.1, 8 25, 26 and 26).
+// Keys of 256, where one block fits, the whole call (slots for two and for one): state-space, 8 groups of 8, 24 chunks 164 and 155 us, 5 chunks 65 and 56;
+// delta rule, 16 key heads of 2, 11 chunks 170 and 156.
 uint32_t prep_heads(bool delta, uint32_t chunks, uint32_t key_heads, uint32_t ratio, uint32_t slots) {
     uint32_t best = 1;
     uint64_t least = ~0ull;
@@ -69,7 +71,8 @@ int chunked(const ScanParams& p, uint32_t chunks, bool fast, uint32_t cus, hipSt
     else if (fast) filter<DELTA, 4, true>(p, s);
     else filter<DELTA, 4, false>(p, s);
     if (p.taps > 1) scan_history_kernel<<<dim3((p.channels + 255) / 256, p.taps - 1), 256, 0, s>>>(p);
-    const uint32_t ratio = p.heads / p.key_heads, per = prep_heads(DELTA, chunks, p.key_heads, ratio, 2 * cus);
+    const uint32_t resident = 2 * (lds + scan_prep_static_lds(DELTA)) <= 160 * 1024 ? 2 : 1;       // two up to keys of 128, then one
+    const uint32_t ratio = p.heads / p.key_heads, per = prep_heads(DELTA, chunks, p.key_heads, ratio, resident * cus);
     scan_prep_kernel<DELTA><<<dim3(chunks, p.key_heads * ((ratio + per - 1) / per)), 256, lds, s>>>(p, per);
     const dim3 grid(p.heads, p.dv / 16);
     if (p.dk <= 64) scan_chain_kernel<DELTA, 4, 2><<<grid, 512, 0, s>>>(p, chunks);

@@ -274,6 +274,9 @@ __global__ __launch_bounds__(256) void scan_history_kernel(ScanParams p) {
 //   (I + L) X = R for X = [Kt | U0], sixteen rows at a time: the four diagonal blocks of I + L are inverted by forward
 //   substitution (a lane per column), X_b = inv_b (R_b - sum_{m < b} L_bm X_m) runs on the matrix cores, a wave per
 //   sixteen columns, its X in the accumulators, where it stands as the next product's B operand.
+// LDS beside the dynamic part: X, beta and bg, and inv and turn of the delta rule.
+constexpr size_t scan_prep_static_lds(bool delta) { return 64 * 8 + 2 * 64 * 4 + (delta ? 2 * 4 * 16 * 20 * 4 : 0); }
+
 template <bool DELTA>
 __global__ __launch_bounds__(256, 2) void scan_prep_kernel(ScanParams p, uint32_t per) {
     constexpr int JOBS = DELTA ? 5 : 3;              // tiles of one wave: ten of q k^T, ten of k k^T

@@ -500,6 +500,42 @@ def test_scan_chunks_whose_blocks_take_several_heads(kind, shape, n):
     assert s.state_error(0) < tol
 
 
+def grids(call):
+    """(x, y) of the grids that a call launches, by a graph that records it."""
+    import ctypes as C
+
+    class Node(C.Structure):                         # hipKernelNodeParams
+        _fields_ = [("block", C.c_uint32 * 3), ("extra", C.c_void_p), ("func", C.c_void_p), ("grid", C.c_uint32 * 3), ("params", C.c_void_p), ("shared", C.c_uint32)]
+    call()
+    graph, stream, hip = torch.cuda.CUDAGraph(keep_graph=True), torch.cuda.Stream(), C.CDLL("libamdhip64.so")
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(graph, stream=stream):
+            call()
+    n, raw = C.c_size_t(0), C.c_void_p(graph.raw_cuda_graph())
+    assert hip.hipGraphGetNodes(raw, None, C.byref(n)) == 0
+    nodes, out = (C.c_void_p * n.value)(), []
+    assert hip.hipGraphGetNodes(raw, nodes, C.byref(n)) == 0
+    for node in nodes:
+        p = Node()
+        assert hip.hipGraphKernelNodeGetParams(C.c_void_p(node), C.byref(p)) == 0
+        out.append((p.grid[0], p.grid[1]))
+    return out
+
+
+@pytest.mark.parametrize("dk,groups", [(128, 16), (144, 16), (160, 8), (256, 8)])
+def test_heads_of_a_block_by_the_blocks_that_fit(dk, groups):
+    """Eight key heads of eight in 24 chunks: four heads per block where two blocks fit a compute unit (512 slots for 384 blocks), all eight where
+    one does, with tiles of keys past 80 KB (192 blocks; twice as many would take two rounds)."""
+    import nvmai_amd as nv
+    s = Scan(1, 64, 8, dk, 16, 4)
+    proj = torch.zeros((1501, s.cols), device="cuda")
+    out = torch.zeros((s.H, 1501, s.vp), device="cuda")
+    say("heads of a block", dk)
+    got = grids(lambda: s.op.encode(proj, s.conv_p, s.bias_p, s.a_log, s.dt_bias, s.skip, s.history, s.state, nv.row_map(0, 0), out, nv.SCAN_CHUNKED))
+    assert (24, groups) in got, got
+
+
 @pytest.mark.parametrize("kind", [0, 1])
 @pytest.mark.parametrize("taps", [1, 4, 6])
 def test_scan_portions_carry_state_and_filter_inputs(kind, taps):
