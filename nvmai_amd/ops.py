@@ -24,9 +24,11 @@ def _ptr(t):
 
 def _stream():
     """The current stream of the current device.  torch.cuda.current_stream() makes a Stream object of it by way of a dozen Python
-    calls, a third of what a call here takes on the host; until the first CUDA call of a process it also sets the device up."""
-    if torch.cuda.is_initialized():
-        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    calls, a third of what a call here takes on the host; until the first CUDA call of a process it also sets the device up.  The
+    functions behind it are torch's own and may be absent."""
+    raw, device = getattr(torch._C, "_cuda_getCurrentRawStream", None), getattr(torch._C, "_cuda_getDevice", None)
+    if raw is not None and device is not None and torch.cuda.is_initialized():
+        return raw(device())
     return torch.cuda.current_stream().cuda_stream
 
 

@@ -1,0 +1,30 @@
+"""The handle of the current stream, with and without the functions of torch that give it directly."""
+import types
+
+import pytest
+import torch
+
+from nvmai_amd import ops
+
+NAMES = ("_cuda_getCurrentRawStream", "_cuda_getDevice")
+
+
+@pytest.mark.parametrize("absent", [(), NAMES[:1], NAMES[1:], NAMES])
+def test_a_torch_without_the_direct_functions(monkeypatch, absent):
+    for n in NAMES:
+        monkeypatch.setattr(torch._C, n, (lambda: 3) if n == "_cuda_getDevice" else (lambda device: 100 + device), raising=False)
+    for n in absent:
+        monkeypatch.delattr(torch._C, n)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=7))
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+    assert ops._stream() == (7 if absent else 103)
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: False)
+    assert ops._stream() == 7
+
+
+@pytest.mark.gpu
+def test_the_stream_that_is_current():
+    side = torch.cuda.Stream()
+    assert ops._stream() == torch.cuda.current_stream().cuda_stream
+    with torch.cuda.stream(side):
+        assert ops._stream() == side.cuda_stream
