@@ -101,12 +101,13 @@ class DenseDecoder(StepDecoder):
     def pass_context(self, rows):
         return self.few_ctx if rows <= FEW_ROWS else self.ctx
 
-    def _buf(self, name, rows, cols, dtype):
-        """Scratch rows.  Columns past a producer's own stay zero: a buffer's name goes with one width."""
+    def _buf(self, name, rows, cols, dtype, most=None):
+        """Scratch rows; most: how many of them a pass takes at most.  Columns past a producer's own stay zero: a buffer's name goes
+        with one width."""
         key = (name, cols, dtype)
         if key not in self._buffers:
             # buffers of passes in another type than the context's never see more than FEW_ROWS rows
-            most = self.max_rows if dtype == self.ctx.dtype or name in self.long_f32 else FEW_ROWS
+            most = most or (self.max_rows if dtype == self.ctx.dtype or name in self.long_f32 else FEW_ROWS)
             self._buffers[key] = torch.zeros((most, cols), dtype=dtype, device=self.ctx.device)
         return self._buffers[key][:rows]
 

@@ -14,7 +14,7 @@ them."""
 import torch
 
 from . import ops
-from .dense_model import DenseDecoder, bf16_reader, blocks_of, check_shapes, need, open_directory, pad_columns, up
+from .dense_model import FEW_ROWS, DenseDecoder, bf16_reader, blocks_of, check_shapes, need, open_directory, pad_columns, up
 from .gturbo import ModelError
 
 
@@ -381,7 +381,7 @@ class KemuzenDecoder(DenseDecoder):
         h, last = self._buf("input", T, cfg.width_p, ctx.dtype), self._buf("normed", T, cfg.width_p, self.ctx.dtype)
         # Short passes: the end of a sublayer goes with the product that opens the next one, from one of two residuals to the other.
         joined = self.residual_hook is None and D == cfg.width_p and ops.joins_rms(ctx, T, D)
-        other, ended = self._buf("residual2", T, D, torch.float32) if joined else None, None
+        other, ended = self._buf("residual2", T, D, torch.float32, FEW_ROWS) if joined else None, None
         ops.embed_positions(ctx, self.w.embed, tokens, D, cfg.vocab, cfg.embed_scale, self.inv_freq, rows_at, x, h)
 
         def linear(weight, y=None, y_f32=None, **epilogue):      # of the layer's input

@@ -112,6 +112,18 @@ def test_prompts_longer_than_a_chunk(folder, dtype):
             session.end(what)
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_the_second_residual_holds_the_rows_of_short_passes(folder, dtype):
+    """Passes of one or two tokens go from one residual to another; long ones have one residual."""
+    from nvmai_amd.registry import open_model
+    path, cfg, _ = model(folder, "aligned")
+    dec = open_model(path, dtype, max_context=64, max_chunk=48)
+    for n in (1, 2, 40):
+        dec.prefill_chunked(torch.tensor(random_tokens(cfg, n, 7), dtype=torch.int32, device="cuda"))
+    assert {b.shape[0] for (name, _, _), b in dec._buffers.items() if name == "residual2"} == {2}
+    assert {b.shape[0] for (name, _, _), b in dec._buffers.items() if name == "residual"} == {48}
+
+
 @pytest.mark.parametrize("name", ["mixed", "wide", "open"])
 def test_residual_after_every_layer(folder, name):
     from nvmai_amd.registry import open_model
