@@ -244,8 +244,8 @@ __global__ __launch_bounds__(256) void dense_gemv_kernel(DenseLinearParams p) {
 // A block norms the rows once, four values of every 1024 per thread as norm_residual_kernel does (the same bits as the two launches), and hands them to its waves through LDS while their first weight rows are on
 // their way; a wave keeps them in registers (k <= 512 S) and goes over `turns` times RW weight rows, the next ones requested before the
 // current ones are multiplied.  The first block stores the sum.  (With each wave norming for itself and one weight row per wave the loads of x, delta and
-// w, five times a weight row's, took the time: 16.1 us for 12,352 x 2048.)  As fast as dense_gemv_kernel alone (11.5 us, 12.5 with the norm; 11,264
-// rows in pairs 11.0 and 10.6; 256 rows 3.7 and 4.6): the norm's own launch, 3.0 us, is saved.
+// w, five times a weight row's, took the time: 16.1 us for 12,352 x 2048.)  Little longer than dense_gemv_kernel alone (cold weights: 10.6 us, 12.0 with the norm; 11,264
+// rows in pairs 10.3 and 10.9; 256 rows 2.3 and 2.9): the norm's own launch, 3.0 us, is saved.
 template <int EPI, int NT, int RW, int S>
 __global__ __launch_bounds__(256) void dense_gemv_rms_kernel(DenseLinearParams p, uint32_t turns) {
     __shared__ __attribute__((aligned(16))) float rows[NT][512 * S];
@@ -389,8 +389,8 @@ __device__ __forceinline__ void dense_read() {
 // ---- 5 .. 64 input rows: 16 NR weight rows per block (HALF: eight), the waves split k, MFMA, sums through LDS ---------
 // Steps of 64 k go round the NW waves, and every wave has a ring of S steps of its own in LDS: weights and inputs are requested in whole
 // lines of 128 bytes and read back as operands (no barrier: a wave waits for its own requests alone).  Requested as operands, which is
-// sixteen rows by lane, a load costs the address unit a cycle per lane, and that was what it took.  16 rows: 2048 x 8192 18 -> 13.3 us, 8192 x 2048
-// 10.1 -> 9.6, 2048 x 2048 6.0 -> 4.2, 1024 x 4096 9.5 -> 5.2, 49,664 x 2048 49 -> 44 (4.6 TB/s).  A line's pieces of 16 bytes lie in the order piece ^ skinny_swizzle(row): the sixteen lanes that a read serves at once cover 256
+// sixteen rows by lane, a load costs the address unit a cycle per lane, and that was what it took.  16 rows, cold weights, against sixteen
+// and fewer waves that did: 2048 x 8192 18.6 -> 11.6 us, 8192 x 2048 11.5 -> 10.3, 2048 x 2048 6.1 -> 4.8, 1024 x 4096 10.3 -> 6.3, 49,664 x 2048 57 -> 48 (4.3 TB/s).  A line's pieces of 16 bytes lie in the order piece ^ skinny_swizzle(row): the sixteen lanes that a read serves at once cover 256
 // bytes.  Stages are arrays of their own, so that a read does not wait for the requests behind it.
 // An output is the sum of P = NW V partial sums: step s goes to the (s mod P)th, a wave's V of them in accumulators of its own, and they are added in
 // order.  P is the launch's rule of n and k alone (skinny_sums), so that neither the waves nor the rows of a block change a bit; with
@@ -527,7 +527,7 @@ __global__ __launch_bounds__(skinny_threads(TT, NW, V)) void dense_skinny_kernel
 // which requests a read of LDS has to wait for.
 //   32-bit activations come as three BF16 planes (dense_split), [row][plane][k], the smallest first: the products of a step
 // of 64 k are exact, and their sum goes to a running total of its own, which keeps the rounding of a long k small.
-// Measured (tiles of 128 x 128 x 64 in two stages before): 2048 x 8192 x 2048 77 -> 61 us, 2048 x 2048 x 8192 140 -> 67, 1501 x
+// Measured (tiles of 128 x 128 x 64 in two stages before): 2048 x 8192 x 2048 77 -> 64 us, 2048 x 2048 x 8192 140 -> 67, 1501 x
 // 2048 x 2048 34 -> 17, 512 x 2048 x 2048 33 -> 9.5 (rows x n x k, cold weights).
 typedef float dn_f16 __attribute__((ext_vector_type(16)));
 
@@ -756,9 +756,10 @@ __global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_ker
 // last two products of the stage before run and the halves 1 during the first two; a half is then out of LDS for registers (128 of them hold a
 // stage) one to one and a half stages before its successor is needed.  Barriers stand behind the first four of the sixteen matrix instructions of
 // a product: the reads before them arrive in the meantime.  Requests go out evenly over the stage.  Pieces lie in the order piece ^ (r / 2 % 8):
-// the sixteen lanes that a read serves at once cover 256 bytes.  Bound by the rate of requests into LDS (49 us of the 61 below without the products) and the
-// clock that the products leave.  Rows x n x k, cold weights, former ring of two stages: 2048 x 8192 x 2048 67 -> 61 us, 4096 x 8192 x 2048
-// 126 -> 116, 8192 x 8192 x 8192 823 -> 759.  Not kept: a third place for the halves 0 (no change), requests of 64 bytes per row in stages of 32 k (half
+// the sixteen lanes that a read serves at once cover 256 bytes.  Bound by the rate of requests into LDS (49 us of the 62 below without the products) and the
+// clock that the products leave.  Rows x n x k, cold weights, former ring of two stages, one call after another: 2048 x 8192 x 2048 63.9 -> 62.2 us, 4096 x 8192 x 2048
+// 123.6 -> 120.5, 2048 x 12,352 x 2048 112 -> 105, 8192 x 8192 x 8192 806 -> 772; in the traces of prompts 64.4 -> 62.3, with GELU 76.8 -> 75.7, pairs of 1501 rows
+// 64.5 -> 63.8.  The costs of the plan below are a little lower than that and choose no worse (156 sizes 1.8 % faster, with costs to the letter 1.4 %).  Not kept: a third place for the halves 0 (no change), requests of 64 bytes per row in stages of 32 k (half
 // the rate).
 template <int EPI>
 __global__ __launch_bounds__(256, 1) void dense_wide_kernel(DenseLinearParams p, uint32_t tiles_n, uint32_t tiles_m) {

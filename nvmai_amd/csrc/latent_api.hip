@@ -39,7 +39,7 @@ int launch_partial(const LatentAttnParams& p, hipStream_t s) {
 }
 
 // How many splits of `most`: of the form through LDS one block per compute unit is resident, so the fewest whose rounds per split are not
-// a tenth above the least (16 rows of 4096 keys: 16 splits 23.7 us and 8.5 to combine them).
+// a tenth above the least (16 rows of 4096 keys: 15 splits 24.5 us and 8.6 to combine them).
 uint32_t latent_splits(uint32_t blocks, uint32_t cus, uint32_t most) {
     uint32_t best = 1, best_rounds = (blocks + cus - 1) / cus;
     for (uint32_t n = 2; n <= most; ++n) {

@@ -266,8 +266,8 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(LatentAttnParams p) 
 // read as 4 g .. 4 g + 3 and 16 + 4 g .. 16 + 4 g + 3.  P enters as two BF16 halves (hi + lo): fp32 weights.
 // A row's pieces of 16 bytes lie in the order piece ^ swizzle(row): sixteen rows read at one piece then cover 256 bytes.  A stage ends
 // with the split and at the end of the ring; rows past it, and stages past the last, are filled with zeros.
-// 16 sequences x 4096 keys of 1152 bytes, 16 heads: 31.3 -> 23.7 us (3.2 TB/s of rows with the launch; every row was loaded twice, once by sixteen rows a
-// lane apart, transposed in registers, and nothing was on its way while a tile was worked on), and half as many splits to combine: 9.6 -> 8.5.
+// 16 sequences x 4096 keys of 1152 bytes, 16 heads: 31.3 -> 24.5 us (3.1 TB/s of rows with the launch; every row was loaded twice, once by sixteen rows a
+// lane apart, transposed in registers, and nothing was on its way while a tile was worked on), and half as many splits to combine: 9.6 -> 8.6.
 constexpr int latent_stages(int nt) { return nt <= 8 ? 3 : 2; }          // of 160 KB, one block per compute unit
 
 template <int NT>

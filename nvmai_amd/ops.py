@@ -1155,7 +1155,8 @@ def joins_rms(ctx, rows, k):
 
 
 def rms_residual_linear(ctx, x, delta, post, post_add, x_out, weight, y, eps=1e-6, activation=LINEAR_NONE, bias=None, mul=None, mul_ids=None):
-    """x_out = x + RMS(delta) * (post_add + post), then dense_linear of x_out, in one launch (32-bit contexts, joins_rms)."""
+    """x_out = x + RMS(delta) * (post_add + post), then dense_linear of x_out, in one launch (32-bit contexts, joins_rms).  x_out and y
+    share no memory with each other, x or delta."""
     n, k = weight.shape
     e = LinearEpilogue(activation, _ptr(bias), _ptr(mul), _ptr(mul_ids), 0 if mul is None else mul.stride(0), 0 if mul is None else mul.shape[0])
     check(lib.nvmai_hip_rms_residual_linear(ctx.handle, _stream(), _ptr(x), x.stride(0), _ptr(delta), delta.stride(0), _ptr(post), post_add, eps, _ptr(x_out),
