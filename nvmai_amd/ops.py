@@ -22,13 +22,15 @@ def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
+# torch's own functions behind torch.cuda.current_stream(), which a torch may lack
+_raw_stream, _raw_device = (getattr(torch._C, n, None) for n in ("_cuda_getCurrentRawStream", "_cuda_getDevice"))
+
+
 def _stream():
     """The current stream of the current device.  torch.cuda.current_stream() makes a Stream object of it by way of a dozen Python
-    calls, a third of what a call here takes on the host; until the first CUDA call of a process it also sets the device up.  The
-    functions behind it are torch's own and may be absent."""
-    raw, device = getattr(torch._C, "_cuda_getCurrentRawStream", None), getattr(torch._C, "_cuda_getDevice", None)
-    if raw is not None and device is not None and torch.cuda.is_initialized():
-        return raw(device())
+    calls, a third of what a call here takes on the host; until the first CUDA call of a process it also sets the device up."""
+    if _raw_stream is not None and _raw_device is not None and torch.cuda.is_initialized():
+        return _raw_stream(_raw_device())
     return torch.cuda.current_stream().cuda_stream
 
 

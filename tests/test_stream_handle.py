@@ -6,15 +6,10 @@ import torch
 
 from nvmai_amd import ops
 
-NAMES = ("_cuda_getCurrentRawStream", "_cuda_getDevice")
-
-
-@pytest.mark.parametrize("absent", [(), NAMES[:1], NAMES[1:], NAMES])
+@pytest.mark.parametrize("absent", [(), ("_raw_stream",), ("_raw_device",), ("_raw_stream", "_raw_device")])
 def test_a_torch_without_the_direct_functions(monkeypatch, absent):
-    for n in NAMES:
-        monkeypatch.setattr(torch._C, n, (lambda: 3) if n == "_cuda_getDevice" else (lambda device: 100 + device), raising=False)
-    for n in absent:
-        monkeypatch.delattr(torch._C, n)
+    for name, function in (("_raw_stream", lambda device: 100 + device), ("_raw_device", lambda: 3)):
+        monkeypatch.setattr(ops, name, None if name in absent else function)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=7))
     monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
     assert ops._stream() == (7 if absent else 103)
