@@ -22,6 +22,8 @@
  *     nvmai_hip_dense_linear[_ex] and the expanded nvmai_hip_latent_attention of a 32-bit
  *     context (products without BF16 planes), and nvmai_hip_attention_decode_ragged (chunks of
  *     one length for every sequence).  They do the same where memory cannot be allocated.
+ *     Beside the workspace a ctx holds 16 MB from its creation on, where the blocks that share an output tile
+ *     meet; if they cannot be allocated, no tile is shared (slower products of few rows, other roundings).
  * Data formats (reference file:line):
  *   - weights: affine group-64 codes, 4 bit (two per byte, element 2k in the low
  *     nibble of byte k) or 8 bit, plus one BF16 scale and one BF16 bias per group

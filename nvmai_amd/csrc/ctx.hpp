@@ -23,6 +23,7 @@ struct nvmai_hip_ctx {
     std::vector<void*> ws_retired;
     uint8_t* static_scratch; // device address of the library's static scratch array on this device (ctx_api.hip)
     uint32_t* tickets;       // zero-initialised device words for last-block-done kernels (TICKET_WORDS)
+    float* cut_sums;         // sums of blocks that share a tile (CUT_SUMS_BYTES), or nullptr: no tile is shared
     // Optional per-kernel timing: event pairs recorded around tagged launches.
     bool prof_on;
     struct ProfSpan { int tag; hipEvent_t start, stop; };
@@ -33,9 +34,14 @@ struct nvmai_hip_ctx {
 namespace nvmai {
 
 // The context's persistent zeroed words: [0] work-list ticket, [8] prefill grouping error word,
-// [16, 48) sampler block counters, [TICKET_GROUPS, TICKET_WORDS) router token-group tickets.
+// [16, 48) sampler block counters, [TICKET_CUTS, + CUT_BLOCKS) tiles that several blocks share.
 constexpr uint32_t TICKET_WORDS = 2048;
-constexpr uint32_t TICKET_GROUPS = 64;
+constexpr uint32_t TICKET_CUTS = 64;
+
+// Blocks that share tiles in one launch at most, and their sums: a tile of 128 x 128 floats each.
+constexpr uint32_t CUT_BLOCKS = 256;
+constexpr size_t CUT_SUMS_BYTES = (size_t)CUT_BLOCKS * 128 * 128 * 4;
+static_assert(TICKET_CUTS + CUT_BLOCKS <= TICKET_WORDS, "a ticket per shared tile");
 
 // The static device array of the allocation-free decode entry point (ctx_api.hip).
 constexpr size_t STATIC_SCRATCH_BYTES = (size_t)4 << 20;

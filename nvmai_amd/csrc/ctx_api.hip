@@ -63,6 +63,12 @@ extern "C" int nvmai_hip_ctx_create(int device, int act_dtype, nvmai_hip_ctx** o
         delete ctx;
         return NVMAI_ERR_HIP;
     }
+    // allocated here and not by the call that first needs it, which may be captured; products are made without it too
+    ctx->cut_sums = nullptr;
+    if (hipMalloc(reinterpret_cast<void**>(&ctx->cut_sums), CUT_SUMS_BYTES) != hipSuccess) {
+        (void)hipGetLastError();
+        ctx->cut_sums = nullptr;
+    }
     // device address of this device's static scratch array (nullptr if the lookup fails: only the
     // allocation-free entry point needs it, and it then reports the failure)
     ctx->static_scratch = nullptr;
@@ -76,6 +82,7 @@ extern "C" void nvmai_hip_ctx_destroy(nvmai_hip_ctx* ctx) {
     if (ctx->ws) (void)hipFree(ctx->ws);
     for (void* block : ctx->ws_retired) (void)hipFree(block);
     if (ctx->tickets) (void)hipFree(ctx->tickets);
+    if (ctx->cut_sums) (void)hipFree(ctx->cut_sums);
     for (auto& sp : ctx->prof_spans) { (void)hipEventDestroy(sp.start); (void)hipEventDestroy(sp.stop); }
     for (auto& e : ctx->prof_free) (void)hipEventDestroy(e);
     delete ctx;

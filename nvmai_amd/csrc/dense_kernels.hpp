@@ -9,6 +9,7 @@ namespace nvmai {
 
 typedef __bf16 dn_b8 __attribute__((ext_vector_type(8)));
 typedef float dn_f4 __attribute__((ext_vector_type(4)));
+typedef uint32_t dn_u4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ dn_f4 dn_mfma(const uint4& a, const uint4& b, dn_f4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_b8, a), __builtin_bit_cast(dn_b8, b), c, 0, 0, 0);
@@ -564,20 +565,93 @@ __device__ __forceinline__ float dense_sum_again(const DenseLinearParams& p, uin
     return wave_sum_bcast(sum);
 }
 
-// Which tile a block takes.
+// Which tile a block takes, and which part of its k.
 struct DenseTileAt {
-    uint32_t m, n;
+    uint32_t m, n, tile, part;
 };
 
-__device__ __forceinline__ DenseTileAt dense_tile_at(uint32_t tiles_n, uint32_t tiles_m) {
-    // blocks are dealt to the eight XCDs in turn: give each XCD a run of neighbouring tiles (shared L2 lines)
-    const uint32_t all = tiles_n * tiles_m, xcd = blockIdx.x & 7u, nth = blockIdx.x >> 3;
+__device__ __forceinline__ DenseTileAt dense_tile_at(uint32_t tiles_n, uint32_t tiles_m, uint32_t parts = 1) {
+    // blocks are dealt to the eight XCDs in turn: give each XCD a run of neighbouring tiles (shared L2 lines); parts of k
+    // outermost, so that an XCD reads as little of both operands as can be
+    const uint32_t tiles = tiles_n * tiles_m, all = tiles * parts, xcd = blockIdx.x & 7u, nth = blockIdx.x >> 3;
     const uint32_t base = all / 8u, extra = all % 8u;
-    const uint32_t tile = xcd * base + min(xcd, extra) + nth;
+    uint32_t tile = xcd * base + min(xcd, extra) + nth, part = 0;
+    if (parts > 1u) {                                        // a division that a launch without parts is spared
+        part = tile / tiles;
+        tile -= part * tiles;
+    }
     // in bands of eight token tiles, weight tiles outermost within the band
     const uint32_t band = tile / (8u * tiles_n), in_band = tile % (8u * tiles_n);
     const uint32_t band_m = min(8u, tiles_m - band * 8u);
-    return {band * 8u + in_band % band_m, in_band / band_m};
+    return {band * 8u + in_band % band_m, in_band / band_m, tile, part};
+}
+
+// Tiles cut along k: `parts` blocks per tile, whose sums meet in `sums` (one tile of floats per block).  tickets: a zeroed word per tile.
+struct DenseCut {
+    uint32_t parts;
+    float* sums;
+    uint32_t* tickets;
+};
+
+constexpr uint32_t DENSE_PARTS = 16;
+constexpr int COHERENT = 16;                                 // sc1: a store goes through this XCD's L2, a load does not stop at it
+
+// A block's sums of a tile go to memory, and the block that ends last takes all of them back and adds them in the order of k.  Nobody waits: a
+// block that is not the last one has ended.  The stores are written through and have all arrived before the ticket is drawn (a release
+// at device scope would write back everything that this XCD's L2 holds).  Returns whether this block holds the tile's sums.
+template <int TN, int TM>
+__device__ __forceinline__ bool dense_join(dn_f16 (&sum)[TN][TM], const DenseCut& cut, const DenseTileAt& at, uint32_t* shared) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    constexpr uint32_t WAVE = TN * TM * 4096u, TILE = 4u * WAVE;                    // bytes
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, own = wave * WAVE + lane * 16u;
+    float* const sums = cut.sums + (size_t)at.tile * cut.parts * (TILE / 4u);
+    const __amdgpu_buffer_rsrc_t all = __builtin_amdgcn_make_buffer_rsrc(sums, 0, (int)(cut.parts * TILE), 0x00020000);
+#pragma unroll
+    for (int a = 0; a < TN; ++a)
+#pragma unroll
+        for (int b = 0; b < TM; ++b)
+#pragma unroll
+            for (int h = 0; h < 4; ++h) {
+                const dn_f16& v = sum[a][b];
+                const dn_f4 q{v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]};
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(dn_u4, q), all, own + ((a * TM + b) * 4 + h) * 1024u, at.part * TILE, COHERENT);
+            }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t before = __hip_atomic_fetch_add(cut.tickets + at.tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const bool last = before == cut.parts - 1u;
+        if (last) __hip_atomic_store(cut.tickets + at.tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // ready for the next launch
+        *shared = last;
+    }
+    __syncthreads();
+    if (*shared == 0u) return false;
+    __syncthreads();                                         // the word is read: its place is free
+#pragma unroll
+    for (int a = 0; a < TN; ++a)
+#pragma unroll
+        for (int b = 0; b < TM; ++b) sum[a][b] = dn_f16{};
+#pragma unroll 2
+    for (uint32_t part = 0; part < cut.parts; ++part) {
+        dn_f4 q[TN][TM][4];
+#pragma unroll
+        for (int a = 0; a < TN; ++a)
+#pragma unroll
+            for (int b = 0; b < TM; ++b)
+#pragma unroll
+                for (int h = 0; h < 4; ++h)
+                    q[a][b][h] = __builtin_bit_cast(dn_f4, __builtin_amdgcn_raw_buffer_load_b128(all, own + ((a * TM + b) * 4 + h) * 1024u, part * TILE, COHERENT));
+#pragma unroll
+        for (int a = 0; a < TN; ++a)
+#pragma unroll
+            for (int b = 0; b < TM; ++b)
+#pragma unroll
+                for (int h = 0; h < 4; ++h)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sum[a][b][4 * h + e] += q[a][b][h][e];
+    }
+#endif
+    return true;
 }
 
 // Of 160 KB, one block per compute unit; 64 x 64 tiles of 16-bit inputs fit twice.  Planes come in threes: six stages where they fit
@@ -589,7 +663,7 @@ constexpr int dense_stages(int act, int bn, int bm) {
 constexpr int dense_blocks(int act, int bn, int bm) { return 2 * dense_stages(act, bn, bm) * (bn + bm) * 128 <= 160 * 1024 ? 2 : 1; }
 
 template <int EPI, int ACT, int BN, int BM>
-__global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_kernel(DenseLinearParams p, uint32_t tiles_n, uint32_t tiles_m) {
+__global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_kernel(DenseLinearParams p, uint32_t tiles_n, uint32_t tiles_m, DenseCut cut) {
     constexpr bool SPLIT = ACT == ACT_FP32;
     constexpr int S = dense_stages(ACT, BN, BM);
     constexpr int LA = BN / 32, LB = BM / 32, L = LA + LB;   // 1 KB requests per wave and stage
@@ -597,10 +671,17 @@ __global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_ker
     constexpr uint32_t STAGE = (BN + BM) * 128u;
     __shared__ __attribute__((aligned(1024))) uint8_t l0[STAGE], l1[STAGE], l2[STAGE], l3[S > 3 ? STAGE : 16], l4[S > 4 ? STAGE : 16], l5[S > 5 ? STAGE : 16];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const DenseTileAt at = dense_tile_at(tiles_n, tiles_m);
+    const DenseTileAt at = dense_tile_at(tiles_n, tiles_m, cut.parts);
     const uint32_t m0 = at.m * BM, n0 = at.n * BN;
 
-    const uint32_t steps = p.k / 64u * (SPLIT ? 3u : 1u);
+    // the part's first 64 k and how many: all of them, or an even share
+    uint32_t first = 0, steps = p.k / 64u;
+    if (cut.parts > 1u) {
+        const uint32_t all = steps;
+        first = all * at.part / cut.parts;
+        steps = all * (at.part + 1u) / cut.parts - first;
+    }
+    if (SPLIT) steps *= 3u;
     [[maybe_unused]] const uint32_t w_bytes = (p.n - 1u) * p.w_stride * 2u + p.k * 2u;
     [[maybe_unused]] const uint32_t x_bytes = (p.rows - 1u) * p.x_stride * 2u + p.k * (SPLIT ? 6u : 2u);
     const uint32_t lr = lane >> 3, piece = ((lane & 7u) ^ (lr & 7u)) * 16u;
@@ -614,7 +695,7 @@ __global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_ker
         const bool live = st < steps;
         const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.w), 0, live ? (int)w_bytes : 0, 0x00020000);
         const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.x), 0, live ? (int)x_bytes : 0, 0x00020000);
-        const uint32_t wk = (SPLIT ? st / 3u : st) * 128u, xk = SPLIT ? wk + j % 3 * p.k * 2u : wk;
+        const uint32_t wk = (first + (SPLIT ? st / 3u : st)) * 128u, xk = SPLIT ? wk + j % 3 * p.k * 2u : wk;
         uint8_t* dst = buf(j);
 #pragma unroll
         for (int r = 0; r < L; ++r) {
@@ -697,6 +778,13 @@ __global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_ker
     for (int j = 0; j < S - 1; ++j)
         if (st + (uint32_t)j < steps) step(st + j, j);
     dense_stage_barrier<0>();                                // no request outlives its block; the stages' places are free
+    if (cut.parts > 1u) {
+        if constexpr (SPLIT) {
+            if (!dense_join<TN, TM>(total, cut, at, reinterpret_cast<uint32_t*>(l2))) return;
+        } else {
+            if (!dense_join<TN, TM>(acc, cut, at, reinterpret_cast<uint32_t*>(l2))) return;
+        }
+    }
     // The sums change places through LDS, 32 tokens of the wave's part at a time, so that neighbouring lanes hold
     // neighbouring outputs of one token (stores of whole lines) and what stands between sum and store is a short loop: unrolled
     // over the sums of a tile it is longer than the instruction cache (GELU on 256 x 128: 122 us instead of 71 for 2048 x 8192 x 2048).
@@ -970,28 +1058,44 @@ int gemv(const DenseLinearParams& p, hipStream_t s) {
     return launch_status();
 }
 
-// Which tile: the one whose rounds over the compute units take the least time.  A step of 64 k takes `full` where every unit
+// Which tile, and how many parts of k: those whose rounds over the compute units take the least time.  A step of 64 k takes `full` where every unit
 // has a tile and `lone` where few have one (in 10 ns; measured at k 2048 and 8192 over 65 .. 4096 rows and 256 .. 11264 weight
 // rows: the choice is the fastest of the five or within a tenth of it).  Large tiles read each operand less often, small
 // ones leave fewer units idle.
+//   Tiles that are fewer than the units are cut along k, in 2, 3, 4, 6, 8, 12 or 16 parts of two steps at least, as long as every part has a unit of its
+// own: a step's latency is then paid by all units at once.  The join costs a trip to memory and back, the parts' sums that the last block takes back and
+// the sums of all.  Rows x n x k, cold weights, uncut and cut, us: 65 x 2048 x 8192 27.6 and 14.0, 128 x 2048 x 5632 28.9 and 13.7, 300 x 1024 x 4096
+// 18.4 and 11.6, 700 x 2048 x 8192 47.9 and 39.9, 128 x 256 x 2048 8.8 and 6.7; 32-bit rows 20 x 1024 x 4096 43 and 15, 128 x 1024 x 2816 34 and 16,
+// 500 x 1024 x 4096 50 and 31; level at 300 x 1024 x 2816 uncut 11.1, cut 10.0.  Over 140 sizes the choice is 1 % from the fastest, 21 % at most.
 struct DenseTile {
     uint32_t bn, bm, lone, full;
 };
 constexpr DenseTile DENSE_TILES[] = {{64, 64, 19, 21}, {128, 64, 24, 34}, {128, 128, 30, 55}, {256, 128, 50, 100}, {256, 256, 105, 168}};
+constexpr int DENSE_CUT_TILES = 3;                           // of these the first may be cut along k
 
 struct DensePlan {
     int tile;
+    uint32_t parts;
     uint64_t ns;
 };
 
-inline DensePlan dense_plan_tile(uint32_t n, uint32_t rows, uint32_t steps, uint32_t cus, int count) {
-    DensePlan best{0, ~0ull};
+// planes: the stages of 64 k.  cut: whether there is a place for the sums of parts.
+inline DensePlan dense_plan_tile(uint32_t n, uint32_t rows, uint32_t k, uint32_t planes, uint32_t cus, int count, bool cut) {
+    DensePlan best{0, 1, ~0ull};
+    const uint32_t steps = k / 64u;
     for (int c = 0; c < count; ++c) {
         const DenseTile& t = DENSE_TILES[c];
         const uint64_t tiles = (uint64_t)((n + t.bn - 1) / t.bn) * ((rows + t.bm - 1) / t.bm), rest = tiles % cus;
         const uint64_t cost = tiles / cus * t.full + (rest ? t.lone + (t.full - t.lone) * rest / cus : 0);
-        const uint64_t ns = cost * 10 * steps + 4000;        // and a launch, the first requests, the stores
-        if (ns < best.ns) best = {c, ns};
+        const uint64_t ns = cost * 10 * steps * planes + 4000;           // and a launch, the first requests, the stores
+        if (ns < best.ns) best = {c, 1, ns};
+        if (!cut || c >= DENSE_CUT_TILES) continue;
+        for (uint32_t parts = 2; parts * 2u <= steps && parts <= DENSE_PARTS && tiles * parts <= cus; parts += parts < 4u ? 1u : parts / 4u * 2u) {
+            const uint64_t step = t.lone + (t.full - t.lone) * tiles * parts / cus;
+            const uint64_t join = 1750 + (uint64_t)parts * t.bn * t.bm / 15 + tiles * parts * t.bn * t.bm / 5000;
+            const uint64_t ns = step * 10 * ((steps + parts - 1) / parts) * planes + 4000 + join;
+            if (ns < best.ns) best = {c, parts, ns};
+        }
     }
     return best;
 }
@@ -999,40 +1103,43 @@ inline DensePlan dense_plan_tile(uint32_t n, uint32_t rows, uint32_t steps, uint
 // The matrix's rows in one launch, or in two where that is shorter: a last round that few units take part in is left to
 // smaller tiles (8208 weight rows, 2048 tokens: one round of 256 x 256 and a sixteenth of one, 105 -> 76 us in all).
 // Returns how many rows the first launch takes.
-inline uint32_t dense_plan(uint32_t n, uint32_t rows, uint32_t steps, uint32_t cus, int count) {
-    DensePlan best = dense_plan_tile(n, rows, steps, cus, count);
+inline uint32_t dense_plan(uint32_t n, uint32_t rows, uint32_t k, uint32_t planes, uint32_t cus, int count, bool split) {
+    DensePlan best = dense_plan_tile(n, rows, k, planes, cus, count, split);
     uint32_t first = n;
     for (int c = 0; c < count; ++c) {
         const uint32_t tm = (rows + DENSE_TILES[c].bm - 1) / DENSE_TILES[c].bm, tn = n / DENSE_TILES[c].bn;
         const uint32_t rounds = (uint32_t)((uint64_t)tn * tm / cus);
         const uint32_t cut = rounds ? (uint32_t)((uint64_t)rounds * cus / tm) * DENSE_TILES[c].bn : 0;
         if (cut == 0 || cut >= n) continue;
-        const uint64_t ns = dense_plan_tile(cut, rows, steps, cus, count).ns + dense_plan_tile(n - cut, rows, steps, cus, count).ns;
+        const uint64_t ns = dense_plan_tile(cut, rows, k, planes, cus, count, split).ns + dense_plan_tile(n - cut, rows, k, planes, cus, count, split).ns;
         if (ns < best.ns) { best.ns = ns; first = cut; }
     }
     return first;
 }
 
 template <int EPI, int ACT, int COUNT>
-void launch_tile(hipStream_t s, const DenseLinearParams& p, int c) {
-    const uint32_t tn = (p.n + DENSE_TILES[c].bn - 1) / DENSE_TILES[c].bn, tm = (p.rows + DENSE_TILES[c].bm - 1) / DENSE_TILES[c].bm;
-    if (c == 0) dense_tile_kernel<EPI, ACT, 64, 64><<<tn * tm, 256, 0, s>>>(p, tn, tm);
-    else if (c == 1) dense_tile_kernel<EPI, ACT, 128, 64><<<tn * tm, 256, 0, s>>>(p, tn, tm);
-    else if (c == 2) dense_tile_kernel<EPI, ACT, 128, 128><<<tn * tm, 256, 0, s>>>(p, tn, tm);
+void launch_tile(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p, const DensePlan& plan) {
+    const int c = plan.tile;
+    const uint32_t tn = (p.n + DENSE_TILES[c].bn - 1) / DENSE_TILES[c].bn, tm = (p.rows + DENSE_TILES[c].bm - 1) / DENSE_TILES[c].bm, blocks = tn * tm * plan.parts;
+    const DenseCut cut{plan.parts, ctx->cut_sums, ctx->tickets + TICKET_CUTS};
+    if (c == 0) dense_tile_kernel<EPI, ACT, 64, 64><<<blocks, 256, 0, s>>>(p, tn, tm, cut);
+    else if (c == 1) dense_tile_kernel<EPI, ACT, 128, 64><<<blocks, 256, 0, s>>>(p, tn, tm, cut);
+    else if (c == 2) dense_tile_kernel<EPI, ACT, 128, 128><<<blocks, 256, 0, s>>>(p, tn, tm, cut);
     if constexpr (COUNT > 3) {
-        if (c == 3) dense_tile_kernel<EPI, ACT, 256, 128><<<tn * tm, 256, 0, s>>>(p, tn, tm);
-        else if (c == 4) dense_wide_kernel<EPI><<<tn * tm, 256, 0, s>>>(p, tn, tm);
+        if (c == 3) dense_tile_kernel<EPI, ACT, 256, 128><<<blocks, 256, 0, s>>>(p, tn, tm, cut);
+        else if (c == 4) dense_wide_kernel<EPI><<<blocks, 256, 0, s>>>(p, tn, tm);
     }
 }
 
 template <int EPI, int ACT>
 void launch_tiles(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p) {
     constexpr int COUNT = ACT == ACT_FP32 ? 3 : 5;           // 32-bit inputs keep a running total beside the sums: no registers for the larger tiles
-    const uint32_t cus = (uint32_t)ctx->compute_units, steps = p.k / 64u * (ACT == ACT_FP32 ? 3u : 1u);
-    const uint32_t first = dense_plan(p.n, p.rows, steps, cus, COUNT);
+    const uint32_t cus = (uint32_t)ctx->compute_units, planes = ACT == ACT_FP32 ? 3u : 1u;
+    const bool cut = ctx->cut_sums != nullptr && cus <= CUT_BLOCKS;
+    const uint32_t first = dense_plan(p.n, p.rows, p.k, planes, cus, COUNT, cut);
     DenseLinearParams q = p;
     q.n = first;
-    launch_tile<EPI, ACT, COUNT>(s, q, dense_plan_tile(q.n, q.rows, steps, cus, COUNT).tile);
+    launch_tile<EPI, ACT, COUNT>(ctx, s, q, dense_plan_tile(q.n, q.rows, q.k, planes, cus, COUNT, cut));
     if (first == p.n) return;
     q.n = p.n - first;                                       // first is a multiple of 64: every operand stays aligned
     q.w = p.w + (size_t)first * p.w_stride;
@@ -1041,7 +1148,7 @@ void launch_tiles(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p)
     if (p.y_f32) q.y_f32 = p.y_f32 + out;
     if (p.bias) q.bias = p.bias + first;
     if (p.mul) q.mul = p.mul + first;
-    launch_tile<EPI, ACT, COUNT>(s, q, dense_plan_tile(q.n, q.rows, steps, cus, COUNT).tile);
+    launch_tile<EPI, ACT, COUNT>(ctx, s, q, dense_plan_tile(q.n, q.rows, q.k, planes, cus, COUNT, cut));
 }
 
 // 32-bit inputs: their planes, in portions of rows, then the product.
