@@ -15,6 +15,23 @@ __device__ __forceinline__ dn_f4 dn_mfma(const uint4& a, const uint4& b, dn_f4 c
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_b8, a), __builtin_bit_cast(dn_b8, b), c, 0, 0, 0);
 }
 
+// The same onto a sum that stays where it is, in the second half of the register file: with 64 sums and 32 operands the compiler moves sums about between
+// products (three copies per product).  The compiler does not see a product here: operands must not come straight from vector instructions, and
+// dn_mfma_done stands before the first use of a sum.
+__device__ __forceinline__ void dn_mfma_in_place(const uint4& a, const uint4& b, dn_f4& c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(__builtin_bit_cast(dn_u4, a)), "v"(__builtin_bit_cast(dn_u4, b)));
+#endif
+}
+
+// The last product's sum is written.
+__device__ __forceinline__ void dn_mfma_done() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#endif
+}
+
 // z/2 (1 + erf(z / sqrt 2))
 __device__ __forceinline__ float gelu_erf(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
 
@@ -514,15 +531,19 @@ __global__ __launch_bounds__(skinny_threads(TT, NW, V)) void dense_skinny_kernel
 }
 
 // ---- many input rows: tiles of BN weight rows x BM tokens, k in steps of 64 through a ring of S stages in LDS ----------
-// Four waves, each a quarter of the tile (BN / 2 x BM / 2) in 32 x 32 x 16 products.  Bound by the rate at which a compute
-// unit takes operands into LDS (about 60 bytes per ns; a tile of 256 x 256 is where the products take as long) and, below
-// one tile per compute unit, by the latency of a step.  A tile's rows are 128 bytes of LDS; the eight 16-byte pieces of
-// row r lie in the order piece ^ (r % 8), so that the rows of an operand read fall into different banks.
-//   A stage is multiplied in four phases of 16 k.  The operands of the next phase are read, and a quarter of the stage S - 1
-// ahead is requested, between the products of a phase: a wave alone on its SIMD has products to issue at all times, and
+// Four waves, each a quarter of the tile (BN / 2 x BM / 2) in 16 x 16 x 32 products.  Bound by the rate at which a compute
+// unit takes operands into LDS (about 60 bytes per ns; a tile of 256 x 256 is where the products take as long), below
+// one tile per compute unit by the latency of a step, and where all units multiply by the clock that the card's power leaves.  A tile's rows are 128 bytes
+// of LDS, whose eight 16-byte pieces lie in the order piece ^ skinny_swizzle(row); an operand is read as there.
+//   Which products, and in which order, is a matter of power.  From registers alone, random values, all units: 32 x 32 x 16 1,750 TFLOP/s,
+// 16 x 16 x 32 with the first operand held for runs and the second going to and fro 2,070, in any order that changes the first each time 1,570 to 1,750.
+// With 32 x 32 x 16 these kernels also left the clock of whatever ran next 13 % lower (a router product of 58 us took 66 beside them; 59 now).
+// 2048 x 2048 x 2048 22.5 -> 19.9 us, 4096 x 12,288 x 2048 in the tiles of 256 x 256 below 176 -> 160.
+//   A stage is multiplied in four phases, half of the weight rows by 32 k each.  The operands of the phases after the next one are read, and a quarter of a
+// stage ahead is requested, between the products of a phase: a wave alone on its SIMD has products to issue at all times, and
 // requests spread over the phases keep the wave from waiting at the memory pipe (in one burst behind the barrier: 96 us for
 // 2048 x 2048 x 8192 in tiles of 256 x 128, spread 93, and 125 with a branch around the burst).  One barrier per stage,
-// before its last phase: by then every wave has read the stage to its end (its place is free for stage + S) and waits for
+// in its middle: by then every wave has read the stage to its end (its place is free for stage + S) and waits for
 // its own part of the next one.  Requests are never conditional, so the counter's meaning is the same in every step; a
 // stage past the last reads no bytes (a buffer of size 0).  Stages are separate arrays: the compiler then knows
 // which requests a read of LDS has to wait for.
@@ -530,12 +551,6 @@ __global__ __launch_bounds__(skinny_threads(TT, NW, V)) void dense_skinny_kernel
 // of 64 k are exact, and their sum goes to a running total of its own, which keeps the rounding of a long k small.
 // Measured (tiles of 128 x 128 x 64 in two stages before): 2048 x 8192 x 2048 77 -> 64 us, 2048 x 2048 x 8192 140 -> 67, 1501 x
 // 2048 x 2048 34 -> 17, 512 x 2048 x 2048 33 -> 9.5 (rows x n x k, cold weights).
-typedef float dn_f16 __attribute__((ext_vector_type(16)));
-
-__device__ __forceinline__ dn_f16 dn_mfma32(const uint4& a, const uint4& b, dn_f16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(dn_b8, a), __builtin_bit_cast(dn_b8, b), c, 0, 0, 0);
-}
-
 // One sum of the planes again by a whole wave, in fp32 multiply-adds of the values that the planes stand for.  An infinite weight makes
 // NaN of a value's lower planes where they are zero, and planes of sums that overflow can cancel: a NaN comes from here or not
 // at all.  It ends where the sum has become NaN, which it stays; poisoned: by an input that is NaN, so that all sums of its row are.
@@ -600,9 +615,9 @@ constexpr int COHERENT = 16;                                 // sc1: a store goe
 // block that is not the last one has ended.  The stores are written through and have all arrived before the ticket is drawn (a release
 // at device scope would write back everything that this XCD's L2 holds).  Returns whether this block holds the tile's sums.
 template <int TN, int TM>
-__device__ __forceinline__ bool dense_join(dn_f16 (&sum)[TN][TM], const DenseCut& cut, const DenseTileAt& at, uint32_t* shared) {
+__device__ __forceinline__ bool dense_join(dn_f4 (&sum)[TN][TM], const DenseCut& cut, const DenseTileAt& at, uint32_t* shared) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    constexpr uint32_t WAVE = TN * TM * 4096u, TILE = 4u * WAVE;                    // bytes
+    constexpr uint32_t WAVE = TN * TM * 1024u, TILE = 4u * WAVE;                    // bytes
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, own = wave * WAVE + lane * 16u;
     float* const sums = cut.sums + (size_t)at.tile * cut.parts * (TILE / 4u);
     const __amdgpu_buffer_rsrc_t all = __builtin_amdgcn_make_buffer_rsrc(sums, 0, (int)(cut.parts * TILE), 0x00020000);
@@ -610,12 +625,7 @@ __device__ __forceinline__ bool dense_join(dn_f16 (&sum)[TN][TM], const DenseCut
     for (int a = 0; a < TN; ++a)
 #pragma unroll
         for (int b = 0; b < TM; ++b)
-#pragma unroll
-            for (int h = 0; h < 4; ++h) {
-                const dn_f16& v = sum[a][b];
-                const dn_f4 q{v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]};
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(dn_u4, q), all, own + ((a * TM + b) * 4 + h) * 1024u, at.part * TILE, COHERENT);
-            }
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(dn_u4, sum[a][b]), all, own + (a * TM + b) * 1024u, at.part * TILE, COHERENT);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -630,25 +640,19 @@ __device__ __forceinline__ bool dense_join(dn_f16 (&sum)[TN][TM], const DenseCut
 #pragma unroll
     for (int a = 0; a < TN; ++a)
 #pragma unroll
-        for (int b = 0; b < TM; ++b) sum[a][b] = dn_f16{};
+        for (int b = 0; b < TM; ++b) sum[a][b] = dn_f4{};
 #pragma unroll 2
     for (uint32_t part = 0; part < cut.parts; ++part) {
-        dn_f4 q[TN][TM][4];
+        dn_f4 q[TN][TM];
 #pragma unroll
         for (int a = 0; a < TN; ++a)
 #pragma unroll
             for (int b = 0; b < TM; ++b)
-#pragma unroll
-                for (int h = 0; h < 4; ++h)
-                    q[a][b][h] = __builtin_bit_cast(dn_f4, __builtin_amdgcn_raw_buffer_load_b128(all, own + ((a * TM + b) * 4 + h) * 1024u, part * TILE, COHERENT));
+                q[a][b] = __builtin_bit_cast(dn_f4, __builtin_amdgcn_raw_buffer_load_b128(all, own + (a * TM + b) * 1024u, part * TILE, COHERENT));
 #pragma unroll
         for (int a = 0; a < TN; ++a)
 #pragma unroll
-            for (int b = 0; b < TM; ++b)
-#pragma unroll
-                for (int h = 0; h < 4; ++h)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) sum[a][b][4 * h + e] += q[a][b][h][e];
+            for (int b = 0; b < TM; ++b) sum[a][b] += q[a][b];
     }
 #endif
     return true;
@@ -667,7 +671,7 @@ __global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_ker
     constexpr bool SPLIT = ACT == ACT_FP32;
     constexpr int S = dense_stages(ACT, BN, BM);
     constexpr int LA = BN / 32, LB = BM / 32, L = LA + LB;   // 1 KB requests per wave and stage
-    constexpr int TN = BN / 64, TM = BM / 64;                // 32 x 32 tiles per wave
+    constexpr int TN = BN / 32, TM = BM / 32;                // 16 x 16 tiles per wave
     constexpr uint32_t STAGE = (BN + BM) * 128u;
     __shared__ __attribute__((aligned(1024))) uint8_t l0[STAGE], l1[STAGE], l2[STAGE], l3[S > 3 ? STAGE : 16], l4[S > 4 ? STAGE : 16], l5[S > 5 ? STAGE : 16];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -684,10 +688,12 @@ __global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_ker
     if (SPLIT) steps *= 3u;
     [[maybe_unused]] const uint32_t w_bytes = (p.n - 1u) * p.w_stride * 2u + p.k * 2u;
     [[maybe_unused]] const uint32_t x_bytes = (p.rows - 1u) * p.x_stride * 2u + p.k * (SPLIT ? 6u : 2u);
-    const uint32_t lr = lane >> 3, piece = ((lane & 7u) ^ (lr & 7u)) * 16u;
+    const uint32_t lr = lane >> 3;
+    // request r of a wave: rows 8 r .. 8 r + 7 of its part (8 r + lane / 8 has two values of the swizzle)
+    [[maybe_unused]] const uint32_t piece[2] = {((lane & 7u) ^ skinny_swizzle(lr)) * 16u, ((lane & 7u) ^ skinny_swizzle(lr + 8u)) * 16u};
     // rows past the last: the last one, whose sums are not stored
-    [[maybe_unused]] const uint32_t a8 = p.w_stride * 16u, a0 = (n0 + wave * (LA * 8u) + lr) * p.w_stride * 2u + piece, amax = (p.n - 1u) * p.w_stride * 2u + piece;
-    [[maybe_unused]] const uint32_t b8 = p.x_stride * 16u, b0 = (m0 + wave * (LB * 8u) + lr) * p.x_stride * 2u + piece, bmax = (p.rows - 1u) * p.x_stride * 2u + piece;
+    [[maybe_unused]] const uint32_t a8 = p.w_stride * 16u, a0 = (n0 + wave * (LA * 8u) + lr) * p.w_stride * 2u, amax = (p.n - 1u) * p.w_stride * 2u;
+    [[maybe_unused]] const uint32_t b8 = p.x_stride * 16u, b0 = (m0 + wave * (LB * 8u) + lr) * p.x_stride * 2u, bmax = (p.rows - 1u) * p.x_stride * 2u;
     auto buf = [&](int j) -> uint8_t* { return j == 0 ? l0 : j == 1 ? l1 : j == 2 ? l2 : j == 3 ? l3 : j == 4 ? l4 : l5; };
     // requests [from, to) of stage st into its place j = st % S (of a 32-bit input: plane j % 3, S is 3 or 6)
     auto request = [&](uint32_t st, int j, int from, int to) {
@@ -700,61 +706,71 @@ __global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_ker
 #pragma unroll
         for (int r = 0; r < L; ++r) {
             if (r < from || r >= to) continue;
-            if (r < LA) __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (__attribute__((address_space(3))) void*)(dst + (wave * LA + r) * 1024u), 16, min(a0 + r * a8, amax), wk, 0, 0);
-            else __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void*)(dst + BN * 128u + (wave * LB + r - LA) * 1024u), 16, min(b0 + (r - LA) * b8, bmax), xk, 0, 0);
+            if (r < LA) __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (__attribute__((address_space(3))) void*)(dst + (wave * LA + r) * 1024u), 16, min(a0 + r * a8, amax) + piece[r & 1], wk, 0, 0);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void*)(dst + BN * 128u + (wave * LB + r - LA) * 1024u), 16, min(b0 + (r - LA) * b8, bmax) + piece[(r - LA) & 1], xk, 0, 0);
         }
 #endif
     };
-    const uint32_t i = lane & 31u, g = lane >> 5;
+    const uint32_t i = lane & 15u, g = lane >> 4;
     const uint32_t wn = (wave >> 1) * (BN / 2), wm = (wave & 1u) * (BM / 2);
     const uint32_t arow = (wn + i) * 128u, brow = BN * 128u + (wm + i) * 128u;
     uint4 fa[2][TN], fb[2][TM];
-    auto fetch = [&](int j, uint32_t q) {                    // the operands of phase q of the stage at place j
-        const uint32_t sw = ((q * 2u + g) ^ (i & 7u)) * 16u;
+    // operands of the half h (32 k: the pieces 2 g + h) of the stage at place j: the tokens' and the first half of the weights' (part 0), the rest (part 1)
+    auto fetch = [&](int j, int h, int part) {
+        const uint32_t sw = ((2u * g + h) ^ skinny_swizzle(i)) * 16u;
+        if (part == 0) {
 #pragma unroll
-        for (int b = 0; b < TM; ++b) fb[q & 1u][b] = *reinterpret_cast<const uint4*>(buf(j) + brow + 4096u * b + sw);
+            for (int b = 0; b < TM; ++b) fb[h][b] = *reinterpret_cast<const uint4*>(buf(j) + brow + 2048u * b + sw);
+        }
 #pragma unroll
-        for (int a = 0; a < TN; ++a) fa[q & 1u][a] = *reinterpret_cast<const uint4*>(buf(j) + arow + 4096u * a + sw);
+        for (int a = part * (TN / 2); a < (part + 1) * (TN / 2); ++a) fa[h][a] = *reinterpret_cast<const uint4*>(buf(j) + arow + 2048u * a + sw);
     };
-    dn_f16 acc[TN][TM];
-    [[maybe_unused]] dn_f16 total[SPLIT ? TN : 1][SPLIT ? TM : 1];
+    dn_f4 acc[TN][TM];
+    [[maybe_unused]] dn_f4 total[SPLIT ? TN : 1][SPLIT ? TM : 1];
 #pragma unroll
     for (int a = 0; a < TN; ++a)
 #pragma unroll
         for (int b = 0; b < TM; ++b) {
-            acc[a][b] = dn_f16{};
-            if constexpr (SPLIT) total[a][b] = dn_f16{};
+            acc[a][b] = dn_f4{};
+            if constexpr (SPLIT) total[a][b] = dn_f4{};
         }
-    auto multiply = [&](int q, auto requests, bool fresh) {
-        constexpr int NP = TN * TM, NF = TN + TM, NR = decltype(requests)::value;
+    // phase q: half q / 2 of the stage, the weights' half q % 2; a weight operand stays for a run, a token operand from one run to the next
+    auto multiply = [&](auto phase, auto requests, bool fresh) {
+        constexpr int Q = decltype(phase)::value, H = Q / 2, NP = TN * TM / 2, NF = TN / 2 + (Q % 2 == 0 ? TM : 0), NR = decltype(requests)::value;
 #pragma unroll
-        for (int a = 0; a < TN; ++a)
-#pragma unroll
-            for (int b = 0; b < TM; ++b) acc[a][b] = dn_mfma32(fa[q & 1][a], fb[q & 1][b], fresh ? dn_f16{} : acc[a][b]);
+        for (int e = 0; e < NP; ++e) {
+            const int a = Q % 2 * (TN / 2) + e / TM, b = a & 1 ? TM - 1 - e % TM : e % TM;
+            acc[a][b] = dn_mfma(fa[H][a], fb[H][b], fresh ? dn_f4{} : acc[a][b]);
+        }
 #pragma unroll
         for (int k = 0; k < NP; ++k) {
             __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);                                     // a product,
-            __builtin_amdgcn_sched_group_barrier(0x100, (NF + NP - 1) / NP, 0);                  // the next phase's operands,
+            __builtin_amdgcn_sched_group_barrier(0x100, (NF + NP - 1) / NP, 0);                  // operands to come,
             if constexpr (NR > 0) __builtin_amdgcn_sched_group_barrier(0x20, (NR + NP - 1) / NP, 0);  // and the requests
         }
         __builtin_amdgcn_sched_barrier(0);
     };
 #define NVMAI_SHARE(q) (L * (q) / 4)
+#define NVMAI_SHARES(q) std::integral_constant<int, NVMAI_SHARE(q + 1) - NVMAI_SHARE(q)>{}
+    constexpr std::integral_constant<int, 0> q0{};
+    constexpr std::integral_constant<int, 1> q1{};
+    constexpr std::integral_constant<int, 2> q2{};
+    constexpr std::integral_constant<int, 3> q3{};
     auto step = [&](uint32_t st, int j) {
         constexpr int B = S - 1;
-        fetch(j, 1);
-        request(st + B, (j + B) % S, NVMAI_SHARE(1), NVMAI_SHARE(2));
-        multiply(0, std::integral_constant<int, NVMAI_SHARE(2) - NVMAI_SHARE(1)>{}, SPLIT && j % 3 == 0);
-        fetch(j, 2);
+        fetch(j, 1, 0);
         request(st + B, (j + B) % S, NVMAI_SHARE(2), NVMAI_SHARE(3));
-        multiply(1, std::integral_constant<int, NVMAI_SHARE(3) - NVMAI_SHARE(2)>{}, false);
-        fetch(j, 3);
+        multiply(q0, NVMAI_SHARES(2), SPLIT && j % 3 == 0);
+        fetch(j, 1, 1);
         request(st + B, (j + B) % S, NVMAI_SHARE(3), NVMAI_SHARE(4));
-        multiply(2, std::integral_constant<int, NVMAI_SHARE(4) - NVMAI_SHARE(3)>{}, false);
+        multiply(q1, NVMAI_SHARES(3), SPLIT && j % 3 == 0);
         dense_stage_barrier<(S - 2) * L>();
-        fetch((j + 1) % S, 0);
-        request(st + S, j, 0, NVMAI_SHARE(1));
-        multiply(3, std::integral_constant<int, NVMAI_SHARE(1)>{}, false);
+        fetch((j + 1) % S, 0, 0);
+        request(st + S, j, NVMAI_SHARE(0), NVMAI_SHARE(1));
+        multiply(q2, NVMAI_SHARES(0), false);
+        fetch((j + 1) % S, 0, 1);
+        request(st + S, j, NVMAI_SHARE(1), NVMAI_SHARE(2));
+        multiply(q3, NVMAI_SHARES(1), false);
         if constexpr (SPLIT) {
             if (j % 3 == 2) {
 #pragma unroll
@@ -765,10 +781,12 @@ __global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_ker
         }
     };
 #pragma unroll
-    for (int j = 0; j < S; ++j) request(j, j, 0, j == S - 1 ? NVMAI_SHARE(1) : L);
-    dense_stage_barrier<(S - 2) * L + NVMAI_SHARE(1)>();
+    for (int j = 0; j < S; ++j) request(j, j, 0, j == S - 1 ? NVMAI_SHARE(2) : L);
+    dense_stage_barrier<(S - 2) * L + NVMAI_SHARE(2)>();
+#undef NVMAI_SHARES
 #undef NVMAI_SHARE
-    fetch(0, 0);
+    fetch(0, 0, 0);
+    fetch(0, 0, 1);
     uint32_t st = 0;
     for (; st + (uint32_t)S <= steps; st += S) {
 #pragma unroll
@@ -795,22 +813,22 @@ __global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_ker
     const uint32_t r = n0 + wn + lane % PER * 4u;
     const dn_f4 bias = dense_bias4<EPI>(p, r);
 #pragma unroll
-    for (int b = 0; b < TM; ++b) {
+    for (int b = 0; b < TM / 2; ++b) {
         [[maybe_unused]] bool again = false;
 #pragma unroll
-        for (int a = 0; a < TN; ++a) {
-            dn_f16 v = acc[a][b];
-            if constexpr (SPLIT) v = total[a][b];
+        for (int a = 0; a < TN; ++a)
 #pragma unroll
-            for (int h = 0; h < 4; ++h)                      // element 4 h + e of a lane: row 8 h + 4 g + e, token i
-                *reinterpret_cast<dn_f4*>(turn + i * PITCH + 32 * a + 8 * h + 4u * g) = dn_f4{v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]};
-            if constexpr (SPLIT) {
-                bool none = false;
+            for (int t = 0; t < 2; ++t) {                    // element e of a lane: row 4 g + e, token i
+                dn_f4 v = acc[a][2 * b + t];
+                if constexpr (SPLIT) v = total[a][2 * b + t];
+                *reinterpret_cast<dn_f4*>(turn + (16 * t + i) * PITCH + 16 * a + 4u * g) = v;
+                if constexpr (SPLIT) {
+                    bool none = false;
 #pragma unroll
-                for (int e = 0; e < 16; ++e) none |= v[e] != v[e];
-                again |= none;
+                    for (int e = 0; e < 4; ++e) none |= v[e] != v[e];
+                    again |= none;
+                }
             }
-        }
         if constexpr (SPLIT) {
             if (__any(again)) {
                 uint32_t poisoned_token = 32;                // sums of one token follow each other
@@ -842,12 +860,10 @@ __global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_ker
 // stage to arrive.  Here a stage is two halves of both operands (rows 0 .. 63 of every 128, and the others), freed and asked for one by one:
 // a wave's part is four products of half by half, in the order (0, 0), (1, 0), (1, 1), (0, 1), so that the halves 0 are read while the
 // last two products of the stage before run and the halves 1 during the first two; a half is then out of LDS for registers (128 of them hold a
-// stage) one to one and a half stages before its successor is needed.  Barriers stand behind the first four of the sixteen matrix instructions of
-// a product: the reads before them arrive in the meantime.  Requests go out evenly over the stage.  Pieces lie in the order piece ^ (r / 2 % 8):
-// the sixteen lanes that a read serves at once cover 256 bytes.  Bound by the rate of requests into LDS (49 us of the 62 below without the products) and the
-// clock that the products leave.  Rows x n x k, cold weights, former ring of two stages, one call after another: 2048 x 8192 x 2048 63.9 -> 62.2 us, 4096 x 8192 x 2048
-// 123.6 -> 120.5, 2048 x 12,352 x 2048 112 -> 105, 8192 x 8192 x 8192 806 -> 772; in the traces of prompts 64.4 -> 62.3, with GELU 76.8 -> 75.7, pairs of 1501 rows
-// 64.5 -> 63.8.  The costs of the plan below are a little lower than that and choose no worse (156 sizes 1.8 % faster, with costs to the letter 1.4 %).  Not kept: a third place for the halves 0 (no change), requests of 64 bytes per row in stages of 32 k (half
+// stage) one to one and a half stages before its successor is needed.  Barriers stand behind the first eight of the 32 matrix instructions of
+// a product: the reads before them arrive in the meantime.  Requests go out evenly over the stage.  Bound by the rate of requests into LDS and the
+// power of the products.  Rows x n x k, cold weights, with 32 x 32 x 16 products: 4096 x 12,288 x 2048 176 -> 160 us (1,290 TFLOP/s).
+// Not kept: a third place for the halves 0 (no change), requests of 64 bytes per row in stages of 32 k (half
 // the rate).
 template <int EPI>
 __global__ __launch_bounds__(256, 1) void dense_wide_kernel(DenseLinearParams p, uint32_t tiles_n, uint32_t tiles_m) {
@@ -859,10 +875,9 @@ __global__ __launch_bounds__(256, 1) void dense_wide_kernel(DenseLinearParams p,
     const uint32_t m0 = at.m * 256u, n0 = at.n * 256u;
     const uint32_t steps = p.k / 64u;
     [[maybe_unused]] const uint32_t w_bytes = (p.n - 1u) * p.w_stride * 2u + p.k * 2u, x_bytes = (p.rows - 1u) * p.x_stride * 2u + p.k * 2u;
-    auto swizzle = [](uint32_t row) { return (row >> 1) & 7u; };
     // request r of a wave: rows 32 wave + 8 r .. + 7 of a half (8 r + lane / 8 has two values of the swizzle)
     const uint32_t lr = lane >> 3;
-    [[maybe_unused]] const uint32_t piece[2] = {((lane & 7u) ^ swizzle(lr)) * 16u, ((lane & 7u) ^ swizzle(lr + 8u)) * 16u};
+    [[maybe_unused]] const uint32_t piece[2] = {((lane & 7u) ^ skinny_swizzle(lr)) * 16u, ((lane & 7u) ^ skinny_swizzle(lr + 8u)) * 16u};
     const uint32_t row = (wave & 1u) * 32u + (wave >> 1) * 128u + lr;
     [[maybe_unused]] const uint32_t w8 = p.w_stride * 16u, w0 = (n0 + row) * p.w_stride * 2u, wmax = (p.n - 1u) * p.w_stride * 2u;
     [[maybe_unused]] const uint32_t x8 = p.x_stride * 16u, x0 = (m0 + row) * p.x_stride * 2u, xmax = (p.rows - 1u) * p.x_stride * 2u;
@@ -882,22 +897,22 @@ __global__ __launch_bounds__(256, 1) void dense_wide_kernel(DenseLinearParams p,
         }
 #endif
     };
-    const uint32_t i = lane & 31u, g = lane >> 5;
+    const uint32_t i = lane & 15u, g = lane >> 4;
     const uint32_t wn = (wave >> 1) * 128u, wm = (wave & 1u) * 128u;
     const uint32_t arow = ((wave >> 1) * 64u + i) * 128u, brow = ((wave & 1u) * 64u + i) * 128u;
-    uint4 A[2][2][4], B[2][2][4];                            // [half][tile of 32][16 k]
+    uint4 A[2][2][4], B[2][2][4];                            // [half][32 k][tile of 16]
     // operand e of eight of a half
-    auto read_w = [&](int j, int h, int e) { A[h][e & 1][e >> 1] = *reinterpret_cast<const uint4*>(wbuf(j, h) + arow + 4096u * (e & 1) + (((e & ~1u) + g) ^ swizzle(i)) * 16u); };
-    auto read_x = [&](int j, int h, int e) { B[h][e & 1][e >> 1] = *reinterpret_cast<const uint4*>(xbuf(j, h) + brow + 4096u * (e & 1) + (((e & ~1u) + g) ^ swizzle(i)) * 16u); };
-    dn_f16 acc[4][4];
+    auto read_w = [&](int j, int h, int e) { A[h][e >> 2][e & 3] = *reinterpret_cast<const uint4*>(wbuf(j, h) + arow + 2048u * (e & 3) + (((2u * g + (e >> 2)) ^ skinny_swizzle(i)) * 16u)); };
+    auto read_x = [&](int j, int h, int e) { B[h][e >> 2][e & 3] = *reinterpret_cast<const uint4*>(xbuf(j, h) + brow + 2048u * (e & 3) + (((2u * g + (e >> 2)) ^ skinny_swizzle(i)) * 16u)); };
+    dn_f4 acc[8][8];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < 8; ++a)
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = dn_f16{};
-    // matrix instruction e of sixteen of the product of two halves
+        for (int b = 0; b < 8; ++b) acc[a][b] = dn_f4{};
+    // matrix instruction e of 32 of the product of two halves: a weight operand stays for four, a token operand from one four to the next
     auto multiply = [&](int ha, int hb, int e) {
-        const int k = e >> 2, a = (e >> 1) & 1, b = e & 1;
-        acc[2 * ha + a][2 * hb + b] = dn_mfma32(A[ha][a][k], B[hb][b][k], acc[2 * ha + a][2 * hb + b]);
+        const int k = e >> 4, a = (e >> 2) & 3, b = a & 1 ? 3 - (e & 3) : e & 3;
+        dn_mfma_in_place(A[ha][k][a], B[hb][k][b], acc[4 * ha + a][4 * hb + b]);
     };
     // The half products (h, h) and (1 - h, h): the halves 1 - of the weights, then of the tokens, are read under the first two, those of the
     // next stage under the last two, where the weights' half 0 is still an operand and is replaced behind its last use.
@@ -906,29 +921,28 @@ __global__ __launch_bounds__(256, 1) void dense_wide_kernel(DenseLinearParams p,
         for (int h = 0; h < 2; ++h) {
             const int next = h == 0 ? j : 1 - j;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) multiply(h, h, e);
+            for (int e = 0; e < 8; ++e) multiply(h, h, e);
             __builtin_amdgcn_sched_barrier(0);
             dense_stage_barrier<16>();                       // two halves of both operands stay on their way
 #pragma unroll
-            for (int e = 4; e < 16; ++e) {
+            for (int e = 8; e < 32; ++e) {
                 multiply(h, h, e);
-                if (e < 12) {
-                    if (h == 0) read_w(next, 1, e - 4);
-                    else read_x(next, 0, e - 4);
+                if ((e & 1) == 0 && e < 24) {
+                    if (h == 0) read_w(next, 1, (e - 8) / 2);
+                    else read_x(next, 0, (e - 8) / 2);
                 }
-                if (e % 3 == 0) request(st + 2u, j, h, e / 3 - 2);
+                if (e % 6 == 1) request(st + 2u, j, h, e / 6 - 2);
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
+            for (int e = 0; e < 32; ++e) {
                 multiply(1 - h, h, e);
                 if (h == 0) {
-                    if (e < 8) read_x(next, 1, e);
+                    if ((e & 1) == 0 && e < 16) read_x(next, 1, e / 2);
                 } else if ((e & 3) == 3) {
-                    read_w(next, 0, e >> 2 << 1);
-                    read_w(next, 0, (e >> 2 << 1) + 1);
+                    read_w(next, 0, e >> 2);
                 }
-                if (e % 4 == 1) request(st + 2u, j, h, 4 + e / 4);
+                if (e % 8 == 2) request(st + 2u, j, h, 4 + e / 8);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -951,6 +965,7 @@ __global__ __launch_bounds__(256, 1) void dense_wide_kernel(DenseLinearParams p,
         stage(st + 1u, 1);
     }
     if (st < steps) stage(st, 0);
+    dn_mfma_done();
     dense_stage_barrier<0>();                                // no request outlives its block; the places are free
     // The sums change places as in dense_tile_kernel, in a row of 128 per token whose pieces of four are exchanged by the token.
     float* turn = reinterpret_cast<float*>(wave == 0u ? w00 : wave == 1u ? w01 : wave == 2u ? w10 : w11);
@@ -960,12 +975,10 @@ __global__ __launch_bounds__(256, 1) void dense_wide_kernel(DenseLinearParams p,
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
 #pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            const dn_f16 v = acc[a][b];
+        for (int a = 0; a < 8; ++a)
 #pragma unroll
-            for (int h = 0; h < 4; ++h)                      // element 4 h + e of a lane: row 8 h + 4 g + e, token i
-                *reinterpret_cast<dn_f4*>(turn + i * 128u + (((8u * a + 2u * h + g) ^ i) * 4u)) = dn_f4{v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]};
-        }
+            for (int h = 0; h < 2; ++h)                      // element e of a lane: row 4 g + e, token i
+                *reinterpret_cast<dn_f4*>(turn + (16u * h + i) * 128u + (((4u * a + g) ^ (16u * h + i)) * 4u)) = acc[a][2 * b + h];
 #pragma unroll UNROLL
         for (uint32_t k = 0; k < 16u; ++k) {
             const uint32_t token = lane / 32u + k * 2u, t = m0 + wm + 32 * b + token;
@@ -1059,41 +1072,46 @@ int gemv(const DenseLinearParams& p, hipStream_t s) {
 }
 
 // Which tile, and how many parts of k: those whose rounds over the compute units take the least time.  A step of 64 k takes `full` where every unit
-// has a tile and `lone` where few have one (in 10 ns; measured at k 2048 and 8192 over 65 .. 4096 rows and 256 .. 11264 weight
-// rows: the choice is the fastest of the five or within a tenth of it).  Large tiles read each operand less often, small
+// has a tile and `lone` where few have one (in 10 ns; fitted to every tile and part at k 1024 .. 8192 over 20 .. 2900 rows and 128 .. 11,264 weight
+// rows).  Large tiles read each operand less often, small
 // ones leave fewer units idle.
 //   Tiles that are fewer than the units are cut along k, in 2, 3, 4, 6, 8, 12 or 16 parts of two steps at least, as long as every part has a unit of its
 // own: a step's latency is then paid by all units at once.  The join costs a trip to memory and back, the parts' sums that the last block takes back and
 // the sums of all.  Rows x n x k, cold weights, uncut and cut, us: 65 x 2048 x 8192 27.6 and 14.0, 128 x 2048 x 5632 28.9 and 13.7, 300 x 1024 x 4096
 // 18.4 and 11.6, 700 x 2048 x 8192 47.9 and 39.9, 128 x 256 x 2048 8.8 and 6.7; 32-bit rows 20 x 1024 x 4096 43 and 15, 128 x 1024 x 2816 34 and 16,
-// 500 x 1024 x 4096 50 and 31; level at 300 x 1024 x 2816 uncut 11.1, cut 10.0.  Over 140 sizes the choice is 1 % from the fastest, 21 % at most.
+// 500 x 1024 x 4096 50 and 31; level at 300 x 1024 x 2816 uncut 11.1, cut 10.0.  Over 155 sizes the choice is 0.7 % from the fastest, 15 % at most.
 struct DenseTile {
     uint32_t bn, bm, lone, full;
 };
-constexpr DenseTile DENSE_TILES[] = {{64, 64, 19, 21}, {128, 64, 24, 34}, {128, 128, 30, 55}, {256, 128, 50, 100}, {256, 256, 105, 168}};
+constexpr DenseTile DENSE_TILES[] = {{64, 64, 16, 23}, {128, 64, 25, 38}, {128, 128, 43, 58}, {256, 128, 76, 100}, {256, 256, 114, 162}};
 constexpr int DENSE_CUT_TILES = 3;                           // of these the first may be cut along k
 
 struct DensePlan {
     int tile;
     uint32_t parts;
-    uint64_t ns;
+    float ns;
 };
 
-// planes: the stages of 64 k.  cut: whether there is a place for the sums of parts.
+// planes: the stages of 64 k.  cut: whether there is a place for the sums of parts.  (Few divisions, and those of 32 bits: the choice is made in every
+// call, and short prompts are bound by the host.)
 inline DensePlan dense_plan_tile(uint32_t n, uint32_t rows, uint32_t k, uint32_t planes, uint32_t cus, int count, bool cut) {
-    DensePlan best{0, 1, ~0ull};
+    DensePlan best{0, 1, 1e30f};
     const uint32_t steps = k / 64u;
+    const float units = 1.0f / (float)cus, stages = 10.0f * (float)planes;
     for (int c = 0; c < count; ++c) {
         const DenseTile& t = DENSE_TILES[c];
-        const uint64_t tiles = (uint64_t)((n + t.bn - 1) / t.bn) * ((rows + t.bm - 1) / t.bm), rest = tiles % cus;
-        const uint64_t cost = tiles / cus * t.full + (rest ? t.lone + (t.full - t.lone) * rest / cus : 0);
-        const uint64_t ns = cost * 10 * steps * planes + 4000;           // and a launch, the first requests, the stores
+        const uint64_t all = (uint64_t)((n + t.bn - 1) / t.bn) * ((rows + t.bm - 1) / t.bm);
+        const uint32_t tiles = all > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)all, rounds = tiles < cus ? 0u : tiles / cus, rest = tiles - rounds * cus;
+        const float lone = (float)t.lone, rise = (float)(t.full - t.lone) * units;
+        const float cost = (float)rounds * (float)t.full + (rest ? lone + rise * (float)rest : 0.0f);
+        const float ns = cost * stages * (float)steps + 4750.0f;             // and a launch, the first requests, the stores
         if (ns < best.ns) best = {c, 1, ns};
-        if (!cut || c >= DENSE_CUT_TILES) continue;
+        if (!cut || rounds != 0 || c >= DENSE_CUT_TILES) continue;
+        const float area = (float)(t.bn * t.bm);
         for (uint32_t parts = 2; parts * 2u <= steps && parts <= DENSE_PARTS && tiles * parts <= cus; parts += parts < 4u ? 1u : parts / 4u * 2u) {
-            const uint64_t step = t.lone + (t.full - t.lone) * tiles * parts / cus;
-            const uint64_t join = 1750 + (uint64_t)parts * t.bn * t.bm / 15 + tiles * parts * t.bn * t.bm / 5000;
-            const uint64_t ns = step * 10 * ((steps + parts - 1) / parts) * planes + 4000 + join;
+            const float blocks = (float)(tiles * parts);
+            const float join = 1000.0f + area * ((float)parts * (1.0f / 16.0f) + blocks * (1.0f / 3500.0f));
+            const float ns = (lone + rise * blocks) * stages * (float)((steps + parts - 1) / parts) + 4750.0f + join;
             if (ns < best.ns) best = {c, parts, ns};
         }
     }
@@ -1102,20 +1120,28 @@ inline DensePlan dense_plan_tile(uint32_t n, uint32_t rows, uint32_t k, uint32_t
 
 // The matrix's rows in one launch, or in two where that is shorter: a last round that few units take part in is left to
 // smaller tiles (8208 weight rows, 2048 tokens: one round of 256 x 256 and a sixteenth of one, 105 -> 76 us in all).
-// Returns how many rows the first launch takes.
-inline uint32_t dense_plan(uint32_t n, uint32_t rows, uint32_t k, uint32_t planes, uint32_t cus, int count, bool split) {
-    DensePlan best = dense_plan_tile(n, rows, k, planes, cus, count, split);
-    uint32_t first = n;
+struct DenseSplit {
+    uint32_t first;                                          // rows of the first launch
+    DensePlan head, tail;
+    float ns;
+};
+
+inline DenseSplit dense_plan(uint32_t n, uint32_t rows, uint32_t k, uint32_t planes, uint32_t cus, int count, bool split) {
+    DenseSplit best{n, dense_plan_tile(n, rows, k, planes, cus, count, split), DensePlan{}, 0.0f};
+    best.ns = best.head.ns;
     for (int c = 0; c < count; ++c) {
         const uint32_t tm = (rows + DENSE_TILES[c].bm - 1) / DENSE_TILES[c].bm, tn = n / DENSE_TILES[c].bn;
+        if ((uint64_t)tn * tm < cus) continue;
         const uint32_t rounds = (uint32_t)((uint64_t)tn * tm / cus);
-        const uint32_t cut = rounds ? (uint32_t)((uint64_t)rounds * cus / tm) * DENSE_TILES[c].bn : 0;
+        const uint32_t cut = (uint32_t)((uint64_t)rounds * cus / tm) * DENSE_TILES[c].bn;
         if (cut == 0 || cut >= n) continue;
-        const uint64_t ns = dense_plan_tile(cut, rows, k, planes, cus, count, split).ns + dense_plan_tile(n - cut, rows, k, planes, cus, count, split).ns;
-        if (ns < best.ns) { best.ns = ns; first = cut; }
+        const DensePlan head = dense_plan_tile(cut, rows, k, planes, cus, count, split), tail = dense_plan_tile(n - cut, rows, k, planes, cus, count, split);
+        if (head.ns + tail.ns < best.ns) best = {cut, head, tail, head.ns + tail.ns};
     }
-    return first;
+    return best;
 }
+
+inline bool dense_may_cut(const nvmai_hip_ctx* ctx) { return ctx->cut_sums != nullptr && (uint32_t)ctx->compute_units <= CUT_BLOCKS; }
 
 template <int EPI, int ACT, int COUNT>
 void launch_tile(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p, const DensePlan& plan) {
@@ -1135,11 +1161,11 @@ template <int EPI, int ACT>
 void launch_tiles(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p) {
     constexpr int COUNT = ACT == ACT_FP32 ? 3 : 5;           // 32-bit inputs keep a running total beside the sums: no registers for the larger tiles
     const uint32_t cus = (uint32_t)ctx->compute_units, planes = ACT == ACT_FP32 ? 3u : 1u;
-    const bool cut = ctx->cut_sums != nullptr && cus <= CUT_BLOCKS;
-    const uint32_t first = dense_plan(p.n, p.rows, p.k, planes, cus, COUNT, cut);
+    const DenseSplit plan = dense_plan(p.n, p.rows, p.k, planes, cus, COUNT, dense_may_cut(ctx));
+    const uint32_t first = plan.first;
     DenseLinearParams q = p;
     q.n = first;
-    launch_tile<EPI, ACT, COUNT>(ctx, s, q, dense_plan_tile(q.n, q.rows, q.k, planes, cus, COUNT, cut));
+    launch_tile<EPI, ACT, COUNT>(ctx, s, q, plan.head);
     if (first == p.n) return;
     q.n = p.n - first;                                       // first is a multiple of 64: every operand stays aligned
     q.w = p.w + (size_t)first * p.w_stride;
@@ -1148,7 +1174,7 @@ void launch_tiles(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p)
     if (p.y_f32) q.y_f32 = p.y_f32 + out;
     if (p.bias) q.bias = p.bias + first;
     if (p.mul) q.mul = p.mul + first;
-    launch_tile<EPI, ACT, COUNT>(ctx, s, q, dense_plan_tile(q.n, q.rows, q.k, planes, cus, COUNT, cut));
+    launch_tile<EPI, ACT, COUNT>(ctx, s, q, plan.tail);
 }
 
 // 32-bit inputs: their planes, in portions of rows, then the product.
