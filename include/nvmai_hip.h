@@ -17,11 +17,13 @@
  *     nvmai_hip_ctx_destroy, so a captured graph stays valid whatever is called
  *     later.  A call that would have to grow while its stream is being captured
  *     returns NVMAI_ERR_SCRATCH and launches nothing: run the same call eagerly once,
- *     or nvmai_hip_ctx_reserve, before capturing.  Three kinds of call that have a form with
+ *     or nvmai_hip_ctx_reserve, before capturing.  Four kinds of call that have a form with
  *     less or no workspace record that one instead, slower and with other roundings:
  *     nvmai_hip_dense_linear[_ex] and the expanded nvmai_hip_latent_attention of a 32-bit
- *     context (products without BF16 planes), and nvmai_hip_attention_decode_ragged (chunks of
- *     one length for every sequence).  They do the same where memory cannot be allocated.
+ *     context (products without BF16 planes), nvmai_hip_attention_decode_ragged (chunks of
+ *     one length for every sequence), and in a BF16 context nvmai_hip_affine_qmm, nvmai_hip_affine_gemv
+ *     and nvmai_hip_shared_expert over many rows (codes dequantized per tile; the other form keeps
+ *     the matrix as BF16 in the workspace for the call, up to 256 MB).  They do the same where memory cannot be allocated.
  *     Beside the workspace a ctx holds 16 MB from its creation on, where the blocks that share an output tile
  *     meet; if they cannot be allocated, no tile is shared (slower products of few rows, other roundings).
  * Data formats (reference file:line):

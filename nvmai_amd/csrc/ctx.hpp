@@ -116,7 +116,9 @@ struct ProfScope {
 // One expert over all rows through the grouped-GEMM kernels (prefill_api.hip).
 int expert_ffn_dense(nvmai_hip_ctx* ctx, hipStream_t s, const uint8_t* blob, const nvmai_expert_offsets* off,
                      uint32_t bits, const void* x, uint32_t x_stride, uint32_t tokens, uint32_t d, uint32_t f,
-                     void* act, void* tmp, const float* gate_logit, void* y, uint32_t y_stride);
+                     void* act, void* tmp, uint16_t* wide, const float* gate_logit, void* y, uint32_t y_stride);
+// Whether it is faster with its matrices widened to BF16 once (d * f * 6 bytes of scratch).
+bool expert_widen_pays(const nvmai_hip_ctx* ctx, uint32_t bits, uint32_t tokens, uint32_t d, uint32_t f);
 
 // Dense BF16 rows against BF16 inputs on the matrix cores (step_api.hip).
 int dense_bf16_gemv(nvmai_hip_ctx* ctx, hipStream_t s, const uint16_t* w, const void* x, uint32_t x_stride,

@@ -70,6 +70,10 @@ int dense_linear(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p) 
     return p.activation == NVMAI_LINEAR_GELU_ERF ? dense_launch_erf(ctx, s, p) : dense_launch<DE_PLAIN>(ctx, s, p);
 }
 
+uint64_t dense_linear_ns(const nvmai_hip_ctx* ctx, uint32_t rows, uint32_t n, uint32_t k) {
+    return (uint64_t)dense_plan(n, rows < 65u ? 65u : rows, k, 1, (uint32_t)ctx->compute_units, 5, dense_may_cut(ctx)).ns;
+}
+
 }  // namespace nvmai
 
 namespace {

@@ -41,6 +41,8 @@ inline size_t dense_plane_bytes(uint32_t rows, uint32_t k) {
 }
 
 int dense_linear_check(const nvmai_hip_ctx* ctx, const DenseLinearParams& p);
+// What a call of more than 64 rows in a 16-bit context is expected to take, in ns.
+uint64_t dense_linear_ns(const nvmai_hip_ctx* ctx, uint32_t rows, uint32_t n, uint32_t k);
 // The launches behind it by what stands between sum and store (dense_*_api.hip, built side by side).
 int dense_launch_erf(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p);
 int dense_launch_bias(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p);

@@ -825,13 +825,16 @@ extern "C" int nvmai_hip_shared_expert(nvmai_hip_ctx* ctx, nvmai_stream stream, 
     if (n_tokens >= 192 && (uint64_t)n_tokens * x_stride * 2 <= 0xFFFFFFFFull &&
         (uint64_t)n_tokens * d * 2 <= 0xFFFFFFFFull && (uint64_t)d * f * bits / 8 <= 0xFFFFFFFFull) {
         const bool gated_d = shared_gate && shared_gate->kind;
-        rc = ws_begin(ctx, stream, ws_round((size_t)n_tokens * f * 2) + ws_round((size_t)n_tokens * d * 2) +
-                               ws_round(n_tokens * 4u) + ws_round(16));
-        if (rc) return rc;
+        const size_t rows = ws_round((size_t)n_tokens * f * 2) + ws_round((size_t)n_tokens * d * 2) + ws_round(n_tokens * 4u) + ws_round(16),
+                     widened = ws_round((size_t)d * f * 6);
+        const bool widen = (uint64_t)n_tokens * x_stride * 4 <= 0xFFFFFFFFull && nvmai::expert_widen_pays(ctx, bits, n_tokens, d, f) &&
+                           ws_begin(ctx, stream, rows + widened) == NVMAI_OK;
+        if (!widen && (rc = ws_begin(ctx, stream, rows))) return rc;
         uint16_t* act = ws_take<uint16_t>(ctx, (size_t)n_tokens * f);
         uint16_t* tmp = ws_take<uint16_t>(ctx, (size_t)n_tokens * d);
         float* gate_logit = ws_take<float>(ctx, n_tokens);
         float* dummy_logits = ws_take<float>(ctx, 4);
+        uint16_t* wide = widen ? ws_take<uint16_t>(ctx, (size_t)d * f * 3) : nullptr;
         if (gated_d) {
             RouterParams rp{};
             rp.gate = to_desc(shared_gate);
@@ -840,7 +843,7 @@ extern "C" int nvmai_hip_shared_expert(nvmai_hip_ctx* ctx, nvmai_stream stream, 
             rc = run_router(ctx, rp, s);
             if (rc) return rc;
         }
-        return nvmai::expert_ffn_dense(ctx, s, (const uint8_t*)blob, off, bits, x, x_stride, n_tokens, d, f, act, tmp,
+        return nvmai::expert_ffn_dense(ctx, s, (const uint8_t*)blob, off, bits, x, x_stride, n_tokens, d, f, act, tmp, wide,
                                        gated_d ? gate_logit : nullptr, y, y_stride);
     }
     const int maxtok = n_tokens == 1 ? 1 : MAX_TOK;

@@ -1,5 +1,6 @@
 // Entry points: token-expert pairs, grouping by expert, grouped expert GEMMs, rank-order reduce.
 #include "ctx.hpp"
+#include "dense_internal.hpp"
 #include "prefill_kernels.hpp"
 
 using namespace nvmai;
@@ -35,6 +36,7 @@ extern "C" int nvmai_hip_prefill_make_pairs(nvmai_hip_ctx* ctx, nvmai_stream str
 namespace {
 
 constexpr uint32_t MAX_GROUP_EXPERTS = 2048;   // five u32 arrays of the scan kernel in 40 KB of LDS
+constexpr size_t WIDEN_BYTES = (size_t)256 << 20;   // of the workspace at most, for the widened rows of a dense product
 constexpr int ERR_WORD = 8;                    // index into the context's persistent zeroed words
 
 int check_grouping(const nvmai_prefill_grouping* g, uint64_t n_pairs) {
@@ -176,14 +178,110 @@ void launch_gemms(const GemmParams& g1, const GemmParams& g2, uint32_t tiles, nv
 
 }  // namespace
 
+namespace {
+
+// Widens up to three matrices in one launch.
+void widen_rows(hipStream_t s, uint32_t bits, const WidenParams& p, uint32_t matrices) {
+    uint64_t most = 0;
+    for (uint32_t i = 0; i < matrices; ++i) most = p.m[i].pieces > most ? p.m[i].pieces : most;
+    const dim3 grid((uint32_t)((most + 255) / 256), matrices);
+    if (bits == 4) widen_rows_kernel<4><<<grid, 256, 0, s>>>(p);
+    else widen_rows_kernel<8><<<grid, 256, 0, s>>>(p);
+}
+
+// ns of a dense product whose tiles dequantize for themselves: what one, and what two blocks of a compute unit take for a super-step of 128 k
+// (bits 4 and 8, M tiles of 64 rows and of 128), and the rounds of the XCD that has the most of them.
+uint64_t dequantizing_ns(const nvmai_hip_ctx* ctx, uint32_t bits, uint32_t rows, uint32_t n, uint32_t k) {
+    const uint32_t cols = bits == 4 ? 256 : 128, tiles_n = (n + cols - 1) / cols, bm = dense_bm_for(rows, tiles_n), tiles_m = (rows + bm - 1) / bm;
+    const bool tall = (rows < bm ? rows : bm) > 64;
+    const uint64_t lone = bits == 4 ? (tall ? 2500 : 1600) : (tall ? 1500 : 1000), pair = bits == 4 ? (tall ? 4200 : 2600) : (tall ? 2500 : 1600);
+    const uint32_t units = (uint32_t)ctx->compute_units / GEMM_XCDS ? (uint32_t)ctx->compute_units / GEMM_XCDS : 1u;
+    const uint64_t blocks = tiles_m >= 8 ? (uint64_t)(tiles_m + 7) / 8 * tiles_n : (uint64_t)(tiles_n + 7) / 8 * tiles_m;
+    const uint64_t rest = blocks % (2 * units), step = blocks / (2 * units) * pair + (rest == 0 ? 0 : rest <= units ? lone : pair * 9 / 10);
+    return step * ((k + GEMM_SK - 1) / GEMM_SK) + 4000;
+}
+
+// Whether the codes are widened to BF16 once, in the workspace, and multiplied by the dense product (whose tiles are larger, are cut along k
+// where they are few, and need no instructions for codes), or dequantized in every tile that needs them.  Widening writes and reads two bytes per
+// code; over 140 sizes (n 1024 .. 12,352, k 512 .. 4096, 33 .. 4096 rows, both widths) the rule is 0.3 % from the faster, 14 % at most.  Rows x n x k,
+// cold codes of 4 bits, dequantized per tile and widened, us: 128 x 2048 x 4096 52.4 and 22.1, 300 x 1024 x 2048 30.8 and 13.0, 1500 x 9216 x 2048 95 and 60,
+// 4096 x 12,352 x 2048 209 and 175, 4096 x 2048 x 4096 78 and 65; but 128 x 12,352 x 2048 31.1 and 34.2, 4096 x 2048 x 512 19.0 and 20.1.
+bool widen_pays(const nvmai_hip_ctx* ctx, uint32_t bits, uint32_t rows, uint32_t n, uint32_t k) {
+    if (ctx->act != NVMAI_ACT_BF16 || rows <= 32 || (uint64_t)n * k * 2 > WIDEN_BYTES) return false;
+    return 500 + (uint64_t)n * k * 26 / 35000 + dense_linear_ns(ctx, rows, n, k) < dequantizing_ns(ctx, bits, rows, n, k);
+}
+
+// Widens and multiplies, if that pays and the workspace can hold the rows; false: nothing is launched.
+bool widened_product(nvmai_hip_ctx* ctx, nvmai_stream stream, uint32_t bits, const uint8_t* weights, const uint16_t* scales, const uint16_t* biases,
+                     DenseLinearParams d, int* rc) {
+    if (!widen_pays(ctx, bits, d.rows, d.n, d.k) || (uint64_t)d.rows * d.x_stride * 4 > 0xFFFFFFFFull) return false;
+    if (ws_begin(ctx, stream, ws_round((size_t)d.n * d.k * 2)) != NVMAI_OK) return false;
+    uint16_t* wide = ws_take<uint16_t>(ctx, (size_t)d.n * d.k);
+    WidenParams p{};
+    p.m[0] = WidenMatrix{weights, scales, biases, wide, (uint64_t)d.n * d.k / 16, d.k, 1};
+    widen_rows((hipStream_t)stream, bits, p, 1);
+    d.w = wide;
+    d.w_stride = d.k;
+    *rc = dense_linear(ctx, (hipStream_t)stream, d);
+    return true;
+}
+
+// rows * sigmoid(gate logit of the row) -> y
+int gate_rows(nvmai_hip_ctx* ctx, hipStream_t s, const void* tmp, const float* gate_logit, void* y, uint32_t tokens, uint32_t d, uint32_t y_stride) {
+    if (d % 8 == 0 && y_stride % 8 == 0 && aligned16(tmp) && aligned16(y)) {       // sixteen bytes per thread
+        dim3 grid8((d / 8 + 255) / 256, tokens);
+        if (ctx->act == ACT_BF16)
+            gate_rows8_kernel<ACT_BF16><<<grid8, 256, 0, s>>>((const uint16_t*)tmp, gate_logit, (uint16_t*)y, tokens, d, y_stride);
+        else
+            gate_rows8_kernel<ACT_FP16><<<grid8, 256, 0, s>>>((const uint16_t*)tmp, gate_logit, (uint16_t*)y, tokens, d, y_stride);
+        return launch_status();
+    }
+    dim3 grid((d + 255) / 256, tokens);
+    if (ctx->act == ACT_BF16)
+        gate_rows_kernel<ACT_BF16><<<grid, 256, 0, s>>>((const uint16_t*)tmp, gate_logit, (uint16_t*)y, tokens, d, y_stride);
+    else
+        gate_rows_kernel<ACT_FP16><<<grid, 256, 0, s>>>((const uint16_t*)tmp, gate_logit, (uint16_t*)y, tokens, d, y_stride);
+    return launch_status();
+}
+
+}  // namespace
+
 // One expert over every row of x (the shared expert of a prefill block): gate/up + SwiGLU and
 // down through the grouped-GEMM kernels in their dense mode, then the optional scalar gate.
 // x [tokens, x_stride] and y [tokens, y_stride] in the context's activation type; act and tmp
-// are 16-bit scratch [tokens, f] and [tokens, d], 16-byte aligned.
+// are 16-bit scratch [tokens, f] and [tokens, d], 16-byte aligned; wide: 3 d f BF16 of scratch for the widened matrices, or nullptr.
 namespace nvmai {
+bool expert_widen_pays(const nvmai_hip_ctx* ctx, uint32_t bits, uint32_t tokens, uint32_t d, uint32_t f) {
+    if (ctx->act != NVMAI_ACT_BF16 || tokens <= 32 || (uint64_t)d * f * 6 > WIDEN_BYTES) return false;
+    return 500 + (uint64_t)d * f * 3 * 26 / 35000 + dense_linear_ns(ctx, tokens, 2 * f, d) + dense_linear_ns(ctx, tokens, d, f) <
+           dequantizing_ns(ctx, bits, tokens, 2 * f, d) + dequantizing_ns(ctx, bits, tokens, d, f);
+}
+
 int expert_ffn_dense(nvmai_hip_ctx* ctx, hipStream_t s, const uint8_t* blob, const nvmai_expert_offsets* off,
                      uint32_t bits, const void* x, uint32_t x_stride, uint32_t tokens, uint32_t d, uint32_t f,
-                     void* act, void* tmp, const float* gate_logit, void* y, uint32_t y_stride) {
+                     void* act, void* tmp, uint16_t* wide, const float* gate_logit, void* y, uint32_t y_stride) {
+    if (wide) {                            // gate and up as pairs of rows, then down
+        const uint64_t pieces = (uint64_t)d * f / 16;
+        WidenParams p{};
+        auto at = [&](uint32_t o) { return blob + o; };
+        auto meta = [&](uint32_t o) { return reinterpret_cast<const uint16_t*>(blob + o); };
+        p.m[0] = WidenMatrix{at(off->gate_w), meta(off->gate_s), meta(off->gate_b), wide, pieces, d, 2};
+        p.m[1] = WidenMatrix{at(off->up_w), meta(off->up_s), meta(off->up_b), wide + d, pieces, d, 2};
+        p.m[2] = WidenMatrix{at(off->down_w), meta(off->down_s), meta(off->down_b), wide + (size_t)2 * f * d, pieces, f, 1};
+        int rc;
+        {
+            ProfScope prof(ctx, NVMAI_PROF_PREFILL_GEMM1, s);
+            widen_rows(s, bits, p, 3);
+            rc = dense_linear(ctx, s, DenseLinearParams{wide, x, act, nullptr, d, x_stride, f, tokens, 2 * f, d, NVMAI_LINEAR_SILU_PAIRS});
+        }
+        if (rc) return rc;
+        {
+            ProfScope prof(ctx, NVMAI_PROF_PREFILL_GEMM2, s);
+            rc = dense_linear(ctx, s, DenseLinearParams{wide + (size_t)2 * f * d, act, tmp, nullptr, f, f, d, tokens, d, f, NVMAI_LINEAR_NONE});
+        }
+        if (rc) return rc;
+        return gate_rows(ctx, s, tmp, gate_logit, y, tokens, d, y_stride);
+    }
     const uint32_t nt = bits == 4 ? 4 : 2;
     const uint32_t tiles = (tokens + GEMM_BM - 1) / GEMM_BM;
     GemmParams g1{};
@@ -207,20 +305,7 @@ int expert_ffn_dense(nvmai_hip_ctx* ctx, hipStream_t s, const uint8_t* blob, con
         if (bits == 4) launch_gemms<ACT_FP16, 4, 4>(g1, g2, tiles, ctx, s);
         else launch_gemms<ACT_FP16, 8, 2>(g1, g2, tiles, ctx, s);
     }
-    if (d % 8 == 0 && y_stride % 8 == 0 && aligned16(tmp) && aligned16(y)) {       // sixteen bytes per thread
-        dim3 grid8((d / 8 + 255) / 256, tokens);
-        if (ctx->act == ACT_BF16)
-            gate_rows8_kernel<ACT_BF16><<<grid8, 256, 0, s>>>((const uint16_t*)tmp, gate_logit, (uint16_t*)y, tokens, d, y_stride);
-        else
-            gate_rows8_kernel<ACT_FP16><<<grid8, 256, 0, s>>>((const uint16_t*)tmp, gate_logit, (uint16_t*)y, tokens, d, y_stride);
-        return launch_status();
-    }
-    dim3 grid((d + 255) / 256, tokens);
-    if (ctx->act == ACT_BF16)
-        gate_rows_kernel<ACT_BF16><<<grid, 256, 0, s>>>((const uint16_t*)tmp, gate_logit, (uint16_t*)y, tokens, d, y_stride);
-    else
-        gate_rows_kernel<ACT_FP16><<<grid, 256, 0, s>>>((const uint16_t*)tmp, gate_logit, (uint16_t*)y, tokens, d, y_stride);
-    return launch_status();
+    return gate_rows(ctx, s, tmp, gate_logit, y, tokens, d, y_stride);
 }
 }  // namespace nvmai
 
@@ -398,6 +483,9 @@ extern "C" int nvmai_hip_affine_qmm(nvmai_hip_ctx* ctx, nvmai_stream stream, con
         return NVMAI_ERR_UNSUPPORTED;
     hipStream_t s = (hipStream_t)stream;
     ProfScope prof(ctx, NVMAI_PROF_PREFILL_GEMM2, s);
+    int rc = NVMAI_OK;
+    if (widened_product(ctx, stream, bits, weights, scales, biases, DenseLinearParams{nullptr, x, y, nullptr, 0, x_stride, y_stride, m, n, k, NVMAI_LINEAR_NONE}, &rc))
+        return rc;
     const uint32_t nt = bits == 4 ? 4 : 2;
     GemmParams g{};
     g.pool = weights; g.pool_stride = 0;

@@ -1451,6 +1451,48 @@ __global__ __launch_bounds__(256) void gate_rows8_kernel(const uint16_t* rows, c
     *reinterpret_cast<uint4*>(y + (size_t)t * y_stride + c) = uint4{r[0], r[1], r[2], r[3]};
 }
 
+// ---- weights of a dense product, widened once -------------------------------------------------------------
+// Codes of up to three matrices -> BF16 rows, w = q * scale + bias in fp32 rounded once, as the tiles above make them; a matrix's row i
+// goes to row step * i of its place (gate and up take turns: pairs).  Sixteen codes of a group per thread, 32 bytes stored.
+// Bound by its bytes: 12,352 x 2048 from four bits about 13 us with its launch, 64 MB.
+struct WidenMatrix {
+    const uint8_t* codes;
+    const uint16_t *scales, *biases;
+    uint16_t* out;
+    uint64_t pieces;                       // n k / 16
+    uint32_t k, step;
+};
+struct WidenParams {
+    WidenMatrix m[3];
+};
+
+template <int BITS>
+__global__ __launch_bounds__(256) void widen_rows_kernel(WidenParams p) {
+    const WidenMatrix m = blockIdx.y == 0 ? p.m[0] : blockIdx.y == 1 ? p.m[1] : p.m[2];
+    const uint64_t at = (uint64_t)blockIdx.x * 256u + threadIdx.x;
+    if (at >= m.pieces) return;
+    uint32_t c[BITS / 2];
+    if (BITS == 8) {
+        const uint4 v = *reinterpret_cast<const uint4*>(m.codes + at * 16u);
+        c[0] = v.x; c[1] = v.y; c[2] = v.z; c[3] = v.w;
+    } else {
+        const uint2 v = *reinterpret_cast<const uint2*>(m.codes + at * 8u);
+        c[0] = v.x; c[1] = v.y;
+    }
+    const float s = bf16_to_f32(m.scales[at / 4u]), b = bf16_to_f32(m.biases[at / 4u]);
+    uint32_t o[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const uint32_t lo = BITS == 8 ? (c[e / 2] >> (16 * (e & 1))) & 0xFFu : (c[e / 4] >> (8 * (e & 3))) & 0xFu;
+        const uint32_t hi = BITS == 8 ? (c[e / 2] >> (16 * (e & 1) + 8)) & 0xFFu : (c[e / 4] >> (8 * (e & 3) + 4)) & 0xFu;
+        o[e] = pack_act2<ACT_BF16>(fmaf((float)lo, s, b), fmaf((float)hi, s, b));
+    }
+    uint64_t to = at * 16u;
+    if (m.step > 1u) to += at * 16u / m.k * (m.step - 1u) * m.k;
+    *reinterpret_cast<uint4*>(m.out + to) = uint4{o[0], o[1], o[2], o[3]};
+    *reinterpret_cast<uint4*>(m.out + to + 8) = uint4{o[4], o[5], o[6], o[7]};
+}
+
 // ---- combine (prefill.metal:437-458) -------------------------------------------------------
 // h2[t, d] = sum over ranks in rank order of fma(w[t, r], partial[t, r, d], acc).  VEC = 8:
 // sixteen bytes of a row per thread (rows 16-byte aligned); VEC = 2: any even d.
