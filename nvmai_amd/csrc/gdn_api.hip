@@ -200,8 +200,11 @@ bool launch_decode_fused(const GdnDecodeParams& p, uint32_t ratio, bool state_bf
     const dim3 grid(p.d.sh.k_heads, p.d.sh.batch);
 #define NVMAI_GDN_FUSED(R)                                                                             \
     do {                                                                                               \
-        if (state_bf16) gdn_decode_fused_kernel<ACT, DK, DV, R, true><<<grid, 256 * R, 0, s>>>(p);      \
-        else gdn_decode_fused_kernel<ACT, DK, DV, R, false><<<grid, 256 * R, 0, s>>>(p);                \
+        if (p.d.sh.taps == 4) {                                                                         \
+            if (state_bf16) gdn_decode_fused_kernel<ACT, DK, DV, R, true, 4><<<grid, 256 * R, 0, s>>>(p); \
+            else gdn_decode_fused_kernel<ACT, DK, DV, R, false, 4><<<grid, 256 * R, 0, s>>>(p);         \
+        } else if (state_bf16) gdn_decode_fused_kernel<ACT, DK, DV, R, true, GDN_MAX_TAPS><<<grid, 256 * R, 0, s>>>(p); \
+        else gdn_decode_fused_kernel<ACT, DK, DV, R, false, GDN_MAX_TAPS><<<grid, 256 * R, 0, s>>>(p);  \
         return true;                                                                                   \
     } while (0)
     if (ratio == 1) NVMAI_GDN_FUSED(1);

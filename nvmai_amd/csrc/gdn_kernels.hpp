@@ -646,8 +646,10 @@ __global__ __launch_bounds__(256) void gdn_delta_rows_kernel(GdnDeltaParams p) {
 // and then its delta rule and gated norm exactly as gdn_delta_gated_kernel does, with q, k and v
 // taken from LDS instead of a conv_out row in memory.  The thread that computes a channel holds the
 // channel's tail column in registers and writes it back shifted: the block is the only reader of
-// its channels, so the tail is updated in place with no ordering between blocks.  The state rows
-// are requested before the conv so that they arrive while it runs.
+// its channels, so the tail is updated in place with no ordering between blocks.  Bound by two trips to memory and the chain of
+// sums behind them, from a few dozen blocks on by the state's bytes: 16 key heads of two value heads of 128 x 128, 16 sequences 14.3 -> 10.3 us (67 MB, 6.5 TB/s)
+// and one 7.7, with the inputs of all conv channels requested before the state instead of channel by channel behind it; the two kernels
+// one after the other took 10.1 for one sequence and 10.5 for four, where this one takes 6.9.
 struct GdnDecodeParams {
     GdnDeltaParams d;           // conv_out unused
     const uint16_t* qkv_raw;    // [batch, qkv_stride]
@@ -656,7 +658,8 @@ struct GdnDecodeParams {
     const uint16_t* conv_w;     // BF16 [C, taps]
 };
 
-template <int ACT, int DK, int DV, int R, bool STATE_BF16>
+// TAPS: the taps of the conv, or the most there can be.
+template <int ACT, int DK, int DV, int R, bool STATE_BF16, int TAPS>
 __global__ __launch_bounds__(256 * R) void gdn_decode_fused_kernel(GdnDecodeParams pp) {
     constexpr int EPL = DK / 16;
     constexpr int GROUPS = DV / 16;
@@ -672,7 +675,31 @@ __global__ __launch_bounds__(256 * R) void gdn_decode_fused_kernel(GdnDecodePara
     const uint32_t h = hk * R + r;
     const uint32_t sub = lt & 15u, row_in_pass = lt >> 4;
     const uint32_t C = 2 * sh.k_heads * DK + sh.v_heads * DV;
-    const uint32_t hist = sh.taps - 1;
+    const uint32_t taps = TAPS < GDN_MAX_TAPS ? (uint32_t)TAPS : sh.taps, hist = taps - 1;
+
+    // ---- everything from memory is requested at once: first what the conv needs, so that it runs while the state is on its way (results
+    // come back in the order of the requests).  q: threads 0 .. DK - 1 of group 0; k: threads 128 .. 128 + DK - 1 of group 0; v: a channel
+    // per thread of each group.  A thread without a channel reads another one's and drops it: a load under a condition is waited for on the spot.
+    const bool is_q = r == 0 && lt < (uint32_t)DK, is_k = r == 0 && lt >= 128u && lt < 128u + (uint32_t)DK, is_v = lt < (uint32_t)DV;
+    const uint32_t ch_v = 2 * sh.k_heads * DK + h * DV + min(lt, (uint32_t)DV - 1u);
+    const uint32_t ch_qk = is_q ? hk * DK + lt : is_k ? sh.k_heads * DK + hk * DK + (lt - 128u) : ch_v;
+    uint16_t* tl = pp.tail + (size_t)b * hist * C;
+    const uint16_t* raw = pp.qkv_raw + (size_t)b * pp.qkv_stride;
+    uint16_t xq[TAPS], xv[TAPS], wq[TAPS], wv[TAPS];
+    auto request = [&](uint32_t ch, uint16_t* x, uint16_t* w) {
+#pragma unroll
+        for (uint32_t j = 0; j < TAPS; ++j) {                       // taps past the last reread it
+            const uint32_t jj = min(j, hist);
+            x[j] = *(jj < hist ? tl + (size_t)jj * C + ch : raw + ch);
+            w[j] = pp.conv_w[ch * taps + jj];
+        }
+    };
+    if (r == 0) request(ch_qk, xq, wq);                             // uniform per wave
+    request(ch_v, xv, wv);
+    const size_t row = b;
+    const uint16_t a_raw = p.a_proj[row * p.ab_stride + h], b_raw = p.b_proj[row * p.ab_stride + h];
+    const uint16_t a_log_raw = p.a_log[h], dt_raw = p.dt_bias[h];
+    const uint16_t z_raw = p.z[row * p.z_stride + h * DV + min(lt, (uint32_t)DV - 1u)], nw_raw = p.norm_w[min(lt, (uint32_t)DV - 1u)];
 
     // ---- the state rows of this value head
     const size_t state_base = (((size_t)b * sh.v_heads + h) * DV) * DK;
@@ -686,42 +713,20 @@ __global__ __launch_bounds__(256 * R) void gdn_decode_fused_kernel(GdnDecodePara
                                  : reinterpret_cast<const float*>(p.state)[at + e];
     }
 
-    // everything else the token needs from memory is requested now as well, ahead of the conv's barriers
-    const size_t row = b;
-    const uint16_t a_raw = p.a_proj[row * p.ab_stride + h], b_raw = p.b_proj[row * p.ab_stride + h];
-    const uint16_t a_log_raw = p.a_log[h], dt_raw = p.dt_bias[h];
-    const uint16_t z_raw = lt < (uint32_t)DV ? p.z[row * p.z_stride + h * DV + lt] : (uint16_t)0;
-    const uint16_t nw_raw = lt < (uint32_t)DV ? p.norm_w[lt] : (uint16_t)0;
-
     // ---- conv + SiLU of one channel, tail column shifted in place; returns the 16-bit result as a float
-    uint16_t* tl = pp.tail + (size_t)b * hist * C;
-    const uint16_t* raw = pp.qkv_raw + (size_t)b * pp.qkv_stride;
-    auto conv_channel = [&](uint32_t ch) -> float {
-        uint16_t x[GDN_MAX_TAPS];
-#pragma unroll
-        for (uint32_t j = 0; j < GDN_MAX_TAPS; ++j) {
-            if (j > hist) break;
-            x[j] = j < hist ? tl[(size_t)j * C + ch] : raw[ch];
-        }
+    auto conv_channel = [&](uint32_t ch, const uint16_t* x, const uint16_t* w) -> float {
         float acc = 0.0f;
 #pragma unroll
-        for (uint32_t j = 0; j < GDN_MAX_TAPS; ++j) {
-            if (j > hist) break;
-            acc = fmaf(act_to_f32<ACT>(x[j]), bf16_to_f32(pp.conv_w[ch * sh.taps + j]), acc);
-        }
+        for (uint32_t j = 0; j < TAPS; ++j)
+            if (j < taps) acc = fmaf(act_to_f32<ACT>(x[j]), bf16_to_f32(w[j]), acc);
 #pragma unroll
-        for (uint32_t j = 0; j < GDN_MAX_TAPS; ++j) {
-            if (j >= hist) break;
-            tl[(size_t)j * C + ch] = x[j + 1];
-        }
+        for (uint32_t j = 0; j + 1 < TAPS; ++j)
+            if (j < hist) tl[(size_t)j * C + ch] = x[j + 1];
         return act_to_f32<ACT>(f32_to_act<ACT>(gdn_silu(acc)));
     };
-    // q: threads 0 .. DK - 1 of group 0; k: threads 128 .. 128 + DK - 1 of group 0
-    const bool is_q = r == 0 && lt < (uint32_t)DK, is_k = r == 0 && lt >= 128u && lt < 128u + (uint32_t)DK;
     float qk = 0.0f;
-    if (is_q) qk = conv_channel(hk * DK + lt);
-    if (is_k) qk = conv_channel(sh.k_heads * DK + hk * DK + (lt - 128u));
-    if (lt < (uint32_t)DV) v_s[r][lt] = conv_channel(2 * sh.k_heads * DK + h * DV + lt);
+    if (is_q || is_k) qk = conv_channel(ch_qk, xq, wq);
+    if (is_v) v_s[r][lt] = conv_channel(ch_v, xv, wv);
     if (r == 0) {
         const float ws = wave_sum_bcast(qk * qk);               // fma(x, x, 0) of the separate kernel
         if (lane == 0) part_qk[wave] = ws;

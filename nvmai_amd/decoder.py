@@ -404,27 +404,14 @@ class HybridDecoder(StepDecoder):
         b = self.lin_proj[:, cfg.gdn_qkv_dim + cfg.gdn_value_dim + vh:]
         tail, state = self.gdn_states[L]
         g = self.gdn
-        if B >= 8:
-            # conv + q / k norm + tail update + delta rule + gated norm of the token in one launch (same
-            # bits; measured: 6.07 -> 6.00 ms per step at 16 sequences, no gain below -- one block per key
-            # head is half as many blocks as the delta kernel's, and a single token leaves the device empty)
-            check(lib.nvmai_hip_gdn_decode_step(self.ctx.handle, ops._stream(), C.byref(g.cfg), ops._ptr(qkv), self.lin_rows,
-                                                ops._ptr(tail), ops._ptr(w["conv_w"]), ops._ptr(self.conv_out),
-                                                cfg.gdn_qkv_dim, ops._ptr(a), ops._ptr(b), self.lin_rows,
-                                                ops._ptr(w["a_log"]), ops._ptr(w["dt_bias"]), ops._ptr(state),
-                                                int(state.dtype == torch.bfloat16), ops._ptr(z), self.lin_rows,
-                                                ops._ptr(w["gdn_norm"]), ops._ptr(self.gdn_out), cfg.gdn_value_dim, B),
-                  "gdn_decode_step")
-        else:
-            check(lib.nvmai_hip_gdn_conv_norm(self.ctx.handle, ops._stream(), C.byref(g.cfg), ops._ptr(qkv), self.lin_rows,
-                                              ops._ptr(tail), ops._ptr(w["conv_w"]), ops._ptr(self.conv_out),
-                                              cfg.gdn_qkv_dim, 1, B), "gdn_conv_norm")
-            check(lib.nvmai_hip_gdn_delta_gated_norm(self.ctx.handle, ops._stream(), C.byref(g.cfg), ops._ptr(self.conv_out),
-                                                     cfg.gdn_qkv_dim, ops._ptr(a), ops._ptr(b), self.lin_rows,
-                                                     ops._ptr(w["a_log"]), ops._ptr(w["dt_bias"]), ops._ptr(state),
-                                                     int(state.dtype == torch.bfloat16), ops._ptr(z), self.lin_rows,
-                                                     ops._ptr(w["gdn_norm"]), ops._ptr(self.gdn_out), cfg.gdn_value_dim, 1, B),
-                  "gdn_delta_gated_norm")
+        # conv + q / k norm + tail update + delta rule + gated norm of the token in one launch (the bits of two)
+        check(lib.nvmai_hip_gdn_decode_step(self.ctx.handle, ops._stream(), C.byref(g.cfg), ops._ptr(qkv), self.lin_rows,
+                                            ops._ptr(tail), ops._ptr(w["conv_w"]), ops._ptr(self.conv_out),
+                                            cfg.gdn_qkv_dim, ops._ptr(a), ops._ptr(b), self.lin_rows,
+                                            ops._ptr(w["a_log"]), ops._ptr(w["dt_bias"]), ops._ptr(state),
+                                            int(state.dtype == torch.bfloat16), ops._ptr(z), self.lin_rows,
+                                            ops._ptr(w["gdn_norm"]), ops._ptr(self.gdn_out), cfg.gdn_value_dim, B),
+              "gdn_decode_step")
         p_, s_, b_ = w["out_proj"]
         ops.affine_gemv(self.ctx, p_, s_, b_, cfg.attn_bits, self.gdn_out, cfg.hidden, cfg.gdn_value_dim, y=self.branch)
 
