@@ -627,6 +627,12 @@ int nvmai_hip_embed_lookup(nvmai_hip_ctx* ctx, nvmai_stream stream, const uint8_
                            const uint16_t* scales, const uint16_t* biases, uint32_t bits,
                            const uint32_t* token_ids, uint32_t token_id, uint32_t n_tokens, void* out,
                            uint32_t out_stride, uint32_t d, uint32_t vocab, float out_scale);
+/* The lookup and the RMSNorm of its rows (nvmai_hip_rmsnorm), the same bits: one launch for a decode step's rows. */
+int nvmai_hip_embed_lookup_rmsnorm(nvmai_hip_ctx* ctx, nvmai_stream stream, const uint8_t* table,
+                                   const uint16_t* scales, const uint16_t* biases, uint32_t bits,
+                                   const uint32_t* token_ids, uint32_t token_id, uint32_t n_tokens, void* out,
+                                   uint32_t out_stride, uint32_t d, uint32_t vocab, float out_scale,
+                                   const uint16_t* weight, void* normed, uint32_t normed_stride, float eps);
 
 /* LMHeadChainInt4.encodeGreedyDecode (LMHeadChainInt4.swift:58-130; kernels rmsnorm_bf16w,
  * lm_head_greedy_int4_rows_chunk_raw, lm_head_greedy_int4_rows_reduce, logit.metal:761-937):

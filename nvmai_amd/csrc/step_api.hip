@@ -259,6 +259,29 @@ extern "C" int nvmai_hip_embed_lookup(nvmai_hip_ctx* ctx, nvmai_stream stream, c
     return launch_status();
 }
 
+extern "C" int nvmai_hip_embed_lookup_rmsnorm(nvmai_hip_ctx* ctx, nvmai_stream stream, const uint8_t* table,
+                                              const uint16_t* scales, const uint16_t* biases, uint32_t bits,
+                                              const uint32_t* token_ids, uint32_t token_id, uint32_t n_tokens, void* out,
+                                              uint32_t out_stride, uint32_t d, uint32_t vocab, float out_scale,
+                                              const uint16_t* weight, void* normed, uint32_t normed_stride, float eps) {
+    if (!normed || normed_stride < d) return NVMAI_ERR_INVALID_ARG;
+    if (d != 2048 || n_tokens > RMS_DIRECT_ROWS || vocab == 0) {
+        const int rc = nvmai_hip_embed_lookup(ctx, stream, table, scales, biases, bits, token_ids, token_id, n_tokens, out, out_stride, d, vocab, out_scale);
+        return rc ? rc : nvmai_hip_rmsnorm(ctx, stream, out, out_stride, weight, normed, normed_stride, n_tokens, d, eps);
+    }
+    if (!act16(ctx) || !table || !scales || !biases || !out) return NVMAI_ERR_INVALID_ARG;
+    if (bits != 4 && bits != 8) return NVMAI_ERR_UNSUPPORTED;
+    if (out_stride < d) return NVMAI_ERR_INVALID_ARG;
+    if (n_tokens == 0) return NVMAI_OK;
+#define NVMAI_EMBED(ACT, BITS)                                                                                                          \
+    embed_norm_direct_kernel<ACT, 2048, BITS><<<n_tokens, 64, 0, (hipStream_t)stream>>>(table, scales, biases, token_ids, token_id, (uint16_t*)out, out_stride, \
+                                                                                        vocab, out_scale, weight, (uint16_t*)normed, normed_stride, eps)
+    if (ctx->act == ACT_BF16) { if (bits == 4) NVMAI_EMBED(ACT_BF16, 4); else NVMAI_EMBED(ACT_BF16, 8); }
+    else { if (bits == 4) NVMAI_EMBED(ACT_FP16, 4); else NVMAI_EMBED(ACT_FP16, 8); }
+#undef NVMAI_EMBED
+    return launch_status();
+}
+
 namespace {
 
 template <int ACT, int BITS>

@@ -479,6 +479,48 @@ __global__ __launch_bounds__(256) void embed_lookup_kernel(const uint8_t* table,
     }
 }
 
+// The rows of a decode step and their RMSNorm in one launch, for a width known at compile time: embed_lookup_kernel's arithmetic, then
+// rms_direct_kernel's (a wave per row, lane l has the elements l, l + 64, ..: group j at place j).  The bits of the two.  Two trips to
+// memory and a launch of 4.5 us less.
+template <int ACT, int DFIX, int BITS>
+__global__ __launch_bounds__(64) void embed_norm_direct_kernel(const uint8_t* table, const uint16_t* scales, const uint16_t* biases,
+                                                               const uint32_t* token_ids, uint32_t token_id, uint16_t* out,
+                                                               uint32_t out_stride, uint32_t vocab, float out_scale, const uint16_t* weight,
+                                                               uint16_t* normed, uint32_t normed_stride, float eps) {
+    constexpr int N = DFIX / 64;
+    static_assert(NVMAI_GROUP == 64 && N <= 64, "a lane holds a group's scale and bias");
+    const uint32_t t = blockIdx.x, lane = threadIdx.x;
+    const uint32_t tok = token_ids ? token_ids[t] : token_id, at = tok < vocab ? tok : 0u;
+    const uint8_t* row = table + (size_t)at * (DFIX * BITS / 8);
+    uint8_t code[N];
+    uint16_t wv[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) code[j] = row[BITS == 8 ? lane + 64 * j : lane / 2 + 32 * j];
+    const float gs = bf16_to_f32(scales[(size_t)at * N + min(lane, (uint32_t)N - 1u)]), gb = bf16_to_f32(biases[(size_t)at * N + min(lane, (uint32_t)N - 1u)]);
+    if (weight) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) wv[j] = weight[lane + 64 * j];
+    }
+    float v[N];
+    float acc = 0.0f;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        const uint32_t q = BITS == 8 ? code[j] : (code[j] >> ((lane & 1u) * 4u)) & 0xFu;
+        uint16_t x = f32_to_act<ACT>(__fmul_rn(__fadd_rn(__fmul_rn((float)q, readlane_f(gs, j)), readlane_f(gb, j)), out_scale));
+        if (tok >= vocab) x = 0;
+        out[(size_t)t * out_stride + lane + 64 * j] = x;
+        v[j] = act_to_f32<ACT>(x);
+        acc = fmaf(v[j], v[j], acc);
+    }
+    const float inv = rms_inverse(rms_wave_sum(acc), DFIX, eps);
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        float y = __fmul_rn(v[j], inv);
+        if (weight) y = __fmul_rn(y, bf16_to_f32(wv[j]));
+        normed[(size_t)t * normed_stride + lane + 64 * j] = f32_to_act<ACT>(y);
+    }
+}
+
 // ---- greedy LM head ------------------------------------------------------------------------
 // LMHeadChainInt4.encodeGreedyDecode (LMHeadChainInt4.swift:58-130; kernels logit.metal:761-937):
 // token = argmax over the vocabulary rows of W[row] . norm(hidden), finite logits only, ties to

@@ -455,10 +455,10 @@ class HybridDecoder(StepDecoder):
         self.normed.  `position` is the index of these tokens in their sequences."""
         cfg, ctx = self.cfg, self.ctx
         e_p, e_s, e_b = self.w.embed
-        check(lib.nvmai_hip_embed_lookup(ctx.handle, ops._stream(), ops._ptr(e_p), ops._ptr(e_s), ops._ptr(e_b),
-                                         cfg.embed_bits, ops._ptr(self.tokens), 0, self.batch, ops._ptr(self.hidden),
-                                         cfg.hidden, cfg.hidden, cfg.vocab, 1.0), "embed_lookup")
-        ops.RMSNorm(ctx).encode_bf16w(self.hidden, self.w.layers[0]["in_norm"], out=self.normed, eps=cfg.rms_eps)
+        check(lib.nvmai_hip_embed_lookup_rmsnorm(ctx.handle, ops._stream(), ops._ptr(e_p), ops._ptr(e_s), ops._ptr(e_b),
+                                                 cfg.embed_bits, ops._ptr(self.tokens), 0, self.batch, ops._ptr(self.hidden),
+                                                 cfg.hidden, cfg.hidden, cfg.vocab, 1.0, ops._ptr(self.w.layers[0]["in_norm"]),
+                                                 ops._ptr(self.normed), cfg.hidden, cfg.rms_eps), "embed_lookup_rmsnorm")
         # up to four sequences: the residual add after a MoE block and the input norm of the next layer
         # run inside that layer's projection launch (one launch less per layer)
         fold = self.batch <= 4
