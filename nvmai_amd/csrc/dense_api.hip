@@ -54,7 +54,7 @@ int dense_linear_check(const nvmai_hip_ctx* ctx, const DenseLinearParams& p) {
     if (pairs && (p.n % 2 || p.y_stride % 2 || p.bias || p.mul)) return NVMAI_ERR_INVALID_ARG;
     if (p.mul && (!p.mul_ids || p.mul_stride < p.n)) return NVMAI_ERR_INVALID_ARG;
     if (!aligned16(p.w) || !aligned16(p.x) || p.w_stride % 8 || p.x_stride % 8) return NVMAI_ERR_ALIGNMENT;
-    if ((p.y && !aligned16(p.y)) || (p.y_f32 && !aligned16(p.y_f32))) return NVMAI_ERR_ALIGNMENT;
+    if (!p.loose && ((p.y && !aligned16(p.y)) || (p.y_f32 && !aligned16(p.y_f32)))) return NVMAI_ERR_ALIGNMENT;
     // 32-bit byte offsets inside an operand
     if ((uint64_t)p.n * p.w_stride * 2 > 0xFFFFFFFFull || (uint64_t)p.rows * p.x_stride * 4 > 0xFFFFFFFFull) return NVMAI_ERR_UNSUPPORTED;
     return NVMAI_OK;

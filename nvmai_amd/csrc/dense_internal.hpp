@@ -23,6 +23,7 @@ struct DenseLinearParams {
     float* rms_out;
     uint32_t rms_delta_stride, rms_out_stride;
     float rms_add, rms_eps;
+    bool loose;             // plain outputs need not lie at 16-byte boundaries: one value at a time
 };
 
 // What the form with rms_delta takes beside a 32-bit context: a row is held in the registers of one wave.

@@ -156,7 +156,7 @@ __device__ __forceinline__ void dense_store4(const DenseLinearParams& p, uint32_
         } else if (r0 < p.n) {
             dense_put<ACT>(p, t, r0 / 2u, a);
         }
-    } else if (r0 + 4u <= p.n && (p.y_stride & 3u) == 0) {
+    } else if (r0 + 4u <= p.n && (p.y_stride & 3u) == 0 && !(EPI == DE_PLAIN && p.loose)) {
         v = dense_finish4<EPI, PARTS>(p, t, r0, v, bias);
         if (p.y) {
             act_t<ACT>* y = static_cast<act_t<ACT>*>(p.y) + (size_t)t * p.y_stride + r0;

@@ -2,6 +2,7 @@
 #include <initializer_list>
 
 #include "ctx.hpp"
+#include "dense_internal.hpp"
 #include "step_kernels.hpp"
 
 using namespace nvmai;
@@ -134,46 +135,34 @@ extern "C" int nvmai_hip_attn_qkv_epilogue_kv(nvmai_hip_ctx* ctx, nvmai_stream s
                              position, theta, eps, k_cache, v_cache);
 }
 
-// Dense BF16 rows [m, n] against n_tokens BF16 inputs: the bits == 16 case of nvmai_hip_affine_gemv.
+// Dense BF16 rows [m, n] against n_tokens BF16 inputs: the bits == 16 case of nvmai_hip_affine_gemv, by the dense models' products (a kernel of
+// its own, which loaded sixteen rows by lane, took 24.5 us for 24,832 x 2048 and one input, 18.0 now, 31.1 and 26.2 for sixteen, 185 and 173 for 248,320 rows and
+// one, 421 and 221 for 32; sums against 64 bits 2.7e-7 and 0.7 to 1.3e-7).  Their operands have 32-bit byte offsets: larger ones in portions.
 namespace nvmai {
 int dense_bf16_gemv(nvmai_hip_ctx* ctx, hipStream_t s, const uint16_t* w, const void* x, uint32_t x_stride,
                     uint32_t n_tokens, uint32_t m, uint32_t n, void* y, float* y_f32, uint32_t y_stride) {
     if (ctx->act != ACT_BF16) return NVMAI_ERR_UNSUPPORTED;
     if (n == 0 || n % 64 || n > 4096 || x_stride < n || y_stride < m) return NVMAI_ERR_INVALID_ARG;
     if (!aligned16(w) || !aligned16(x) || x_stride % 8) return NVMAI_ERR_ALIGNMENT;
-    if (m == 0 || n_tokens == 0) return NVMAI_OK;
-    static bool lds_raised = false;
-    if (!lds_raised) {
-        NVMAI_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(dense_bf16_gemv_kernel),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, DENSE_TOK * (4096 * 2 + 16)));
-        lds_raised = true;
-    }
-    const uint32_t groups = (m + 63) / 64;                   // 64 rows per block pass
-    // Blocks per compute unit follow from the staged inputs (4 KB of LDS each at the usual width):
-    // five at one input, two at sixteen.  With three or more the hardware's own hand-out of short
-    // blocks is the fastest form (one pass per block; two or three passes, or one resident round,
-    // measured 3 to 14 % slower at 1..12 inputs: 180 us = 5.7 TB/s for 1.02 GB at one input).  At two
-    // blocks per unit the 64 KB staging of every block is what costs, and one resident round of long
-    // blocks wins (217 -> 202 us at sixteen inputs).
-    static int resident[DENSE_TOK + 1] = {};                 // blocks per compute unit by staged inputs
-    for (uint32_t t0 = 0; t0 < n_tokens; t0 += DENSE_TOK) {
-        const uint32_t nt = n_tokens - t0 < (uint32_t)DENSE_TOK ? n_tokens - t0 : (uint32_t)DENSE_TOK;
-        const uint32_t lds = nt * (n * 2 + 16);
-        int occ = n == 2048 ? resident[nt] : 0;              // cached for the usual width only
-        if (occ == 0) {
-            NVMAI_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, dense_bf16_gemv_kernel, 256, lds));
-            if (occ < 1) occ = 1;
-            if (n == 2048) resident[nt] = occ;
+    const uint32_t most_rows = 0xFFFFFFFFu / (n * 2u) / 256u * 256u;
+    const uint64_t fit = 0xFFFFFFFFull / ((uint64_t)x_stride * 4u);
+    const uint32_t most_tokens = fit > 65536 ? 65536u : fit ? (uint32_t)fit : 1u;
+    for (uint64_t t0 = 0; t0 < n_tokens; t0 += most_tokens)
+        for (uint64_t r0 = 0; r0 < m; r0 += most_rows) {
+            DenseLinearParams p{};
+            p.w = w + (size_t)r0 * n; p.w_stride = n;
+            p.x = static_cast<const uint16_t*>(x) + (size_t)t0 * x_stride;
+            if (y) p.y = static_cast<uint16_t*>(y) + (size_t)t0 * y_stride + r0;
+            if (y_f32) p.y_f32 = y_f32 + (size_t)t0 * y_stride + r0;
+            p.y_stride = y_stride;
+            p.rows = (uint32_t)(n_tokens - t0 < most_tokens ? n_tokens - t0 : most_tokens);
+            p.x_stride = p.rows == 1 ? n : x_stride;
+            p.n = (uint32_t)(m - r0 < most_rows ? m - r0 : most_rows); p.k = n; p.activation = NVMAI_LINEAR_NONE;
+            p.loose = !aligned16(p.y) || !aligned16(p.y_f32);
+            const int rc = dense_linear(ctx, s, p);
+            if (rc) return rc;
         }
-        const uint32_t places = (uint32_t)occ * (uint32_t)ctx->compute_units;
-        const uint32_t per_block = occ >= 3 ? 1u : (groups + places - 1) / places;
-        const dim3 grid((groups + per_block - 1) / per_block);
-        dense_bf16_gemv_kernel<<<grid, 256, lds, s>>>(
-            w, (const uint16_t*)x + (size_t)t0 * x_stride, x_stride, nt, m, n,
-            y ? (uint16_t*)y + (size_t)t0 * y_stride : nullptr, y_f32 ? y_f32 + (size_t)t0 * y_stride : nullptr, y_stride,
-            per_block);
-    }
-    return launch_status();
+    return NVMAI_OK;
 }
 }  // namespace nvmai
 
