@@ -124,6 +124,11 @@ bool expert_widen_pays(const nvmai_hip_ctx* ctx, uint32_t bits, uint32_t tokens,
 int dense_bf16_gemv(nvmai_hip_ctx* ctx, hipStream_t s, const uint16_t* w, const void* x, uint32_t x_stride,
                     uint32_t n_tokens, uint32_t m, uint32_t n, void* y, float* y_f32, uint32_t y_stride);
 
+// sum = hidden (+ delta, if any), rows of their own, out = RMSNorm(sum): residual_add_rmsnorm out of place, in one launch.  False, having launched nothing,
+// for widths that have no such form.
+bool residual_norm_apart(nvmai_hip_ctx* ctx, hipStream_t s, const void* hidden, uint32_t hidden_stride, const void* delta, uint32_t delta_stride,
+                         const uint16_t* weight, void* sum, uint32_t sum_stride, void* out, uint32_t out_stride, uint32_t rows, uint32_t d, float eps);
+
 // Affine 4 / 8-bit rows against 1 .. 32 input rows on the matrix cores, the matrix read once
 // (gemv_mfma_api.hip).  gemv_mfma_ok: the shapes and alignments it takes.
 bool gemv_mfma_ok(const uint8_t* w, const uint16_t* s, const uint16_t* b, uint32_t bits, const void* x,

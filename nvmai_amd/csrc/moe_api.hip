@@ -500,6 +500,17 @@ int affine_gemv_any(nvmai_hip_ctx* ctx, nvmai_stream stream, const uint8_t* weig
 }
 }  // namespace
 
+namespace {
+// Whether three or four input rows take the matrix-core product too: where it is faster than the row engine, which takes the inputs in fp16 pieces as well (engine
+// and product, us, 4 bits, four rows: 12,352 x 2048 13.0 and 9.7, 2048 x 4096 10.1 and 9.3, 512 x 1024 6.7 and 5.4; three: 12,352 x 2048 11.3 and 9.8, 4096 x 2048 6.6 and
+// 6.5; 8 bits, four: 12,352 x 2048 15.4 and 12.0, 4096 x 2048 8.2 and 8.2; sums against 64 bits 8e-6 and 2e-6, 8 bits 5e-7 and 3e-7).  8-bit rows of more than
+// 2048 stay: there the engine's inputs are floats.
+bool few_rows_mfma(uint32_t bits, uint32_t n_tokens, uint32_t m, uint32_t n) {
+    if (n_tokens == 4) return bits == 4 || (n == 2048 && m >= 8192);
+    return n_tokens == 3 && n == 2048 && m >= 8192;
+}
+}  // namespace
+
 extern "C" int nvmai_hip_affine_gemv(nvmai_hip_ctx* ctx, nvmai_stream stream, const uint8_t* weights,
                                      const uint16_t* scales, const uint16_t* biases, uint32_t bits,
                                      const void* x, uint32_t x_stride, uint32_t n_tokens,
@@ -514,7 +525,7 @@ extern "C" int nvmai_hip_affine_gemv(nvmai_hip_ctx* ctx, nvmai_stream stream, co
     // once for all of them.  (Every block of it stages the inputs for itself, which a matrix of
     // LM-head size pays thousands of times: 165 / 280 us at 16 / 32 rows against 116 us through the
     // dense product below -- so that one keeps the large matrices unless fp32 results are asked for.)
-    if (ctx && n_tokens > 4 && n_tokens <= 32 && (m < 32768 || y_f32 || !y) &&
+    if (ctx && (n_tokens > 4 || few_rows_mfma(bits, n_tokens, m, n)) && n_tokens <= 32 && (m < 32768 || y_f32 || !y) &&
         nvmai::gemv_mfma_ok(weights, scales, biases, bits, x, x_stride, n_tokens, m, n, y, y_f32, y_stride))
         return nvmai::gemv_mfma(ctx, (hipStream_t)stream, weights, scales, biases, bits, x, x_stride, n_tokens, m, n, y,
                                 y_f32, y_stride);
@@ -577,6 +588,19 @@ extern "C" int nvmai_hip_affine_gemv_prenorm(nvmai_hip_ctx* ctx, nvmai_stream st
                         aligned16(norm_weight) && (!delta || (aligned16(delta) && delta_stride % 8 == 0));
     // every block norms the rows for itself when they are few, short and may be moved 16 bytes at a time,
     // and the updated residual rows do not overwrite the ones other blocks still read
+    // Rows that take the matrix-core product: the norm in a launch of its own, into the workspace (12,352 x 2048, 4 bits, four rows: 23.6 us in the one
+    // launch, whose blocks norm and stage four rows each, 4.7 + 9.7 so).
+    const bool two_launches = normed_scratch && normed_stride >= n;      // other calls are refused without scratch rows
+    if (few_rows_mfma(bits, n_tokens, m, n) && n == 2048 && m < 32768 && hidden_out != hidden && (two_launches || (m <= 16384 && rows16 && aligned16(weights)))) {
+        const uint16_t* rows = nullptr;
+        uint32_t stride = n;
+        if (ws_begin(ctx, stream, ws_round((size_t)n_tokens * n * 2)) == NVMAI_OK) rows = ws_take<uint16_t>(ctx, (size_t)n_tokens * n);
+        else if (two_launches) { rows = static_cast<const uint16_t*>(normed_scratch); stride = normed_stride; }
+        if (rows && nvmai::gemv_mfma_ok(weights, scales, biases, bits, rows, stride, n_tokens, m, n, y, nullptr, y_stride) &&
+            nvmai::residual_norm_apart(ctx, s, hidden, hidden_stride, delta, delta_stride, norm_weight, hidden_out, hidden_out_stride,
+                                       const_cast<uint16_t*>(rows), stride, n_tokens, n, eps))
+            return nvmai::gemv_mfma(ctx, s, weights, scales, biases, bits, rows, stride, n_tokens, m, n, y, nullptr, y_stride);
+    }
     if (n_tokens <= (uint32_t)MAX_TOK && n <= 2048 && rows16 && aligned16(weights) && hidden_out != hidden) {
         RowsParams p{};
         p.src.slot[0] = weights;

@@ -135,6 +135,20 @@ extern "C" int nvmai_hip_attn_qkv_epilogue_kv(nvmai_hip_ctx* ctx, nvmai_stream s
                              position, theta, eps, k_cache, v_cache);
 }
 
+namespace nvmai {
+bool residual_norm_apart(nvmai_hip_ctx* ctx, hipStream_t s, const void* hidden, uint32_t hidden_stride, const void* delta, uint32_t delta_stride,
+                         const uint16_t* weight, void* sum, uint32_t sum_stride, void* out, uint32_t out_stride, uint32_t rows, uint32_t d, float eps) {
+    if (d != 2048 || rows > RMS_DIRECT_ROWS || rows == 0) return false;
+#define NVMAI_APART(ACT, RESIDUAL)                                                                                                           \
+    rms_direct_kernel<ACT, 2048, RESIDUAL><<<rows, 64, 0, s>>>(static_cast<uint16_t*>(const_cast<void*>(hidden)), hidden_stride, static_cast<const uint16_t*>(delta), \
+                                                           delta_stride, weight, static_cast<uint16_t*>(out), out_stride, eps, static_cast<uint16_t*>(sum), sum_stride)
+    if (ctx->act == ACT_BF16) { if (delta) NVMAI_APART(ACT_BF16, true); else NVMAI_APART(ACT_BF16, false); }
+    else { if (delta) NVMAI_APART(ACT_FP16, true); else NVMAI_APART(ACT_FP16, false); }
+#undef NVMAI_APART
+    return true;
+}
+}  // namespace nvmai
+
 // Dense BF16 rows [m, n] against n_tokens BF16 inputs: the bits == 16 case of nvmai_hip_affine_gemv, by the dense models' products (a kernel of
 // its own, which loaded sixteen rows by lane, took 24.5 us for 24,832 x 2048 and one input, 18.0 now, 31.1 and 26.2 for sixteen, 185 and 173 for 248,320 rows and
 // one, 421 and 221 for 32; sums against 64 bits 2.7e-7 and 0.7 to 1.3e-7).  Their operands have 32-bit byte offsets: larger ones in portions.

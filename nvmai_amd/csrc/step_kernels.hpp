@@ -126,10 +126,11 @@ __global__ __launch_bounds__(256) void residual_add_rmsnorm_kernel(uint16_t* hid
 template <int ACT, int DFIX, bool RESIDUAL>
 __global__ __launch_bounds__(64) void rms_direct_kernel(uint16_t* x, uint32_t x_stride, const uint16_t* delta,
                                                         uint32_t delta_stride, const uint16_t* weight, uint16_t* out,
-                                                        uint32_t out_stride, float eps) {
+                                                        uint32_t out_stride, float eps, uint16_t* sum = nullptr, uint32_t sum_stride = 0) {
     constexpr int N = DFIX / 64;
     const uint32_t row = blockIdx.x, lane = threadIdx.x;
     uint16_t* xr = x + (size_t)row * x_stride;
+    [[maybe_unused]] uint16_t* to = sum ? sum + (size_t)row * sum_stride : xr;      // x (+ delta): in place, or rows of their own
     const uint16_t* dr = RESIDUAL ? delta + (size_t)row * delta_stride : nullptr;
     uint16_t* o = out + (size_t)row * out_stride;
     uint16_t xv[N], dv[N], wv[N];
@@ -149,7 +150,9 @@ __global__ __launch_bounds__(64) void rms_direct_kernel(uint16_t* x, uint32_t x_
     for (int j = 0; j < N; ++j) {
         if (RESIDUAL) {
             xv[j] = f32_to_act<ACT>(__fadd_rn(act_to_f32<ACT>(xv[j]), act_to_f32<ACT>(dv[j])));
-            xr[lane + 64 * j] = xv[j];
+            to[lane + 64 * j] = xv[j];
+        } else if (sum) {
+            to[lane + 64 * j] = xv[j];
         }
         v[j] = act_to_f32<ACT>(xv[j]);
         acc = fmaf(v[j], v[j], acc);

@@ -1,0 +1,59 @@
+"""Three and four input rows against quantized matrices at the lines of the rule that gives them to the matrix cores, and the norm before them."""
+import pytest
+import torch
+
+from gpu_util import say
+from test_gpu_widened import quantized, values
+
+pytestmark = pytest.mark.gpu
+
+
+# Inputs rounded to eleven bits, sums in fp32: off by 2^-11 of the largest value at most, and half a unit of BF16's last place, 2^-8.
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("tokens", [3, 4])
+@pytest.mark.parametrize("m,n", [(8191, 2048), (8192, 2048), (70, 512), (300, 4096), (1000, 2048)])
+def test_products(bits, tokens, m, n):
+    import nvmai_amd as nv
+    from nvmai_amd import ops
+    say("few rows", bits, tokens, m, n)
+    ctx = nv.Context(0, nv.ACT_BF16)
+    w = quantized(ctx, m, n, bits, m + n)
+    x = torch.randn((tokens, n), device="cuda").to(torch.bfloat16)
+    want = x.double() @ values(*w, bits).T
+    y = ops.affine_gemv(ctx, *w, bits, x, m, n)
+    y32 = ops.affine_gemv(ctx, *w, bits, x, m, n, out_f32=True)
+    top = float(want.abs().max())
+    assert float((y.double() - want).abs().max()) <= (2 ** -8 + 2 ** -11) * top
+    assert float((y32.double() - want).abs().max()) <= 2 ** -11 * top
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("tokens,m", [(3, 8192), (4, 8192), (4, 100), (3, 100), (4, 16400)])
+@pytest.mark.parametrize("with_delta", [False, True])
+def test_the_norm_before_them_has_the_bits_of_the_separate_calls(bits, tokens, m, with_delta):
+    import nvmai_amd as nv
+    from nvmai_amd import ops
+    say("few rows behind their norm", bits, tokens, m, with_delta)
+    ctx, fresh = nv.Context(0, nv.ACT_BF16), nv.Context(0, nv.ACT_BF16)
+    n = 2048
+    w = quantized(ctx, m, n, bits, m)
+    hidden, delta = (torch.randn((tokens, n), device="cuda").to(torch.bfloat16) for _ in range(2))
+    weight = torch.randn(n, device="cuda").to(torch.bfloat16).view(torch.int16)
+    want_h = hidden.clone()
+    normed = ops.residual_add_rmsnorm(ctx, want_h, delta, weight) if with_delta else ops.RMSNorm(ctx).encode_bf16w(want_h, weight)
+    want = ops.affine_gemv(ctx, *w, bits, normed, m, n)
+    got_h, scratch = torch.zeros_like(hidden), torch.zeros_like(hidden)
+    y = ops.affine_gemv_prenorm(ctx, *w, bits, hidden, delta if with_delta else None, weight, got_h, m, n, normed_scratch=scratch)
+    assert torch.equal(got_h, want_h) and torch.equal(y, want)
+    # recorded by a context without a workspace, and replayed
+    y, stream, graph = torch.zeros_like(want), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(graph, stream=stream):
+            ops.affine_gemv_prenorm(fresh, *w, bits, hidden, delta if with_delta else None, weight, got_h, m, n, y=y, normed_scratch=scratch)
+    for _ in range(3):
+        y.zero_()
+        got_h.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got_h, want_h) and torch.equal(y, want)
