@@ -6,15 +6,15 @@ using namespace nvmai;
 
 namespace {
 
-template <bool DELTA, int CP>
+template <bool DELTA, int CP, int TAPS>
 int recurrent_launch(const ScanParams& p, uint32_t sequences, uint32_t seq_rows, hipStream_t s) {
     const uint32_t per = (p.dk + 15) / 16;
     const dim3 grid(p.heads, p.dv / (16 * CP), sequences);
-    if (per <= 2) scan_recurrent_kernel<DELTA, 2, CP><<<grid, 256, 0, s>>>(p, seq_rows);
-    else if (per <= 4) scan_recurrent_kernel<DELTA, 4, CP><<<grid, 256, 0, s>>>(p, seq_rows);
-    else if (per <= 8) scan_recurrent_kernel<DELTA, 8, CP><<<grid, 256, 0, s>>>(p, seq_rows);
-    else if (CP == 1 && per <= 16) scan_recurrent_kernel<DELTA, 16, 1><<<grid, 256, 0, s>>>(p, seq_rows);
-    else if (CP == 1) scan_recurrent_kernel<DELTA, 32, 1><<<grid, 256, 0, s>>>(p, seq_rows);
+    if (per <= 2) scan_recurrent_kernel<DELTA, 2, CP, TAPS><<<grid, 256, 0, s>>>(p, seq_rows);
+    else if (per <= 4) scan_recurrent_kernel<DELTA, 4, CP, TAPS><<<grid, 256, 0, s>>>(p, seq_rows);
+    else if (per <= 8) scan_recurrent_kernel<DELTA, 8, CP, TAPS><<<grid, 256, 0, s>>>(p, seq_rows);
+    else if (CP == 1 && per <= 16) scan_recurrent_kernel<DELTA, 16, 1, TAPS><<<grid, 256, 0, s>>>(p, seq_rows);
+    else if (CP == 1) scan_recurrent_kernel<DELTA, 32, 1, 0><<<grid, 256, 0, s>>>(p, seq_rows);
     return launch_status();
 }
 
@@ -22,13 +22,14 @@ template <bool DELTA>
 int recurrent(ScanParams p, bool by_arrays, uint32_t compute_units, hipStream_t s) {
     // four columns per thread when blocks of sixteen columns would come in several rounds
     const bool wide = by_arrays && p.dv % 64 == 0 && p.dk <= 128 && aligned16(p.state) && (uint64_t)p.heads * (p.dv / 16) * p.n_rows > 4ull * compute_units;
-    if (wide) return recurrent_launch<DELTA, 4>(p, p.n_rows, 1, s);
-    if (by_arrays) return recurrent_launch<DELTA, 1>(p, p.n_rows, 1, s);
+    const bool four = p.taps == 4;                   // the filters of the models that have one
+    if (wide) return four ? recurrent_launch<DELTA, 4, 4>(p, p.n_rows, 1, s) : recurrent_launch<DELTA, 4, 0>(p, p.n_rows, 1, s);
+    if (by_arrays || p.n_rows == 1) return four ? recurrent_launch<DELTA, 1, 4>(p, p.n_rows, 1, s) : recurrent_launch<DELTA, 1, 0>(p, p.n_rows, 1, s);
     // consecutive rows: SCAN_AHEAD of them per launch, so that a launch overwrites no history it reads
     const uint32_t rows = p.n_rows;
     for (uint32_t t0 = 0; t0 < rows; t0 += SCAN_AHEAD) {
         p.n_rows = rows - t0 < SCAN_AHEAD ? rows - t0 : SCAN_AHEAD;
-        const int rc = recurrent_launch<DELTA, 1>(p, 1, p.n_rows, s);
+        const int rc = recurrent_launch<DELTA, 1, 0>(p, 1, p.n_rows, s);
         if (rc) return rc;
         p.proj += (size_t)p.n_rows * p.proj_stride;
         p.out += (size_t)p.n_rows * p.out_stride;
