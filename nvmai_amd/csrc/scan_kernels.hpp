@@ -86,7 +86,7 @@ __device__ __forceinline__ void scan_barrier() {
 // TAPS 0: any filter, any number of rows of a sequence.  Otherwise one row, TAPS taps and dk <= 256, so that a thread filters at most one channel each of
 // q, k and v: all that the filters read is requested before the state, from addresses that are valid without a condition (a load under one is waited
 // for on the spot, and tap after tap each waited behind the state).  128 x 128 states, 32 heads of the delta rule or 64 of the state-space form: one
-// sequence 8.4 -> 5.2 and 5.6 us, 16 sequences 23 -> 17.6 us; 64 MB of state each way there, 12.6 us at the rate of a large copy.
+// sequence 8.4 -> 4.9 and 4.5 us, 16 sequences 23 -> 16.5 and 15.2 us; 34 MB of state each way there, 13.4 us at the rate of a large copy.
 template <bool DELTA, int PER, int CP, int TAPS>
 __global__ __launch_bounds__(256) void scan_recurrent_kernel(ScanParams p, uint32_t seq_rows) {
     constexpr uint32_t COLS = 16u * CP;
@@ -103,13 +103,14 @@ __global__ __launch_bounds__(256) void scan_recurrent_kernel(ScanParams p, uint3
     float x[3][N];
     uint16_t w[3][N], bias[3] = {};
     float a_in = 0.0f, b_in = 0.0f;
+    const uint16_t rate_raw = p.a_log[head], dt_bias_raw = p.dt_bias[head], skip_raw = DELTA ? (uint16_t)0 : p.skip[head];
     if constexpr (TAPS != 0) {
         const float* row = p.proj + (size_t)base * p.proj_stride;
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
 #pragma unroll
             for (int n = 0; n < TAPS; ++n) w[i][n] = p.conv[(size_t)ch[i] * TAPS + n];
-            if (p.conv_bias) bias[i] = p.conv_bias[ch[i]];
+            bias[i] = (p.conv_bias ? p.conv_bias : p.conv)[ch[i]];
             x[i][TAPS - 1] = row[p.conv_at + ch[i]];
         }
         a_in = row[p.a_at + head];
@@ -120,13 +121,10 @@ __global__ __launch_bounds__(256) void scan_recurrent_kernel(ScanParams p, uint3
         for (int n = 0; n + 1 < TAPS; ++n) {
             const uint32_t back = TAPS - 1 - n, at = newest >= back ? newest - back : newest + p.history_rows - back;
 #pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                const float old = past[(size_t)at * p.channels + ch[i]];
-                x[i][n] = first >= back ? old : 0.0f;
-            }
+            for (int i = 0; i < 3; ++i) x[i][n] = past[(size_t)at * p.channels + ch[i]];
         }
     }
-    const uint16_t rate_raw = p.a_log[head], dt_bias_raw = p.dt_bias[head], skip_raw = DELTA ? (uint16_t)0 : p.skip[head];
+    if (TAPS) __builtin_amdgcn_sched_barrier(0);     // results come back in the order of the requests: the compiler would put the state's first
     float* S = p.state + (((size_t)slot * p.heads + head) * dk) * p.dv + c0 + CP * j;
     float st[PER][CP];
 #pragma unroll
@@ -138,7 +136,7 @@ __global__ __launch_bounds__(256) void scan_recurrent_kernel(ScanParams p, uint3
     auto filtered = [&](int i) {
         float z = p.conv_bias ? bf16_to_f32(bias[i]) : 0.0f;
 #pragma unroll
-        for (int n = 0; n < TAPS; ++n) z = fmaf(bf16_to_f32(w[i][n]), x[i][n], z);
+        for (int n = 0; n < TAPS; ++n) z = fmaf(bf16_to_f32(w[i][n]), first + n + 1u >= (uint32_t)TAPS ? x[i][n] : 0.0f, z);      // zeros before the sequence
         return silu(z);
     };
     const float rate = expf(bf16_to_f32(rate_raw)), dt_bias = bf16_to_f32(dt_bias_raw), skip = DELTA ? 0.0f : bf16_to_f32(skip_raw);
