@@ -73,6 +73,8 @@ __device__ __forceinline__ void gla_unpack8(const uint4& q, float* w) {
 // rows of the call (PER = 0: any number of them, in memory, where only this thread touches them).  Key channels past
 // the last one have zero decay, key and query in LDS, so that no load or product stands under a condition; a row's
 // operands are requested before the row ahead of it is finished, the first row's before the state.
+// One row of 16 sequences, 16 heads of 128 x 128: 12.9 -> 9.8 us for 17 MB of state each way (6.7 at the rate of a large copy) since the requests are issued in
+// that order too, a single row requests no second one, and the stores of a state without rest stand under no condition.
 template <int ACT, int PER, uint32_t NTH>
 __global__ __launch_bounds__(NTH) void gla_recurrent_kernel(GlaParams p) {
     extern __shared__ __attribute__((aligned(16))) float gla_lds[];
@@ -87,7 +89,10 @@ __global__ __launch_bounds__(NTH) void gla_recurrent_kernel(GlaParams p) {
     float* part = red + 16;              // [groups, dv]
     float* a1s = part + groups * dv;     // [rank]
     const uint32_t slot = p.slots ? p.slots[seq] : p.slot0 + seq;
-    float* S = p.state + ((size_t)slot * p.heads + head) * dk * dv + j;
+    float* const S0 = p.state + ((size_t)slot * p.heads + head) * dk * dv;
+    float* const S = S0 + j;
+    const bool whole = PER > 0 && groups * PER == dk && groups * dv == NTH;      // uniform: every thread has PER rows of the state
+    const uint32_t at0 = c * PER * dv + j;
     const float *qp = p.q + head * dk, *kp = p.k + head * dk, *vp = p.v + head * dv, *gp = p.g + head * dv;
     const uint32_t dc = min(tid, dk - 1u), jc = min(tid, dv - 1u), rc = min(tid, p.rank - 1u), ch = head * dk + dc;
     float a1v, q0, k0, vj, gj;
@@ -103,10 +108,14 @@ __global__ __launch_bounds__(NTH) void gla_recurrent_kernel(GlaParams p) {
     const uint16_t* a2 = p.a2 + (size_t)ch * p.rank;
     const uint4 w0 = *reinterpret_cast<const uint4*>(a2), w1 = *reinterpret_cast<const uint4*>(a2 + (p.rank > 8u ? 8u : 0u));
     const float b0 = bf16_to_f32(p.a2_bias[ch]), nw = bf16_to_f32(p.norm_weight[jc]);
+    __builtin_amdgcn_sched_barrier(0);               // results come back in the order of the requests: the compiler would put the state's first
     float st[PER > 0 ? PER : 1];
-    if (PER > 0) {
+    if (PER > 0 && whole) {
 #pragma unroll
-        for (int e = 0; e < PER; ++e) st[e] = S[(size_t)min(c * PER + e, dk - 1u) * dv];
+        for (int e = 0; e < PER; ++e) st[e] = (S0 + e * dv)[at0];
+    } else if (PER > 0) {
+#pragma unroll
+        for (int e = 0; e < PER; ++e) st[e] = S0[min(c * PER + e, dk - 1u) * dv + j];
     }
     for (uint32_t t = 0; t < p.rows; ++t) {
         const size_t row = (size_t)seq * p.rows + t;
@@ -138,7 +147,7 @@ __global__ __launch_bounds__(NTH) void gla_recurrent_kernel(GlaParams p) {
             al[tid] = real ? __builtin_amdgcn_exp2f(gla_log2_decay(z, p.inv_tau)) : 0.0f;
         }
         const float v = vj, gate = gj;
-        fetch(min(t + 1u, p.rows - 1u));
+        if (t + 1u < p.rows) fetch(t + 1u);
         __syncthreads();
         float o = 0.0f;
         if (PER > 0) {
@@ -181,7 +190,10 @@ __global__ __launch_bounds__(NTH) void gla_recurrent_kernel(GlaParams p) {
             static_cast<act_t<ACT>*>(p.out)[row * p.out_stride + head * dv + tid] = f32_to_act<ACT>(o * inv * nw * gla_silu(gate));
         }
     }
-    if (PER > 0 && owner) {
+    if (PER > 0 && whole) {
+#pragma unroll
+        for (int e = 0; e < PER; ++e) (S0 + e * dv)[at0] = st[e];
+    } else if (PER > 0 && owner) {
 #pragma unroll
         for (int e = 0; e < PER; ++e)
             if (c * PER + e < dk) S[(size_t)(c * PER + e) * dv] = st[e];
