@@ -94,22 +94,28 @@ class DenseDecoder(StepDecoder):
         self.few_ctx = ctx if ctx.act == ops.ACT_FP32 else ops.Context(ctx.device.index, ops.ACT_FP32)
         self.contexts = {ctx, self.few_ctx}
         self.slots = torch.arange(batch, dtype=torch.int32, device=ctx.device)
-        self._buffers = {}
+        self._buffers, self._views = {}, {}
         self.residual_hook = None        # called with (layer index, residual rows) after every layer
         self.logits_f32 = torch.zeros((batch, cfg.vocab), dtype=torch.float32, device=ctx.device)
 
     def pass_context(self, rows):
         return self.few_ctx if rows <= FEW_ROWS else self.ctx
 
-    def _buf(self, name, rows, cols, dtype, most=None):
-        """Scratch rows; most: how many of them a pass takes at most.  Columns past a producer's own stay zero: a buffer's name goes
-        with one width."""
+    def _buf(self, name, rows, cols, dtype, most=None, at=0):
+        """Scratch rows from column `at` on; most: how many of them a pass takes at most.  Columns past a producer's own stay zero: a
+        buffer's name goes with one width.  The view of the last number of rows is kept, one for each place of a buffer: making one takes
+        1.7 to 2.2 us, and a served Pakirax step of 8 layers, bound by the host up to 9 sequences, asks for 75 (430-480 us a step, 360-397 with them kept)."""
+        held = self._views.get((name, cols, dtype, at))
+        if held is not None and held[0] == rows:
+            return held[1]
         key = (name, cols, dtype)
         if key not in self._buffers:
             # buffers of passes in another type than the context's never see more than FEW_ROWS rows
             most = most or (self.max_rows if dtype == self.ctx.dtype or name in self.long_f32 else FEW_ROWS)
             self._buffers[key] = torch.zeros((most, cols), dtype=dtype, device=self.ctx.device)
-        return self._buffers[key][:rows]
+        view = self._buffers[key][:rows, at:]
+        self._views[name, cols, dtype, at] = rows, view
+        return view
 
     def _prefill_chunk_rows(self, tokens, b, start):
         return self._forward(tokens, ops.row_map(b, start))

@@ -357,19 +357,20 @@ class KemuzenDecoder(DenseDecoder):
 
     def _mix(self, ctx, i, linear, T, rows_at):
         m, w = self.cfg.layers[i][0], self.w.layers[i]
-        proj = linear(w["in_proj"], y_f32=self._buf("proj", T, w["in_proj"].shape[0], torch.float32), bias=w["in_bias"])
+        part = lambda n: self._buf("proj", T, w["in_proj"].shape[0], torch.float32, at=n)
+        proj = linear(w["in_proj"], y_f32=part(0), bias=w["in_bias"])
         out, at = self._buf("mixed", T, w["o"].shape[1], ctx.dtype), w["at"]
         if m.kind == "attention":
             self._window(ctx, i, m, proj, rows_at, out)
         elif m.kind == "delta":
             y = self._scan(ctx, i, proj, rows_at, m.heads, m.vdim_p)
-            ops.gated_norm(ctx, y, proj[:, at["g"]:], w["norm"], out, m.vdim, m.heads, False, self.cfg.eps)
+            ops.gated_norm(ctx, y, part(at["g"]), w["norm"], out, m.vdim, m.heads, False, self.cfg.eps)
         else:
             a, r = m.left, m.right
-            self._window(ctx, i, a, proj, rows_at, out, proj[:, at["gate"]:], m.left_scale)
+            self._window(ctx, i, a, proj, rows_at, out, part(at["gate"]), m.left_scale)
             y = self._scan(ctx, i, proj, rows_at, r.heads, r.vdim_p)
-            ops.gated_norm(ctx, y, proj[:, at["z"]:], w["norm"], out[:, a.heads * a.vdim_p:], r.vdim, r.norm_groups, True, self.cfg.eps,
-                           m.right_scale)
+            right = self._buf("mixed", T, w["o"].shape[1], ctx.dtype, at=a.heads * a.vdim_p)
+            ops.gated_norm(ctx, y, part(at["z"]), w["norm"], right, r.vdim, r.norm_groups, True, self.cfg.eps, m.right_scale)
         return ops.dense_linear(ctx, w["o"], out, y_f32=self._buf("delta", T, self.cfg.width_p, torch.float32), bias=w.get("o_bias"))
 
     # -- the layers -------------------------------------------------------------------------------------

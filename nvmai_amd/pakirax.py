@@ -217,8 +217,8 @@ class PakiraxDecoder(DenseDecoder):
     # -- mixers: normed rows in, the sublayer's output as 32-bit rows ---------------------------------------
     def _gla(self, ctx, i, h, rows_at, T, slots):
         m, w, op = self.cfg.layers[i][0], self.w.layers[i], self.mixers[i, ctx]
-        proj = ops.dense_linear(ctx, w["in_proj"], h, y_f32=self._buf("gla_proj", T, w["in_proj"].shape[0], torch.float32))
-        part = lambda n: proj[:, w["at"][n]:]
+        part = lambda n: self._buf("gla_proj", T, w["in_proj"].shape[0], torch.float32, at=w["at"][n])
+        ops.dense_linear(ctx, w["in_proj"], h, y_f32=self._buf("gla_proj", T, w["in_proj"].shape[0], torch.float32))
         out = self._buf("gla_out%d" % (m.heads * m.vdim_p), T, w["o"].shape[1], ctx.dtype)
         batch, rows = (1, T) if slots is None else (T, 1)
         op.encode(part("q"), part("k"), part("v"), part("g"), part("a1"), w["a2"], w["a2_bias"], w["norm"], self.states[i], out,
@@ -233,7 +233,7 @@ class PakiraxDecoder(DenseDecoder):
         op.encode_epilogue(proj, at["q"], m.q_rank, w["q_norm"], at["kv"], at["rope"], w["kv_norm"], cq, self.caches[i], rows_at)
         q = ops.dense_linear(ctx, w["uq"], cq, y=self._buf("latent_q", T, w["uq"].shape[0], dt))
         out = self._buf("latent_out%d" % (m.heads * m.vdim_p), T, w["o"].shape[1], dt)
-        op.encode(q, proj[:, at["g"]:], w["uk"], w["uv"], self.caches[i], rows_at, out)
+        op.encode(q, self._buf("latent_proj", T, w["in_proj"].shape[0], dt, at=at["g"]), w["uk"], w["uv"], self.caches[i], rows_at, out)
         return ops.dense_linear(ctx, w["o"], out, y_f32=self._buf("delta", T, self.cfg.width_p, torch.float32))
 
     # -- the layers -------------------------------------------------------------------------------------
