@@ -177,6 +177,9 @@ struct WindowTiles {
 // sum and outputs of its own, and add them up at the end.  Per tile S^T[key, head] = K Q^T and O^T[value, head] += V^T P^T;
 // row m of score tile 0 (1) is key 8 (m / 4) + m % 4 (+ 4), so a lane's score registers are the keys 8 g .. 8 g + 7 in order
 // and stand as the second product's B operand beside 16 contiguous bytes of V^T.  P enters as two BF16 halves.
+// Bound by the cached rows' bytes and a wave's one or two trips for them: a tile's keys and values are requested together.  16 sequences x 2048 keys, 4 kv
+// heads of 128: 19.9 -> 17.1 us (67 MB, 13.4 at the rate of a large copy) since the values' requests are kept ahead of the softmax.  The next tile's keys
+// requested behind the first product were no faster (16.8 to 19.1; the body twice or more registers).
 template <int DK, int DV>
 __global__ __launch_bounds__(256) void window_split_kernel(WindowParams p) {
     constexpr int KS = DK / 32, VS = DV / 16;
@@ -198,12 +201,14 @@ __global__ __launch_bounds__(256) void window_split_kernel(WindowParams p) {
     const uint16_t* kc = static_cast<const uint16_t*>(p.cache.k) + own * total * dk;
     const uint16_t* vc = static_cast<const uint16_t*>(p.cache.v) + own * dv * total;
     const uint16_t* q = static_cast<const uint16_t*>(p.q) + (size_t)row * p.q_stride + head * dk;
-    const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
     uint4 qf[KS];
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-        const uint4 v = *reinterpret_cast<const uint4*>(q + min(32u * s, dk - 32u) + 8u * g);
-        qf[s] = 32u * s < dk ? v : zero;
+    for (int s = 0; s < KS; ++s) qf[s] = *reinterpret_cast<const uint4*>(q + min(32u * s, dk - 32u) + 8u * g);
+    if (dk < (uint32_t)DK) {                         // only here are the queries waited for ahead of the first tile's requests
+        asm volatile("" ::: "memory");               // a branch, not a selection
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+            if (32u * s >= dk) qf[s] = make_uint4(0u, 0u, 0u, 0u);
     }
     wa_f4 acc[VS];
 #pragma unroll
@@ -222,6 +227,7 @@ __global__ __launch_bounds__(256) void window_split_kernel(WindowParams p) {
         }
 #pragma unroll
         for (int t = 0; t < VS; ++t) vf[t] = *reinterpret_cast<const uint4*>(vc + (size_t)min(16u * t + i, dv - 1u) * total + row0 + 8u * g);
+        __builtin_amdgcn_sched_barrier(0);           // values too are requested here: the compiler would have them wait for the softmax
         wa_f4 s0 = wa_f4{0.0f, 0.0f, 0.0f, 0.0f}, s1 = s0;
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
