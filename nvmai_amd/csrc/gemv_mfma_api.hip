@@ -1,4 +1,4 @@
-// Host side of the matrix-core GEMV for 5 .. 32 input rows.
+// Host side of the matrix-core GEMV for 3 .. 32 input rows.
 #include "ctx.hpp"
 #include "gemv_mfma_kernels.hpp"
 

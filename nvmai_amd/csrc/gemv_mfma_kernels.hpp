@@ -1,4 +1,4 @@
-// Affine 4 / 8-bit group-64 matrix times 5 .. 32 input rows on the matrix cores, for gfx950: the
+// Affine 4 / 8-bit group-64 matrix times 5 .. 32 input rows (three and four where that is faster than the row engine) on the matrix cores, for gfx950: the
 // product a decode step of a small batch needs for its projections and its LM head
 // (dequant_int4.metal:93-215 and dequant_int8.metal's GEMV kernels, issued once per token there).
 // The row engine streams the matrix once per four inputs; here a block reads its 64 rows once for

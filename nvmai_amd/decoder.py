@@ -383,7 +383,7 @@ class HybridDecoder(StepDecoder):
     def _input_projection(self, p_, s_, b_, rows, out, pre):
         """The fused input projections of a layer over its normed input rows.  pre = the norm weight
         of this layer when the residual add of the MoE block before it and this norm are still to
-        be done: the projection launch then does both itself (up to four sequences; same bits)
+        be done: the projection's call then does both itself (up to four sequences; same bits)
         and the updated residual rows go to the second buffer."""
         cfg = self.cfg
         if pre is None:

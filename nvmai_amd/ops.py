@@ -833,8 +833,9 @@ def residual_add_rmsnorm(ctx, hidden, delta, weight, out=None, eps=1e-6):
 def affine_gemv_prenorm(ctx, weights, scales, biases, bits, hidden, delta, norm_weight, hidden_out, m, n, y=None,
                         normed_scratch=None, eps=1e-6):
     """hidden_out = round(hidden + delta); y = W . (rmsnorm(hidden_out) * norm_weight): a layer's input norm
-    and its input projection in one launch for up to four rows (same bits as the two calls).  delta may
-    be None; normed_scratch [rows, n] is only used for shapes without the one-launch form."""
+    and its input projection in one call for up to four rows (same bits as the two calls; one launch, or two where
+    the matrix cores take the rows).  delta may
+    be None; normed_scratch [rows, n] is used for shapes without the one-launch form, and by the two launches without workspace."""
     h2 = hidden.reshape(-1, hidden.shape[-1])
     rows = h2.shape[0]
     if y is None:
