@@ -534,7 +534,8 @@ __global__ __launch_bounds__(skinny_threads(TT, NW, V)) void dense_skinny_kernel
 // Four waves, each a quarter of the tile (BN / 2 x BM / 2) in 16 x 16 x 32 products.  Bound by the rate at which a compute
 // unit takes operands into LDS (about 60 bytes per ns; a tile of 256 x 256 is where the products take as long), below
 // one tile per compute unit by the latency of a step, and where all units multiply by the clock that the card's power leaves.  A tile's rows are 128 bytes
-// of LDS, whose eight 16-byte pieces lie in the order piece ^ skinny_swizzle(row); an operand is read as there.
+// of LDS, whose eight 16-byte pieces lie in the order piece ^ tile_swizzle(row).  An operand is four pieces in a row, and a product adds them in their order:
+// the bits of 32 x 32 x 16 products one after another, whatever the tile.
 //   Which products, and in which order, is a matter of power.  From registers alone, random values, all units: 32 x 32 x 16 1,750 TFLOP/s,
 // 16 x 16 x 32 with the first operand held for runs and the second going to and fro 2,070, in any order that changes the first each time 1,570 to 1,750.
 // With 32 x 32 x 16 these kernels also left the clock of whatever ran next 13 % lower (a router product of 58 us took 66 beside them; 59 now).
@@ -551,6 +552,10 @@ __global__ __launch_bounds__(skinny_threads(TT, NW, V)) void dense_skinny_kernel
 // of 64 k are exact, and their sum goes to a running total of its own, which keeps the rounding of a long k small.
 // Measured (tiles of 128 x 128 x 64 in two stages before): 2048 x 8192 x 2048 77 -> 64 us, 2048 x 2048 x 8192 140 -> 67, 1501 x
 // 2048 x 2048 34 -> 17, 512 x 2048 x 2048 33 -> 9.5 (rows x n x k, cold weights).
+// A read serves the rows 0 .. 3 and 12 .. 15 of one g with 4 .. 11 of the next at once, or sixteen rows of one: pairs of rows in their own order cover eight
+// pieces either way where neighbouring g read neighbouring pieces.
+__device__ __forceinline__ uint32_t tile_swizzle(uint32_t row) { return (row >> 1) & 7u; }
+
 // One sum of the planes again by a whole wave, in fp32 multiply-adds of the values that the planes stand for.  An infinite weight makes
 // NaN of a value's lower planes where they are zero, and planes of sums that overflow can cancel: a NaN comes from here or not
 // at all.  It ends where the sum has become NaN, which it stays; poisoned: by an input that is NaN, so that all sums of its row are.
@@ -690,7 +695,7 @@ __global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_ker
     [[maybe_unused]] const uint32_t x_bytes = (p.rows - 1u) * p.x_stride * 2u + p.k * (SPLIT ? 6u : 2u);
     const uint32_t lr = lane >> 3;
     // request r of a wave: rows 8 r .. 8 r + 7 of its part (8 r + lane / 8 has two values of the swizzle)
-    [[maybe_unused]] const uint32_t piece[2] = {((lane & 7u) ^ skinny_swizzle(lr)) * 16u, ((lane & 7u) ^ skinny_swizzle(lr + 8u)) * 16u};
+    [[maybe_unused]] const uint32_t piece[2] = {((lane & 7u) ^ tile_swizzle(lr)) * 16u, ((lane & 7u) ^ tile_swizzle(lr + 8u)) * 16u};
     // rows past the last: the last one, whose sums are not stored
     [[maybe_unused]] const uint32_t a8 = p.w_stride * 16u, a0 = (n0 + wave * (LA * 8u) + lr) * p.w_stride * 2u, amax = (p.n - 1u) * p.w_stride * 2u;
     [[maybe_unused]] const uint32_t b8 = p.x_stride * 16u, b0 = (m0 + wave * (LB * 8u) + lr) * p.x_stride * 2u, bmax = (p.rows - 1u) * p.x_stride * 2u;
@@ -715,9 +720,9 @@ __global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_ker
     const uint32_t wn = (wave >> 1) * (BN / 2), wm = (wave & 1u) * (BM / 2);
     const uint32_t arow = (wn + i) * 128u, brow = BN * 128u + (wm + i) * 128u;
     uint4 fa[2][TN], fb[2][TM];
-    // operands of the half h (32 k: the pieces 2 g + h) of the stage at place j: the tokens' and the first half of the weights' (part 0), the rest (part 1)
+    // operands of the half h (32 k: the pieces 4 h + g) of the stage at place j: the tokens' and the first half of the weights' (part 0), the rest (part 1)
     auto fetch = [&](int j, int h, int part) {
-        const uint32_t sw = ((2u * g + h) ^ skinny_swizzle(i)) * 16u;
+        const uint32_t sw = ((4u * h + g) ^ tile_swizzle(i)) * 16u;
         if (part == 0) {
 #pragma unroll
             for (int b = 0; b < TM; ++b) fb[h][b] = *reinterpret_cast<const uint4*>(buf(j) + brow + 2048u * b + sw);
@@ -877,7 +882,7 @@ __global__ __launch_bounds__(256, 1) void dense_wide_kernel(DenseLinearParams p,
     [[maybe_unused]] const uint32_t w_bytes = (p.n - 1u) * p.w_stride * 2u + p.k * 2u, x_bytes = (p.rows - 1u) * p.x_stride * 2u + p.k * 2u;
     // request r of a wave: rows 32 wave + 8 r .. + 7 of a half (8 r + lane / 8 has two values of the swizzle)
     const uint32_t lr = lane >> 3;
-    [[maybe_unused]] const uint32_t piece[2] = {((lane & 7u) ^ skinny_swizzle(lr)) * 16u, ((lane & 7u) ^ skinny_swizzle(lr + 8u)) * 16u};
+    [[maybe_unused]] const uint32_t piece[2] = {((lane & 7u) ^ tile_swizzle(lr)) * 16u, ((lane & 7u) ^ tile_swizzle(lr + 8u)) * 16u};
     const uint32_t row = (wave & 1u) * 32u + (wave >> 1) * 128u + lr;
     [[maybe_unused]] const uint32_t w8 = p.w_stride * 16u, w0 = (n0 + row) * p.w_stride * 2u, wmax = (p.n - 1u) * p.w_stride * 2u;
     [[maybe_unused]] const uint32_t x8 = p.x_stride * 16u, x0 = (m0 + row) * p.x_stride * 2u, xmax = (p.rows - 1u) * p.x_stride * 2u;
@@ -902,8 +907,8 @@ __global__ __launch_bounds__(256, 1) void dense_wide_kernel(DenseLinearParams p,
     const uint32_t arow = ((wave >> 1) * 64u + i) * 128u, brow = ((wave & 1u) * 64u + i) * 128u;
     uint4 A[2][2][4], B[2][2][4];                            // [half][32 k][tile of 16]
     // operand e of eight of a half
-    auto read_w = [&](int j, int h, int e) { A[h][e >> 2][e & 3] = *reinterpret_cast<const uint4*>(wbuf(j, h) + arow + 2048u * (e & 3) + (((2u * g + (e >> 2)) ^ skinny_swizzle(i)) * 16u)); };
-    auto read_x = [&](int j, int h, int e) { B[h][e >> 2][e & 3] = *reinterpret_cast<const uint4*>(xbuf(j, h) + brow + 2048u * (e & 3) + (((2u * g + (e >> 2)) ^ skinny_swizzle(i)) * 16u)); };
+    auto read_w = [&](int j, int h, int e) { A[h][e >> 2][e & 3] = *reinterpret_cast<const uint4*>(wbuf(j, h) + arow + 2048u * (e & 3) + (((4u * (e >> 2) + g) ^ tile_swizzle(i)) * 16u)); };
+    auto read_x = [&](int j, int h, int e) { B[h][e >> 2][e & 3] = *reinterpret_cast<const uint4*>(xbuf(j, h) + brow + 2048u * (e & 3) + (((4u * (e >> 2) + g) ^ tile_swizzle(i)) * 16u)); };
     dn_f4 acc[8][8];
 #pragma unroll
     for (int a = 0; a < 8; ++a)
@@ -1085,6 +1090,7 @@ struct DenseTile {
 };
 constexpr DenseTile DENSE_TILES[] = {{64, 64, 16, 23}, {128, 64, 25, 38}, {128, 128, 43, 58}, {256, 128, 76, 100}, {256, 256, 114, 162}};
 constexpr int DENSE_CUT_TILES = 3;                           // of these the first may be cut along k
+constexpr float DENSE_CUT_BELOW = 0.875f;                    // where the time falls below this share: parts end in other roundings than a sum in one piece
 
 struct DensePlan {
     int tile;
@@ -1095,7 +1101,7 @@ struct DensePlan {
 // planes: the stages of 64 k.  cut: whether there is a place for the sums of parts.  (Few divisions, and those of 32 bits: the choice is made in every
 // call, and short prompts are bound by the host.)
 inline DensePlan dense_plan_tile(uint32_t n, uint32_t rows, uint32_t k, uint32_t planes, uint32_t cus, int count, bool cut) {
-    DensePlan best{0, 1, 1e30f};
+    DensePlan whole{0, 1, 1e30f}, parted{0, 1, 1e30f};
     const uint32_t steps = k / 64u;
     const float units = 1.0f / (float)cus, stages = 10.0f * (float)planes;
     for (int c = 0; c < count; ++c) {
@@ -1105,21 +1111,23 @@ inline DensePlan dense_plan_tile(uint32_t n, uint32_t rows, uint32_t k, uint32_t
         const float lone = (float)t.lone, rise = (float)(t.full - t.lone) * units;
         const float cost = (float)rounds * (float)t.full + (rest ? lone + rise * (float)rest : 0.0f);
         const float ns = cost * stages * (float)steps + 4750.0f;             // and a launch, the first requests, the stores
-        if (ns < best.ns) best = {c, 1, ns};
+        if (ns < whole.ns) whole = {c, 1, ns};
         if (!cut || rounds != 0 || c >= DENSE_CUT_TILES) continue;
         const float area = (float)(t.bn * t.bm);
         for (uint32_t parts = 2; parts * 2u <= steps && parts <= DENSE_PARTS && tiles * parts <= cus; parts += parts < 4u ? 1u : parts / 4u * 2u) {
             const float blocks = (float)(tiles * parts);
             const float join = 1000.0f + area * ((float)parts * (1.0f / 16.0f) + blocks * (1.0f / 3500.0f));
             const float ns = (lone + rise * blocks) * stages * (float)((steps + parts - 1) / parts) + 4750.0f + join;
-            if (ns < best.ns) best = {c, parts, ns};
+            if (ns < parted.ns) parted = {c, parts, ns};
         }
     }
-    return best;
+    return parted.ns < whole.ns * DENSE_CUT_BELOW ? parted : whole;
 }
 
 // The matrix's rows in one launch, or in two where that is shorter: a last round that few units take part in is left to
 // smaller tiles (8208 weight rows, 2048 tokens: one round of 256 x 256 and a sixteenth of one, 105 -> 76 us in all).
+// Neither is cut along k: all outputs of such a product are sums in one order, that of a product which fills the units (cut, those sixteen rows would save
+// 3 us of the 76, and end in other roundings than the rows beside them).
 struct DenseSplit {
     uint32_t first;                                          // rows of the first launch
     DensePlan head, tail;
@@ -1135,7 +1143,7 @@ inline DenseSplit dense_plan(uint32_t n, uint32_t rows, uint32_t k, uint32_t pla
         const uint32_t rounds = (uint32_t)((uint64_t)tn * tm / cus);
         const uint32_t cut = (uint32_t)((uint64_t)rounds * cus / tm) * DENSE_TILES[c].bn;
         if (cut == 0 || cut >= n) continue;
-        const DensePlan head = dense_plan_tile(cut, rows, k, planes, cus, count, split), tail = dense_plan_tile(n - cut, rows, k, planes, cus, count, split);
+        const DensePlan head = dense_plan_tile(cut, rows, k, planes, cus, count, false), tail = dense_plan_tile(n - cut, rows, k, planes, cus, count, false);
         if (head.ns + tail.ns < best.ns) best = {cut, head, tail, head.ns + tail.ns};
     }
     return best;
