@@ -5,6 +5,7 @@
 
 #include "ctx.hpp"
 #include "moe_kernels.hpp"
+#include "rules.hpp"
 
 using namespace nvmai;
 
@@ -497,17 +498,6 @@ int affine_gemv_any(nvmai_hip_ctx* ctx, nvmai_stream stream, const uint8_t* weig
         else store_rows_kernel<ACT_FP16><<<grid, 256, 0, s>>>(tmp, y, y_f32, m, y_stride);
     }
     return launch_status();
-}
-}  // namespace
-
-namespace {
-// Whether three or four input rows take the matrix-core product too: where it is faster than the row engine, which takes the inputs in fp16 pieces as well (engine
-// and product, us, 4 bits, four rows: 12,352 x 2048 13.0 and 9.7, 2048 x 4096 10.1 and 9.3, 512 x 1024 6.7 and 5.4; three: 12,352 x 2048 11.3 and 9.8, 4096 x 2048 6.6 and
-// 6.5; 8 bits, four: 12,352 x 2048 15.4 and 12.0, 4096 x 2048 8.2 and 8.2; sums against 64 bits 8e-6 and 2e-6, 8 bits 5e-7 and 3e-7).  8-bit rows of more than
-// 2048 stay: there the engine's inputs are floats.
-bool few_rows_mfma(uint32_t bits, uint32_t n_tokens, uint32_t m, uint32_t n) {
-    if (n_tokens == 4) return bits == 4 || (n == 2048 && m >= 8192);
-    return n_tokens == 3 && n == 2048 && m >= 8192;
 }
 }  // namespace
 

@@ -1,0 +1,27 @@
+// Choices between the forms of a call that sizes alone decide: plain C++, without a device.
+#pragma once
+
+#include <stdint.h>
+
+namespace nvmai {
+
+// Widths whose rows the row engine reads in 16, 32, 64 or 128 pieces of sixteen bytes, with its inputs as fp16 numbers (moe_kernels.hpp).  At
+// others it takes floats.
+inline bool rows_engine_fp16(uint32_t bits, uint32_t n) {
+    const uint64_t width = (uint64_t)n * bits;
+    return width == 16u * 128u || width == 32u * 128u || width == 64u * 128u || width == 128u * 128u;
+}
+
+// Whether three or four input rows of an affine matrix take the matrix-core product, as five do: where it is faster than the row engine and the engine
+// takes the inputs as fp16 numbers too.  Engine and product, us, 4 bits, four rows: 12,352 x 2048 13.0 and 9.7, 2048 x 4096 10.1 and 9.3, 512 x 1024 6.7 and 5.4,
+// 2048 x 512 5.6 and 5.4; three: 12,352 x 2048 11.3 and 9.8, 4096 x 2048 6.6 and 6.5, 1024 x 2048 5.5 and 5.7, 2048 x 4096 8.2 and 9.4; 8 bits, four: 12,352 x 2048 15.4
+// and 12.0, 4096 x 2048 8.2 and 8.2, 512 x 1024 5.6 and 6.1; sums against 64 bits 8e-6 and 2e-6, 8 bits 5e-7 and 3e-7.  Three rows and 8 bits: the widths of one
+// size are level below 8192 matrix rows (6 % for either), so the line lies where the gain is sure.  Up to 30,000 rows were measured (20.8 and 18.8); larger
+// matrices stay.
+inline bool few_rows_mfma(uint32_t bits, uint32_t n_tokens, uint32_t m, uint32_t n) {
+    if (m >= 32768u || !rows_engine_fp16(bits, n)) return false;
+    if (n_tokens == 4) return bits == 4 || (n == 2048 && m >= 8192);
+    return n_tokens == 3 && n == 2048 && m >= 8192;
+}
+
+}  // namespace nvmai

@@ -57,3 +57,20 @@ def test_the_norm_before_them_has_the_bits_of_the_separate_calls(bits, tokens, m
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(got_h, want_h) and torch.equal(y, want)
+
+
+# Widths for which the row engine has no instantiation with its inputs in fp16: sums of floats, each of a lane's n / 64 products and the lanes' sums rounded to
+# 24 bits, 2^-24 sqrt(n / 64 + 6) = 6e-7 of the value at most at these n (2-norm; inputs rounded to eleven bits as for the matrix cores give 1.2e-6 to 3.7e-6).
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("tokens", [3, 4])
+@pytest.mark.parametrize("n", [1536, 2560, 3584, 5120])
+def test_other_widths_keep_inputs_of_32_bits(bits, tokens, n):
+    import nvmai_amd as nv
+    from nvmai_amd import ops
+    say("few rows, other widths", bits, tokens, n)
+    ctx, m = nv.Context(0, nv.ACT_BF16), 300
+    w = quantized(ctx, m, n, bits, n)
+    x = torch.randn((tokens, n), device="cuda").to(torch.bfloat16)
+    want = x.double() @ values(*w, bits).T
+    got = ops.affine_gemv(ctx, *w, bits, x, m, n, out_f32=True)
+    assert float((got.double() - want).norm() / want.norm()) <= 6e-7

@@ -1,0 +1,29 @@
+"""Choices between forms of a call that sizes alone decide, compiled for the host."""
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "nvmai_amd", "csrc")
+
+
+@pytest.fixture(scope="module")
+def rule(tmp_path_factory):
+    """Answers of one expression of nvmai's rules for a list of values of its variables."""
+    def answers(names, rows, expression):
+        at = tmp_path_factory.mktemp("rules")
+        (at / "rules.cpp").write_text('#include <stdio.h>\n#include "rules.hpp"\nusing namespace nvmai;\nint main() {\n    unsigned %s;\n    while (scanf("%s", %s) == %d) printf("%%lld\\n", (long long)(%s));\n}\n'
+                                      % (", ".join(names), "%u " * len(names), ", ".join("&" + n for n in names), len(names), expression))
+        subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, "-o", str(at / "rules"), str(at / "rules.cpp")], check=True)
+        out = subprocess.run([str(at / "rules")], input="\n".join(" ".join(str(v) for v in r) for r in rows), text=True, check=True, stdout=subprocess.PIPE).stdout
+        return [int(v) for v in out.split()]
+    return answers
+
+
+def test_few_rows_take_the_matrix_cores_only_in_place_of_inputs_in_fp16(rule):
+    cases = [(b, t, m, n) for b in (4, 8) for t in (3, 4) for m in (1, 8192, 32767, 32768, 248320) for n in range(64, 8193, 64)]
+    for (bits, tokens, m, n), taken in zip(cases, rule(("bits", "tokens", "m", "n"), cases, "few_rows_mfma(bits, tokens, m, n)")):
+        in_fp16 = n in ((512, 1024, 2048, 4096) if bits == 4 else (256, 512, 1024, 2048))
+        assert not taken or (in_fp16 and m < 32768), (bits, tokens, m, n)
+        if tokens == 4 and bits == 4 and in_fp16 and m < 32768:
+            assert taken
