@@ -3,6 +3,7 @@
 #include "ctx.hpp"
 #include "dense_kernels.hpp"
 #include "ends_kernels.hpp"
+#include "rules.hpp"
 
 using namespace nvmai;
 
@@ -56,7 +57,7 @@ int dense_linear_check(const nvmai_hip_ctx* ctx, const DenseLinearParams& p) {
     if (!aligned16(p.w) || !aligned16(p.x) || p.w_stride % 8 || p.x_stride % 8) return NVMAI_ERR_ALIGNMENT;
     if (!p.loose && ((p.y && !aligned16(p.y)) || (p.y_f32 && !aligned16(p.y_f32)))) return NVMAI_ERR_ALIGNMENT;
     // 32-bit byte offsets inside an operand
-    if ((uint64_t)p.n * p.w_stride * 2 > 0xFFFFFFFFull || (uint64_t)p.rows * p.x_stride * 4 > 0xFFFFFFFFull) return NVMAI_ERR_UNSUPPORTED;
+    if ((uint64_t)p.n * p.w_stride * 2 > 0xFFFFFFFFull || !dense_rows_fit(p.rows, p.x_stride)) return NVMAI_ERR_UNSUPPORTED;
     return NVMAI_OK;
 }
 

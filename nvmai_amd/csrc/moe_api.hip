@@ -841,7 +841,7 @@ extern "C" int nvmai_hip_shared_expert(nvmai_hip_ctx* ctx, nvmai_stream stream, 
         const bool gated_d = shared_gate && shared_gate->kind;
         const size_t rows = ws_round((size_t)n_tokens * f * 2) + ws_round((size_t)n_tokens * d * 2) + ws_round(n_tokens * 4u) + ws_round(16),
                      widened = ws_round((size_t)d * f * 6);
-        const bool widen = (uint64_t)n_tokens * x_stride * 4 <= 0xFFFFFFFFull && nvmai::expert_widen_pays(ctx, bits, n_tokens, d, f) &&
+        const bool widen = expert_rows_fit(n_tokens, x_stride, f) && nvmai::expert_widen_pays(ctx, bits, n_tokens, d, f) &&
                            ws_begin(ctx, stream, rows + widened) == NVMAI_OK;
         if (!widen && (rc = ws_begin(ctx, stream, rows))) return rc;
         uint16_t* act = ws_take<uint16_t>(ctx, (size_t)n_tokens * f);

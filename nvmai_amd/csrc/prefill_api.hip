@@ -2,6 +2,7 @@
 #include "ctx.hpp"
 #include "dense_internal.hpp"
 #include "prefill_kernels.hpp"
+#include "rules.hpp"
 
 using namespace nvmai;
 
@@ -214,7 +215,7 @@ bool widen_pays(const nvmai_hip_ctx* ctx, uint32_t bits, uint32_t rows, uint32_t
 // Widens and multiplies, if that pays and the workspace can hold the rows; false: nothing is launched.
 bool widened_product(nvmai_hip_ctx* ctx, nvmai_stream stream, uint32_t bits, const uint8_t* weights, const uint16_t* scales, const uint16_t* biases,
                      DenseLinearParams d, int* rc) {
-    if (!widen_pays(ctx, bits, d.rows, d.n, d.k) || (uint64_t)d.rows * d.x_stride * 4 > 0xFFFFFFFFull) return false;
+    if (!widen_pays(ctx, bits, d.rows, d.n, d.k) || !dense_rows_fit(d.rows, d.x_stride)) return false;
     if (ws_begin(ctx, stream, ws_round((size_t)d.n * d.k * 2)) != NVMAI_OK) return false;
     uint16_t* wide = ws_take<uint16_t>(ctx, (size_t)d.n * d.k);
     WidenParams p{};

@@ -24,4 +24,10 @@ inline bool few_rows_mfma(uint32_t bits, uint32_t n_tokens, uint32_t m, uint32_t
     return n_tokens == 3 && n == 2048 && m >= 8192;
 }
 
+// Whether a dense product can address `rows` input rows of `stride` values with 32-bit byte offsets (values of up to four bytes).
+inline bool dense_rows_fit(uint32_t rows, uint32_t stride) { return (uint64_t)rows * stride * 4 <= 0xFFFFFFFFull; }
+
+// The same of both products of a shared expert: its tokens, and the f values that it holds of each between them.
+inline bool expert_rows_fit(uint32_t tokens, uint32_t x_stride, uint32_t f) { return dense_rows_fit(tokens, x_stride) && dense_rows_fit(tokens, f); }
+
 }  // namespace nvmai

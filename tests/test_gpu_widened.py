@@ -92,3 +92,27 @@ def test_shared_expert(bits, tokens, d, f):
     want = (torch.nn.functional.silu(xd @ w[0].T) * (xd @ w[1].T)) @ w[2].T
     y = ops.SharedExpertRuntime(ctx, bits).encode(blob, off, x, d, f)
     assert float((y.double() - want).abs().max() / want.abs().max()) < 2 * TOL
+
+
+def test_a_shared_expert_past_the_offsets_of_the_widened_form():
+    """f values of 131,200 tokens lie 4.3 GB apart as the dense products count them: the form that dequantizes per tile takes the call."""
+    import nvmai_amd as nv
+    from nvmai_amd import ops
+    bits, tokens, d, f = 4, 131200, 2048, 8192
+    say("shared expert of many tokens", bits, tokens, d, f)
+    ctx = nv.Context(0, nv.ACT_BF16)
+    off, stride = nv.expert_offsets(d, f, bits)
+    blob = torch.empty(stride, dtype=torch.uint8, device="cuda")
+    w = []
+    for i, (n, k, wo, so, bo) in enumerate(((f, d, off.gate_w, off.gate_s, off.gate_b), (f, d, off.up_w, off.up_s, off.up_b), (d, f, off.down_w, off.down_s, off.down_b))):
+        q = quantized(ctx, n, k, bits, i)
+        for t, o in zip(q, (wo, so, bo)):
+            flat = t.view(torch.uint8).view(-1)
+            blob[o:o + flat.numel()] = flat
+        w.append(values(*q, bits))
+    x = torch.empty((tokens, d), device="cuda", dtype=torch.bfloat16).normal_()
+    y = ops.SharedExpertRuntime(ctx, bits).encode(blob, off, x, d, f)
+    at = torch.tensor([0, 1, 65535, 65536, 131071, 131072, 131199], device="cuda")
+    xd = x[at].double()
+    want = (torch.nn.functional.silu(xd @ w[0].T) * (xd @ w[1].T)) @ w[2].T
+    assert float((y[at].double() - want).abs().max() / want.abs().max()) < 2 * TOL

@@ -27,3 +27,12 @@ def test_few_rows_take_the_matrix_cores_only_in_place_of_inputs_in_fp16(rule):
         assert not taken or (in_fp16 and m < 32768), (bits, tokens, m, n)
         if tokens == 4 and bits == 4 and in_fp16 and m < 32768:
             assert taken
+
+
+def test_a_shared_expert_is_widened_only_where_both_products_take_its_rows(rule):
+    cases = [(t, s, f) for t in (192, 131071, 131072, 140000, 262143, 262144, 600000) for s in (2048, 4096, 8192) for f in (512, 8192, 16384)]
+    for (tokens, stride, f), fits, x, act in zip(cases, rule(("t", "s", "f"), cases, "expert_rows_fit(t, s, f)"), rule(("t", "s", "f"), cases, "dense_rows_fit(t, s)"),
+                                                 rule(("t", "s", "f"), cases, "dense_rows_fit(t, f)")):
+        assert x == (tokens * stride * 4 < 2 ** 32) and act == (tokens * f * 4 < 2 ** 32)
+        assert fits == (x and act), (tokens, stride, f)
+    assert rule(("t", "s", "f"), [(140000, 2048, 8192)], "expert_rows_fit(t, s, f)") == [0]      # taken, and refused after its first product
