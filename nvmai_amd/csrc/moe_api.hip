@@ -834,10 +834,19 @@ extern "C" int nvmai_hip_shared_expert(nvmai_hip_ctx* ctx, nvmai_stream stream, 
     hipStream_t s = (hipStream_t)stream;
     // A block of tokens (prefill): the expert's matrices are read once for all of them by the
     // grouped-GEMM kernels instead of once per four tokens (the reference runs its dense QMM
-    // there, MPPPrefillInt4QMM.swift:18-128).  Operands past the kernels' 32-bit offsets, and
-    // small batches (the two ways cost the same at about 200 tokens), take the row engine below.
-    if (n_tokens >= 192 && (uint64_t)n_tokens * x_stride * 2 <= 0xFFFFFFFFull &&
-        (uint64_t)n_tokens * d * 2 <= 0xFFFFFFFFull && (uint64_t)d * f * bits / 8 <= 0xFFFFFFFFull) {
+    // there, MPPPrefillInt4QMM.swift:18-128), in portions where operands pass the kernels' 32-bit
+    // offsets.  Small batches (the two ways cost the same at about 200 tokens) take the row engine below.
+    const uint32_t most = expert_block_tokens(x_stride, d, f, bits);
+    if (n_tokens >= 192 && most >= 192) {
+        if (n_tokens > most) {
+            for (uint32_t t = 0; t < n_tokens; t += most) {
+                rc = nvmai_hip_shared_expert(ctx, stream, blob, off, bits, shared_gate, static_cast<const uint16_t*>(x) + (size_t)t * x_stride, x_stride,
+                                             n_tokens - t < most ? n_tokens - t : most, static_cast<uint16_t*>(y) + (size_t)t * y_stride, y_stride, d, f);
+                if (rc) return rc;
+                if (n_tokens - t <= most) break;             // t + most may pass 32 bits
+            }
+            return NVMAI_OK;
+        }
         const bool gated_d = shared_gate && shared_gate->kind;
         const size_t rows = ws_round((size_t)n_tokens * f * 2) + ws_round((size_t)n_tokens * d * 2) + ws_round(n_tokens * 4u) + ws_round(16),
                      widened = ws_round((size_t)d * f * 6);

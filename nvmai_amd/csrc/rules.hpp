@@ -30,4 +30,12 @@ inline bool dense_rows_fit(uint32_t rows, uint32_t stride) { return (uint64_t)ro
 // The same of both products of a shared expert: its tokens, and the f values that it holds of each between them.
 inline bool expert_rows_fit(uint32_t tokens, uint32_t x_stride, uint32_t f) { return dense_rows_fit(tokens, x_stride) && dense_rows_fit(tokens, f); }
 
+// How many tokens of a shared expert the products that dequantize per tile take in one call: x, the f values between them and the output have 32-bit
+// byte offsets, in 16 bits.  0: the codes themselves are too many.
+inline uint32_t expert_block_tokens(uint32_t x_stride, uint32_t d, uint32_t f, uint32_t bits) {
+    if ((uint64_t)d * f * bits / 8 > 0xFFFFFFFFull) return 0;
+    const uint32_t widest = x_stride > d ? (x_stride > f ? x_stride : f) : (d > f ? d : f);
+    return 0xFFFFFFFFu / 2u / widest / 128u * 128u;
+}
+
 }  // namespace nvmai

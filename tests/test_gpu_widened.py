@@ -94,11 +94,12 @@ def test_shared_expert(bits, tokens, d, f):
     assert float((y.double() - want).abs().max() / want.abs().max()) < 2 * TOL
 
 
-def test_a_shared_expert_past_the_offsets_of_the_widened_form():
-    """f values of 131,200 tokens lie 4.3 GB apart as the dense products count them: the form that dequantizes per tile takes the call."""
+@pytest.mark.parametrize("tokens", [131200, 270000])
+def test_a_shared_expert_past_offsets_of_32_bits(tokens):
+    """f values of 131,200 tokens lie 4.3 GB apart as the dense products count them: the form that dequantizes per tile takes the call; 270,000 in two portions."""
     import nvmai_amd as nv
     from nvmai_amd import ops
-    bits, tokens, d, f = 4, 131200, 2048, 8192
+    bits, d, f = 4, 2048, 8192
     say("shared expert of many tokens", bits, tokens, d, f)
     ctx = nv.Context(0, nv.ACT_BF16)
     off, stride = nv.expert_offsets(d, f, bits)
@@ -112,7 +113,7 @@ def test_a_shared_expert_past_the_offsets_of_the_widened_form():
         w.append(values(*q, bits))
     x = torch.empty((tokens, d), device="cuda", dtype=torch.bfloat16).normal_()
     y = ops.SharedExpertRuntime(ctx, bits).encode(blob, off, x, d, f)
-    at = torch.tensor([0, 1, 65535, 65536, 131071, 131072, 131199], device="cuda")
+    at = torch.tensor([0, 1, 65535, 65536, 131071, 131072, 131199, tokens - 7985, tokens - 7984, tokens - 1], device="cuda")
     xd = x[at].double()
     want = (torch.nn.functional.silu(xd @ w[0].T) * (xd @ w[1].T)) @ w[2].T
     assert float((y[at].double() - want).abs().max() / want.abs().max()) < 2 * TOL

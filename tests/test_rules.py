@@ -36,3 +36,12 @@ def test_a_shared_expert_is_widened_only_where_both_products_take_its_rows(rule)
         assert x == (tokens * stride * 4 < 2 ** 32) and act == (tokens * f * 4 < 2 ** 32)
         assert fits == (x and act), (tokens, stride, f)
     assert rule(("t", "s", "f"), [(140000, 2048, 8192)], "expert_rows_fit(t, s, f)") == [0]      # taken, and refused after its first product
+
+
+def test_a_shared_expert_takes_the_tiles_in_portions_whose_operands_have_offsets_of_32_bits(rule):
+    cases = [(s, d, f, b) for d in (64, 1024, 2048, 8192) for s in (d, d + 64, 1 << 24, 1 << 31) for f in (64, 512, 8192, 131072, 1 << 24) for b in (4, 8)]
+    for (s, d, f, b), most in zip(cases, rule(("s", "d", "f", "b"), cases, "expert_block_tokens(s, d, f, b)")):
+        widest = max(s, d, f) * 2
+        assert most * widest < 2 ** 32 and (most + 128) * widest > 2 ** 32 - 2 * widest or (most == 0 and d * f * b // 8 >= 2 ** 32), (s, d, f, b)
+    # 270,000 tokens x 8192 had offsets that wrapped: outputs past token 262,143 were other tokens'
+    assert rule(("s", "d", "f", "b"), [(2048, 2048, 8192, 4)], "expert_block_tokens(s, d, f, b)") == [262016]
