@@ -659,8 +659,11 @@ int nvmai_hip_residual_add_rmsnorm(nvmai_hip_ctx* ctx, nvmai_stream stream, void
  * launch for up to four rows of at most 2048 elements against a projection of at most 16,384 rows:
  * every block norms the rows for itself (same arithmetic and order, so the same bits), the first
  * block stores the updated residual rows to hidden_out, which must not be `hidden` (other blocks
- * still read it).  delta may be NULL (norm only).  Any other shape runs the steps one after the other
- * through normed_scratch ([n_tokens, normed_stride] activations; NVMAI_ERR_UNSUPPORTED when NULL). */
+ * still read it).  Three and four rows that nvmai_hip_affine_gemv gives to the matrix cores (2048 elements,
+ * fewer than 32,768 projection rows) take two launches, their normed rows in 16 KB of the ctx: eager and captured alike,
+ * with and without a workspace, the bits are those of the two calls.  delta may be NULL (norm only).  Any other shape
+ * runs the steps one after the other through normed_scratch ([n_tokens, normed_stride] activations, not touched
+ * otherwise; NVMAI_ERR_UNSUPPORTED when NULL). */
 int nvmai_hip_affine_gemv_prenorm(nvmai_hip_ctx* ctx, nvmai_stream stream, const uint8_t* weights,
                                   const uint16_t* scales, const uint16_t* biases, uint32_t bits, const void* hidden,
                                   uint32_t hidden_stride, const void* delta, uint32_t delta_stride,

@@ -23,6 +23,7 @@ struct nvmai_hip_ctx {
     std::vector<void*> ws_retired;
     uint8_t* static_scratch; // device address of the library's static scratch array on this device (ctx_api.hip)
     uint32_t* tickets;       // zero-initialised device words for last-block-done kernels (TICKET_WORDS)
+    uint16_t* norm_rows;     // behind them: normed rows between the two launches of affine_gemv_prenorm (NORM_ROWS x NORM_WIDTH)
     float* cut_sums;         // sums of blocks that share a tile (CUT_SUMS_BYTES), or nullptr: no tile is shared
     // Optional per-kernel timing: event pairs recorded around tagged launches.
     bool prof_on;
@@ -37,6 +38,10 @@ namespace nvmai {
 // [16, 48) sampler block counters, [TICKET_CUTS, + CUT_BLOCKS) tiles that several blocks share.
 constexpr uint32_t TICKET_WORDS = 2048;
 constexpr uint32_t TICKET_CUTS = 64;
+
+// Rows of the context's own, so that a call with them takes the same launches with and without a workspace.
+constexpr uint32_t NORM_ROWS = 4, NORM_WIDTH = 2048;
+constexpr size_t TICKET_BYTES = TICKET_WORDS * 4, NORM_BYTES = (size_t)NORM_ROWS * NORM_WIDTH * 2;
 
 // Blocks that share tiles in one launch at most, and their sums: a tile of 128 x 128 floats each.
 constexpr uint32_t CUT_BLOCKS = 256;

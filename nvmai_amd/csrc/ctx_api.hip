@@ -58,11 +58,12 @@ extern "C" int nvmai_hip_ctx_create(int device, int act_dtype, nvmai_hip_ctx** o
     ctx->ws_used = 0;
     ctx->prof_on = false;
     ctx->tickets = nullptr;
-    if (hipMalloc(reinterpret_cast<void**>(&ctx->tickets), TICKET_WORDS * 4) != hipSuccess ||
-        hipMemset(ctx->tickets, 0, TICKET_WORDS * 4) != hipSuccess) {
+    if (hipMalloc(reinterpret_cast<void**>(&ctx->tickets), TICKET_BYTES + NORM_BYTES) != hipSuccess ||
+        hipMemset(ctx->tickets, 0, TICKET_BYTES) != hipSuccess) {
         delete ctx;
         return NVMAI_ERR_HIP;
     }
+    ctx->norm_rows = reinterpret_cast<uint16_t*>(ctx->tickets + TICKET_WORDS);
     // allocated here and not by the call that first needs it, which may be captured; products are made without it too
     ctx->cut_sums = nullptr;
     if (hipMalloc(reinterpret_cast<void**>(&ctx->cut_sums), CUT_SUMS_BYTES) != hipSuccess) {

@@ -576,21 +576,16 @@ extern "C" int nvmai_hip_affine_gemv_prenorm(nvmai_hip_ctx* ctx, nvmai_stream st
     hipStream_t s = (hipStream_t)stream;
     const bool rows16 = aligned16(hidden) && hidden_stride % 8 == 0 && aligned16(hidden_out) && hidden_out_stride % 8 == 0 &&
                         aligned16(norm_weight) && (!delta || (aligned16(delta) && delta_stride % 8 == 0));
+    // Rows that take the matrix-core product: the norm in a launch of its own, into rows of the context (12,352 x 2048, 4 bits, four rows: 23.6 us in the
+    // one launch below, whose blocks norm and stage four rows each, 4.7 + 9.7 so).  Calls that would need scratch rows are refused without them all the same.
+    const bool taken = (normed_scratch && normed_stride >= n) || (m <= 16384 && rows16 && aligned16(weights));
+    if (few_rows_mfma(bits, n_tokens, m, n) && n == NORM_WIDTH && hidden_out != hidden && taken &&
+        nvmai::gemv_mfma_ok(weights, scales, biases, bits, ctx->norm_rows, n, n_tokens, m, n, y, nullptr, y_stride) &&
+        nvmai::residual_norm_apart(ctx, s, hidden, hidden_stride, delta, delta_stride, norm_weight, hidden_out, hidden_out_stride, ctx->norm_rows, n,
+                                   n_tokens, n, eps))
+        return nvmai::gemv_mfma(ctx, s, weights, scales, biases, bits, ctx->norm_rows, n, n_tokens, m, n, y, nullptr, y_stride);
     // every block norms the rows for itself when they are few, short and may be moved 16 bytes at a time,
     // and the updated residual rows do not overwrite the ones other blocks still read
-    // Rows that take the matrix-core product: the norm in a launch of its own, into the workspace (12,352 x 2048, 4 bits, four rows: 23.6 us in the one
-    // launch, whose blocks norm and stage four rows each, 4.7 + 9.7 so).
-    const bool two_launches = normed_scratch && normed_stride >= n;      // other calls are refused without scratch rows
-    if (few_rows_mfma(bits, n_tokens, m, n) && n == 2048 && m < 32768 && hidden_out != hidden && (two_launches || (m <= 16384 && rows16 && aligned16(weights)))) {
-        const uint16_t* rows = nullptr;
-        uint32_t stride = n;
-        if (ws_begin(ctx, stream, ws_round((size_t)n_tokens * n * 2)) == NVMAI_OK) rows = ws_take<uint16_t>(ctx, (size_t)n_tokens * n);
-        else if (two_launches) { rows = static_cast<const uint16_t*>(normed_scratch); stride = normed_stride; }
-        if (rows && nvmai::gemv_mfma_ok(weights, scales, biases, bits, rows, stride, n_tokens, m, n, y, nullptr, y_stride) &&
-            nvmai::residual_norm_apart(ctx, s, hidden, hidden_stride, delta, delta_stride, norm_weight, hidden_out, hidden_out_stride,
-                                       const_cast<uint16_t*>(rows), stride, n_tokens, n, eps))
-            return nvmai::gemv_mfma(ctx, s, weights, scales, biases, bits, rows, stride, n_tokens, m, n, y, nullptr, y_stride);
-    }
     if (n_tokens <= (uint32_t)MAX_TOK && n <= 2048 && rows16 && aligned16(weights) && hidden_out != hidden) {
         RowsParams p{};
         p.src.slot[0] = weights;

@@ -835,7 +835,7 @@ def affine_gemv_prenorm(ctx, weights, scales, biases, bits, hidden, delta, norm_
     """hidden_out = round(hidden + delta); y = W . (rmsnorm(hidden_out) * norm_weight): a layer's input norm
     and its input projection in one call for up to four rows (same bits as the two calls; one launch, or two where
     the matrix cores take the rows).  delta may
-    be None; normed_scratch [rows, n] is used for shapes without the one-launch form, and by the two launches without workspace."""
+    be None; normed_scratch [rows, n] is only used for shapes without these forms."""
     h2 = hidden.reshape(-1, hidden.shape[-1])
     rows = h2.shape[0]
     if y is None:

@@ -74,3 +74,32 @@ def test_other_widths_keep_inputs_of_32_bits(bits, tokens, n):
     want = x.double() @ values(*w, bits).T
     got = ops.affine_gemv(ctx, *w, bits, x, m, n, out_f32=True)
     assert float((got.double() - want).norm() / want.norm()) <= 6e-7
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("tokens,m", [(3, 8192), (4, 8192), (4, 100), (3, 100)])
+def test_the_norm_before_them_needs_neither_workspace_nor_scratch_rows(bits, tokens, m):
+    """A context that has made no call yet records the launches that it makes eagerly, and scratch rows stay as they are."""
+    import nvmai_amd as nv
+    from nvmai_amd import ops
+    say("few rows behind their norm, without workspace", bits, tokens, m)
+    ctx, fresh, n = nv.Context(0, nv.ACT_BF16), nv.Context(0, nv.ACT_BF16), 2048
+    w = quantized(ctx, m, n, bits, m)
+    hidden, delta = (torch.randn((tokens, n), device="cuda").to(torch.bfloat16) for _ in range(2))
+    weight = torch.randn(n, device="cuda").to(torch.bfloat16).view(torch.int16)
+    want_h = hidden.clone()
+    want = ops.affine_gemv(ctx, *w, bits, ops.residual_add_rmsnorm(ctx, want_h, delta, weight), m, n)
+    got_h, scratch = torch.zeros_like(hidden), torch.full_like(hidden, 7.0)
+    y = ops.affine_gemv_prenorm(ctx, *w, bits, hidden, delta, weight, got_h, m, n, normed_scratch=scratch)
+    assert torch.equal(y, want) and bool((scratch == 7).all())
+    y, stream, graph = torch.zeros_like(want), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(graph, stream=stream):
+            ops.affine_gemv_prenorm(fresh, *w, bits, hidden, delta, weight, got_h, m, n, y=y)
+    for _ in range(3):
+        y.zero_()
+        got_h.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got_h, want_h) and torch.equal(y, want)
