@@ -12,7 +12,7 @@ def rule(tmp_path_factory):
     """Answers of one expression of nvmai's rules for a list of values of its variables."""
     def answers(names, rows, expression):
         at = tmp_path_factory.mktemp("rules")
-        (at / "rules.cpp").write_text('#include <stdio.h>\n#include "rules.hpp"\nusing namespace nvmai;\nint main() {\n    unsigned %s;\n    while (scanf("%s", %s) == %d) printf("%%lld\\n", (long long)(%s));\n}\n'
+        (at / "rules.cpp").write_text('#include <stdio.h>\n#include "dense_plan.hpp"\n#include "rules.hpp"\nusing namespace nvmai;\nint main() {\n    unsigned %s;\n    while (scanf("%s", %s) == %d) printf("%%lld\\n", (long long)(%s));\n}\n'
                                       % (", ".join(names), "%u " * len(names), ", ".join("&" + n for n in names), len(names), expression))
         subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, "-o", str(at / "rules"), str(at / "rules.cpp")], check=True)
         out = subprocess.run([str(at / "rules")], input="\n".join(" ".join(str(v) for v in r) for r in rows), text=True, check=True, stdout=subprocess.PIPE).stdout
@@ -45,3 +45,37 @@ def test_a_shared_expert_takes_the_tiles_in_portions_whose_operands_have_offsets
         assert most * widest < 2 ** 32 and (most + 128) * widest > 2 ** 32 - 2 * widest or (most == 0 and d * f * b // 8 >= 2 ** 32), (s, d, f, b)
     # 270,000 tokens x 8192 had offsets that wrapped: outputs past token 262,143 were other tokens'
     assert rule(("s", "d", "f", "b"), [(2048, 2048, 8192, 4)], "expert_block_tokens(s, d, f, b)") == [262016]
+
+
+PLAN = "dense_plan(n, rows, k, planes, 256, planes == 3 ? 3 : 5, cut)"
+
+
+def test_which_tiles_the_cut_sizes_take(rule):
+    """The sizes of the test on the device between them take every tile that may be cut, and the fewest and most parts."""
+    from test_gpu_dense_cut import SHAPES
+    names = ("rows", "n", "k", "planes", "cut")
+    for planes, tiles, parts in ((1, {0, 1, 2}, {2, 12}), (3, {0, 1, 2}, {2, 12})):
+        cases = [(*shape, planes, 1) for shape in SHAPES]
+        got = list(zip(rule(names, cases, PLAN + ".head.tile"), rule(names, cases, PLAN + ".head.parts")))
+        assert {t for t, p in got if p > 1} == tiles and parts <= {p for _, p in got}, got
+        assert got[-1][1] == 1
+
+
+def test_parts_have_a_unit_each_and_are_taken_where_they_save_time(rule):
+    names = ("rows", "n", "k", "planes", "cut")
+    cases = [(r, n, k, p, 1) for r in (5, 20, 65, 130, 300, 700, 1501, 2048, 4096) for n in (64, 250, 1024, 2048, 4160, 8256, 11264) for k in (64, 256, 1024, 2048, 8192, 32768)
+             for p in (1, 3) if p == 3 or r > 64]
+    value = lambda what, at=cases: rule(names, at, what)
+    sizes = ((64, 64), (128, 64), (128, 128), (256, 128), (256, 256))
+    whole = value(PLAN + ".ns", [(*c[:4], 0) for c in cases])
+    for (rows, n, k, planes, _), first, tile, parts, tail, ns, uncut in zip(cases, value(PLAN + ".first"), value(PLAN + ".head.tile"), value(PLAN + ".head.parts"),
+                                                                            value(PLAN + ".tail.parts"), value(PLAN + ".ns"), whole):
+        bn, bm = sizes[tile]
+        if first < n:                                # two launches: neither is cut
+            assert parts == 1 and tail == 1
+        if parts > 1:
+            assert parts in (2, 3, 4, 6, 8, 12) and 2 * parts <= k // 64
+            assert -(-n // bn) * -(-rows // bm) * parts <= 256 and ns <= uncut - 1699
+    # what one sum per output is for: prompts of 4096 tokens in portions of 2048, and of 1501
+    long = [(2048, n, 2048, 1, 1) for n in (2048, 4160, 8192, 8256)] + [(2048, 2048, 8192, 1, 1), (1501, 256, 2048, 1, 1), (1501, 2048, 5632, 1, 1), (1501, 11264, 2048, 1, 1)]
+    assert set(value(PLAN + ".head.parts", long)) == {1}
