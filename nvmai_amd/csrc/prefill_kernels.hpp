@@ -915,17 +915,20 @@ __global__ __launch_bounds__(256, 2) void prefill_gemm_kernel(GemmParams p) {
     const int ld_t = lane >> 4;
     const bool ld_on = NT == 4 || ld_t < NT;
     const bool ld_second = DUAL && (ld_t & 1);
+    // A dense product's arrays are taken from the dword at or below their first entry to the one that holds their last: a dword that
+    // sticks out of a resource reads as zero, the entry in it too (the last scale of an odd number of them).
+    const uint32_t s_odd = DUAL ? 0u : (uint32_t)reinterpret_cast<uintptr_t>(blob + p.sA) & 2u, b_odd = DUAL ? 0u : (uint32_t)reinterpret_cast<uintptr_t>(blob + p.bA) & 2u;
     uint32_t so_lane, bo_lane;
     {
         uint32_t c = DUAL ? n0 + wave * (8 * NT) + (ld_t >> 1) * 16 + li : n0 + wave * (16 * NT) + ld_t * 16 + li;
         c = min(c, p.N - 1) * groups * 2u;
-        so_lane = (DUAL ? (uint32_t)(ld_second ? p.sB : p.sA) : 0u) + c;
-        bo_lane = (DUAL ? (uint32_t)(ld_second ? p.bB : p.bA) : 0u) + c;
+        so_lane = (DUAL ? (uint32_t)(ld_second ? p.sB : p.sA) : s_odd) + c;
+        bo_lane = (DUAL ? (uint32_t)(ld_second ? p.bB : p.bA) : b_odd) + c;
     }
     // DUAL: gate and up arrays are reached from the expert's base (the lane picks the matrix)
     const uint32_t blob_bytes = (uint32_t)(p.pool_stride < 0xFFFFFFFFull ? p.pool_stride : 0xFFFFFFFFull);
-    const __amdgpu_buffer_rsrc_t s_rs = DUAL ? rsrc_of(0, blob_bytes) : rsrc_of(p.sA, sb_bytes);
-    const __amdgpu_buffer_rsrc_t b_rs = DUAL ? rsrc_of(0, blob_bytes) : rsrc_of(p.bA, sb_bytes);
+    const __amdgpu_buffer_rsrc_t s_rs = DUAL ? rsrc_of(0, blob_bytes) : rsrc_of(p.sA - s_odd, (sb_bytes + s_odd + 3u) & ~3u);
+    const __amdgpu_buffer_rsrc_t b_rs = DUAL ? rsrc_of(0, blob_bytes) : rsrc_of(p.bA - b_odd, (sb_bytes + b_odd + 3u) & ~3u);
     // raw: CS + 1 dwords from the dword at or below the row's chunk
     auto load_sb = [&](auto csc, uint32_t* rs_, uint32_t* rb_, uint32_t chunk) {
         constexpr int CS = decltype(csc)::value;
@@ -1310,8 +1313,8 @@ __global__ __launch_bounds__(256, 2) void prefill_gemm_kernel(GemmParams p) {
                 const uint32_t t = row >> 4, c16 = row & 15u;
                 uint32_t c = DUAL ? n0 + wave * (8 * NT) + (t >> 1) * 16 + c16 : n0 + wave * (16 * NT) + t * 16 + c16;
                 c = min(c, p.N - 1) * g2 + piece * 16u;
-                const uint32_t so = (DUAL ? (uint32_t)((t & 1) ? p.sB : p.sA) : 0u) + c;
-                const uint32_t bo = (DUAL ? (uint32_t)((t & 1) ? p.bB : p.bA) : 0u) + c;
+                const uint32_t so = (DUAL ? (uint32_t)((t & 1) ? p.sB : p.sA) : s_odd) + c;
+                const uint32_t bo = (DUAL ? (uint32_t)((t & 1) ? p.bB : p.bA) : b_odd) + c;
                 const uint32_t at = wave * (NT * 16u) * g2 + i * 1024u;
                 if (q < total) {
                     __builtin_amdgcn_raw_ptr_buffer_load_lds(s_rs, (__attribute__((address_space(3))) void*)(tab_s + at), 16, so, 0, 0, 0);

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 import oracle as O
-from gpu_util import act_np, act_tensor, dev, gauss, say, u32
+from gpu_util import act_np, act_tensor, dev, gauss, round_act, say, u32
 
 pytestmark = pytest.mark.gpu
 
@@ -527,3 +527,20 @@ def test_streamed_tiles_equal_the_resident_pool_call(nv, ctx_bf16, bits):
     with pytest.raises(nv.NvmaiError):
         moe.encode_streamed_batched(xd, routes.sorted_pairs, got, act, crooked,
                                     nv.prefill_streamed_params(0, 4, d, f, k, xd.stride(0), crooked, off))
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m,n,k", [(16, 33, 64), (40, 257, 192), (130, 1999, 320), (300, 65, 2112)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_dense_qmm_uses_the_last_scale_of_an_odd_number(nv, ctx, bits, m, n, k, shift):
+    """Odd rows of an odd number of groups: the last scale and bias fill half of a dword, whichever half word the arrays start at.  The last column alone,
+    whose last group weighs 64 / k of it and more."""
+    say("dense qmm, odd number of scales", ctx.act, bits, m, n, k, shift)
+    rng = np.random.default_rng(m + n + k + bits)
+    p, s, b = O.quantize_affine(gauss(rng, (n, k), 0.05), bits)
+    x = round_act(gauss(rng, (m, k)), ctx.act)
+    meta = [torch.empty(n * k // 64 + shift, dtype=torch.int16, device="cuda")[shift:].copy_(dev(t.view(np.int16)).view(-1)).view(n, -1) for t in (s, b)]
+    y = nv.MPPPrefillInt4QMM(ctx, bits).encode(dev(p), *meta, act_tensor(x, ctx), n, k)
+    torch.cuda.synchronize()
+    want = np.stack([O.affine_gemv(p, s, b, x[t], bits) for t in range(m)])
+    assert O.rel_error(act_np(y)[:, -1], want[:, -1]) <= TOL_ACT and O.rel_error(act_np(y), want) <= TOL_ACT

@@ -70,6 +70,34 @@ def test_a_captured_product_without_workspace_dequantizes_per_tile():
             assert float((y.double() - want).abs().max() / want.abs().max()) < TOL
 
 
+# The two forms round the same values to the same weights (a scale and a bias of eight bits each: the shifted bias of the form per tile is exact) and add in
+# another order: sums apart by 2^-20 of their size at most.  Outputs then are, where a sum lies that near the middle of two BF16 values, which are 2^-8 of it
+# apart or half that: one output in 2^11, by 2^-8 of itself on average.  In all 2^-5.5 2^-8 of the outputs; not nothing, which would be one form twice.
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("rows,n,k", [(65, 2048, 4096), (130, 1999, 2112), (700, 1024, 2048), (257, 2048, 4096)])
+def test_both_forms_round_alike(bits, rows, n, k):
+    import nvmai_amd as nv
+    from nvmai_amd import ops
+    say("product over quantized rows, both forms", bits, rows, n, k)
+    ctx, fresh = nv.Context(0, nv.ACT_BF16), nv.Context(0, nv.ACT_BF16)
+    w = quantized(ctx, n, k, bits, n + k)
+    x = torch.randn((rows, k), device="cuda").to(torch.bfloat16)
+    widened, per_tile = torch.empty((rows, n), dtype=torch.bfloat16, device="cuda"), torch.empty((rows, n), dtype=torch.bfloat16, device="cuda")
+    encode = lambda c, y: ops.MPPPrefillInt4QMM(c, bits).encode(*w, x, n, k, y=y)
+    encode(ctx, widened)
+    torch.cuda.synchronize()
+    assert ctx.workspace_bytes >= n * k * 2                           # the form in question
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(graph, stream=stream):
+            encode(fresh, per_tile)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert fresh.workspace_bytes == 0
+    a, b = widened.double(), per_tile.double()
+    assert 0 < float((a - b).norm() / b.norm()) <= 2 ** -13.5
+
+
 # The hidden row is rounded to BF16 between the products and the output once more: TOL for each of the two products covers them.
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("tokens,d,f", [(192, 1024, 256), (333, 2048, 512), (2100, 512, 320)])
