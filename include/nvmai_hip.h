@@ -26,6 +26,9 @@
  *     the matrix as BF16 in the workspace for the call, up to 256 MB).  They do the same where memory cannot be allocated.
  *     Beside the workspace a ctx holds 16 MB from its creation on, where the blocks that share an output tile
  *     meet; if they cannot be allocated, no tile is shared (slower products of few rows, other roundings).
+ *     They and a word per tile that counts its blocks belong to the one stream of the ctx, as the workspace does: products
+ *     of one ctx that run at the same time, on two streams or in two replayed graphs, may add each other's sums, and may leave
+ *     a count behind that spoils later products of that ctx.
  * Data formats (reference file:line):
  *   - weights: affine group-64 codes, 4 bit (two per byte, element 2k in the low
  *     nibble of byte k) or 8 bit, plus one BF16 scale and one BF16 bias per group
