@@ -202,7 +202,7 @@ __global__ __launch_bounds__(256) void dense_gemv_kernel(DenseLinearParams p) {
         uint4 wv[U][RW], xv[U][NT][XP];
 #pragma unroll
         for (int s = 0; s < U; ++s) {
-            const uint32_t at = min(k0 + 512u * s + lane * 8u, p.k - 8u);        // past the end: the last piece, taken as zeros
+            const uint32_t at = min(k0 + 512u * s + lane * 8u, p.k - 8u);        // past the end: the last piece, whose sums are dropped
 #pragma unroll
             for (int r = 0; r < RW; ++r) wv[s][r] = *reinterpret_cast<const uint4*>(wp[r] + at);
 #pragma unroll
@@ -211,47 +211,42 @@ __global__ __launch_bounds__(256) void dense_gemv_kernel(DenseLinearParams p) {
                 for (int u = 0; u < XP; ++u) xv[s][t][u] = reinterpret_cast<const uint4*>(x + (size_t)t * p.x_stride + at)[u];
         }
         __builtin_amdgcn_sched_barrier(0);
-        auto multiply = [&](auto tail) {
 #pragma unroll
-            for (int s = 0; s < U; ++s) {
-                const bool live = !decltype(tail)::value || k0 + 512u * s + lane * 8u < p.k;
-                const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
-                float wf[RW][8];
+        for (int s = 0; s < U; ++s) {
+            const bool live = k0 + 512u * s + lane * 8u < p.k;
+            float wf[RW][8];
+#pragma unroll
+            for (int r = 0; r < RW; ++r) {
+                const uint4 q = wv[s][r];
+                act2_to_f32<ACT_BF16>(q.x, wf[r][0], wf[r][1]);
+                act2_to_f32<ACT_BF16>(q.y, wf[r][2], wf[r][3]);
+                act2_to_f32<ACT_BF16>(q.z, wf[r][4], wf[r][5]);
+                act2_to_f32<ACT_BF16>(q.w, wf[r][6], wf[r][7]);
+            }
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                float xf[8];
+                if constexpr (ACT == ACT_FP32) {
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        xf[4 * u] = __uint_as_float(xv[s][t][u].x); xf[4 * u + 1] = __uint_as_float(xv[s][t][u].y);
+                        xf[4 * u + 2] = __uint_as_float(xv[s][t][u].z); xf[4 * u + 3] = __uint_as_float(xv[s][t][u].w);
+                    }
+                } else {
+                    act2_to_f32<ACT_BF16>(xv[s][t][0].x, xf[0], xf[1]);
+                    act2_to_f32<ACT_BF16>(xv[s][t][0].y, xf[2], xf[3]);
+                    act2_to_f32<ACT_BF16>(xv[s][t][0].z, xf[4], xf[5]);
+                    act2_to_f32<ACT_BF16>(xv[s][t][0].w, xf[6], xf[7]);
+                }
 #pragma unroll
                 for (int r = 0; r < RW; ++r) {
-                    const uint4 q = live ? wv[s][r] : zero;
-                    act2_to_f32<ACT_BF16>(q.x, wf[r][0], wf[r][1]);
-                    act2_to_f32<ACT_BF16>(q.y, wf[r][2], wf[r][3]);
-                    act2_to_f32<ACT_BF16>(q.z, wf[r][4], wf[r][5]);
-                    act2_to_f32<ACT_BF16>(q.w, wf[r][6], wf[r][7]);
-                }
+                    float sum = acc[t][r];
 #pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    float xf[8];
-                    uint4 q[XP];                             // an input past the end is zero too: no weight makes zero of an infinity
-#pragma unroll
-                    for (int u = 0; u < XP; ++u) q[u] = live ? xv[s][t][u] : zero;
-                    if constexpr (ACT == ACT_FP32) {
-#pragma unroll
-                        for (int u = 0; u < 2; ++u) {
-                            xf[4 * u] = __uint_as_float(q[u].x); xf[4 * u + 1] = __uint_as_float(q[u].y);
-                            xf[4 * u + 2] = __uint_as_float(q[u].z); xf[4 * u + 3] = __uint_as_float(q[u].w);
-                        }
-                    } else {
-                        act2_to_f32<ACT_BF16>(q[0].x, xf[0], xf[1]);
-                        act2_to_f32<ACT_BF16>(q[0].y, xf[2], xf[3]);
-                        act2_to_f32<ACT_BF16>(q[0].z, xf[4], xf[5]);
-                        act2_to_f32<ACT_BF16>(q[0].w, xf[6], xf[7]);
-                    }
-#pragma unroll
-                    for (int r = 0; r < RW; ++r)
-#pragma unroll
-                        for (int j = 0; j < 8; ++j) acc[t][r] = fmaf(wf[r][j], xf[j], acc[t][r]);
+                    for (int j = 0; j < 8; ++j) sum = fmaf(wf[r][j], xf[j], sum);
+                    acc[t][r] = live ? sum : acc[t][r];
                 }
             }
-        };
-        if (p.k - k0 >= 512u * U) multiply(std::false_type{});
-        else multiply(std::true_type{});
+        }
     }
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
