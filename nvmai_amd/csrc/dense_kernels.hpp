@@ -182,7 +182,8 @@ __device__ __forceinline__ void dense_store4(const DenseLinearParams& p, uint32_
 // Bound by the matrix's bytes.  The inputs are read from L1 / L2 beside the weights (no LDS, no barrier): every
 // load of a k step is independent of the others, so a wave has RW + NT (32-bit inputs: RW + 2 NT) 16-byte loads per lane
 // in flight.
-template <int EPI, int ACT, int NT, int RW>
+// U steps of 512 k whose loads are all issued before the first product.
+template <int EPI, int ACT, int NT, int RW, int U>
 __global__ __launch_bounds__(256) void dense_gemv_kernel(DenseLinearParams p) {
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t r0 = (blockIdx.x * 4u + wave) * RW;
@@ -197,7 +198,6 @@ __global__ __launch_bounds__(256) void dense_gemv_kernel(DenseLinearParams p) {
 #pragma unroll
         for (int r = 0; r < RW; ++r) acc[t][r] = 0.0f;
     constexpr int XP = ACT == ACT_FP32 ? 2 : 1;
-    constexpr int U = NT * XP + RW <= 3 ? 4 : 2;             // steps of 512 k whose loads are all issued before the first product
     for (uint32_t k0 = 0; k0 < p.k; k0 += 512u * U) {
         uint4 wv[U][RW], xv[U][NT][XP];
 #pragma unroll
@@ -1046,10 +1046,32 @@ __global__ __launch_bounds__(256) void dense_f32_kernel(DenseLinearParams p) {
 // ---- launches ---------------------------------------------------------------------------------------------
 template <int EPI, int ACT, int NT>
 void launch_gemv(const DenseLinearParams& p, hipStream_t s) {
-    // rows per wave: one (short blocks, many of them) until the inputs' own loads weigh more than that
-    if (p.n >= 65536) dense_gemv_kernel<EPI, ACT, NT, 4><<<(p.n + 15) / 16, 256, 0, s>>>(p);
-    else if (EPI == DE_PAIRS || (NT * (ACT == ACT_FP32 ? 2 : 1) > 2 && p.n >= 8192)) dense_gemv_kernel<EPI, ACT, NT, 2><<<(p.n + 7) / 8, 256, 0, s>>>(p);
-    else if constexpr (EPI != DE_PAIRS) dense_gemv_kernel<EPI, ACT, NT, 1><<<(p.n + 3) / 4, 256, 0, s>>>(p);
+    constexpr int X = NT * (ACT == ACT_FP32 ? 2 : 1);        // loads of the inputs per step
+    auto go = [&](auto rw, auto u) {
+        constexpr int RW = decltype(rw)::value, U = decltype(u)::value;
+        dense_gemv_kernel<EPI, ACT, NT, RW, U><<<(p.n + 4 * RW - 1) / (4 * RW), 256, 0, s>>>(p);
+    };
+    constexpr std::integral_constant<int, 1> one{};
+    constexpr std::integral_constant<int, 2> two{};
+    constexpr std::integral_constant<int, 4> four{};
+    constexpr bool PAIRS = EPI == DE_PAIRS;
+    // Rows per wave: one (short blocks, many of them) until the inputs' own loads weigh more than that.  Steps past the end of k are loads for nothing: where k ends
+    // before they do, fewer steps and more rows (BF16 us, one row per wave and four steps, and so: 24,833 x 576 one input 11.2 and 7.2, two 14.8 and 8.4; 21,845 x 1024
+    // 12.1 and 9.9, 15.3 and 10.2; 2048 x 1024 3.0 and 2.8; 4096 x 512 3.3 and 2.8, 4.1 and 3.2; 30,000 x 192 11.1 and 5.2; three inputs of 4096 x 512 in two steps 3.8 and 3.2).
+    // The bits depend on neither.
+    if (p.k <= 512) {
+        if (p.n >= 8192) go(four, one);
+        else if (PAIRS || (X <= 2 && p.n >= 2048)) go(two, one);
+        else if constexpr (!PAIRS) go(one, one);
+    } else if (p.n >= 65536) {
+        go(four, two);
+    } else if (X <= 2 && p.k <= 1024 && p.n >= 2048) {
+        go(two, two);
+    } else if (PAIRS || (X > 2 && p.n >= 8192)) {
+        go(two, std::integral_constant<int, X == 1 ? 4 : 2>{});
+    } else if constexpr (!PAIRS) {
+        go(one, std::integral_constant<int, X <= 2 ? 4 : 2>{});
+    }
 }
 
 template <int EPI, int NT, int S>
