@@ -13,8 +13,9 @@ namespace nvmai {
 // own: a step's latency is then paid by all units at once.  The join costs a trip to memory and back, the parts' sums that the last block takes back and
 // the sums of all.  Rows x n x k, cold weights, uncut and cut, us: 65 x 2048 x 8192 26.9 and 13.8, 128 x 2048 x 5632 28.8 and 13.9, 300 x 1024 x 4096
 // 18.4 and 11.7, 700 x 2048 x 8192 48.6 and 40.5, 300 x 2048 x 4096 18.9 and 17.1, 128 x 256 x 2048 7.9 and 6.4; 32-bit rows 20 x 1024 x 4096 39 and 14, 128 x 1024 x 2816
-// 27.6 and 15.1, 500 x 1024 x 4096 48 and 32, 300 x 1024 x 1024 14.5 and 13.3.  Products that would save less than 1.7 us by these costs stay whole, one
-// sum per output: 1000 x 256 x 2048 7.7 and 8.7, 1501 x 256 x 2048 7.9 and 8.3, 700 x 512 x 2048 8.0 and 8.1, 65 x 2048 x 2048 9.6 and 9.3, 32-bit 70 x 4112 x 1024 14.4 and 15.5.
+// 27.6 and 15.1, 500 x 1024 x 4096 48 and 32, 300 x 1024 x 1024 14.5 and 13.3.  A cut has to save 0.3 us by these costs (700 x 2048 x 4096 saves 0.4 by them, 28.2 and 24.5;
+// 32-bit 70 x 4112 x 1024 less, 14.4 and 15.5), and 1 us past 1024 rows, where little is left to gain and a prompt of any length keeps one sum per output: 1250 x 256 x 2048 10.2
+// and 9.3 is cut, 1501 x 256 x 2048 10.0 and 9.0 and 2048 x 256 x 2048 10.9 and 9.7 are not (weights from memory; where the caches hold them whole is the faster, 7.9 and 8.3).
 // Sums against 64 bits, whole and in parts: 5.7e-7 and 2.7e-7 (65 x 2048 x 8192), 4.0e-7 and 2.7e-7 (500 x 1024 x 4096), 32-bit 1.6e-7 and 1.0e-7 there.
 struct DenseTile {
     uint32_t bn, bm, lone, full;
@@ -22,7 +23,8 @@ struct DenseTile {
 constexpr DenseTile DENSE_TILES[] = {{64, 64, 16, 23}, {128, 64, 25, 38}, {128, 128, 43, 58}, {256, 128, 76, 100}, {256, 256, 114, 162}};
 constexpr uint32_t DENSE_PARTS[] = {2, 3, 4, 6, 8, 12};
 constexpr int DENSE_CUT_TILES = 3;                           // of these the first may be cut along k
-constexpr float DENSE_CUT_SAVES = 1700.0f;                   // ns at least: parts end in other roundings than a sum in one piece
+constexpr float DENSE_CUT_SAVES = 300.0f, DENSE_CUT_SAVES_TALL = 1000.0f;      // ns at least: parts end in other roundings than a sum in one piece
+constexpr uint32_t DENSE_TALL = 1024;                        // rows past which the larger saving is asked for
 
 struct DensePlan {
     int tile;
@@ -54,13 +56,13 @@ inline DensePlan dense_plan_tile(uint32_t n, uint32_t rows, uint32_t k, uint32_t
             if (ns < parted.ns) parted = {c, parts, ns};
         }
     }
-    return parted.ns + DENSE_CUT_SAVES <= whole.ns ? parted : whole;
+    return parted.ns + (rows > DENSE_TALL ? DENSE_CUT_SAVES_TALL : DENSE_CUT_SAVES) <= whole.ns ? parted : whole;
 }
 
 // The matrix's rows in one launch, or in two where that is shorter: a last round that few units take part in is left to
 // smaller tiles (8208 weight rows, 2048 tokens: one round of 256 x 256 and a sixteenth of one, 105 -> 76 us in all).
-// Neither is cut along k: all outputs of such a product are sums in one order, that of a product which fills the units (cut, those sixteen rows would save
-// 3 us of the 76, and end in other roundings than the rows beside them).
+// Past 1024 rows the second is not cut along k: all outputs of such a product are sums in one order (cut, those sixteen rows would save 3 us of the 76, and end in
+// other roundings than the rows beside them).
 struct DenseSplit {
     uint32_t first;                                          // rows of the first launch
     DensePlan head, tail;
@@ -76,7 +78,7 @@ inline DenseSplit dense_plan(uint32_t n, uint32_t rows, uint32_t k, uint32_t pla
         const uint32_t rounds = (uint32_t)((uint64_t)tn * tm / cus);
         const uint32_t cut = (uint32_t)((uint64_t)rounds * cus / tm) * DENSE_TILES[c].bn;
         if (cut == 0 || cut >= n) continue;
-        const DensePlan head = dense_plan_tile(cut, rows, k, planes, cus, count, false), tail = dense_plan_tile(n - cut, rows, k, planes, cus, count, false);
+        const DensePlan head = dense_plan_tile(cut, rows, k, planes, cus, count, false), tail = dense_plan_tile(n - cut, rows, k, planes, cus, count, split && rows <= DENSE_TALL);
         if (head.ns + tail.ns < best.ns) best = {cut, head, tail, head.ns + tail.ns};
     }
     return best;

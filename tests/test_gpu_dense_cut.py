@@ -8,10 +8,10 @@ from test_gpu_dense_tiles import KINDS, check, epilogue, operands
 pytestmark = pytest.mark.gpu
 
 
-# Tiles of 64 x 64, 128 x 64 and 128 x 128 in 2 .. 12 parts (test_rules.py says which) and the last size in one; 37, 67 and 129 steps of 64 k leave parts of unequal
+# Tiles of 64 x 64, 128 x 64 and 128 x 128 in 2 .. 12 parts (test_rules.py says which; the last but one in its second launch) and the last size in one; 37, 67 and 129 steps of 64 k leave parts of unequal
 # length; one weight row and one token past a tile.  Sums as in the uncut form or of more, shorter chains: below 1e-6 of the largest value at these k (2^-24
 # sqrt(k / 16 + 16) of a part), the bound is twice that, and 1e-6 for a GELU or SiLU by hardware exponentials.
-SHAPES = [(65, 66, 2368), (129, 250, 4288), (300, 2048, 4288), (700, 2048, 4096), (400, 1000, 8192), (1200, 1000, 8256), (500, 1024, 4096), (70, 66, 16384), (65, 64, 128)]
+SHAPES = [(65, 66, 2368), (129, 250, 4288), (300, 2048, 4288), (700, 2048, 4096), (400, 1000, 8192), (1200, 1000, 8256), (500, 1024, 4096), (70, 66, 16384), (700, 11264, 2048), (65, 64, 128)]
 
 
 @pytest.mark.parametrize("act", ["bf16", "fp32"])
