@@ -543,7 +543,7 @@ __global__ __launch_bounds__(skinny_threads(TT, NW, V)) void dense_skinny_kernel
 //   Which products, and in which order, is a matter of power.  From registers alone, random values, all units: 32 x 32 x 16 1,750 TFLOP/s,
 // 16 x 16 x 32 with the first operand held for runs and the second going to and fro 2,070, in any order that changes the first each time 1,570 to 1,750.
 // With 32 x 32 x 16 these kernels also left the clock of whatever ran next 13 % lower (a router product of 58 us took 66 beside them; 59 now).
-// 2048 x 2048 x 2048 22.5 -> 19.9 us, 4096 x 12,288 x 2048 in the tiles of 256 x 256 below 176 -> 160.
+// Cold weights, one call after another: 2048 x 2048 x 2048 23.7 -> 22.8 us, in the tiles of 256 x 256 below 4096 x 12,288 x 2048 179 -> 170 and 8192 x 8192 x 8192 769 -> 718.
 //   A stage is multiplied in four phases, half of the weight rows by 32 k each.  The operands of the phases after the next one are read, and a quarter of a
 // stage ahead is requested, between the products of a phase: a wave alone on its SIMD has products to issue at all times, and
 // requests spread over the phases keep the wave from waiting at the memory pipe (in one burst behind the barrier: 96 us for
@@ -870,7 +870,7 @@ __global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_ker
 // last two products of the stage before run and the halves 1 during the first two; a half is then out of LDS for registers (128 of them hold a
 // stage) one to one and a half stages before its successor is needed.  Barriers stand behind the first eight of the 32 matrix instructions of
 // a product: the reads before them arrive in the meantime.  Requests go out evenly over the stage.  Bound by the rate of requests into LDS and the
-// power of the products.  Rows x n x k, cold weights, with 32 x 32 x 16 products: 4096 x 12,288 x 2048 176 -> 160 us (1,290 TFLOP/s).
+// power of the products.  Rows x n x k, cold weights, 32 x 32 x 16 products and these: 4096 x 12,288 x 2048 179 and 170 us (1,210 TFLOP/s).
 // Not kept: a third place for the halves 0 (no change), requests of 64 bytes per row in stages of 32 k (half
 // the rate).
 template <int EPI>
