@@ -319,8 +319,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_prefill_fa_kern
     }
 
     // ---- finish: d over the four quarters, O / d, rows out through LDS in 16-byte pieces
-    d_run += shfl_xor_f(d_run, 16);
-    d_run += shfl_xor_f(d_run, 32);
+    d_run = add_xor<16>(d_run);
+    d_run = add_xor<32>(d_run);
     if (r == 0) bc[i] = d_run;
     __builtin_amdgcn_wave_barrier();
     const float4 d4 = *reinterpret_cast<const float4*>(bc + 4 * r);

@@ -118,13 +118,17 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
+// Lanes without a source read 0, which changes no maximum of unsigned numbers: so one instruction per step (a lane that kept its own value would cost four, with the
+// wait between them), and no row masks: the last lane still sees every row.
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-    v = max(v, (uint32_t)dpp_keep<0xB1, 0xF>((int)v));
-    v = max(v, (uint32_t)dpp_keep<0x4E, 0xF>((int)v));
-    v = max(v, (uint32_t)dpp_keep<0x141, 0xF>((int)v));
-    v = max(v, (uint32_t)dpp_keep<0x140, 0xF>((int)v));
-    v = max(v, (uint32_t)dpp_keep<0x142, 0xA>((int)v));
-    v = max(v, (uint32_t)dpp_keep<0x143, 0xC>((int)v));
+#define NVMAI_STEP(CTRL) v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true))
+    NVMAI_STEP(0xB1);            // quad_perm [1,0,3,2]
+    NVMAI_STEP(0x4E);            // quad_perm [2,3,0,1]
+    NVMAI_STEP(0x141);           // row_half_mirror
+    NVMAI_STEP(0x140);           // row_mirror
+    NVMAI_STEP(0x142);           // row_bcast15
+    NVMAI_STEP(0x143);           // row_bcast31
+#undef NVMAI_STEP
     return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
@@ -150,6 +154,34 @@ __device__ __forceinline__ float shfl_xor_f(float v, int mask) {
 __device__ __forceinline__ uint32_t shfl_xor_u(uint32_t v, int mask) {
     return (uint32_t)__shfl_xor((int)v, mask, 64);
 }
+
+// f(v, its value in the lane whose number differs in bit M): the step of a butterfly, on the vector pipe (through LDS, as __shfl_xor goes, a step is a trip of
+// some 120 cycles).  f has to be symmetric: for M of 16 and 32 half of the lanes see its arguments exchanged.
+template <int M, typename F>
+__device__ __forceinline__ float with_xor(float v, const F& f) {
+    static_assert(M == 1 || M == 2 || M == 4 || M == 8 || M == 16 || M == 32, "one bit");
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (M == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        return f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    } else if constexpr (M == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        return f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    } else if constexpr (M == 8) {
+        return f(v, dpp_mov<0x128, 0xF>(v));                           // row_ror 8
+    } else if constexpr (M == 4) {
+        return f(v, dpp_mov<0x1B, 0xF>(dpp_mov<0x141, 0xF>(v)));       // 7 - i, then 3 - i
+    } else {
+        return f(v, dpp_mov<M == 2 ? 0x4E : 0xB1, 0xF>(v));
+    }
+#else
+    return v;
+#endif
+}
+template <int M>
+__device__ __forceinline__ float add_xor(float v) { return with_xor<M>(v, [](float a, float b) { return __fadd_rn(a, b); }); }
+template <int M>
+__device__ __forceinline__ float max_xor(float v) { return with_xor<M>(v, [](float a, float b) { return fmaxf(a, b); }); }
 
 // ---- packed codes -----------------------------------------------------------
 // 4 codes of one dword at 8 bits -> floats, element order = byte order.
@@ -200,9 +232,7 @@ __device__ __forceinline__ void unpack4(uint32_t w, float* q) {
 // Sum of squares in a stated order: lane l runs acc = fma(x, x, acc) over the elements l, l + 64,
 // ..., then this xor butterfly 32, 16, 8, 4, 2, 1; mean, sqrt and the divide are single IEEE steps.
 __device__ __forceinline__ float rms_wave_sum(float acc) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) acc = __fadd_rn(acc, shfl_xor_f(acc, off));
-    return acc;
+    return add_xor<1>(add_xor<2>(add_xor<4>(add_xor<8>(add_xor<16>(add_xor<32>(acc))))));
 }
 
 __device__ __forceinline__ float rms_inverse(float sum, uint32_t d, float eps) {

@@ -59,8 +59,8 @@ __device__ __forceinline__ void flash32_block(uint32_t tiles, float* shared, Que
             for (int j = 0; j < 4; ++j) s[j] = sees(t, j, i) ? s[j] : 2.0f * FLASH32_NONE;
         }
         float tm = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
-        tm = fmaxf(tm, shfl_xor_f(tm, 16));
-        tm = fmaxf(tm, shfl_xor_f(tm, 32));
+        tm = max_xor<16>(tm);
+        tm = max_xor<32>(tm);
         if (__any(tm > m)) {
             const float mn = fmaxf(m, tm), alpha = __builtin_amdgcn_exp2f(m - mn);
             m = mn;
@@ -102,8 +102,8 @@ __device__ __forceinline__ void flash32_block(uint32_t tiles, float* shared, Que
 #pragma unroll
             for (int n = 0; n < NV; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(value(n, j), s[j], acc[n], 0, 0, 0);
     }
-    l += shfl_xor_f(l, 16);
-    l += shfl_xor_f(l, 32);
+    l = add_xor<16>(l);
+    l = add_xor<32>(l);
     float* ml = shared + NV * 1024;
     if (g == 0) {
         ml[wave * 32u + i] = m;

@@ -372,8 +372,8 @@ __global__ __launch_bounds__(256, 1) void latent_partial_mfma_kernel(LatentAttnP
         float tm = s[0];
 #pragma unroll
         for (int e = 1; e < 8; ++e) tm = fmaxf(tm, s[e]);
-        tm = fmaxf(tm, shfl_xor_f(tm, 16));
-        tm = fmaxf(tm, shfl_xor_f(tm, 32));
+        tm = max_xor<16>(tm);
+        tm = max_xor<32>(tm);
         const float mn = fmaxf(m, tm), alpha = __builtin_amdgcn_exp2f(m - mn);
         m = mn;
         float ts = 0.0f;
@@ -385,8 +385,8 @@ __global__ __launch_bounds__(256, 1) void latent_partial_mfma_kernel(LatentAttnP
             ph[j8] = f32_to_bf16(e);
             pl[j8] = f32_to_bf16(e - bf16_to_f32(ph[j8]));
         }
-        ts += shfl_xor_f(ts, 16);
-        ts += shfl_xor_f(ts, 32);
+        ts = add_xor<16>(ts);
+        ts = add_xor<32>(ts);
         l = fmaf(l, alpha, ts);
         uint4 bh, bl;
         bh.x = ph[0] | ((uint32_t)ph[1] << 16); bh.y = ph[2] | ((uint32_t)ph[3] << 16);
@@ -813,8 +813,8 @@ __device__ __forceinline__ void latent_flash_body(const LatentAttnParams& p) {
             float tm = fmaxf(fmaxf(s[b][0][0], s[b][0][1]), fmaxf(s[b][0][2], s[b][0][3]));
 #pragma unroll
             for (int t = 1; t < 4; ++t) tm = fmaxf(fmaxf(fmaxf(s[b][t][0], s[b][t][1]), fmaxf(s[b][t][2], s[b][t][3])), tm);
-            tm = fmaxf(tm, shfl_xor_f(tm, 16));
-            tm = fmaxf(tm, shfl_xor_f(tm, 32));
+            tm = max_xor<16>(tm);
+            tm = max_xor<32>(tm);
             if (__any(tm > m[b])) {
                 const float mn = fmaxf(m[b], tm), alpha = __builtin_amdgcn_exp2f(m[b] - mn);
                 m[b] = mn;
@@ -881,8 +881,8 @@ __device__ __forceinline__ void latent_flash_body(const LatentAttnParams& p) {
 #pragma unroll
     for (int b = 0; b < QB; ++b) {
         float sum = l[b];
-        sum += shfl_xor_f(sum, 16);
-        sum += shfl_xor_f(sum, 32);
+        sum = add_xor<16>(sum);
+        sum = add_xor<32>(sum);
         const uint32_t t = wt0 + 16u * b + i;
         if (t >= p.n_rows) continue;
         const float gate = p.gate ? la_sigmoid(bf16_to_f32(static_cast<const uint16_t*>(p.gate)[(size_t)t * p.gate_stride + head])) : 1.0f;

@@ -794,12 +794,25 @@ __device__ __forceinline__ void router_row_prefetch(const RouterParams& p, const
     }
 }
 
-template <int ACT, int KIND, int CPL>
-__device__ __forceinline__ void router_row_dots(const RouterParams& p, const RouterRowRegs<CPL>& g,
+template <int ACT, int KIND, int CPL, int HELD>
+__device__ __forceinline__ void router_row_dots(const RouterParams& p, const RouterRowRegs<HELD>& g,
                                                 const uint16_t* xl, uint32_t nt, int hl, float* acc) {
     constexpr int EPC = KIND == 16 ? 8 : (KIND == 8 ? 16 : 32);
     constexpr int XV = EPC / 8;
     const uint32_t chunks = p.d / EPC;
+    // the lane's inputs, where they are up to eight pieces all requested before the first is used (a trip to LDS per chunk is as long as the rest)
+    static_assert(ROUTER_TOK == 1, "one token's inputs");
+    constexpr bool AHEAD = CPL * XV <= 8;
+    uint4 mine[AHEAD ? CPL : 1][XV];
+    if constexpr (AHEAD) {
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) {
+            const uint32_t c = hl + 32 * i;
+            if (c >= chunks) break;
+#pragma unroll
+            for (int v = 0; v < XV; ++v) mine[i][v] = *reinterpret_cast<const uint4*>(xl + c * EPC + 8 * v);
+        }
+    }
 #pragma unroll
     for (int t = 0; t < ROUTER_TOK; ++t) acc[t] = 0.0f;
 #pragma unroll
@@ -817,10 +830,11 @@ __device__ __forceinline__ void router_row_dots(const RouterParams& p, const Rou
         for (int t = 0; t < ROUTER_TOK; ++t) {
             if ((uint32_t)t >= nt) break;
             float xv[EPC];
-            uint4 xraw[XV];
+            if constexpr (!AHEAD) {
 #pragma unroll
-            for (int v = 0; v < XV; ++v) xraw[v] = *reinterpret_cast<const uint4*>(xl + (size_t)t * p.d + c * EPC + 8 * v);
-            router_x_from_raw<ACT, EPC>(p, xraw, c * EPC, xv);
+                for (int v = 0; v < XV; ++v) mine[0][v] = *reinterpret_cast<const uint4*>(xl + c * EPC + 8 * v);
+            }
+            router_x_from_raw<ACT, EPC>(p, mine[AHEAD ? i : 0], c * EPC, xv);
             if (KIND == 16) {
 #pragma unroll
                 for (int j = 0; j < EPC; ++j) acc[t] = fmaf(q[j], xv[j], acc[t]);
@@ -837,17 +851,18 @@ __device__ __forceinline__ void router_row_dots(const RouterParams& p, const Rou
         }
     }
 #pragma unroll
-    for (int t = 0; t < ROUTER_TOK; ++t)
-#pragma unroll
-        for (int off = 16; off >= 1; off >>= 1) acc[t] = __fadd_rn(acc[t], shfl_xor_f(acc[t], off));
+    for (int t = 0; t < ROUTER_TOK; ++t) acc[t] = add_xor<1>(add_xor<2>(add_xor<4>(add_xor<8>(add_xor<16>(acc[t])))));
 }
 
-template <int ACT, int CPL>
+// MOST: the largest d that the caller takes, which bounds the chunks of a lane by their kind.
+template <int ACT, int CPL, int MOST = 65536>
 __device__ __forceinline__ void router_row_any(const RouterParams& p, int kind, const RouterRowRegs<CPL>& g,
                                                const uint16_t* xl, uint32_t nt, int hl, float* acc) {
-    if (kind == 16) router_row_dots<ACT, 16, CPL>(p, g, xl, nt, hl, acc);
-    else if (kind == 8) router_row_dots<ACT, 8, CPL>(p, g, xl, nt, hl, acc);
-    else router_row_dots<ACT, 4, CPL>(p, g, xl, nt, hl, acc);
+    constexpr int C16 = MOST / 8 / 32 < CPL ? MOST / 8 / 32 : CPL, C8 = MOST / 16 / 32 < CPL ? MOST / 16 / 32 : CPL,
+                  C4 = MOST / 32 / 32 < CPL ? MOST / 32 / 32 : CPL;
+    if (kind == 16) router_row_dots<ACT, 16, C16>(p, g, xl, nt, hl, acc);
+    else if (kind == 8) router_row_dots<ACT, 8, C8>(p, g, xl, nt, hl, acc);
+    else router_row_dots<ACT, 4, C4>(p, g, xl, nt, hl, acc);
 }
 
 // Largest chunk count per lane over the router and gate rows must be <= CPL.
@@ -1242,52 +1257,66 @@ __device__ __forceinline__ void select_topk_pairs(const SelectParams& p, const f
     }
 }
 
-// Selection for token t by one wave: lane r < top_k ends with the r-th best (score, index).  PER: scores per lane.
-// A round is one maximum over the wave of unsigned images that order like the scores (0: taken, or past the last expert), and a
-// compare per score that finds the lowest index that has it: about thirty vector instructions at 256 experts, where a compare of (score, index)
-// pairs within the lanes and two reductions were a hundred (one token, 4 bits: the launch that selects for itself 8.7 -> 7.1 us).  Rows with a NaN go the
-// other way, in which it hides what stands behind it in its lane.
+// Selection by one wave from scores in registers: val[j] of a lane is expert PER * lane + j's (any value past the last expert).  Lane r < rounds (top_k, or fewer) ends with the r-th best (score, index).
+// A round is one maximum over the wave of unsigned images that order like the scores (0: taken, or past the last expert), and the lowest lane that has it: experts
+// lie in the lanes in their order, so that lane's first image that equals it is the lowest index that does.  One token, 4 bits, in the launch that holds the
+// block: 1.65 -> 0.6 us for eight of 256, where experts that lay 64 apart took a compare over the wave per score.  Rows with a NaN go the
+// other way, in which it hides what stands behind it in its lane, experts 64 apart.
 template <int PER>
-__device__ __forceinline__ void select_topk_core(const SelectParams& p, uint32_t t, int lane, float& my_score,
-                                                 uint32_t& my_idx) {
-    float val[PER];
+__device__ __forceinline__ void select_topk_values(const SelectParams& p, const float (&val)[PER], int lane, float& my_score,
+                                                   uint32_t& my_idx, uint32_t rounds) {
     bool none = false;
 #pragma unroll
-    for (int j = 0; j < PER; ++j) {
-        const uint32_t e = lane + 64 * j;
-        val[j] = p.logits[(size_t)t * p.num_experts + min(e, p.num_experts - 1u)];
-    }
-#pragma unroll
-    for (int j = 0; j < PER; ++j) none |= (uint32_t)(lane + 64 * j) < p.num_experts && val[j] != val[j];
+    for (int j = 0; j < PER; ++j) none |= (uint32_t)(PER * lane + j) < p.num_experts && val[j] != val[j];
     my_score = 0.0f;
     my_idx = 0;
     if (__any(none)) {
-        select_topk_pairs<PER>(p, val, lane, my_score, my_idx);
+        float apart[PER];
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            apart[j] = 0.0f;
+#pragma unroll
+            for (int i = 0; i < PER; ++i) {
+                const float v = __shfl(val[i], (lane + 64 * j) / PER, 64);
+                apart[j] = (lane + 64 * j) % PER == i ? v : apart[j];
+            }
+        }
+        select_topk_pairs<PER>(p, apart, lane, my_score, my_idx);
         return;
     }
     uint32_t key[PER], mine = 0;
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
         const uint32_t u = __float_as_uint(val[j] + 0.0f);             // -0 and 0 are equal
-        key[j] = (uint32_t)(lane + 64 * j) < p.num_experts ? u ^ ((uint32_t)((int)u >> 31) | 0x80000000u) : 0u;
+        key[j] = (uint32_t)(PER * lane + j) < p.num_experts ? u ^ ((uint32_t)((int)u >> 31) | 0x80000000u) : 0u;
     }
-    for (uint32_t round = 0; round < p.top_k; ++round) {
+    for (uint32_t round = 0; round < rounds; ++round) {
         uint32_t most = key[0];
 #pragma unroll
         for (int j = 1; j < PER; ++j) most = max(most, key[j]);
-        most = wave_max_u32(most);
-        uint32_t best = 0;                                             // where no candidate is left: expert 0, -inf
+        uint32_t at = PER - 1;
 #pragma unroll
-        for (int j = PER - 1; j >= 0; --j) {
-            const uint64_t has = __ballot(key[j] == most);
-            best = has ? 64u * j + (uint32_t)__builtin_ctzll(has) : best;
-        }
-        best = most ? best : 0u;
+        for (int j = PER - 2; j >= 0; --j) at = key[j] == most ? (uint32_t)j : at;
+        const uint32_t top = wave_max_u32(most);
+        const int first = __builtin_ctzll(__ballot(most == top));      // some lane has it; where no candidate is left: expert 0, -inf
+        const uint32_t best = (uint32_t)__builtin_amdgcn_readlane((int)(PER * lane + at), first);
+        at = lane == first ? at : (uint32_t)PER;
 #pragma unroll
-        for (int j = 0; j < PER; ++j) key[j] = (uint32_t)(lane + 64 * j) == best ? 0u : key[j];
-        if ((uint32_t)lane == round) { mine = most; my_idx = best; }
+        for (int j = 0; j < PER; ++j) key[j] = at == (uint32_t)j ? 0u : key[j];
+        mine = (uint32_t)lane == round ? top : mine;
+        my_idx = (uint32_t)lane == round ? best : my_idx;
     }
     if ((uint32_t)lane < p.top_k) my_score = mine ? __uint_as_float(mine ^ ((uint32_t)((int)~mine >> 31) | 0x80000000u)) : -INFINITY;
+}
+
+// Selection for token t.  PER: scores per lane.
+template <int PER>
+__device__ __forceinline__ void select_topk_core(const SelectParams& p, uint32_t t, int lane, float& my_score,
+                                                 uint32_t& my_idx) {
+    float val[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) val[j] = p.logits[(size_t)t * p.num_experts + min((uint32_t)(PER * lane + j), p.num_experts - 1u)];
+    select_topk_values<PER>(p, val, lane, my_score, my_idx, p.top_k);
 }
 
 __device__ __forceinline__ void select_topk_core(const SelectParams& p, uint32_t t, int lane, float& my_score,
@@ -1298,17 +1327,21 @@ __device__ __forceinline__ void select_topk_core(const SelectParams& p, uint32_t
 
 // Softmax over the selected scores (in the lanes below top_k) times the expert's gain; stores
 // index and fp16 weight of token t.
-__device__ __forceinline__ void select_store_routes(const SelectParams& p, uint32_t t, int lane, float my_score,
-                                                    uint32_t my_idx) {
+__device__ __forceinline__ uint16_t select_weight(const SelectParams& p, int lane, float my_score, uint32_t my_idx) {
     const float max_s = readlane_f(my_score, 0);
     const float ex = expf(my_score - max_s);
     float sum = 0.0f;
     for (uint32_t i = 0; i < p.top_k; ++i) sum = __fadd_rn(sum, readlane_f(ex, (int)i));
+    const float gain = p.per_expert_scale && (uint32_t)lane < p.top_k ? bf16_to_f32(p.per_expert_scale[my_idx]) : 1.0f;
+    return f32_to_f16(__fmul_rn(__fdiv_rn(ex, sum), gain));
+}
+
+__device__ __forceinline__ void select_store_routes(const SelectParams& p, uint32_t t, int lane, float my_score,
+                                                    uint32_t my_idx) {
+    const uint16_t w = select_weight(p, lane, my_score, my_idx);
     if ((uint32_t)lane < p.top_k) {
-        const float gain = p.per_expert_scale ? bf16_to_f32(p.per_expert_scale[my_idx]) : 1.0f;
-        const float w = __fmul_rn(__fdiv_rn(ex, sum), gain);
         p.out_idx[(size_t)t * p.top_k + lane] = my_idx;
-        p.out_w[(size_t)t * p.top_k + lane] = f32_to_f16(w);
+        p.out_w[(size_t)t * p.top_k + lane] = w;
     }
 }
 
@@ -1747,6 +1780,43 @@ struct DownCombineParams {
     void* y;
 };
 
+// 64 / SEG rows of one slot: their codes against the activations a[] of the lane's chunk and their sum xs; the sum of a row, in the lanes seg_result_lane names.
+template <int BITS, int SEG>
+__device__ __forceinline__ float down_rows(const uint4& q, uint16_t sc, uint16_t bi, const float (&a)[Chunk<BITS>::elems], float xs) {
+    constexpr int EPC = Chunk<BITS>::elems;
+    float qf[EPC];
+    unpack_chunk<BITS>(q, qf);
+    float dot = 0.0f;
+#pragma unroll
+    for (int e = 0; e < EPC; ++e) dot = fmaf(qf[e], a[e], dot);
+    return seg_reduce_sum<SEG>(fmaf(bf16_to_f32(sc), dot, bf16_to_f32(bi) * xs));
+}
+
+// The weighted sum over the slots, by one wave: lanes below DC_ROWS own an output row each, all 64 serve the lane reads.  Every slot's part is requested before the
+// first is added.
+template <int ACT>
+__device__ __forceinline__ void down_store(const DownCombineParams& p, uint32_t t, uint32_t row0, int lane, const float (*part)[DC_ROWS],
+                                           float wk, float gate, float res) {
+    constexpr uint32_t SLOTS = 4 * DC_SLOTS_PER_WAVE;
+    const uint32_t r = lane < DC_ROWS ? lane : 0, last = p.top_k + (p.has_shared ? 1u : 0u) - 1u;
+    float v[SLOTS];
+#pragma unroll
+    for (uint32_t k = 0; k < SLOTS; ++k) v[k] = part[min(k, last)][r];
+    float acc = res;
+    if (p.has_shared) {
+        float s = part[last][r];
+        if (p.gate_logit) s = __fdiv_rn(s, __fadd_rn(1.0f, expf(-gate)));
+        acc = __fadd_rn(acc, s);
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < SLOTS; ++k) {
+        if (k >= p.top_k) break;
+        acc = __fadd_rn(acc, __fmul_rn(readlane_f(wk, (int)k), v[k]));
+    }
+    if (lane < DC_ROWS && row0 + r < p.rows)
+        ((uint16_t*)p.y)[(size_t)t * p.y_stride + row0 + r] = f32_to_act<ACT>(acc);
+}
+
 // (Handing a slot's activation row to the lanes through LDS -- one fetch per wave instead of one
 // per row of a load instruction -- was measured slower: 12 us against 9.6 us per launch at one
 // token; the step is a chain of latencies, and the LDS round trip lengthens it.)
@@ -1798,36 +1868,17 @@ __global__ __launch_bounds__(256) void down_combine_kernel(DownCombineParams p) 
     for (int j = 0; j < DC_SLOTS_PER_WAVE; ++j) {
         const uint32_t slot = wave + 4 * j;
         if (slot >= n_slots) break;
-        const float* aj = a[j];
         float xs = 0.0f;
 #pragma unroll
-        for (int e = 0; e < EPC; ++e) xs += aj[e];
+        for (int e = 0; e < EPC; ++e) xs += a[j][e];
 #pragma unroll
         for (int i = 0; i < PASSES; ++i) {
-            float qf[EPC];
-            unpack_chunk<BITS>(q[j][i], qf);
-            float dot = 0.0f;
-#pragma unroll
-            for (int e = 0; e < EPC; ++e) dot = fmaf(qf[e], aj[e], dot);
-            float acc = fmaf(bf16_to_f32(sc[j][i]), dot, bf16_to_f32(bi[j][i]) * xs);
-            acc = seg_reduce_sum<SEG>(acc);
+            const float acc = down_rows<BITS, SEG>(q[j][i], sc[j][i], bi[j][i], a[j], xs);
             if (seg_result_lane<SEG>(lane)) part[slot][i * RPL + seg_id] = acc;
         }
     }
     __syncthreads();
-    if (wave == 0) {              // lanes below DC_ROWS own an output row each; all 64 serve the lane reads
-        const uint32_t r = lane < DC_ROWS ? lane : 0;
-        float acc = res;
-        if (p.has_shared) {
-            float s = part[p.top_k][r];
-            if (p.gate_logit) s = __fdiv_rn(s, __fadd_rn(1.0f, expf(-gate)));
-            acc = __fadd_rn(acc, s);
-        }
-        for (uint32_t k = 0; k < p.top_k; ++k)
-            acc = __fadd_rn(acc, __fmul_rn(readlane_f(wk, (int)k), part[k][r]));
-        if (lane < DC_ROWS && row0 + r < p.rows)
-            ((uint16_t*)p.y)[(size_t)t * p.y_stride + row0 + r] = f32_to_act<ACT>(acc);
-    }
+    if (wave == 0) down_store<ACT>(p, t, row0, lane, part, wk, gate, res);
 }
 
 // fp32 rows [tokens, m] -> the caller's rows with its own stride: 16-bit activations (y) and /

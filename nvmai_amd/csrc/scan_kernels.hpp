@@ -185,9 +185,9 @@ __global__ __launch_bounds__(256) void scan_recurrent_kernel(ScanParams p, uint3
         }
 #pragma unroll
         for (int u = 0; u < CP; ++u) {
-            sq[u] += shfl_xor_f(sq[u], 16);
-            sq[u] += shfl_xor_f(sq[u], 32);
-            if (DELTA) { sk[u] += shfl_xor_f(sk[u], 16); sk[u] += shfl_xor_f(sk[u], 32); }
+            sq[u] = add_xor<16>(sq[u]);
+            sq[u] = add_xor<32>(sq[u]);
+            if (DELTA) { sk[u] = add_xor<16>(sk[u]); sk[u] = add_xor<32>(sk[u]); }
             if (lane < 16u) { part[0][wave][CP * j + u] = sq[u]; if (DELTA) part[1][wave][CP * j + u] = sk[u]; }
         }
         const float sum_qk = (red[2][0] + red[2][1]) + (red[2][2] + red[2][3]);

@@ -246,8 +246,8 @@ __global__ __launch_bounds__(256) void window_split_kernel(WindowParams p) {
         float tm = s[0];
 #pragma unroll
         for (int e = 1; e < 8; ++e) tm = fmaxf(tm, s[e]);
-        tm = fmaxf(tm, shfl_xor_f(tm, 16));
-        tm = fmaxf(tm, shfl_xor_f(tm, 32));
+        tm = max_xor<16>(tm);
+        tm = max_xor<32>(tm);
         const float mn = fmaxf(m, tm), alpha = __builtin_amdgcn_exp2f(m - mn);
         m = mn;
         float ts = 0.0f, hi8[8], lo8[8];
@@ -258,8 +258,8 @@ __global__ __launch_bounds__(256) void window_split_kernel(WindowParams p) {
             hi8[e] = bf16_to_f32(f32_to_bf16(x));
             lo8[e] = x - hi8[e];
         }
-        ts += shfl_xor_f(ts, 16);
-        ts += shfl_xor_f(ts, 32);
+        ts = add_xor<16>(ts);
+        ts = add_xor<32>(ts);
         l = fmaf(l, alpha, ts);
         const uint4 bh = make_uint4(wa_pack2(hi8[0], hi8[1]), wa_pack2(hi8[2], hi8[3]), wa_pack2(hi8[4], hi8[5]), wa_pack2(hi8[6], hi8[7]));
         const uint4 bl = make_uint4(wa_pack2(lo8[0], lo8[1]), wa_pack2(lo8[2], lo8[3]), wa_pack2(lo8[4], lo8[5]), wa_pack2(lo8[6], lo8[7]));
@@ -611,8 +611,8 @@ __device__ __forceinline__ void window_flash_body(const WindowParams& p) {
             float tm = fmaxf(fmaxf(s[b][0][0], s[b][0][1]), fmaxf(s[b][0][2], s[b][0][3]));
 #pragma unroll
             for (int t = 1; t < 4; ++t) tm = fmaxf(fmaxf(fmaxf(s[b][t][0], s[b][t][1]), fmaxf(s[b][t][2], s[b][t][3])), tm);
-            tm = fmaxf(tm, shfl_xor_f(tm, 16));
-            tm = fmaxf(tm, shfl_xor_f(tm, 32));
+            tm = max_xor<16>(tm);
+            tm = max_xor<32>(tm);
             if (__any(tm > m[b])) {
                 const float mn = fmaxf(m[b], tm), alpha = __builtin_amdgcn_exp2f(m[b] - mn);
                 m[b] = mn;
@@ -678,8 +678,8 @@ __device__ __forceinline__ void window_flash_body(const WindowParams& p) {
 #pragma unroll
     for (int b = 0; b < QB; ++b) {
         float sum = l[b];
-        sum += shfl_xor_f(sum, 16);
-        sum += shfl_xor_f(sum, 32);
+        sum = add_xor<16>(sum);
+        sum = add_xor<32>(sum);
         const uint32_t t0 = wt0 + 16u * b + i;
         if (t0 >= p.n_rows) continue;
         const float gate = p.gate ? wa_sigmoid(p.gate[(size_t)t0 * p.gate_stride + head]) : 1.0f;
