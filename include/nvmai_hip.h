@@ -89,6 +89,9 @@ void nvmai_hip_ctx_destroy(nvmai_hip_ctx* ctx);
  * buffers allocated in init, Attention.swift:117-126, LogitOutput.swift:244-258), so that no
  * later call has to; nvmai_hip_ctx_workspace_bytes reports the current size. */
 int nvmai_hip_ctx_reserve(nvmai_hip_ctx* ctx, size_t bytes);
+/* How often a block of a launch that hands values from block to block looks for them before it makes
+ * them itself (the result is the same; 2^14 looks, about 15 ms, in a new context).  Of use to tests. */
+int nvmai_hip_ctx_wait_limit(nvmai_hip_ctx* ctx, uint32_t looks);
 size_t nvmai_hip_ctx_workspace_bytes(const nvmai_hip_ctx* ctx);
 const char* nvmai_hip_status_string(int status);
 

@@ -135,6 +135,7 @@ class ScanConfig(C.Structure):
 SIGNATURES = {
     "nvmai_hip_ctx_create": [C.c_int, C.c_int, C.POINTER(vp)],
     "nvmai_hip_ctx_reserve": [vp, C.c_size_t],
+    "nvmai_hip_ctx_wait_limit": [vp, u32],
     "nvmai_hip_profile_enable": [vp, C.c_int],
     "nvmai_hip_profile_read": [vp, C.c_int, C.POINTER(C.c_double), C.POINTER(u32)],
     "nvmai_hip_read_probe": [vp, vp, vp, u64, vp],

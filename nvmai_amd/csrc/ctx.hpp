@@ -7,8 +7,10 @@
 #include <vector>
 
 #include "../../include/nvmai_hip.h"
+#include "hand.hpp"
 
 struct nvmai_hip_ctx {
+    using Hand = nvmai::Hand;
     int device;
     int compute_units;       // of the device (persistent grids are sized from it)
     int act;                 // NVMAI_ACT_BF16 / NVMAI_ACT_FP16 / NVMAI_ACT_FP32
@@ -23,7 +25,8 @@ struct nvmai_hip_ctx {
     std::vector<void*> ws_retired;
     uint8_t* static_scratch; // device address of the library's static scratch array on this device (ctx_api.hip)
     uint32_t* tickets;       // zero-initialised device words for last-block-done kernels (TICKET_WORDS)
-    uint16_t* norm_rows;     // behind them: normed rows between the two launches of affine_gemv_prenorm (NORM_ROWS x NORM_WIDTH)
+    uint16_t* norm_rows;     // behind those words: normed rows between the two launches of affine_gemv_prenorm (NORM_ROWS x NORM_WIDTH)
+    Hand hand;               // behind the tickets: words handed from block to block inside a launch (hand.hpp)
     float* cut_sums;         // sums of blocks that share a tile (CUT_SUMS_BYTES), or nullptr: no tile is shared
     // Optional per-kernel timing: event pairs recorded around tagged launches.
     bool prof_on;

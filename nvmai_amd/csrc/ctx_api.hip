@@ -58,12 +58,14 @@ extern "C" int nvmai_hip_ctx_create(int device, int act_dtype, nvmai_hip_ctx** o
     ctx->ws_used = 0;
     ctx->prof_on = false;
     ctx->tickets = nullptr;
-    if (hipMalloc(reinterpret_cast<void**>(&ctx->tickets), TICKET_BYTES + NORM_BYTES) != hipSuccess ||
-        hipMemset(ctx->tickets, 0, TICKET_BYTES) != hipSuccess) {
+    if (hipMalloc(reinterpret_cast<void**>(&ctx->tickets), TICKET_BYTES + HAND_BYTES + NORM_BYTES) != hipSuccess ||
+        hipMemset(ctx->tickets, 0, TICKET_BYTES + HAND_BYTES) != hipSuccess) {
         delete ctx;
         return NVMAI_ERR_HIP;
     }
-    ctx->norm_rows = reinterpret_cast<uint16_t*>(ctx->tickets + TICKET_WORDS);
+    uint8_t* const words = reinterpret_cast<uint8_t*>(ctx->tickets) + TICKET_BYTES;
+    ctx->hand = Hand{reinterpret_cast<uint32_t*>(words), reinterpret_cast<uint64_t*>(words + HAND_BLOCKS * 4), 0, HAND_POLLS};
+    ctx->norm_rows = reinterpret_cast<uint16_t*>(words + HAND_BYTES);
     // allocated here and not by the call that first needs it, which may be captured; products are made without it too
     ctx->cut_sums = nullptr;
     if (hipMalloc(reinterpret_cast<void**>(&ctx->cut_sums), CUT_SUMS_BYTES) != hipSuccess) {
@@ -93,6 +95,12 @@ extern "C" int nvmai_hip_ctx_reserve(nvmai_hip_ctx* ctx, size_t bytes) {
     if (!ctx) return NVMAI_ERR_INVALID_ARG;
     NVMAI_HIP_TRY(hipSetDevice(ctx->device));
     return ws_begin(ctx, nullptr, bytes);
+}
+
+extern "C" int nvmai_hip_ctx_wait_limit(nvmai_hip_ctx* ctx, uint32_t looks) {
+    if (!ctx) return NVMAI_ERR_INVALID_ARG;
+    ctx->hand.polls = looks;
+    return NVMAI_OK;
 }
 
 extern "C" size_t nvmai_hip_ctx_workspace_bytes(const nvmai_hip_ctx* ctx) { return ctx ? ctx->ws_cap : 0; }

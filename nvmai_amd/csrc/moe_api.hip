@@ -5,6 +5,7 @@
 
 #include "ctx.hpp"
 #include "moe_kernels.hpp"
+#include "moe_one_kernels.hpp"
 #include "rules.hpp"
 
 using namespace nvmai;
@@ -406,6 +407,62 @@ void launch_down_combine(int act, uint32_t bits, const DownCombineParams& p, hip
         if (bits == 8) launch_down_combine_t<ACT_FP16, 8>(p, s);
         else launch_down_combine_t<ACT_FP16, 4>(p, s);
     }
+}
+
+// The same in one launch (moe_one_kernels.hpp), for one token.  False, having launched nothing, for shapes that have no such form: rows of gate and up that a wave reads
+// whole and whose inputs a block holds (d up to 2048), rows of the down projection of 16 or 32 pieces (64 would be held in more registers than the others leave), more blocks than one launch
+// numbers, an output that lies over what the launch reads.
+template <int ACT, int BITS, int NCH>
+bool launch_moe_one_t(const MoeOneParams& p, uint32_t blocks, hipStream_t s) {
+    const size_t rows_lds = moe_one_rows_lds(p.rows.n, NCH);
+    const uint32_t chunks = p.down.n * BITS / 128;
+#define NVMAI_ONE(SEG)                                                                               \
+    do {                                                                                             \
+        const size_t down_lds = moe_one_down_lds<BITS, SEG>(p.slots);                                \
+        const size_t lds = rows_lds > down_lds ? rows_lds : down_lds;                                \
+        if (lds > 60 * 1024) return false;                                                           \
+        moe_one_kernel<ACT, BITS, NCH, SEG><<<blocks, MOE_ONE_THREADS, lds, s>>>(p);                             \
+        return true;                                                                                 \
+    } while (0)
+    if (chunks == 16) NVMAI_ONE(16);
+    if (chunks == 32) NVMAI_ONE(32);
+#undef NVMAI_ONE
+    return false;
+}
+
+template <int ACT>
+bool launch_moe_one_act(uint32_t bits, const MoeOneParams& p, uint32_t blocks, hipStream_t s) {
+    if (p.rows.n * bits == 64 * 128) return bits == 8 ? launch_moe_one_t<ACT, 8, 1>(p, blocks, s) : launch_moe_one_t<ACT, 4, 1>(p, blocks, s);
+    if (p.rows.n * bits == 128 * 128 && bits == 8) return launch_moe_one_t<ACT, 8, 2>(p, blocks, s);
+    return false;
+}
+
+// Whether rows of `d` 16-bit values `stride` apart at a and at b have bytes in common.
+bool rows_overlap(const void* a, uint32_t a_stride, const void* b, uint32_t b_stride, uint32_t rows, uint32_t d) {
+    if (!a || !b) return false;
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    const uintptr_t nx = ((uintptr_t)(rows - 1) * a_stride + d) * 2, ny = ((uintptr_t)(rows - 1) * b_stride + d) * 2;
+    return x < y + ny && y < x + nx;
+}
+
+bool launch_moe_one(const nvmai_hip_ctx* ctx, uint32_t bits, MoeOneParams& p, hipStream_t s) {
+    const uint32_t T = p.sel.tokens, D = p.rows.n, F = p.rows.rows;
+    if (T != 1 || D > 2048 || D % 256 || F < 64) return false;
+    const RouterParams& r = p.router;
+    if ((rows_chunks(r.router.kind, D) + 31) / 32 > 8) return false;
+    const struct { const void* at; uint32_t stride; } outs[3] = {{p.down.y, p.down.y_stride}, {r.pre_hidden_out, r.pre_hidden_stride}, {r.pre_normed_out, r.pre_normed_stride}};
+    for (const auto& o : outs)
+        if (rows_overlap(o.at, o.stride, r.x, r.x_stride, T, D) || rows_overlap(o.at, o.stride, r.pre_delta, r.pre_delta_stride, T, D)) return false;
+    p.router_blocks = (r.num_experts + (r.gate.kind ? 1u : 0u) + MOE_ONE_LOGITS - 1) / MOE_ONE_LOGITS;
+    p.slots = p.sel.top_k + (p.down.has_shared ? 1u : 0u);
+    p.rows.blocks_per_entry = (F + MOE_ONE_ROWS - 1) / MOE_ONE_ROWS;
+    p.down_blocks = (D + DC_ROWS - 1) / DC_ROWS;
+    const uint64_t blocks = (uint64_t)T * (p.router_blocks + p.slots * p.rows.blocks_per_entry + 1 + p.down_blocks);
+    const uint64_t words = (uint64_t)T * moe_one_token_words(r.num_experts, p.slots, F);
+    if (blocks > HAND_BLOCKS || words > HAND_WORDS) return false;
+    p.hand = ctx->hand;
+    p.hand.used = (uint32_t)words;
+    return ctx->act == ACT_BF16 ? launch_moe_one_act<ACT_BF16>(bits, p, (uint32_t)blocks, s) : launch_moe_one_act<ACT_FP16>(bits, p, (uint32_t)blocks, s);
 }
 
 }  // namespace
@@ -1056,8 +1113,6 @@ int decode_layer_impl(nvmai_hip_ctx* ctx, nvmai_stream stream, const nvmai_moe_l
     GroupParams gp{sp, (uint32_t)maxtok, has_shared ? 1 : 0, entries, n_entries, stats, pair_token, pair_id,
                    ctx->tickets};
     if (fused_decode_ok(T, K, has_shared, D, F, L->bits)) {
-        { ProfScope ps(ctx, NVMAI_PROF_ROUTER, s); rc = run_router(ctx, rp, s); }
-        if (rc) return rc;
         RowsParams p{};
         p.src.pool_base = (const uint8_t*)L->experts_base;
         p.src.pool_stride = L->expert_stride;
@@ -1065,6 +1120,28 @@ int decode_layer_impl(nvmai_hip_ctx* ctx, nvmai_stream stream, const nvmai_moe_l
         set_phase1(p, L->offsets, D, F);
         p.x = x; p.x_stride = x_stride; p.out = acts; p.out_stride = F;
         const RoutedStats rs{stats, has_shared ? 1 : 0};
+        {
+            MoeOneParams one{};
+            one.router = rp;
+            one.router.x_vec = 1;
+            one.sel = sp;
+            one.rows = p;
+            if (pre) {
+                one.rows.x = rp.x; one.rows.x_stride = rp.x_stride;
+                one.rows.pre_delta = rp.pre_delta; one.rows.pre_delta_stride = rp.pre_delta_stride;
+                one.rows.pre_weight = rp.pre_weight; one.rows.pre_eps = rp.pre_eps;
+            }
+            one.down.src = p.src;
+            one.down.wA = L->offsets.down_w; one.down.sA = L->offsets.down_s; one.down.bA = L->offsets.down_b;
+            one.down.gate_logit = gated ? gate_logit : nullptr;
+            one.down.has_shared = has_shared ? 1 : 0; one.down.tokens = T; one.down.top_k = K; one.down.rows = D; one.down.n = F;
+            one.down.y_stride = y_stride; one.down.y = y;
+            one.stats = rs;
+            ProfScope ps(ctx, NVMAI_PROF_PHASE1, s);
+            if (launch_moe_one(ctx, L->bits, one, s)) return launch_status();
+        }
+        { ProfScope ps(ctx, NVMAI_PROF_ROUTER, s); rc = run_router(ctx, rp, s); }
+        if (rc) return rc;
         {
             ProfScope ps(ctx, NVMAI_PROF_PHASE1, s);
             launch_routed(ctx->act, L->bits, p, sp, rs, K + (has_shared ? 1u : 0u), s);
