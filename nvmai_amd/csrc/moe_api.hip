@@ -6,6 +6,7 @@
 #include "ctx.hpp"
 #include "moe_kernels.hpp"
 #include "moe_one_kernels.hpp"
+#include "router_group_kernels.hpp"
 #include "rules.hpp"
 
 using namespace nvmai;
@@ -445,14 +446,22 @@ bool rows_overlap(const void* a, uint32_t a_stride, const void* b, uint32_t b_st
     return x < y + ny && y < x + nx;
 }
 
+// Whether what a launch with the prologue stores lies over the rows that all of its blocks read.
+bool prologue_overlaps(const RouterParams& r) {
+    const struct { const void* at; uint32_t stride; } outs[2] = {{r.pre_hidden_out, r.pre_hidden_stride}, {r.pre_normed_out, r.pre_normed_stride}};
+    for (const auto& o : outs)
+        if (rows_overlap(o.at, o.stride, r.x, r.x_stride, r.tokens, r.d) || rows_overlap(o.at, o.stride, r.pre_delta, r.pre_delta_stride, r.tokens, r.d)) return true;
+    return false;
+}
+
 bool launch_moe_one(const nvmai_hip_ctx* ctx, uint32_t bits, MoeOneParams& p, hipStream_t s) {
     const uint32_t T = p.sel.tokens, D = p.rows.n, F = p.rows.rows;
     if (T != 1 || D > 2048 || D % 256 || F < 64) return false;
     const RouterParams& r = p.router;
     if ((rows_chunks(r.router.kind, D) + 31) / 32 > 8) return false;
-    const struct { const void* at; uint32_t stride; } outs[3] = {{p.down.y, p.down.y_stride}, {r.pre_hidden_out, r.pre_hidden_stride}, {r.pre_normed_out, r.pre_normed_stride}};
-    for (const auto& o : outs)
-        if (rows_overlap(o.at, o.stride, r.x, r.x_stride, T, D) || rows_overlap(o.at, o.stride, r.pre_delta, r.pre_delta_stride, T, D)) return false;
+    if (prologue_overlaps(r) || rows_overlap(p.down.y, p.down.y_stride, r.x, r.x_stride, T, D) ||
+        rows_overlap(p.down.y, p.down.y_stride, r.pre_delta, r.pre_delta_stride, T, D))
+        return false;
     p.router_blocks = (r.num_experts + (r.gate.kind ? 1u : 0u) + MOE_ONE_LOGITS - 1) / MOE_ONE_LOGITS;
     p.slots = p.sel.top_k + (p.down.has_shared ? 1u : 0u);
     p.rows.blocks_per_entry = (F + MOE_ONE_ROWS - 1) / MOE_ONE_ROWS;
@@ -463,6 +472,31 @@ bool launch_moe_one(const nvmai_hip_ctx* ctx, uint32_t bits, MoeOneParams& p, hi
     p.hand = ctx->hand;
     p.hand.used = (uint32_t)words;
     return ctx->act == ACT_BF16 ? launch_moe_one_act<ACT_BF16>(bits, p, (uint32_t)blocks, s) : launch_moe_one_act<ACT_FP16>(bits, p, (uint32_t)blocks, s);
+}
+
+// Router, selection and work list in one launch (router_group_kernels.hpp).  False, having launched nothing, for what has no such form: tokens
+// for the router's tiles, more blocks or words than one launch numbers, an output that lies over what the launch reads.
+template <int ACT>
+bool launch_router_group_act(const RouterGroupParams& p, uint32_t cpl, uint32_t blocks, size_t lds, hipStream_t s) {
+    if (cpl <= 2) router_group_kernel<ACT, 2><<<blocks, RG_THREADS, lds, s>>>(p);
+    else if (cpl <= 4) router_group_kernel<ACT, 4><<<blocks, RG_THREADS, lds, s>>>(p);
+    else router_group_kernel<ACT, 8><<<blocks, RG_THREADS, lds, s>>>(p);
+    return true;
+}
+
+bool launch_router_group(const nvmai_hip_ctx* ctx, const RouterParams& rp, const GroupParams& gp, hipStream_t s) {
+    const uint32_t T = rp.tokens, E = rp.num_experts, D = rp.d, pairs = T * gp.sel.top_k;
+    const uint32_t words = rg_words(T, E, gp.sel.top_k);
+    uint32_t chunks = rows_chunks(rp.router.kind, D);
+    if (rp.gate.kind && rows_chunks(rp.gate.kind, D) > chunks) chunks = rows_chunks(rp.gate.kind, D);
+    const uint32_t cpl = (chunks + 31) / 32;
+    RouterGroupParams p{rp, gp, ctx->hand, (E + (rp.gate.kind ? 1u : 0u) + RG_ROWS - 1) / RG_ROWS};
+    const uint32_t blocks = T * p.router_blocks + (T + RG_TOKENS - 1) / RG_TOKENS + 1;
+    const size_t row = (size_t)D * (rp.pre_weight ? 4 : 2) + 16, list = (4 * (size_t)E + 8 + 2 * (size_t)pairs) * 4, lds = row > list ? row : list;
+    if (T >= 64 || cpl > 8 || blocks > HAND_BLOCKS || words > HAND_WORDS || lds > 60 * 1024 || prologue_overlaps(rp)) return false;
+    p.router.x_vec = aligned16(rp.x) && rp.x_stride % 8 == 0;
+    p.hand.used = words;
+    return ctx->act == ACT_BF16 ? launch_router_group_act<ACT_BF16>(p, cpl, blocks, lds, s) : launch_router_group_act<ACT_FP16>(p, cpl, blocks, lds, s);
 }
 
 }  // namespace
@@ -1155,18 +1189,15 @@ int decode_layer_impl(nvmai_hip_ctx* ctx, nvmai_stream stream, const nvmai_moe_l
         { ProfScope ps(ctx, NVMAI_PROF_PHASE2, s); launch_down_combine(ctx->act, L->bits, dc, s); }
         return launch_status();
     }
-    // Two launches on purpose: one that also selects and groups in its last blocks needs a
-    // device-scope release (an L2 write-back on this multi-die part) from every one of its
-    // hundreds of producer blocks, and measured 18 us slower per step.
-    { ProfScope ps(ctx, NVMAI_PROF_ROUTER, s); rc = run_router(ctx, rp, s); }
-    if (rc) return rc;
+    bool routed;
     {
+        ProfScope ps(ctx, NVMAI_PROF_ROUTER, s);
+        routed = launch_router_group(ctx, rp, gp, s);
+        if (!routed && (rc = run_router(ctx, rp, s))) return rc;
+    }
+    if (!routed) {
         ProfScope ps(ctx, NVMAI_PROF_GROUP, s);
-        // a wave per token of one block (8 tokens 5.9 us, 16 7.2), or several blocks that meet at a ticket (7.4, 8.6; 24 tokens 9.3, 32 10.0 where
-        // one block takes 10.0 and 11.8: four selections on a SIMD are bound by their instructions)
-        const size_t one = (4 * E + 8 + 2 * (size_t)pairs) * 4;
-        if (T <= 16 && one <= 64 * 1024) select_group_one_block_kernel<<<1, 64 * (T < 4 ? 4 : T), one, s>>>(gp);
-        else select_group_kernel<<<(T + 3) / 4, 256, (4 * E + 8 + pairs) * 4, s>>>(gp);
+        select_group_kernel<<<(T + 3) / 4, 256, (4 * E + 8 + pairs) * 4, s>>>(gp);
     }
 
     RowsParams p{};

@@ -1380,7 +1380,12 @@ struct GroupParams {
     uint32_t* ticket;          // zero between launches; counts finished blocks
 };
 
-// The work list from every token's routed experts, idx[token * top_k + rank]; one block, after all indices are written.
+// The counters of build_work_list; a barrier stands between.
+__device__ __forceinline__ void clear_work_list(const GroupParams& p, uint32_t* lds) {
+    for (uint32_t i = threadIdx.x; i < 4 * p.sel.num_experts + 8; i += blockDim.x) lds[i] = 0;
+}
+
+// The work list from every token's routed experts, idx[token * top_k + rank]; one block, after all indices are written and the counters cleared.
 template <typename Idx>
 __device__ __forceinline__ void build_work_list(const GroupParams& p, uint32_t* lds, const Idx* idx) {
     const uint32_t tokens = p.sel.tokens, top_k = p.sel.top_k, E = p.sel.num_experts;
@@ -1392,8 +1397,6 @@ __device__ __forceinline__ void build_work_list(const GroupParams& p, uint32_t* 
     uint32_t* slotr = lds + 3 * E;        // [E] remainder entry of the expert inside its class
     uint32_t* misc = lds + 4 * E;         // [0] pair cursor, [1..4] entries per class, [5] distinct
     uint32_t* rank = lds + 4 * E + 8;     // [n_pairs] rank of the pair inside its expert
-    for (uint32_t i = tid; i < 4 * E + 8; i += blockDim.x) lds[i] = 0;
-    __syncthreads();
     for (uint32_t i = tid; i < n_pairs; i += blockDim.x) rank[i] = atomicAdd(&cnt[idx[i]], 1u);
     __syncthreads();
     const uint32_t tpe = p.tok_per_entry;
@@ -1455,21 +1458,9 @@ __global__ __launch_bounds__(256) void select_group_kernel(GroupParams p) {
     __syncthreads();
     if (lds[0] != gridDim.x - 1) return;  // uniform per block
     __syncthreads();
+    clear_work_list(p, lds);
+    __syncthreads();
     build_work_list(p, lds, const_cast<const volatile uint32_t*>(p.sel.out_idx));       // written by other blocks: read past L1
-}
-
-// The same in ONE block, a wave per token: nothing crosses a block, so the device-scope
-// release of the multi-block kernel (an L2 write-back on this multi-die part) and its ticket
-// are not needed, and the indices stay in LDS.
-__global__ __launch_bounds__(1024) void select_group_one_block_kernel(GroupParams p) {
-    extern __shared__ uint32_t lds[];
-    const uint32_t tokens = p.sel.tokens, top_k = p.sel.top_k, lane = threadIdx.x & 63u, waves = blockDim.x >> 6;
-    uint32_t* idx = lds + 4u * p.sel.num_experts + 8u + tokens * top_k;
-    for (uint32_t t = threadIdx.x >> 6; t < tokens; t += waves) {
-        const uint32_t mine = select_topk_wave(p.sel, t, (int)lane);
-        if (lane < top_k) idx[t * top_k + lane] = mine;
-    }
-    build_work_list(p, lds, idx);                    // its first barrier stands before the first index is read
 }
 
 // Dense work list: `count` inputs through the expert in slot `slot`.
