@@ -824,6 +824,19 @@ int nvmai_hip_rms_residual(nvmai_hip_ctx* ctx, nvmai_stream stream, float* x, ui
                            uint32_t delta_stride, const uint16_t* post_weight, float post_add, const uint16_t* next_weight,
                            float next_add, void* out, uint32_t out_stride, uint32_t rows, uint32_t d, float eps);
 
+/* The same with rows of 32-bit contexts as planes, [rows][3][k] BF16: three parts of every value that add up to it (see nvmai_hip_dense_linear), the smallest first.
+ * What nvmai_hip_dense_linear_ex makes of the rows in its workspace, for rows that only products read.  dense_linear_planes: x is planes (5 rows or more, 6 k rows
+ * at most 128 MB), either y or y_planes (of y_k values a row, n and y_k multiples of 4) is given.  The norms: out is planes of out_k values a row, the first d of them written.
+ * The same bits as the calls on rows of floats; NVMAI_ERR_UNSUPPORTED otherwise. */
+int nvmai_hip_dense_linear_planes(nvmai_hip_ctx* ctx, nvmai_stream stream, const uint16_t* w, uint32_t w_stride, const uint16_t* x, uint32_t rows, uint32_t n,
+                                  uint32_t k, float* y, uint32_t y_stride, uint16_t* y_planes, uint32_t y_k, const nvmai_linear_epilogue* epilogue);
+int nvmai_hip_norm_residual_planes(nvmai_hip_ctx* ctx, nvmai_stream stream, float* x, uint32_t x_stride, const float* delta, uint32_t delta_stride,
+                                   const uint16_t* post_weight, const uint16_t* post_bias, float mult, const uint16_t* next_weight, const uint16_t* next_bias,
+                                   uint16_t* out, uint32_t out_k, uint32_t rows, uint32_t d, float eps);
+int nvmai_hip_rms_residual_planes(nvmai_hip_ctx* ctx, nvmai_stream stream, float* x, uint32_t x_stride, const float* delta, uint32_t delta_stride,
+                                  const uint16_t* post_weight, float post_add, const uint16_t* next_weight, float next_add, uint16_t* out, uint32_t out_k,
+                                  uint32_t rows, uint32_t d, float eps);
+
 /* The end of a sublayer and the product that opens the next one, in 32-bit contexts, for one or two rows of at most 2048:
  *   x_out  = x + RMS(delta) * (post_add + post_weight)
  *   y      = the product of nvmai_hip_dense_linear_ex with x_out as its input

@@ -215,6 +215,9 @@ SIGNATURES = {
     "nvmai_hip_norm_residual": [vp, vp, vp, u32, vp, u32, vp, vp, C.c_float, vp, vp, vp, u32, u32, u32, C.c_float],
     "nvmai_hip_embed_rows": [vp, vp, vp, u32, vp, u32, vp, u32, u32, u32],
     "nvmai_hip_dense_linear_ex": [vp, vp, vp, u32, vp, u32, u32, u32, u32, vp, vp, u32, C.POINTER(LinearEpilogue)],
+    "nvmai_hip_dense_linear_planes": [vp, vp, vp, u32, vp, u32, u32, u32, vp, u32, vp, u32, C.POINTER(LinearEpilogue)],
+    "nvmai_hip_norm_residual_planes": [vp, vp, vp, u32, vp, u32, vp, vp, C.c_float, vp, vp, vp, u32, u32, u32, C.c_float],
+    "nvmai_hip_rms_residual_planes": [vp, vp, vp, u32, vp, u32, vp, C.c_float, vp, C.c_float, vp, u32, u32, u32, C.c_float],
     "nvmai_hip_rms_residual_linear": [vp, vp, vp, u32, vp, u32, vp, C.c_float, C.c_float, vp, u32, vp, u32, u32, u32, u32, vp, u32, C.POINTER(LinearEpilogue)],
     "nvmai_hip_rms_residual": [vp, vp, vp, u32, vp, u32, vp, C.c_float, vp, C.c_float, vp, u32, u32, u32, C.c_float],
     "nvmai_hip_embed_positions": [vp, vp, vp, u32, vp, u32, C.c_float, vp, C.POINTER(RowMap), vp, u32, vp, u32, u32, u32],

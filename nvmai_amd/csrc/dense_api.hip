@@ -9,18 +9,6 @@ using namespace nvmai;
 
 namespace nvmai {
 
-// A float as three BF16 values that add up to it exactly (8 + 8 + 8 bits of mantissa, by truncation; below 2^-110 the
-// last bits may be lost).  Infinities and NaN stay in the first one.
-__device__ __forceinline__ void dense_split3(float x, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
-    const uint32_t u = __float_as_uint(x);
-    const bool finite = (u & 0x7F800000u) != 0x7F800000u;
-    const float r1 = x - __uint_as_float(u & 0xFFFF0000u);
-    const float r2 = r1 - __uint_as_float(__float_as_uint(r1) & 0xFFFF0000u);
-    hi = (u >> 16) | (!finite && (u & 0x007FFFFFu) ? 0x40u : 0u);
-    mid = finite ? __float_as_uint(r1) >> 16 : 0u;
-    lo = finite ? __float_as_uint(r2) >> 16 : 0u;
-}
-
 // Rows of floats -> [row][3][k] BF16, the smallest part first.  Bound by its bytes (4 read, 6 written per value).
 __global__ __launch_bounds__(256) void dense_split_kernel(const float* x, uint32_t x_stride, uint32_t k, uint16_t* planes) {
     const uint32_t at = (blockIdx.x * 256u + threadIdx.x) * 8u, row = blockIdx.y;
@@ -31,8 +19,8 @@ __global__ __launch_bounds__(256) void dense_split_kernel(const float* x, uint32
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         uint32_t a[3], b[3];
-        dense_split3(f[2 * e], a[0], a[1], a[2]);
-        dense_split3(f[2 * e + 1], b[0], b[1], b[2]);
+        split3(f[2 * e], a[0], a[1], a[2]);
+        split3(f[2 * e + 1], b[0], b[1], b[2]);
 #pragma unroll
         for (int q = 0; q < 3; ++q) out[q][e] = a[q] | (b[q] << 16);
     }
@@ -122,6 +110,20 @@ extern "C" int nvmai_hip_dense_linear_ex(nvmai_hip_ctx* ctx, nvmai_stream stream
     const DenseLinearParams p{w, x, y, y_f32, w_stride, x_stride, y_stride, rows, n, k, e->activation, e->bias, e->mul, e->mul_ids,
                               e->mul_stride, e->mul_rows};
     return dense_linear_call(ctx, stream, p);
+}
+
+extern "C" int nvmai_hip_dense_linear_planes(nvmai_hip_ctx* ctx, nvmai_stream stream, const uint16_t* w, uint32_t w_stride, const uint16_t* x, uint32_t rows,
+                                             uint32_t n, uint32_t k, float* y, uint32_t y_stride, uint16_t* y_planes, uint32_t y_k,
+                                             const nvmai_linear_epilogue* e) {
+    if (!ctx || !e || (y == nullptr) == (y_planes == nullptr)) return NVMAI_ERR_INVALID_ARG;
+    if (ctx->act != NVMAI_ACT_FP32 || rows < 5 || !planes_fit(rows, k)) return NVMAI_ERR_UNSUPPORTED;
+    // planes are stored two or four values at a time
+    if (y_planes && (n % 4 || y_k % 4 || !planes_fit(rows, y_k))) return NVMAI_ERR_UNSUPPORTED;
+    if (y_planes && y_k < (e->activation == NVMAI_LINEAR_SILU_PAIRS ? n / 2 : n)) return NVMAI_ERR_INVALID_ARG;
+    DenseLinearParams p{w, x, y, nullptr, w_stride, 3 * k, y_stride, rows, n, k, e->activation, e->bias, e->mul, e->mul_ids, e->mul_stride, e->mul_rows};
+    p.x_planes = true;
+    if (y_planes) { p.y = y_planes; p.y_stride = 3 * y_k; p.y_k = y_k; }
+    return dense_linear(ctx, (hipStream_t)stream, p);
 }
 
 extern "C" int nvmai_hip_rms_residual_linear(nvmai_hip_ctx* ctx, nvmai_stream stream, const float* x, uint32_t x_stride, const float* delta,

@@ -23,6 +23,8 @@ struct DenseLinearParams {
     float* rms_out;
     uint32_t rms_delta_stride, rms_out_stride;
     float rms_add, rms_eps;
+    bool x_planes;          // x: planes (planes.hpp), x_stride 3 k, five rows or more
+    uint32_t y_k;           // y: planes of y_k values, y_stride 3 y_k (x_planes too); 0: activations
     bool loose;             // plain outputs need not lie at 16-byte boundaries: one value at a time
 };
 
@@ -36,6 +38,8 @@ inline uint32_t dense_plane_rows(uint32_t k) {
     return rows >= 32768u ? 32768u : rows >= 256u ? (uint32_t)(rows / 256u * 256u) : rows ? (uint32_t)rows : 1u;
 }
 void dense_split(hipStream_t s, const float* x, uint32_t x_stride, uint32_t rows, uint32_t k, uint16_t* planes);
+// Whether a call takes rows that are planes already.
+inline bool planes_fit(uint32_t rows, uint32_t k) { return (uint64_t)rows * k * 6u <= (128u << 20); }
 inline size_t dense_plane_bytes(uint32_t rows, uint32_t k) {
     const uint32_t most = dense_plane_rows(k);
     return (size_t)(rows < most ? rows : most) * k * 6u;

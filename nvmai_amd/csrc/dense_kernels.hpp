@@ -5,6 +5,7 @@
 #include "dense_internal.hpp"
 #include "dense_plan.hpp"
 #include "common.hpp"
+#include "planes.hpp"
 
 namespace nvmai {
 
@@ -175,6 +176,20 @@ __device__ __forceinline__ void dense_store4(const DenseLinearParams& p, uint32_
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             if (r0 + j < p.n) dense_store<EPI, ACT, PARTS>(p, t, r0 + j, v[j]);
+    }
+}
+
+// The same as planes (n a multiple of 4).
+template <int EPI>
+__device__ __forceinline__ void dense_store_planes(const DenseLinearParams& p, uint32_t t, uint32_t r0, dn_f4 v, dn_f4 bias) {
+    uint16_t* const row = static_cast<uint16_t*>(p.y) + (size_t)t * p.y_stride;
+    if constexpr (EPI == DE_PAIRS) {
+        const float out[2] = {dense_pair<ACT_FP32>(v[0], v[1]), dense_pair<ACT_FP32>(v[2], v[3])};
+        planes_put<2>(row, p.y_k, r0 / 2u, out);
+    } else {
+        v = dense_finish4<EPI, false>(p, t, r0, v, bias);
+        const float out[4] = {v[0], v[1], v[2], v[3]};
+        planes_put<4>(row, p.y_k, r0, out);
     }
 }
 
@@ -858,7 +873,14 @@ __global__ __launch_bounds__(256, dense_blocks(ACT, BN, BM)) void dense_tile_ker
         for (uint32_t k = 0; k < 32u / AT_ONCE; ++k) {
             const uint32_t token = lane / PER + k * AT_ONCE, t = m0 + wm + 32 * b + token;
             const dn_f4 v = *reinterpret_cast<const dn_f4*>(turn + token * PITCH + lane % PER * 4u);
-            if (t < p.rows && r < p.n) dense_store4<EPI, ACT, !SPLIT>(p, t, r, v, bias);
+            if (t >= p.rows || r >= p.n) continue;
+            if constexpr (SPLIT) {
+                if (p.y_k) {
+                    dense_store_planes<EPI>(p, t, r, v, bias);
+                    continue;
+                }
+            }
+            dense_store4<EPI, ACT, !SPLIT>(p, t, r, v, bias);
         }
     }
 }
@@ -1130,7 +1152,7 @@ void launch_tiles(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p)
     q.n = p.n - first;                                       // first is a multiple of 64: every operand stays aligned
     q.w = p.w + (size_t)first * p.w_stride;
     const uint32_t out = EPI == DE_PAIRS ? first / 2 : first;
-    if (p.y) q.y = static_cast<act_t<ACT>*>(p.y) + out;
+    if (p.y) q.y = p.y_k ? static_cast<void*>(static_cast<uint16_t*>(p.y) + out) : static_cast<void*>(static_cast<act_t<ACT>*>(p.y) + out);
     if (p.y_f32) q.y_f32 = p.y_f32 + out;
     if (p.bias) q.bias = p.bias + first;
     if (p.mul) q.mul = p.mul + first;
@@ -1162,6 +1184,7 @@ int dense_launch(nvmai_hip_ctx* ctx, hipStream_t s, const DenseLinearParams& p) 
     if (ctx->act == NVMAI_ACT_FP32) {
         const dim3 grid((p.n + 63) / 64, (p.rows + 63) / 64);
         if (grid.y > 65535) return NVMAI_ERR_UNSUPPORTED;
+        if (p.x_planes) return launch_tiles<EPI, ACT_FP32>(ctx, s, p), launch_status();
         if (p.planes) return launch_split<EPI>(ctx, s, p);
         dense_f32_kernel<EPI><<<grid, 256, 0, s>>>(p);
         return launch_status();

@@ -11,6 +11,7 @@
 //   * expanded, for prompts: keys and values of the range are formed by two matrix products, then flash attention.
 #pragma once
 
+#include "planes.hpp"
 #include "flash32.hpp"
 #include "rows.hpp"
 
@@ -193,6 +194,7 @@ struct LatentAttnParams {
     uint32_t splits, split_keys;
     // expanded form
     void *lat, *kn, *v;                  // [nk_pad, row_stride], [nk_pad, kn_stride], V (or V^T) rows of v_stride
+    uint16_t* planes;                    // the latents go here (planes.hpp, [nk_pad][3][rank]) and not to lat, whose rotated parts alone are written; nullptr: all to lat
     uint32_t nk, nk_pad, key0;           // keys of the call, the position of the first
     uint32_t kn_stride, v_stride;
 };
@@ -574,8 +576,16 @@ __global__ __launch_bounds__(256) void latent_gather_kernel(LatentAttnParams p) 
                             (size_t)((p.key0 + min(key, p.nk - 1u)) % p.cache.capacity) * p.cache.row_stride;
     act_t<ACT>* dst = static_cast<act_t<ACT>*>(p.lat) + (size_t)key * p.cache.row_stride;
     for (uint32_t j = threadIdx.x; j < pieces; j += 256u) {
-        const uint4 v = reinterpret_cast<const uint4*>(src)[j];
-        reinterpret_cast<uint4*>(dst)[j] = key < p.nk ? v : make_uint4(0u, 0u, 0u, 0u);
+        uint4 v = reinterpret_cast<const uint4*>(src)[j];
+        v = key < p.nk ? v : make_uint4(0u, 0u, 0u, 0u);
+        if constexpr (ACT == ACT_FP32) {
+            if (p.planes && PER * j < p.rank) {          // rank is a multiple of 64
+                const float f[4] = {__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w)};
+                planes_put<4>(p.planes + (size_t)key * 3u * p.rank, p.rank, PER * j, f);
+                continue;
+            }
+        }
+        reinterpret_cast<uint4*>(dst)[j] = v;
     }
 }
 

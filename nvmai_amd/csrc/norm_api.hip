@@ -47,6 +47,7 @@ int norm_residual_checked(nvmai_hip_ctx* ctx, nvmai_stream stream, const NormRes
     if (!ctx || !p.x || p.d == 0 || p.x_stride < p.d || (p.delta && p.delta_stride < p.d)) return NVMAI_ERR_INVALID_ARG;
     if ((next == NORM_NONE) != (p.out == nullptr) || (p.out && p.out_stride < p.d)) return NVMAI_ERR_INVALID_ARG;
     if (ctx->act != NVMAI_ACT_BF16 && ctx->act != NVMAI_ACT_FP32) return NVMAI_ERR_UNSUPPORTED;
+    if (p.planes_k && ctx->act != NVMAI_ACT_FP32) return NVMAI_ERR_UNSUPPORTED;
     if (p.d > 16384) return NVMAI_ERR_UNSUPPORTED;
     if (rows == 0) return NVMAI_OK;
     if (post != NORM_NONE && !p.delta) return NVMAI_ERR_INVALID_ARG;
@@ -73,4 +74,21 @@ extern "C" int nvmai_hip_rms_residual(nvmai_hip_ctx* ctx, nvmai_stream stream, f
                                       float next_add, void* out, uint32_t out_stride, uint32_t rows, uint32_t d, float eps) {
     const NormResidualParams p{x, delta, post_weight, nullptr, next_weight, nullptr, out, x_stride, delta_stride, out_stride, d, 1.0f, eps, post_add, next_add};
     return norm_residual_checked(ctx, stream, p, post_weight ? NORM_RMS : NORM_NONE, next_weight ? NORM_RMS : out ? NORM_COPY : NORM_NONE, rows);
+}
+
+extern "C" int nvmai_hip_norm_residual_planes(nvmai_hip_ctx* ctx, nvmai_stream stream, float* x, uint32_t x_stride, const float* delta,
+                                              uint32_t delta_stride, const uint16_t* post_weight, const uint16_t* post_bias, float mult,
+                                              const uint16_t* next_weight, const uint16_t* next_bias, uint16_t* out, uint32_t out_k, uint32_t rows,
+                                              uint32_t d, float eps) {
+    if (!out || !next_weight || out_k < d) return NVMAI_ERR_INVALID_ARG;
+    const NormResidualParams p{x, delta, post_weight, post_bias, next_weight, next_bias, out, x_stride, delta_stride, 3 * out_k, d, mult, eps, 0.0f, 0.0f, out_k};
+    return norm_residual_checked(ctx, stream, p, post_weight ? NORM_LAYER : NORM_NONE, NORM_LAYER, rows);
+}
+
+extern "C" int nvmai_hip_rms_residual_planes(nvmai_hip_ctx* ctx, nvmai_stream stream, float* x, uint32_t x_stride, const float* delta,
+                                             uint32_t delta_stride, const uint16_t* post_weight, float post_add, const uint16_t* next_weight,
+                                             float next_add, uint16_t* out, uint32_t out_k, uint32_t rows, uint32_t d, float eps) {
+    if (!out || out_k < d) return NVMAI_ERR_INVALID_ARG;
+    const NormResidualParams p{x, delta, post_weight, nullptr, next_weight, nullptr, out, x_stride, delta_stride, 3 * out_k, d, 1.0f, eps, post_add, next_add, out_k};
+    return norm_residual_checked(ctx, stream, p, post_weight ? NORM_RMS : NORM_NONE, next_weight ? NORM_RMS : NORM_COPY, rows);
 }

@@ -3,6 +3,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "planes.hpp"
 
 namespace nvmai {
 
@@ -66,6 +67,7 @@ struct NormResidualParams {
     void* out;
     uint32_t x_stride, delta_stride, out_stride, d;
     float mult, eps, post_add, next_add;
+    uint32_t planes_k;               // 32-bit contexts: out is planes of that many values (planes.hpp), out_stride 3 planes_k; 0: activations
 };
 
 __device__ __forceinline__ void norm_bf4(const uint16_t* p, float* v) {
@@ -138,6 +140,26 @@ __global__ __launch_bounds__(256) void norm_residual_kernel(NormResidualParams p
     if (NEXT == NORM_NONE) return;
     if (NEXT == NORM_LAYER) block_layernorm<VPT>(xv, p.d, p.eps, lds + 8);
     if (NEXT == NORM_RMS) block_rmsnorm<VPT>(xv, p.d, p.eps, lds + 8);
+    if constexpr (ACT == ACT_FP32) {
+        if (p.planes_k) {
+            uint16_t* to = static_cast<uint16_t*>(p.out) + (size_t)row * p.out_stride;
+#pragma unroll
+            for (int j = 0; j < VPT; ++j) {
+                const uint32_t at = 4u * (tid + 256u * j);
+                float o[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = NEXT == NORM_LAYER ? fmaf(xv[j][e], nw[j][e], nb[j][e]) : NEXT == NORM_RMS ? xv[j][e] * nw[j][e] : xv[j][e];
+                if (VEC) {
+                    if (at < p.d) planes_put<4>(to, p.planes_k, at, o);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (at + e < p.d) planes_put<1>(to, p.planes_k, at + e, o + e);
+                }
+            }
+            return;
+        }
+    }
     act_t<ACT>* out = static_cast<act_t<ACT>*>(p.out) + (size_t)row * p.out_stride;
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {

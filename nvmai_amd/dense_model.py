@@ -117,6 +117,13 @@ class DenseDecoder(StepDecoder):
         self._views[name, cols, dtype, at] = rows, view
         return view
 
+    def _operand(self, ctx, name, rows, cols, made, x=None):
+        """Scratch rows that only products read, of `made` values by a norm or the product of x with as many rows of a matrix: planes where the context multiplies
+        those (and x is planes)."""
+        if made % 4 or not ops.takes_planes(ctx, rows, cols) or (x is not None and x.dim() != 3):
+            return self._buf(name, rows, cols, ctx.dtype)
+        return self._buf(name + "_planes", rows, 3 * cols, torch.bfloat16, self.max_rows).view(rows, 3, cols)
+
     def _prefill_chunk_rows(self, tokens, b, start):
         return self._forward(tokens, ops.row_map(b, start))
 

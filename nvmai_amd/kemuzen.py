@@ -380,6 +380,7 @@ class KemuzenDecoder(DenseDecoder):
         ctx, D = self.pass_context(T), cfg.width
         x = self._buf("residual", T, D, torch.float32)
         h, last = self._buf("input", T, cfg.width_p, ctx.dtype), self._buf("normed", T, cfg.width_p, self.ctx.dtype)
+        normed = self._operand(ctx, "input", T, cfg.width_p, D)
         # Short passes: the end of a sublayer goes with the product that opens the next one, from one of two residuals to the other.
         joined = self.residual_hook is None and D == cfg.width_p and ops.joins_rms(ctx, T, D)
         other, ended = self._buf("residual2", T, D, torch.float32, FEW_ROWS) if joined else None, None
@@ -398,22 +399,23 @@ class KemuzenDecoder(DenseDecoder):
             left = (ff is not None) + (cfg.side > 0)         # sublayers of this layer still to come
 
             def close(delta, weight, add):           # the end of a sublayer; behind the model's last one the final norm (in the head's type)
-                nonlocal ended
+                nonlocal ended, h
                 if i + 1 == len(cfg.layers) and left == 0:
                     ops.rms_residual(self.ctx, x, D, delta, weight, add, self.w.final_norm, 1.0, last, cfg.eps)
                 elif joined:
                     ended = delta, weight, add
                 else:
-                    ops.rms_residual(ctx, x, D, delta, weight, add, out=h, eps=cfg.eps)
+                    ops.rms_residual(ctx, x, D, delta, weight, add, out=normed, eps=cfg.eps)
+                    h = normed
             close(self._mix(ctx, i, linear, T, rows_at), w["norm1"], 1.0)
             if ff is not None:
                 left -= 1
-                act = linear(w["gate_up"], y=self._buf("ff", T, w["down"].shape[1], ctx.dtype), activation=ops.LINEAR_SILU_PAIRS)
+                act = linear(w["gate_up"], y=self._operand(ctx, "ff", T, w["down"].shape[1], w["gate_up"].shape[0], h), activation=ops.LINEAR_SILU_PAIRS)
                 close(ops.dense_linear(ctx, w["down"], act, y_f32=self._buf("delta", T, cfg.width_p, torch.float32)), w["norm2"], 1.0)
             if cfg.side:
                 left -= 1
-                g = linear(w["side_gate"], y=self._buf("side", T, w["side_proj"].shape[1], ctx.dtype), activation=ops.LINEAR_GELU_TANH, mul=w["side_embed"],
-                           mul_ids=tokens)
+                g = linear(w["side_gate"], y=self._operand(ctx, "side", T, w["side_proj"].shape[1], w["side_gate"].shape[0], h), activation=ops.LINEAR_GELU_TANH,
+                           mul=w["side_embed"], mul_ids=tokens)
                 close(ops.dense_linear(ctx, w["side_proj"], g, y_f32=self._buf("delta", T, cfg.width_p, torch.float32)), w["side_norm"], 0.0)
             if self.residual_hook is not None:
                 self.residual_hook(i, x)
