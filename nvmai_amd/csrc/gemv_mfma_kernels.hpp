@@ -131,29 +131,26 @@ __global__ __launch_bounds__(64 * NW) void gemv_mfma_kernel(GemvMfmaParams p) {
                                                  meta_off, st * 16u, 0, 0);
 #endif
     };
-    // this wave's stages: wave_k, wave_k + KW, ...; its j-th one lands in the A arrays for even j
-    const uint32_t n_my = (uint32_t)wave_k < n_stages ? (n_stages - wave_k + KW - 1) / KW : 0u;
-    if (n_my > 0) issue_stage(wave_k, wa_w, ma_w);
-    if (n_my > 1) issue_stage(wave_k + KW, wb_w, mb_w);
-
     // ---- inputs of one panel: a wave converts whole rows (tokens wave, wave + NW, ...)
-    auto stage_inputs = [&](uint32_t k0) {
-        constexpr int CH = KP / 512;                         // 16-byte pieces per lane and row
+    constexpr int CH = KP / 512;                             // 16-byte pieces per lane and row
+    constexpr int TPW = NTOK / NW;                           // rows per wave
+    uint4 raw_all[TPW][CH];                                  // every load of the wave's rows is issued before the first is used
+    auto request_inputs = [&](uint32_t k0) {
         const uint32_t kp_len = min(KP, p.n - k0);
-        // every load of the wave's rows is issued before the first is used
-        constexpr int TPW = NTOK / NW;                       // rows per wave
-        uint4 raw_all[TPW][CH];
 #pragma unroll
-        for (int q = 0; q < TPW; ++q) {
-            const uint32_t t = wave + NW * q;
+        for (int q = 0; q < TPW; ++q)
 #pragma unroll
-            for (int c = 0; c < CH; ++c) {
-                const uint32_t e = (c * 64 + lane) * 8;
-                raw_all[q][c] = (t < p.n_tokens && e < kp_len)
-                                    ? *reinterpret_cast<const uint4*>(p.x + (size_t)t * p.x_stride + k0 + e)
-                                    : uint4{0u, 0u, 0u, 0u};
-            }
-        }
+            for (int c = 0; c < CH; ++c)                     // past the end: the last piece, the last row
+                raw_all[q][c] = *reinterpret_cast<const uint4*>(p.x + (size_t)min((uint32_t)(wave + NW * q), p.n_tokens - 1u) * p.x_stride + k0 +
+                                                                min((uint32_t)(c * 64 + lane) * 8u, kp_len - 8u));
+    };
+    auto stage_inputs = [&](uint32_t k0) {
+        const uint32_t kp_len = min(KP, p.n - k0);
+#pragma unroll
+        for (int q = 0; q < TPW; ++q)
+#pragma unroll
+            for (int c = 0; c < CH; ++c)
+                if (wave + NW * q >= p.n_tokens || (uint32_t)(c * 64 + lane) * 8u >= kp_len) raw_all[q][c] = uint4{0u, 0u, 0u, 0u};
 #pragma unroll
         for (int q = 0; q < TPW; ++q) {
             const uint32_t t = wave + NW * q;
@@ -195,6 +192,15 @@ __global__ __launch_bounds__(64 * NW) void gemv_mfma_kernel(GemvMfmaParams p) {
         }
         __syncthreads();
     };
+
+    // The first panel's inputs ahead of the weights: loads come back in their order, and the inputs, which the caches hold, are converted while the weights are on their way
+    // (16 tokens, 4 bits: 12,352 x 2048 10.1 -> 9.4 us, 2048 x 4096 10.5 -> 9.9).
+    request_inputs(0);
+    __builtin_amdgcn_sched_barrier(0);
+    // this wave's stages: wave_k, wave_k + KW, ...; its j-th one lands in the A arrays for even j
+    const uint32_t n_my = (uint32_t)wave_k < n_stages ? (n_stages - wave_k + KW - 1) / KW : 0u;
+    if (n_my > 0) issue_stage(wave_k, wa_w, ma_w);
+    if (n_my > 1) issue_stage(wave_k + KW, wb_w, mb_w);
 
     gm_f4_t total[TT];
     float ys[TT][4], yb[TT][4];
@@ -330,6 +336,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_mfma_kernel(GemvMfmaParams p) {
             close_panel();
             __syncthreads();                                     // every wave is through with the old panel
         }
+        if (k0 != 0) request_inputs(k0);
         stage_inputs(k0);
         while (j < n_my && (wave_k + j * KW) / SPP == panel) {   // wave-uniform
             const uint32_t st = wave_k + j * KW;
