@@ -419,6 +419,13 @@ int nvmai_hip_prefill_moe_reduce_token_major(nvmai_hip_ctx* ctx, nvmai_stream st
                                              void* h2, uint32_t h2_stride, uint32_t query_count,
                                              uint32_t top_k, uint32_t d);
 
+/* The same sum in the rows of a layer's end: hidden += round(sum + add), normed = rmsnorm(hidden) * norm_weight, with the roundings and
+ * the bits of nvmai_hip_prefill_moe_reduce_token_major, nvmai_hip_residual_add and nvmai_hip_residual_add_rmsnorm one after the other.  d a multiple of 8, at most 8192
+ * (NVMAI_ERR_UNSUPPORTED); rows at 16-byte boundaries. */
+int nvmai_hip_prefill_reduce_norm(nvmai_hip_ctx* ctx, nvmai_stream stream, const void* route_partials, const uint16_t* route_weights,
+                                  const void* add, uint32_t add_stride, void* hidden, uint32_t hidden_stride, const uint16_t* norm_weight, float eps,
+                                  void* normed, uint32_t normed_stride, uint32_t query_count, uint32_t top_k, uint32_t d);
+
 
 /* ---- KV cache -------------------------------------------------------------------------- */
 

@@ -184,6 +184,7 @@ SIGNATURES = {
     "nvmai_hip_prefill_grouped_moe_streamed": [vp, vp, C.POINTER(PrefillStreamedParams), C.POINTER(vp), u32, vp, vp, u64,
                                                vp, vp, vp],
     "nvmai_hip_affine_qmm": [vp, vp, vp, vp, vp, u32, vp, u32, vp, u32, u32, u32, u32],
+    "nvmai_hip_prefill_reduce_norm": [vp, vp, vp, vp, vp, u32, vp, u32, vp, C.c_float, vp, u32, u32, u32, u32],
     "nvmai_hip_prefill_moe_reduce_token_major": [vp, vp, vp, vp, vp, u32, u32, u32, u32],
     "nvmai_hip_silu_mul": [vp, vp, vp, vp, vp, u32],
     "nvmai_hip_sigmoid_gate_mul": [vp, vp, vp, vp, u32],

@@ -521,3 +521,28 @@ extern "C" int nvmai_hip_prefill_moe_reduce_token_major(nvmai_hip_ctx* ctx, nvma
 #undef NVMAI_REDUCE
     return launch_status();
 }
+
+extern "C" int nvmai_hip_prefill_reduce_norm(nvmai_hip_ctx* ctx, nvmai_stream stream, const void* route_partials, const uint16_t* route_weights,
+                                             const void* add, uint32_t add_stride, void* hidden, uint32_t hidden_stride, const uint16_t* norm_weight, float eps,
+                                             void* normed, uint32_t normed_stride, uint32_t query_count, uint32_t top_k, uint32_t d) {
+    if (!act16(ctx) || !route_partials || !route_weights || !add || !hidden || !norm_weight || !normed) return NVMAI_ERR_INVALID_ARG;
+    if (query_count == 0 || top_k == 0 || d == 0 || add_stride < d || hidden_stride < d || normed_stride < d) return NVMAI_ERR_INVALID_ARG;
+    if (d % 8 || d > 8192) return NVMAI_ERR_UNSUPPORTED;
+    if (!aligned16(route_partials) || !aligned16(add) || !aligned16(hidden) || !aligned16(norm_weight) || !aligned16(normed) || add_stride % 8 ||
+        hidden_stride % 8 || normed_stride % 8)
+        return NVMAI_ERR_ALIGNMENT;
+    hipStream_t s = (hipStream_t)stream;
+    ProfScope prof(ctx, NVMAI_PROF_PREFILL_COMBINE, s);
+    const ReduceNormParams p{(const uint16_t*)route_partials, route_weights, (const uint16_t*)add, (uint16_t*)hidden, norm_weight, (uint16_t*)normed,
+                             top_k, d, add_stride, hidden_stride, normed_stride, eps};
+#define NVMAI_REDUCE_NORM(PIECES)                                                                        \
+    do {                                                                                                 \
+        if (ctx->act == ACT_BF16) prefill_reduce_norm_kernel<ACT_BF16, PIECES><<<query_count, 256, 0, s>>>(p); \
+        else prefill_reduce_norm_kernel<ACT_FP16, PIECES><<<query_count, 256, 0, s>>>(p);                \
+    } while (0)
+    if (d <= 2048) NVMAI_REDUCE_NORM(1);
+    else if (d <= 4096) NVMAI_REDUCE_NORM(2);
+    else NVMAI_REDUCE_NORM(4);
+#undef NVMAI_REDUCE_NORM
+    return launch_status();
+}

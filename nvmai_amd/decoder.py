@@ -524,9 +524,8 @@ class HybridDecoder(StepDecoder):
             else:
                 branch = self._full_attention_prefill(L, w, normed, b, start, positions, T)
             routed_x = ops.residual_add_rmsnorm(ctx, hidden, branch, w["post_norm"], eps=cfg.rms_eps)
-            y = self._routed_moe_prefill(w, routed_x, T)
             nxt = self.w.layers[L + 1]["in_norm"] if L + 1 < cfg.layers else self.w.final_norm
-            normed = ops.residual_add_rmsnorm(ctx, hidden, y, nxt, eps=cfg.rms_eps)
+            normed = self._routed_moe_prefill(w, routed_x, T, hidden, nxt)
         return normed
 
     def _linear_attention_prefill(self, L, w, normed, b, T):
@@ -573,10 +572,11 @@ class HybridDecoder(StepDecoder):
         p_, s_, b_ = w["o_proj"]
         return ops.affine_gemv(ctx, p_, s_, b_, cfg.attn_bits, out.view(T, cfg.q_dim), cfg.hidden, cfg.q_dim)
 
-    def _routed_moe_prefill(self, w, x, T):
+    def _routed_moe_prefill(self, w, x, T, hidden, next_norm):
         """The MoE block of a chunk: below 64 rows the decode call (a work list over the distinct
         experts), from 64 rows on the prefill path -- tiled router, permutation by expert, grouped
-        GEMM, rank-order reduce -- with the shared expert beside it."""
+        GEMM, rank-order reduce -- with the shared expert beside it.  Its rows go into the residual stream; returns the
+        next layer's normed ones."""
         cfg, ctx = self.cfg, self.ctx
         D, F, E, K = cfg.hidden, cfg.moe_intermediate, cfg.num_experts, cfg.top_k
         sh = w.get("shared")                 # a shared expert of another width: beside the routed block
@@ -585,19 +585,21 @@ class HybridDecoder(StepDecoder):
             if sh is not None:
                 self.ew.encode_residual_add(y, ops.SharedExpertRuntime(ctx, sh["bits"]).encode(
                     sh["blob"], sh["offsets"], x, D, F, shared_gate=sh["gate"]))
-            return y
+            return ops.residual_add_rmsnorm(ctx, hidden, y, next_norm, eps=cfg.rms_eps)
         layer = w["moe"]
         idx, wts = self.moe.encode_router(layer.router, x, E, D, K)
         routes = ops.PrefillMoEGrouping(ctx).group_routes(idx, wts, E)
         pool = w["pool"]
         partials, _ = ops.PrefillGroupedRoutedMoE(ctx, cfg.expert_bits).encode(pool[:E], layer.offsets, x, D, F, routes)
-        h2 = ops.PrefillMoE(ctx).encode_reduce_token_major(partials, wts, T, K, D)
         if sh is not None:
             shared = ops.SharedExpertRuntime(ctx, sh["bits"]).encode(sh["blob"], sh["offsets"], x, D, F, shared_gate=sh["gate"])
         else:
             shared = ops.SharedExpertRuntime(ctx, cfg.expert_bits).encode(pool[E], layer.offsets, x, D, F,
                                                                           shared_gate=layer.shared_gate)
-        return self.ew.encode_residual_add(h2, shared)
+        if D % 8 == 0 and D <= 8192:
+            return ops.PrefillMoE(ctx).encode_reduce_norm(partials, wts, K, shared, hidden, next_norm, cfg.rms_eps)
+        h2 = ops.PrefillMoE(ctx).encode_reduce_token_major(partials, wts, T, K, D)
+        return ops.residual_add_rmsnorm(ctx, hidden, self.ew.encode_residual_add(h2, shared), next_norm, eps=cfg.rms_eps)
 
     def head(self):
         """LM head over the final-normed rows: logits in self.logits."""

@@ -602,6 +602,14 @@ class PrefillMoE:
                                                            top_k, d), "prefill_moe_reduce_token_major")
         return h2
 
+    def encode_reduce_norm(self, route_partials, route_weights, top_k, add, hidden, norm_weight, eps=1e-6):
+        """hidden += the reduced rows + add, in place; the rows normed for the next layer (rows of a multiple of 8 values, at most 8192)."""
+        rows, d = hidden.shape
+        normed = torch.empty_like(hidden)
+        check(lib.nvmai_hip_prefill_reduce_norm(self.ctx.handle, _stream(), _ptr(route_partials), _ptr(route_weights), _ptr(add), add.stride(0), _ptr(hidden),
+                                                hidden.stride(0), _ptr(norm_weight), eps, _ptr(normed), normed.stride(0), rows, top_k, d), "prefill_reduce_norm")
+        return normed
+
 
 def kv_row_layout(elements, bits):
     """KVCacheManager.rowLayout (KVCacheManager.swift:437-446) -> (stride, value_bytes)."""
