@@ -67,7 +67,7 @@ void launch_softmax_top64(const void* logits, uint32_t logits_stride, uint16_t* 
                           float softcap, float* tmax, float* tsum, uint64_t* keys, uint32_t runs, hipStream_t s) {
     const uint32_t tiles = (v + SOFTMAX_TILE - 1) / SOFTMAX_TILE;
     softmax_stage1_kernel<ACT><<<dim3(tiles, rows), 256, 0, s>>>(logits, v, logits_stride, softcap, tmax, tsum, tiles);
-    softmax_top64_kernel<ACT><<<dim3(tiles, rows), 1024, 0, s>>>(logits, v, logits_stride, softcap, tmax, tsum, tiles, probs, probs_stride, keys,
+    softmax_top64_kernel<ACT><<<dim3(runs, rows), 256, 0, s>>>(logits, v, logits_stride, softcap, tmax, tsum, tiles, probs, probs_stride, keys,
                                                                  runs * SAMPLE_KEEP);
 }
 }  // namespace

@@ -320,19 +320,19 @@ __global__ __launch_bounds__(256) void sample_topk64_stage1_kernel(const uint16_
     if (valid) out[(size_t)row * out_row_stride + blockIdx.x * SAMPLE_KEEP + threadIdx.x] = tile_key_64(best, base);
 }
 
-// Merge, normalize and the top 64 of each 1024 entries in one launch: a block takes the 4096 entries of a softmax tile, a thread four
-// neighbouring ones, four waves a tile of the sampler.  The same bits as the two kernels above (v <= 262144: the tiles' partial
-// states are one wave's, whatever the block's size).
+// Merge, normalize and the top 64 of each 1024 entries in one launch: a block takes 1024 entries, a tile of the sampler, a thread four
+// neighbouring ones.  The same bits as the two kernels above (v <= 262144: the tiles' partial states are one wave's).  Bound by the instructions of the selection, so
+// with a wave on a SIMD: blocks of four tiles, four waves on a SIMD, left most compute units idle (one row of 24,832 entries 8.6 -> 5.9 us, with the launches around it 18.0 -> 15.1; sixteen rows 19.7 -> 16.9, sixteen of 248,320 42.9 -> 41.1).
 template <int ACT>
-__global__ __launch_bounds__(1024) void softmax_top64_kernel(const void* logits, uint32_t v, uint32_t row_stride, float softcap,
+__global__ __launch_bounds__(256) void softmax_top64_kernel(const void* logits, uint32_t v, uint32_t row_stride, float softcap,
                                                              const float* tile_max, const float* tile_sum, uint32_t tiles,
                                                              uint16_t* probs, uint32_t probs_stride, uint64_t* out,
                                                              uint32_t out_row_stride) {
-    __shared__ float lds[32];
-    __shared__ uint32_t cand[4][256];
-    const uint32_t row = blockIdx.y, base = blockIdx.x * SOFTMAX_TILE, first = base + 4u * threadIdx.x;
+    __shared__ float lds[8];
+    __shared__ uint32_t cand[256];
+    const uint32_t row = blockIdx.y, base = blockIdx.x * SAMPLE_TILE, first = base + 4u * threadIdx.x;
     const act_t<ACT>* z = (const act_t<ACT>*)logits + (size_t)row * row_stride;
-    const bool whole = base + SOFTMAX_TILE <= v;
+    const bool whole = base + SAMPLE_TILE <= v;
     float x[4];
     if (whole && (reinterpret_cast<uintptr_t>(z + base) & (4u * sizeof(act_t<ACT>) - 1u)) == 0) {
         if constexpr (ACT == ACT_FP32) {
@@ -352,11 +352,11 @@ __global__ __launch_bounds__(1024) void softmax_top64_kernel(const void* logits,
 #pragma unroll
     for (int j = 0; j < 4; ++j) x[j] = first + j < v ? softcap_value(x[j], softcap) : -INFINITY;
     float m = threadIdx.x < tiles ? tm : -INFINITY, d = threadIdx.x < tiles && tm != -INFINITY ? ts : 0.0f;
-    block_softmax_merge<16>(m, d, lds);
+    block_softmax_merge<4>(m, d, lds);
     const float inv = d > 0.0f ? 1.0f / d : 0.0f;
     uint16_t* to = probs + (size_t)row * probs_stride;
     uint32_t mine[4], pr[4];
-    const uint32_t place = 4u * (threadIdx.x & 255u);
+    const uint32_t place = 4u * threadIdx.x;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         pr[j] = f32_to_f16(__expf(x[j] - m) * inv);
@@ -369,11 +369,9 @@ __global__ __launch_bounds__(1024) void softmax_top64_kernel(const void* logits,
         for (int j = 0; j < 4; ++j)
             if (first + j < v) to[first + j] = (uint16_t)pr[j];
     }
-    const uint32_t group = threadIdx.x >> 8, tile = 4u * blockIdx.x + group;
     bool valid;
-    const uint32_t best = tile_top64(mine, cand[group], valid);
-    if (valid && tile * SAMPLE_TILE < v)
-        out[(size_t)row * out_row_stride + tile * SAMPLE_KEEP + (threadIdx.x & 63u)] = tile_key_64(best, tile * SAMPLE_TILE);
+    const uint32_t best = tile_top64(mine, cand, valid);
+    if (valid) out[(size_t)row * out_row_stride + blockIdx.x * SAMPLE_KEEP + threadIdx.x] = tile_key_64(best, base);
 }
 
 // Selection over the sorted candidates (logit.metal:704-757 == :517-571): cap at k,
