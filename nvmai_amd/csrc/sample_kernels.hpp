@@ -425,7 +425,11 @@ __global__ __launch_bounds__(1024) void sample_topk64_final_kernel(const uint64_
     uint64_t k[4], ahead[4], best = none;
     const uint32_t rounds = (runs + 63u) / 64u;
     fetch(0, ahead);
-    for (uint32_t n = 0; n < rounds; ++n) {
+    if (runs <= 32u) {                                             // two runs a wave: one merge (25 runs 8.7 -> 7.7 us)
+        const uint64_t a = wave < runs ? ahead[0] : none, b = wave + 16u < runs ? ahead[1] : none;
+        best = lane_merge64(a > b ? a : b, lane, true);
+    }
+    for (uint32_t n = 0; n < rounds && runs > 32u; ++n) {
 #pragma unroll
         for (uint32_t r = 0; r < 4; ++r) k[r] = wave + 16u * (4u * n + r) < runs ? ahead[r] : none;
         if (n + 1u < rounds) fetch(n + 1u, ahead);
