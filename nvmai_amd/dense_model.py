@@ -118,9 +118,13 @@ class DenseDecoder(StepDecoder):
         return view
 
     def _operand(self, ctx, name, rows, cols, made, x=None):
-        """Scratch rows that only products read, of `made` values by a norm or the product of x with as many rows of a matrix: planes where the context multiplies
+        """Scratch rows that only products read, of `made` values by a norm, or by the product of x with the matrix `made`: planes where the context multiplies
         those (and x is planes)."""
-        if made % 4 or not ops.takes_planes(ctx, rows, cols) or (x is not None and x.dim() != 3):
+        if ctx.act != ops.ACT_FP32:
+            return self._buf(name, rows, cols, ctx.dtype)
+        if x is not None:
+            made = made.shape[0] if x.dim() == 3 else 1
+        if made % 4 or not ops.takes_planes(ctx, rows, cols):
             return self._buf(name, rows, cols, ctx.dtype)
         return self._buf(name + "_planes", rows, 3 * cols, torch.bfloat16, self.max_rows).view(rows, 3, cols)
 

@@ -410,11 +410,11 @@ class KemuzenDecoder(DenseDecoder):
             close(self._mix(ctx, i, linear, T, rows_at), w["norm1"], 1.0)
             if ff is not None:
                 left -= 1
-                act = linear(w["gate_up"], y=self._operand(ctx, "ff", T, w["down"].shape[1], w["gate_up"].shape[0], h), activation=ops.LINEAR_SILU_PAIRS)
+                act = linear(w["gate_up"], y=self._operand(ctx, "ff", T, w["down"].shape[1], w["gate_up"], h), activation=ops.LINEAR_SILU_PAIRS)
                 close(ops.dense_linear(ctx, w["down"], act, y_f32=self._buf("delta", T, cfg.width_p, torch.float32)), w["norm2"], 1.0)
             if cfg.side:
                 left -= 1
-                g = linear(w["side_gate"], y=self._operand(ctx, "side", T, w["side_proj"].shape[1], w["side_gate"].shape[0], h), activation=ops.LINEAR_GELU_TANH,
+                g = linear(w["side_gate"], y=self._operand(ctx, "side", T, w["side_proj"].shape[1], w["side_gate"], h), activation=ops.LINEAR_GELU_TANH,
                            mul=w["side_embed"], mul_ids=tokens)
                 close(ops.dense_linear(ctx, w["side_proj"], g, y_f32=self._buf("delta", T, cfg.width_p, torch.float32)), w["side_norm"], 0.0)
             if self.residual_hook is not None:

@@ -1128,7 +1128,7 @@ def dense_linear(ctx, weight, x, y=None, y_f32=None, n=None, activation=LINEAR_N
     (activations) and / or y_f32 are buffers [tokens, >= n] with one row stride.  bias: BF16 [n]; mul: BF16 columns [.., n]
     of a table.  LINEAR_SILU_PAIRS: y[t, j] = silu(row 2 j) * (row 2 j + 1).  x [tokens, 3, k] BF16: planes (takes_planes); y may be planes then."""
     rows, k = weight.shape
-    if x.dim() == 3:
+    if ctx.act == ACT_FP32 and x.dim() == 3:
         y = y_f32 if y is None else y
         to = (None, 0, _ptr(y), y.shape[2]) if y.dim() == 3 else (_ptr(y), y.stride(0), None, 0)
         e = LinearEpilogue(activation, _ptr(bias), _ptr(mul), _ptr(mul_ids), 0 if mul is None else mul.stride(0), 0 if mul is None else mul.shape[0])
@@ -1157,7 +1157,7 @@ def norm_residual(ctx, x, d, delta=None, post=None, mult=1.0, next_norm=None, ou
     (weight, bias): the end of a sublayer and the start of the next over the 32-bit residual x [tokens, >= d].  out may be planes."""
     pw, pb = post if post is not None else (None, None)
     nw, nb = next_norm if next_norm is not None else (None, None)
-    if out is not None and out.dim() == 3:
+    if ctx.act == ACT_FP32 and out is not None and out.dim() == 3:
         check(lib.nvmai_hip_norm_residual_planes(ctx.handle, _stream(), _ptr(x), x.stride(0), _ptr(delta), 0 if delta is None else delta.stride(0), _ptr(pw),
                                                  _ptr(pb), mult, _ptr(nw), _ptr(nb), _ptr(out), out.shape[2], x.shape[0], d, eps), "norm_residual_planes")
         return out
@@ -1170,7 +1170,7 @@ def norm_residual(ctx, x, d, delta=None, post=None, mult=1.0, next_norm=None, ou
 def rms_residual(ctx, x, d, delta=None, post=None, post_add=0.0, next_norm=None, next_add=0.0, out=None, eps=1e-6):
     """x += RMS(delta) * (post_add + post), then out = RMS(x) * (next_add + next_norm), or x as activations where
     next_norm is None.  out may be planes."""
-    if out is not None and out.dim() == 3:
+    if ctx.act == ACT_FP32 and out is not None and out.dim() == 3:
         check(lib.nvmai_hip_rms_residual_planes(ctx.handle, _stream(), _ptr(x), x.stride(0), _ptr(delta), 0 if delta is None else delta.stride(0), _ptr(post),
                                                 post_add, _ptr(next_norm), next_add, _ptr(out), out.shape[2], x.shape[0], d, eps), "rms_residual_planes")
         return out

@@ -259,7 +259,7 @@ class PakiraxDecoder(DenseDecoder):
                 close(delta, w["norm1b"], i + 1)
             else:
                 ops.norm_residual(ctx, x, D, delta, w["norm1b"], mult, w["norm2"], h, cfg.eps)
-                act = ops.dense_linear(ctx, w["up"], h, y=self._operand(ctx, "ff%d" % ff, T, w["down"].shape[1], w["up"].shape[0], h), activation=ops.LINEAR_GELU_ERF)
+                act = ops.dense_linear(ctx, w["up"], h, y=self._operand(ctx, "ff%d" % ff, T, w["down"].shape[1], w["up"], h), activation=ops.LINEAR_GELU_ERF)
                 delta = ops.dense_linear(ctx, w["down"], act, y_f32=self._buf("delta", T, cfg.width_p, torch.float32))
                 close(delta, w["norm2b"], i + 1)
             if self.residual_hook is not None:

@@ -1,4 +1,6 @@
 """Rows of 32-bit contexts that their producer stores as three BF16 planes: the bits of the calls on rows of floats."""
+import ctypes as C
+
 import pytest
 import torch
 
@@ -77,9 +79,12 @@ def test_refusals(nv):
     ctx, half, ops = nv.Context(0, nv.ACT_FP32), nv.Context(0, nv.ACT_BF16), nv.ops
     w, x = torch.zeros((66, 64), dtype=torch.bfloat16, device="cuda"), torch.zeros((8, 3, 64), dtype=torch.bfloat16, device="cuda")
     y = torch.zeros((8, 66), device="cuda")
-    for c, a, out in ((half, x, y), (ctx, x[:4], y), (ctx, x, torch.zeros((8, 3, 128), dtype=torch.bfloat16, device="cuda"))):
-        with pytest.raises(Exception):
-            ops.dense_linear(c, w, a, y=out)
+    # fewer than five rows; planes of an odd number of rows of the matrix; a context of 16 bits
+    for a, out in ((x[:4], y), (x, torch.zeros((8, 3, 128), dtype=torch.bfloat16, device="cuda"))):
+        with pytest.raises(nv.NvmaiError):
+            ops.dense_linear(ctx, w, a, y=out)
+    e = nv.ops.LinearEpilogue(ops.LINEAR_NONE, None, None, None, 0, 0)
+    assert nv.lib.nvmai_hip_dense_linear_planes(half.handle, ops._stream(), w.data_ptr(), 64, x.data_ptr(), 8, 66, 64, y.data_ptr(), 66, None, 0, C.byref(e)) != 0
     ops.dense_linear(ctx, w, x, y=y)
     ctx.close()
     half.close()

@@ -31,7 +31,7 @@ def _both(nv, ctx, layer, x, delta, weight):
 @pytest.mark.parametrize("looks", [1 << 14, 0])
 # tokens of one choosing block and of the next, of several; experts at the edges of a lane's share and of a block of rows; rows of one to eight pieces a lane
 @pytest.mark.parametrize("tokens,d,E,k,kind,gated", [
-    (5, 2048, 256, 8, 16, True), (8, 1024, 257, 7, 16, True), (16, 2048, 255, 8, 8, True), (17, 512, 8, 8, 16, False), (32, 2048, 256, 8, 16, True),
+    (1, 512, 40, 3, 4, True), (2, 1024, 256, 8, 16, False), (5, 2048, 256, 8, 16, True), (8, 1024, 257, 7, 16, True), (16, 2048, 255, 8, 8, True), (17, 512, 8, 8, 16, False), (32, 2048, 256, 8, 16, True),
     (33, 256, 40, 3, 4, True), (63, 1024, 512, 4, 16, True)])
 def test_one_launch_equals_two(nv, act, looks, tokens, d, E, k, kind, gated):
     print("router and work list", act, looks, tokens, d, E, k, flush=True)
