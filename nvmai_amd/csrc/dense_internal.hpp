@@ -2,6 +2,7 @@
 #pragma once
 
 #include "ctx.hpp"
+#include "rules.hpp"
 
 namespace nvmai {
 
@@ -31,19 +32,7 @@ struct DenseLinearParams {
 // What the form with rms_delta takes beside a 32-bit context: a row is held in the registers of one wave.
 constexpr uint32_t DENSE_RMS_ROWS = 2, DENSE_RMS_K = 2048;
 
-// 32-bit rows are multiplied as three BF16 planes, at most this many rows at a time: 128 MB of planes, or one row's (1.3 GB for
-// the longest that a call accepts), so that byte offsets inside them stay within 32 bits.
-inline uint32_t dense_plane_rows(uint32_t k) {
-    const uint64_t rows = (128u << 20) / (6ull * k);
-    return rows >= 32768u ? 32768u : rows >= 256u ? (uint32_t)(rows / 256u * 256u) : rows ? (uint32_t)rows : 1u;
-}
 void dense_split(hipStream_t s, const float* x, uint32_t x_stride, uint32_t rows, uint32_t k, uint16_t* planes);
-// Whether a call takes rows that are planes already.
-inline bool planes_fit(uint32_t rows, uint32_t k) { return (uint64_t)rows * k * 6u <= (128u << 20); }
-inline size_t dense_plane_bytes(uint32_t rows, uint32_t k) {
-    const uint32_t most = dense_plane_rows(k);
-    return (size_t)(rows < most ? rows : most) * k * 6u;
-}
 
 int dense_linear_check(const nvmai_hip_ctx* ctx, const DenseLinearParams& p);
 // What a call of more than 64 rows in a 16-bit context is expected to take, in ns.

@@ -209,7 +209,7 @@ extern "C" int nvmai_hip_latent_attention(nvmai_hip_ctx* ctx, nvmai_stream strea
     DenseLinearParams lv = flash ? DenseLinearParams{static_cast<const uint16_t*>(p.lat), uv, p.v, nullptr, cache->row_stride, c.rank, p.v_stride, vh, p.nk_pad, c.rank, NVMAI_LINEAR_NONE}
                                        : DenseLinearParams{uv, p.lat, p.v, nullptr, c.rank, cache->row_stride, p.v_stride, p.nk_pad, vh, c.rank, NVMAI_LINEAR_NONE};
     if (planes) lk.planes = lv.planes = ws_take<uint16_t>(ctx, n_planes);
-    if (planes && planes_fit(p.nk_pad, c.rank)) {        // both products multiply the same planes
+    if (planes && planes_at_once(p.nk_pad, c.rank)) {    // both products multiply the same planes
         p.planes = lk.planes;
         lk.x = lv.x = p.planes;
         lk.x_stride = lv.x_stride = 3 * c.rank;

@@ -1,6 +1,7 @@
 // Choices between the forms of a call that sizes alone decide: plain C++, without a device.
 #pragma once
 
+#include <stddef.h>
 #include <stdint.h>
 
 namespace nvmai {
@@ -37,5 +38,21 @@ inline uint32_t expert_block_tokens(uint32_t x_stride, uint32_t d, uint32_t f, u
     const uint32_t widest = x_stride > d ? (x_stride > f ? x_stride : f) : (d > f ? d : f);
     return 0xFFFFFFFFu / 2u / widest / 128u * 128u;
 }
+
+// 32-bit rows are multiplied as three BF16 planes, at most this many rows at a time: 128 MB of planes, or one row's (1.3 GB for
+// the longest that a call accepts), so that byte offsets inside them stay within 32 bits.
+inline uint32_t dense_plane_rows(uint32_t k) {
+    const uint64_t rows = (128u << 20) / (6ull * k);
+    return rows >= 32768u ? 32768u : rows >= 256u ? (uint32_t)(rows / 256u * 256u) : rows ? (uint32_t)rows : 1u;
+}
+inline size_t dense_plane_bytes(uint32_t rows, uint32_t k) {
+    const uint32_t most = dense_plane_rows(k);
+    return (size_t)(rows < most ? rows : most) * k * 6u;
+}
+// Whether a call takes rows that are planes already, in memory of its caller's.
+inline bool planes_fit(uint32_t rows, uint32_t k) { return (uint64_t)rows * k * 6u <= (128u << 20); }
+// Whether dense_plane_bytes is room for the planes of all rows at once, which products that share them need: the latents of an expanded 32-bit attention.
+// Past it each product makes its own, in portions.
+inline bool planes_at_once(uint32_t rows, uint32_t k) { return rows <= dense_plane_rows(k); }
 
 }  // namespace nvmai

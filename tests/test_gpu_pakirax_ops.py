@@ -402,6 +402,18 @@ def test_latent_decode_batch_of_unequal_positions(ctx):
     close(y, L.plain(lengths), 2e-5 if is32(ctx) else 2e-2)
 
 
+@pytest.mark.parametrize("n", [32768, 32768 + 100])
+def test_latent_attention_over_more_keys_than_planes_are_made_of_at_once(ctx, n):
+    """A portion behind a long context: up to 32,768 keys both products of a 32-bit context share their planes, past it each makes its own in portions."""
+    import nvmai_amd as nv
+    say("latent keys", ctx.dtype, n)
+    L = Latent(ctx, np.random.default_rng(n), 1, 16, 16, 16, 64, 0, n)
+    L.op.encode_epilogue(L.proj, 0, L.qc, L.qn, L.qc, L.qc + L.rank, L.kvn, torch.zeros((n, 64), dtype=ctx.dtype, device="cuda"), L.cache, nv.row_map(0, 0))
+    y = torch.zeros((40, 16), dtype=ctx.dtype, device="cuda")
+    L.op.encode(L.q[n - 40:].clone(), L.proj[n - 40:, L.qc + L.rank + L.rot:], L.uk, L.uv, L.cache, nv.row_map(0, n - 40), y, nv.LATENT_EXPANDED)
+    close(y, L.plain(range(n - 40, n)), 2e-5 if is32(ctx) else 2e-2)
+
+
 def test_latent_attention_in_32_bit_over_a_bf16_cache():
     """32-bit rows beside a BF16 cache: what passes of one or two rows use.  The cached rows and the query on its way to them are
     BF16, everything else 32-bit; the expanded form is refused."""

@@ -79,3 +79,16 @@ def test_parts_have_a_unit_each_and_are_taken_where_they_save_time(rule):
     # what one sum per output is for: prompts of 4096 tokens in portions of 2048, and of 1501
     long = [(2048, n, 2048, 1, 1) for n in (2048, 4160, 8192, 8256)] + [(2048, 2048, 8192, 1, 1), (1501, 256, 2048, 1, 1), (1501, 2048, 5632, 1, 1), (1501, 11264, 2048, 1, 1)]
     assert set(value(PLAN + ".head.parts", long)) == {1}
+
+
+def test_planes_that_products_share_lie_in_the_room_they_were_given(rule):
+    # latents of an expanded attention: keys in steps of 64, beside what the room's own steps of 256 rows and its end at 32,768 leave
+    cases = [(rows, k) for k in (*range(64, 1600, 64), 4096, 1 << 20, 1 << 26) for rows in (64, 4096, 14336, 14400, 14464, 14528, 21824, 21888, 32704, *range(32768, 400000, 64 * 13), 43648, 46656,
+                                                                             48704, 87360, 349504)]
+    names = ("rows", "k")
+    at_once = rule(names, cases, "planes_at_once(rows, k)")
+    for (rows, k), whole, room in zip(cases, at_once, rule(names, cases, "dense_plane_bytes(rows, k)")):
+        assert room <= max(128 << 20, 6 * k) and (not whole or room == 6 * rows * k), (rows, k)
+    # past 32,768 rows they had been taken as whole wherever 128 MB hold all of them
+    answer = dict(zip(cases, at_once))
+    assert answer[32768, 256] and not answer[32768 + 64 * 13, 64] and not answer[46656, 256] and not answer[14400, 1536] and answer[14336, 1536]
