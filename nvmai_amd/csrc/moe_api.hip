@@ -412,7 +412,7 @@ void launch_down_combine(int act, uint32_t bits, const DownCombineParams& p, hip
 
 // The same in one launch (moe_one_kernels.hpp), for one token.  False, having launched nothing, for shapes that have no such form: rows of gate and up that a wave reads
 // whole and whose inputs a block holds (d up to 2048), rows of the down projection of 16 or 32 pieces (64 would be held in more registers than the others leave), more blocks than one launch
-// numbers, an output that lies over what the launch reads.
+// numbers, outputs that lie over what the launch reads or over one another (block_overlaps).
 template <int ACT, int BITS, int NCH>
 bool launch_moe_one_t(const MoeOneParams& p, uint32_t blocks, hipStream_t s) {
     const size_t rows_lds = moe_one_rows_lds(p.rows.n, NCH);
@@ -438,20 +438,11 @@ bool launch_moe_one_act(uint32_t bits, const MoeOneParams& p, uint32_t blocks, h
     return false;
 }
 
-// Whether rows of `d` 16-bit values `stride` apart at a and at b have bytes in common.
-bool rows_overlap(const void* a, uint32_t a_stride, const void* b, uint32_t b_stride, uint32_t rows, uint32_t d) {
-    if (!a || !b) return false;
-    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
-    const uintptr_t nx = ((uintptr_t)(rows - 1) * a_stride + d) * 2, ny = ((uintptr_t)(rows - 1) * b_stride + d) * 2;
-    return x < y + ny && y < x + nx;
-}
+Rows16 rows16(const void* at, uint32_t stride) { return Rows16{reinterpret_cast<uintptr_t>(at), stride}; }
 
-// Whether what a launch with the prologue stores lies over the rows that all of its blocks read.
 bool prologue_overlaps(const RouterParams& r) {
-    const struct { const void* at; uint32_t stride; } outs[2] = {{r.pre_hidden_out, r.pre_hidden_stride}, {r.pre_normed_out, r.pre_normed_stride}};
-    for (const auto& o : outs)
-        if (rows_overlap(o.at, o.stride, r.x, r.x_stride, r.tokens, r.d) || rows_overlap(o.at, o.stride, r.pre_delta, r.pre_delta_stride, r.tokens, r.d)) return true;
-    return false;
+    return nvmai::prologue_overlaps(rows16(r.x, r.x_stride), rows16(r.pre_delta, r.pre_delta_stride), rows16(r.pre_hidden_out, r.pre_hidden_stride),
+                                    rows16(r.pre_normed_out, r.pre_normed_stride), r.tokens, r.d);
 }
 
 bool launch_moe_one(const nvmai_hip_ctx* ctx, uint32_t bits, MoeOneParams& p, hipStream_t s) {
@@ -459,8 +450,8 @@ bool launch_moe_one(const nvmai_hip_ctx* ctx, uint32_t bits, MoeOneParams& p, hi
     if (T != 1 || D > 2048 || D % 256 || F < 64) return false;
     const RouterParams& r = p.router;
     if ((rows_chunks(r.router.kind, D) + 31) / 32 > 8) return false;
-    if (prologue_overlaps(r) || rows_overlap(p.down.y, p.down.y_stride, r.x, r.x_stride, T, D) ||
-        rows_overlap(p.down.y, p.down.y_stride, r.pre_delta, r.pre_delta_stride, T, D))
+    if (block_overlaps(rows16(r.x, r.x_stride), rows16(r.pre_delta, r.pre_delta_stride), rows16(r.pre_hidden_out, r.pre_hidden_stride),
+                       rows16(r.pre_normed_out, r.pre_normed_stride), rows16(p.down.y, p.down.y_stride), T, D))
         return false;
     p.router_blocks = (r.num_experts + (r.gate.kind ? 1u : 0u) + MOE_ONE_LOGITS - 1) / MOE_ONE_LOGITS;
     p.slots = p.sel.top_k + (p.down.has_shared ? 1u : 0u);

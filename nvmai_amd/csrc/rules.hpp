@@ -55,4 +55,29 @@ inline bool planes_fit(uint32_t rows, uint32_t k) { return (uint64_t)rows * k * 
 // Past it each product makes its own, in portions.
 inline bool planes_at_once(uint32_t rows, uint32_t k) { return rows <= dense_plane_rows(k); }
 
+// Rows of values of 16 bits by their addresses, 0: none.
+struct Rows16 {
+    uint64_t at;
+    uint32_t stride;
+};
+
+// Whether `rows` rows of `d` values at a and at b have bytes in common.
+inline bool rows_overlap(const Rows16& a, const Rows16& b, uint32_t rows, uint32_t d) {
+    if (!a.at || !b.at) return false;
+    const uint64_t na = ((uint64_t)(rows - 1) * a.stride + d) * 2, nb = ((uint64_t)(rows - 1) * b.stride + d) * 2;
+    return a.at < b.at + nb && b.at < a.at + na;
+}
+
+// Whether what the prologue of a launch stores lies over the rows that all of its blocks read.
+inline bool prologue_overlaps(const Rows16& x, const Rows16& delta, const Rows16& hidden_out, const Rows16& normed_out, uint32_t rows, uint32_t d) {
+    return rows_overlap(hidden_out, x, rows, d) || rows_overlap(hidden_out, delta, rows, d) || rows_overlap(normed_out, x, rows, d) || rows_overlap(normed_out, delta, rows, d);
+}
+
+// The same of a launch that holds the whole MoE block: y, too, lies over nothing that other blocks read, nor over what another block stores, which nothing orders (a block
+// that waits in vain stores the prologue's rows once more, after others have stored y).
+inline bool block_overlaps(const Rows16& x, const Rows16& delta, const Rows16& hidden_out, const Rows16& normed_out, const Rows16& y, uint32_t rows, uint32_t d) {
+    return prologue_overlaps(x, delta, hidden_out, normed_out, rows, d) || rows_overlap(y, x, rows, d) || rows_overlap(y, delta, rows, d) ||
+           rows_overlap(y, hidden_out, rows, d) || rows_overlap(y, normed_out, rows, d);
+}
+
 }  // namespace nvmai

@@ -114,3 +114,24 @@ def test_one_launch_with_scores_that_are_not_numbers(nv):
             assert torch.equal(one[1], three[1]) and torch.equal(one[2].view(torch.int16), three[2].view(torch.int16)), (E, at)
             assert torch.equal(torch.isnan(one[0]), torch.isnan(three[0]))
     ctx.close()
+
+
+@pytest.mark.parametrize("looks", [1 << 14, 0])
+def test_output_in_place_of_the_prologues_rows(nv, looks):
+    # y over normed or hidden_out takes three launches: the rows of separate buffers, y last
+    print("one launch, y over the prologue's rows", looks, flush=True)
+    ctx = nv.Context(0, nv.ACT_BF16)
+    assert nv.lib.nvmai_hip_ctx_wait_limit(ctx.handle, looks) == 0
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    row = lambda: torch.empty((1, 2048), device="cuda").normal_(0.0, 1.0, generator=gen).to(torch.bfloat16)
+    layer, keep = _layer(nv, ctx, gen, 2048, 512, 64, 8, 4, True, True)
+    moe, hidden, delta, weight = nv.MoE(ctx, 4), row(), row(), row()[0]
+    h, normed, y = row(), row(), row()
+    moe.decode_layer_prenorm(layer, hidden, delta, weight, h, normed, y)
+    h2, both = row(), row()
+    moe.decode_layer_prenorm(layer, hidden, delta, weight, h2, both, both)
+    assert torch.equal(h2, h) and torch.equal(both, y)
+    n2, both = row(), row()
+    moe.decode_layer_prenorm(layer, hidden, delta, weight, both, n2, both)
+    assert torch.equal(n2, normed) and torch.equal(both, y)
+    ctx.close()

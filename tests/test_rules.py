@@ -92,3 +92,20 @@ def test_planes_that_products_share_lie_in_the_room_they_were_given(rule):
     # past 32,768 rows they had been taken as whole wherever 128 MB hold all of them
     answer = dict(zip(cases, at_once))
     assert answer[32768, 256] and not answer[32768 + 64 * 13, 64] and not answer[46656, 256] and not answer[14400, 1536] and answer[14336, 1536]
+
+
+def test_rows_that_one_launch_of_the_expert_block_does_not_take(rule):
+    # y in the place of any row that the launch reads or stores, whole or by its ends; x, delta, hidden_out and normed apart
+    D, at = 2048, dict(x=1 << 20, delta=2 << 20, hidden_out=3 << 20, normed=4 << 20)
+    names = ("x", "delta", "hidden", "normed", "y", "d")
+    row = lambda a: "Rows16{%s, 4096}" % a
+    overlaps = lambda cases: rule(names, cases, "block_overlaps(%s, %s, %s, %s, %s, 1, d)" % tuple(map(row, names[:5])))
+    places = tuple(at.values())
+    assert overlaps([(*places, p + o, D) for p in places for o in (0, 2 * D - 2, 2 - 2 * D)]) == [1] * 12
+    assert overlaps([(*places, p + o, D) for p in places for o in (2 * D, -2 * D)]) == [0] * 8
+    assert overlaps([(at["x"], 0, 0, 0, at["x"], D), (at["x"], 0, 0, 0, at["delta"], D)]) == [1, 0]
+    # the prologue's rows over what it reads
+    assert overlaps([(*(at[k] for k in order), 5 << 20, D) for order in (("x", "delta", "x", "normed"), ("x", "delta", "delta", "normed"), ("x", "delta", "hidden_out", "delta"))]) == [1] * 3
+    # several tokens: by the ends of their rows
+    several = "rows_overlap(Rows16{x, 4096}, Rows16{y, 4096}, 3, 2048)"
+    assert rule(("x", "y"), [(1 << 20, (1 << 20) + 2 * 4096 * 2 + 4094), (1 << 20, (1 << 20) + 2 * 4096 * 2 + 4096)], several) == [1, 0]
