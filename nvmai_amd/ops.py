@@ -1123,14 +1123,19 @@ SCAN_DELTA, SCAN_SSD = 0, 1
 LINEAR_NONE, LINEAR_GELU_ERF, LINEAR_GELU_TANH, LINEAR_SILU_PAIRS = range(4)
 
 
+def _are_planes(rows):
+    """Whether rows of a 32-bit context are planes, [rows, 3, k] BF16: floats may have three dimensions too (heads)."""
+    return rows.dim() == 3 and rows.dtype == torch.bfloat16
+
+
 def dense_linear(ctx, weight, x, y=None, y_f32=None, n=None, activation=LINEAR_NONE, bias=None, mul=None, mul_ids=None):
     """y[t] = act(W x[t] + bias) * mul[mul_ids[t]]: weight [n, k] BF16 (k a multiple of 64), x [tokens, >= k] activations; y
     (activations) and / or y_f32 are buffers [tokens, >= n] with one row stride.  bias: BF16 [n]; mul: BF16 columns [.., n]
     of a table.  LINEAR_SILU_PAIRS: y[t, j] = silu(row 2 j) * (row 2 j + 1).  x [tokens, 3, k] BF16: planes (takes_planes); y may be planes then."""
     rows, k = weight.shape
-    if ctx.act == ACT_FP32 and x.dim() == 3:
+    if ctx.act == ACT_FP32 and _are_planes(x):
         y = y_f32 if y is None else y
-        to = (None, 0, _ptr(y), y.shape[2]) if y.dim() == 3 else (_ptr(y), y.stride(0), None, 0)
+        to = (None, 0, _ptr(y), y.shape[2]) if _are_planes(y) else (_ptr(y), y.stride(0), None, 0)
         e = LinearEpilogue(activation, _ptr(bias), _ptr(mul), _ptr(mul_ids), 0 if mul is None else mul.stride(0), 0 if mul is None else mul.shape[0])
         check(lib.nvmai_hip_dense_linear_planes(ctx.handle, _stream(), _ptr(weight), weight.stride(0), _ptr(x), x.shape[0], rows if n is None else n, k, *to,
                                                 C.byref(e)), "dense_linear_planes")
@@ -1157,7 +1162,7 @@ def norm_residual(ctx, x, d, delta=None, post=None, mult=1.0, next_norm=None, ou
     (weight, bias): the end of a sublayer and the start of the next over the 32-bit residual x [tokens, >= d].  out may be planes."""
     pw, pb = post if post is not None else (None, None)
     nw, nb = next_norm if next_norm is not None else (None, None)
-    if ctx.act == ACT_FP32 and out is not None and out.dim() == 3:
+    if ctx.act == ACT_FP32 and out is not None and _are_planes(out):
         check(lib.nvmai_hip_norm_residual_planes(ctx.handle, _stream(), _ptr(x), x.stride(0), _ptr(delta), 0 if delta is None else delta.stride(0), _ptr(pw),
                                                  _ptr(pb), mult, _ptr(nw), _ptr(nb), _ptr(out), out.shape[2], x.shape[0], d, eps), "norm_residual_planes")
         return out
@@ -1170,7 +1175,7 @@ def norm_residual(ctx, x, d, delta=None, post=None, mult=1.0, next_norm=None, ou
 def rms_residual(ctx, x, d, delta=None, post=None, post_add=0.0, next_norm=None, next_add=0.0, out=None, eps=1e-6):
     """x += RMS(delta) * (post_add + post), then out = RMS(x) * (next_add + next_norm), or x as activations where
     next_norm is None.  out may be planes."""
-    if ctx.act == ACT_FP32 and out is not None and out.dim() == 3:
+    if ctx.act == ACT_FP32 and out is not None and _are_planes(out):
         check(lib.nvmai_hip_rms_residual_planes(ctx.handle, _stream(), _ptr(x), x.stride(0), _ptr(delta), 0 if delta is None else delta.stride(0), _ptr(post),
                                                 post_add, _ptr(next_norm), next_add, _ptr(out), out.shape[2], x.shape[0], d, eps), "rms_residual_planes")
         return out

@@ -88,3 +88,20 @@ def test_refusals(nv):
     ops.dense_linear(ctx, w, x, y=y)
     ctx.close()
     half.close()
+
+
+def test_rows_of_floats_by_heads(nv):
+    # three dimensions do not make planes: [tokens, 3, values] floats are rows of 3 * values
+    print("floats by heads", flush=True)
+    ctx, ops = nv.Context(0, nv.ACT_FP32), nv.ops
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    w, norm, x = _normal(gen, 96, 192).to(torch.bfloat16), _normal(gen, 192).to(torch.bfloat16), _normal(gen, 40, 192)
+    want, got = torch.zeros((40, 96), device="cuda"), torch.zeros((40, 3, 32), device="cuda")
+    ops.dense_linear(ctx, w, x, y=want)
+    ops.dense_linear(ctx, w, x.view(40, 3, 64), y=got)
+    assert torch.equal(got.view(40, 96), want)
+    for call in (lambda out: ops.norm_residual(ctx, x, 192, next_norm=(norm, norm), out=out), lambda out: ops.rms_residual(ctx, x, 192, next_norm=norm, out=out)):
+        want, got = torch.zeros((40, 192), device="cuda"), torch.zeros((40, 3, 64), device="cuda")
+        call(want), call(got)
+        assert torch.equal(got.view(40, 192), want)
+    ctx.close()
