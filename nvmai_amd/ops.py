@@ -1134,6 +1134,7 @@ def dense_linear(ctx, weight, x, y=None, y_f32=None, n=None, activation=LINEAR_N
     of a table.  LINEAR_SILU_PAIRS: y[t, j] = silu(row 2 j) * (row 2 j + 1).  x [tokens, 3, k] BF16: planes (takes_planes); y may be planes then."""
     rows, k = weight.shape
     if ctx.act == ACT_FP32 and _are_planes(x):
+        assert x.shape[2] == k and (y is None or y_f32 is None), "rows of planes have the matrix's length, their product one output"
         y = y_f32 if y is None else y
         to = (None, 0, _ptr(y), y.shape[2]) if _are_planes(y) else (_ptr(y), y.stride(0), None, 0)
         e = LinearEpilogue(activation, _ptr(bias), _ptr(mul), _ptr(mul_ids), 0 if mul is None else mul.stride(0), 0 if mul is None else mul.shape[0])

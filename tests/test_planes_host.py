@@ -45,3 +45,14 @@ def test_planes_take_the_calls_on_planes(calls):
     ops.rms_residual(CTX, flat, 64, out=x)
     assert [name for name, _ in calls] == ["nvmai_hip_dense_linear_planes"] * 2 + ["nvmai_hip_norm_residual_planes", "nvmai_hip_rms_residual_planes"]
     assert calls[1][1][8:12] == (by_heads.data_ptr(), 8, None, 0)
+
+
+def test_a_product_of_planes_has_one_output_and_rows_of_the_matrix(calls):
+    w, x, y = torch.zeros((8, 64), dtype=torch.bfloat16), torch.zeros((6, 3, 64), dtype=torch.bfloat16), torch.zeros((6, 8))
+    with pytest.raises(AssertionError):
+        ops.dense_linear(CTX, w, x, y=y, y_f32=torch.zeros((6, 8)))
+    with pytest.raises(AssertionError):
+        ops.dense_linear(CTX, w, torch.zeros((6, 3, 128), dtype=torch.bfloat16), y=y)
+    assert not calls
+    ops.dense_linear(CTX, w, x, y_f32=y)
+    assert calls[0][1][8] == y.data_ptr()
