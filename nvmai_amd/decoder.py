@@ -596,7 +596,7 @@ class HybridDecoder(StepDecoder):
         else:
             shared = ops.SharedExpertRuntime(ctx, cfg.expert_bits).encode(pool[E], layer.offsets, x, D, F,
                                                                           shared_gate=layer.shared_gate)
-        if D % 8 == 0 and D <= 8192:
+        if ops.PrefillMoE.takes_reduce_norm(D, next_norm):
             return ops.PrefillMoE(ctx).encode_reduce_norm(partials, wts, K, shared, hidden, next_norm, cfg.rms_eps)
         h2 = ops.PrefillMoE(ctx).encode_reduce_token_major(partials, wts, T, K, D)
         return ops.residual_add_rmsnorm(ctx, hidden, self.ew.encode_residual_add(h2, shared), next_norm, eps=cfg.rms_eps)

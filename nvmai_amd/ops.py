@@ -602,6 +602,11 @@ class PrefillMoE:
                                                            top_k, d), "prefill_moe_reduce_token_major")
         return h2
 
+    @staticmethod
+    def takes_reduce_norm(d, norm_weight):
+        """Whether encode_reduce_norm takes rows of d values (at 16-byte boundaries) and this weight, which may be a view into a model's file at any address."""
+        return d % 8 == 0 and d <= 8192 and norm_weight is not None and norm_weight.data_ptr() % 16 == 0
+
     def encode_reduce_norm(self, route_partials, route_weights, top_k, add, hidden, norm_weight, eps=1e-6):
         """hidden += the reduced rows + add, in place; the rows normed for the next layer (rows of a multiple of 8 values, at most 8192)."""
         rows, d = hidden.shape

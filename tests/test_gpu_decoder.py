@@ -343,3 +343,24 @@ def test_full_size_configs4_step_properties():
         dec.logits.zero_()                                   # eager work between the replays
     torch.cuda.synchronize()
     ctx.close()
+
+
+def test_prompts_with_norms_at_any_address():
+    # weights that are views into a file lie where it has them: at an odd multiple of two bytes a prompt takes the launches that read them so, with the same bits
+    import nvmai_amd as nv
+    from nvmai_amd.decoder import HybridConfig, HybridDecoder, HybridWeights
+    say("prompt with norms at odd addresses")
+    ctx = nv.Context(0, nv.ACT_BF16)
+    cfg = HybridConfig(hidden=256, layers=2, full_every=2, num_heads=4, num_kv_heads=2, head_dim=64, rotary_dim=16,
+                       rope_theta=1e4, gdn=(2, 4, 32, 32, 4), num_experts=4, top_k=4, moe_intermediate=128, vocab=1024,
+                       expert_bits=4, attn_bits=4, kv_bits=8, head_bits=16, gdn_state_bf16=False)
+    w = HybridWeights(ctx, cfg, seed=11, std=0.06)
+    tokens = torch.arange(100, dtype=torch.int32, device="cuda") * 7 % cfg.vocab
+    prompt = lambda: HybridDecoder(ctx, cfg, w, 1, 256)._prefill_chunk_rows(tokens, 0, 0).clone()
+    want, held = prompt(), torch.zeros(2 * 256 + 1, dtype=w.final_norm.dtype, device="cuda")
+    for at, (place, name) in enumerate(((w.layers[1], "in_norm"), (w.__dict__, "final_norm"))):
+        odd = held[at * 256 + 1:(at + 1) * 256 + 1]
+        odd.copy_(place[name])
+        place[name] = odd
+    assert torch.equal(prompt(), want)
+    ctx.close()
