@@ -1,6 +1,7 @@
 // Host side of the matrix-core GEMV for 3 .. 32 input rows.
 #include "ctx.hpp"
 #include "gemv_mfma_kernels.hpp"
+#include "rules.hpp"
 
 namespace nvmai {
 
@@ -23,15 +24,17 @@ int gemv_mfma(nvmai_hip_ctx* ctx, hipStream_t s, const uint8_t* w, const uint16_
     const int wr = m >= 8192 ? 4 : m >= 4096 ? 2 : 1;
     const dim3 grid((m + 16 * wr - 1) / (16 * wr));
     // eight waves per block for 4-bit rows (8-bit rows would need 200 KB of LDS for them)
-#define NVMAI_GM_N(ACT, BITS, TT, NW)                                                          \
-    do {                                                                                       \
-        if (wr == 4) gemv_mfma_kernel<ACT, BITS, TT, 4, NW><<<grid, 64 * NW, 0, s>>>(p);       \
-        else if (wr == 2) gemv_mfma_kernel<ACT, BITS, TT, 2, NW><<<grid, 64 * NW, 0, s>>>(p);  \
-        else gemv_mfma_kernel<ACT, BITS, TT, 1, NW><<<grid, 64 * NW, 0, s>>>(p);               \
+    const bool first = gemv_inputs_first(bits, n_tokens, n);
+#define NVMAI_GM_N(ACT, BITS, TT, NW, FIRST)                                                          \
+    do {                                                                                              \
+        if (wr == 4) gemv_mfma_kernel<ACT, BITS, TT, 4, NW, FIRST><<<grid, 64 * NW, 0, s>>>(p);       \
+        else if (wr == 2) gemv_mfma_kernel<ACT, BITS, TT, 2, NW, FIRST><<<grid, 64 * NW, 0, s>>>(p);  \
+        else gemv_mfma_kernel<ACT, BITS, TT, 1, NW, FIRST><<<grid, 64 * NW, 0, s>>>(p);               \
     } while (0)
 #define NVMAI_GM_T(ACT, BITS, TT)                                                              \
     do {                                                                                       \
-        NVMAI_GM_N(ACT, BITS, TT, (BITS == 4 ? 8 : 4));                                        \
+        if (first) NVMAI_GM_N(ACT, BITS, TT, (BITS == 4 ? 8 : 4), true);                       \
+        else NVMAI_GM_N(ACT, BITS, TT, (BITS == 4 ? 8 : 4), false);                            \
     } while (0)
 #define NVMAI_GM(ACT, BITS)                                                                    \
     do {                                                                                       \

@@ -64,7 +64,8 @@ constexpr uint32_t GM_STAGE_CODES = 512;        // codes of a row per stage: 8 g
 
 // NW = waves per block (4 or 8): eight halve what a wave has to stage and to multiply, which is
 // what a projection of a few thousand rows -- one block per compute unit at most -- is short of.
-template <int ACT, int BITS, int TT, int WR, int NW>
+// FIRST: the inputs are requested ahead of the weights, all rows of the tile, whole panels (gemv_inputs_first).
+template <int ACT, int BITS, int TT, int WR, int NW, bool FIRST>
 __global__ __launch_bounds__(64 * NW) void gemv_mfma_kernel(GemvMfmaParams p) {
     constexpr int KW = NW / WR;                          // waves sharing out the stages of K
     constexpr uint32_t KP = 2048 / TT;                   // elements of an input panel
@@ -140,17 +141,24 @@ __global__ __launch_bounds__(64 * NW) void gemv_mfma_kernel(GemvMfmaParams p) {
 #pragma unroll
         for (int q = 0; q < TPW; ++q)
 #pragma unroll
-            for (int c = 0; c < CH; ++c)                     // past the end: the last piece, the last row
-                raw_all[q][c] = *reinterpret_cast<const uint4*>(p.x + (size_t)min((uint32_t)(wave + NW * q), p.n_tokens - 1u) * p.x_stride + k0 +
-                                                                min((uint32_t)(c * 64 + lane) * 8u, kp_len - 8u));
+            for (int c = 0; c < CH; ++c) {
+                const uint32_t t = wave + NW * q, e = (c * 64 + lane) * 8;
+                if constexpr (FIRST)                         // past the last row: that one again
+                    raw_all[q][c] = *reinterpret_cast<const uint4*>(p.x + (size_t)min(t, p.n_tokens - 1u) * p.x_stride + k0 + e);
+                else
+                    raw_all[q][c] = (t < p.n_tokens && e < kp_len)
+                                        ? *reinterpret_cast<const uint4*>(p.x + (size_t)t * p.x_stride + k0 + e)
+                                        : uint4{0u, 0u, 0u, 0u};
+            }
     };
-    auto stage_inputs = [&](uint32_t k0) {
-        const uint32_t kp_len = min(KP, p.n - k0);
+    auto stage_inputs = [&]() {
+        if constexpr (FIRST) {
 #pragma unroll
-        for (int q = 0; q < TPW; ++q)
+            for (int q = 0; q < TPW; ++q)
 #pragma unroll
-            for (int c = 0; c < CH; ++c)
-                if (wave + NW * q >= p.n_tokens || (uint32_t)(c * 64 + lane) * 8u >= kp_len) raw_all[q][c] = uint4{0u, 0u, 0u, 0u};
+                for (int c = 0; c < CH; ++c)
+                    if (wave + NW * q >= p.n_tokens) raw_all[q][c] = uint4{0u, 0u, 0u, 0u};
+        }
 #pragma unroll
         for (int q = 0; q < TPW; ++q) {
             const uint32_t t = wave + NW * q;
@@ -194,9 +202,11 @@ __global__ __launch_bounds__(64 * NW) void gemv_mfma_kernel(GemvMfmaParams p) {
     };
 
     // The first panel's inputs ahead of the weights: loads come back in their order, and the inputs, which the caches hold, are converted while the weights are on their way
-    // (16 tokens, 4 bits: 12,352 x 2048 10.1 -> 9.4 us, 2048 x 4096 10.5 -> 9.9).
-    request_inputs(0);
-    __builtin_amdgcn_sched_barrier(0);
+    // (16 tokens, 4 bits: 12,352 x 2048 9.9 -> 9.3 us, 2048 x 4096 9.6 -> 8.9).
+    if constexpr (FIRST) {
+        request_inputs(0);
+        __builtin_amdgcn_sched_barrier(0);
+    }
     // this wave's stages: wave_k, wave_k + KW, ...; its j-th one lands in the A arrays for even j
     const uint32_t n_my = (uint32_t)wave_k < n_stages ? (n_stages - wave_k + KW - 1) / KW : 0u;
     if (n_my > 0) issue_stage(wave_k, wa_w, ma_w);
@@ -336,8 +346,8 @@ __global__ __launch_bounds__(64 * NW) void gemv_mfma_kernel(GemvMfmaParams p) {
             close_panel();
             __syncthreads();                                     // every wave is through with the old panel
         }
-        if (k0 != 0) request_inputs(k0);
-        stage_inputs(k0);
+        if (!FIRST || k0 != 0) request_inputs(k0);
+        stage_inputs();
         while (j < n_my && (wave_k + j * KW) / SPP == panel) {   // wave-uniform
             const uint32_t st = wave_k + j * KW;
             if (j + 1 < n_my) __builtin_amdgcn_s_waitcnt(gm_vmcnt(N_LOADS)); else __builtin_amdgcn_s_waitcnt(gm_vmcnt(0));

@@ -25,6 +25,15 @@ inline bool few_rows_mfma(uint32_t bits, uint32_t n_tokens, uint32_t m, uint32_t
     return n_tokens == 3 && n == 2048 && m >= 8192;
 }
 
+// Whether the matrix-core product of few rows requests its inputs ahead of the weights, without a look at which there are: all rows of a tile of 16 or 32, so that it
+// pays where few are missing, and whole panels of 2048 or 1024 values.  4 bits, 2048 x 4096: 16 rows 9.6 -> 8.9 us, 9 rows 9.4 -> 9.0, 8 rows 9.4 both ways; 28 rows 18.2 -> 17.9, 24
+// rows 18.0 -> 17.9 and at 512 x 2048 9.7 -> 9.9.  8 bits, 12,352 x 2048: 16 rows 12.0 -> 11.2, 14 rows 11.9 -> 11.7, 12 rows 11.8 both ways and at 2048 x 4096 12.0 -> 12.2; 32 rows
+// 18.5 -> 18.0, 28 rows 18.2 -> 18.5.  Panels that are not whole, 16 rows of 1024 x 4096: 5.6 -> 5.8.
+inline bool gemv_inputs_first(uint32_t bits, uint32_t n_tokens, uint32_t n) {
+    if (n_tokens <= 16) return n % 2048 == 0 && n_tokens >= (bits == 4 ? 9u : 14u);
+    return n % 1024 == 0 && n_tokens >= (bits == 4 ? 28u : 31u);
+}
+
 // Whether a dense product can address `rows` input rows of `stride` values with 32-bit byte offsets (values of up to four bytes).
 inline bool dense_rows_fit(uint32_t rows, uint32_t stride) { return (uint64_t)rows * stride * 4 <= 0xFFFFFFFFull; }
 

@@ -103,3 +103,24 @@ def test_the_norm_before_them_needs_neither_workspace_nor_scratch_rows(bits, tok
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(got_h, want_h) and torch.equal(y, want)
+
+
+# panels of 2048 and of 1024 values, whole and not; one block of rows and a part of it, every number of them side by side
+@pytest.mark.parametrize("bits,below,from_", [(4, 8, 9), (8, 13, 14), (4, 27, 28), (8, 30, 31)])
+@pytest.mark.parametrize("m,n", [(10, 2048), (4100, 4096), (8200, 2048), (64, 3072), (64, 512)])
+def test_rows_are_the_same_whether_inputs_or_weights_are_requested_first(bits, below, from_, m, n):
+    import nvmai_amd as nv
+    from nvmai_amd import ops
+    say("inputs first", bits, from_, m, n)
+    ctx, gen = nv.Context(0, nv.ACT_BF16), torch.Generator(device="cuda").manual_seed(m + n)
+    w = nv.quantize_affine(ctx, torch.empty((m, n), device="cuda").normal_(0.0, 0.05, generator=gen).to(torch.bfloat16), bits)
+    x = torch.empty((32, n), device="cuda").normal_(0.0, 1.0, generator=gen).to(torch.bfloat16)
+    full = 16 if from_ <= 16 else 32
+    want = ops.affine_gemv(ctx, *w, bits, x[:below], m, n)
+    for tokens in (from_, full - 1, full):
+        got = ops.affine_gemv(ctx, *w, bits, x[:tokens], m, n)
+        assert torch.equal(got[:below], want), tokens
+        if tokens > below:      # a row among others and alone in the last place
+            swapped = ops.affine_gemv(ctx, *w, bits, x[:tokens].flip(0).contiguous(), m, n)
+            assert torch.equal(swapped.flip(0), got), tokens
+    ctx.close()

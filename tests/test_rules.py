@@ -109,3 +109,11 @@ def test_rows_that_one_launch_of_the_expert_block_does_not_take(rule):
     # several tokens: by the ends of their rows
     several = "rows_overlap(Rows16{x, 4096}, Rows16{y, 4096}, 3, 2048)"
     assert rule(("x", "y"), [(1 << 20, (1 << 20) + 2 * 4096 * 2 + 4094), (1 << 20, (1 << 20) + 2 * 4096 * 2 + 4096)], several) == [1, 0]
+
+
+def test_inputs_are_requested_first_for_whole_panels_of_nearly_whole_tiles(rule):
+    cases = [(b, t, n) for b in (4, 8) for t in range(3, 33) for n in range(512, 8193, 512)]
+    for (bits, tokens, n), first in zip(cases, rule(("bits", "tokens", "n"), cases, "gemv_inputs_first(bits, tokens, n)")):
+        tile = 16 if tokens <= 16 else 32
+        assert not first or (n % (2048 if tile == 16 else 1024) == 0 and tokens > tile // 2), (bits, tokens, n)
+        assert first or tokens < tile or n % 2048, (bits, tokens, n)
