@@ -402,7 +402,10 @@ __device__ __forceinline__ void expert_rows_body(const RowsParams& p, const Work
     load_stage(s0, 0);                            // both in flight while the inputs are staged
     load_stage(s1, 1);
 
-    if constexpr (HELD) {
+    // 8 bits of an expert: a question at run time, whose answer is known (rows of a form are never longer), keeps what stands in front of it apart from the staging.  Without it
+    // the compiler takes two registers more, and a wave less fits a SIMD (grouped down projection of 32 tokens: 98 and four, 42.4 us; 96 and five, 40.3; a layer 129.6 -> 127.7).
+    // At 4 bits it costs 1 us of a layer instead (16 tokens 63.3, 65.2 with it), and one row with the norm in front 0.9 (12,352 x 2048, 8 bits: 13.5, 14.4).
+    if (HELD && (BITS == 4 || MODE == ROWS_DENSE || p.n <= 2048u * PC)) {
         float m[MT];
         if constexpr (PRENORM) {
             // the normed rows are made here, in LDS behind the engine's own arrays, and read from there
