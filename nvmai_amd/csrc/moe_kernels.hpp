@@ -377,10 +377,10 @@ __device__ __forceinline__ void expert_rows_body(const RowsParams& p, const Work
     // Rows of up to 2048 (one input: 4096): every thread holds its PC pieces of eight elements of every input, which are read once, all loads in flight together,
     // and scaled from registers.  Of a dense launch, whose rows no table names, they are requested ahead of the weights: loads come back in their order, and
     // the inputs, which the caches hold, are staged while the weights are on their way (one token, 12,352 x 2048 codes of 4 bits 6.6 -> 5.9 us, 2048 x 4096 5.3 -> 5.1; the
-    // same for a norm's inputs changed nothing).
+    // same for a norm's inputs changed nothing).  One input in the longest blocks, which a large matrix takes, is staged behind them: 30,000 x 2048 at 8 bits 14.3 us, 14.7 ahead of them.
     constexpr int MT = TOKS ? TOKS : MAX_TOK;
     constexpr int PC = (NCH * SEG * EPC + 2047) / 2048;
-    constexpr bool HELD = PC == 1 || (PC == 2 && MT == 1 && MODE == ROWS_DENSE), AHEAD = HELD && MODE == ROWS_DENSE && !PRENORM;
+    constexpr bool HELD = PC == 1 || (PC == 2 && MT == 1 && MODE == ROWS_DENSE), AHEAD = HELD && MODE == ROWS_DENSE && !PRENORM && !(MT == 1 && ITERS == 8);
     float v[HELD ? MT * PC : 1][8];
     const uint32_t e0 = threadIdx.x * 8;
     auto load_inputs = [&]() {
