@@ -136,17 +136,21 @@ def run_config(nv, ctx, torch, layers, stride, bits, batch, steps, warmup, profi
             moe.decode_layer(layers[i % len(layers)]["desc"], xs[i % n_x], y)
         torch.cuda.synchronize()
         ctx.profile_enable(False)
-        names = ["router", "select", "group", "phase1", "phase2", "combine"]
+        names = {"router": nv.PROF_ROUTER, "select": nv.PROF_SELECT, "group": nv.PROF_GROUP, "phase1": nv.PROF_PHASE1, "phase2": nv.PROF_PHASE2,
+                 "combine": nv.PROF_COMBINE, "block": nv.PROF_MOE_ONE}
         kern = {}
-        for tag, name in enumerate(names):
+        for name, tag in names.items():
             ms, n = ctx.profile_read(tag)
             kern[name] = ms / max(n, 1) * 1e3      # microseconds per launch
         out["kernel_us"] = kern
         # phase 1 streams gate+up of every distinct routed expert and of the shared expert
         gate_up = 2 * (F * D * bits // 8 + 2 * F * (D // 64) * 2)
         p1_bytes = float(np.mean((distinct + 1) * gate_up + batch * D * 2 + (distinct + 1) * F * 4))
-        out["phase1_bytes"] = p1_bytes
-        out["phase1_gbps"] = p1_bytes / (kern["phase1"] * 1e-6) / 1e9
+        # (one token: the launch that holds the whole block, all bytes of the step)
+        out["one_launch"] = not kern["phase1"]
+        out["kernel_bytes"] = total / steps if out["one_launch"] else p1_bytes
+        out["kernel_name"] = "block" if out["one_launch"] else "phase1"
+        out["kernel_gbps"] = out["kernel_bytes"] / (kern[out["kernel_name"]] * 1e-6) / 1e9
     return out
 
 
@@ -983,9 +987,9 @@ def main():
             for b in (1, 2, 4, 8, 16, 32):
                 s = run_config(nv, ctx, torch, ls, st, bits, b, a.steps, a.warmup, profile=True)
                 print("sweep bits=%d batch=%d: %.1f GB/s (%.1f%% of HBM peak) %.2f us/step distinct=%.1f "
-                      "phase1 %.1f GB/s kernels(us)=%s"
+                      "%s %.1f GB/s kernels(us)=%s"
                       % (bits, b, s["gbps"], 100 * s["gbps"] / HBM_PEAK_GBPS, s["ms_per_step"] * 1e3,
-                         s["mean_distinct"], s["phase1_gbps"],
+                         s["mean_distinct"], s["kernel_name"], s["kernel_gbps"],
                          {k: round(v, 1) for k, v in s["kernel_us"].items()}), file=sys.stderr, flush=True)
             if bits != a.bits:
                 del ls
@@ -1022,14 +1026,15 @@ def decode_line(a, r, bits, batch, steps, warmup):
                    "mean_distinct_experts": round(r["mean_distinct"], 2),
                    "frac_of_hbm_peak": round(r["gbps"] / HBM_PEAK_GBPS, 4),
                    "kernel_us": {k: round(v, 2) for k, v in r["kernel_us"].items()}},
-        "roofline": {"kernel": "expert_rows_fast (routed + shared gate/up SwiGLU, phase 1)" if batch > 4 else
+        "roofline": {"kernel": "moe_one_kernel (router, selection, gate/up SwiGLU, down and sum)" if r["one_launch"] else
+                               "expert_rows_fast (routed + shared gate/up SwiGLU, phase 1)" if batch > 4 else
                                "expert_rows_routed / expert_rows_fast (gate/up SwiGLU, phase 1)", "bound": "hbm",
-                     "achieved": round(r["phase1_gbps"], 2), "peak": HBM_PEAK_GBPS, "unit": "GB/s",
-                     "frac": round(r["phase1_gbps"] / HBM_PEAK_GBPS, 4),
-                     "traffic": recorded_traffic(("decode", bits, batch))[0],
-                     "traffic_source": recorded_traffic(("decode", bits, batch))[1],
-                     "bytes_per_launch": round(r["phase1_bytes"]),
-                     "avg_launch_us": round(r["kernel_us"]["phase1"], 2)},
+                     "achieved": round(r["kernel_gbps"], 2), "peak": HBM_PEAK_GBPS, "unit": "GB/s",
+                     "frac": round(r["kernel_gbps"] / HBM_PEAK_GBPS, 4),
+                     "traffic": None if r["one_launch"] else recorded_traffic(("decode", bits, batch))[0],
+                     "traffic_source": None if r["one_launch"] else recorded_traffic(("decode", bits, batch))[1],
+                     "bytes_per_launch": round(r["kernel_bytes"]),
+                     "avg_launch_us": round(r["kernel_us"][r["kernel_name"]], 2)},
     }
 
 

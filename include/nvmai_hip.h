@@ -99,13 +99,15 @@ const char* nvmai_hip_status_string(int status);
  * (RealForwardRunner.swift:1129-1188): while enabled, each tagged kernel launch is
  * bracketed by events on its stream.  profile_read waits for the recorded events,
  * returns the summed milliseconds and launch count of one tag and leaves the
- * records in place; profile_enable(…, 1) clears them. */
+ * records in place; profile_enable(…, 1) clears them.  A launch that holds several steps has one
+ * tag: NVMAI_PROF_MOE_ONE the whole MoE block of one token, NVMAI_PROF_ROUTER the router, the selection
+ * and the work list of a small batch (NVMAI_PROF_GROUP where these are launches of their own). */
 enum {
     NVMAI_PROF_ROUTER = 0, NVMAI_PROF_SELECT = 1, NVMAI_PROF_GROUP = 2, NVMAI_PROF_PHASE1 = 3,
     NVMAI_PROF_PHASE2 = 4, NVMAI_PROF_COMBINE = 5, NVMAI_PROF_KV_QUANT = 6, NVMAI_PROF_ATTN_PARTIAL = 7,
     NVMAI_PROF_ATTN_COMBINE = 8, NVMAI_PROF_SOFTMAX = 9, NVMAI_PROF_SAMPLE = 10,
     NVMAI_PROF_PREFILL_GROUP = 11, NVMAI_PROF_PREFILL_GEMM1 = 12, NVMAI_PROF_PREFILL_GEMM2 = 13,
-    NVMAI_PROF_PREFILL_COMBINE = 14, NVMAI_PROF_TAGS = 16
+    NVMAI_PROF_PREFILL_COMBINE = 14, NVMAI_PROF_MOE_ONE = 15, NVMAI_PROF_TAGS = 16
 };
 int nvmai_hip_profile_enable(nvmai_hip_ctx* ctx, int on);
 int nvmai_hip_profile_read(nvmai_hip_ctx* ctx, int tag, double* total_ms, uint32_t* launches);

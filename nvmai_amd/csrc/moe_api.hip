@@ -410,34 +410,6 @@ void launch_down_combine(int act, uint32_t bits, const DownCombineParams& p, hip
     }
 }
 
-// The same in one launch (moe_one_kernels.hpp), for one token.  False, having launched nothing, for shapes that have no such form: rows of gate and up that a wave reads
-// whole and whose inputs a block holds (d up to 2048), rows of the down projection of 16 or 32 pieces (64 would be held in more registers than the others leave), more blocks than one launch
-// numbers, outputs that lie over what the launch reads or over one another (block_overlaps).
-template <int ACT, int BITS, int NCH>
-bool launch_moe_one_t(const MoeOneParams& p, uint32_t blocks, hipStream_t s) {
-    const size_t rows_lds = moe_one_rows_lds(p.rows.n, NCH);
-    const uint32_t chunks = p.down.n * BITS / 128;
-#define NVMAI_ONE(SEG)                                                                               \
-    do {                                                                                             \
-        const size_t down_lds = moe_one_down_lds<BITS, SEG>(p.slots);                                \
-        const size_t lds = rows_lds > down_lds ? rows_lds : down_lds;                                \
-        if (lds > 60 * 1024) return false;                                                           \
-        moe_one_kernel<ACT, BITS, NCH, SEG><<<blocks, MOE_ONE_THREADS, lds, s>>>(p);                             \
-        return true;                                                                                 \
-    } while (0)
-    if (chunks == 16) NVMAI_ONE(16);
-    if (chunks == 32) NVMAI_ONE(32);
-#undef NVMAI_ONE
-    return false;
-}
-
-template <int ACT>
-bool launch_moe_one_act(uint32_t bits, const MoeOneParams& p, uint32_t blocks, hipStream_t s) {
-    if (p.rows.n * bits == 64 * 128) return bits == 8 ? launch_moe_one_t<ACT, 8, 1>(p, blocks, s) : launch_moe_one_t<ACT, 4, 1>(p, blocks, s);
-    if (p.rows.n * bits == 128 * 128 && bits == 8) return launch_moe_one_t<ACT, 8, 2>(p, blocks, s);
-    return false;
-}
-
 Rows16 rows16(const void* at, uint32_t stride) { return Rows16{reinterpret_cast<uintptr_t>(at), stride}; }
 
 bool prologue_overlaps(const RouterParams& r) {
@@ -445,9 +417,12 @@ bool prologue_overlaps(const RouterParams& r) {
                                     rows16(r.pre_normed_out, r.pre_normed_stride), r.tokens, r.d);
 }
 
-bool launch_moe_one(const nvmai_hip_ctx* ctx, uint32_t bits, MoeOneParams& p, hipStream_t s) {
-    const uint32_t T = p.sel.tokens, D = p.rows.n, F = p.rows.rows;
-    if (T != 1 || D > 2048 || D % 256 || F < 64) return false;
+// Whether the same is made in one launch (moe_one_kernels.hpp), for one token, and the rest of what that launch takes: rows of gate and up that a wave reads
+// whole and whose inputs a block holds (d up to 2048), rows of the down projection of 16 or 32 pieces (64 would be held in more registers than the others leave), no more blocks than one
+// launch numbers, no outputs that lie over what the launch reads or over one another (block_overlaps).
+bool moe_one_fits(const nvmai_hip_ctx* ctx, uint32_t bits, MoeOneParams& p) {
+    const uint32_t T = p.sel.tokens, D = p.rows.n, F = p.rows.rows, chunks = D * bits / 128, seg = F * bits / 128;
+    if (T != 1 || D > 2048 || D % 256 || F < 64 || (chunks != 64 && (chunks != 128 || bits != 8)) || (seg != 16 && seg != 32)) return false;
     const RouterParams& r = p.router;
     if ((rows_chunks(r.router.kind, D) + 31) / 32 > 8) return false;
     if (block_overlaps(rows16(r.x, r.x_stride), rows16(r.pre_delta, r.pre_delta_stride), rows16(r.pre_hidden_out, r.pre_hidden_stride),
@@ -459,10 +434,32 @@ bool launch_moe_one(const nvmai_hip_ctx* ctx, uint32_t bits, MoeOneParams& p, hi
     p.down_blocks = (D + DC_ROWS - 1) / DC_ROWS;
     const uint64_t blocks = (uint64_t)T * (p.router_blocks + p.slots * p.rows.blocks_per_entry + 1 + p.down_blocks);
     const uint64_t words = (uint64_t)T * moe_one_token_words(r.num_experts, p.slots, F);
-    if (blocks > HAND_BLOCKS || words > HAND_WORDS) return false;
+    const size_t rows_lds = moe_one_rows_lds(D, chunks / 64), down_lds = moe_one_down_lds(bits, seg, p.slots);
+    p.blocks = (uint32_t)blocks;
+    p.lds = (uint32_t)(rows_lds > down_lds ? rows_lds : down_lds);
+    if (blocks > HAND_BLOCKS || words > HAND_WORDS || p.lds > 60 * 1024) return false;
     p.hand = ctx->hand;
     p.hand.used = (uint32_t)words;
-    return ctx->act == ACT_BF16 ? launch_moe_one_act<ACT_BF16>(bits, p, (uint32_t)blocks, s) : launch_moe_one_act<ACT_FP16>(bits, p, (uint32_t)blocks, s);
+    return true;
+}
+
+template <int ACT, int BITS, int NCH>
+void launch_moe_one_t(const MoeOneParams& p, hipStream_t s) {
+    if (p.down.n * BITS / 128 == 16) moe_one_kernel<ACT, BITS, NCH, 16><<<p.blocks, MOE_ONE_THREADS, p.lds, s>>>(p);
+    else moe_one_kernel<ACT, BITS, NCH, 32><<<p.blocks, MOE_ONE_THREADS, p.lds, s>>>(p);
+}
+
+template <int ACT>
+void launch_moe_one_act(uint32_t bits, const MoeOneParams& p, hipStream_t s) {
+    if (bits == 4) launch_moe_one_t<ACT, 4, 1>(p, s);
+    else if (p.rows.n == 1024) launch_moe_one_t<ACT, 8, 1>(p, s);
+    else launch_moe_one_t<ACT, 8, 2>(p, s);
+}
+
+// p as moe_one_fits left it.
+void launch_moe_one(int act, uint32_t bits, const MoeOneParams& p, hipStream_t s) {
+    if (act == ACT_BF16) launch_moe_one_act<ACT_BF16>(bits, p, s);
+    else launch_moe_one_act<ACT_FP16>(bits, p, s);
 }
 
 // Router, selection and work list in one launch (router_group_kernels.hpp).  False, having launched nothing, for what has no such form: tokens
@@ -1162,8 +1159,10 @@ int decode_layer_impl(nvmai_hip_ctx* ctx, nvmai_stream stream, const nvmai_moe_l
             one.down.has_shared = has_shared ? 1 : 0; one.down.tokens = T; one.down.top_k = K; one.down.rows = D; one.down.n = F;
             one.down.y_stride = y_stride; one.down.y = y;
             one.stats = rs;
-            ProfScope ps(ctx, NVMAI_PROF_PHASE1, s);
-            if (launch_moe_one(ctx, L->bits, one, s)) return launch_status();
+            if (moe_one_fits(ctx, L->bits, one)) {
+                { ProfScope ps(ctx, NVMAI_PROF_MOE_ONE, s); launch_moe_one(ctx->act, L->bits, one, s); }
+                return launch_status();
+            }
         }
         { ProfScope ps(ctx, NVMAI_PROF_ROUTER, s); rc = run_router(ctx, rp, s); }
         if (rc) return rc;

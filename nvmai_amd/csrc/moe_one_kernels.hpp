@@ -23,6 +23,7 @@ struct MoeOneParams {
     uint32_t router_blocks;      // per token
     uint32_t slots;
     uint32_t down_blocks;        // per token
+    uint32_t blocks, lds;        // of the launch
 };
 
 constexpr uint32_t MOE_ONE_THREADS = 512;                // fewer blocks than of 256, and so fewer that ask for the same words
@@ -50,8 +51,7 @@ struct DownActs {
     static __device__ uint32_t at(uint32_t f) { return ((f % EPC / 4) * (SEG + 1) + f / EPC) * 4 + f % 4; }
 };
 
-template <int BITS, int SEG>
-__host__ __device__ inline size_t moe_one_down_lds(uint32_t slots) { return (size_t)slots * (Chunk<BITS>::elems / 4) * (SEG + 1) * 16; }
+inline size_t moe_one_down_lds(uint32_t bits, uint32_t seg, uint32_t slots) { return (size_t)slots * (128 / bits / 4) * (seg + 1) * 16; }
 
 struct MoeOneToken {
     uint64_t *first, *acts;      // copy 0
@@ -287,7 +287,7 @@ __device__ __forceinline__ bool moe_one_rows(const MoeOneParams& p, uint32_t e, 
 }
 
 // Bytes of LDS of a block of gate and up.
-__host__ __device__ inline size_t moe_one_rows_lds(uint32_t n, int nch) { return (size_t)n * 2 + (size_t)nch * 64 * 8 + 16 + (size_t)2 * n * 2; }
+inline size_t moe_one_rows_lds(uint32_t n, uint32_t nch) { return (size_t)n * 2 + (size_t)nch * 64 * 8 + 16 + (size_t)2 * n * 2; }
 
 // A unit is 64 / SEG output rows of one slot; the block's waves share those of its DC_ROWS rows.
 template <int ACT, int BITS, int SEG>

@@ -14,7 +14,7 @@ from ._lib import (ExpertOffsets, GdnConfig, GemvPart, GenerationConfig as _CGen
 ACT_BF16, ACT_FP16, ACT_FP32 = 0, 1, 2
 (PROF_ROUTER, PROF_SELECT, PROF_GROUP, PROF_PHASE1, PROF_PHASE2, PROF_COMBINE, PROF_KV_QUANT,
  PROF_ATTN_PARTIAL, PROF_ATTN_COMBINE, PROF_SOFTMAX, PROF_SAMPLE, PROF_PREFILL_GROUP,
- PROF_PREFILL_GEMM1, PROF_PREFILL_GEMM2, PROF_PREFILL_COMBINE) = range(15)
+ PROF_PREFILL_GEMM1, PROF_PREFILL_GEMM2, PROF_PREFILL_COMBINE, PROF_MOE_ONE) = range(16)
 _ACT_TORCH = {ACT_BF16: torch.bfloat16, ACT_FP16: torch.float16, ACT_FP32: torch.float32}
 
 

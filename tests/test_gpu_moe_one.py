@@ -135,3 +135,20 @@ def test_output_in_place_of_the_prologues_rows(nv, looks):
     moe.decode_layer_prenorm(layer, hidden, delta, weight, both, n2, both)
     assert torch.equal(n2, normed) and torch.equal(both, y)
     ctx.close()
+
+
+def test_time_is_booked_under_the_launches_that_are_made(nv):
+    # the one launch under a tag of its own; its refusal (an output in place of the input, more tokens) books nothing
+    print("one launch, spans", flush=True)
+    ctx = nv.Context(0, nv.ACT_BF16)
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    layer, keep = _layer(nv, ctx, gen, 2048, 512, 16, 8, 4, True, True)
+    moe = nv.MoE(ctx, 4)
+    tags = (nv.PROF_MOE_ONE, nv.PROF_ROUTER, nv.PROF_PHASE1, nv.PROF_PHASE2)
+    for tokens, in_place, want in ((1, False, (1, 0, 0, 0)), (1, True, (0, 1, 1, 1)), (2, False, (0, 1, 1, 1)), (4, False, (0, 1, 1, 1))):
+        x = torch.zeros((tokens, 2048), dtype=torch.bfloat16, device="cuda")
+        ctx.profile_enable(True)
+        moe.decode_layer(layer, x, x if in_place else torch.empty_like(x))
+        ctx.profile_enable(False)
+        assert tuple(ctx.profile_read(tag)[1] for tag in tags) == want, (tokens, in_place)
+    ctx.close()
