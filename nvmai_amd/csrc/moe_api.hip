@@ -422,7 +422,7 @@ bool prologue_overlaps(const RouterParams& r) {
 // launch numbers, no outputs that lie over what the launch reads or over one another (block_overlaps).
 bool moe_one_fits(const nvmai_hip_ctx* ctx, uint32_t bits, MoeOneParams& p) {
     const uint32_t T = p.sel.tokens, D = p.rows.n, F = p.rows.rows, chunks = D * bits / 128, seg = F * bits / 128;
-    if (T != 1 || D > 2048 || D % 256 || F < 64 || (chunks != 64 && (chunks != 128 || bits != 8)) || (seg != 16 && seg != 32)) return false;
+    if (T != MOE_ONE_TOKENS || D > 2048 || D % 256 || F < 64 || (chunks != 64 && (chunks != 128 || bits != 8)) || (seg != 16 && seg != 32)) return false;
     const RouterParams& r = p.router;
     if ((rows_chunks(r.router.kind, D) + 31) / 32 > 8) return false;
     if (block_overlaps(rows16(r.x, r.x_stride), rows16(r.pre_delta, r.pre_delta_stride), rows16(r.pre_hidden_out, r.pre_hidden_stride),

@@ -152,3 +152,18 @@ def test_time_is_booked_under_the_launches_that_are_made(nv):
         ctx.profile_enable(False)
         assert tuple(ctx.profile_read(tag)[1] for tag in tags) == want, (tokens, in_place)
     ctx.close()
+
+
+def test_statistics_where_scores_are_not_numbers(nv):
+    # experts are chosen again where no score is left that is a number; one token's statistics name its slots and top_k either way, as the three launches do
+    print("one launch, statistics", flush=True)
+    ctx = nv.Context(0, nv.ACT_BF16)
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    layer, keep = _layer(nv, ctx, gen, 1024, 256, 12, 8, 8, True, True)
+    router = keep[1].view(torch.bfloat16)
+    for bad in (0, 1, 5, 12):
+        router[:] = 0.01
+        router[12 - bad:] = float("nan")
+        one, three = _both(nv, ctx, layer, torch.ones((1, 1024), device="cuda", dtype=torch.bfloat16))
+        assert torch.equal(one[1], three[1]) and one[3].tolist() == three[3].tolist() == [9, 8], bad
+    ctx.close()
