@@ -167,3 +167,39 @@ def test_statistics_where_scores_are_not_numbers(nv):
         one, three = _both(nv, ctx, layer, torch.ones((1, 1024), device="cuda", dtype=torch.bfloat16))
         assert torch.equal(one[1], three[1]) and one[3].tolist() == three[3].tolist() == [9, 8], bad
     ctx.close()
+
+
+@pytest.mark.parametrize("act", ["ACT_BF16", "ACT_FP16"])
+@pytest.mark.parametrize("looks", [1 << 14, 0])
+@pytest.mark.parametrize("with_delta", [False, True])
+@pytest.mark.parametrize("bits,d,f,E,k,shared,gated,kind,scales", [
+    (4, 2048, 512, 256, 8, True, True, 16, False), (8, 2048, 512, 30, 8, True, True, 16, True), (8, 1024, 256, 300, 4, False, False, 8, False)])
+def test_with_the_norm_before_it(nv, act, looks, with_delta, bits, d, f, E, k, shared, gated, kind, scales):
+    # the residual add and the norm inside the launch, as a layer of a decode step takes it, against the norm's own launch and the three
+    print("one launch with its norm", act, looks, with_delta, bits, d, f, E, k, flush=True)
+    ctx = nv.Context(0, getattr(nv, act))
+    assert nv.lib.nvmai_hip_ctx_wait_limit(ctx.handle, looks) == 0
+    gen = torch.Generator(device="cuda").manual_seed(E + d)
+    layer, keep = _layer(nv, ctx, gen, d, f, E, k, bits, shared, gated, kind, scales)
+    row = lambda: torch.empty((1, d), device="cuda").normal_(0.0, 1.0, generator=gen).to(ctx.dtype)
+    weight, closing = (torch.empty(d, device="cuda").uniform_(0.5, 1.5, generator=gen).to(torch.bfloat16) for _ in range(2))
+    moe, eps = nv.MoE(ctx, bits), 1e-5
+    new = lambda: (torch.zeros((1, k), dtype=torch.int32, device="cuda"), torch.zeros((1, k), dtype=torch.float16, device="cuda"), torch.zeros(2, dtype=torch.int32, device="cuda"))
+    for turn in range(3):
+        hidden, delta = row(), row() if with_delta else None
+        stream, stats = hidden.clone(), torch.zeros(2, dtype=torch.int32, device="cuda")
+        zero = torch.zeros_like(hidden)
+        normed = nv.ops.residual_add_rmsnorm(ctx, stream, delta if with_delta else zero, weight, eps=eps)
+        want = normed.clone()
+        want, want_idx, want_w = moe.decode_layer(layer, want, want, want_routes=True, stats=stats)
+        h, n, y, (idx, w, s) = row(), row(), row(), new()
+        moe.decode_layer_prenorm(layer, hidden, delta, weight, h, n, y, eps, idx, w, s)
+        for got, wanted in zip((h, n, y, idx, w, s), (stream, normed, want, want_idx, want_w, stats)):
+            assert torch.equal(got.view(torch.uint8), wanted.view(torch.uint8)), turn
+        # with the end of the layer behind it
+        ended = nv.ops.residual_add_rmsnorm(ctx, stream, want, closing, eps=eps)
+        h, n, y, (idx, w, s), after = row(), row(), row(), new(), row()
+        moe.decode_layer_norms(layer, hidden, delta, weight, h, n, y, closing, after, eps, idx, w, s)
+        for got, wanted in zip((h, n, y, after, idx, w, s), (stream, normed, want, ended, want_idx, want_w, stats)):
+            assert torch.equal(got.view(torch.uint8), wanted.view(torch.uint8)), turn
+    ctx.close()
