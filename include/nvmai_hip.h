@@ -29,6 +29,10 @@
  *     They and a word per tile that counts its blocks belong to the one stream of the ctx, as the workspace does: products
  *     of one ctx that run at the same time, on two streams or in two replayed graphs, may add each other's sums, and may leave
  *     a count behind that spoils later products of that ctx.
+ *     The same holds for the words in which the blocks of an MoE step of one token, or of a few, hand values to one another (2 MB): they carry
+ *     the number of the launch, which every block counts for itself.  Two such steps of one ctx that run at the same time may take each other's
+ *     values, and may leave blocks with different numbers behind, after which every later such step of that ctx may be wrong without
+ *     an error.  Streams that run at the same time each need a ctx of their own.
  * Data formats (reference file:line):
  *   - weights: affine group-64 codes, 4 bit (two per byte, element 2k in the low
  *     nibble of byte k) or 8 bit, plus one BF16 scale and one BF16 bias per group
