@@ -3,7 +3,7 @@
 // As three launches (router_logits_kernel, expert_rows_routed, down_combine_kernel) the block is bound by their chain: 4.4 + 7.2 + 7.4 us at 4
 // bits, 17 MB of weights among them, which HBM delivers in 3.4.  Here the steps are blocks of one launch that hand their values on (hand.hpp): the inputs of gate and up are
 // staged while the router's rows are summed, and a block of the down projection asks for its experts' rows as soon as the router has chosen, beside gate and up.  One token, 2048 x 512, 256
-// experts: 18.2 -> 14.4 us a block, 24 -> 19 with the norm before it, at 4 and at 8 bits.  By the clock in its blocks: inputs staged at 1.9 us, logits at 3.0, seen at 5.3, experts chosen at
+// experts: 18.2 -> 14.3 to 15.2 us a block, from process to process, 24 -> 19 with the norm before it, at 4 and at 8 bits.  By the clock in its blocks: inputs staged at 1.9 us, logits at 3.0, seen at 5.3, experts chosen at
 // 5.6 to 6.5, the first rows of gate and up at 7.4 and the last at 8.4, all seen at 10.0, taken at 11.6, summed at 13.2.  Two tokens take longer so than in three launches (23.3 and 21.7 us at 4 bits, 27.7 and
 // 23.1 at 8): the blocks do not all fit the device at once, and each asks for all activations of its token.
 #pragma once
